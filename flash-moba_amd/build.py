@@ -15,6 +15,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libflash_moba_hip.so")
+HOST_MODULE = "flash_moba_host"  # the eager host path (csrc/torch_ops.cpp), a Python extension beside the library
+HOST_LIB = os.path.join(LIBDIR, HOST_MODULE + ".so")
 SOURCES = ["fmoba_host.hip", "mean_pool.hip", "topk_csc.hip", "varlen_sort.hip", "attn_fwd.hip", "attn_fwd_rows.hip", "attn_bwd.hip", "attn_bwd_wide.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -40,11 +42,43 @@ def _compile(src: str, objdir: str) -> str:
     return obj
 
 
+def _run(cmd, what):
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("%s failed:\n%s\n%s" % (what, r.stdout, r.stderr))
+
+
+def _compile_host_module(objdir: str) -> str:
+    """torch_ops.cpp against the installed torch (host code only: the host compiler)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    inc = include_paths() + [os.path.join(os.path.dirname(os.path.dirname(hipcc())), "include"), sysconfig.get_paths()["include"]]
+    obj = os.path.join(objdir, "torch_ops.o")
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          "-DTORCH_EXTENSION_NAME=" + HOST_MODULE, "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
+         + ["-isystem" + d for d in inc] + ["-c", os.path.join(CSRC, "torch_ops.cpp"), "-o", obj], "compiling the host module")
+    return obj
+
+
+def _link_host_module(obj: str) -> None:
+    from torch.utils.cpp_extension import library_paths
+
+    tmp = HOST_LIB + ".tmp"
+    _run([os.environ.get("CXX", "g++"), "-shared", "-o", tmp, obj, "-L" + LIBDIR, "-lflash_moba_hip", "-Wl,-rpath,$ORIGIN"]
+         + ["-L" + d for d in library_paths()] + ["-l" + x for x in ("torch", "torch_cpu", "torch_hip", "torch_python", "c10", "c10_hip")],
+         "linking the host module")
+    os.replace(tmp, HOST_LIB)
+
+
 def build_library(verbose: bool = True, jobs: int = 6) -> str:
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_compile_host_module, objdir)
         objs = list(ex.map(lambda s: _compile(s, objdir), SOURCES))
     tmp = LIB + ".tmp"
     cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp] + objs
@@ -52,6 +86,7 @@ def build_library(verbose: bool = True, jobs: int = 6) -> str:
     if r.returncode != 0:
         raise RuntimeError("link failed:\n%s\n%s" % (r.stdout, r.stderr))
     os.replace(tmp, LIB)
+    _link_host_module(host.result())
     if verbose:
         print("built", LIB, os.path.getsize(LIB), "bytes")
     return LIB

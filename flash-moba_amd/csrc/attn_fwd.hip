@@ -685,7 +685,8 @@ extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phase
     FMOBA_LAUNCH_CHECK("attn_fwd(empty)");
     return 0;
   }
-  FMOBA_REQUIRE(a->k && a->v && a->col_offsets && a->col_nnz && a->row_indices, "attn_fwd: null k/v/CSC pointer");
+  FMOBA_REQUIRE(a->k && a->v, "attn_fwd: null k/v pointer");
+  FMOBA_REQUIRE((a->col_offsets && a->col_nnz && a->row_indices) || (a->selection_bits && fwd_use_rows(*a)), "attn_fwd: null CSC pointer");
   const int64_t st[] = {a->q_row_stride, a->q_head_stride, a->k_row_stride, a->k_head_stride,
                         a->v_row_stride, a->v_head_stride, a->o_row_stride, a->o_head_stride};
   for (int64_t x : st) FMOBA_REQUIRE(x % 8 == 0, "attn_fwd: strides must be multiples of 8 elements");

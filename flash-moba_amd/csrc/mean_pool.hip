@@ -5,14 +5,41 @@
 
 namespace fmoba {
 
+// What the first launch of the gated path does besides the pooling, so that it need not be a launch of its own (about
+// five microseconds each on the device, and as much on the host): offsets of the pooled sequences, and counters of the
+// gating that have to be zero.
+struct PoolExtra {
+  int32_t *cu_km;   // null: the offsets are an input (a.cu_seqlens_km)
+  int32_t *clear;   // 16-byte aligned, clear_vec16 pieces of 16 bytes
+  int64_t clear_vec16;
+};
+
 // grid (max_chunks, batch, ceil(vecs / 64)), block 256 = 4 waves.
 // A wave owns 64 consecutive 16-byte vectors of the (heads_k*head_dim) axis; the four
 // waves of the block split the rows of the chunk and reduce through LDS.
 template <typename T>
-__global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a) {
+__global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x) {
   const int c = blockIdx.x, b = blockIdx.y;
   const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1];
   const int row0 = seq_start + c * a.chunk;
+  if (x.clear_vec16) {
+    const int64_t nthr = (int64_t)gridDim.x * gridDim.y * gridDim.z * 256;
+    int64_t i = (((int64_t)blockIdx.z * gridDim.y + b) * gridDim.x + c) * 256 + threadIdx.x;
+    for (; i < x.clear_vec16; i += nthr) *reinterpret_cast<Pack8 *>(x.clear + 4 * i) = zero_pack8();
+  }
+  // first pooled row of the sequence: the chunks of the sequences before it, counted by the wave that writes the row
+  const bool offsets = x.cu_km != nullptr;
+  const bool tells = offsets && c == 0 && blockIdx.z == 0;
+  int before = 0;
+  if (offsets && threadIdx.x < 64 && (tells || row0 < seq_end)) {
+    for (int i = threadIdx.x; i < b; i += 64) before += (a.cu_seqlens_k[i + 1] - a.cu_seqlens_k[i] + a.chunk - 1) / a.chunk;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) before += __shfl_xor(before, o, 64);
+    if (tells && threadIdx.x == 0) {
+      x.cu_km[b] = before;
+      if (b == a.batch - 1) x.cu_km[a.batch] = before + (seq_end - seq_start + a.chunk - 1) / a.chunk;
+    }
+  }
   if (row0 >= seq_end) return;
   const int n = min(a.chunk, seq_end - row0);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -63,7 +90,7 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a) 
     Pack8 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o.w[i] = pack2<T>(s[2 * i], s[2 * i + 1]);
-    const int out_row = a.cu_seqlens_km[b] + c;
+    const int out_row = (offsets ? before : a.cu_seqlens_km[b]) + c;
     uint16_t *dst = reinterpret_cast<uint16_t *>(a.km) + (int64_t)out_row * a.km_row_stride + (int64_t)head * a.km_head_stride + d0;
     *reinterpret_cast<Pack8 *>(dst) = o;
   }
@@ -106,7 +133,8 @@ extern "C" int fmoba_chunk_offsets(const int32_t *cu_seqlens, int32_t *cu_seqlen
   return 0;
 }
 
-extern "C" int fmoba_mean_pool(const fmoba_mean_pool_args *a, void *stream) {
+// `extra`: cu_km and clear_* of PoolExtra
+static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &extra, void *stream) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "mean_pool: null args");
   FMOBA_REQUIRE(a->dtype == FMOBA_DTYPE_F16 || a->dtype == FMOBA_DTYPE_BF16, "mean_pool: only fp16 and bf16 are supported");
@@ -124,9 +152,25 @@ extern "C" int fmoba_mean_pool(const fmoba_mean_pool_args *a, void *stream) {
   FMOBA_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "mean_pool: batch or heads*dim too large for the launch grid");
   hipStream_t s = (hipStream_t)stream;
   if (a->dtype == FMOBA_DTYPE_BF16)
-    hipLaunchKernelGGL(mean_pool_kernel<bf16_t>, grid, dim3(256), 0, s, *a);
+    hipLaunchKernelGGL(mean_pool_kernel<bf16_t>, grid, dim3(256), 0, s, *a, extra);
   else
-    hipLaunchKernelGGL(mean_pool_kernel<f16_t>, grid, dim3(256), 0, s, *a);
+    hipLaunchKernelGGL(mean_pool_kernel<f16_t>, grid, dim3(256), 0, s, *a, extra);
   FMOBA_LAUNCH_CHECK("mean_pool");
   return 0;
 }
+
+extern "C" int fmoba_mean_pool(const fmoba_mean_pool_args *a, void *stream) { return mean_pool_run(a, fmoba::PoolExtra{nullptr, nullptr, 0}, stream); }
+
+namespace fmoba {
+// every block counts the sequences before its own: up to this many it is no more than a handful of loads per lane
+constexpr int kPoolOffsetsBatch = 1024;
+
+int mean_pool_with_offsets(const fmoba_mean_pool_args *a, int32_t *clear, int64_t clear_vec16, void *stream) {
+  int32_t *cu_km = const_cast<int32_t *>(a->cu_seqlens_km);
+  if (a->batch > kPoolOffsetsBatch) {
+    if (int rc = fmoba_chunk_offsets(a->cu_seqlens_k, cu_km, a->batch, a->chunk, stream)) return rc;
+    cu_km = nullptr;
+  }
+  return mean_pool_run(a, PoolExtra{cu_km, clear, clear_vec16}, stream);
+}
+}  // namespace fmoba

@@ -21,7 +21,7 @@ constexpr int kSegRows = 2048;   // rows per counting segment (fewer for small p
 struct TopkParams {
   fmoba_fused_topk_args a;
   uint32_t *sel;      // [heads][W][total_q] selection bits, word w covers chunks 32w..32w+31
-  int32_t *segcnt;    // [batch][heads][nseg][max_cols]
+  int32_t *segcnt;    // [batch][heads][nseg][max_cols], null if no lists are wanted
   int32_t W, nseg, max_cols, seg_rows;
 };
 
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
       if (!valid) w = 0u;
       if (valid && hh == 0) selp[(int64_t)t * a.total_q] = w;
       // per-chunk counts of this wave's 32 rows (both halves of the wave hold the rows' words)
-      if (__any(w != 0u)) {
+      if (p.segcnt != nullptr && __any(w != 0u)) {
         const int mycnt = bit_column_count32(w, lane);
         if (lane < 32 && mycnt) atomicAdd(&sHist[t * 32 + lane], mycnt);
       }
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
   __syncthreads();
   for (int c = tid; c < p.W * 32 && c < p.max_cols; c += 256) {
     const int v = sHist[c];
-    if (v) atomicAdd(&p.segcnt[(((int64_t)b * a.heads + h) * p.nseg + seg) * p.max_cols + c], v);
+    if (v && p.segcnt != nullptr) atomicAdd(&p.segcnt[(((int64_t)b * a.heads + h) * p.nseg + seg) * p.max_cols + c], v);
   }
 }
 
@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256, CAP < kBigCap ? 2 : 1) void topk_gate_big_kern
     }
     for (int c = tid; c < wn * 32; c += 256) {
       const int v = sHist[c];
-      if (v) atomicAdd(&p.segcnt[(((int64_t)b * a.heads + h) * p.nseg + seg) * p.max_cols + 32 * w0 + c], v);
+      if (v && p.segcnt != nullptr) atomicAdd(&p.segcnt[(((int64_t)b * a.heads + h) * p.nseg + seg) * p.max_cols + 32 * w0 + c], v);
     }
   }
 }
@@ -1413,7 +1413,7 @@ __global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void topk_gate_stream_kernel(
     }
     for (int c = tid; c < wn * 32; c += 256) {
       const int v = sHist[c];
-      if (v) atomicAdd(&p.segcnt[(((int64_t)b * a.heads + h) * p.nseg + seg) * p.max_cols + 32 * w0 + c], v);
+      if (v && p.segcnt != nullptr) atomicAdd(&p.segcnt[(((int64_t)b * a.heads + h) * p.nseg + seg) * p.max_cols + 32 * w0 + c], v);
     }
   }
 }
@@ -1741,8 +1741,13 @@ static int launch_gate_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
 }
 }  // namespace fmoba
 
-// The call behind both entry points: everything of `a` except its workspace fields, which come as arguments.
-static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_t workspace_bytes, void *stream) {
+namespace fmoba {
+int mean_pool_with_offsets(const fmoba_mean_pool_args *a, int32_t *clear, int64_t clear_vec16, void *stream);
+}
+// The call behind the entry points: everything of `a` except its workspace fields, which come as arguments.  `pool`: the
+// pooling pass that comes first and clears the segment counts; null: the chunk means are there already.
+static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_t workspace_bytes, const fmoba_mean_pool_args *pool, bool lists,
+                          void *stream) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "fused_topk: null args");
   FMOBA_REQUIRE(a->dtype == FMOBA_DTYPE_F16 || a->dtype == FMOBA_DTYPE_BF16, "FlashMoBA only supports fp16 and bf16 data types");
@@ -1754,8 +1759,8 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   FMOBA_REQUIRE(a->chunk > 0, "moba_chunk_size must be positive");
   FMOBA_REQUIRE(a->total_q >= 0 && a->max_seqlen_q >= 0 && a->max_seqlen_k >= 0, "negative size");
   FMOBA_REQUIRE(a->cu_seqlens_q && a->cu_seqlens_k && a->cu_seqlens_km, "fused_topk: null cu_seqlens pointer");
-  FMOBA_REQUIRE((a->col_offsets && a->col_nnz) || a->max_seqlen_k == 0, "fused_topk: null col_offsets/col_nnz pointer");
-  FMOBA_REQUIRE(a->flat_indices || (int64_t)a->total_q * a->heads * a->topk == 0, "fused_topk: null flat_indices pointer");
+  FMOBA_REQUIRE((a->col_offsets && a->col_nnz) || a->max_seqlen_k == 0 || !lists, "fused_topk: null col_offsets/col_nnz pointer");
+  FMOBA_REQUIRE(a->flat_indices || (int64_t)a->total_q * a->heads * a->topk == 0 || !lists, "fused_topk: null flat_indices pointer");
   FMOBA_REQUIRE((a->raw_indices == nullptr) == (a->raw_values == nullptr), "fused_topk: raw_indices and raw_values go together");
   hipStream_t s = (hipStream_t)stream;
   const int max_cols = ceil_div(a->max_seqlen_k, a->chunk);
@@ -1810,7 +1815,12 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
     return 0;
   }
 
-  hipLaunchKernelGGL(fill_i32_kernel, dim3(512), dim3(256), 0, s, p.segcnt, (int64_t)(seg_bytes / 4), 0);
+  if (pool != nullptr) {
+    if (int rc = mean_pool_with_offsets(pool, p.segcnt, lists ? (int64_t)(seg_bytes / 16) : 0, stream)) return rc;
+  } else {
+    hipLaunchKernelGGL(fill_i32_kernel, dim3(512), dim3(256), 0, s, p.segcnt, (int64_t)(seg_bytes / 4), 0);
+  }
+  if (!lists) p.segcnt = nullptr;
   dim3 ggrid(ceil_div(a->max_seqlen_q, kGateRows), a->heads, a->batch);
   int rc;
   if (big)
@@ -1819,6 +1829,7 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_hd<bf16_t>(p, ggrid, s) : launch_gate_hd<f16_t>(p, ggrid, s);
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("topk_gate_kernel");
+  if (!lists) return 0;
   hipLaunchKernelGGL(csc_scan_kernel, dim3(a->heads, a->batch), dim3(256), 0, s, p);
   FMOBA_LAUNCH_CHECK("csc_scan_kernel");
   hipLaunchKernelGGL(csc_fill_kernel, dim3(p.nseg * p.W, a->heads, a->batch), dim3(64), 0, s, p);
@@ -1837,7 +1848,18 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
 
 extern "C" int fmoba_fused_topk(const fmoba_fused_topk_args *a, void *stream) {
   FMOBA_REQUIRE(a != nullptr, "fused_topk: null args");
-  return fused_topk_run(a, a->workspace, a->workspace_bytes, stream);
+  return fused_topk_run(a, a->workspace, a->workspace_bytes, nullptr, true, stream);
+}
+
+extern "C" int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, int32_t want_lists, void *stream) {
+  FMOBA_REQUIRE(m != nullptr && g != nullptr, "pool_and_gate: null args");
+  FMOBA_REQUIRE(m->km == g->km && m->cu_seqlens_km == g->cu_seqlens_km && m->cu_seqlens_k == g->cu_seqlens_k && m->batch == g->batch &&
+                    m->heads_k == g->heads_k && m->head_dim == g->head_dim && m->chunk == g->chunk && m->dtype == g->dtype,
+                "pool_and_gate: the two argument structs describe different problems");
+  FMOBA_REQUIRE(g->total_q > 0 && g->max_seqlen_q > 0 && g->max_seqlen_k > 0, "pool_and_gate: empty problem");
+  FMOBA_REQUIRE(m->max_chunks == fmoba::ceil_div(g->max_seqlen_k, g->chunk), "pool_and_gate: max_chunks is ceil(max_seqlen_k / chunk)");
+  FMOBA_REQUIRE(want_lists || g->raw_indices == nullptr, "pool_and_gate: the ordered lists come with the column lists only");
+  return fused_topk_run(g, g->workspace, g->workspace_bytes, m, want_lists != 0, stream);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1873,5 +1895,5 @@ extern "C" int fmoba_fused_topk_static(const fmoba_fused_topk_args *a, void *str
     }
     ptr = g_scratch_ptr[dev];
   }
-  return fused_topk_run(a, ptr, (size_t)FMOBA_STATIC_SCRATCH_BYTES, stream);
+  return fused_topk_run(a, ptr, (size_t)FMOBA_STATIC_SCRATCH_BYTES, nullptr, true, stream);
 }

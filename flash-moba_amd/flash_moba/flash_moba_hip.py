@@ -20,6 +20,8 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 import os
 from typing import List, Optional
@@ -28,6 +30,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libflash_moba_hip.so")
+HOST_PATH = os.path.join(os.path.dirname(_HERE), "lib", "flash_moba_host.so")
 
 c_i32, c_i64, c_f32, c_vp, c_sz = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t
 
@@ -88,6 +91,7 @@ EXPORTS = {
     "fmoba_chunk_offsets": (c_i32, [c_vp, c_vp, c_i32, c_i32, c_vp]),
     "fmoba_fused_topk_workspace_bytes": (c_sz, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
     "fmoba_fused_topk": (c_i32, [ctypes.POINTER(FusedTopkArgs), c_vp]),
+    "fmoba_pool_and_gate": (c_i32, [ctypes.POINTER(MeanPoolArgs), ctypes.POINTER(FusedTopkArgs), c_i32, c_vp]),
     "fmoba_fused_topk_static": (c_i32, [ctypes.POINTER(FusedTopkArgs), c_vp]),
     "fmoba_varlen_sort_workspace_bytes": (c_sz, [c_i64]),
     "fmoba_varlen_sort": (c_i32, [c_vp, c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_sz, c_vp]),
@@ -104,6 +108,7 @@ EXPORTS = {
 }
 
 _lib = None
+_host = None
 _device_ok = set()
 
 
@@ -122,6 +127,21 @@ def load_library() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+def host_module():
+    """The eager host path (csrc/torch_ops.cpp), loaded once from beside the kernel library."""
+    global _host
+    if _host is None:
+        load_library()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python flash-moba_amd/build.py`")
+        loader = importlib.machinery.ExtensionFileLoader("flash_moba_host", HOST_PATH)
+        spec = importlib.util.spec_from_loader("flash_moba_host", loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def _check(rc: int):
@@ -322,6 +342,11 @@ def _reject_unsupported(p_dropout, softcap, alibi_slopes, seqused_k=None, leftpa
 # What the last forward / backward call of this thread ran.  Read-only diagnostics for tests and benchmarks: nothing
 # in here influences a later call (bounds and selection bits are explicit arguments).
 _last = threading.local()
+
+
+def note_eager_forward():
+    """Takes over what the eager host path ran last on this thread."""
+    _last.fwd_visits, _last.fwd_row_blocks = _host.last_forward()
 
 
 def last_fwd_visits():

@@ -434,6 +434,11 @@ def flash_topk_varlen_func(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_s
     col_offsets: (batch, num_heads, ceil(max_seqlen_k / chunk)) int64, col_nnz: same shape
     int32, indices: (total_q * num_heads * moba_topk,) int32.
     """
+    if not torch.compiler.is_compiling():  # plain eager calls: one native call (None: not of its form)
+        pattern = flash_moba_gpu.host_module().topk_varlen(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, moba_topk,
+                                                           moba_chunk_size, causal)
+        if pattern is not None:
+            return pattern
     q, k = _pad8(q, k)
     km, cu_seqlens_km = _wrapped_mean_pool(maybe_contiguous(k), cu_seqlens_k, max_seqlen_k, moba_chunk_size)
     # The row lists come back ascending, so the reference's second step
@@ -462,6 +467,12 @@ def flash_moba_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_
     return_attn_probs=True the triple (out, softmax_lse (nheads, total_q) fp32, S_dmask
     (empty)).
     """
+    if not torch.compiler.is_compiling() and dropout_p == 0.0 and softcap == 0.0 and alibi_slopes is None and not return_attn_probs:
+        out = flash_moba_gpu.host_module().attn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, moba_col_offsets,
+                                                       moba_col_nnz, moba_row_indices, lg_block_m, lg_block_n, softmax_scale, causal, deterministic)
+        if out is not None:
+            flash_moba_gpu.note_eager_forward()
+            return out
     return FlashMobaAttnVarlenFunc.apply(
         q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
         moba_col_offsets, moba_col_nnz, moba_row_indices, lg_block_m, lg_block_n,
@@ -472,6 +483,12 @@ def flash_moba_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_
 def flash_moba_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                            moba_chunk_size, moba_topk, causal=True):
     """MoBA attention end to end: gate (mean-pool + top-k + CSC), then sparse attention."""
+    if not torch.compiler.is_compiling():
+        out = flash_moba_gpu.host_module().moba_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, moba_chunk_size,
+                                                       moba_topk, causal)
+        if out is not None:
+            flash_moba_gpu.note_eager_forward()
+            return out
     qp, kp = _pad8(q, k)
     km, cu_seqlens_km = _wrapped_mean_pool(maybe_contiguous(kp), cu_seqlens_k, max_seqlen_k, moba_chunk_size)
     col_offsets, col_nnz, indices, selection = _wrapped_gated_topk(

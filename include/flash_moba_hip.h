@@ -95,6 +95,12 @@ typedef struct {
 size_t fmoba_fused_topk_workspace_bytes(int32_t batch, int32_t total_q, int32_t heads,
                                         int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t chunk);
 int fmoba_fused_topk(const fmoba_fused_topk_args *a, void *stream);
+/* fmoba_chunk_offsets, fmoba_mean_pool and fmoba_fused_topk of one path in fewer launches: m->cu_seqlens_km (an
+ * output here) is written by the pooling pass itself, which also clears the gating's counters.  want_lists = 0 leaves
+ * the column lists out: only the selection bits are made (col_offsets, col_nnz and flat_indices of g may then be NULL),
+ * for callers whose attention form reads nothing else.  g->km and g->cu_seqlens_km must be m->km and m->cu_seqlens_km;
+ * max_seqlen_k of g must be positive. */
+int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, int32_t want_lists, void *stream);
 /* The same call without a workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
  * reference, whose host code allocates on every call.  `workspace` / `workspace_bytes` of `a` are
@@ -149,8 +155,9 @@ typedef struct {
   const int32_t *cu_seqlens_q, *cu_seqlens_k;
   /* optional (may be NULL): the same pattern as one bit per (row, head, chunk), word
    * [(h * ceil(max_cols/32) + c/32) * total_q + global row] bit c%32 -- what fmoba_fused_topk leaves
-   * at the first 256-byte boundary of its workspace.  Only the row-block form reads it; without it
-   * that form derives the bits from the lists first. */
+   * at the first 256-byte boundary of its workspace.  Only the row-block form reads it (and
+   * then no list: col_offsets, col_nnz and row_indices may be NULL); without it that form derives the
+   * bits from the lists first. */
   const uint32_t *selection_bits;
   void *workspace;
   size_t workspace_bytes;

@@ -1,0 +1,65 @@
+"""The native eager host path against the path through the custom ops, which stays for traced calls: same bits."""
+import numpy as np
+import pytest
+import torch
+
+import flash_moba
+from flash_moba import flash_moba_hip as hip
+
+pytestmark = pytest.mark.gpu
+
+
+class _NoHost:
+    """A host module that takes no call."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def _both(monkeypatch, fn):
+    got = fn()
+    with monkeypatch.context() as m:
+        m.setattr(hip, "host_module", lambda: _NoHost())
+        want = fn()
+    for x, y in zip(got, want):
+        assert x.shape == y.shape and x.dtype == y.dtype and torch.equal(x, y)
+    return got
+
+
+# one row, uneven lengths with empty sequences, more sequences than a wave has lanes, more than the pooling counts itself
+@pytest.mark.parametrize("lens_q,lens_k,H,Hk,D,chunk,topk", [
+    ([1], [1], 1, 1, 8, 64, 1), ([300, 0, 77], [300, 0, 77], 4, 2, 64, 64, 3), ([5, 900], [700, 2000], 4, 1, 128, 128, 4),
+    ([7] * 70, [7] * 70, 2, 2, 72, 64, 2), ([2] * 1030, [3] * 1030, 1, 1, 64, 64, 2), ([600], [600], 2, 2, 256, 64, 3),
+    ([2500], [2500], 4, 4, 128, 64, 2)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_native_host_path_gives_the_bits_of_the_op_path(monkeypatch, lens_q, lens_k, H, Hk, D, chunk, topk, grad):
+    g = torch.Generator(device="cuda").manual_seed(sum(lens_q) + D)
+    mk = lambda n, h: torch.randn((n, h, D), generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v, dout = mk(sum(lens_q), H), mk(sum(lens_k), Hk), mk(sum(lens_k), Hk), mk(sum(lens_q), H)
+    cu = lambda lens: torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device="cuda")
+    cq, ck = cu(lens_q), cu(lens_k)
+    where = (cq, ck, max(lens_q), max(lens_k))
+
+    def fused():
+        qg, kg, vg = (t.clone().requires_grad_(grad) for t in (q, k, v))
+        out = flash_moba.flash_moba_varlen_func(qg, kg, vg, *where, chunk, topk, causal=True)
+        return (out.detach(),) + (torch.autograd.grad(out, (qg, kg, vg), dout) if grad else ())
+
+    def two_step():
+        qg, kg, vg = (t.clone().requires_grad_(grad) for t in (q, k, v))
+        pattern = flash_moba.flash_topk_varlen_func(q, k, *where, topk, chunk, causal=True)
+        out = flash_moba.flash_moba_attn_varlen_func(qg, kg, vg, *where, *pattern, lg_block_m=128, lg_block_n=chunk, causal=True)
+        return (out.detach(), *pattern) + (torch.autograd.grad(out, (qg, kg, vg), dout) if grad else ())
+
+    one = _both(monkeypatch, fused)
+    two = _both(monkeypatch, two_step)
+    assert torch.equal(one[0], two[0])
+
+
+def test_gradients_have_no_gradients():
+    x = torch.randn((200, 2, 64), device="cuda").to(torch.bfloat16).requires_grad_(True)
+    cu = torch.tensor([0, 200], dtype=torch.int32, device="cuda")
+    out = flash_moba.flash_moba_varlen_func(x, x, x, cu, cu, 200, 200, 64, 2)
+    (dx,) = torch.autograd.grad(out.sum(), x, create_graph=True)
+    with pytest.raises(RuntimeError):
+        dx.sum().backward()
