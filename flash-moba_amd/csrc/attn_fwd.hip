@@ -1,10 +1,11 @@
 // Sparse attention forward over a CSC pattern: the entry points, and the column-stationary form in two
 // launches (sparse patterns; the row-block form for dense ones is in attn_fwd_rows.hip).
 //
-//   attn_fwd_col_kernel     : one workgroup per (key block of KB = 64 or 128 keys, head,
-//                             sequence).  K of the block lives in MFMA operand registers, V in
-//                             LDS; the block's ascending row list is walked in gathered 32-row
-//                             tiles: S^T = K Q^T (one lane owns one query row, so the softmax
+//   attn_fwd_col_kernel     : one workgroup per (key block of KB = 64 or 128 keys, KEY head,
+//                             sequence).  K and V of the block lie in LDS; the ascending row lists
+//                             of the query heads that share the key head are walked in gathered
+//                             32-row tiles, each wave taking tiles of its own:
+//                             S^T = K Q^T (one lane owns one query row, so the softmax
 //                             reductions over the block's keys stay in registers), P^T goes from
 //                             the accumulators straight into the operand registers of
 //                             O^T = V^T P^T (V^T through transposing LDS reads).  Every visit of
@@ -18,9 +19,6 @@
 // Work and traffic are proportional to the number of (row, key block) visits whatever the number of
 // chunks per sequence; a row-stationary formulation degenerates when every 128-row block touches
 // thousands of chunks with one or two rows each.
-// In the first kernel all four waves compute (one tile each per round, one wave per SIMD: K of the block and
-// the operands of a tile take most of its registers); the gathered Q rows go from global memory straight to
-// LDS (global_load_lds), one round ahead.
 #include "fmoba_common.h"
 
 #include <algorithm>
@@ -33,24 +31,6 @@ namespace fmoba {
 // measured break-even points (16 heads of 128, 8K and 16K tokens per sequence, top-k 8 to 32)
 constexpr int kFwdRowsDensity64 = 50, kFwdRowsDensity128 = 27;
 
-constexpr int kFwdRoundRows = 128;  // rows of a column list per round: one 32-row tile per wave
-
-template <int HD, int KB>
-struct FwdColSmem {
-  static constexpr int LDQ = HD + 16;  // elements, K / V rows (conflict-free for the 16-byte row reads and the transposing reads)
-  static constexpr int LDO = HD + 8;   // elements, per-wave output tile [32 rows][LDO]
-  static constexpr size_t tileBytes = (size_t)32 * HD * 2;  // a gathered Q tile: rows of exactly HD elements, swizzled
-  static constexpr size_t oV = 0;
-  static constexpr size_t oQ = oV + (size_t)KB * LDQ * 2;           // [2 buffers][4 tiles][32][HD]; K passes through it on its way to registers
-  static constexpr size_t oOut = oQ + 8 * tileBytes;                 // [4 waves][32][LDO]
-  static constexpr size_t oRid = oOut + (size_t)4 * 32 * LDO * 2;    // int[2][128]: row ids, one round before the rest
-  static constexpr size_t oRow = oRid + 2 * kFwdRoundRows * 4;       // int[2][128]
-  static constexpr size_t oSlot = oRow + 2 * kFwdRoundRows * 4;      // int[2][128]
-  static constexpr size_t bytes = oSlot + 2 * kFwdRoundRows * 4;
-  static_assert((size_t)KB * LDQ * 2 <= 8 * tileBytes + (size_t)4 * 32 * LDO * 2, "K passes through the Q tiles and the output tiles");
-  static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
-};
-
 struct FwdWs {
   int32_t *cnt;      // [total_q * heads] visits handed out per (row, head)
   float4 *hdr;       // [total_q * heads * cap] {m (log2 domain), l, key block id, -}
@@ -58,356 +38,284 @@ struct FwdWs {
   int32_t cap;
 };
 
-template <typename T, int HD, int KB>
-__global__ __launch_bounds__(256) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws) {
-  typedef FwdColSmem<HD, KB> SM;
-  constexpr int NTHR = 256;
-  constexpr int KS = HD / 16, LDQ = SM::LDQ, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
-  constexpr int KT = KB / 32;                 // 32-key tiles of the block
-  constexpr uint32_t TB = (uint32_t)SM::tileBytes;
-  constexpr int RB = HD * 2;                  // bytes of a tile row
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint16_t *sV = reinterpret_cast<uint16_t *>(smem + SM::oV);
-  int *sRid = reinterpret_cast<int *>(smem + SM::oRid);
-  int *sRow = reinterpret_cast<int *>(smem + SM::oRow);
-  int *sSlot = reinterpret_cast<int *>(smem + SM::oSlot);
+template <int HD, int KB>
+struct FwdColSmem {
+  static constexpr size_t tile = (size_t)KB * HD * 2;  // K or V of the block: rows of exactly HD elements, swizzled
+  static constexpr size_t oOut = 2 * tile;             // [4 waves][32 rows][64 features]: half a tile of partial rows on its way out
+  static constexpr size_t bytes = oOut + 4 * 4096;
+  static_assert(2 * bytes <= 160 * 1024, "two workgroups per compute unit");
+};
 
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + KB - 1) / KB, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
-  const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
-  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+// *p += 1 in the lanes of `lanes`; the old value arrives with the wave's other loads (the caller waits), what the other
+// lanes get is undefined
+__device__ __forceinline__ int take_slot(int32_t *p, unsigned long long lanes) {
+  int old = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+  unsigned long long saved;
+  asm volatile("s_mov_b64 %1, exec\n\t"
+               "s_mov_b64 exec, %2\n\t"
+               "global_atomic_add %0, %3, %4, off sc0\n\t"
+               "s_mov_b64 exec, %1"
+               : "=&v"(old), "=&s"(saved)
+               : "s"(lanes), "v"(p), "v"(1)
+               : "memory");
+#else
+  (void)p, (void)lanes;
+#endif
+  return old;
+}
+
+// Two workgroups per compute unit, two waves per SIMD, no barrier after the block's K and V have arrived.  What bounds it
+// depends on the lists.  Long ones (32768 tokens, 32 heads, top-k 16 of 256 chunks: 2000 rows per list): the partial
+// results on their way out and the gathered Q rows, together about 4 TB/s.  Short ones (a part of a prompt against the
+// keys so far, 1000 query rows: 28 rows per list): the three dependent loads before a workgroup's first product, hence
+// small workgroups that share a unit and serve all heads of a group.  The kernel this one replaces had one workgroup of
+// 512-register waves per unit and head and walked 128 rows between barriers: on those two shapes 2.32 -> 2.17 ms and
+// 530 -> 162 us, 8192 tokens with top-k 8 148 -> 132 us, 262144 tokens 9.99 -> 9.12 ms, and one row per sequence against
+// 16 sequences of up to 32768 keys 651 -> 113 us.
+template <typename T, int HD, int KB>
+__global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws) {
+  typedef FwdColSmem<HD, KB> SM;
+  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, KT = KB / 32, RB = HD * 2;
+  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads_k, (a.max_seqlen_k + KB - 1) / KB, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
+  const int nb = item.idx, b = item.pair / a.heads_k, hk = item.pair - b * a.heads_k;
+  const int grp = a.heads / a.heads_k, h0 = hk * grp;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
   const int key0 = nb * KB;
-  if (key0 >= Lk) return;
+  const int c = key0 / a.lg_block_n;
+  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+  if (key0 >= Lk || c >= a.max_cols) return;
   const int off = Lk - Lq;
   const int D = a.head_dim;
-  const int hk = h / (a.heads / a.heads_k);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hh = lane >> 5;
   const bool causal = a.is_causal != 0;
   const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
+  const uint32_t ldsK = (uint32_t)(uintptr_t)smem, ldsV = ldsK + (uint32_t)SM::tile, ldsOut = ldsK + (uint32_t)(SM::oOut + wave * 4096);
 
-  // ---- K and V of the block: the loads are issued first and stored after the look-up of the column list, so
-  // that the two chains of dependent loads wait together (one workgroup per compute unit: nothing else covers them)
-  constexpr int NKV = KB * VPR / NTHR;
-  Pack8 xk[NKV], xv[NKV];
-  {
-    const uint16_t *kp = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
-    const uint16_t *vp = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
+  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
+  const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
+  const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
+  bool loaded = false;
+
+  for (int g0 = 0; g0 < grp; g0 += 64) {  // (a turn per 64 heads of the group)
+    // lane j: the list of head g0 + j of the group
+    int nnz = 0;
+    int64_t lbase = 0;
+    if (g0 + lane < grp) {
+      const int64_t ci = ((int64_t)b * a.heads + h0 + g0 + lane) * a.max_cols + c;
+      nnz = a.col_nnz[ci];
+      lbase = a.col_offsets[ci];
+    }
+    int incl = (nnz + 31) >> 5;  // tiles of the lists up to this one
 #pragma unroll
-    for (int i = 0; i < NKV; ++i) {
-      const int v = tid + NTHR * i;
-      const int key = v / VPR, e = (v - key * VPR) * 8;
-      xk[i] = zero_pack8();
-      xv[i] = zero_pack8();
-      if (key0 + key < Lk && e < D) {
-        xk[i] = ld_global16(kp + (int64_t)key * a.k_row_stride + e);
-        xv[i] = ld_global16(vp + (int64_t)key * a.v_row_stride + e);
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(incl, o, 64);
+      incl += lane >= o ? up : 0;
+    }
+    const int ntile = __builtin_amdgcn_readlane(incl, 63);
+    if (ntile == 0) continue;
+    if (!loaded) {
+      constexpr int RPI = 64 / VPR, NI = KB / RPI / 4;
+      const int rl = lane / VPR, pc = lane % VPR;
+      const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
+      const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int key = (wave * NI + i) * RPI + rl;
+        const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
+        const int64_t kc = min(key, Lk - 1 - key0);
+        global_to_lds16(kg + kc * a.k_row_stride + e, ldsK + (uint32_t)((wave * NI + i) * 1024));
+        global_to_lds16(vg + kc * a.v_row_stride + e, ldsV + (uint32_t)((wave * NI + i) * 1024));
       }
     }
-  }
-
-  // ---- the block's column list --------------------------------------------------------------------
-  const int Bn = a.lg_block_n;
-  const int c = key0 / Bn;
-  const int64_t bh = (int64_t)b * a.heads + h;
-  int nnz = 0;
-  int64_t lbase = 0;
-  int start = 0;
-  if (c < a.max_cols) {
-    nnz = a.col_nnz[bh * a.max_cols + c];
-    lbase = a.col_offsets[bh * a.max_cols + c];
-    if (causal && nnz > 0) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off);  // earlier rows see no key of the block
-  }
-  const int32_t *list = a.row_indices + lbase + start;
-  const int n = nnz - start;  // rows of the list that the block walks
-  const int nround = (n + kFwdRoundRows - 1) / kFwdRoundRows;
-  const int ntile = (n + 31) >> 5;
-  const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride + (int64_t)h * a.q_head_stride;
-  int32_t *cntg = ws.cnt + (int64_t)q0 * a.heads + h;       // counter of local row r: cntg[r * heads]
-  if (nround == 0) return;
-  int rid01[2] = {-1, -1};  // threads 0..127: row ids of rounds 0 and 1
-  if (tid < kFwdRoundRows) {
-#pragma unroll
-    for (int sr = 0; sr < 2; ++sr) {
-      const int j = sr * kFwdRoundRows + tid;
-      const int r = list[min(j, n - 1)];
-      rid01[sr] = tile_row_code(r, j < n, Lq);
-    }
-  }
-  {
-    uint16_t *sK = reinterpret_cast<uint16_t *>(smem + SM::oQ);
-#pragma unroll
-    for (int i = 0; i < NKV; ++i) {
-      const int v = tid + NTHR * i;
-      const int key = v / VPR, e = (v - key * VPR) * 8;
-      *reinterpret_cast<Pack8 *>(sK + key * LDQ + e) = xk[i];
-      *reinterpret_cast<Pack8 *>(sV + key * LDQ + e) = xv[i];
-    }
-  }
-  __syncthreads();
-  // K of this block as the A operand of S^T = K Q^T: lane -> key (lane % 32) of each 32-key tile
-  // (kept in accumulation registers, where the MFMAs read them; S^T and O^T tiles are produced in ordinary registers,
-  // where the softmax and the packing read them: no copy between the two register files in the loop)
-  u32x4_t kfr[KT][KS];
-  {
-    const uint16_t *sK = reinterpret_cast<const uint16_t *>(smem + SM::oQ);
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        kfr[kt][ks] = pack8_vec(*reinterpret_cast<const Pack8 *>(sK + (kt * 32 + (lane & 31)) * LDQ + (hh * KS + ks) * 8));
-#if defined(__HIP_DEVICE_COMPILE__)
-        asm volatile("" : "+a"(kfr[kt][ks]));
-#endif
-      }
-  }
-  if (tid < kFwdRoundRows) {
-    sRid[tid] = rid01[0];
-    sRid[kFwdRoundRows + tid] = rid01[1];
-  }
-  __syncthreads();  // K is in registers; the row ids of rounds 0 and 1 are in LDS
-
-  // ---- feeding the tiles: all four waves compute, nothing passes through registers.  Every wave fetches the tile
-  // it will work on in the NEXT round with loads that write straight to LDS, issued at the start of a round and
-  // awaited at its end.  Threads 0..127 carry the per-row scalars: the row id of round s+2 (it has to be in LDS one
-  // round before the tile loads that use it) and the partial slot of round s+1.
-  typedef std::integral_constant<int, 0> C0;
-  typedef std::integral_constant<int, 1> C1;
-  const uint32_t ldsQ = (uint32_t)(uintptr_t)(smem + SM::oQ);
-  int n_rid = -1, v_rid = rid01[1], m_rid = -1, m_slot = 0;  // v_rid: the checked row id that was stored last = the one of the next round
-  int ft = tid;  // thread index for the feeding code, re-made opaque in every round: what is derived from it must not be kept in registers across rounds
-  auto rid_issue = [&](int sr) {
-    if (tid < kFwdRoundRows) {
-      n_rid = list[min(sr * kFwdRoundRows + ft, n - 1)];  // used (and checked) only when it is stored: no wait for it here
-    }
-  };
-  auto rid_store = [&](int sr) {
-    if (tid < kFwdRoundRows) {
-      const int j = sr * kFwdRoundRows + ft;
-      v_rid = tile_row_code(n_rid, j < n, Lq);
-      sRid[(sr & 1) * kFwdRoundRows + ft] = v_rid;
-    }
-  };
-  auto meta_issue = [&](int rid) {  // rid: this thread's row of the round after the current one
-    if (tid < kFwdRoundRows) {
-      m_rid = rid;
-      // every visit of a (row, key block) pair takes one slot of the row (a shared dummy counter for absent
-      // rows would serialise the whole grid on one address)
-      if (m_rid >= 0) m_slot = atomicAdd(cntg + (int64_t)m_rid * a.heads, 1);
-    }
-  };
-  auto meta_store = [&](int sr) {
-    if (tid < kFwdRoundRows) {
-      sRow[(sr & 1) * kFwdRoundRows + ft] = m_rid;
-      // where the visit's partial goes, as an index of partial rows (it fits 32 bits: 2^31 partial rows would be half a
-      // terabyte), or -1 for a row that is absent or has more visits than the caller's bound
-      sSlot[(sr & 1) * kFwdRoundRows + ft] = (m_rid >= 0 && m_slot < ws.cap) ? ((q0 + m_rid) * a.heads + h) * ws.cap + m_slot : -1;
-    }
-  };
-  auto tile_issue = [&](int sr) {  // tile `wave` of round sr
-    constexpr int RPI = 64 / VPR, NI = 32 / RPI;  // tile rows per instruction, instructions per tile
-    const int fl = ft & 63, rl = fl / VPR, p = fl - rl * VPR;
-    const uint32_t dst = ldsQ + (uint32_t)__builtin_amdgcn_readfirstlane(((sr & 1) * 4 + wave) * (int)TB);
-    const uint32_t qs = (uint32_t)a.q_row_stride;  // (32 x 32 -> 64-bit product: one instruction)
-    // Absent rows and features past head_dim are fetched from a row and a piece that exist (tile_row_code): every load
-    // is unconditional; the scores of absent rows are masked, and K is zero in the features past head_dim.
-    int src[NI];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) src[i] = sRid[(sr & 1) * kFwdRoundRows + wave * 32 + i * RPI + rl] & 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const uint32_t e = (uint32_t)min((p ^ tile_swz<HD>(i * RPI + rl)) * 8, D - 8);
-      global_to_lds16(qg + ((uint64_t)(uint32_t)src[i] * qs + e), dst + (uint32_t)(i * RPI * RB));
-    }
-  };
-  meta_issue(rid01[0]);
-  tile_issue(0);
-  meta_store(0);
-  wait_all_loads();
-  __syncthreads();
-
-  lds_cu16 *trV = tr_lane_base(sV, LDQ, lane) + 4 * hh * LDQ;
-  uint16_t *sOut = reinterpret_cast<uint16_t *>(smem + SM::oOut) + (size_t)wave * 32 * LDO;
-  // byte address of this lane's row (lane % 32 of the wave's tile, buffer 0), piece hh * KS; the other pieces
-  // are an exclusive-or on the piece bits
-  const uint32_t qrow = ldsQ + (uint32_t)wave * TB + (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
-
-  // LDS addresses are one register (made opaque to the compiler where it is used) plus an offset in the instruction:
-  // left alone, the compiler computes every address of a tile outside the loop and parks them in spare registers
-  auto opaque = [](uint32_t &x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(x));
-#else
-    (void)x;
-#endif
-  };
-  const uint32_t ldsOut = (uint32_t)(uintptr_t)sOut, ldsRow = (uint32_t)(uintptr_t)(smem + SM::oRow) + (uint32_t)(wave * 32 * 4);
-  // A tile in two steps: the products and the softmax (the partial goes to the wave's LDS tile), then the stores.
-  // Between them the round waits for the loads of the next tile: one counter covers loads and stores alike, so
-  // stores issued before that wait would be waited for as well instead of completing under the next round.
-  float t_m = 0.f, t_l = 0.f;
-  int t_rid = -1;
-  auto compute_tile = [&](auto pc) {
-    constexpr int PB = decltype(pc)::value;
-    const int sidx = PB * kFwdRoundRows + wave * 32 + (lane & 31);
-    const int rid = sRow[sidx];
-    // this lane's query row as the B operand
+    // The wave's tiles: tile t + 8 is picked (its row ids are asked for) and the rows of tile t + 4 are fetched while tile t
+    // is worked on, and all of these loads are awaited at one place, before the stores of tile t: one counter covers
+    // loads and stores alike, and a load issued after the stores would be waited for together with them.
+    int g = 0, rem = 0, ridn = 0;
     Pack8 qb[KS];
-    uint32_t bq = qrow;
-    opaque(bq);
+    int slot = 0;
+    // (no branch around the loads: where two paths join, the compiler copies what was loaded, and waits for it there)
+    auto pick = [&](int t) {
+      t = min(t, ntile - 1);
+      g = __popcll(__ballot(incl <= t));
+      const int first = t - (g ? __builtin_amdgcn_readlane(incl, g - 1) : 0);
+      const int n = __builtin_amdgcn_readlane(nnz, g);
+      const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)lbase, g), bhi = __builtin_amdgcn_readlane((uint32_t)(lbase >> 32), g);
+      const int32_t *list = a.row_indices + (int64_t)(((uint64_t)bhi << 32) | blo) + first * 32;
+      rem = n - first * 32;
+      ridn = list[min(lane & 31, rem - 1)];
+    };
+    int rid = -1, hcur = 0;
+    auto fetch = [&](int t) {  // Q rows and partial slots of the picked tile
+      rid = tile_row_code(ridn, (lane & 31) < rem, Lq);
+      hcur = h0 + g0 + g;
+      const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + (rid & 0x7fffffff)) * a.q_row_stride + (int64_t)hcur * a.q_head_stride;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qb[ks] = lds_read16((bq ^ (uint32_t)(ks * 16)) + (uint32_t)(PB * 4) * TB);
-    __builtin_amdgcn_sched_barrier(0);
-    // block-local softmax of the row, log2 domain; keys beyond lim are masked: in a tile that has such pairs S^T starts
-    // from 0 / -inf per pair and the products add to that (the exponential of -inf is 0), in the others it starts from
-    // nothing, and the softmax has no comparison in either
-    const int lim = rid < 0 ? -1 : min(causal ? rid + off : 0x7fffffff, Lk - 1) - key0;  // last visible key, relative
-    f32x16 st[KT];  // S^T: register i of tile kt <-> key kt*32 + acc_row(i, hh), this lane's row
-    const bool masked = !__all(lim >= KB - 1);
-    if (masked) {
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int jrel = kt * 32 + 8 * (i >> 2) + (i & 3) + 4 * hh;
-          st[kt][i] = jrel <= lim ? 0.f : -INFINITY;
-        }
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) mfma32_a_acc<T, false>(st[kt], kfr[kt][0], qb[0]);
-    } else {
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) mfma32_a_acc<T, true>(st[kt], kfr[kt][0], qb[0]);
-    }
-#pragma unroll
-    for (int ks = 1; ks < KS; ++ks)
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) mfma32_a_acc<T, false>(st[kt], kfr[kt][ks], qb[ks]);
-    static_assert(KT == 2 || KT == 4, "key blocks of 64 or 128 keys");
-    if constexpr (KT == 2) {
-      mfma_results_ready(st[0], st[1]);
-    } else {
-      mfma_results_ready(st[0], st[1]);
-      mfma_results_ready(st[2], st[3]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // V^T operands of the first half of the feature tiles: their LDS latency runs under the softmax arithmetic
-    Pack8 vt[NDT][KT][2];
-#pragma unroll
-    for (int dt = 0; dt < NDT / 2; ++dt)
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const int lo = (kt * 32 + 16 * s2) * LDQ + dt * 32;
-          vt[dt][kt][s2] = tr_frag8_at(trV, lo, lo + 8 * LDQ);
-        }
-    __builtin_amdgcn_sched_barrier(0);
-    // (the scores stay raw: the scale, positive, goes into the exponent's multiply-add)
-    float m = -INFINITY;
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) m = fmaxf(m, st[kt][i]);
-    m = max_xor32_f(m) * scale_log2;
-    const float m_use = m == -INFINITY ? 0.f : m;
-    float l = 0.f;
-    Pack8 pf[KT][2];  // P^T as the B operand of O^T = V^T P^T, straight from the accumulators
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w], scale_log2, -m_use));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w + 1], scale_log2, -m_use));
-          l += p0 + p1;
-          pf[kt][s2].w[w] = pack2<T>(p0, p1);
-        }
-    l = sum_xor32_f(l);
-    __builtin_amdgcn_sched_barrier(0);
-    // O^T[d][row] = sum_key V^T[d][key] P^T[key][row]; register i of d-tile dt <-> d = dt*32 + acc_row(i, hh)
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      if (dt == 0) {  // second half of the V^T operands, under the first products
-#pragma unroll
-        for (int d2 = NDT / 2; d2 < NDT; ++d2)
-#pragma unroll
-          for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-              const int lo = (kt * 32 + 16 * s2) * LDQ + d2 * 32;
-              vt[d2][kt][s2] = tr_frag8_at(trV, lo, lo + 8 * LDQ);
-            }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      f32x16 o;
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          if (kt == 0 && s2 == 0)
-            mfma32_vv<T, true>(o, vt[dt][kt][s2], pf[kt][s2]);
-          else
-            mfma32_vv<T, false>(o, vt[dt][kt][s2], pf[kt][s2]);
-        }
-      mfma_results_ready(o);
-      // to the wave's row-major output tile, four features (8 bytes) at a time
-      uint32_t bo = ldsOut + (uint32_t)(((lane & 31) * LDO + 4 * hh) * 2);
-      opaque(bo);
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        lds_write_vec<uint2>(bo + (uint32_t)((dt * 32 + 8 * g) * 2), make_uint2(pack2<T>(o[4 * g], o[4 * g + 1]), pack2<T>(o[4 * g + 2], o[4 * g + 3])));
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    t_m = m;
-    t_l = l;
-    t_rid = rid;
-  };
-  auto store_tile = [&](auto pc) {
-    constexpr int PB = decltype(pc)::value;
-    const int sidx = PB * kFwdRoundRows + wave * 32 + (lane & 31);
-    const int rid = t_rid;
-    const float m = t_m, l = t_l;
-    // header of the partial
-    const int pidx = sSlot[sidx];
-    if (pidx >= 0 && hh == 0) ws.hdr[pidx] = make_float4(m, l, __int_as_float(nb), 0.f);
-    wave_lds_fence();
-    // rows leave as 16-byte pieces: lane -> (row 4k + lane / 16, features 8 * (lane % 16))
-    if ((lane & 15) * 8 < D) {
-      uint32_t br = ldsRow + (uint32_t)((lane >> 4) * 4), bx = ldsOut + (uint32_t)(((lane >> 4) * LDO + (lane & 15) * 8) * 2);
-      opaque(br);
-      opaque(bx);
-      // all indices, then all rows, then the stores: one LDS latency each instead of sixteen in a chain
-      int p2[8];
-      Pack8 x[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) p2[k] = lds_read_vec<int>(br + (uint32_t)((PB * kFwdRoundRows + 4 * k) * 4) + (uint32_t)(SM::oSlot - SM::oRow));
-#pragma unroll
-      for (int k = 0; k < 8; ++k) x[k] = lds_read16(bx + (uint32_t)(4 * k * LDO * 2));
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (p2[k] >= 0) st_stream16(ws.part + ((uint64_t)(uint32_t)p2[k] * (uint32_t)D + (uint32_t)((lane & 15) * 8)), x[k]);
-    }
-    wave_lds_fence();
-  };
-
-  auto round = [&](auto pc, int r) {
+      for (int ks = 0; ks < KS; ++ks) qb[ks] = ld_global16(qp + min((hh * KS + ks) * 8, D - 8));  // (features past D: zeroed in arrived())
+      slot = take_slot(ws.cnt + ((int64_t)(q0 + (rid & 0x7fffffff)) * a.heads + hcur), __ballot(rid >= 0 && hh == 0 && t < ntile));
+    };
+    auto arrived = [&]() {
+      wait_all_loads();
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(ft));
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
+      asm volatile("" : "+v"(slot), "+v"(ridn));
 #endif
-    rid_issue(r + 2);
-    meta_issue(v_rid);
-    tile_issue(r + 1);
-    const bool mine = 4 * r + wave < ntile;
-    if (mine) compute_tile(pc);
-    wait_all_loads();
-    meta_store(r + 1);
-    rid_store(r + 2);
-    if (mine) store_tile(pc);
-    __syncthreads();  // round r + 1 is in LDS; everyone is done with round r
-  };
-  for (int r = 0; r < nround; r += 2) {
-    round(C0{}, r);
-    if (r + 1 < nround) round(C1{}, r + 1);
+      if (D < HD) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) qb[ks].w[w] = (hh * KS + ks) * 8 < D ? qb[ks].w[w] : 0u;
+      }
+    };
+    pick(wave);
+    fetch(wave);
+    pick(wave + 4);
+    arrived();
+    if (!loaded) {
+      wait_all_loads();
+      __syncthreads();
+      loaded = true;
+    }
+    for (int t = wave; t < ntile; t += 4) {
+      const int r = rid, h = hcur;
+      const int s0 = __shfl(slot, lane & 31, 64);
+      const int pidx = (r >= 0 && s0 < ws.cap) ? ((q0 + r) * a.heads + h) * ws.cap + s0 : -1;
+      // keys beyond lim are masked
+      const int lim = r < 0 ? -1 : min(causal ? r + off : 0x7fffffff, Lk - 1) - key0;
+      f32x16 st[KT];
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[kt][i] = 0.f;
+      uint32_t ak = ldsK + rowoff;
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(ak));
+#endif
+      // (the K operands of a k-step are read while the step before it is on the matrix cores; the fences keep the compiler
+      // from moving every read next to its product)
+      Pack8 kf[2][KT];
+      auto k_read = [&](auto kc) {
+        constexpr int ks = decltype(kc)::value;
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) kf[ks & 1][kt] = lds_read16((ak ^ (uint32_t)(ks * 16)) + (uint32_t)(kt * 32 * RB));
+      };
+      k_read(std::integral_constant<int, 0>{});
+      static_for<KS>([&](auto kc) {
+        constexpr int ks = decltype(kc)::value;
+        if constexpr (ks + 1 < KS) k_read(std::integral_constant<int, ks + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) st[kt] = mfma32<T>(kf[ks & 1][kt], qb[ks], st[kt]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      fetch(t + 4);
+      pick(t + 8);
+      if (!__all(lim >= KB - 1)) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int jrel = kt * 32 + 8 * (i >> 2) + (i & 3) + 4 * hh;
+            st[kt][i] = jrel <= lim ? st[kt][i] : -INFINITY;
+          }
+      }
+      float m = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m = fmaxf(m, st[kt][i]);
+      m = max_xor32_f(m) * scale_log2;
+      const float m_use = m == -INFINITY ? 0.f : m;
+      float l = 0.f;
+      Pack8 pf[KT][2];
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w], scale_log2, -m_use));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w + 1], scale_log2, -m_use));
+            l += p0 + p1;
+            pf[kt][s2].w[w] = pack2<T>(p0, p1);
+          }
+      l = sum_xor32_f(l);
+      Pack8 x[NDT][2];
+      uint32_t tv = ldsV + troff;
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(tv));
+#endif
+      // V^T operands: those of the next KT products are read while KT products run
+      Pack8 vt[2][KT];
+      auto v_read = [&](auto hc) {  // half hc & 1 of feature tile hc / 2
+        constexpr int hb = decltype(hc)::value, dt = hb >> 1;
+        const uint32_t xlo = (uint32_t)(dt * 4 * 16), xhi = (uint32_t)(((dt * 4) ^ TileSwz<HD>::kRow8) * 16);
+#pragma unroll
+        for (int u = 0; u < KT; ++u) {
+          const int q = (hb & 1) * KT + u;  // key tile q / 2, half q & 1
+          const uint32_t olo = (uint32_t)(q * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
+          vt[hb & 1][u] = lds_tr8((tv ^ xlo) + olo, (tv ^ xhi) + ohi);
+        }
+      };
+      v_read(std::integral_constant<int, 0>{});
+      f32x16 o;
+      static_for<2 * NDT>([&](auto hc) {
+        constexpr int hb = decltype(hc)::value, dt = hb >> 1;
+        if constexpr (hb + 1 < 2 * NDT) v_read(std::integral_constant<int, hb + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr ((hb & 1) == 0) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[i] = 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < KT; ++u) {
+          const int q = (hb & 1) * KT + u;
+          o = mfma32<T>(vt[hb & 1][u], pf[q >> 1][q & 1], o);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr ((hb & 1) == 0) return;
+        // four features per lane and group of eight: the two halves of the wave exchange, so that a lane stores eight
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const uint32_t ev = pack2<T>(o[8 * j + 2 * w], o[8 * j + 2 * w + 1]), od = pack2<T>(o[8 * j + 4 + 2 * w], o[8 * j + 4 + 2 * w + 1]);
+#if defined(__HIP_DEVICE_COMPILE__)
+            auto sw = __builtin_amdgcn_permlane32_swap(ev, od, false, false);
+            x[dt][j].w[w] = sw[0];
+            x[dt][j].w[2 + w] = sw[1];
+#else
+            x[dt][j].w[w] = ev, x[dt][j].w[2 + w] = od;
+#endif
+          }
+        }
+      });
+      arrived();
+      if (pidx >= 0 && hh == 0) st_stream16(ws.hdr + pidx, Pack8{{__float_as_uint(m), __float_as_uint(l), (uint32_t)nb, 0u}});
+      // (the header past the caches, as the rows: written the ordinary way it cost 6 to 8 % of the kernel)
+      // Rows leave through LDS, 64 features at a time, so that eight lanes store the 128 bytes of a row together: stored
+      // from where the products leave them (16 bytes per lane, 32 per row and instruction) every line went to memory
+      // in pieces, and the kernel took nearly twice as long (275 against 146 us at 8192 tokens).  Piece p of row r lies at piece p ^ (r & 7).
+#pragma unroll
+      for (int half = 0; half < HD / 64; ++half) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          lds_write_vec<u32x4_t>(ldsOut + (uint32_t)((lane & 31) * 128 + (((2 * e + hh) ^ (lane & 7)) * 16)), pack8_vec(x[2 * half + (e >> 1)][e & 1]));
+        wave_lds_fence();
+        Pack8 y[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y[k] = lds_read16(ldsOut + (uint32_t)((8 * k + (lane >> 3)) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) * 16)));
+        wave_lds_fence();
+        const int f = half * 64 + (lane & 7) * 8;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int p2 = __shfl(pidx, 8 * k + (lane >> 3), 64);
+          if (p2 >= 0 && f < D) st_stream16(ws.part + ((uint64_t)(uint32_t)p2 * (uint32_t)D + (uint32_t)f), y[k]);
+        }
+      }
+    }
   }
 }
 
@@ -575,7 +483,7 @@ static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStre
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_k, KB);
+  const int64_t items = (int64_t)a.batch * a.heads_k * ceil_div(a.max_seqlen_k, KB);
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_fwd: too many (sequence, head, key block) work items");
     return 1;
