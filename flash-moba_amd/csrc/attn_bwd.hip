@@ -804,6 +804,265 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
 }
 
 // ------------------------------------------------------------------------------------
+// dK / dV, dS tiles form: TODO comment
+// ------------------------------------------------------------------------------------
+template <int HD>
+struct DkdvSmem {
+  static constexpr size_t tile = (size_t)64 * HD * 2;        // 64 gathered rows of Q or dO, swizzled (tile_swz)
+  static constexpr size_t oQ = 0;                             // [2 buffers]
+  static constexpr size_t odO = oQ + 2 * tile;                // [2 buffers]
+  static constexpr size_t oP = odO + 2 * tile;                // [64 rows][64 keys], piece p (8 keys) of row r at p ^ (r & 7)
+  static constexpr size_t odS = oP + 64 * 128;
+  static constexpr size_t bytes_loop = odS + 64 * 128;
+  static constexpr int LDR = HD + 4;                          // floats, output staging [2][64 keys][LDR]
+  static constexpr size_t bytes = bytes_loop > (size_t)2 * 64 * LDR * 4 ? bytes_loop : (size_t)2 * 64 * LDR * 4;
+};
+
+template <typename T, int HD>
+__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws) {
+  typedef DkdvSmem<HD> SM;
+  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, NDW = NDT / 2, LDR = SM::LDR;
+  constexpr float kLog2e = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + 63) / 64, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
+  const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
+  const int key0 = nb * 64;
+  const int Bn = a.lg_block_n, c = key0 / Bn;
+  const int64_t bh = (int64_t)b * a.heads + h;
+  int nnz = 0;
+  int64_t lbase = 0;
+  if (c < a.max_cols) {
+    nnz = a.col_nnz[bh * a.max_cols + c];
+    lbase = a.col_offsets[bh * a.max_cols + c];
+  }
+  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+  if (key0 >= Lk) return;
+  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+  const int off = Lk - Lq;
+  const int D = a.head_dim;
+  const int hk = h / (a.heads / a.heads_k);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
+  const int kq = wave & 1, rt = wave >> 1;  // S and dP: this wave's 32 keys and 32 rows
+  const int fw = wave & 1, sel = wave >> 1;      // sums: dV (sel = 0) or dK (1), all keys of the block, half of the features
+  const bool causal = a.is_causal != 0;
+  const float scale_log2 = a.softmax_scale * kLog2e;
+  const uint32_t lds = (uint32_t)(uintptr_t)smem, ldsQ = lds + (uint32_t)SM::oQ, ldsdO = lds + (uint32_t)SM::odO, ldsP = lds + (uint32_t)SM::oP, ldsdS = lds + (uint32_t)SM::odS;
+  constexpr uint32_t TILE = (uint32_t)SM::tile;
+  constexpr int RPI = 64 / VPR;      // tile rows per load instruction
+  constexpr int NI = 16 / RPI;       // load instructions per wave and operand: 16 rows
+
+  // K and V of the block pass through the tiles on their way to registers
+  {
+    const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
+    const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
+    const int rl = lane / VPR, pc = lane % VPR;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int key = (wave * NI + i) * RPI + rl;
+      const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
+      const int64_t kc = min(key, Lk - 1 - key0);
+      global_to_lds16(kg + kc * a.k_row_stride + e, ldsQ + (uint32_t)((wave * NI + i) * 1024));
+      global_to_lds16(vg + kc * a.v_row_stride + e, ldsdO + (uint32_t)((wave * NI + i) * 1024));
+    }
+  }
+  int start = 0;
+  if (causal && nnz > 0 && Bn > 64) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off);  // earlier rows see no key of the block
+  const int32_t *list = a.row_indices + lbase + start;
+  const int n = nnz - start;
+  const int nround = (n + 63) >> 6;
+  const int koff = key0 - c * Bn;
+
+  const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride + (int64_t)h * a.q_head_stride;
+  const uint16_t *dog = reinterpret_cast<const uint16_t *>(a.dout) + (int64_t)q0 * a.do_row_stride + (int64_t)h * a.do_head_stride;
+  const float *lseg = a.softmax_lse + (int64_t)h * a.total_q + q0;
+  const float *delg = a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b;
+
+  f32x16 acc[NDW][2];  // register i of tile [d][kk] <-> feature (fw * NDW + d) * 32 + acc_row(i, hh), key kk * 32 + lane % 32
+#pragma unroll
+  for (int d = 0; d < NDW; ++d)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[d][kk][i] = 0.f;
+
+  // lane -> row rt * 32 + lane % 32 of a round
+  const int myrow = rt * 32 + (lane & 31);
+  int rid_nx = nround > 0 ? list[min(myrow, n - 1)] : 0;
+  auto code = [&](int raw, int r) { return tile_row_code(raw, r * 64 + myrow < n, Lq); };
+  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
+  const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
+  const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
+
+  wait_all_loads();
+  __syncthreads();
+  Pack8 kf[KS], vf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    kf[ks] = lds_read16(((ldsQ + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
+    vf[ks] = lds_read16(((ldsdO + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
+    if (D < HD && (hh * KS + ks) * 8 >= D) kf[ks] = vf[ks] = zero_pack8();
+  }
+  __syncthreads();
+  if (nround > 0) {
+    // rows of round r + 1 (ids `rid`): Q and dO into the other buffer, 16 rows per wave
+    auto feed = [&](int rid, uint32_t buf) {
+      const int rl = lane / VPR, pc = lane % VPR;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int tr = kq * 16 + i * RPI + rl;  // row of the tile of 32
+        const uint32_t src = (uint32_t)__shfl(rid, tr, 64) & 0x7fffffffu;
+        const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
+        const uint32_t dst = buf + (uint32_t)((rt * 32 + kq * 16 + i * RPI) * RB);
+        global_to_lds16(qg + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
+        global_to_lds16(dog + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
+      }
+    };
+    int rid = code(rid_nx, 0);
+    feed(rid, 0);
+    float lse = lseg[rid & 0x7fffffff], del = delg[rid & 0x7fffffff];
+    rid_nx = list[min(64 + myrow, n - 1)];
+    auto arrived = [&]() {
+      wait_all_loads();
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(lse), "+v"(del), "+v"(rid_nx));
+#endif
+    };
+    arrived();
+    __syncthreads();
+    const uint32_t pw = (uint32_t)(myrow * 128 + hh * 8), psw = (uint32_t)(myrow & 7);
+    const uint32_t ptr_ = (uint32_t)(r0t * 128 + (((((lane >> 4) & 1) * 2 + ((li & 3) >> 1)) ^ (r0t & 7)) * 16) + (li & 1) * 8);
+    for (int r = 0; r < nround; ++r) {
+      const uint32_t buf = (r & 1) ? TILE : 0u;
+      const int rcur = rid;
+      const float lse2 = rcur >= 0 ? lse * kLog2e : INFINITY, delta = del;
+      // the next round's rows
+      rid = code(rid_nx, r + 1);
+      if (r + 1 < nround) feed(rid, buf ^ TILE);
+      lse = lseg[rid & 0x7fffffff];
+      del = delg[rid & 0x7fffffff];
+      rid_nx = list[min((r + 2) * 64 + myrow, n - 1)];
+      // S^T and dP^T: lane -> row, register i -> key kq * 32 + acc_row(i, hh)
+      f32x16 s, dp;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
+      uint32_t aq = ldsQ + buf + (uint32_t)(rt * 32 * RB) + rowoff, ad = ldsdO + buf + (uint32_t)(rt * 32 * RB) + rowoff;
+      constexpr int NB = 2;  // k-steps per batch of reads
+      Pack8 qf[2][NB], df[2][NB];
+      auto rd = [&](auto bc) {
+        constexpr int B = decltype(bc)::value;
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          qf[B & 1][u] = lds_read16(aq ^ (uint32_t)((B * NB + u) * 16));
+          df[B & 1][u] = lds_read16(ad ^ (uint32_t)((B * NB + u) * 16));
+        }
+      };
+      rd(std::integral_constant<int, 0>{});
+      static_for<KS / NB>([&](auto bc) {
+        constexpr int B = decltype(bc)::value;
+        if constexpr (B + 1 < KS / NB) rd(std::integral_constant<int, B + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          s = mfma32<T>(kf[B * NB + u], qf[B & 1][u], s);
+          dp = mfma32<T>(vf[B * NB + u], df[B & 1][u], dp);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      const int lim = rcur < 0 ? -1 : min(causal ? rcur + off : 0x7fffffff, Lk - 1) - key0 - kq * 32;  // last visible key of this wave's 32
+      if (!__all(lim >= 31)) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 8 * (i >> 2) + (i & 3) + 4 * hh <= lim ? s[i] : -INFINITY;
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float p[4], d[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          p[j] = __builtin_amdgcn_exp2f(fmaf(s[4 * g + j], scale_log2, -lse2));
+          d[j] = p[j] * (dp[4 * g + j] - delta);
+        }
+        const uint32_t at = pw + (((uint32_t)(kq * 4 + g) ^ psw) * 16u);
+        lds_write_vec<uint2>(ldsP + at, make_uint2(pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3])));
+        lds_write_vec<uint2>(ldsdS + at, make_uint2(pack2<T>(d[0], d[1]), pack2<T>(d[2], d[3])));
+      }
+      __syncthreads();  // P and dS of the round are in LDS
+      // dV^T[f][key] += dO^T[f][row] P[row][key], dK^T[f][key] += Q^T[f][row] dS[row][key]
+      const uint32_t tx = (sel ? ldsQ : ldsdO) + buf + troff, px = (sel ? ldsdS : ldsP) + ptr_;
+      Pack8 pb[2][2], xa[2][NDW];
+      auto rd2 = [&](auto sc) {
+        constexpr int S4 = decltype(sc)::value;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          const uint32_t po = (px ^ (uint32_t)(kk * 64)) + (uint32_t)(S4 * 16 * 128);
+          pb[S4 & 1][kk] = lds_tr8(po, po + 8 * 128);
+        }
+#pragma unroll
+        for (int d = 0; d < NDW; ++d) {
+          const uint32_t dt = (uint32_t)(fw * NDW + d), xlo = dt * 64u, xhi = ((dt * 4u) ^ (uint32_t)TileSwz<HD>::kRow8) * 16u;
+          const uint32_t olo = (uint32_t)(S4 * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
+          xa[S4 & 1][d] = lds_tr8((tx ^ xlo) + olo, (tx ^ xhi) + ohi);
+        }
+      };
+      rd2(std::integral_constant<int, 0>{});
+      static_for<4>([&](auto sc) {
+        constexpr int S4 = decltype(sc)::value;
+        if constexpr (S4 < 3) rd2(std::integral_constant<int, S4 + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < NDW; ++d)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      arrived();
+      // dS of row `lane`, key groups 2 wave and 2 wave + 1: consecutive lanes write consecutive pieces of the dS tile
+      {
+        const int p = r * 64 + lane;
+        Pack8 x[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) x[u] = lds_read16(ldsdS + (uint32_t)(lane * 128) + (((uint32_t)(2 * wave + u) ^ (uint32_t)(lane & 7)) * 16u));
+        if (p < n) {
+          const int64_t pos = lbase + start + p;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(ds_ws + ds_piece_offset(pos, (koff >> 3) + 2 * wave + u, Bn >> 3)) = x[u];
+        }
+      }
+      __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
+    }
+  }
+
+  // ---- dK^T / dV^T leave as rows, once ----
+  float *red = reinterpret_cast<float *>(smem);
+#pragma unroll
+  for (int d = 0; d < NDW; ++d)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 x4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x4[j] = acc[d][kk][4 * g + j];
+        *reinterpret_cast<f32x4 *>(red + (size_t)(sel * 64 + kk * 32 + (lane & 31)) * LDR + (fw * NDW + d) * 32 + 8 * g + 4 * hh) = x4;
+      }
+  __syncthreads();
+  uint16_t *dkg = reinterpret_cast<uint16_t *>(a.dk) + (int64_t)(k0 + key0) * a.dk_row_stride + (int64_t)h * a.dk_head_stride;
+  uint16_t *dvg = reinterpret_cast<uint16_t *>(a.dv) + (int64_t)(k0 + key0) * a.dv_row_stride + (int64_t)h * a.dv_head_stride;
+  for (int v = tid; v < 64 * VPR; v += 256) {
+    const int key = v / VPR, e = (v - key * VPR) * 8;
+    if (key0 + key >= Lk || e >= D) continue;
+    const float *s0 = red + (size_t)key * LDR + e, *s1 = s0 + 64 * LDR;
+    Pack8 ov, ok;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      ov.w[w] = pack2<T>(s0[2 * w], s0[2 * w + 1]);
+      ok.w[w] = pack2<T>(s1[2 * w] * a.softmax_scale, s1[2 * w + 1] * a.softmax_scale);
+    }
+    *reinterpret_cast<Pack8 *>(dvg + (int64_t)key * a.dv_row_stride + e) = ov;
+    *reinterpret_cast<Pack8 *>(dkg + (int64_t)key * a.dk_row_stride + e) = ok;
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // dQ, first form: row blocks.  One workgroup owns 256 or 512 consecutive query rows of one (sequence, head) and
 // walks the 64-key blocks of every column in which one of its rows appears.  The dS rows of a step (written by the
 // dK/dV pass in list order) go from global memory straight into the registers of the lane that owns the query row;
@@ -1384,6 +1643,18 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
       hipLaunchKernelGGL(zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, (int64_t)a.total_q * a.heads);
       rc = a.head_dim <= 64 ? launch_dkdv<T, 64, true, 1>(a, ws, s) : (wide ? launch_dkdv<T, 128, true, 2>(a, ws, s) : launch_dkdv<T, 128, true, 1>(a, ws, s));
     } else {
+      if (getenv("FM_OLD") == nullptr) {
+        if (a.head_dim <= 64) {
+          auto kern = attn_bwd_dkdv_rows_kernel<T, 64>;
+          hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)DkdvSmem<64>::bytes);
+          hipLaunchKernelGGL(kern, dim3(a.batch * a.heads * ceil_div(a.max_seqlen_k, 64)), dim3(256), DkdvSmem<64>::bytes, s, a, ws.ds);
+        } else {
+          auto kern = attn_bwd_dkdv_rows_kernel<T, 128>;
+          hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)DkdvSmem<128>::bytes);
+          hipLaunchKernelGGL(kern, dim3(a.batch * a.heads * ceil_div(a.max_seqlen_k, 64)), dim3(256), DkdvSmem<128>::bytes, s, a, ws.ds);
+        }
+        rc = 0;
+      } else
       rc = a.head_dim <= 64 ? launch_dkdv<T, 64, false, 1>(a, ws, s) : (wide ? launch_dkdv<T, 128, false, 2>(a, ws, s) : launch_dkdv<T, 128, false, 1>(a, ws, s));
     }
     if (rc) return rc;

@@ -1,245 +1,286 @@
-// dK / dV (and the dS tiles of the row-block dQ pass) for head dimensions above 128, up to 256.
+// dK / dV and the dS tiles of the row-block dQ pass for head dimensions above 128, up to 256.
 //
-// Same column-stationary scheme as attn_bwd_dkdv_kernel -- one workgroup per (64-key block, head, sequence) walks the
-// block's ascending row list in gathered 32-row tiles: S = Q K^T, dP = dO V^T, P = exp2(S*scale*log2e - LSE*log2e),
-// dS = P o (dP - delta), dV^T += dO^T P, dK^T += Q^T dS -- with the feature axis split, because 32 keys x 256 features
-// of dK^T and dV^T no longer fit one wave's registers next to the K / V operands: wave w owns the keys 32 (w % 2) ..
-// and the features 128 (w / 2) .. of the accumulators.  S and dP need the whole head dimension, so the two waves of a
-// key half both form them (6 instead of 4 units of MFMA work per pair, the price of the split), and K / V stay in LDS
-// instead of registers.  One tile at a time, loaded by all threads between two barriers: this is the plain form, kept
-// simple; the tuned kernels serve head dimensions up to 128 (the reference gives its head dimensions 192 and 256 their
-// own, smaller tilings for the same reason: run_moba_bwd_hdim192 / run_moba_bwd_hdim256, flash_bwd_launch_template.h:237-279).
+// The column-stationary scheme of attn_bwd_dkdv_kernel -- one workgroup per (64-key block, head, sequence) walks the
+// block's ascending row list: S = Q K^T, dP = dO V^T, P = exp2(S*scale*log2e - LSE*log2e), dS = P o (dP - delta),
+// dV^T += dO^T P, dK^T += Q^T dS -- cut so that a wave fits 256 registers and two waves share a SIMD.  dK^T and dV^T of 64
+// keys x 256 features are 512 accumulator registers of one wave; here eight waves hold 64 each (a quarter of the
+// features, all keys, of one of the two), and the four (key half, row half) tiles of S and the four of dP are one wave's
+// each, with K resp. V of its key half in registers.  A round takes 64 gathered rows, which loads bring straight into LDS one
+// round ahead; dP - delta goes to the wave that holds S of the same tile through LDS (fp32), P and dS to everybody (16 bits).
+// 2 x 4096 tokens, 8 heads of 256, 8 of 128-key chunks: 1223 us with one 32-row tile at a time between two barriers and
+// K and V as LDS operands, @US@ us now.  What bounds it: one operand from LDS per product, and the two exchanges.
 #include "fmoba_common.h"
+
+#include <type_traits>
+#include <utility>
 
 namespace fmoba {
 
-constexpr int kWideHD = 256;
-
 struct BwdWideSmem {
-  static constexpr int LD = kWideHD + 8;   // elements, K / V / Q / dO rows
-  static constexpr int LDX = 64 + 8;       // elements, dS tile rows [32 rows][64 keys]
-  static constexpr int LDR = kWideHD + 4;  // floats, output staging [64 keys][LDR]
-  static constexpr size_t oK = 0;                                    // [64][LD]
-  static constexpr size_t oV = oK + (size_t)64 * LD * 2;
-  static constexpr size_t oQ = oV + (size_t)64 * LD * 2;             // [32][LD]
-  static constexpr size_t odO = oQ + (size_t)32 * LD * 2;
-  static constexpr size_t odS = odO + (size_t)32 * LD * 2;           // [32][LDX]
-  static constexpr size_t oRow = odS + (size_t)32 * LDX * 2;         // int[32]
-  static constexpr size_t oLse = oRow + 32 * 4;                      // float[32]: LSE * log2(e), +inf for absent rows
-  static constexpr size_t oDelta = oLse + 32 * 4;
-  static constexpr size_t bytes = oDelta + 32 * 4;
-  static_assert((size_t)64 * LDR * 4 <= oQ, "one output staging buffer fits where K and V were");
+  static constexpr int HD = 256;
+  static constexpr size_t tile = (size_t)64 * HD * 2;  // 64 gathered rows of Q or dO, swizzled (tile_swz)
+  static constexpr size_t oQ = 0;                       // [2 buffers]
+  static constexpr size_t odO = oQ + 2 * tile;          // [2 buffers]
+  static constexpr size_t oP = odO + 2 * tile;          // [64 rows][64 keys], piece p (8 keys) of row r at p ^ (r & 7)
+  static constexpr size_t odS = oP + 64 * 128;
+  static constexpr size_t oX = odS + 64 * 128;          // dP - delta of the four tiles: [tile][4][64 lanes][4] fp32
+  static constexpr size_t bytes = oX + 4 * 4096;
+  static constexpr int LDR = HD + 4;                    // floats, output staging [64 keys][LDR], dV then dK
+  static_assert(2 * (size_t)64 * LDR * 4 <= bytes, "the output staging reuses the tiles");
   static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
 };
 
-// grid (key blocks of 64, heads, batch), block 256
 template <typename T>
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_wide_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws) {
+__global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws) {
   typedef BwdWideSmem SM;
-  constexpr int HD = kWideHD, KS = HD / 16, LD = SM::LD, LDX = SM::LDX, LDR = SM::LDR, VPR = HD / 8;
-  constexpr int NDTW = HD / 64;  // feature tiles of 32 per wave (its half of the head dimension)
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint16_t *sK = reinterpret_cast<uint16_t *>(smem + SM::oK), *sV = reinterpret_cast<uint16_t *>(smem + SM::oV);
-  uint16_t *sQ = reinterpret_cast<uint16_t *>(smem + SM::oQ), *sdO = reinterpret_cast<uint16_t *>(smem + SM::odO);
-  uint16_t *sdS = reinterpret_cast<uint16_t *>(smem + SM::odS);
-  int *sRow = reinterpret_cast<int *>(smem + SM::oRow);
-  float *sLse = reinterpret_cast<float *>(smem + SM::oLse), *sDelta = reinterpret_cast<float *>(smem + SM::oDelta);
-
-  const int nb = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+  constexpr int HD = SM::HD, KS = HD / 16, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR;
+  constexpr float kLog2e = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + 63) / 64);
+  const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
   const int key0 = nb * 64;
+  const int Bn = a.lg_block_n, c = key0 / Bn;
+  const int64_t bh = (int64_t)b * a.heads + h;
+  int nnz = 0;
+  int64_t lbase = 0;
+  if (c < a.max_cols) {
+    nnz = a.col_nnz[bh * a.max_cols + c];
+    lbase = a.col_offsets[bh * a.max_cols + c];
+  }
+  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
   if (key0 >= Lk) return;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   const int off = Lk - Lq;
   const int D = a.head_dim;
   const int hk = h / (a.heads / a.heads_k);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hh = lane >> 5;
-  const int kq = wave & 1, fh = wave >> 1;  // key half, feature half
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
+  const int rt = wave & 1, kq = (wave >> 1) & 1, is_s = wave >> 2;  // S (waves 4..7) or dP (0..3) of this wave's 32 rows and 32 keys
+  const int fw = wave & 3, is_k = wave >> 2;                        // sums: dV (0..3) or dK (4..7), features 64 fw ..
   const bool causal = a.is_causal != 0;
-  const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
-  constexpr float kLog2e = 1.4426950408889634f;
+  const float scale_log2 = a.softmax_scale * kLog2e;
+  const uint32_t lds = (uint32_t)(uintptr_t)smem, ldsQ = lds + (uint32_t)SM::oQ, ldsdO = lds + (uint32_t)SM::odO, ldsP = lds + (uint32_t)SM::oP, ldsdS = lds + (uint32_t)SM::odS;
+  const uint32_t ldsX = lds + (uint32_t)(SM::oX + (wave & 3) * 4096 + lane * 16);
+  constexpr uint32_t TILE = (uint32_t)SM::tile;
+  constexpr int RPI = 64 / VPR;  // tile rows per load instruction
+  const int rl = lane / VPR, pc = lane % VPR;
 
-  // ---- K and V of the block into LDS (keys past the sequence and features past head_dim: zeros) ----
+  // K and V of the block pass through the tiles on their way to registers
   {
-    const uint16_t *kp = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
-    const uint16_t *vp = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
-    for (int v = tid; v < 64 * VPR; v += 256) {
-      const int key = v / VPR, e = (v - key * VPR) * 8;
-      Pack8 xk = zero_pack8(), xv = zero_pack8();
-      if (key0 + key < Lk && e < D) {
-        xk = ld_global16(kp + (int64_t)key * a.k_row_stride + e);
-        xv = ld_global16(vp + (int64_t)key * a.v_row_stride + e);
-      }
-      *reinterpret_cast<Pack8 *>(sK + key * LD + e) = xk;
-      *reinterpret_cast<Pack8 *>(sV + key * LD + e) = xv;
+    const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
+    const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = (wave * 4 + i) * RPI + rl;
+      const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
+      const int64_t kc = min(key, Lk - 1 - key0);
+      global_to_lds16(kg + kc * a.k_row_stride + e, ldsQ + (uint32_t)((wave * 4 + i) * 1024));
+      global_to_lds16(vg + kc * a.v_row_stride + e, ldsdO + (uint32_t)((wave * 4 + i) * 1024));
     }
   }
-  // ---- this block's column list ----
-  const int Bn = a.lg_block_n;
-  const int c = key0 / Bn;
-  const int64_t bh = (int64_t)b * a.heads + h;
-  int nnz = 0, start = 0;
-  int64_t lbase = 0;
-  if (c < a.max_cols) {
-    nnz = a.col_nnz[bh * a.max_cols + c];
-    lbase = a.col_offsets[bh * a.max_cols + c];
-    if (causal && nnz > 0) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off);  // earlier rows see no key of the block
-  }
+  int start = 0;
+  if (causal && nnz > 0 && Bn > 64) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off);  // earlier rows see no key of the block
   const int32_t *list = a.row_indices + lbase + start;
   const int n = nnz - start;
-  const int ntile = (n + 31) / 32;
-  const int koff = key0 - c * Bn;  // offset of this 64-key block inside its column
+  const int nround = (n + 63) >> 6;
+  const int koff = key0 - c * Bn;  // offset of the block inside its column
 
   const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride + (int64_t)h * a.q_head_stride;
   const uint16_t *dog = reinterpret_cast<const uint16_t *>(a.dout) + (int64_t)q0 * a.do_row_stride + (int64_t)h * a.do_head_stride;
-  const float *lseg = a.softmax_lse + (int64_t)h * a.total_q + q0;
-  const float *delg = a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b;
+  // the per-row scalar of this wave's part: LSE for S, delta for dP
+  const float *sclg = is_s ? a.softmax_lse + (int64_t)h * a.total_q + q0 : a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b;
 
-  f32x16 dv[NDTW], dk[NDTW];  // register i of tile dt <-> feature fh*128 + dt*32 + acc_row(i, hh), key kq*32 + lane % 32
+  f32x16 acc[2][2];  // register i of tile [d][kk] <-> feature 64 fw + 32 d + acc_row(i, hh), key 32 kk + lane % 32
 #pragma unroll
-  for (int dt = 0; dt < NDTW; ++dt)
+  for (int d = 0; d < 2; ++d)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      dv[dt][i] = 0.f;
-      dk[dt][i] = 0.f;
-    }
-  // this lane's key; key j is visible to row r iff r >= row_thr
-  const int j = key0 + kq * 32 + (lane & 31);
-  const int row_thr = j >= Lk ? 0x7fffffff : (causal ? max(0, j - off) : 0);
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[d][kk][i] = 0.f;
 
-  for (int tile = 0; tile < ntile; ++tile) {
-    __syncthreads();  // the previous tile is no longer read (first pass: K and V are in LDS)
-    // gathered Q / dO rows and the per-row scalars of the tile; absent rows: zeros, LSE = +inf
-    for (int v = tid; v < 32 * VPR; v += 256) {
-      const int rl = v / VPR, e = (v - rl * VPR) * 8;
-      const int jj = tile * 32 + rl;
-      const int r = jj < n ? list[jj] : -1;
-      Pack8 xq = zero_pack8(), xo = zero_pack8();
-      if (r >= 0 && r < Lq && e < D) {
-        xq = ld_global16(qg + (int64_t)r * a.q_row_stride + e);
-        xo = ld_global16(dog + (int64_t)r * a.do_row_stride + e);
+  const int myrow = rt * 32 + (lane & 31);  // this lane's row of a round
+  int rid_nx = nround > 0 ? list[min(myrow, n - 1)] : 0;
+  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
+  const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
+  const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
+  wait_all_loads();
+  __syncthreads();
+  Pack8 kf[KS];  // K or V of this wave's keys, the A operand
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    kf[ks] = lds_read16(((is_s ? ldsQ : ldsdO) + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16));
+    if (D < HD && (hh * KS + ks) * 8 >= D) kf[ks] = zero_pack8();
+  }
+  __syncthreads();
+  if (nround > 0) {
+    auto code = [&](int raw, int r) { return tile_row_code(raw, r * 64 + myrow < n, Lq); };
+    auto feed = [&](int rid, uint32_t buf) {  // eight rows per wave, of its own 32
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int tr = (wave >> 1) * 8 + i * RPI + rl;
+        const uint32_t src = (uint32_t)__shfl(rid, tr, 64) & 0x7fffffffu;
+        const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
+        const uint32_t dst = buf + (uint32_t)((rt * 32 + (wave >> 1) * 8 + i * RPI) * RB);
+        global_to_lds16(qg + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
+        global_to_lds16(dog + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
       }
-      *reinterpret_cast<Pack8 *>(sQ + rl * LD + e) = xq;
-      *reinterpret_cast<Pack8 *>(sdO + rl * LD + e) = xo;
-    }
-    if (tid < 32) {
-      const int jj = tile * 32 + tid;
-      const int r = jj < n ? list[jj] : -1;
-      const bool ok = r >= 0 && r < Lq;
-      sRow[tid] = ok ? r : -1;
-      sLse[tid] = ok ? lseg[r] * kLog2e : INFINITY;
-      sDelta[tid] = ok ? delg[r] : 0.f;
-    }
+    };
+    int rid = code(rid_nx, 0);
+    feed(rid, 0);
+    float scl = sclg[rid & 0x7fffffff];
+    rid_nx = list[min(64 + myrow, n - 1)];
+    auto arrived = [&]() {
+      wait_all_loads();
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(scl), "+v"(rid_nx));
+#endif
+    };
+    arrived();
     __syncthreads();
-    // S and dP of this wave's 32 keys over the whole head dimension (contraction index permuted so that each half of
-    // the wave reads one contiguous half of a row)
-    f32x16 s, dp;
+    const uint32_t pw = (uint32_t)(myrow * 128 + hh * 8), psw = (uint32_t)(myrow & 7);
+    const uint32_t ptr0 = (is_k ? ldsdS : ldsP) + (uint32_t)(r0t * 128 + (((((lane >> 4) & 1) * 2 + ((li & 3) >> 1)) ^ (r0t & 7)) * 16) + (li & 1) * 8);
+    for (int r = 0; r < nround; ++r) {
+      const uint32_t buf = (r & 1) ? TILE : 0u;
+      const int rcur = rid;
+      const float x0 = is_s ? (rcur >= 0 ? scl * kLog2e : INFINITY) : scl;
+      rid = code(rid_nx, r + 1);
+      if (r + 1 < nround) feed(rid, buf ^ TILE);
+      scl = sclg[rid & 0x7fffffff];
+      rid_nx = list[min((r + 2) * 64 + myrow, n - 1)];
+      // S^T or dP^T: lane -> row, register i -> key 32 kq + acc_row(i, hh)
+      f32x16 s;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      s[i] = 0.f;
-      dp[i] = 0.f;
-    }
+      for (int i = 0; i < 16; ++i) s[i] = 0.f;
+      const uint32_t aq = (is_s ? ldsQ : ldsdO) + buf + (uint32_t)(rt * 32 * RB) + rowoff;
+      constexpr int NB = 4;  // k-steps per batch of reads
+      Pack8 qf[2][NB];
+      auto rd = [&](auto bc) {
+        constexpr int B = decltype(bc)::value;
 #pragma unroll
-    for (int t = 0; t < KS; ++t) {
-      const int e = (hh * KS + t) * 8;
-      const Pack8 qa = *reinterpret_cast<const Pack8 *>(sQ + (lane & 31) * LD + e);
-      const Pack8 kb = *reinterpret_cast<const Pack8 *>(sK + (kq * 32 + (lane & 31)) * LD + e);
-      s = mfma32<T>(qa, kb, s);
-      const Pack8 da = *reinterpret_cast<const Pack8 *>(sdO + (lane & 31) * LD + e);
-      const Pack8 vb = *reinterpret_cast<const Pack8 *>(sV + (kq * 32 + (lane & 31)) * LD + e);
-      dp = mfma32<T>(da, vb, dp);
-    }
-    // P and dS: register i <-> row acc_row(i, hh) of the tile, this lane's key
-    Pack8 pf[2], dsf[2];
+        for (int u = 0; u < NB; ++u) qf[B & 1][u] = lds_read16(aq ^ (uint32_t)((B * NB + u) * 16));
+      };
+      rd(std::integral_constant<int, 0>{});
+      static_for<KS / NB>([&](auto bc) {
+        constexpr int B = decltype(bc)::value;
+        if constexpr (B + 1 < KS / NB) rd(std::integral_constant<int, B + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float pr[4], dsv[4];
+        for (int u = 0; u < NB; ++u) s = mfma32<T>(kf[B * NB + u], qf[B & 1][u], s);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      const uint32_t at = pw + ((uint32_t)(kq * 4) ^ psw) * 16u;
+      if (is_s) {
+        const int lim = rcur < 0 ? -1 : min(causal ? rcur + off : 0x7fffffff, Lk - 1) - key0 - kq * 32;  // last visible key of this wave's 32
+        if (!__all(lim >= 31)) {
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int i = 4 * g + jj, rl = acc_row(i, hh);
-        const float x = sRow[rl] >= row_thr ? fmaf(s[i], scale_log2, -sLse[rl]) : -INFINITY;  // (absent rows: row id -1, LSE +inf)
-        pr[jj] = __builtin_amdgcn_exp2f(x);
-        dsv[jj] = pr[jj] * (dp[i] - sDelta[rl]);
-        if (fh == 0) sdS[rl * LDX + kq * 32 + (lane & 31)] = float_to_elem_bits<T>(dsv[jj]);
+          for (int i = 0; i < 16; ++i) s[i] = 8 * (i >> 2) + (i & 3) + 4 * hh <= lim ? s[i] : -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -x0));
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          lds_write_vec<uint2>(ldsP + (at ^ (uint32_t)(g * 16)), make_uint2(pack2<T>(s[4 * g], s[4 * g + 1]), pack2<T>(s[4 * g + 2], s[4 * g + 3])));
+      } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          lds_write_vec<f32x4>(ldsX + (uint32_t)(g * 1024), f32x4{s[4 * g] - x0, s[4 * g + 1] - x0, s[4 * g + 2] - x0, s[4 * g + 3] - x0});
       }
-      // operand register s2 = g / 2 holds rows 16 s2 + 8 (w / 2) + 4 hh + ..: words 2 (g % 2), 2 (g % 2) + 1
-      pf[g >> 1].w[2 * (g & 1)] = pack2<T>(pr[0], pr[1]);
-      pf[g >> 1].w[2 * (g & 1) + 1] = pack2<T>(pr[2], pr[3]);
-      dsf[g >> 1].w[2 * (g & 1)] = pack2<T>(dsv[0], dsv[1]);
-      dsf[g >> 1].w[2 * (g & 1) + 1] = pack2<T>(dsv[2], dsv[3]);
-    }
-    // dV^T[d][key] += dO^T[d][row] P[row][key];  dK^T[d][key] += Q^T[d][row] dS[row][key], this wave's features
+      __syncthreads();  // dP - delta is there
+      if (is_s) {
 #pragma unroll
-    for (int dt = 0; dt < NDTW; ++dt)
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        const int col0 = fh * (HD / 2) + dt * 32;
-        const Pack8 dot = tr_frag8(sdO, LD, 16 * s2 + 4 * hh, 16 * s2 + 8 + 4 * hh, col0, lane);
-        const Pack8 qt = tr_frag8(sQ, LD, 16 * s2 + 4 * hh, 16 * s2 + 8 + 4 * hh, col0, lane);
-        dv[dt] = mfma32<T>(dot, pf[s2], dv[dt]);
-        dk[dt] = mfma32<T>(qt, dsf[s2], dk[dt]);
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 x = lds_read_vec<f32x4>(ldsX + (uint32_t)(g * 1024));
+          lds_write_vec<uint2>(ldsdS + (at ^ (uint32_t)(g * 16)),
+                               make_uint2(pack2<T>(s[4 * g] * x[0], s[4 * g + 1] * x[1]), pack2<T>(s[4 * g + 2] * x[2], s[4 * g + 3] * x[3])));
+        }
       }
-    // the dS tile leaves in 16-byte pieces (8 keys of one list entry), one per thread
-    if (ds_ws != nullptr) {
-      __syncthreads();
-      const int rl = tid & 31, piece = tid >> 5;  // consecutive threads: consecutive list positions of one key group
-      if (sRow[rl] >= 0)
-        *reinterpret_cast<Pack8 *>(ds_ws + ds_piece_offset(lbase + start + tile * 32 + rl, (koff >> 3) + piece, Bn >> 3)) = *reinterpret_cast<const Pack8 *>(sdS + rl * LDX + piece * 8);
+      __syncthreads();  // P and dS of the round are there
+      // dV^T[f][key] += dO^T[f][row] P[row][key] or dK^T[f][key] += Q^T[f][row] dS[row][key]
+      const uint32_t tx = (is_k ? ldsQ : ldsdO) + buf + troff;
+      Pack8 pb[2][2], xa[2][2];
+      auto rd2 = [&](auto sc) {
+        constexpr int S4 = decltype(sc)::value;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          const uint32_t po = (ptr0 ^ (uint32_t)(kk * 64)) + (uint32_t)(S4 * 16 * 128);
+          pb[S4 & 1][kk] = lds_tr8(po, po + 8 * 128);
+        }
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          const uint32_t dt = (uint32_t)(fw * 2 + d), xlo = dt * 64u, xhi = ((dt * 4u) ^ (uint32_t)TileSwz<HD>::kRow8) * 16u;
+          const uint32_t olo = (uint32_t)(S4 * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
+          xa[S4 & 1][d] = lds_tr8((tx ^ xlo) + olo, (tx ^ xhi) + ohi);
+        }
+      };
+      rd2(std::integral_constant<int, 0>{});
+      static_for<4>([&](auto sc) {
+        constexpr int S4 = decltype(sc)::value;
+        if constexpr (S4 < 3) rd2(std::integral_constant<int, S4 + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      arrived();
+      // dS of row `lane`, key group `wave`: consecutive lanes write consecutive pieces of the dS tile
+      {
+        const int p = r * 64 + lane;
+        const Pack8 x = lds_read16(ldsdS + (uint32_t)(lane * 128) + (((uint32_t)wave ^ (uint32_t)(lane & 7)) * 16u));
+        if (p < n) *reinterpret_cast<Pack8 *>(ds_ws + ds_piece_offset(lbase + start + p, (koff >> 3) + wave, Bn >> 3)) = x;
+      }
+      __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
     }
   }
 
-  // ---- dK^T / dV^T leave as rows: through LDS, dV first, then dK (one staging buffer) ----
-  float *red = reinterpret_cast<float *>(smem);  // [64 keys][LDR]
+  // ---- dK^T / dV^T leave as rows, once ----
+  float *red = reinterpret_cast<float *>(smem);  // [dV, dK][64 keys][LDR]
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4 *>(red + (size_t)(is_k * 64 + kk * 32 + (lane & 31)) * LDR + fw * 64 + d * 32 + 8 * g + 4 * hh) =
+            f32x4{acc[d][kk][4 * g], acc[d][kk][4 * g + 1], acc[d][kk][4 * g + 2], acc[d][kk][4 * g + 3]};
+  __syncthreads();
   uint16_t *dkg = reinterpret_cast<uint16_t *>(a.dk) + (int64_t)(k0 + key0) * a.dk_row_stride + (int64_t)h * a.dk_head_stride;
   uint16_t *dvg = reinterpret_cast<uint16_t *>(a.dv) + (int64_t)(k0 + key0) * a.dv_row_stride + (int64_t)h * a.dv_head_stride;
+  for (int v = tid; v < 64 * VPR; v += 512) {
+    const int key = v / VPR, e = (v - key * VPR) * 8;
+    if (key0 + key >= Lk || e >= D) continue;
+    const float *s0 = red + (size_t)key * LDR + e, *s1 = s0 + 64 * LDR;
+    Pack8 ov, ok;
 #pragma unroll
-  for (int which = 0; which < 2; ++which) {
-    __syncthreads();  // the staging buffer (K / V at first) is no longer read
-#pragma unroll
-    for (int dt = 0; dt < NDTW; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4 x;
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) x[jj] = which == 0 ? dv[dt][4 * g + jj] : dk[dt][4 * g + jj];
-        *reinterpret_cast<f32x4 *>(red + (size_t)(kq * 32 + (lane & 31)) * LDR + fh * (HD / 2) + dt * 32 + 8 * g + 4 * hh) = x;
-      }
-    __syncthreads();
-    const float mul = which == 0 ? 1.f : a.softmax_scale;
-    uint16_t *og = which == 0 ? dvg : dkg;
-    const int64_t ostride = which == 0 ? a.dv_row_stride : a.dk_row_stride;
-    for (int v = tid; v < 64 * VPR; v += 256) {
-      const int key = v / VPR, e = (v - key * VPR) * 8;
-      if (key0 + key >= Lk || e >= D) continue;
-      const float *sp = red + (size_t)key * LDR + e;
-      Pack8 o;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) o.w[w] = pack2<T>(sp[2 * w] * mul, sp[2 * w + 1] * mul);
-      *reinterpret_cast<Pack8 *>(og + (int64_t)key * ostride + e) = o;
+    for (int w = 0; w < 4; ++w) {
+      ov.w[w] = pack2<T>(s0[2 * w], s0[2 * w + 1]);
+      ok.w[w] = pack2<T>(s1[2 * w] * a.softmax_scale, s1[2 * w + 1] * a.softmax_scale);
     }
+    *reinterpret_cast<Pack8 *>(dvg + (int64_t)key * a.dv_row_stride + e) = ov;
+    *reinterpret_cast<Pack8 *>(dkg + (int64_t)key * a.dk_row_stride + e) = ok;
   }
+}
+
+template <typename T>
+static int launch_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, hipStream_t s) {
+  auto kern = attn_bwd_dkdv_wide_kernel<T>;
+  const size_t smem = BwdWideSmem::bytes;
+  if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
+    set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
+    return 2;
+  }
+  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_k, 64);
+  if (items >= ((int64_t)1 << 31)) {
+    set_error("attn_bwd: too many (sequence, head, key block) work items");
+    return 1;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(512), smem, s, a, ds_ws);
+  return 0;
 }
 
 // dK / dV and the dS tiles for head dimensions above 128 (ds_ws: the dS workspace, laid out by ds_piece_offset)
 int run_bwd_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, hipStream_t s) {
-  const size_t smem = BwdWideSmem::bytes;
-  const dim3 grid(ceil_div(a.max_seqlen_k, 64), a.heads, a.batch);
-  if (a.dtype == FMOBA_DTYPE_BF16) {
-    auto kern = attn_bwd_dkdv_wide_kernel<bf16_t>;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
-      set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
-      return 2;
-    }
-    hipLaunchKernelGGL(kern, grid, dim3(256), smem, s, a, ds_ws);
-  } else {
-    auto kern = attn_bwd_dkdv_wide_kernel<f16_t>;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
-      set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
-      return 2;
-    }
-    hipLaunchKernelGGL(kern, grid, dim3(256), smem, s, a, ds_ws);
-  }
-  return 0;
+  return a.dtype == FMOBA_DTYPE_BF16 ? launch_dkdv_wide<bf16_t>(a, ds_ws, s) : launch_dkdv_wide<f16_t>(a, ds_ws, s);
 }
 
 }  // namespace fmoba

@@ -30,6 +30,7 @@ namespace fmoba {
 // row-block form when a row selects at least 10/50 (64-key blocks) resp. 10/27 (128-key blocks) of the chunks it may see:
 // measured break-even points (16 heads of 128, 8K and 16K tokens per sequence, top-k 8 to 32)
 constexpr int kFwdRowsDensity64 = 50, kFwdRowsDensity128 = 27;
+constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 
 struct FwdWs {
   int32_t *cnt;      // [total_q * heads] visits handed out per (row, head)
@@ -322,7 +323,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
 // One 16-lane group per (row, head), four per wave, sixteen per block of 256: a row's chain of dependent steps (count,
 // headers, order, rows) is mostly waiting, so a wave runs four of them side by side.  Lane li of a group owns the
 // 16-byte piece li of the row.
-template <typename T>
+// (head dimensions above 128: pieces li and li + 16, NP = 2)
+template <typename T, int NP>
 __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_args a, FwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
   __shared__ float sWgt[16][16], sWl[16][16];
@@ -342,10 +344,10 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   int nmax = max(n, __shfl_xor(n, 16, 64));
   nmax = max(nmax, __shfl_xor(nmax, 32, 64));  // the wave walks the longest of its four rows
   const int c8 = li * 8;
-  const bool mine = c8 < D;
-  float acc[8];
+  const bool mine = c8 < D, mine2 = NP > 1 && c8 + 128 < D;
+  float acc[8 * NP];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+  for (int i = 0; i < 8 * NP; ++i) acc[i] = 0.f;
   float L = 0.f, M = -INFINITY;
   const float4 *hdr = ws.hdr + rh * ws.cap;
   const uint16_t *part = ws.part + rh * ws.cap * D;
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
     const float Mu = Mn == -INFINITY ? 0.f : Mn;
     const float resc = __builtin_amdgcn_exp2f(M - Mu);  // M = -inf: nothing accumulated yet, factor 0 on zeros
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] *= resc;
+    for (int i = 0; i < 8 * NP; ++i) acc[i] *= resc;
     L *= resc;
     M = Mn;
     const float wj = (li < cntb) ? __builtin_amdgcn_exp2f(mj - Mu) : 0.f;
@@ -383,36 +385,49 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
     // sums in rank order: every lane of the group adds the same sequence
     for (int t = 0; t < cntb; ++t) L += sWl[sg][t];
     if (mine) {
-      auto add = [&](const Pack8 &x, float w) {
+      auto add = [&](const Pack8(&x)[NP], float w) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          acc[2 * k] = fmaf(w, elem_to_float<T>((uint16_t)(x.w[k] & 0xffffu)), acc[2 * k]);
-          acc[2 * k + 1] = fmaf(w, elem_to_float<T>((uint16_t)(x.w[k] >> 16)), acc[2 * k + 1]);
-        }
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            acc[8 * p + 2 * k] = fmaf(w, elem_to_float<T>((uint16_t)(x[p].w[k] & 0xffffu)), acc[8 * p + 2 * k]);
+            acc[8 * p + 2 * k + 1] = fmaf(w, elem_to_float<T>((uint16_t)(x[p].w[k] >> 16)), acc[8 * p + 2 * k + 1]);
+          }
+      };
+      auto load = [&](Pack8(&x)[NP], int slot) {
+        const uint16_t *row = part + (int64_t)slot * D + c8;
+        x[0] = ld_stream16(row);
+        if constexpr (NP > 1) x[1] = ld_stream16(mine2 ? row + 128 : row);
       };
       int t = 0;
       for (; t + 4 <= cntb; t += 4) {  // independent loads, four in flight
-        Pack8 x[4];
+        Pack8 x[4][NP];
         float w[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          x[u] = ld_stream16(part + (int64_t)sOrd[base + t + u] * D + c8);
+          load(x[u], sOrd[base + t + u]);
           w[u] = sWgt[sg][t + u];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) add(x[u], w[u]);
       }
-      for (; t < cntb; ++t) add(ld_stream16(part + (int64_t)sOrd[base + t] * D + c8), sWgt[sg][t]);
+      for (; t < cntb; ++t) {
+        Pack8 x[NP];
+        load(x, sOrd[base + t]);
+        add(x, sWgt[sg][t]);
+      }
     }
   }
   if (!valid) return;
   const bool empty = !(L > 0.f);
   const float inv = empty ? 0.f : 1.f / L;
-  if (mine) {
+  uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + row * a.o_row_stride + (int64_t)h * a.o_head_stride + c8;
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
     Pack8 o;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o.w[k] = pack2<T>(acc[2 * k] * inv, acc[2 * k + 1] * inv);
-    *reinterpret_cast<Pack8 *>(reinterpret_cast<uint16_t *>(a.out) + row * a.o_row_stride + (int64_t)h * a.o_head_stride + c8) = o;
+    for (int k = 0; k < 4; ++k) o.w[k] = pack2<T>(acc[8 * p + 2 * k] * inv, acc[8 * p + 2 * k + 1] * inv);
+    if (p == 0 ? mine : mine2) *reinterpret_cast<Pack8 *>(op + 128 * p) = o;
   }
   if (li == 0) a.softmax_lse[(int64_t)h * a.total_q + row] = empty ? INFINITY : (M + __builtin_amdgcn_logf(L)) * 0.6931471805599453f;
 }
@@ -454,6 +469,11 @@ __global__ __launch_bounds__(256) void max_i32_kernel(const int32_t *p, int64_t 
 
 static inline size_t fwd_align256(size_t x) { return (x + 255) & ~(size_t)255; }
 static inline int fwd_key_block(int lg_block_n) { return lg_block_n % 128 == 0 ? 128 : 64; }
+// partial slots per (row, head): the caller's bound counts key blocks of fwd_key_block keys, and head dimensions above 128
+// have blocks of 64 (K and V of 128 keys would not leave room for a second workgroup on the unit)
+static inline int64_t fwd_partial_cap(const fmoba_attn_fwd_args &a) {
+  return (int64_t)a.max_visits_per_row * (a.head_dim > 128 ? fwd_key_block(a.lg_block_n) / 64 : 1);
+}
 
 // the row-block form (attn_fwd_rows.hip)
 bool fwd_rows_feasible(const fmoba_attn_fwd_args &a);
@@ -465,10 +485,16 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s);
 // visit: the first wins while a row selects more than about a fifth of the chunks it may see (64-key blocks) or
 // more than about three eighths of them (128-key blocks, whose visits cost the column form less per key).
 static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
-  if (a.head_dim > 128) return true;  // head dimensions above 128 only have the row-block form
   if (a.fwd_mode == 1) return false;
   if (!fwd_rows_feasible(a)) return false;
   if (a.fwd_mode == 2) return true;
+  // Head dimensions above 128: a visit costs the column form a third of what the (row, 64 keys) step costs the row-block form
+  // (2 x 4096 tokens, 8 heads of 256, 8 of 128-key chunks: 1023 -> 275 us), so it serves dense patterns too,
+  // up to the size of the partial results that a call may ask for.
+  if (a.head_dim > 128) {
+    const int64_t partials = (int64_t)a.total_q * a.heads * fwd_partial_cap(a);
+    return partials >= ((int64_t)1 << 31) || partials * (a.head_dim * 2 + 16) > kWidePartialBytes;
+  }
   const int64_t chunks_per_seq = std::max<int64_t>(1, ceil_div64(ceil_div64(std::max(a.total_k, 1), a.batch), a.lg_block_n));
   const int64_t chunks_per_row = std::max<int64_t>(1, (int64_t)a.max_visits_per_row * fwd_key_block(a.lg_block_n) / a.lg_block_n);
   const int64_t seen = a.is_causal ? (chunks_per_seq + 1) / 2 : chunks_per_seq;
@@ -498,7 +524,9 @@ static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hi
     hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, rows);
     const int kb = fwd_key_block(a.lg_block_n);
     int rc;
-    if (a.head_dim <= 64)
+    if (a.head_dim > 128)
+      rc = launch_fwd_col<T, 256, 64>(a, ws, s);
+    else if (a.head_dim <= 64)
       rc = kb == 128 ? launch_fwd_col<T, 64, 128>(a, ws, s) : launch_fwd_col<T, 64, 64>(a, ws, s);
     else
       rc = kb == 128 ? launch_fwd_col<T, 128, 128>(a, ws, s) : launch_fwd_col<T, 128, 64>(a, ws, s);
@@ -507,7 +535,7 @@ static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hi
   if (phases & FMOBA_FWD_COMBINE) {
     const int capl = combine_order_entries(ws.cap);
     const size_t smem = (size_t)16 * capl * 4;
-    auto kern = attn_fwd_combine_kernel<T>;
+    auto kern = a.head_dim > 128 ? attn_fwd_combine_kernel<T, 2> : attn_fwd_combine_kernel<T, 1>;
     if (smem > 32 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
       set_error("attn_fwd: a row with up to %d visits needs %zu bytes of LDS for the order of its partial results", ws.cap, smem);
       return 2;
@@ -521,18 +549,18 @@ static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hi
 
 extern "C" int32_t fmoba_attn_fwd_key_block(int32_t lg_block_n) { return fmoba::fwd_key_block(lg_block_n); }
 
-static size_t fwd_cols_workspace_bytes(int32_t total_q, int32_t heads, int32_t head_dim, int32_t max_visits_per_row) {
+static size_t fwd_cols_workspace_bytes(const fmoba_attn_fwd_args &a) {
   using namespace fmoba;
-  if (total_q <= 0 || heads <= 0 || head_dim <= 0 || max_visits_per_row <= 0) return 256;
-  const size_t rows = (size_t)total_q * heads;
-  return fwd_align256((rows + 1) * 4) + fwd_align256(rows * max_visits_per_row * 16) + fwd_align256(rows * max_visits_per_row * head_dim * 2) + 256;
+  if (a.max_visits_per_row <= 0) return 256;
+  const size_t rows = (size_t)a.total_q * a.heads, cap = (size_t)fwd_partial_cap(a);
+  return fwd_align256((rows + 1) * 4) + fwd_align256(rows * cap * 16) + fwd_align256(rows * cap * a.head_dim * 2) + 256;
 }
 
 extern "C" size_t fmoba_attn_fwd_workspace_bytes(const fmoba_attn_fwd_args *a) {
   using namespace fmoba;
   if (a == nullptr || a->total_q <= 0 || a->heads <= 0 || a->head_dim <= 0 || a->batch <= 0 || a->lg_block_n <= 0) return 256;
   if (fwd_use_rows(*a)) return fwd_rows_workspace_bytes(*a);
-  return fwd_cols_workspace_bytes(a->total_q, a->heads, a->head_dim, a->max_visits_per_row);
+  return fwd_cols_workspace_bytes(*a);
 }
 
 extern "C" int32_t fmoba_attn_fwd_uses_row_blocks(const fmoba_attn_fwd_args *a) {
@@ -603,8 +631,7 @@ extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phase
                 "attn_fwd: q, k, v and out must be 16-byte aligned");
   FMOBA_REQUIRE(a->max_visits_per_row > 0, "attn_fwd: max_visits_per_row must be positive");
   FMOBA_REQUIRE(a->fwd_mode >= 0 && a->fwd_mode <= 2, "attn_fwd: fwd_mode must be 0 (automatic), 1 (columns) or 2 (row blocks)");
-  FMOBA_REQUIRE(a->fwd_mode != 1 || a->head_dim <= 128, "attn_fwd: head dimensions above 128 only have the row-block form");
-  FMOBA_REQUIRE((a->fwd_mode != 2 && a->head_dim <= 128) || fwd_rows_feasible(*a), "attn_fwd: the row-block form does not take this shape (more than %d chunks or %d keys per sequence)",
+  FMOBA_REQUIRE(a->fwd_mode != 2 || fwd_rows_feasible(*a), "attn_fwd: the row-block form does not take this shape (more than %d chunks or %d keys per sequence)",
                 32 * 128, 64 * 4096);
   const size_t need = fmoba_attn_fwd_workspace_bytes(a);
   FMOBA_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= need, "attn_fwd: workspace too small (%zu < %zu)", a->workspace_bytes, need);
@@ -614,12 +641,12 @@ extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phase
     return 0;
   }
   const size_t rows = (size_t)a->total_q * a->heads;
-  FMOBA_REQUIRE(rows * (size_t)a->max_visits_per_row < ((size_t)1 << 31),
+  FMOBA_REQUIRE(rows * (size_t)fwd_partial_cap(*a) < ((size_t)1 << 31),
                 "attn_fwd: %zu partial rows exceed the 2^31 the column form indexes (their workspace would not fit any device either)",
-                rows * (size_t)a->max_visits_per_row);
+                rows * (size_t)fwd_partial_cap(*a));
   uintptr_t p = ((uintptr_t)a->workspace + 255) & ~(uintptr_t)255;
   FwdWs ws;
-  ws.cap = a->max_visits_per_row;
+  ws.cap = (int32_t)fwd_partial_cap(*a);
   ws.cnt = reinterpret_cast<int32_t *>(p);
   p += fwd_align256((rows + 1) * 4);
   ws.hdr = reinterpret_cast<float4 *>(p);
