@@ -806,21 +806,23 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
 // ------------------------------------------------------------------------------------
 // dK / dV, dS tiles form: TODO comment
 // ------------------------------------------------------------------------------------
-template <int HD>
+template <int HD, bool DQP>
 struct DkdvSmem {
   static constexpr size_t tile = (size_t)64 * HD * 2;        // 64 gathered rows of Q or dO, swizzled (tile_swz)
   static constexpr size_t oQ = 0;                             // [2 buffers]
   static constexpr size_t odO = oQ + 2 * tile;                // [2 buffers]
   static constexpr size_t oP = odO + 2 * tile;                // [64 rows][64 keys], piece p (8 keys) of row r at p ^ (r & 7)
   static constexpr size_t odS = oP + 64 * 128;
-  static constexpr size_t bytes_loop = odS + 64 * 128;
+  static constexpr size_t oOut = odS + 64 * 128;              // partials form: [64 rows][HD], dQ part rows on their way out
+  static constexpr size_t oSlot = oOut + (DQP ? (size_t)64 * HD * 2 : 0);  // int[2][64]: places of the part rows
+  static constexpr size_t bytes_loop = oSlot + (DQP ? 2 * 64 * 4 : 0);
   static constexpr int LDR = HD + 4;                          // floats, output staging [2][64 keys][LDR]
   static constexpr size_t bytes = bytes_loop > (size_t)2 * 64 * LDR * 4 ? bytes_loop : (size_t)2 * 64 * LDR * 4;
 };
 
-template <typename T, int HD>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws) {
-  typedef DkdvSmem<HD> SM;
+template <typename T, int HD, bool DQP>
+__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
+  typedef DkdvSmem<HD, DQP> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, NDW = NDT / 2, LDR = SM::LDR;
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
@@ -902,6 +904,22 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_b
     vf[ks] = lds_read16(((ldsdO + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
     if (D < HD && (hh * KS + ks) * 8 >= D) kf[ks] = vf[ks] = zero_pack8();
   }
+  // partials form: K^T of this wave's half of the features, the A operand of dQ^T = K^T dS^T (keys 16 s4 + 8 hh .. + 7)
+  Pack8 ktf[DQP ? NDW : 1][4];
+  if constexpr (DQP) {
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+      for (int d = 0; d < NDW; ++d) {
+        uint32_t ad[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int key = 16 * s4 + 8 * hh + 4 * u + (li >> 2);
+          ad[u] = ldsQ + (uint32_t)(key * RB + ((((kq * NDW + d) * 4 + ((lane >> 4) & 1) * 2 + ((li & 3) >> 1)) ^ tile_swz<HD>(key)) * 16) + (li & 1) * 8);
+        }
+        ktf[d][s4] = lds_tr8(ad[0], ad[1]);
+      }
+  }
   __syncthreads();
   if (nround > 0) {
     // rows of round r + 1 (ids `rid`): Q and dO into the other buffer, 16 rows per wave
@@ -920,11 +938,20 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_b
     int rid = code(rid_nx, 0);
     feed(rid, 0);
     float lse = lseg[rid & 0x7fffffff], del = delg[rid & 0x7fffffff];
+    // partials form: the waves of key half 0 hand out the part rows of their 32 rows, a round ahead (a spare row takes what
+    // absent rows and visits beyond the caller's bound write)
+    int slot = 0;
+    int *sSlot = reinterpret_cast<int *>(smem + SM::oSlot);
+    const int trash = a.total_q * a.heads * ws.cap;
+    auto take = [&](int rd, int r) {
+      if constexpr (DQP) slot = take_slot(ws.cnt + ((int64_t)(q0 + (rd & 0x7fffffff)) * a.heads + h), __ballot(rd >= 0 && hh == 0 && kq == 0 && r < nround));
+    };
+    take(rid, 0);
     rid_nx = list[min(64 + myrow, n - 1)];
     auto arrived = [&]() {
       wait_all_loads();
 #if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(lse), "+v"(del), "+v"(rid_nx));
+      asm volatile("" : "+v"(lse), "+v"(del), "+v"(rid_nx), "+v"(slot));
 #endif
     };
     arrived();
@@ -935,11 +962,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_b
       const uint32_t buf = (r & 1) ? TILE : 0u;
       const int rcur = rid;
       const float lse2 = rcur >= 0 ? lse * kLog2e : INFINITY, delta = del;
+      if constexpr (DQP) {
+        if (kq == 0 && hh == 0) sSlot[(r & 1) * 64 + myrow] = (rcur >= 0 && slot < ws.cap) ? ((q0 + rcur) * a.heads + h) * ws.cap + slot : trash;
+      }
       // the next round's rows
       rid = code(rid_nx, r + 1);
       if (r + 1 < nround) feed(rid, buf ^ TILE);
       lse = lseg[rid & 0x7fffffff];
       del = delg[rid & 0x7fffffff];
+      take(rid, r + 1);
       rid_nx = list[min((r + 2) * 64 + myrow, n - 1)];
       // S^T and dP^T: lane -> row, register i -> key kq * 32 + acc_row(i, hh)
       f32x16 s, dp;
@@ -1014,9 +1045,40 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_b
           for (int kk = 0; kk < 2; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
         __builtin_amdgcn_sched_barrier(0);
       });
-      arrived();
-      // dS of row `lane`, key groups 2 wave and 2 wave + 1: consecutive lanes write consecutive pieces of the dS tile
-      {
+      if constexpr (DQP) {
+        // dQ^T[f][row] of this wave's 32 rows and its half (kq) of the features, over all keys of the block
+        f32x16 dq[NDW];
+        Pack8 sf[4];
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) sf[s4] = lds_read16(ldsdS + (uint32_t)(myrow * 128) + (((uint32_t)(2 * s4 + hh) ^ psw) * 16u));
+#pragma unroll
+        for (int d = 0; d < NDW; ++d) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) dq[d][i] = 0.f;
+#pragma unroll
+          for (int s4 = 0; s4 < 4; ++s4) dq[d] = mfma32<T>(ktf[d][s4], sf[s4], dq[d]);
+        }
+        // rows through LDS, so that a row's 16-byte pieces leave together (piece p of row r at p ^ (r & 7))
+        const uint32_t ldsOut = lds + (uint32_t)SM::oOut;
+#pragma unroll
+        for (int d = 0; d < NDW; ++d)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            lds_write_vec<uint2>(ldsOut + (uint32_t)(myrow * RB + hh * 8) + (((uint32_t)((kq * NDW + d) * 4 + g) ^ psw) * 16u),
+                                 make_uint2(pack2<T>(dq[d][4 * g], dq[d][4 * g + 1]), pack2<T>(dq[d][4 * g + 2], dq[d][4 * g + 3])));
+        arrived();
+        __syncthreads();  // the part rows are there (and the next round's rows)
+#pragma unroll
+        for (int v = tid; v < 64 * VPR; v += 256) {
+          const int row = v / VPR, pcs = v - row * VPR;
+          const uint32_t p = (uint32_t)sSlot[(r & 1) * 64 + row];
+          const Pack8 x = lds_read16(ldsOut + (uint32_t)(row * RB) + (((uint32_t)pcs ^ (uint32_t)(row & 7)) * 16u));
+          if (pcs * 8 < D) st_stream16(ws.part + ((uint64_t)p * (uint32_t)D + (uint32_t)(pcs * 8)), x);
+          if (pcs == 0) ws.pid[p] = nb;
+        }
+      } else {
+        arrived();
+        // dS of row `lane`, key groups 2 wave and 2 wave + 1: consecutive lanes write consecutive pieces of the dS tile
         const int p = r * 64 + lane;
         Pack8 x[2];
 #pragma unroll
@@ -1024,7 +1086,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_b
         if (p < n) {
           const int64_t pos = lbase + start + p;
 #pragma unroll
-          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(ds_ws + ds_piece_offset(pos, (koff >> 3) + 2 * wave + u, Bn >> 3)) = x[u];
+          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(ws.ds + ds_piece_offset(pos, (koff >> 3) + 2 * wave + u, Bn >> 3)) = x[u];
         }
       }
       __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
@@ -1573,6 +1635,23 @@ static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_
   return near_rows ? launch_dkdv_form<T, HD, DQP, KB, true>(a, ws, s) : launch_dkdv_form<T, HD, DQP, KB, false>(a, ws, s);
 }
 
+template <typename T, int HD, bool DQP>
+static int launch_dkdv_rows(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
+  auto kern = attn_bwd_dkdv_rows_kernel<T, HD, DQP>;
+  const size_t smem = DkdvSmem<HD, DQP>::bytes;
+  if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
+    set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
+    return 2;
+  }
+  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_k, 64);
+  if (items >= ((int64_t)1 << 31)) {
+    set_error("attn_bwd: too many (sequence, head, key block) work items");
+    return 1;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws);
+  return 0;
+}
+
 template <typename T, int HD, int RT>
 static int launch_dq(const fmoba_attn_bwd_args &a, const uint16_t *ws, hipStream_t s) {
   auto kern = attn_bwd_dq_kernel<T, HD, RT>;
@@ -1641,21 +1720,9 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
     const bool wide = bwd_wide_blocks(a);
     if (partials) {
       hipLaunchKernelGGL(zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, (int64_t)a.total_q * a.heads);
-      rc = a.head_dim <= 64 ? launch_dkdv<T, 64, true, 1>(a, ws, s) : (wide ? launch_dkdv<T, 128, true, 2>(a, ws, s) : launch_dkdv<T, 128, true, 1>(a, ws, s));
+      rc = a.head_dim <= 64 ? launch_dkdv_rows<T, 64, true>(a, ws, s) : (wide ? launch_dkdv<T, 128, true, 2>(a, ws, s) : launch_dkdv<T, 128, true, 1>(a, ws, s));
     } else {
-      if (getenv("FM_OLD") == nullptr) {
-        if (a.head_dim <= 64) {
-          auto kern = attn_bwd_dkdv_rows_kernel<T, 64>;
-          hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)DkdvSmem<64>::bytes);
-          hipLaunchKernelGGL(kern, dim3(a.batch * a.heads * ceil_div(a.max_seqlen_k, 64)), dim3(256), DkdvSmem<64>::bytes, s, a, ws.ds);
-        } else {
-          auto kern = attn_bwd_dkdv_rows_kernel<T, 128>;
-          hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)DkdvSmem<128>::bytes);
-          hipLaunchKernelGGL(kern, dim3(a.batch * a.heads * ceil_div(a.max_seqlen_k, 64)), dim3(256), DkdvSmem<128>::bytes, s, a, ws.ds);
-        }
-        rc = 0;
-      } else
-      rc = a.head_dim <= 64 ? launch_dkdv<T, 64, false, 1>(a, ws, s) : (wide ? launch_dkdv<T, 128, false, 2>(a, ws, s) : launch_dkdv<T, 128, false, 1>(a, ws, s));
+      rc = a.head_dim <= 64 ? launch_dkdv_rows<T, 64, false>(a, ws, s) : launch_dkdv_rows<T, 128, false>(a, ws, s);
     }
     if (rc) return rc;
   }

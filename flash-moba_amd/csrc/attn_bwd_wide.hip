@@ -8,7 +8,7 @@
 // each, with K resp. V of its key half in registers.  A round takes 64 gathered rows, which loads bring straight into LDS one
 // round ahead; dP - delta goes to the wave that holds S of the same tile through LDS (fp32), P and dS to everybody (16 bits).
 // 2 x 4096 tokens, 8 heads of 256, 8 of 128-key chunks: 1223 us with one 32-row tile at a time between two barriers and
-// K and V as LDS operands, @US@ us now.  What bounds it: one operand from LDS per product, and the two exchanges.
+// K and V as LDS operands, 235 us now.  What bounds it: one operand from LDS per product, and the two exchanges.
 #include "fmoba_common.h"
 
 #include <type_traits>

@@ -47,25 +47,6 @@ struct FwdColSmem {
   static_assert(2 * bytes <= 160 * 1024, "two workgroups per compute unit");
 };
 
-// *p += 1 in the lanes of `lanes`; the old value arrives with the wave's other loads (the caller waits), what the other
-// lanes get is undefined
-__device__ __forceinline__ int take_slot(int32_t *p, unsigned long long lanes) {
-  int old = 0;
-#if defined(__HIP_DEVICE_COMPILE__)
-  unsigned long long saved;
-  asm volatile("s_mov_b64 %1, exec\n\t"
-               "s_mov_b64 exec, %2\n\t"
-               "global_atomic_add %0, %3, %4, off sc0\n\t"
-               "s_mov_b64 exec, %1"
-               : "=&v"(old), "=&s"(saved)
-               : "s"(lanes), "v"(p), "v"(1)
-               : "memory");
-#else
-  (void)p, (void)lanes;
-#endif
-  return old;
-}
-
 // Two workgroups per compute unit, two waves per SIMD, no barrier after the block's K and V have arrived.  What bounds it
 // depends on the lists.  Long ones (32768 tokens, 32 heads, top-k 16 of 256 chunks: 2000 rows per list): the partial
 // results on their way out and the gathered Q rows, together about 4 TB/s.  Short ones (a part of a prompt against the

@@ -677,6 +677,25 @@ __device__ __forceinline__ void wait_all_loads() {
 __host__ __device__ __forceinline__ int64_t ds_piece_offset(int64_t p, int kg, int kgs) { return ((((p >> 5) * kgs + kg) << 5) + (p & 31)) << 3; }
 static inline size_t ds_workspace_tiles(int64_t positions) { return (size_t)((positions > 0 ? positions : 0) + 31) / 32 + 1; }
 
+// *p += 1 in the lanes of `lanes`; the old value arrives with the wave's other loads (the caller waits), what the other
+// lanes get is undefined
+__device__ __forceinline__ int take_slot(int32_t *p, unsigned long long lanes) {
+  int old = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+  unsigned long long saved;
+  asm volatile("s_mov_b64 %1, exec\n\t"
+               "s_mov_b64 exec, %2\n\t"
+               "global_atomic_add %0, %3, %4, off sc0\n\t"
+               "s_mov_b64 exec, %1"
+               : "=&v"(old), "=&s"(saved)
+               : "s"(lanes), "v"(p), "v"(1)
+               : "memory");
+#else
+  (void)p, (void)lanes;
+#endif
+  return old;
+}
+
 // Row id of a gathered tile row as it is kept in LDS: r itself if the entry is present and the row exists, else
 // negative with a row that exists in the low 31 bits (the entry's own if it exists: past the end of a list that is the
 // list's last row, whose data the column meets anyway; else row 0).  The tile loads fetch that row unconditionally, the
