@@ -17,7 +17,7 @@ LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libflash_moba_hip.so")
 HOST_MODULE = "flash_moba_host"  # the eager host path (csrc/torch_ops.cpp), a Python extension beside the library
 HOST_LIB = os.path.join(LIBDIR, HOST_MODULE + ".so")
-SOURCES = ["fmoba_host.hip", "mean_pool.hip", "topk_csc.hip", "varlen_sort.hip", "attn_fwd.hip", "attn_fwd_rows.hip", "attn_bwd.hip", "attn_bwd_wide.hip"]
+SOURCES = ["fmoba_host.hip", "mean_pool.hip", "topk_csc.hip", "varlen_sort.hip", "attn_fwd.hip", "attn_fwd_rows.hip", "attn_fwd_few.hip", "attn_bwd.hip", "attn_bwd_wide.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # keep packed-fp32 VALU ops out of the generated code

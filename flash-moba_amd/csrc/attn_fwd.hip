@@ -458,6 +458,7 @@ static inline int64_t fwd_partial_cap(const fmoba_attn_fwd_args &a) {
 
 // the row-block form (attn_fwd_rows.hip)
 bool fwd_rows_feasible(const fmoba_attn_fwd_args &a);
+bool fwd_few_rows(const fmoba_attn_fwd_args &a);  // its variant for calls with a handful of rows (attn_fwd_few.hip)
 size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a);
 int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s);
 
@@ -468,7 +469,7 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s);
 static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   if (a.fwd_mode == 1) return false;
   if (!fwd_rows_feasible(a)) return false;
-  if (a.fwd_mode == 2) return true;
+  if (a.fwd_mode == 2 || fwd_few_rows(a)) return true;
   // Head dimensions above 128: a visit costs the column form a third of what the (row, 64 keys) step costs the row-block form
   // (2 x 4096 tokens, 8 heads of 256, 8 of 128-key chunks: 1023 -> 275 us), so it serves dense patterns too,
   // up to the size of the partial results that a call may ask for.

@@ -848,6 +848,10 @@ static int launch_rows_loader(const fmoba_attn_fwd_args &a, const uint32_t *bm, 
   return 0;
 }
 
+// a call with a handful of rows (attn_fwd_few.hip)
+bool fwd_few_rows(const fmoba_attn_fwd_args &a);
+void run_fwd_few(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s);
+
 bool fwd_rows_feasible(const fmoba_attn_fwd_args &a) {
   return a.head_dim <= 256 && ceil_div(a.max_cols, 32) <= kRowsWordCap && ceil_div(a.max_seqlen_k, 64) <= kRowsStepCap &&
          a.max_cols < 32768 && a.lg_block_n % 64 == 0;
@@ -871,6 +875,10 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
       hipLaunchKernelGGL(fwd_zero_u32_kernel, dim3(512), dim3(256), 0, s, own, rows * nw);
       hipLaunchKernelGGL(csc_bitmap_kernel, dim3(a.max_cols, a.heads, a.batch), dim3(256), 0, s, a, own, nw);
     }
+  }
+  if ((phases & 2) && fwd_few_rows(a)) {
+    run_fwd_few(a, bm, nw, s);
+    return 0;
   }
   if (phases & 2) {
     const bool bf = a.dtype == FMOBA_DTYPE_BF16;

@@ -11,6 +11,7 @@
 //                      ascending, so no sort pass is needed afterwards.
 #include "fmoba_common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace fmoba {
@@ -1418,6 +1419,133 @@ __global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void topk_gate_stream_kernel(
   }
 }
 
+// ------------------------------------------------------------------------------------
+// The gate for calls with at most eight query rows per sequence (decode steps).  The kernels above give a row to a pair
+// of lanes and let four waves work on 128 rows; with one row three of the waves and 63 of 64 lanes idle through a chain of
+// LDS reads, products and a dozen probes (20 us for 16 requests of up to 256 chunks, 32 heads).  Here the eight waves share the
+// chunks (their means straight from memory as the A operand: nothing is read twice), the scores of the few rows meet in
+// LDS, and a whole wave searches the cut of a row: a chunk per lane and register, a count is a ballot.  The products are
+// the same as above, so are the scores, and the order (score descending, chunk descending) is total: the same selection.
+// 20 -> 13.6 us there.
+// ------------------------------------------------------------------------------------
+constexpr int kFewGateRows = 8, kFewGateChunks = 4096;
+
+// NJ: chunks per lane of a row's wave
+template <typename T, int HD, int NJ>
+__global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
+  constexpr int KS = HD / 16;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  float *sScore = reinterpret_cast<float *>(smem);  // [rows][NJ * 64]
+  const fmoba_fused_topk_args &a = p.a;
+  const int h = blockIdx.x, b = blockIdx.y;
+  const int q0 = a.cu_seqlens_q[b];
+  const int Lq = min(a.cu_seqlens_q[b + 1] - q0, a.max_seqlen_q);  // (at most kFewGateRows)
+  if (Lq <= 0) return;
+  const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b];
+  const int km0 = a.cu_seqlens_km[b];
+  const int Cb = min(min(a.cu_seqlens_km[b + 1] - km0, p.max_cols), NJ * 64);
+  const int off = Lk - (a.cu_seqlens_q[b + 1] - q0);
+  const int B = a.chunk, D = a.head_dim;
+  const int hk = h / (a.heads / a.heads_k);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
+  int nsc = Cb;  // chunks that are candidates of the last row
+  if (a.is_causal) {
+    const int rmax = Lq - 1 + off;
+    nsc = rmax < 0 ? 0 : min(Cb, rmax / B);
+  }
+  const int r = lane & 31;
+  Pack8 qf[KS];
+  {
+    const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + min(r, Lq - 1)) * a.q_row_stride + (int64_t)h * a.q_head_stride;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int e = (hh * KS + ks) * 8;
+      qf[ks] = (r < Lq && e < D) ? ld_global16(qp + e) : zero_pack8();
+    }
+  }
+  const uint16_t *kmp = reinterpret_cast<const uint16_t *>(a.km) + (int64_t)km0 * a.km_row_stride + (int64_t)hk * a.km_head_stride;
+  for (int t = wave; t * 32 < nsc; t += 8) {
+    const uint16_t *row = kmp + (int64_t)min(t * 32 + (lane & 31), nsc - 1) * a.km_row_stride;
+    Pack8 af[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) af[ks] = ld_global16(row + min((hh * KS + ks) * 8, D - 8));
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) s = mfma32<T>(af[ks], qf[ks], s);
+    if (r < Lq) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4 *>(sScore + r * (NJ * 64) + t * 32 + 8 * g + 4 * hh) = f32x4{s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
+    }
+  }
+  __syncthreads();
+  if (wave >= Lq) return;
+  {
+    const int row = wave, rp = row + off;
+    const bool self = a.is_causal && rp >= 0;
+    const int nc = a.is_causal ? (rp >= 0 ? min(min(rp / B, Cb), nsc) : 0) : Cb;
+    const int kp = a.is_causal ? a.topk - 1 : a.topk;
+    const int pself = self ? rp / B : -1;
+    // keys in the order of the scores; 0: no candidate, or a score that no cut lies below (-inf, not a number)
+    uint32_t key[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int c = j * 64 + lane;
+      key[j] = 0u;
+      if (j * 64 < nc) {
+        const float x = sScore[row * (NJ * 64) + c] + 0.f;  // (-0 is +0)
+        key[j] = (c < nc && x > -INFINITY) ? float_order_key(x) : 0u;
+      }
+    }
+    auto count_ge = [&](uint32_t v) {
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (j * 64 < nc) n += __popcll(__ballot(key[j] >= v));
+      return n;
+    };
+    // the largest cut with at least K' keys at or above it (1: all of them, if there are no more than K')
+    uint32_t cut = 1u;
+    if (kp > 0 && count_ge(1u) > kp) {
+      cut = 0u;
+      for (int bit = 31; bit >= 0; --bit) {
+        const uint32_t trial = cut | (1u << bit);
+        if (count_ge(trial) >= kp) cut = trial;
+      }
+    }
+    int spare = kp - (cut == 0xffffffffu ? 0 : count_ge(cut + 1u));  // places left for the keys equal to the cut: the highest chunks
+    uint32_t w_lo = 0u, w_hi = 0u;                                  // lane w: words w and 64 + w of the row
+#pragma unroll
+    for (int j = NJ - 1; j >= 0; --j) {
+      if (j * 64 >= p.max_cols) continue;
+      unsigned long long m = 0ull;
+      if (kp > 0 && j * 64 < nc) {
+        m = __ballot(key[j] > cut);
+        unsigned long long eq = __ballot(key[j] == cut);
+        int n = __popcll(eq);
+        while (n > spare) {
+          eq &= eq - 1ull;  // the lowest chunk goes
+          --n;
+        }
+        spare -= n;
+        m |= eq;
+      }
+      if (self && (pself >> 6) == j) m |= 1ull << (pself & 63);
+      if (p.segcnt != nullptr && ((m >> lane) & 1ull) && j * 64 + lane < p.max_cols)
+        atomicAdd(&p.segcnt[((int64_t)b * a.heads + h) * p.nseg * p.max_cols + j * 64 + lane], 1);
+      const uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+      uint32_t &w = j < 32 ? w_lo : w_hi;
+      const int at = (2 * j) & 63;
+      w = lane == at ? lo : lane == at + 1 ? hi : w;
+    }
+    uint32_t *selp = p.sel + (int64_t)h * p.W * a.total_q + q0 + row;
+    if (lane < p.W) selp[(int64_t)lane * a.total_q] = w_lo;
+    if (64 + lane < p.W) selp[(int64_t)(64 + lane) * a.total_q] = w_hi;
+  }
+}
+
 // grid (heads, batch), block 256
 __global__ __launch_bounds__(256) void csc_scan_kernel(TopkParams p) {
   const fmoba_fused_topk_args &a = p.a;
@@ -1733,6 +1861,29 @@ static int launch_gate_big_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
   if (kp <= 16) return launch_gate_stream<T, 256, 2>(p, grid, s);
   return launch_gate_big<T, 256, 4, kBigCap>(p, grid, s);
 }
+template <typename T, int HD, int NJ>
+static int launch_gate_few_nj(const TopkParams &p, hipStream_t s) {
+  const size_t smem = (size_t)std::min(p.a.max_seqlen_q, kFewGateRows) * NJ * 64 * 4;
+  auto kern = topk_gate_few_kernel<T, HD, NJ>;
+  if (smem > 32 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
+    set_error("fused_topk: cannot reserve %zu bytes of LDS", smem);
+    return 2;
+  }
+  hipLaunchKernelGGL(kern, dim3(p.a.heads, p.a.batch), dim3(512), smem, s, p);
+  return 0;
+}
+template <typename T, int HD>
+static int launch_gate_few(const TopkParams &p, hipStream_t s) {
+  if (p.max_cols <= 256) return launch_gate_few_nj<T, HD, 4>(p, s);
+  if (p.max_cols <= 1024) return launch_gate_few_nj<T, HD, 16>(p, s);
+  return launch_gate_few_nj<T, HD, 64>(p, s);
+}
+template <typename T>
+static int launch_gate_few_hd(const TopkParams &p, hipStream_t s) {
+  if (p.a.head_dim <= 64) return launch_gate_few<T, 64>(p, s);
+  if (p.a.head_dim <= 128) return launch_gate_few<T, 128>(p, s);
+  return launch_gate_few<T, 256>(p, s);
+}
 template <typename T>
 static int launch_gate_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
   if (p.a.head_dim <= 64) return launch_gate_nt<T, 64>(p, grid, s);
@@ -1823,7 +1974,9 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   if (!lists) p.segcnt = nullptr;
   dim3 ggrid(ceil_div(a->max_seqlen_q, kGateRows), a->heads, a->batch);
   int rc;
-  if (big)
+  if (a->max_seqlen_q <= kFewGateRows && max_cols <= kFewGateChunks)
+    rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_few_hd<bf16_t>(p, s) : launch_gate_few_hd<f16_t>(p, s);
+  else if (big)
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_big_hd<bf16_t>(p, ggrid, s) : launch_gate_big_hd<f16_t>(p, ggrid, s);
   else
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_hd<bf16_t>(p, ggrid, s) : launch_gate_hd<f16_t>(p, ggrid, s);

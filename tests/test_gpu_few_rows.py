@@ -1,0 +1,56 @@
+"""Calls with at most eight query rows per sequence: their own gate and attention kernels."""
+import numpy as np
+import pytest
+import torch
+
+import flash_moba
+from flash_moba import flash_moba_hip as hip
+from flash_moba.mean_pool import flash_topk_mean_pool
+from gpu_utils import assert_close
+from oracle import moba_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(lens_q, lens_k, H, Hk, D, dtype, seed, integer=False):
+    g = torch.Generator().manual_seed(seed)
+    mk = lambda n, h: (torch.randint(-2, 3, (n, h, D), generator=g).float() if integer else torch.randn((n, h, D), generator=g)).to(dtype)
+    cu = lambda lens: torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    return mk(sum(lens_q), H), mk(sum(lens_k), Hk), mk(sum(lens_k), Hk), cu(lens_q), cu(lens_k)
+
+
+# chunks per sequence: none before the row's own, one tile of 32, at and past 64 and 256 (registers of a lane), past 1024;
+# rows: one, eight, none; ties everywhere with integer inputs
+@pytest.mark.parametrize("lens_q,lens_k,chunk,topk", [
+    ([1], [5], 64, 3), ([1, 1, 0, 1], [2048, 64, 100, 65], 64, 4), ([8, 3], [64 * 65 + 1, 700], 64, 7), ([1, 2], [64 * 257, 64 * 40], 64, 33),
+    ([4], [3000], 2, 16), ([1, 1], [4096, 2500], 1, 64), ([5], [3], 64, 2)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("integer", [True, False])
+@pytest.mark.parametrize("D", [64, 96, 256])
+def test_gate_selects_what_the_wide_gates_select(lens_q, lens_k, chunk, topk, causal, integer, D):
+    # the same rows inside a longer query block go through the gates with 128 rows per workgroup
+    q, k, _, cuq, cuk = (t.cuda() for t in _case(lens_q, lens_k, 4, 2, D, torch.bfloat16, len(lens_k) + topk, integer))
+    mq, mk = max(lens_q), max(lens_k)
+    km, cu_km, _ = flash_topk_mean_pool(k, cuk, mk, chunk)
+    few = hip.moba_fused_topk(q, km, cuq, cuk, cu_km, mq, mk, topk, chunk, causal, return_raw=False, return_selection=True)
+    wide = hip.moba_fused_topk(q, km, cuq, cuk, cu_km, 9, mk, topk, chunk, causal, return_raw=False, return_selection=True)
+    assert all(torch.equal(few[i], wide[i]) for i in (0, 1, 2, 5))
+
+
+@pytest.mark.parametrize("lens_q,lens_k,chunk,topk", [
+    ([1], [5], 64, 3), ([1, 1, 1, 0, 1], [2048, 64, 129, 100, 3000], 128, 4), ([3, 8], [1000, 4097], 64, 5), ([1, 2], [64 * 257, 64 * 40], 256, 9)])
+@pytest.mark.parametrize("H,Hk", [(4, 4), (8, 1)])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (40, torch.float16), (128, torch.float16), (96, torch.bfloat16), (256, torch.bfloat16), (160, torch.float16)])
+def test_attention_of_a_few_rows(lens_q, lens_k, chunk, topk, H, Hk, D, dtype):
+    q, k, v, cuq, cuk = _case(lens_q, lens_k, H, Hk, D, dtype, D + topk)
+    mq, mk = max(lens_q), max(lens_k)
+    where = (cuq.cuda(), cuk.cuda(), mq, mk)
+    out = flash_moba.flash_moba_varlen_func(q.cuda(), k.cuda(), v.cuda(), *where, chunk, topk, causal=True)
+    co, cn, ind = flash_moba.flash_topk_varlen_func(q.cuda(), k.cuda(), *where, topk, chunk, causal=True)
+    cols, lse, _, _ = hip.moba_varlen_fwd(q.cuda(), k.cuda(), v.cuda(), None, co, cn, ind, *where[:2], None, None, None, mq, mk, 0.0, D ** -0.5,
+                                          False, True, 0.0, False, 128, chunk, None, _fwd_mode=1)
+    out2, lse2, _, _ = hip.moba_varlen_fwd(q.cuda(), k.cuda(), v.cuda(), None, co, cn, ind, *where[:2], None, None, None, mq, mk, 0.0, D ** -0.5,
+                                           False, True, 0.0, False, 128, chunk, None)
+    assert torch.equal(out, out2)
+    assert_close("out", out, cols.float().cpu(), 2e-2, 1e-2)
+    assert_close("lse", lse2, lse.float().cpu(), 2e-3, 1e-3)
