@@ -400,66 +400,83 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 }
 
 // ------------------------------------------------------------------------------------
-// The same walk with EIGHT compute waves (256 query rows per workgroup, two waves per SIMD) and no loader waves, for
-// head dimensions up to 128: the matrix products of one wave run under the softmax arithmetic of the other wave of
-// its SIMD.  K and V tiles go from global memory straight into LDS (every wave issues an eighth of a tile's loads,
-// three steps ahead for K and two for V, rings of three stages) in rows of exactly HD elements, swizzled instead of
-// padded (piece c of row r lies at piece c ^ tile_swz(r)): the 16-byte row reads of the K operands and the transposing
-// reads of the V^T operands both spread over all banks.  Keys past the sequence and features past head_dim are fetched
-// from a key and a piece that exist: the scores of such keys are masked, Q is zero in such features and the
-// corresponding output features are never stored.
+// The same walk without loader waves, for head dimensions up to 128: four waves of 32 rows and 256 registers, two
+// workgroups per compute unit, so that the matrix products of one run under the softmax arithmetic of the other whatever
+// their steps wait for.  K and V tiles go from global memory straight into LDS (every wave issues a quarter of a tile's
+// loads, one step ahead, rings of two stages each) in rows of exactly HD elements, swizzled instead of padded (piece c of row
+// r lies at piece c ^ tile_swz(r)): the 16-byte row reads of the K operands and the transposing reads of the V^T operands
+// both spread over all banks.  Keys past the sequence and features past head_dim are fetched from a key and a piece that
+// exist: the scores of such keys are masked, Q is zero in such features and the corresponding output features are never
+// stored.
+// With eight waves of one workgroup in step (256 rows, the second four a part of a step late, rings two and three steps
+// ahead), half of the tile loads but one barrier for all: 65536 tokens in eight sequences, top-k 32 of 64-key chunks 3.08 ms
+// against 2.87 here, 2 x 4096 tokens 247 against 205 us, 12037 tokens in five sequences 290 against 253, 8191 tokens of short
+// documents with heads of 64 51 against 40 (two workgroups cover each other's first loads, and 128 rows are less padding).
+// SPLIT = 2: a second set of four waves takes every other step of the same rows, with rings of its own; the two results of a
+// row meet in LDS at the end.
 // ------------------------------------------------------------------------------------
-constexpr int kRows8 = 256;  // rows of a workgroup
-constexpr int kRows8Words = 16;  // selection words per row that the workgroup keeps in LDS (512 chunks)
+constexpr int kRowsWords = 16;  // selection words per row that the workgroup keeps in LDS (512 chunks)
 
-template <int HD>
-struct FwdRows8Smem {
+template <int HD, int SPLIT>
+struct FwdRowsDirectSmem {
+  static constexpr int ROWS = 128;  // rows of a workgroup: 32 for each of four waves
   static constexpr int LDO = HD + 8;   // elements, per-wave output tile [32 rows][LDO]
   static constexpr size_t tile = (size_t)64 * HD * 2;       // one 64-key tile of K or V
-  static constexpr size_t oK = 0;                             // [3 stages]
-  static constexpr size_t oV = oK + 3 * tile;                 // [4 stages]; the output tiles reuse both rings at the end
-  static constexpr size_t oStep = oV + 4 * tile;              // int[kRowsStepCap]: key block | chunk << 16
-  static constexpr size_t oUnion = oStep + (size_t)kRowsStepCap * 4;
-  static constexpr size_t oOff = oUnion + (size_t)kRowsWordCap * 4;  // int[8]
-  static constexpr size_t oBits = oOff + (size_t)(kRowsWordCap + 1) * 4 + 12;  // uint32[kRows8Words][256]: the rows' selection words
-  static constexpr size_t bytes = oBits + (size_t)kRows8Words * kRows8 * 4;
-  static_assert((size_t)8 * 32 * LDO * 2 <= 7 * tile, "output tiles must fit the K/V rings");
-  static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
+  static constexpr size_t ring = 4 * tile;                    // K, K, V, V: the rings of one set of four waves
+  static constexpr size_t oStep = SPLIT * ring;               // int[step_cap]: key block | chunk << 16
+  // behind the steps, sized by the call: uint32[nw] union, int[8], uint32[nw][ROWS] the rows' selection words
+  static size_t bytes(int step_cap, int nw) { return oStep + ((size_t)step_cap + nw + 8 + (size_t)nw * ROWS) * 4; }
+  static_assert((size_t)4 * 32 * LDO * 2 <= ring && (size_t)4 * HD * 128 <= ring, "output tiles must fit the K/V rings");
 };
 
-template <typename T, int HD>
-__global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw) {
-  typedef FwdRows8Smem<HD> SM;
+template <typename T, int HD, int SPLIT>
+__global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap) {
+  typedef FwdRowsDirectSmem<HD, SPLIT> SM;
+  constexpr int kRows = SM::ROWS;
   constexpr int KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
-  constexpr int NTHR = 512;
+  constexpr int NTHR = SPLIT * 256;
   constexpr int RB = HD * 2;            // bytes of a tile row
   constexpr int RPI = 64 / VPR;         // tile rows per direct-to-LDS instruction (64 lanes x 16 bytes)
   constexpr int NI = 64 / RPI / 4;      // such instructions per tile and feeding wave
   static_assert(NI >= 1, "four waves share the loads of a tile");
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   int *sStep = reinterpret_cast<int *>(smem + SM::oStep);
-  uint32_t *sUnion = reinterpret_cast<uint32_t *>(smem + SM::oUnion);
-  int *sOff = reinterpret_cast<int *>(smem + SM::oOff);
-  uint32_t *sBits = reinterpret_cast<uint32_t *>(smem + SM::oBits);
+  uint32_t *sUnion = reinterpret_cast<uint32_t *>(sStep + step_cap);
+  int *sOff = reinterpret_cast<int *>(sUnion + nw);
+  uint32_t *sBits = reinterpret_cast<uint32_t *>(sOff + 8);
 
-  const int nrb = (a.max_seqlen_q + kRows8 - 1) / kRows8;
+  const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
   const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb);
   const int b = item.pair / a.heads, h = item.pair - b * a.heads;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   const int rb = nrb - 1 - item.idx;  // the longest walks (last rows of a causal sequence) start first
-  const int r0 = rb * kRows8;
+  const int r0 = rb * kRows;
   if (r0 >= Lq) return;
   const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
   const int off = Lk - Lq;
   const int D = a.head_dim;
   const int hk = h / (a.heads / a.heads_k);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hh = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
+  const int wave = wave_all & 3, set = wave_all >> 2;  // rows 32 wave .., steps set, set + SPLIT, ..
   const bool causal = a.is_causal != 0;
   const int Bn = a.lg_block_n, sub = Bn >> 6;
   const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
 
+  const int row = r0 + wave * 32 + (lane & 31);
+  const bool valid = row < Lq;
+  // this lane's query row as the B operand of S^T = K Q^T: asked for first, on its way while the steps are counted
+  Pack8 qb[KS];
+  {
+    const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + min(row, Lq - 1)) * a.q_row_stride + (int64_t)h * a.q_head_stride;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int e = (hh * KS + ks) * 8;
+      qb[ks] = (valid && e < D) ? ld_global16(qg + e) : zero_pack8();
+    }
+  }
+
   // ---- the steps of this row block -------------------------------------------------------------
-  const int rlast = min(r0 + kRows8 - 1, Lq - 1);
+  const int rlast = min(r0 + kRows - 1, Lq - 1);
   const int kend = min(Lk, causal ? rlast + off + 1 : Lk);  // keys [0, kend) are visible to some row
   const int nchunk = kend > 0 ? (kend + Bn - 1) / Bn : 0;
   const int nwu = min((nchunk + 31) >> 5, nw);
@@ -473,7 +490,7 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
     for (int i = tid; i < nrow * nwu; i += NTHR) {
       const int w = i / nrow, row = i - w * nrow;
       const uint32_t x = bp[(int64_t)w * a.total_q + row];
-      sBits[w * kRows8 + row] = x;
+      sBits[w * kRows + row] = x;
       if (x) atomicOr(&sUnion[w], x);
     }
   }
@@ -492,29 +509,29 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
       const int up = __shfl_up(incl, o, 64);
       incl += lane >= o ? up : 0;
     }
-    if (lane == 63) sOff[wave] = incl;
+    if (lane == 63) sOff[wave_all] = incl;
     __syncthreads();
     int before = 0, total = 0;
 #pragma unroll
     for (int w = 0; w < NTHR / 64; ++w) {
       const int v = sOff[w];
-      before += w < wave ? v : 0;
+      before += w < wave_all ? v : 0;
       total += v;
     }
     int pos = nstep_all + before + incl - cnt;
     for (int jb = 0; jb < cnt; ++jb, ++pos)
-      if (pos < kRowsStepCap) sStep[pos] = (c * sub + jb) | (c << 16);
+      if (pos < step_cap) sStep[pos] = (c * sub + jb) | (c << 16);
     nstep_all += total;
     __syncthreads();
   }
-  const int nstep = min(nstep_all, kRowsStepCap);
+  const int nstep_wg = min(nstep_all, step_cap);
+  const int nstep = (nstep_wg - set + SPLIT - 1) / SPLIT, nturn = (nstep_wg + SPLIT - 1) / SPLIT;  // this set's steps, the turns of the loop
+  auto entry = [&](int t) { return sStep[min(t * SPLIT + set, nstep_wg - 1)]; };
 
   typedef std::integral_constant<int, 0> C0;
   typedef std::integral_constant<int, 1> C1;
-  const int row = r0 + wave * 32 + (lane & 31);
-  const bool valid = row < Lq;
-  if (nstep == 0) {  // no visible selected key: out = 0, lse = +inf for the rows of this block
-    if (valid) {
+  if (nstep_wg == 0) {  // no visible selected key: out = 0, lse = +inf for the rows of this block
+    if (valid && set == 0) {
       uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + row) * a.o_row_stride + (int64_t)h * a.o_head_stride;
       for (int e = hh * 8; e < D; e += 16) *reinterpret_cast<Pack8 *>(op + e) = zero_pack8();
       if (hh == 0) a.softmax_lse[(int64_t)h * a.total_q + q0 + row] = INFINITY;
@@ -525,7 +542,7 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
   // ---- feeding the rings: the waves 0..3 fetch the tiles, rows wave * 16 .. wave * 16 + 15 each.  They reach the
   // barrier of a step well before the waves 4..7 (which run a step's last part one step late and meet them on the
   // matrix cores at the end of the step), so the loads are theirs ---------------------------------------------------
-  const uint32_t ldsK = (uint32_t)(uintptr_t)(smem + SM::oK), ldsV = (uint32_t)(uintptr_t)(smem + SM::oV);
+  const uint32_t ldsK = (uint32_t)(uintptr_t)smem + (uint32_t)(set * (int)SM::ring), ldsV = ldsK + (uint32_t)(2 * SM::tile);
   const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)k0 * a.k_row_stride + (int64_t)hk * a.k_head_stride;
   const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)k0 * a.v_row_stride + (int64_t)hk * a.v_head_stride;
   // A lane's piece of row tr = wave * 16 + i * RPI + lane / VPR of a tile: its byte offset from the tile's first key, for K
@@ -543,8 +560,7 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
     }
   }
   auto feed = [&](const uint16_t *g, uint32_t row_stride, const uint32_t(&lof)[NI], uint32_t lds_ring, int stage, int t) {
-    if (wave >= 4) return;
-    const int key0 = __builtin_amdgcn_readfirstlane((sStep[min(t, nstep - 1)] & 0xffff) << 6);
+    const int key0 = __builtin_amdgcn_readfirstlane((entry(t) & 0xffff) << 6);
     const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + wave * (64 / 4) * RB);
     if (key0 + 64 <= Lk) {
       const uint16_t *base = g + (uint64_t)(uint32_t)key0 * row_stride;
@@ -561,22 +577,9 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
       }
     }
   };
-  auto feed_k = [&](int t) { feed(kg, (uint32_t)a.k_row_stride, lofK, ldsK, t % 3, t); };
-  auto feed_v = [&](int t) { feed(vg, (uint32_t)a.v_row_stride, lofV, ldsV, t & 3, t); };
-  // the loads of a step, once per feeding wave: the wait before the next barrier lets exactly these stay in flight
-  constexpr int kLoadsPerStep = 2 * NI;
-
+  auto feed_k = [&](int t) { feed(kg, (uint32_t)a.k_row_stride, lofK, ldsK, t & 1, t); };
+  auto feed_v = [&](int t) { feed(vg, (uint32_t)a.v_row_stride, lofV, ldsV, t & 1, t); };
   const int lim = valid ? min(causal ? row + off : 0x7fffffff, Lk - 1) : -1;  // last visible key
-  // this lane's query row as the B operand of S^T = K Q^T
-  Pack8 qb[KS];
-  {
-    const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + min(row, Lq - 1)) * a.q_row_stride + (int64_t)h * a.q_head_stride;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int e = (hh * KS + ks) * 8;
-      qb[ks] = (valid && e < D) ? ld_global16(qg + e) : zero_pack8();
-    }
-  }
   // (Q is in registers before the first tile loads are issued: from here on the wave counts its outstanding loads)
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
@@ -586,8 +589,6 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
   feed_k(0);
   feed_k(1);
   feed_v(0);
-  feed_k(2);
-  feed_v(1);
 
   f32x16 o[NDT];  // O^T: register i of feature tile dt <-> feature dt*32 + acc_row(i, hh), this lane's row
 #pragma unroll
@@ -639,13 +640,13 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
   Pack8 kf[KS];        // K operands of S(t + 1): read at the start of part0, their latency runs under its arithmetic
   Pack8 vt[2][2];      // V^T operands of the first feature tile of step t: read at the end of part1
   float neg_mc = 0.f;  // minus the reference point of the row's exponentials, scaled; -inf for a row that skips the step
-  int s_nx = sStep[0];  // entry of the next step and this row's word of selection bits for its chunk
-  uint32_t word_nx = sBits[((s_nx >> 16) >> 5) * kRows8 + wave * 32 + (lane & 31)];
+  int s_nx = entry(0);  // entry of the next step and this row's word of selection bits for its chunk
+  uint32_t word_nx = sBits[((s_nx >> 16) >> 5) * kRows + wave * 32 + (lane & 31)];
   auto part0 = [&](auto par, int t) {
     constexpr int P = decltype(par)::value;
     f32x16(&sc)[2] = st[P];
     {
-      uint32_t akn = ldsK + (uint32_t)(((t + 1) % 3) * (int)SM::tile) + rowoff;  // K(t + 1)
+      uint32_t akn = ldsK + (uint32_t)(((t + 1) & 1) * (int)SM::tile) + rowoff;  // K(t + 1)
       opaque(akn);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) kf[ks] = k_frag(akn, 0, ks);
@@ -691,11 +692,11 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
   };
   auto part1 = [&](auto par, int t) {
     constexpr int P = decltype(par)::value;
-    uint32_t akn = ldsK + (uint32_t)(((t + 1) % 3) * (int)SM::tile) + rowoff;  // K(t + 1)
+    uint32_t akn = ldsK + (uint32_t)(((t + 1) & 1) * (int)SM::tile) + rowoff;  // K(t + 1)
     opaque(akn);
     f32x16(&sc)[2] = st[P];
     f32x16(&sn)[2] = st[P ^ 1];
-    uint32_t tv = ldsV + (uint32_t)((t & 3) * (int)SM::tile) + troff;  // V(t)
+    uint32_t tv = ldsV + (uint32_t)((t & 1) * (int)SM::tile) + troff;  // V(t)
     opaque(tv);
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
@@ -716,8 +717,8 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
       const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[kte][2 * j + 1], scale_log2, neg_mc));
       lsum += p0 + p1;
       pf[kte][j / 4].w[j % 4] = pack2<T>(p0, p1);
-      if (g == 2) s_nx = sStep[min(t + 1, nstep - 1)];
-      if (g == 8) word_nx = sBits[((s_nx >> 16) >> 5) * kRows8 + wave * 32 + (lane & 31)];
+      if (g == 2) s_nx = entry(t + 1);
+      if (g == 8) word_nx = sBits[((s_nx >> 16) >> 5) * kRows + wave * 32 + (lane & 31)];
       if (g == 14) {  // V^T operands of the first feature tile
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
@@ -729,7 +730,7 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
     l_run += lsum;
   };
   auto part2 = [&](int t) {
-    uint32_t tv = ldsV + (uint32_t)((t & 3) * (int)SM::tile) + troff;  // V(t)
+    uint32_t tv = ldsV + (uint32_t)((t & 1) * (int)SM::tile) + troff;  // V(t)
     opaque(tv);
     static_for<NDT>([&](auto di) {
       constexpr int dt = decltype(di)::value;
@@ -743,56 +744,61 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
       __builtin_amdgcn_sched_barrier(0);
     });
   };
-  auto wait_older_loads = [&]() {  // all but the loads of the current step
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (kLoadsPerStep == 8)
-      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-#endif
-  };
-  static_assert(kLoadsPerStep == 8 || kLoadsPerStep == 4, "wait_older_loads");
-
-  // K(0), K(1), V(0) have to be there for the first step: the two youngest groups of loads (K(2), V(1)) may stay out
-  wait_older_loads();
+  wait_all_loads();  // K(0), K(1), V(0)
   __syncthreads();
   {
     uint32_t ak0 = ldsK + rowoff;
     opaque(ak0);
     s_plain(ak0, st[0]);
   }
-  const int nstep_pad = (nstep + 1) & ~1;
-  const bool late = wave >= 4;
   auto step = [&](auto par, int t) {
-    // K(t + 1) and V(t) are in LDS (the wait before the last barrier); the readers of K(t) and V(t - 2) are done
-    feed_k(t + 3);
-    feed_v(t + 2);
-    if (late) {
-      if (t >= 1 && t - 1 < nstep) part2(t - 1);
-      if (t < nstep) {
-        part0(par, t);
-        part1(par, t);
-      }
-    } else if (t < nstep) {
+    // K(t + 1) and V(t) are in LDS (the wait before the last barrier); the readers of K(t) and V(t - 1) are done
+    feed_k(t + 2);
+    feed_v(t + 1);
+    if (t < nstep) {
       part0(par, t);
       part1(par, t);
       part2(t);
     }
-    wait_older_loads();
+    wait_all_loads();
     __syncthreads();
   };
-  for (int t = 0; t < nstep_pad; t += 2) {
+  for (int t = 0; t < nturn; t += 2) {
     step(C0{}, t);
-    step(C1{}, t + 1);
+    if (t + 1 < nturn) step(C1{}, t + 1);
   }
-  if (late && nstep_pad - 1 < nstep) part2(nstep_pad - 1);  // (an even number of steps: the last one's products are still due)
-  wait_all_loads();
-  __syncthreads();  // every wave is done with the rings and nothing is in flight: they now hold the output tiles
+  // (every wave is done with the rings and nothing is in flight: they now hold the sets' sums, then the output tiles)
+  if constexpr (SPLIT == 2) {
+    float *sO = reinterpret_cast<float *>(smem + SM::ring);                                // [wave][HD / 2 registers][64 lanes], in the second set's rings
+    float *sMl = reinterpret_cast<float *>(smem);                                          // [wave][2][64]
+    if (set == 1) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sO[(wave * (HD / 2) + dt * 16 + i) * 64 + lane] = o[dt][i];
+      sMl[(wave * 2) * 64 + lane] = m_run;
+      sMl[(wave * 2 + 1) * 64 + lane] = l_run;
+    }
+    __syncthreads();
+    if (set == 0) {
+      const float m1 = sMl[(wave * 2) * 64 + lane], l1 = sMl[(wave * 2 + 1) * 64 + lane];
+      const float mn = fmaxf(m_run, m1), mref = mn == -INFINITY ? 0.f : mn;
+      const float f0 = __builtin_amdgcn_exp2f((m_run - mref) * scale_log2), f1 = __builtin_amdgcn_exp2f((m1 - mref) * scale_log2);
+      m_run = mn;
+      l_run = l_run * f0 + l1 * f1;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * f0 + sO[(wave * (HD / 2) + dt * 16 + i) * 64 + lane] * f1;
+    }
+    __syncthreads();  // (the output tiles lie where m and l of the second set did)
+    if (set == 1) return;
+  }
 
   const float l_tot = sum_xor32_f(l_run);
   const bool empty = !(l_tot > 0.f);
   const float inv = empty ? 0.f : 1.f / l_tot;
-  uint16_t *sOut = reinterpret_cast<uint16_t *>(smem + SM::oK) + (size_t)wave * 32 * LDO;
+  uint16_t *sOut = reinterpret_cast<uint16_t *>(smem) + (size_t)wave * 32 * LDO;
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -814,21 +820,31 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_kernel(fmoba_attn_fwd_args 
   }
 }
 
-template <typename T, int HD>
-static int launch_rows_eight(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
-  auto kern = attn_fwd_rows_kernel<T, HD>;
-  const size_t smem = FwdRows8Smem<HD>::bytes;
+template <typename T, int HD, int SPLIT>
+static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
+  typedef FwdRowsDirectSmem<HD, SPLIT> SM;
+  auto kern = attn_fwd_rows_kernel<T, HD, SPLIT>;
+  const int step_cap = ceil_div(a.max_seqlen_k, 64);  // (at most kRowsStepCap: fwd_rows_feasible)
+  const size_t smem = SM::bytes(step_cap, nw);
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_q, kRows8);
+  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_q, SM::ROWS);
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_fwd: too many (sequence, head, row block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(512), smem, s, a, bm, nw);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * 256), smem, s, a, bm, nw, step_cap);
   return 0;
+}
+// Two sets of waves where the launch leaves compute units idle anyway (at most one workgroup for each of the 256): the walk
+// of a row block is half as long (3072 tokens, 8 heads of 64: 38 -> 30 us).  Otherwise a second workgroup beside the first
+// serves a unit better (8191 tokens of short documents: 40 us with one set, 64 with two).
+template <typename T, int HD>
+static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
+  const int64_t blocks = (int64_t)a.heads * (a.total_q / 128 + a.batch);
+  return blocks <= 256 ? launch_rows_split<T, HD, 2>(a, bm, nw, s) : launch_rows_split<T, HD, 1>(a, bm, nw, s);
 }
 
 template <typename T, int HD>
@@ -883,14 +899,14 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
   if (phases & 2) {
     const bool bf = a.dtype == FMOBA_DTYPE_BF16;
     int rc;
-    // eight compute waves when the rows' selection words fit the workgroup's LDS (up to 512 chunks per sequence)
+    // without loader waves when the rows' selection words fit the workgroup's LDS (up to 512 chunks per sequence)
     // (and the rows of a tile lie within 32-bit byte offsets of its first key)
-    const bool eight = nw <= kRows8Words && a.k_row_stride < ((int64_t)1 << 24) && a.v_row_stride < ((int64_t)1 << 24);
+    const bool direct = nw <= kRowsWords && a.k_row_stride < ((int64_t)1 << 24) && a.v_row_stride < ((int64_t)1 << 24);
     if (a.head_dim <= 64)
-      rc = eight ? (bf ? launch_rows_eight<bf16_t, 64>(a, bm, nw, s) : launch_rows_eight<f16_t, 64>(a, bm, nw, s))
+      rc = direct ? (bf ? launch_rows<bf16_t, 64>(a, bm, nw, s) : launch_rows<f16_t, 64>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 64>(a, bm, nw, s) : launch_rows_loader<f16_t, 64>(a, bm, nw, s));
     else if (a.head_dim <= 128)
-      rc = eight ? (bf ? launch_rows_eight<bf16_t, 128>(a, bm, nw, s) : launch_rows_eight<f16_t, 128>(a, bm, nw, s))
+      rc = direct ? (bf ? launch_rows<bf16_t, 128>(a, bm, nw, s) : launch_rows<f16_t, 128>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 128>(a, bm, nw, s) : launch_rows_loader<f16_t, 128>(a, bm, nw, s));
     else
       rc = bf ? launch_rows_loader<bf16_t, 256>(a, bm, nw, s) : launch_rows_loader<f16_t, 256>(a, bm, nw, s);
