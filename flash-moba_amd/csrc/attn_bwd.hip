@@ -1,28 +1,25 @@
 // Sparse attention backward over a CSC pattern, without a single global atomic.
 //
 //   bwd_prep_kernel      : delta[row] = sum_d dO*O (fp32).
-//   attn_bwd_dkdv_kernel : COLUMN-stationary.  One workgroup per (64-key block, head,
+//   attn_bwd_dkdv_kernel : COLUMN-stationary.  One workgroup per (64-key block, query heads that share it,
 //                          sequence) keeps K and V of the block in registers and walks the block's
-//                          ascending row list in gathered 32-row tiles:
-//                            S = Q K^T, dP = dO V^T             (A = gathered rows, B = K / V halves)
+//                          ascending row lists in rounds of 64 gathered rows:
+//                            S = Q K^T, dP = dO V^T
 //                            P = exp2(S*scale*log2e - LSE*log2e), dS = P o (dP - delta)
-//                            dV^T += dO^T P, dK^T += Q^T dS     (P, dS feed the MFMA from registers;
-//                                                                dO^T, Q^T via transposing LDS reads)
+//                            dV^T += dO^T P, dK^T += Q^T dS     (transposing LDS reads)
 //                            dQ^T_partial = K^T dS^T            (per visit of a (row, key block) pair)
-//                          dK/dV live in accumulator registers for the whole list and are written
+//                          dK/dV live in registers for the whole list and are written
 //                          once.  For dQ the kernel leaves either its dS tiles (16-bit, indexed by
 //                          row-list position) or, per visit, a dQ partial row (16-bit, unscaled) in a
 //                          slot that the row hands out from a counter.
+//   attn_bwd_dkdv_partials_kernel : the same for the long calls, dQ partials at head dimension 128.
 //   attn_bwd_dq_kernel   : dQ from the dS tiles, one workgroup per 128 query rows, dQ in registers
 //                          (patterns in which a 128-row block meets a dozen rows or more per step).
 //   attn_bwd_dq_combine_kernel : dQ from the partials, sixteen lanes per (row, head) add them in ascending
 //                          key-block order and scales.  Work and traffic are proportional to
 //                          the number of visits, whatever the number of chunks per sequence.
-// The dK/dV kernel runs four waves of 512 registers, one per SIMD, and all four compute: two pairs
-// (one wave per 32-key half) that take alternate pairs of tiles and add their sums at the end.  A wave keeps
-// 32 keys x head_dim of dK^T and dV^T plus its K and V operands in registers, which leaves no room for a
-// second wave on the SIMD, so nothing moves data through registers: the gathered Q / dO rows go from global
-// memory straight to LDS (global_load_lds), one round (four tiles) ahead.
+// In the dK/dV kernels nothing moves data through registers: the gathered Q / dO rows go from global
+// memory straight to LDS (global_load_lds), one round ahead.
 #include "fmoba_common.h"
 
 #include <type_traits>
@@ -43,7 +40,7 @@ struct BwdSmem {
   static constexpr size_t tileBytes = (size_t)32 * HD * 2;
   static constexpr size_t oQ = 0;                                   // [2 buffers][4 tiles][32][HD]
   static constexpr size_t odO = oQ + 8 * tileBytes;
-  static constexpr size_t odS = odO + 8 * tileBytes;               // partials form: [2 pairs][2 tile slots][64 keys][LDS_] or [2 tile slots][128 keys][LDS_]; dS form: [4 waves][32 keys][LDS_]
+  static constexpr size_t odS = odO + 8 * tileBytes;               // [2 pairs][2 tile slots][64 keys][LDS_] or [2 tile slots][128 keys][LDS_]
   static constexpr size_t oRid = odS + (size_t)2 * 2 * 64 * LDS_ * 2;  // int[2 buffers][128]: row ids, one round before the rest
   static constexpr size_t oRow = oRid + 2 * kBwdRoundRows * 4;     // int[2 buffers][128]
   static constexpr size_t oSlot = oRow + 2 * kBwdRoundRows * 4;
@@ -56,12 +53,398 @@ struct BwdSmem {
 };
 
 struct BwdWs {
+  int32_t dkv_heads;  // heads of dK / dV (of the kernels that sum query heads)
   int32_t *cnt;    // [total_q * heads] visits handed out per (row, head)
   int32_t *pid;    // [total_q * heads * cap] key block id of each partial
   uint16_t *part;  // [total_q * heads * cap][head_dim] dQ partials (unscaled)
   int32_t cap;
   uint16_t *ds;    // dS tiles (row-stationary dQ form): [row list position / 32][key of the column / 8][position % 32][8 keys]
 };
+
+// ------------------------------------------------------------------------------------
+// dK / dV.  One workgroup per (64 keys, query heads that share them, sequence) walks the row lists of its heads, 64
+// gathered rows a round.  S^T and dP^T of a (32 keys, 32 rows) tile are one wave's (A = K / V in registers, B = the rows: one
+// lane owns one row, so LSE and delta are one register each); P and dS go to LDS, [row][key], 16-bit; then every wave adds
+// up dV^T or dK^T of half of the features and all keys over the round's 64 rows (both operands through transposing
+// reads).  Four waves of 256 registers, two workgroups per compute unit: what one waits for (two barriers a round, the next
+// round's rows, which come straight into LDS a round ahead) the other covers.
+// dQ: the dS form leaves dS, by position in the row lists (attn_bwd_dq_kernel); the partials form, built for head
+// dimensions up to 64, multiplies it with K^T (in registers) and leaves a part row per visit in the slot that the row hands
+// out (attn_bwd_dq_combine_kernel).
+// Measured against one workgroup of four 512-register waves per unit, products and softmax interleaved by hand (which stays
+// for the partials form at head dimension 128, attn_bwd_dkdv_partials_kernel): 8191 tokens of short documents, heads of 64
+// 100 -> 49 us; 12037 tokens, heads of 96 227 -> 177 us; 2 x 4096 tokens 223 -> 214 us; 65536-token batch 2.94 -> 2.65 ms.
+// One workgroup of eight waves per 128 keys (half of the gathers, three buffers): 256 us where two of 64 keys take 214.
+// ------------------------------------------------------------------------------------
+template <int HD, bool DQP>
+struct DkdvSmem {
+  static constexpr int NBUF = 2;
+  static constexpr int PRB = 128;                        // bytes of a P / dS row
+  static constexpr size_t tile = (size_t)64 * HD * 2;        // 64 gathered rows of Q or dO, swizzled (tile_swz)
+  static constexpr size_t oQ = 0;                             // [NBUF]
+  static constexpr size_t odO = oQ + NBUF * tile;             // [NBUF]
+  static constexpr size_t oP = odO + NBUF * tile;             // [64 rows][64 keys], piece p (8 keys) of row r at p ^ (r & 7)
+  static constexpr size_t odS = oP + 64 * PRB;
+  static constexpr size_t oOut = odS + 64 * PRB;              // partials form: [64 rows][HD], dQ part rows on their way out
+  static constexpr size_t oSlot = oOut + (DQP ? (size_t)64 * HD * 2 : 0);  // int[2][64]: places of the part rows
+  static constexpr size_t bytes_loop = oSlot + (DQP ? 2 * 64 * 4 : 0);
+  static constexpr int LDR = HD + 4;                          // floats, output staging [2][64 keys][LDR]
+  static constexpr size_t bytes_out = (size_t)2 * 64 * LDR * 4;
+  static constexpr size_t bytes = bytes_loop > bytes_out ? bytes_loop : bytes_out;
+  static_assert(bytes <= 160 * 1024 && (size_t)64 * HD * 2 <= NBUF * tile, "LDS of one compute unit; K and V pass through the tiles");
+};
+
+template <typename T, int HD, bool DQP>
+__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
+  typedef DkdvSmem<HD, DQP> SM;
+  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, NDW = NDT / 2, LDR = SM::LDR, PRB = SM::PRB;
+  constexpr int NKEY = 64;   // keys of the workgroup
+  constexpr float kLog2e = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
+  const int gh = ws.dkv_heads, gs = a.heads / gh;  // heads of dK / dV, query heads that are added up in one
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * gh, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
+  const int nb = item.idx, b = item.pair / gh, hg = item.pair - b * gh, h0 = hg * gs;
+  const int key0 = nb * NKEY;
+  const int Bn = a.lg_block_n, c = key0 / Bn;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
+  // lane j: the row list of head h0 + j (a group larger than a wave is split by the caller)
+  int nnz = 0;
+  int64_t lbase = 0;
+  if (c < a.max_cols && lane < gs) {
+    const int64_t ci = ((int64_t)b * a.heads + h0 + lane) * a.max_cols + c;
+    nnz = a.col_nnz[ci];
+    lbase = a.col_offsets[ci];
+  }
+  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+  if (key0 >= Lk) return;
+  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+  const int off = Lk - Lq;
+  const int D = a.head_dim;
+  const int hk = h0 / (a.heads / a.heads_k);
+  const int kq = wave & 1, rt = wave >> 1;   // S and dP: this wave's 32 keys and 32 rows
+  const int sel = wave >> 1, fw = wave & 1;  // sums: dV (0) or dK (1), half fw of the features, all keys
+  const bool causal = a.is_causal != 0;
+  const float scale_log2 = a.softmax_scale * kLog2e;
+  const uint32_t lds = (uint32_t)(uintptr_t)smem, ldsQ = lds + (uint32_t)SM::oQ, ldsdO = lds + (uint32_t)SM::odO, ldsP = lds + (uint32_t)SM::oP, ldsdS = lds + (uint32_t)SM::odS;
+  constexpr uint32_t TILE = (uint32_t)SM::tile;
+  constexpr int RPI = 64 / VPR;              // tile rows per load instruction
+  constexpr int NI = 16 / RPI;               // load instructions per wave, operand and round: 16 rows
+  const int rl = lane / VPR, pc = lane % VPR;
+
+  // K and V of the block pass through the tiles on their way to registers
+  {
+    const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
+    const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int key = (wave * NI + i) * RPI + rl;
+      const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
+      const int64_t kc = min(key, Lk - 1 - key0);
+      global_to_lds16(kg + kc * a.k_row_stride + e, ldsQ + (uint32_t)((wave * NI + i) * 1024));
+      global_to_lds16(vg + kc * a.v_row_stride + e, ldsdO + (uint32_t)((wave * NI + i) * 1024));
+    }
+  }
+  // Rows that lie before the block see none of its keys; only a block that is not its column's first has any in its lists
+  // (of a gated pattern; others are masked), so only there the lists are searched for their first row.
+  int start = 0;
+  if (causal && key0 != c * Bn) {
+    for (int g = 0; g < gs; ++g) {
+      const int n = __builtin_amdgcn_readlane(nnz, g);
+      const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)lbase, g), bhi = __builtin_amdgcn_readlane((uint32_t)(lbase >> 32), g);
+      const int st = n > 0 ? lower_bound_wave_i32(a.row_indices + (int64_t)(((uint64_t)bhi << 32) | blo), n, key0 - off) : 0;
+      start = lane == g ? st : start;
+    }
+  }
+  nnz -= start;
+  lbase += start;
+  int incl = (nnz + 63) >> 6;  // rounds of the lists up to this lane's
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int up = __shfl_up(incl, o, 64);
+    incl += lane >= o ? up : 0;
+  }
+  const int nround = __builtin_amdgcn_readlane(incl, 63);
+  const int koff = key0 - c * Bn;  // offset of the block inside its column
+
+  // a round: its head, the place of its first entry in the row lists and how many it has
+  struct Round {
+    int h, n;
+    int64_t pos;
+  };
+  auto round_at = [&](int r) {  // (past the end: the last round again)
+    r = min(r, nround - 1);
+    const int g = __popcll(__ballot(incl <= r));
+    const int j = (r - (g ? __builtin_amdgcn_readlane(incl, g - 1) : 0)) * 64;
+    const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)lbase, g), bhi = __builtin_amdgcn_readlane((uint32_t)(lbase >> 32), g);
+    return Round{h0 + g, __builtin_amdgcn_readlane(nnz, g) - j, (int64_t)(((uint64_t)bhi << 32) | blo) + j};
+  };
+  const int64_t dstride = (int64_t)a.total_q + 128 * (int64_t)a.batch;
+  const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride;
+  const uint16_t *dog = reinterpret_cast<const uint16_t *>(a.dout) + (int64_t)q0 * a.do_row_stride;
+
+  f32x16 acc[NDW][2];  // register i of tile [d][kk] <-> feature (fw * NDW + d) * 32 + acc_row(i, hh), key kk * 32 + lane % 32
+#pragma unroll
+  for (int d = 0; d < NDW; ++d)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[d][kk][i] = 0.f;
+
+  const int myrow = rt * 32 + (lane & 31);  // this lane's row of a round
+  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
+  const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
+  const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
+  auto entry_at = [&](const Round &w) { return a.row_indices + w.pos + min(myrow, w.n - 1); };
+  auto code = [&](int raw, const Round &w) { return tile_row_code(raw, myrow < w.n, Lq); };
+  Round w0{}, w1{};  // the round at hand and the one after it
+  int raw0 = 0, raw_nx = 0;
+  if (nround > 0) {
+    w0 = round_at(0), w1 = round_at(1);
+    raw0 = *entry_at(w0), raw_nx = *entry_at(w1);
+  }
+  wait_all_loads();
+  __syncthreads();
+  Pack8 kf[KS], vf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    kf[ks] = lds_read16(((ldsQ + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
+    vf[ks] = lds_read16(((ldsdO + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
+    if (D < HD && (hh * KS + ks) * 8 >= D) kf[ks] = vf[ks] = zero_pack8();
+  }
+  // partials form: K^T of this wave's features, the A operand of dQ^T = K^T dS^T (keys 16 s4 + 8 hh .. + 7)
+  Pack8 ktf[DQP ? NDW : 1][4];
+  if constexpr (DQP) {
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+      for (int d = 0; d < NDW; ++d) {
+        uint32_t ad[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int key = 16 * s4 + 8 * hh + 4 * u + (li >> 2);
+          ad[u] = ldsQ + (uint32_t)(key * RB + ((((kq * NDW + d) * 4 + ((lane >> 4) & 1) * 2 + ((li & 3) >> 1)) ^ tile_swz<HD>(key)) * 16) + (li & 1) * 8);
+        }
+        ktf[d][s4] = lds_tr8(ad[0], ad[1]);
+      }
+  }
+  __syncthreads();
+  if (nround > 0) {
+    // rows of a round (ids `rid`): Q and dO into the buffer, 16 rows per wave, of its own 32
+    int ft = tid;  // thread index for the code around the products, re-made opaque in every round: what is derived from it is not kept in registers
+    auto feed = [&](int rid, const Round &w, uint32_t buf) {
+      const int fl = ft & 63, rl = fl / VPR, pc = fl % VPR;
+      const uint16_t *qh = qg + (int64_t)w.h * a.q_head_stride, *doh = dog + (int64_t)w.h * a.do_head_stride;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int tr = kq * 16 + i * RPI + rl;  // row of the tile of 32
+        const uint32_t src = (uint32_t)__shfl(rid, tr, 64) & 0x7fffffffu;
+        const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
+        const uint32_t dst = buf + (uint32_t)((rt * 32 + kq * 16 + i * RPI) * RB);
+        global_to_lds16(qh + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
+        global_to_lds16(doh + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
+      }
+    };
+    int rid0 = code(raw0, w0), rid1 = code(raw_nx, w1);
+    feed(rid0, w0, 0);
+    float lse = 0.f, del = 0.f;
+    int slot = 0;
+    int *sSlot = reinterpret_cast<int *>(smem + SM::oSlot);
+    const int trash = a.total_q * a.heads * ws.cap;  // a spare part row: takes what absent rows and visits beyond the caller's bound write
+    // LSE, delta and (partials form, handed out by the waves of key quarter 0) the part row of a round's rows
+    auto scalars = [&](int rid, const Round &w, bool counted) {
+      const int rc = rid & 0x7fffffff;
+      lse = a.softmax_lse[(int64_t)w.h * a.total_q + q0 + rc];
+      del = a.softmax_d[(int64_t)w.h * dstride + q0 + 128 * b + rc];
+      if constexpr (DQP) slot = take_slot(ws.cnt + ((int64_t)(q0 + rc) * a.heads + w.h), __ballot(rid >= 0 && hh == 0 && kq == 0 && counted));
+    };
+    auto arrived = [&]() {
+      wait_all_loads();
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(lse), "+v"(del), "+v"(raw_nx), "+v"(slot));
+#endif
+    };
+    scalars(rid0, w0, true);
+    arrived();
+    __syncthreads();
+    uint32_t buf = 0u;
+    for (int r = 0; r < nround; ++r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (DQP) asm volatile("" : "+v"(ft));
+#endif
+      // places of this lane in the P and dS rows (and of its row in a round)
+      const int fl = ft & 63, fh = fl >> 5, fli = fl & 15, frow = rt * 32 + (fl & 31), fr = (fli >> 2) + 4 * fh;
+      const uint32_t pw = (uint32_t)(frow * PRB + fh * 8), psw = (uint32_t)(frow & 7);
+      const uint32_t pread = (uint32_t)(fr * PRB + (((((fl >> 4) & 1) * 2 + ((fli & 3) >> 1)) ^ (fr & 7)) * 16) + (fli & 1) * 8);
+      const Round w2 = round_at(r + 2);
+      const float lse2 = rid0 >= 0 ? lse * kLog2e : INFINITY, delta = del;
+      if constexpr (DQP) {
+        if (kq == 0 && fh == 0) sSlot[(r & 1) * 64 + frow] = (rid0 >= 0 && slot < ws.cap) ? ((q0 + rid0) * a.heads + w0.h) * ws.cap + slot : trash;
+      }
+      // the next round's rows and scalars, the row ids of the one after it
+      if (r + 1 < nround) feed(rid1, w1, buf ^ TILE);
+      scalars(rid1, w1, r + 1 < nround);
+      raw_nx = *entry_at(w2);
+      // S^T and dP^T: lane -> row, register i -> key kq * 32 + acc_row(i, hh)
+      f32x16 s, dp;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
+      const uint32_t aq = ldsQ + buf + (uint32_t)(rt * 32 * RB) + rowoff, ad = ldsdO + buf + (uint32_t)(rt * 32 * RB) + rowoff;
+      constexpr int NB = DQP ? 1 : 2;  // k-steps per batch of reads
+      Pack8 qf[2][NB], df[2][NB];
+      auto rd = [&](auto bc) {
+        constexpr int B = decltype(bc)::value;
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          qf[B & 1][u] = lds_read16(aq ^ (uint32_t)((B * NB + u) * 16));
+          df[B & 1][u] = lds_read16(ad ^ (uint32_t)((B * NB + u) * 16));
+        }
+      };
+      rd(std::integral_constant<int, 0>{});
+      static_for<KS / NB>([&](auto bc) {
+        constexpr int B = decltype(bc)::value;
+        if constexpr (B + 1 < KS / NB) rd(std::integral_constant<int, B + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          s = mfma32<T>(kf[B * NB + u], qf[B & 1][u], s);
+          dp = mfma32<T>(vf[B * NB + u], df[B & 1][u], dp);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      const int lim = rid0 < 0 ? -1 : min(causal ? rid0 + off : 0x7fffffff, Lk - 1) - key0 - kq * 32;  // last visible key of this wave's 32
+      if (!__all(lim >= 31)) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 8 * (i >> 2) + (i & 3) + 4 * hh <= lim ? s[i] : -INFINITY;
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float p[4], d[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          p[j] = __builtin_amdgcn_exp2f(fmaf(s[4 * g + j], scale_log2, -lse2));
+          d[j] = p[j] * (dp[4 * g + j] - delta);
+        }
+        const uint32_t at = pw + (((uint32_t)(kq * 4 + g) ^ psw) * 16u);
+        lds_write_vec<uint2>(ldsP + at, make_uint2(pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3])));
+        lds_write_vec<uint2>(ldsdS + at, make_uint2(pack2<T>(d[0], d[1]), pack2<T>(d[2], d[3])));
+      }
+      __syncthreads();  // P and dS of the round are in LDS
+      // dV^T[f][key] += dO^T[f][row] P[row][key], dK^T[f][key] += Q^T[f][row] dS[row][key]
+      const uint32_t tx = (sel ? ldsQ : ldsdO) + buf + troff, px = (sel ? ldsdS : ldsP) + pread;
+      Pack8 pb[2][2], xa[2][NDW];
+      auto rd2 = [&](auto sc) {
+        constexpr int S4 = decltype(sc)::value;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          const uint32_t po = (px ^ (uint32_t)(kk * 64)) + (uint32_t)(S4 * 16 * PRB);
+          pb[S4 & 1][kk] = lds_tr8(po, po + 8 * PRB);
+        }
+#pragma unroll
+        for (int d = 0; d < NDW; ++d) {
+          const uint32_t dt = (uint32_t)(fw * NDW + d), xlo = dt * 64u, xhi = ((dt * 4u) ^ (uint32_t)TileSwz<HD>::kRow8) * 16u;
+          const uint32_t olo = (uint32_t)(S4 * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
+          xa[S4 & 1][d] = lds_tr8((tx ^ xlo) + olo, (tx ^ xhi) + ohi);
+        }
+      };
+      rd2(std::integral_constant<int, 0>{});
+      static_for<4>([&](auto sc) {
+        constexpr int S4 = decltype(sc)::value;
+        if constexpr (S4 < 3) rd2(std::integral_constant<int, S4 + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < NDW; ++d)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr (DQP) {
+        // dQ^T[f][row] of this wave's 32 rows and its share of the features, over all keys of the block
+        f32x16 dq[NDW];
+#pragma unroll
+        for (int d = 0; d < NDW; ++d)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) dq[d][i] = 0.f;
+        Pack8 sf[2][2];
+        auto rd3 = [&](auto sc) {
+          constexpr int S = decltype(sc)::value;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) sf[S & 1][u] = lds_read16(ldsdS + (uint32_t)(frow * PRB) + (((uint32_t)(2 * (2 * S + u) + fh) ^ psw) * 16u));
+        };
+        rd3(std::integral_constant<int, 0>{});
+        static_for<2>([&](auto sc) {
+          constexpr int S = decltype(sc)::value;
+          if constexpr (S + 1 < 2) rd3(std::integral_constant<int, S + 1>{});
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int d = 0; d < NDW; ++d) dq[d] = mfma32<T>(ktf[d][2 * S + u], sf[S & 1][u], dq[d]);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        // rows through LDS, so that a row's 16-byte pieces leave together (piece p of row r at p ^ (r & 7))
+        const uint32_t ldsOut = lds + (uint32_t)SM::oOut;
+#pragma unroll
+        for (int d = 0; d < NDW; ++d)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            lds_write_vec<uint2>(ldsOut + (uint32_t)(frow * RB + fh * 8) + (((uint32_t)((kq * NDW + d) * 4 + g) ^ psw) * 16u),
+                                 make_uint2(pack2<T>(dq[d][4 * g], dq[d][4 * g + 1]), pack2<T>(dq[d][4 * g + 2], dq[d][4 * g + 3])));
+        arrived();
+        __syncthreads();  // the part rows are there; the next round's rows are, and this one's are no longer read
+#pragma unroll
+        for (int v0 = 0; v0 < 64 * VPR; v0 += 256) {
+          const int v = v0 + ft, row = v / VPR, pcs = v - row * VPR;
+          const uint32_t p = (uint32_t)sSlot[(r & 1) * 64 + row];
+          const Pack8 x = lds_read16(ldsOut + (uint32_t)(row * RB) + (((uint32_t)pcs ^ (uint32_t)(row & 7)) * 16u));
+          if (pcs * 8 < D) st_stream16(ws.part + ((uint64_t)p * (uint32_t)D + (uint32_t)(pcs * 8)), x);
+          if (pcs == 0) ws.pid[p] = nb;
+        }
+      } else {
+        arrived();
+        // dS of row `lane`, key groups 2 wave and 2 wave + 1: consecutive lanes write consecutive pieces of the dS tile
+        Pack8 x[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) x[u] = lds_read16(ldsdS + (uint32_t)(lane * PRB) + (((uint32_t)(2 * wave + u) ^ (uint32_t)(lane & 7)) * 16u));
+        if (lane < w0.n) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(ws.ds + ds_piece_offset(w0.pos + lane, (koff >> 3) + 2 * wave + u, Bn >> 3)) = x[u];
+        }
+        __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
+      }
+      w0 = w1, rid0 = rid1;
+      w1 = w2, rid1 = code(raw_nx, w2);
+      buf ^= TILE;
+    }
+    __syncthreads();  // (the last part rows have left LDS)
+  }
+
+  // ---- dK^T / dV^T leave as rows, once ----
+  float *red = reinterpret_cast<float *>(smem);  // [dV, dK][keys][LDR]
+#pragma unroll
+  for (int d = 0; d < NDW; ++d)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4 *>(red + (size_t)(sel * NKEY + kk * 32 + (lane & 31)) * LDR + (fw * NDW + d) * 32 + 8 * g + 4 * hh) =
+            f32x4{acc[d][kk][4 * g], acc[d][kk][4 * g + 1], acc[d][kk][4 * g + 2], acc[d][kk][4 * g + 3]};
+  __syncthreads();
+  uint16_t *dkg = reinterpret_cast<uint16_t *>(a.dk) + (int64_t)(k0 + key0) * a.dk_row_stride + (int64_t)hg * a.dk_head_stride;
+  uint16_t *dvg = reinterpret_cast<uint16_t *>(a.dv) + (int64_t)(k0 + key0) * a.dv_row_stride + (int64_t)hg * a.dv_head_stride;
+  for (int v = tid; v < NKEY * VPR; v += 256) {
+    const int key = v / VPR, e = (v - key * VPR) * 8;
+    if (key0 + key >= Lk || e >= D) continue;
+    const float *s0 = red + (size_t)key * LDR + e, *s1 = s0 + NKEY * LDR;
+    Pack8 ov, ok;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      ov.w[w] = pack2<T>(s0[2 * w], s0[2 * w + 1]);
+      ok.w[w] = pack2<T>(s1[2 * w] * a.softmax_scale, s1[2 * w + 1] * a.softmax_scale);
+    }
+    *reinterpret_cast<Pack8 *>(dvg + (int64_t)key * a.dv_row_stride + e) = ov;
+    *reinterpret_cast<Pack8 *>(dkg + (int64_t)key * a.dk_row_stride + e) = ok;
+  }
+}
 
 // a * b of two values below 2^24, b the same in every lane: one full-rate instruction (a 32-bit multiply takes four
 // times as long)
@@ -75,15 +458,17 @@ __device__ __forceinline__ uint32_t mul24_u32(uint32_t a, uint32_t b) {
 #endif
 }
 
-// DQP = true: dQ partials per visit (for the combine kernel); false: dS^T tiles to ws.ds (for the row-stationary dQ kernel).
+// dK / dV and dQ partials at head dimension 128 (the long calls).  Four waves of 512 registers, one per SIMD, all of which
+// compute: each keeps 32 keys x head_dim of dK^T and dV^T and its K and V operands in registers, and runs the softmax
+// arithmetic of one tile between the products of another.
 // KB = 1: the workgroup owns 64 keys, wave pair px takes tiles 2 px, 2 px + 1 of a round and wave kq of the pair the
 // key half kq.  KB = 2 (columns of a multiple of 128 keys, whose two 64-key blocks share one row list): it owns 128
 // keys, every wave takes all four tiles for its key quarter kq, so a gathered row serves twice the keys and a visit
 // leaves one dQ partial instead of two.
 // NEAR: the host has checked that a gathered row's place in q and dout is a 32-bit byte offset from the sequence's first
 // row that one 24-bit multiply makes (launch_dkdv); otherwise the loads take 64-bit addresses per lane.
-template <typename T, int HD, bool DQP, int KB, bool NEAR>
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
+template <typename T, int HD, int KB, bool NEAR>
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
   typedef BwdSmem<HD> SM;
   constexpr int KS = HD / 16, LDQ = SM::LDQ, LDS_ = SM::LDS_, NDT = HD / 32, VPR = HD / 8, LDR = SM::LDR;
   constexpr int NKEY = 64 * KB;         // keys of the workgroup
@@ -164,7 +549,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
   const int32_t *list = a.row_indices + lbase + start;
   const int n = nnz - start;               // rows of the list that the block walks
   const int nround = (n + kBwdRoundRows - 1) / kBwdRoundRows;
-  const int koff = key0 - c * Bn;  // offset of this 64-key block inside its column
   int rid01[2] = {-1, -1};         // threads 0..127: row ids of rounds 0 and 1
   if (tid < kBwdRoundRows && n > 0) {
 #pragma unroll
@@ -200,19 +584,17 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
       asm volatile("" : "+a"(kb[t]), "+a"(vb[t]));
 #endif
     }
-    if constexpr (DQP) {
-      lds_cu16 *trK = tr_lane_base(sK, LDQ, lane) + 8 * hh * LDQ;
+    lds_cu16 *trK = tr_lane_base(sK, LDQ, lane) + 8 * hh * LDQ;
 #pragma unroll
-      for (int s4 = 0; s4 < 4 * KB; ++s4)
+    for (int s4 = 0; s4 < 4 * KB; ++s4)
 #pragma unroll
-        for (int d2 = 0; d2 < NDH; ++d2) {
-          const int lo = 16 * s4 * LDQ + (kq * NDH + d2) * 32;
-          kt[d2][s4] = pack8_vec(tr_frag8_at(trK, lo, lo + 4 * LDQ));
+      for (int d2 = 0; d2 < NDH; ++d2) {
+        const int lo = 16 * s4 * LDQ + (kq * NDH + d2) * 32;
+        kt[d2][s4] = pack8_vec(tr_frag8_at(trK, lo, lo + 4 * LDQ));
 #if defined(__HIP_DEVICE_COMPILE__)
-          asm volatile("" : "+a"(kt[d2][s4]));
+        asm volatile("" : "+a"(kt[d2][s4]));
 #endif
-        }
-    }
+      }
   }
 
   const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride + (int64_t)h * a.q_head_stride;
@@ -260,9 +642,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
         m_lse = lseg[rc];
         m_del = delg[rc];
         // every visit of a (row, key block) pair takes one dQ-partial slot of the row
-        if constexpr (DQP) {
-          if (m_rid >= 0) m_slot = atomicAdd(cntg + (int64_t)m_rid * a.heads, 1);
-        }
+        if (m_rid >= 0) m_slot = atomicAdd(cntg + (int64_t)m_rid * a.heads, 1);
       }
     };
     const int64_t trash = (int64_t)a.total_q * a.heads * ws.cap;  // spare row: takes the writes of absent rows, no branch
@@ -273,7 +653,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
         sRow[i] = m_rid;
         // where the visit's dQ partial goes, as an index of partial rows (2^31 of them would be half a terabyte): the
         // row's slot, or the spare row for an absent row and for a visit beyond the caller's bound
-        if constexpr (DQP) sSlot[i] = (ok && m_slot < ws.cap) ? (int)((((int64_t)(q0 + m_rid)) * a.heads + h) * ws.cap + m_slot) : (int)trash;
+        sSlot[i] = (ok && m_slot < ws.cap) ? (int)((((int64_t)(q0 + m_rid)) * a.heads + h) * ws.cap + m_slot) : (int)trash;
         sLse[i] = ok ? m_lse * kLog2e : INFINITY;  // absent rows: exp2(x - inf) = 0
         sDelta[i] = ok ? m_del : 0.f;
       }
@@ -368,34 +748,9 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
     const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
     const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
     const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
-    // The operand addresses derived from them (an exclusive-or per piece) are formed once and stay in registers: the
-    // products leave room for them since their sums live in the accumulation registers.  (Made opaque, or the
-    // compiler forms them again at every read.)
-    // (The form with dQ partials has no registers to spare: there the bases are re-made opaque wherever they are used,
-    // so that nothing derived from them is kept from one use to the next.)
-    constexpr bool kKeepAddresses = !DQP;
+    // (no registers to spare for those: the bases are re-made opaque wherever they are used, so that nothing derived from
+    // them is kept from one use to the next)
     uint32_t aQ = pairQ + rowoff, adO = pairdO + rowoff, tQ = pairQ + troff, tdO = pairdO + troff;
-    uint32_t aQk[KS], adOk[KS];                              // row reads: piece hh * KS + k of this lane's row
-    uint32_t tQlo[NDT], tQhi[NDT], tdOlo[NDT], tdOhi[NDT];  // transposing reads: feature tile dt, rows (0..3) + 4 hh and the same + 8
-#pragma unroll
-    for (int k = 0; k < (kKeepAddresses ? KS : 0); ++k) {
-      aQk[k] = aQ ^ (uint32_t)(k * 16);
-      adOk[k] = adO ^ (uint32_t)(k * 16);
-#if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(aQk[k]), "+v"(adOk[k]));
-#endif
-    }
-#pragma unroll
-    for (int dt = 0; dt < (kKeepAddresses ? NDT : 0); ++dt) {
-      const uint32_t xlo = (uint32_t)(dt * 4 * 16), xhi = (uint32_t)(((dt * 4) ^ TileSwz<HD>::kRow8) * 16);
-      tQlo[dt] = tQ ^ xlo;
-      tQhi[dt] = tQ ^ xhi;
-      tdOlo[dt] = tdO ^ xlo;
-      tdOhi[dt] = tdO ^ xhi;
-#if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(tQlo[dt]), "+v"(tQhi[dt]), "+v"(tdOlo[dt]), "+v"(tdOhi[dt]));
-#endif
-    }
     auto opaque = [](uint32_t &x, uint32_t &y) {
 #if defined(__HIP_DEVICE_COMPILE__)
       asm volatile("" : "+v"(x), "+v"(y));
@@ -410,7 +765,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
       (void)x;
 #endif
     };
-    uint16_t *sdS = reinterpret_cast<uint16_t *>(smem + SM::odS) + (DQP ? (size_t)px * 2 * 64 * LDS_ : (size_t)wave * 32 * LDS_);  // (px = 0 with 128 keys)
+    uint16_t *sdS = reinterpret_cast<uint16_t *>(smem + SM::odS) + (size_t)px * 2 * 64 * LDS_;  // (px = 0 with 128 keys)
     lds_cu16 *trdS = tr_lane_base(sdS, LDS_, lane) + 8 * hh * LDS_;  // dS^T tile: 8 consecutive keys per read
     // the dQ part rows of a tile leave through the first tile of the pair, which nobody reads after the barrier in
     // the middle of the round: Q's for even waves, dO's for odd ones, one half of it each with four key quarters
@@ -429,16 +784,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
     auto ld_a = [&](auto pc, auto pp, auto tsc, auto gc) {
       constexpr uint32_t TO = (uint32_t)(decltype(pc)::value * 4 + decltype(pp)::value * 2 + decltype(tsc)::value) * TB;
       constexpr int G = decltype(gc)::value;
-      if constexpr (!kKeepAddresses) opaque(aQ, adO);
+      opaque(aQ, adO);
 #pragma unroll
       for (int t = 0; t < KC; ++t) {
-        if constexpr (kKeepAddresses) {
-          qa[G & 1][t] = lds_read16(aQk[G * KC + t] + TO);
-          doa[G & 1][t] = lds_read16(adOk[G * KC + t] + TO);
-        } else {
-          qa[G & 1][t] = lds_read16((aQ ^ (uint32_t)((G * KC + t) * 16)) + TO);
-          doa[G & 1][t] = lds_read16((adO ^ (uint32_t)((G * KC + t) * 16)) + TO);
-        }
+        qa[G & 1][t] = lds_read16((aQ ^ (uint32_t)((G * KC + t) * 16)) + TO);
+        doa[G & 1][t] = lds_read16((adO ^ (uint32_t)((G * KC + t) * 16)) + TO);
       }
     };
     // this lane's key; key j is visible to row r iff r >= row_thr (rows that do not exist are stored as -1)
@@ -482,20 +832,15 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
     auto ld_b = [&](auto pc, auto pp, auto tsc, auto gc) {
       constexpr uint32_t TO = (uint32_t)(decltype(pc)::value * 4 + decltype(pp)::value * 2 + decltype(tsc)::value) * TB;
       constexpr int G = decltype(gc)::value;
-      if constexpr (!kKeepAddresses) opaque(tQ, tdO);
+      opaque(tQ, tdO);
 #pragma unroll
       for (int t = 0; t < BC; ++t) {
         const int pi = G * BC + t, dt = pi >> 1, s2 = pi & 1;
         // rows 16 s2 + (0..3) + 4 hh and the same + 8, features dt * 32 ..
         const uint32_t olo = TO + (uint32_t)(16 * s2 * RB), ohi = olo + (uint32_t)(8 * RB);
-        if constexpr (kKeepAddresses) {
-          dot[G & 1][t] = lds_tr8(tdOlo[dt] + olo, tdOhi[dt] + ohi);
-          qt[G & 1][t] = lds_tr8(tQlo[dt] + olo, tQhi[dt] + ohi);
-        } else {
-          const uint32_t xlo = (uint32_t)(dt * 4 * 16), xhi = (uint32_t)(((dt * 4) ^ TileSwz<HD>::kRow8) * 16);
-          dot[G & 1][t] = lds_tr8((tdO ^ xlo) + olo, (tdO ^ xhi) + ohi);
-          qt[G & 1][t] = lds_tr8((tQ ^ xlo) + olo, (tQ ^ xhi) + ohi);
-        }
+        const uint32_t xlo = (uint32_t)(dt * 4 * 16), xhi = (uint32_t)(((dt * 4) ^ TileSwz<HD>::kRow8) * 16);
+        dot[G & 1][t] = lds_tr8((tdO ^ xlo) + olo, (tdO ^ xhi) + ohi);
+        qt[G & 1][t] = lds_tr8((tQ ^ xlo) + olo, (tQ ^ xhi) + ohi);
       }
     };
     auto mm_b = [&](auto tsc, auto gc) {
@@ -543,31 +888,12 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
     // half rows (16-bit, unscaled) go to the partial slot that the row handed out for this visit.
     auto ds_write = [&](auto tsc) {
       constexpr int TS = decltype(tsc)::value;
-      // partials form: tile slot TS of the pair, rows of all keys of the block; else: this wave's private tile
-      uint16_t *t = sdS + (size_t)((DQP ? TS * NKEY + kq * 32 : 0) + (lane & 31)) * LDS_;
+      // tile slot TS of the pair, rows of all keys of the block
+      uint16_t *t = sdS + (size_t)(TS * NKEY + kq * 32 + (lane & 31)) * LDS_;
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
         *reinterpret_cast<uint2 *>(t + 16 * s2 + 4 * hh) = make_uint2(dsf[TS][s2].w[0], dsf[TS][s2].w[1]);
         *reinterpret_cast<uint2 *>(t + 16 * s2 + 8 + 4 * hh) = make_uint2(dsf[TS][s2].w[2], dsf[TS][s2].w[3]);
-      }
-      if constexpr (!DQP) wave_lds_order();  // (the partials form waits for both key halves at a workgroup barrier later)
-    };
-    // dS form: the wave's 32 keys of every row go to the dS tile of the row's list entry
-    int dsrow = -1;
-    auto ds_read = [&](auto pc, auto pp, auto tsc) {
-      constexpr int TS = decltype(pc)::value * 4 + decltype(pp)::value * 2 + decltype(tsc)::value;
-      dsrow = pRow[TS * 32 + (lane & 31)];
-#pragma unroll
-      for (int s4 = 0; s4 < 2; ++s4) dsx[s4] = tr_frag8_at(trdS, 16 * s4 * LDS_, (16 * s4 + 4) * LDS_);
-      wave_lds_order();
-    };
-    auto ds_store = [&](int tile) {
-      if (dsrow >= 0) {
-        // key groups koff / 8 + 4 kq + 2 s4 + hh of list position p: consecutive lanes write consecutive 16-byte pieces
-        const int64_t p = lbase + start + tile * 32 + (lane & 31);
-        uint16_t *wp = ws.ds + ds_piece_offset(p, (koff >> 3) + 4 * kq + hh, Bn >> 3);
-#pragma unroll
-        for (int s4 = 0; s4 < 2; ++s4) *reinterpret_cast<Pack8 *>(wp + s4 * 512) = dsx[s4];
       }
     };
     auto dq_load = [&](auto tsc) {
@@ -635,7 +961,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
     // One round of a pair = its tiles 2 px and 2 px + 1, both already in LDS.  Tiles past the end of the list hold
     // absent rows (row id -1, zero data): they run through the same code and add nothing.
     auto process_round = [&](auto pc, auto pp, int r) {  // pc: parity of r = the LDS buffer that holds the round
-      const int tile0 = 4 * r + 2 * (KB == 1 ? px : decltype(pp)::value);  // position of the pair's first tile in the list
       // (the first row of the pair's first tile is its earliest; -1 if the pair has no row)
       const bool masked = __builtin_amdgcn_readfirstlane(pRow[(decltype(pc)::value * 4 + decltype(pp)::value * 2) * 32]) < all_visible_from;
       // S, dP of the first tile
@@ -672,9 +997,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
       });
       // dV, dK of the first tile between the softmax rows of the second
       // (a second pair of the same waves reuses the dS^T tiles of the first: its readers have to be done)
-      if constexpr (DQP && decltype(pp)::value == 1) __syncthreads();
+      if constexpr (decltype(pp)::value == 1) __syncthreads();
       ds_write(C0{});
-      if constexpr (!DQP) ds_read(pc, pp, C0{});
       fence();
       static_for<4>([&](auto gc) {
         constexpr int G = decltype(gc)::value;
@@ -686,45 +1010,38 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
         }
         mm_b(C0{}, gc);
         smx(C1{}, gc);
-        if constexpr (!DQP && G == 0) ds_store(tile0);
         fence();
       });
-      // dV, dK of the second tile; in the partials form dQ of the first one runs between them: by now all key
+      // dV, dK of the second tile; dQ of the first one runs between them: by now all key
       // groups have put dS^T of both tiles into LDS, so the one barrier the exchange needs hardly ever waits
       ds_write(C1{});
-      if constexpr (DQP) __syncthreads();
-      if constexpr (DQP)
-        dq_load(C0{});
-      else
-        ds_read(pc, pp, C1{});
+      __syncthreads();
+      dq_load(C0{});
       fence();
       static_for<4>([&](auto gc) {
         constexpr int G = decltype(gc)::value;
         if constexpr (G < 3) ld_b(pc, pp, C1{}, std::integral_constant<int, G + 1>{});
         mm_b(C1{}, gc);
-        if constexpr (DQP) dq_mma(gc);
-        if constexpr (!DQP && G == 0) ds_store(tile0 + 1);
+        dq_mma(gc);
         fence();
       });
-      if constexpr (DQP) {
-        dq_store(pc, pp, C0{});
-        // dQ of the second tile
-        dq_load(C1{});
+      dq_store(pc, pp, C0{});
+      // dQ of the second tile
+      dq_load(C1{});
+      fence();
+      static_for<4>([&](auto gc) {
+        dq_mma(gc);
         fence();
-        static_for<4>([&](auto gc) {
-          dq_mma(gc);
-          fence();
-        });
-        // The tiles of the next round must be in LDS before the barrier that ends this one, and one counter covers
-        // loads and stores alike: the round's last partial rows are issued after that wait, so that they complete
-        // under the next round instead of being waited for.
-        if constexpr (KB == 1 || decltype(pp)::value == 1) {
-          wait_all_loads();
-          meta_store(r + 1);
-          rid_store(r + 2);
-        }
-        dq_store(pc, pp, C1{});
+      });
+      // The tiles of the next round must be in LDS before the barrier that ends this one, and one counter covers
+      // loads and stores alike: the round's last partial rows are issued after that wait, so that they complete
+      // under the next round instead of being waited for.
+      if constexpr (KB == 1 || decltype(pp)::value == 1) {
+        wait_all_loads();
+        meta_store(r + 1);
+        rid_store(r + 2);
       }
+      dq_store(pc, pp, C1{});
     };
     auto round = [&](auto pc, int r) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -738,11 +1055,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
         tile_issue(r + 1);
       process_round(pc, C0{}, r);
       if constexpr (KB == 2) process_round(pc, C1{}, r);
-      if constexpr (!DQP) {
-        meta_store(r + 1);
-        rid_store(r + 2);
-        wait_all_loads();
-      }
       __syncthreads();  // round r + 1 is in LDS; everyone is done with round r
     };
     for (int r = 0; r < nround; r += 2) {
@@ -797,327 +1109,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args 
     for (int w = 0; w < 4; ++w) {
       ov.w[w] = pack2<T>(fv[2 * w], fv[2 * w + 1]);
       ok.w[w] = pack2<T>(fk[2 * w] * a.softmax_scale, fk[2 * w + 1] * a.softmax_scale);
-    }
-    *reinterpret_cast<Pack8 *>(dvg + (int64_t)key * a.dv_row_stride + e) = ov;
-    *reinterpret_cast<Pack8 *>(dkg + (int64_t)key * a.dk_row_stride + e) = ok;
-  }
-}
-
-// ------------------------------------------------------------------------------------
-// dK / dV, dS tiles form: TODO comment
-// ------------------------------------------------------------------------------------
-template <int HD, bool DQP>
-struct DkdvSmem {
-  static constexpr size_t tile = (size_t)64 * HD * 2;        // 64 gathered rows of Q or dO, swizzled (tile_swz)
-  static constexpr size_t oQ = 0;                             // [2 buffers]
-  static constexpr size_t odO = oQ + 2 * tile;                // [2 buffers]
-  static constexpr size_t oP = odO + 2 * tile;                // [64 rows][64 keys], piece p (8 keys) of row r at p ^ (r & 7)
-  static constexpr size_t odS = oP + 64 * 128;
-  static constexpr size_t oOut = odS + 64 * 128;              // partials form: [64 rows][HD], dQ part rows on their way out
-  static constexpr size_t oSlot = oOut + (DQP ? (size_t)64 * HD * 2 : 0);  // int[2][64]: places of the part rows
-  static constexpr size_t bytes_loop = oSlot + (DQP ? 2 * 64 * 4 : 0);
-  static constexpr int LDR = HD + 4;                          // floats, output staging [2][64 keys][LDR]
-  static constexpr size_t bytes = bytes_loop > (size_t)2 * 64 * LDR * 4 ? bytes_loop : (size_t)2 * 64 * LDR * 4;
-};
-
-template <typename T, int HD, bool DQP>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_rows_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
-  typedef DkdvSmem<HD, DQP> SM;
-  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, NDW = NDT / 2, LDR = SM::LDR;
-  constexpr float kLog2e = 1.4426950408889634f;
-  extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + 63) / 64, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
-  const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
-  const int key0 = nb * 64;
-  const int Bn = a.lg_block_n, c = key0 / Bn;
-  const int64_t bh = (int64_t)b * a.heads + h;
-  int nnz = 0;
-  int64_t lbase = 0;
-  if (c < a.max_cols) {
-    nnz = a.col_nnz[bh * a.max_cols + c];
-    lbase = a.col_offsets[bh * a.max_cols + c];
-  }
-  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
-  if (key0 >= Lk) return;
-  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
-  const int off = Lk - Lq;
-  const int D = a.head_dim;
-  const int hk = h / (a.heads / a.heads_k);
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
-  const int kq = wave & 1, rt = wave >> 1;  // S and dP: this wave's 32 keys and 32 rows
-  const int fw = wave & 1, sel = wave >> 1;      // sums: dV (sel = 0) or dK (1), all keys of the block, half of the features
-  const bool causal = a.is_causal != 0;
-  const float scale_log2 = a.softmax_scale * kLog2e;
-  const uint32_t lds = (uint32_t)(uintptr_t)smem, ldsQ = lds + (uint32_t)SM::oQ, ldsdO = lds + (uint32_t)SM::odO, ldsP = lds + (uint32_t)SM::oP, ldsdS = lds + (uint32_t)SM::odS;
-  constexpr uint32_t TILE = (uint32_t)SM::tile;
-  constexpr int RPI = 64 / VPR;      // tile rows per load instruction
-  constexpr int NI = 16 / RPI;       // load instructions per wave and operand: 16 rows
-
-  // K and V of the block pass through the tiles on their way to registers
-  {
-    const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
-    const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
-    const int rl = lane / VPR, pc = lane % VPR;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int key = (wave * NI + i) * RPI + rl;
-      const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
-      const int64_t kc = min(key, Lk - 1 - key0);
-      global_to_lds16(kg + kc * a.k_row_stride + e, ldsQ + (uint32_t)((wave * NI + i) * 1024));
-      global_to_lds16(vg + kc * a.v_row_stride + e, ldsdO + (uint32_t)((wave * NI + i) * 1024));
-    }
-  }
-  int start = 0;
-  if (causal && nnz > 0 && Bn > 64) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off);  // earlier rows see no key of the block
-  const int32_t *list = a.row_indices + lbase + start;
-  const int n = nnz - start;
-  const int nround = (n + 63) >> 6;
-  const int koff = key0 - c * Bn;
-
-  const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride + (int64_t)h * a.q_head_stride;
-  const uint16_t *dog = reinterpret_cast<const uint16_t *>(a.dout) + (int64_t)q0 * a.do_row_stride + (int64_t)h * a.do_head_stride;
-  const float *lseg = a.softmax_lse + (int64_t)h * a.total_q + q0;
-  const float *delg = a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b;
-
-  f32x16 acc[NDW][2];  // register i of tile [d][kk] <-> feature (fw * NDW + d) * 32 + acc_row(i, hh), key kk * 32 + lane % 32
-#pragma unroll
-  for (int d = 0; d < NDW; ++d)
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[d][kk][i] = 0.f;
-
-  // lane -> row rt * 32 + lane % 32 of a round
-  const int myrow = rt * 32 + (lane & 31);
-  int rid_nx = nround > 0 ? list[min(myrow, n - 1)] : 0;
-  auto code = [&](int raw, int r) { return tile_row_code(raw, r * 64 + myrow < n, Lq); };
-  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
-  const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
-  const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
-
-  wait_all_loads();
-  __syncthreads();
-  Pack8 kf[KS], vf[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    kf[ks] = lds_read16(((ldsQ + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
-    vf[ks] = lds_read16(((ldsdO + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
-    if (D < HD && (hh * KS + ks) * 8 >= D) kf[ks] = vf[ks] = zero_pack8();
-  }
-  // partials form: K^T of this wave's half of the features, the A operand of dQ^T = K^T dS^T (keys 16 s4 + 8 hh .. + 7)
-  Pack8 ktf[DQP ? NDW : 1][4];
-  if constexpr (DQP) {
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-      for (int d = 0; d < NDW; ++d) {
-        uint32_t ad[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int key = 16 * s4 + 8 * hh + 4 * u + (li >> 2);
-          ad[u] = ldsQ + (uint32_t)(key * RB + ((((kq * NDW + d) * 4 + ((lane >> 4) & 1) * 2 + ((li & 3) >> 1)) ^ tile_swz<HD>(key)) * 16) + (li & 1) * 8);
-        }
-        ktf[d][s4] = lds_tr8(ad[0], ad[1]);
-      }
-  }
-  __syncthreads();
-  if (nround > 0) {
-    // rows of round r + 1 (ids `rid`): Q and dO into the other buffer, 16 rows per wave
-    auto feed = [&](int rid, uint32_t buf) {
-      const int rl = lane / VPR, pc = lane % VPR;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int tr = kq * 16 + i * RPI + rl;  // row of the tile of 32
-        const uint32_t src = (uint32_t)__shfl(rid, tr, 64) & 0x7fffffffu;
-        const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
-        const uint32_t dst = buf + (uint32_t)((rt * 32 + kq * 16 + i * RPI) * RB);
-        global_to_lds16(qg + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
-        global_to_lds16(dog + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
-      }
-    };
-    int rid = code(rid_nx, 0);
-    feed(rid, 0);
-    float lse = lseg[rid & 0x7fffffff], del = delg[rid & 0x7fffffff];
-    // partials form: the waves of key half 0 hand out the part rows of their 32 rows, a round ahead (a spare row takes what
-    // absent rows and visits beyond the caller's bound write)
-    int slot = 0;
-    int *sSlot = reinterpret_cast<int *>(smem + SM::oSlot);
-    const int trash = a.total_q * a.heads * ws.cap;
-    auto take = [&](int rd, int r) {
-      if constexpr (DQP) slot = take_slot(ws.cnt + ((int64_t)(q0 + (rd & 0x7fffffff)) * a.heads + h), __ballot(rd >= 0 && hh == 0 && kq == 0 && r < nround));
-    };
-    take(rid, 0);
-    rid_nx = list[min(64 + myrow, n - 1)];
-    auto arrived = [&]() {
-      wait_all_loads();
-#if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(lse), "+v"(del), "+v"(rid_nx), "+v"(slot));
-#endif
-    };
-    arrived();
-    __syncthreads();
-    const uint32_t pw = (uint32_t)(myrow * 128 + hh * 8), psw = (uint32_t)(myrow & 7);
-    const uint32_t ptr_ = (uint32_t)(r0t * 128 + (((((lane >> 4) & 1) * 2 + ((li & 3) >> 1)) ^ (r0t & 7)) * 16) + (li & 1) * 8);
-    for (int r = 0; r < nround; ++r) {
-      const uint32_t buf = (r & 1) ? TILE : 0u;
-      const int rcur = rid;
-      const float lse2 = rcur >= 0 ? lse * kLog2e : INFINITY, delta = del;
-      if constexpr (DQP) {
-        if (kq == 0 && hh == 0) sSlot[(r & 1) * 64 + myrow] = (rcur >= 0 && slot < ws.cap) ? ((q0 + rcur) * a.heads + h) * ws.cap + slot : trash;
-      }
-      // the next round's rows
-      rid = code(rid_nx, r + 1);
-      if (r + 1 < nround) feed(rid, buf ^ TILE);
-      lse = lseg[rid & 0x7fffffff];
-      del = delg[rid & 0x7fffffff];
-      take(rid, r + 1);
-      rid_nx = list[min((r + 2) * 64 + myrow, n - 1)];
-      // S^T and dP^T: lane -> row, register i -> key kq * 32 + acc_row(i, hh)
-      f32x16 s, dp;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.f;
-      uint32_t aq = ldsQ + buf + (uint32_t)(rt * 32 * RB) + rowoff, ad = ldsdO + buf + (uint32_t)(rt * 32 * RB) + rowoff;
-      constexpr int NB = 2;  // k-steps per batch of reads
-      Pack8 qf[2][NB], df[2][NB];
-      auto rd = [&](auto bc) {
-        constexpr int B = decltype(bc)::value;
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          qf[B & 1][u] = lds_read16(aq ^ (uint32_t)((B * NB + u) * 16));
-          df[B & 1][u] = lds_read16(ad ^ (uint32_t)((B * NB + u) * 16));
-        }
-      };
-      rd(std::integral_constant<int, 0>{});
-      static_for<KS / NB>([&](auto bc) {
-        constexpr int B = decltype(bc)::value;
-        if constexpr (B + 1 < KS / NB) rd(std::integral_constant<int, B + 1>{});
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          s = mfma32<T>(kf[B * NB + u], qf[B & 1][u], s);
-          dp = mfma32<T>(vf[B * NB + u], df[B & 1][u], dp);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      });
-      const int lim = rcur < 0 ? -1 : min(causal ? rcur + off : 0x7fffffff, Lk - 1) - key0 - kq * 32;  // last visible key of this wave's 32
-      if (!__all(lim >= 31)) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = 8 * (i >> 2) + (i & 3) + 4 * hh <= lim ? s[i] : -INFINITY;
-      }
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        float p[4], d[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          p[j] = __builtin_amdgcn_exp2f(fmaf(s[4 * g + j], scale_log2, -lse2));
-          d[j] = p[j] * (dp[4 * g + j] - delta);
-        }
-        const uint32_t at = pw + (((uint32_t)(kq * 4 + g) ^ psw) * 16u);
-        lds_write_vec<uint2>(ldsP + at, make_uint2(pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3])));
-        lds_write_vec<uint2>(ldsdS + at, make_uint2(pack2<T>(d[0], d[1]), pack2<T>(d[2], d[3])));
-      }
-      __syncthreads();  // P and dS of the round are in LDS
-      // dV^T[f][key] += dO^T[f][row] P[row][key], dK^T[f][key] += Q^T[f][row] dS[row][key]
-      const uint32_t tx = (sel ? ldsQ : ldsdO) + buf + troff, px = (sel ? ldsdS : ldsP) + ptr_;
-      Pack8 pb[2][2], xa[2][NDW];
-      auto rd2 = [&](auto sc) {
-        constexpr int S4 = decltype(sc)::value;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const uint32_t po = (px ^ (uint32_t)(kk * 64)) + (uint32_t)(S4 * 16 * 128);
-          pb[S4 & 1][kk] = lds_tr8(po, po + 8 * 128);
-        }
-#pragma unroll
-        for (int d = 0; d < NDW; ++d) {
-          const uint32_t dt = (uint32_t)(fw * NDW + d), xlo = dt * 64u, xhi = ((dt * 4u) ^ (uint32_t)TileSwz<HD>::kRow8) * 16u;
-          const uint32_t olo = (uint32_t)(S4 * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
-          xa[S4 & 1][d] = lds_tr8((tx ^ xlo) + olo, (tx ^ xhi) + ohi);
-        }
-      };
-      rd2(std::integral_constant<int, 0>{});
-      static_for<4>([&](auto sc) {
-        constexpr int S4 = decltype(sc)::value;
-        if constexpr (S4 < 3) rd2(std::integral_constant<int, S4 + 1>{});
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int d = 0; d < NDW; ++d)
-#pragma unroll
-          for (int kk = 0; kk < 2; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
-        __builtin_amdgcn_sched_barrier(0);
-      });
-      if constexpr (DQP) {
-        // dQ^T[f][row] of this wave's 32 rows and its half (kq) of the features, over all keys of the block
-        f32x16 dq[NDW];
-        Pack8 sf[4];
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) sf[s4] = lds_read16(ldsdS + (uint32_t)(myrow * 128) + (((uint32_t)(2 * s4 + hh) ^ psw) * 16u));
-#pragma unroll
-        for (int d = 0; d < NDW; ++d) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) dq[d][i] = 0.f;
-#pragma unroll
-          for (int s4 = 0; s4 < 4; ++s4) dq[d] = mfma32<T>(ktf[d][s4], sf[s4], dq[d]);
-        }
-        // rows through LDS, so that a row's 16-byte pieces leave together (piece p of row r at p ^ (r & 7))
-        const uint32_t ldsOut = lds + (uint32_t)SM::oOut;
-#pragma unroll
-        for (int d = 0; d < NDW; ++d)
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            lds_write_vec<uint2>(ldsOut + (uint32_t)(myrow * RB + hh * 8) + (((uint32_t)((kq * NDW + d) * 4 + g) ^ psw) * 16u),
-                                 make_uint2(pack2<T>(dq[d][4 * g], dq[d][4 * g + 1]), pack2<T>(dq[d][4 * g + 2], dq[d][4 * g + 3])));
-        arrived();
-        __syncthreads();  // the part rows are there (and the next round's rows)
-#pragma unroll
-        for (int v = tid; v < 64 * VPR; v += 256) {
-          const int row = v / VPR, pcs = v - row * VPR;
-          const uint32_t p = (uint32_t)sSlot[(r & 1) * 64 + row];
-          const Pack8 x = lds_read16(ldsOut + (uint32_t)(row * RB) + (((uint32_t)pcs ^ (uint32_t)(row & 7)) * 16u));
-          if (pcs * 8 < D) st_stream16(ws.part + ((uint64_t)p * (uint32_t)D + (uint32_t)(pcs * 8)), x);
-          if (pcs == 0) ws.pid[p] = nb;
-        }
-      } else {
-        arrived();
-        // dS of row `lane`, key groups 2 wave and 2 wave + 1: consecutive lanes write consecutive pieces of the dS tile
-        const int p = r * 64 + lane;
-        Pack8 x[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) x[u] = lds_read16(ldsdS + (uint32_t)(lane * 128) + (((uint32_t)(2 * wave + u) ^ (uint32_t)(lane & 7)) * 16u));
-        if (p < n) {
-          const int64_t pos = lbase + start + p;
-#pragma unroll
-          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(ws.ds + ds_piece_offset(pos, (koff >> 3) + 2 * wave + u, Bn >> 3)) = x[u];
-        }
-      }
-      __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
-    }
-  }
-
-  // ---- dK^T / dV^T leave as rows, once ----
-  float *red = reinterpret_cast<float *>(smem);
-#pragma unroll
-  for (int d = 0; d < NDW; ++d)
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4 x4;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) x4[j] = acc[d][kk][4 * g + j];
-        *reinterpret_cast<f32x4 *>(red + (size_t)(sel * 64 + kk * 32 + (lane & 31)) * LDR + (fw * NDW + d) * 32 + 8 * g + 4 * hh) = x4;
-      }
-  __syncthreads();
-  uint16_t *dkg = reinterpret_cast<uint16_t *>(a.dk) + (int64_t)(k0 + key0) * a.dk_row_stride + (int64_t)h * a.dk_head_stride;
-  uint16_t *dvg = reinterpret_cast<uint16_t *>(a.dv) + (int64_t)(k0 + key0) * a.dv_row_stride + (int64_t)h * a.dv_head_stride;
-  for (int v = tid; v < 64 * VPR; v += 256) {
-    const int key = v / VPR, e = (v - key * VPR) * 8;
-    if (key0 + key >= Lk || e >= D) continue;
-    const float *s0 = red + (size_t)key * LDR + e, *s1 = s0 + 64 * LDR;
-    Pack8 ov, ok;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      ov.w[w] = pack2<T>(s0[2 * w], s0[2 * w + 1]);
-      ok.w[w] = pack2<T>(s1[2 * w] * a.softmax_scale, s1[2 * w + 1] * a.softmax_scale);
     }
     *reinterpret_cast<Pack8 *>(dvg + (int64_t)key * a.dv_row_stride + e) = ov;
     *reinterpret_cast<Pack8 *>(dkg + (int64_t)key * a.dk_row_stride + e) = ok;
@@ -1610,46 +1601,32 @@ __global__ void zero_f32_kernel(float *p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0.f;
 }
 
-template <typename T, int HD, bool DQP, int KB, bool NEAR>
-static int launch_dkdv_form(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
-  auto kern = attn_bwd_dkdv_kernel<T, HD, DQP, KB, NEAR>;
-  const size_t smem = BwdSmem<HD>::bytes;
+template <typename K>
+static int launch_dkdv_kernel(K kern, size_t smem, int heads, int keys, const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_k, 64 * KB);
+  const int64_t items = (int64_t)a.batch * heads * ceil_div(a.max_seqlen_k, keys);
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_bwd: too many (sequence, head, key block) work items");
     return 1;
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws);
   return 0;
+}
+template <typename T, int HD, bool DQP>
+static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
+  return launch_dkdv_kernel(attn_bwd_dkdv_kernel<T, HD, DQP>, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
 }
 // NEAR: every row of a sequence's q and dout lies within 2 GB of the sequence's first row and is less than 2^24 rows
 // and 2^22 elements per row away, so a gathered row's place is a 32-bit offset made by one 24-bit multiply.
-template <typename T, int HD, bool DQP, int KB>
-static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
+template <typename T, int HD, int KB>
+static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   const bool near_rows = a.max_seqlen_q < (1 << 24) && a.q_row_stride < (1 << 22) && a.do_row_stride < (1 << 22) &&
                          (int64_t)a.max_seqlen_q * a.q_row_stride < (int64_t)0x7fff0000 && (int64_t)a.max_seqlen_q * a.do_row_stride < (int64_t)0x7fff0000;
-  return near_rows ? launch_dkdv_form<T, HD, DQP, KB, true>(a, ws, s) : launch_dkdv_form<T, HD, DQP, KB, false>(a, ws, s);
-}
-
-template <typename T, int HD, bool DQP>
-static int launch_dkdv_rows(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
-  auto kern = attn_bwd_dkdv_rows_kernel<T, HD, DQP>;
-  const size_t smem = DkdvSmem<HD, DQP>::bytes;
-  if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
-    set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
-    return 2;
-  }
-  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_k, 64);
-  if (items >= ((int64_t)1 << 31)) {
-    set_error("attn_bwd: too many (sequence, head, key block) work items");
-    return 1;
-  }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws);
-  return 0;
+  return near_rows ? launch_dkdv_kernel(attn_bwd_dkdv_partials_kernel<T, HD, KB, true>, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s)
+                   : launch_dkdv_kernel(attn_bwd_dkdv_partials_kernel<T, HD, KB, false>, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s);
 }
 
 template <typename T, int HD, int RT>
@@ -1690,6 +1667,19 @@ static int bwd_dq_partials(const fmoba_attn_bwd_args &a) {
   const double seen = a.is_causal ? 0.5 * chunks_per_seq : chunks_per_seq;
   return chunks_per_row < (bwd_wide_blocks(a) ? 0.37 : 0.10) * seen;
 }
+// Heads of dK / dV the call is best made with: heads / this many query heads are added up by one workgroup, in fp32, instead
+// of in memory afterwards (24571 tokens, 32 over 8 heads: 1225 us and two sums of 48 us -> 1118 us).  All heads of a group, unless that
+// leaves fewer than two rounds of workgroups for the chip's 512 (two per unit).  The long calls (partials at head dimension
+// 128) have a kernel that takes one head at a time.
+static bool bwd_sums_heads(const fmoba_attn_bwd_args &a) { return a.head_dim <= 64 || (a.head_dim <= 128 && !bwd_dq_partials(a)); }
+static int bwd_dkv_heads(const fmoba_attn_bwd_args &a) {
+  if (!bwd_sums_heads(a)) return a.heads;
+  const int grp = a.heads / a.heads_k;
+  const int64_t blocks = a.total_k / 64 + a.batch;
+  for (int gs = grp < 64 ? grp : 64; gs > 1; --gs)
+    if (grp % gs == 0 && blocks * (a.heads / gs) >= 1024) return a.heads / gs;
+  return a.heads;
+}
 // partial slots per (row, head): max_visits_per_row counts 64-key blocks; with 128-key blocks a row has half as many
 // visits (only the last column of a sequence can have an odd number of 64-key blocks)
 static inline int32_t bwd_partial_cap(const fmoba_attn_bwd_args &a) {
@@ -1716,13 +1706,11 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
   }
   if (phases & FMOBA_BWD_DKDV) {
     int rc;
-    // columns of a multiple of 128 keys: one workgroup per 128 keys (the two 64-key blocks share their row list)
-    const bool wide = bwd_wide_blocks(a);
     if (partials) {
       hipLaunchKernelGGL(zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, (int64_t)a.total_q * a.heads);
-      rc = a.head_dim <= 64 ? launch_dkdv_rows<T, 64, true>(a, ws, s) : (wide ? launch_dkdv<T, 128, true, 2>(a, ws, s) : launch_dkdv<T, 128, true, 1>(a, ws, s));
+      rc = a.head_dim <= 64 ? launch_dkdv<T, 64, true>(a, ws, s) : (bwd_wide_blocks(a) ? launch_dkdv_partials<T, 128, 2>(a, ws, s) : launch_dkdv_partials<T, 128, 1>(a, ws, s));
     } else {
-      rc = a.head_dim <= 64 ? launch_dkdv_rows<T, 64, false>(a, ws, s) : launch_dkdv_rows<T, 128, false>(a, ws, s);
+      rc = a.head_dim <= 64 ? launch_dkdv<T, 64, false>(a, ws, s) : launch_dkdv<T, 128, false>(a, ws, s);
     }
     if (rc) return rc;
   }
@@ -1754,6 +1742,12 @@ extern "C" int32_t fmoba_attn_bwd_uses_partials(const fmoba_attn_bwd_args *a) {
   return fmoba::bwd_dq_partials(*a);
 }
 
+extern "C" int32_t fmoba_attn_bwd_dkv_heads(const fmoba_attn_bwd_args *a) {
+  if (a == nullptr) return 0;
+  if (a->heads_k <= 0 || a->heads % a->heads_k != 0 || a->batch <= 0 || a->lg_block_n <= 0) return a->heads;
+  return fmoba::bwd_dkv_heads(*a);
+}
+
 extern "C" size_t fmoba_attn_bwd_workspace_bytes(const fmoba_attn_bwd_args *a) {
   using namespace fmoba;
   if (a == nullptr || a->total_q <= 0 || a->heads <= 0 || a->head_dim <= 0 || a->batch <= 0 || a->lg_block_n <= 0) return 256;
@@ -1765,7 +1759,9 @@ extern "C" size_t fmoba_attn_bwd_workspace_bytes(const fmoba_attn_bwd_args *a) {
 
 extern "C" int fmoba_attn_bwd(const fmoba_attn_bwd_args *a, void *stream) { return fmoba_attn_bwd_phases(a, 7, stream); }
 
-extern "C" int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phases, void *stream) {
+extern "C" int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phases, void *stream) { return fmoba_attn_bwd_grouped(a, a ? a->heads : 0, phases, stream); }
+
+extern "C" int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_heads, int32_t phases, void *stream) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "attn_bwd: null args");
   FMOBA_REQUIRE(phases > 0 && phases <= 7, "attn_bwd: phases must be a mask of bits 1, 2, 4");
@@ -1774,6 +1770,9 @@ extern "C" int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phase
   FMOBA_REQUIRE(a->head_dim > 0 && a->head_dim % 8 == 0, "head_size should be a multiple of 8");
   FMOBA_REQUIRE(a->head_dim <= 256, "FlashMoBA backward only supports head dimension at most 256");
   FMOBA_REQUIRE(a->heads > 0 && a->heads_k > 0 && a->heads % a->heads_k == 0, "Number of heads in key/value must divide number of heads in query");
+  FMOBA_REQUIRE(dkv_heads == a->heads || (dkv_heads > 0 && dkv_heads % a->heads_k == 0 && a->heads % dkv_heads == 0 && a->heads / dkv_heads <= 64 && a->lg_block_n > 0 &&
+                                          bwd_sums_heads(*a)),
+                "attn_bwd: dkv_heads must be heads, or a multiple of heads_k that divides heads, at most 64 query heads each (not above head dimension 128, nor above 64 with dQ partials)");
   FMOBA_REQUIRE(a->lg_block_m % 64 == 0, "m_lg_block_dim must be a multiple of 64");
   FMOBA_REQUIRE(a->lg_block_n > 0 && a->lg_block_n % 64 == 0, "n_lg_block_dim must be a multiple of 64");
   FMOBA_REQUIRE(a->lg_block_n <= 64 * 256, "attn_bwd: n_lg_block_dim above 16384 is not supported");
@@ -1795,8 +1794,8 @@ extern "C" int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phase
     FMOBA_REQUIRE(a->dk && a->dv, "attn_bwd: null dk/dv");
     if (a->max_seqlen_q == 0 || a->total_q == 0 || a->max_cols == 0) {
       // no query rows: dk = dv = 0 (csrc/flash_moba/flash_moba_api.cpp:834-839)
-      hipLaunchKernelGGL(zero_rows_kernel, dim3(1024), dim3(256), 0, s, a->dk, (int64_t)a->total_k, a->dk_row_stride, a->heads, a->dk_head_stride, a->head_dim);
-      hipLaunchKernelGGL(zero_rows_kernel, dim3(1024), dim3(256), 0, s, a->dv, (int64_t)a->total_k, a->dv_row_stride, a->heads, a->dv_head_stride, a->head_dim);
+      hipLaunchKernelGGL(zero_rows_kernel, dim3(1024), dim3(256), 0, s, a->dk, (int64_t)a->total_k, a->dk_row_stride, dkv_heads, a->dk_head_stride, a->head_dim);
+      hipLaunchKernelGGL(zero_rows_kernel, dim3(1024), dim3(256), 0, s, a->dv, (int64_t)a->total_k, a->dv_row_stride, dkv_heads, a->dv_head_stride, a->head_dim);
     }
   }
   if (a->total_q == 0 || a->max_seqlen_q == 0) {
@@ -1821,6 +1820,7 @@ extern "C" int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phase
   const size_t rows = (size_t)a->total_q * a->heads;
   uintptr_t wp = ((uintptr_t)a->workspace + 255) & ~(uintptr_t)255;
   BwdWs ws;
+  ws.dkv_heads = dkv_heads;
   ws.cap = bwd_partial_cap(*a);
   // (the dK/dV pass keeps the place of a visit's dQ partial as a 32-bit index of partial rows)
   FMOBA_REQUIRE(!fmoba::bwd_dq_partials(*a) || rows * (size_t)ws.cap + 1 < ((size_t)1 << 31),

@@ -205,18 +205,20 @@ struct Attention : public torch::autograd::Function<Attention> {
       TORCH_CHECK(dout.defined(), "flash_moba: no gradient");
       if (!is_rows(dout, q.scalar_type(), q.device())) dout = dout.to(q.scalar_type()).contiguous();
       Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-      const bool grouped = s.heads != s.heads_k;  // per-query-head gradients of keys and values, summed below (flash_moba_api.cpp:842-845)
-      const Tensor dk_e = grouped ? at::empty({s.total_k, s.heads, s.dim}, k.options()) : dk, dv_e = grouped ? at::empty({s.total_k, s.heads, s.dim}, v.options()) : dv;
-      const Tensor softmax_d = at::empty({s.heads, s.total_q + 128 * s.batch}, q.options().dtype(at::kFloat));
       fmoba_attn_bwd_args a{};
-      a.dout = dout.data_ptr(), a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr(), a.out = out.data_ptr(), a.softmax_lse = lse.data_ptr<float>();
-      a.dq = dq.data_ptr(), a.dk = dk_e.data_ptr(), a.dv = dv_e.data_ptr(), a.softmax_d = softmax_d.data_ptr<float>();
-      a.col_offsets = co.data_ptr<int64_t>(), a.col_nnz = cn.data_ptr<int32_t>(), a.row_indices = ind.data_ptr<int32_t>(), a.num_row_indices = ind.numel();
-      a.cu_seqlens_q = cu_q.data_ptr<int32_t>(), a.cu_seqlens_k = cu_k.data_ptr<int32_t>();
       a.batch = s.batch, a.total_q = s.total_q, a.total_k = s.total_k, a.heads = s.heads, a.heads_k = s.heads_k, a.head_dim = s.dim;
       a.max_seqlen_q = s.max_q, a.max_seqlen_k = s.max_k, a.max_cols = co.size(2), a.lg_block_m = 128, a.lg_block_n = s.chunk;
       a.is_causal = s.causal && s.max_q != 1, a.dtype = s.dtype, a.deterministic = ctx->saved_data["deterministic"].toBool();
       a.max_visits_per_row = num("visits"), a.dq_mode = num("dq_mode"), a.softmax_scale = static_cast<float>(ctx->saved_data["scale"].toDouble());
+      // heads of a group that the library does not add up itself are summed below (flash_moba_api.cpp:842-845)
+      const int32_t dkv_heads = fmoba_attn_bwd_dkv_heads(&a);
+      const bool grouped = dkv_heads != s.heads_k;
+      const Tensor dk_e = grouped ? at::empty({s.total_k, dkv_heads, s.dim}, k.options()) : dk, dv_e = grouped ? at::empty({s.total_k, dkv_heads, s.dim}, v.options()) : dv;
+      const Tensor softmax_d = at::empty({s.heads, s.total_q + 128 * s.batch}, q.options().dtype(at::kFloat));
+      a.dout = dout.data_ptr(), a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr(), a.out = out.data_ptr(), a.softmax_lse = lse.data_ptr<float>();
+      a.dq = dq.data_ptr(), a.dk = dk_e.data_ptr(), a.dv = dv_e.data_ptr(), a.softmax_d = softmax_d.data_ptr<float>();
+      a.col_offsets = co.data_ptr<int64_t>(), a.col_nnz = cn.data_ptr<int32_t>(), a.row_indices = ind.data_ptr<int32_t>(), a.num_row_indices = ind.numel();
+      a.cu_seqlens_q = cu_q.data_ptr<int32_t>(), a.cu_seqlens_k = cu_k.data_ptr<int32_t>();
       a.q_row_stride = q.stride(0), a.q_head_stride = q.stride(1), a.k_row_stride = k.stride(0), a.k_head_stride = k.stride(1);
       a.v_row_stride = v.stride(0), a.v_head_stride = v.stride(1), a.o_row_stride = out.stride(0), a.o_head_stride = out.stride(1);
       a.do_row_stride = dout.stride(0), a.do_head_stride = dout.stride(1), a.dq_row_stride = dq.stride(0), a.dq_head_stride = dq.stride(1);
@@ -224,10 +226,10 @@ struct Attention : public torch::autograd::Function<Attention> {
       const size_t n = fmoba_attn_bwd_workspace_bytes(&a);
       const Tensor ws = bytes_like(q, n);
       a.workspace = ws.data_ptr(), a.workspace_bytes = n;
-      check(fmoba_attn_bwd(&a, s.stream));
+      check(fmoba_attn_bwd_grouped(&a, dkv_heads, 7, s.stream));
       if (grouped) {
-        at::sum_out(dk, dk_e.view({s.total_k, s.heads_k, s.heads / s.heads_k, s.dim}), at::IntArrayRef{2});
-        at::sum_out(dv, dv_e.view({s.total_k, s.heads_k, s.heads / s.heads_k, s.dim}), at::IntArrayRef{2});
+        at::sum_out(dk, dk_e.view({s.total_k, s.heads_k, dkv_heads / s.heads_k, s.dim}), at::IntArrayRef{2});
+        at::sum_out(dv, dv_e.view({s.total_k, s.heads_k, dkv_heads / s.heads_k, s.dim}), at::IntArrayRef{2});
       }
       res[0] = dq, res[1] = dk, res[2] = dv;
     }

@@ -101,6 +101,8 @@ EXPORTS = {
     "fmoba_csc_max_row_visits": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp, c_vp, c_vp]),
     "fmoba_attn_fwd": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp]),
     "fmoba_attn_fwd_phases": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_i32, c_vp]),
+    "fmoba_attn_bwd_grouped": (c_i32, [ctypes.POINTER(AttnBwdArgs), c_i32, c_i32, c_vp]),
+    "fmoba_attn_bwd_dkv_heads": (c_i32, [ctypes.POINTER(AttnBwdArgs)]),
     "fmoba_attn_bwd_workspace_bytes": (c_sz, [ctypes.POINTER(AttnBwdArgs)]),
     "fmoba_attn_bwd_uses_partials": (c_i32, [ctypes.POINTER(AttnBwdArgs)]),
     "fmoba_attn_bwd": (c_i32, [ctypes.POINTER(AttnBwdArgs), c_vp]),
@@ -549,11 +551,6 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
         dv = _grad(dv_, v, "dv", (total_k, heads_k, d))
         dev = q.device
         softmax_d = torch.empty((heads, total_q + 128 * batch), dtype=torch.float32, device=dev)
-        if heads_k != heads:  # MQA / GQA: per-query-head gradients, summed below (flash_moba_api.cpp:764-771,842-845)
-            dk_e = torch.empty((total_k, heads, d), dtype=dtype, device=dev)
-            dv_e = torch.empty((total_k, heads, d), dtype=dtype, device=dev)
-        else:
-            dk_e, dv_e = dk, dv
         lib = load_library()
         visits = _max_visits
         if visits is None or int(visits) < 1:
@@ -563,7 +560,7 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
                                                 max_seqlen_k, max_cols, 128, n_lg_block_dim)
         visits = max(1, int(visits))
         a = AttnBwdArgs(dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), softmax_lse.data_ptr(),
-                        dq.data_ptr(), dk_e.data_ptr(), dv_e.data_ptr(), softmax_d.data_ptr(),
+                        dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), softmax_d.data_ptr(),
                         moba_col_offsets.data_ptr(), moba_col_nnz.data_ptr(), moba_row_indices.data_ptr(),
                         cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), None, 0, int(moba_row_indices.numel()),
                         batch, total_q, total_k, heads, heads_k, d, int(max_seqlen_q), int(max_seqlen_k), max_cols,
@@ -571,17 +568,25 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
                         visits, int(_dq_mode), float(softmax_scale),
                         q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
                         out.stride(0), out.stride(1), dout.stride(0), dout.stride(1),
-                        dq.stride(0), dq.stride(1), dk_e.stride(0), dk_e.stride(1), dv_e.stride(0), dv_e.stride(1), _ptr(_overflow))
+                        dq.stride(0), dq.stride(1), dk.stride(0), dk.stride(1), dv.stride(0), dv.stride(1), _ptr(_overflow))
+        # MQA / GQA: the library adds up the query heads of a group, or as many of them as leave it enough to do side by
+        # side; the rest is summed below (flash_moba_api.cpp:764-771,842-845)
+        dkv_heads = lib.fmoba_attn_bwd_dkv_heads(ctypes.byref(a)) if heads_k != heads else heads
+        if dkv_heads != heads_k:
+            dk_e = torch.empty((total_k, dkv_heads, d), dtype=dtype, device=dev)
+            dv_e = torch.empty((total_k, dkv_heads, d), dtype=dtype, device=dev)
+            a.dk, a.dk_row_stride, a.dk_head_stride = dk_e.data_ptr(), dk_e.stride(0), dk_e.stride(1)
+            a.dv, a.dv_row_stride, a.dv_head_stride = dv_e.data_ptr(), dv_e.stride(0), dv_e.stride(1)
         ws_bytes = lib.fmoba_attn_bwd_workspace_bytes(ctypes.byref(a))
         _last.bwd_partials = int(lib.fmoba_attn_bwd_uses_partials(ctypes.byref(a)))
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes
         if _phases is None:
-            _check(lib.fmoba_attn_bwd(ctypes.byref(a), _stream()))
+            _check(lib.fmoba_attn_bwd_grouped(ctypes.byref(a), dkv_heads, 7, _stream()))
         else:  # measurement hook: callable(run) receives run(mask) launching the chosen phases
-            _phases(lambda mask: _check(lib.fmoba_attn_bwd_phases(ctypes.byref(a), mask, _stream())))
-        if heads_k != heads:
-            grp = heads // heads_k
+            _phases(lambda mask: _check(lib.fmoba_attn_bwd_grouped(ctypes.byref(a), dkv_heads, mask, _stream())))
+        if dkv_heads != heads_k:
+            grp = dkv_heads // heads_k
             torch.sum(dk_e.view(total_k, heads_k, grp, d), dim=2, out=dk)
             torch.sum(dv_e.view(total_k, heads_k, grp, d), dim=2, out=dv)
     return [dq, dk, dv, softmax_d]

@@ -198,7 +198,8 @@ int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phases, void *st
  * Sparse attention backward.
  * Replaces moba_varlen_bwd (csrc/flash_moba/flash_moba_api.cpp:610-848).
  *   dq (total_q, heads, d), dk/dv (total_k, heads, d) -- dk/dv are PER QUERY HEAD; for
- *   GQA/MQA the caller sums groups of heads/heads_k (flash_moba_api.cpp:842-845).
+ *   GQA/MQA the caller sums groups of heads/heads_k (flash_moba_api.cpp:842-845), or has
+ *   fmoba_attn_bwd_grouped sum them.
  *   softmax_d (heads, total_q + 128*batch) fp32: row (b, r) of head h is stored at
  *   h*(total_q + 128*batch) + cu_q[b] + 128*b + r (flash_bwd_preprocess_kernel.h:86).
  *   dK/dV come from one column-stationary pass.  dQ has two forms (dq_mode: 0 = the library
@@ -256,6 +257,11 @@ int fmoba_attn_bwd(const fmoba_attn_bwd_args *a, void *stream);
 #define FMOBA_BWD_DKDV 2
 #define FMOBA_BWD_DQ 4
 int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phases, void *stream);
+/* The same with dk/dv (total_k, dkv_heads, d), each head the sum over heads / dkv_heads consecutive query heads, formed in
+ * fp32; dkv_heads is a multiple of heads_k.  fmoba_attn_bwd_dkv_heads says how many are best (and possible) for a call; the
+ * caller sums what is left of a group. */
+int32_t fmoba_attn_bwd_dkv_heads(const fmoba_attn_bwd_args *a);
+int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_heads, int32_t phases, void *stream);
 
 #ifdef __cplusplus
 }
