@@ -37,17 +37,19 @@ def test_groups_add_up(lens_q, lens_k, chunk, topk, causal, H, Hk, counts, D, dq
                                          False, causal, 0.0, False, 128, chunk, None)
     lib = hip.load_library()
 
-    def grads(heads):
+    def grads(heads, k, v):
         monkeypatch.setattr(hip, "load_library", lambda: _Library(lib, heads))
-        return hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, co, cn, ind, cuq, cuk, mq, mk_, 0.0, D ** -0.5,
+        return hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, co, cn, ind, cuq, cuk, None, mq, mk_, 0.0, D ** -0.5,
                                    False, causal, 0.0, False, 128, chunk, _dq_mode=dq_mode)[:3]
 
-    dq, dk, dv = grads(H)
+    dq, dk, dv = grads(H, k.repeat_interleave(H // Hk, 1), v.repeat_interleave(H // Hk, 1))  # a head of keys per query head
+    dk, dv = (t.float().view(-1, Hk, H // Hk, D) for t in (dk, dv))
     for n in counts:
-        dq2, dk2, dv2 = grads(n)
+        dq2, dk2, dv2 = grads(n, k, v)
         if dq_mode == 1:
             assert torch.equal(dq, dq2)
-        else:  # the visits of a row are ordered before they are added
+        else:  # which visit got which slot does not matter: a row's visits are ordered before they are added
             assert_close("dq", dq2, dq.float().cpu(), 2e-2, 1e-2)
-        assert_close("dk", dk2, dk.float().cpu(), 6e-2, 2e-2)  # (the reference adds rows that were rounded to 16 bits)
-        assert_close("dv", dv2, dv.float().cpu(), 6e-2, 2e-2)
+        for name, got, ref in (("dk", dk2, dk), ("dv", dv2, dv)):  # (every term of the sum was rounded to 16 bits, and so are partial sums)
+            worst = (got.float() - ref.sum(2)).abs() - 2.0 ** -7 * ref.abs().sum(2)
+            assert worst.max().item() < 1e-3, f"{name}: {worst.max().item()}"
