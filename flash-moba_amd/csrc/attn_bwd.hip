@@ -1116,11 +1116,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
 }
 
 // ------------------------------------------------------------------------------------
-// dQ, first form: row blocks.  One workgroup owns 256 or 512 consecutive query rows of one (sequence, head) and
+// dQ, first form: row blocks.  One workgroup owns 256 consecutive query rows of one (sequence, head) and
 // walks the 64-key blocks of every column in which one of its rows appears.  The dS rows of a step (written by the
 // dK/dV pass in list order) go from global memory straight into the registers of the lane that owns the query row;
 // rows that are absent contribute zeros, so every wave multiplies its own 32-row tiles and keeps dQ in registers
-// for the whole walk.  All eight waves compute, two per SIMD, and nothing in the workgroup only moves data.  What a
+// for the whole walk.  All waves compute, two per SIMD (four at head dimensions up to 64), and nothing only moves data.  What a
 // step needs from other threads -- its K tile (global memory straight into LDS, global_load_lds, every wave a share
 // of the tile, swizzled rows of exactly head_dim elements) and the list positions of its rows (scattered into LDS by
 // the thread whose index is the row's place in the step's run) -- is prepared for a whole group of G steps at once,
@@ -1128,18 +1128,25 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
 // pace, and a wave's chain of dependent steps (where are my rows in this column's list -> fetch them -> multiply)
 // is covered by the products of the other wave of its SIMD.
 // ------------------------------------------------------------------------------------
-constexpr int kDqWaves = 8;
 constexpr int kDqColBatch = 256;
+//
+// What bounds it: the misses a unit can have in flight (dS pieces of 64 to 512 bytes at scattered places), and in calls of few
+// workgroups the longest walk.  Head dimensions 65 to 128: four waves with two row tiles each, two workgroups per unit and
+// groups of two steps; one workgroup of eight such waves per unit (groups of four steps, 512 rows) read half of the K tiles
+// but met at one barrier and left no unit a second walk: 65536 tokens in eight sequences, top-k 32 of 64-key chunks
+// 1634 -> 1556 us, 24571 tokens, 32 over 8 heads 691 -> 624, 12037 tokens, heads of 96 182 -> 124 (with the order of the items
+// below), 2 x 4096 tokens 143 -> 125.  Up to 64: eight waves of one tile (with two tiles in four waves 4096 tokens 58 -> 67 us).
+// Above 128: eight waves of one tile, one workgroup per unit (its K tiles take 128 KB).
 constexpr int kDqMaxSteps = 512;
 
-template <int HD, int RT>
+template <int HD, int RT, int NW>
 struct DqSmem {
-  static constexpr int ROWS = kDqWaves * 32 * RT;
-  static constexpr int G = HD == 128 ? 4 : 2;  // steps per group (one workgroup barrier per group)
+  static constexpr int ROWS = NW * 32 * RT;
+  static constexpr int G = 2;  // steps per group (one workgroup barrier per group)
   static constexpr int NS = 2 * G;              // K tiles / position slots in LDS: the group in use and the next one
   static constexpr int LDO = HD + 8;   // elements, per-wave output tile [32 rows][LDO] (reuses the K tiles at the end)
   static constexpr size_t tileBytes = (size_t)64 * HD * 2;
-  static constexpr size_t outBytes = (size_t)kDqWaves * 32 * LDO * 2;
+  static constexpr size_t outBytes = (size_t)NW * 32 * LDO * 2;
   static constexpr size_t prepBytes = (size_t)kDqColBatch * 16 + (size_t)kDqMaxSteps * 4;
   static constexpr size_t oK = 0;                                   // [NS][64 keys][HD], swizzled; later the output tiles
   static constexpr size_t ringBytes = NS * tileBytes > outBytes ? NS * tileBytes : outBytes;
@@ -1175,17 +1182,17 @@ __device__ __forceinline__ void wait_loads_but() {  // until at most N of the wa
 #endif
 }
 
-// RT: 32-row tiles per wave.  With two, a workgroup owns 512 rows and every K^T operand read from LDS feeds two MFMAs.
-template <typename T, int HD, int RT>
-__global__ __launch_bounds__(512, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, int nsb_max) {
-  typedef DqSmem<HD, RT> SM;
+// RT: 32-row tiles per wave (with two, every K^T operand read from LDS feeds two MFMAs).  NW: waves.
+template <typename T, int HD, int RT, int NW>
+__global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, int nsb_max) {
+  typedef DqSmem<HD, RT, NW> SM;
   constexpr int ROWS = SM::ROWS;  // query rows of the workgroup
   constexpr int LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
   constexpr int RB = HD * 2;                       // bytes of a K tile row
   constexpr uint32_t TB = (uint32_t)SM::tileBytes;
   constexpr int RPI = 64 / VPR;                    // K rows per load instruction
-  constexpr int NKI = 64 / RPI / kDqWaves;         // K load instructions per wave and tile
-  static_assert(NKI >= 1 && NKI * RPI * kDqWaves == 64, "the waves share a K tile evenly");
+  constexpr int NKI = 64 / RPI / NW;         // K load instructions per wave and tile
+  static_assert(NKI >= 1 && NKI * RPI * NW == 64, "the waves share a K tile evenly");
   constexpr int NS = SM::NS, G = SM::G;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   int *sPos = reinterpret_cast<int *>(smem + SM::oTag);
@@ -1213,7 +1220,7 @@ __global__ __launch_bounds__(512, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool causal = a.is_causal != 0;
 
-  for (int v = tid; v < NS * ROWS; v += 512) sPos[v] = 0;  // step tags start at 1
+  for (int v = tid; v < NS * ROWS; v += 64 * NW) sPos[v] = 0;  // step tags start at 1
 
   int ncols = min((Lk + Bn - 1) / Bn, a.max_cols);
   const int last_rowpos = m0 + rows_sb - 1 + off;
@@ -1228,7 +1235,7 @@ __global__ __launch_bounds__(512, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq
   // no tile is in use or on its way when the workgroup comes here.
   auto prepare_batch = [&](int cb, int cend) {
     __syncthreads();
-    for (int c = cb + tid; c < cend; c += 512) {
+    for (int c = cb + tid; c < cend; c += 64 * NW) {
       const int nnz = a.col_nnz[bh * a.max_cols + c];
       int lo = 0, cnt = 0;
       int64_t base = 0;
@@ -1263,11 +1270,11 @@ __global__ __launch_bounds__(512, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq
     __syncthreads();
     const int nsteps = __builtin_amdgcn_readfirstlane(sMisc[0]);
     // one record per step
-    for (int st = tid; st < nsteps; st += 512) {
+    for (int st = tid; st < nsteps; st += 64 * NW) {
       const int code = sStep[st];
       const int cl = code >> 8, kb = code & 255;
       const int64_t pos0 = sOff[cl];
-      // (y: rows of the run, at most 512, and above them the 64-key block's number inside its column)
+      // (y: rows of the run, at most ROWS, and above them the 64-key block's number inside its column)
       sInfo[st] = make_int4((cb + cl) * Bn + kb * 64, sCnt[cl] | (kb << 16), (int)(uint32_t)(pos0 & 0xffffffffll), (int)(pos0 >> 32));
     }
     __syncthreads();  // (also: everyone has read the scratch arrays before the first tile loads overwrite them)
@@ -1629,21 +1636,21 @@ static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, h
                    : launch_dkdv_kernel(attn_bwd_dkdv_partials_kernel<T, HD, KB, false>, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s);
 }
 
-template <typename T, int HD, int RT>
+template <typename T, int HD, int RT, int NW>
 static int launch_dq(const fmoba_attn_bwd_args &a, const uint16_t *ws, hipStream_t s) {
-  auto kern = attn_bwd_dq_kernel<T, HD, RT>;
-  const size_t smem = DqSmem<HD, RT>::bytes;
+  auto kern = attn_bwd_dq_kernel<T, HD, RT, NW>;
+  const size_t smem = DqSmem<HD, RT, NW>::bytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int nsb_max = ceil_div(a.max_seqlen_q, DqSmem<HD, RT>::ROWS);
+  const int nsb_max = ceil_div(a.max_seqlen_q, DqSmem<HD, RT, NW>::ROWS);
   const int64_t items = (int64_t)a.heads * a.batch * nsb_max;
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_bwd: too many (sequence, head, superblock) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(512), smem, s, a, ws, nsb_max);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * NW), smem, s, a, ws, nsb_max);
   return 0;
 }
 
@@ -1653,7 +1660,7 @@ int run_bwd_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, hipStream_t
 // columns of a multiple of 128 keys: one workgroup (and one dQ partial per visit) per 128 keys
 static inline bool bwd_wide_blocks(const fmoba_attn_bwd_args &a) { return a.head_dim > 64 && a.lg_block_n % 128 == 0; }
 
-// Which form of the dQ computation a call uses.  The row-stationary form works on (128-row block, key block) steps
+// Which form of the dQ computation a call uses.  The row-stationary form works on (256-row block, key block) steps
 // and is the faster one while a step has enough rows; with many chunks per sequence a step has one or two rows and
 // only the per-visit partials scale.  Measured break-even points (16 heads of 128, 8K and 16K tokens per sequence,
 // top-k 8 to 32): a row selects a tenth of the chunks it may see (64-key blocks), three eighths with 128-key blocks,
@@ -1701,7 +1708,7 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
     if (phases & FMOBA_BWD_DKDV)
       if (int rc = run_bwd_dkdv_wide(a, ws.ds, s)) return rc;
     if (phases & FMOBA_BWD_DQ)
-      if (int rc = launch_dq<T, 256, 1>(a, ws.ds, s)) return rc;
+      if (int rc = launch_dq<T, 256, 1, 8>(a, ws.ds, s)) return rc;
     return 0;
   }
   if (phases & FMOBA_BWD_DKDV) {
@@ -1726,7 +1733,7 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
       }
       hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 15) / 16)), dim3(256), smem, s, a, ws, capl);
     } else {
-      int rc = a.head_dim <= 64 ? launch_dq<T, 64, 1>(a, ws.ds, s) : launch_dq<T, 128, 2>(a, ws.ds, s);
+      int rc = a.head_dim <= 64 ? launch_dq<T, 64, 1, 8>(a, ws.ds, s) : launch_dq<T, 128, 2, 4>(a, ws.ds, s);
       if (rc) return rc;
     }
   }
