@@ -102,7 +102,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   const int gh = ws.dkv_heads, gs = a.heads / gh;  // heads of dK / dV, query heads that are added up in one
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * gh, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * gh, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
+                                      longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
   const int nb = item.idx, b = item.pair / gh, hg = item.pair - b * gh, h0 = hg * gs;
   const int key0 = nb * NKEY;
   const int Bn = a.lg_block_n, c = key0 / Bn;
@@ -485,7 +486,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
   float *sLse = reinterpret_cast<float *>(smem + SM::oLse);
   float *sDelta = reinterpret_cast<float *>(smem + SM::oDelta);
 
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
+                                      longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
   const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
   const int key0 = nb * NKEY;
   // One workgroup per compute unit: nothing covers the dependent loads before the first round, so their chain is kept
@@ -1127,8 +1129,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
 // one group ahead, so the workgroup meets at a barrier once per group: inside a group every wave runs at its own
 // pace, and a wave's chain of dependent steps (where are my rows in this column's list -> fetch them -> multiply)
 // is covered by the products of the other wave of its SIMD.
-// ------------------------------------------------------------------------------------
-constexpr int kDqColBatch = 256;
 //
 // What bounds it: the misses a unit can have in flight (dS pieces of 64 to 512 bytes at scattered places), and in calls of few
 // workgroups the longest walk.  Head dimensions 65 to 128: four waves with two row tiles each, two workgroups per unit and
@@ -1138,6 +1138,8 @@ constexpr int kDqColBatch = 256;
 // below), 2 x 4096 tokens 143 -> 125.  Up to 64: eight waves of one tile (with two tiles in four waves 4096 tokens 58 -> 67 us).
 // Above 128: eight waves of one tile, one workgroup per unit (its K tiles take 128 KB).
 constexpr int kDqMaxSteps = 512;
+// ------------------------------------------------------------------------------------
+constexpr int kDqColBatch = 256;
 
 template <int HD, int RT, int NW>
 struct DqSmem {
@@ -1166,9 +1168,14 @@ struct DqSmem {
 struct DqItem {
   int pair, sb;
 };
-__device__ __forceinline__ DqItem dq_decode_item(int id, int npairs, int nsb_max) {
+__device__ __forceinline__ DqItem dq_decode_item(int id, int npairs, int nsb_max, bool longest_first) {
+  // One workgroup each for the slots of the chip (32 units per XCD, two to a unit) start all at once: the second half in
+  // reverse, so that the longest walks share a unit with the shortest (4096 tokens, 32 over 8 heads: 113 -> 104 us, 8192
+  // tokens, 16 heads: 198 -> 186).
+  const int n = npairs % 8 == 0 ? npairs / 8 * nsb_max : 0;
+  if (longest_first && n > 32 && n <= 64 && (id >> 3) >= 32) id = ((n + 31 - (id >> 3)) << 3) | (id & 7);
   // late row blocks (the longest walks) first
-  const PairItem item = xcd_pair_item(id, npairs, nsb_max);
+  const PairItem item = xcd_pair_item(id, npairs, nsb_max, false, longest_first);
   DqItem w;
   w.pair = item.pair < npairs ? item.pair : -1;
   w.sb = nsb_max - 1 - item.idx;
@@ -1204,7 +1211,7 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
   int *sMisc = reinterpret_cast<int *>(smem + SM::oMisc);
   const uint32_t ldsK = (uint32_t)(uintptr_t)(smem + SM::oK);
 
-  const DqItem wi = dq_decode_item(blockIdx.x, a.heads * a.batch, nsb_max);
+  const DqItem wi = dq_decode_item(blockIdx.x, a.heads * a.batch, nsb_max, longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 2));
   if (wi.pair < 0) return;
   const int b = wi.pair / a.heads, h = wi.pair - b * a.heads, sb = wi.sb;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;

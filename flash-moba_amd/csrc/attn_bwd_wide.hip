@@ -36,7 +36,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
   constexpr int HD = SM::HD, KS = HD / 16, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR;
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + 63) / 64);
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + 63) / 64, false, longest_items_first(max(a.total_q, a.total_k), a.heads, 1024));
   const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
   const int key0 = nb * 64;
   const int Bn = a.lg_block_n, c = key0 / Bn;

@@ -446,7 +446,7 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
   uint32_t *sBits = reinterpret_cast<uint32_t *>(sOff + 8);
 
   const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb);
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
   const int b = item.pair / a.heads, h = item.pair - b * a.heads;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   const int rb = nrb - 1 - item.idx;  // the longest walks (last rows of a causal sequence) start first

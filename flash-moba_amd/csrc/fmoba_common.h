@@ -536,16 +536,34 @@ __device__ __forceinline__ void static_for(F &&f) {
 // an L2 still holds a good part of a pair, the same order costs 13 %).
 // ------------------------------------------------------------------------------------
 constexpr long long kOnePairBytes = 64ll << 20;
+// longest_first takes the items of an XCD's pairs in turn instead, item 0 of every pair, then item 1, .. : the callers number
+// the items of a pair from the longest down, so the launch begins with the longest of all pairs and its last round is made of
+// the shortest.  With a few rounds of workgroups, or sequences of different lengths, that is what decides the time: a
+// pair-by-pair launch ends with a whole pair's mixture, its long items among them.  It gives up what a pair's items find in the
+// L2 of each other, so it is for calls whose rows, all pairs together (row_bytes per row and head: what the kernel reads of
+// them again and again), take no more than kLongestFirstBytes and come from the memory-side cache at worst.  The pairs of a turn
+// are rotated by one from turn to turn where their number is even: workgroups go round the shader engines, and without the
+// rotation an engine gets the same pairs, hence the same sequences, in every turn (8192 tokens in four sequences, 32 over 8
+// heads: dK/dV 520 us without, 336 with).  Before and after: row-block forward of 8192 tokens in four sequences 145 -> 111 us,
+// of 2 x 4096 211 -> 195, dK/dV of 8191 tokens of short documents 55 -> 44, column forward of 8192 tokens 134 -> 114.  Where the line
+// lies: 24576 tokens, 16 heads of 128 (201 MB) dK/dV 1031 -> 1061 us, 65536 tokens (537 MB) row-block forward 2787 -> 3203.
+constexpr long long kLongestFirstBytes = 128ll << 20;
+__device__ __forceinline__ bool longest_items_first(int64_t rows, int heads, int row_bytes) { return rows * heads * row_bytes <= kLongestFirstBytes; }
 struct PairItem {
   int pair, idx;
 };
-__device__ __forceinline__ PairItem xcd_pair_item(int id, int npairs, int nper, bool one_pair_at_a_time = false) {
+__device__ __forceinline__ PairItem xcd_pair_item(int id, int npairs, int nper, bool one_pair_at_a_time = false, bool longest_first = false) {
   PairItem w;
   if (npairs % 8 == 0 && !one_pair_at_a_time) {
-    const int s = id >> 3;
-    const int pl = s / nper;
-    w.pair = pl * 8 + (id & 7);
+    const int s = id >> 3, np = npairs >> 3;
+    int pl = s / nper;
     w.idx = s - pl * nper;
+    if (longest_first) {
+      w.idx = s / np;
+      pl = s - w.idx * np;
+      if (np % 2 == 0) pl = (pl + w.idx) % np;
+    }
+    w.pair = pl * 8 + (id & 7);
   } else {
     w.pair = id / nper;
     w.idx = id - w.pair * nper;
