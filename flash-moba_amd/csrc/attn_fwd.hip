@@ -58,13 +58,13 @@ struct FwdColSmem {
 // 530 -> 162 us, 8192 tokens with top-k 8 148 -> 132 us, 262144 tokens 9.99 -> 9.12 ms, and one row per sequence against
 // 16 sequences of up to 32768 keys 651 -> 113 us.
 template <typename T, int HD, int KB>
-__global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws) {
+__global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp) {
   typedef FwdColSmem<HD, KB> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, KT = KB / 32, RB = HD * 2;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads_k, (a.max_seqlen_k + KB - 1) / KB, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes);
-  const int nb = item.idx, b = item.pair / a.heads_k, hk = item.pair - b * a.heads_k;
-  const int grp = a.heads / a.heads_k, h0 = hk * grp;
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * (a.heads / grp), (a.max_seqlen_k + KB - 1) / KB, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
+                                      longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 2));
+  const int ngrp = a.heads / grp, nb = item.idx, b = item.pair / ngrp, h0 = (item.pair - b * ngrp) * grp, hk = h0 / (a.heads / a.heads_k);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
   const int key0 = nb * KB;
   const int c = key0 / a.lg_block_n;
@@ -488,6 +488,20 @@ static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   return chunks_per_row * (large ? 27 : kFwdRowsDensity128) >= seen * 10;
 }
 
+// Query heads per workgroup.  All heads of a group share the block's K and V and a workgroup's first loads, which is most of the
+// time of a call with short lists (1000-row parts of prompts against 9000 to 33000 keys: 164 us, 325 with a head each).  Long
+// lists make few long workgroups of it, so the group is divided until there are three rounds of them for the chip's 512
+// places, as long as each of the four waves keeps two tiles (32 over 8 heads, top-k 4 of 128-key chunks: 4096 tokens
+// 131 -> 68 us, 8192 tokens 190 -> 127, 16384 tokens 292 -> 231; with one head each 24576 tokens take 462 us instead of 419).
+static int fwd_col_heads(const fmoba_attn_fwd_args &a, int kb) {
+  const int grp = a.heads / a.heads_k;
+  const int64_t blocks = (int64_t)a.total_k / kb + a.batch;
+  const int64_t tiles = (int64_t)a.total_q * fwd_partial_cap(a) / 32 / blocks;  // of one head's lists, on average
+  int best = grp;
+  for (int gs = grp - 1; gs >= 1 && blocks * (a.heads / best) < 1536 && tiles * gs >= 8; --gs)
+    if (grp % gs == 0) best = gs;
+  return best;
+}
 template <typename T, int HD, int KB>
 static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStream_t s) {
   auto kern = attn_fwd_col_kernel<T, HD, KB>;
@@ -496,12 +510,13 @@ static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStre
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * a.heads_k * ceil_div(a.max_seqlen_k, KB);
+  const int grp = fwd_col_heads(a, KB);
+  const int64_t items = (int64_t)a.batch * (a.heads / grp) * ceil_div(a.max_seqlen_k, KB);
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_fwd: too many (sequence, head, key block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws, grp);
   return 0;
 }
 template <typename T>
