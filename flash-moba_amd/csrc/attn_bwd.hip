@@ -1673,7 +1673,7 @@ static inline bool bwd_wide_blocks(const fmoba_attn_bwd_args &a) { return a.head
 // only the per-visit partials scale.  Measured, dK/dV and dQ together, partials against dS tiles:
 //  - 128-key blocks at head dimensions 65 to 128 (a visit leaves one partial per 128 keys): even where a row selects 3/8 of
 //    the chunks it may see (32768 tokens, 0.30 of them 5130 against 5433 us, 0.45 7371 against 7048);
-//  - 64-key blocks at head dimension 128: the more chunks, the later (4 x 4096 tokens even below a sixteenth; 8192 tokens at 0.20;
+//  - 64-key blocks at head dimension 128: later with more chunks, hence the constant (4 x 4096 tokens even below 0.06; 8192 at 0.20;
 //    32768 tokens at 0.165, with 0.12 3142 against 3560 us; 16384 tokens, 16 over 4 heads, at 0.35);
 //  - head dimensions up to 64: 0.25 of the chunks at 16384 and 32768 tokens (0.12: 1999 against 2497 us), 0.45 at 8192.
 // Partials take twice the memory of dS tiles: beyond 1/10 (64-key blocks) only up to kPartialBytes of them.
@@ -1688,7 +1688,7 @@ static int bwd_dq_partials(const fmoba_attn_bwd_args &a) {
   if (bwd_wide_blocks(a)) return chunks_per_row < 0.37 * seen;
   if (chunks_per_row < 0.10 * seen) return 1;
   if ((int64_t)a.total_q * a.heads * std::max(a.max_visits_per_row, 1) * a.head_dim * 2 > kPartialBytes) return 0;
-  return a.head_dim > 64 ? chunks_per_row < 0.18 * seen - 3.0 : chunks_per_row < 0.22 * seen;
+  return a.head_dim > 64 ? chunks_per_row < 0.18 * seen - 4.0 : chunks_per_row < 0.22 * seen;
 }
 // Heads of dK / dV the call is best made with: heads / this many query heads are added up by one workgroup, in fp32, instead
 // of in memory afterwards (24571 tokens, 32 over 8 heads: 1225 us and two sums of 48 us -> 1118 us).  All heads of a group, unless that
