@@ -50,11 +50,12 @@ void check_device(int index) {
 
 PyObject *g_parameter_class = nullptr;  // torch.nn.Parameter
 
-// an ordinary tensor (or parameter): no subclass, no wrapper of a transform, no lazy conjugate
+// an ordinary tensor (or parameter): no subclass, no wrapper of a transform, no lazy conjugate, no tangent of forward-mode
+// differentiation (a dual tensor has the key set of an ordinary one; the path in Python refuses it, having no derivative of that kind)
 bool plain(const py::handle &h) {
   if (!THPVariable_CheckExact(h.ptr()) && reinterpret_cast<PyObject *>(Py_TYPE(h.ptr())) != g_parameter_class) return false;
   const Tensor &t = THPVariable_Unpack(h.ptr());
-  return t.defined() && t.is_cuda() && !t.is_sparse() &&
+  return t.defined() && t.is_cuda() && !t.is_sparse() && !t._fw_grad(/*level=*/0).defined() &&
          !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                                    c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative}));
 }

@@ -63,3 +63,19 @@ def test_gradients_have_no_gradients():
     (dx,) = torch.autograd.grad(out.sum(), x, create_graph=True)
     with pytest.raises(RuntimeError):
         dx.sum().backward()
+
+
+# forward-mode differentiation has no rule here: a call on a dual tensor says so instead of returning a result without tangent
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("two_step", [False, True])
+def test_dual_tensors_are_refused(which, two_step):
+    qkv = [torch.randn((200, 2, 64), device="cuda").to(torch.bfloat16) for _ in range(3)]
+    cu = torch.tensor([0, 200], dtype=torch.int32, device="cuda")
+    pattern = flash_moba.flash_topk_varlen_func(qkv[0], qkv[1], cu, cu, 200, 200, 2, 64, causal=True)
+    with torch.autograd.forward_ad.dual_level():
+        qkv[which] = torch.autograd.forward_ad.make_dual(qkv[which], torch.ones_like(qkv[which]))
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            if two_step:
+                flash_moba.flash_moba_attn_varlen_func(*qkv, cu, cu, 200, 200, *pattern, lg_block_m=128, lg_block_n=64, causal=True)
+            else:
+                flash_moba.flash_moba_varlen_func(*qkv, cu, cu, 200, 200, 64, 2)
