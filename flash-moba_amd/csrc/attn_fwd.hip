@@ -11,7 +11,8 @@
 //                             O^T = V^T P^T (V^T through transposing LDS reads).  Every visit of
 //                             a (row, key block) pair leaves a PARTIAL result: the block-local
 //                             maximum m, the sum l of exp2(s - m) and the unnormalised output row
-//                             (16-bit), in a slot that the row hands out from a counter.
+//                             (16-bit; fp32 above head dimension 128), in a slot that the row hands
+//                             out from a counter.
 //   attn_fwd_combine_kernel : sixteen lanes per (row, head) merge the row's partials in ascending
 //                             key-block order (sorted by block id, so the result does not depend
 //                             on which slot a visit happened to get): out, log-sum-exp.
@@ -37,16 +38,22 @@ constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 struct FwdWs {
   int32_t *cnt;      // [total_q * heads] visits handed out per (row, head)
   float4 *hdr;       // [total_q * heads * cap] {m (log2 domain), l, key block id, -}
-  uint16_t *part;    // [total_q * heads * cap][head_dim] unnormalised partial outputs
+  void *part;        // [total_q * heads * cap][head_dim] unnormalised partial outputs (fwd_part_size bytes each)
   int32_t cap;
 };
+
+// Bytes per element of a partial row: the 16-bit type of the call, fp32 at head dimensions above 128.  There this form serves
+// dense patterns too, whose rows the row-block form adds up in fp32 from end to end, and the two agree in precision.
+constexpr size_t fwd_part_size(int head_dim) { return head_dim > 128 ? 4 : 2; }
 
 template <int HD, int KB>
 struct FwdColSmem {
   static constexpr size_t tile = (size_t)KB * HD * 2;  // K or V of the block: rows of exactly HD elements, swizzled
-  static constexpr size_t oOut = 2 * tile;             // [4 waves][32 rows][64 features]: half a tile of partial rows on its way out
-  static constexpr size_t bytes = oOut + 4 * 4096;
-  static_assert(2 * bytes <= 160 * 1024, "two workgroups per compute unit");
+  static constexpr size_t oOut = 2 * tile;             // [NW waves][32 rows][128 bytes]: a part of a tile's partial rows on its way out
+  // Two workgroups of four waves per compute unit; 128 keys of 256 features fill the unit's LDS: one workgroup of eight.
+  static constexpr int NW = 2 * (oOut + 4 * 4096) <= 160 * 1024 ? 4 : 8;
+  static constexpr size_t bytes = oOut + NW * 4096;
+  static_assert(bytes * (8 / NW) <= 160 * 1024, "eight waves per compute unit");
 };
 
 // Two workgroups per compute unit, two waves per SIMD, no barrier after the block's K and V have arrived.  What bounds it
@@ -57,10 +64,14 @@ struct FwdColSmem {
 // 512-register waves per unit and head and walked 128 rows between barriers: on those two shapes 2.32 -> 2.17 ms and
 // 530 -> 162 us, 8192 tokens with top-k 8 148 -> 132 us, 262144 tokens 9.99 -> 9.12 ms, and one row per sequence against
 // 16 sequences of up to 32768 keys 651 -> 113 us.
+// Head dimensions above 128: an fp32 partial row per 128 keys is as many bytes as a 16-bit one per 64, and 128 keys are what one
+// workgroup of eight waves finds room for (2 x 4096 tokens, 8 heads of 256, top-k 8 of 128-key chunks, forward: 16-bit rows
+// per 64 keys 273 us, fp32 rows per 64 keys 450, per 128 keys 269).  Chunks that 128 does not divide pay for the wider rows:
+// top-k 16 of 64-key chunks 259 -> 439 us.
 template <typename T, int HD, int KB>
-__global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp) {
+__global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp) {
   typedef FwdColSmem<HD, KB> SM;
-  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, KT = KB / 32, RB = HD * 2;
+  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, KT = KB / 32, RB = HD * 2, NW = SM::NW;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   const PairItem item = xcd_pair_item(blockIdx.x, a.batch * (a.heads / grp), (a.max_seqlen_k + KB - 1) / KB, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
                                       longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 2));
@@ -100,7 +111,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
     const int ntile = __builtin_amdgcn_readlane(incl, 63);
     if (ntile == 0) continue;
     if (!loaded) {
-      constexpr int RPI = 64 / VPR, NI = KB / RPI / 4;
+      constexpr int RPI = 64 / VPR, NI = KB / RPI / NW;
       const int rl = lane / VPR, pc = lane % VPR;
       const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
       const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
@@ -113,7 +124,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
         global_to_lds16(vg + kc * a.v_row_stride + e, ldsV + (uint32_t)((wave * NI + i) * 1024));
       }
     }
-    // The wave's tiles: tile t + 8 is picked (its row ids are asked for) and the rows of tile t + 4 are fetched while tile t
+    // The wave's tiles: tile t + 2 NW is picked (its row ids are asked for) and the rows of tile t + NW are fetched while tile t
     // is worked on, and all of these loads are awaited at one place, before the stores of tile t: one counter covers
     // loads and stores alike, and a load issued after the stores would be waited for together with them.
     int g = 0, rem = 0, ridn = 0;
@@ -155,14 +166,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
     };
     pick(wave);
     fetch(wave);
-    pick(wave + 4);
+    pick(wave + NW);
     arrived();
     if (!loaded) {
       wait_all_loads();
       __syncthreads();
       loaded = true;
     }
-    for (int t = wave; t < ntile; t += 4) {
+    for (int t = wave; t < ntile; t += NW) {
       const int r = rid, h = hcur;
       const int s0 = __shfl(slot, lane & 31, 64);
       const int pidx = (r >= 0 && s0 < ws.cap) ? ((q0 + r) * a.heads + h) * ws.cap + s0 : -1;
@@ -194,8 +205,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
         for (int kt = 0; kt < KT; ++kt) st[kt] = mfma32<T>(kf[ks & 1][kt], qb[ks], st[kt]);
         __builtin_amdgcn_sched_barrier(0);
       });
-      fetch(t + 4);
-      pick(t + 8);
+      fetch(t + NW);
+      pick(t + 2 * NW);
       if (!__all(lim >= KB - 1)) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
@@ -226,7 +237,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
             pf[kt][s2].w[w] = pack2<T>(p0, p1);
           }
       l = sum_xor32_f(l);
-      Pack8 x[NDT][2];
+      constexpr bool F32 = fwd_part_size(HD) == 4;
+      // a tile's partial rows, 128 bytes of every row at a time: 64 features in 16 bits, 32 features in fp32
+      constexpr int HELD = F32 ? NDT / KT : NDT;  // feature tiles that are kept until the next tile's loads are in
+      Pack8 x[F32 ? HELD : NDT / 2][4];
       uint32_t tv = ldsV + troff;
 #if defined(__HIP_DEVICE_COMPILE__)
       asm volatile("" : "+v"(tv));
@@ -244,6 +258,33 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
         }
       };
       v_read(std::integral_constant<int, 0>{});
+      // Rows leave through LDS, 128 bytes of each at a time, so that eight lanes store the 128 bytes of a row together: stored
+      // from where the products leave them (16 bytes per lane, 32 per row and instruction) every line went to memory
+      // in pieces, and the kernel took nearly twice as long (275 against 146 us at 8192 tokens).  Piece p of row r lies at piece p ^ (r & 7).
+      auto flush = [&](const Pack8(&piece)[4], int part) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lds_write_vec<u32x4_t>(ldsOut + (uint32_t)((lane & 31) * 128 + (((2 * e + hh) ^ (lane & 7)) * 16)), pack8_vec(piece[e]));
+        wave_lds_fence();
+        Pack8 y[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y[k] = lds_read16(ldsOut + (uint32_t)((8 * k + (lane >> 3)) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) * 16)));
+        wave_lds_fence();
+        typedef std::conditional_t<F32, float, uint16_t> E;
+        const int f = (part * 8 + (lane & 7)) * (int)(16 / sizeof(E));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int p2 = __shfl(pidx, 8 * k + (lane >> 3), 64);
+          if (p2 >= 0 && f < D) st_stream16(reinterpret_cast<E *>(ws.part) + ((uint64_t)(uint32_t)p2 * (uint32_t)D + (uint32_t)f), y[k]);
+        }
+      };
+      // once the next tile's loads are in, what is held of this one leaves
+      auto flush_held = [&]() {
+        arrived();
+        if (pidx >= 0 && hh == 0) st_stream16(ws.hdr + pidx, Pack8{{__float_as_uint(m), __float_as_uint(l), (uint32_t)nb, 0u}});
+        // (the header past the caches, as the rows: written the ordinary way it cost 6 to 8 % of the kernel)
+#pragma unroll
+        for (int part = 0; part < (int)(sizeof(x) / sizeof(x[0])); ++part) flush(x[part], part);
+      };
       f32x16 o;
       static_for<2 * NDT>([&](auto hc) {
         constexpr int hb = decltype(hc)::value, dt = hb >> 1;
@@ -260,54 +301,47 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_col_kernel(fmoba_attn_fwd_arg
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr ((hb & 1) == 0) return;
-        // four features per lane and group of eight: the two halves of the wave exchange, so that a lane stores eight
+        if constexpr (F32) {
+          Pack8 y[4];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+          for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            const uint32_t ev = pack2<T>(o[8 * j + 2 * w], o[8 * j + 2 * w + 1]), od = pack2<T>(o[8 * j + 4 + 2 * w], o[8 * j + 4 + 2 * w + 1]);
-#if defined(__HIP_DEVICE_COMPILE__)
-            auto sw = __builtin_amdgcn_permlane32_swap(ev, od, false, false);
-            x[dt][j].w[w] = sw[0];
-            x[dt][j].w[2 + w] = sw[1];
-#else
-            x[dt][j].w[w] = ev, x[dt][j].w[2 + w] = od;
-#endif
+            for (int w = 0; w < 4; ++w) y[e].w[w] = __float_as_uint(o[4 * e + w]);
+          if constexpr (dt < HELD) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[dt][e] = y[e];
+            if constexpr (dt == HELD - 1) flush_held();
+          } else {
+            flush(y, dt);
           }
+        } else {
+          // four features per lane and group of eight: the two halves of the wave exchange, so that a lane stores eight
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+              const uint32_t ev = pack2<T>(o[8 * j + 2 * w], o[8 * j + 2 * w + 1]), od = pack2<T>(o[8 * j + 4 + 2 * w], o[8 * j + 4 + 2 * w + 1]);
+              Pack8 &y = x[dt >> 1][2 * (dt & 1) + j];
+#if defined(__HIP_DEVICE_COMPILE__)
+              auto sw = __builtin_amdgcn_permlane32_swap(ev, od, false, false);
+              y.w[w] = sw[0];
+              y.w[2 + w] = sw[1];
+#else
+              y.w[w] = ev, y.w[2 + w] = od;
+#endif
+            }
+          }
+          if constexpr (dt == NDT - 1) flush_held();
         }
       });
-      arrived();
-      if (pidx >= 0 && hh == 0) st_stream16(ws.hdr + pidx, Pack8{{__float_as_uint(m), __float_as_uint(l), (uint32_t)nb, 0u}});
-      // (the header past the caches, as the rows: written the ordinary way it cost 6 to 8 % of the kernel)
-      // Rows leave through LDS, 64 features at a time, so that eight lanes store the 128 bytes of a row together: stored
-      // from where the products leave them (16 bytes per lane, 32 per row and instruction) every line went to memory
-      // in pieces, and the kernel took nearly twice as long (275 against 146 us at 8192 tokens).  Piece p of row r lies at piece p ^ (r & 7).
-#pragma unroll
-      for (int half = 0; half < HD / 64; ++half) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          lds_write_vec<u32x4_t>(ldsOut + (uint32_t)((lane & 31) * 128 + (((2 * e + hh) ^ (lane & 7)) * 16)), pack8_vec(x[2 * half + (e >> 1)][e & 1]));
-        wave_lds_fence();
-        Pack8 y[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) y[k] = lds_read16(ldsOut + (uint32_t)((8 * k + (lane >> 3)) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) * 16)));
-        wave_lds_fence();
-        const int f = half * 64 + (lane & 7) * 8;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int p2 = __shfl(pidx, 8 * k + (lane >> 3), 64);
-          if (p2 >= 0 && f < D) st_stream16(ws.part + ((uint64_t)(uint32_t)p2 * (uint32_t)D + (uint32_t)f), y[k]);
-        }
-      }
     }
   }
 }
 
 // One 16-lane group per (row, head), four per wave, sixteen per block of 256: a row's chain of dependent steps (count,
 // headers, order, rows) is mostly waiting, so a wave runs four of them side by side.  Lane li of a group owns the
-// 16-byte piece li of the row.
-// (head dimensions above 128: pieces li and li + 16, NP = 2)
-template <typename T, int NP>
+// 16-byte pieces li, li + 16, .. (NP of them) of the row, whose elements are of type E.
+template <typename T, typename E, int NP>
 __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_args a, FwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
   __shared__ float sWgt[16][16], sWl[16][16];
@@ -326,14 +360,15 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   if (nall > ws.cap && li == 0 && a.visits_overflow != nullptr) atomicMax(a.visits_overflow, nall);  // visits were dropped
   int nmax = max(n, __shfl_xor(n, 16, 64));
   nmax = max(nmax, __shfl_xor(nmax, 32, 64));  // the wave walks the longest of its four rows
-  const int c8 = li * 8;
-  const bool mine = c8 < D, mine2 = NP > 1 && c8 + 128 < D;
-  float acc[8 * NP];
+  constexpr int PE = 16 / sizeof(E);  // elements of a piece
+  const int c0 = li * PE;             // the lane's pieces begin at features c0, c0 + 16 * PE, ..
+  const bool mine = c0 < D;
+  float acc[PE * NP];
 #pragma unroll
-  for (int i = 0; i < 8 * NP; ++i) acc[i] = 0.f;
+  for (int i = 0; i < PE * NP; ++i) acc[i] = 0.f;
   float L = 0.f, M = -INFINITY;
   const float4 *hdr = ws.hdr + rh * ws.cap;
-  const uint16_t *part = ws.part + rh * ws.cap * D;
+  const E *part = reinterpret_cast<const E *>(ws.part) + rh * ws.cap * D;
   // The slot a visit got is arbitrary (a counter handed it out), the sum must not depend on it: every partial gets
   // its rank in ascending key-block order over the WHOLE row (equal ids, a malformed pattern, are ordered by slot),
   // and the partials are merged in rank order, 16 at a time.
@@ -355,7 +390,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
     const float Mu = Mn == -INFINITY ? 0.f : Mn;
     const float resc = __builtin_amdgcn_exp2f(M - Mu);  // M = -inf: nothing accumulated yet, factor 0 on zeros
 #pragma unroll
-    for (int i = 0; i < 8 * NP; ++i) acc[i] *= resc;
+    for (int i = 0; i < PE * NP; ++i) acc[i] *= resc;
     L *= resc;
     M = Mn;
     const float wj = (li < cntb) ? __builtin_amdgcn_exp2f(mj - Mu) : 0.f;
@@ -373,14 +408,18 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
         for (int p = 0; p < NP; ++p)
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            acc[8 * p + 2 * k] = fmaf(w, elem_to_float<T>((uint16_t)(x[p].w[k] & 0xffffu)), acc[8 * p + 2 * k]);
-            acc[8 * p + 2 * k + 1] = fmaf(w, elem_to_float<T>((uint16_t)(x[p].w[k] >> 16)), acc[8 * p + 2 * k + 1]);
+            if constexpr (sizeof(E) == 4) {
+              acc[4 * p + k] = fmaf(w, __uint_as_float(x[p].w[k]), acc[4 * p + k]);
+            } else {
+              acc[8 * p + 2 * k] = fmaf(w, elem_to_float<T>((uint16_t)(x[p].w[k] & 0xffffu)), acc[8 * p + 2 * k]);
+              acc[8 * p + 2 * k + 1] = fmaf(w, elem_to_float<T>((uint16_t)(x[p].w[k] >> 16)), acc[8 * p + 2 * k + 1]);
+            }
           }
       };
       auto load = [&](Pack8(&x)[NP], int slot) {
-        const uint16_t *row = part + (int64_t)slot * D + c8;
-        x[0] = ld_stream16(row);
-        if constexpr (NP > 1) x[1] = ld_stream16(mine2 ? row + 128 : row);
+        const E *row = part + (int64_t)slot * D + c0;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) x[p] = ld_stream16(c0 + p * 16 * PE < D ? row + p * 16 * PE : row);
       };
       int t = 0;
       for (; t + 4 <= cntb; t += 4) {  // independent loads, four in flight
@@ -404,13 +443,15 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   if (!valid) return;
   const bool empty = !(L > 0.f);
   const float inv = empty ? 0.f : 1.f / L;
-  uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + row * a.o_row_stride + (int64_t)h * a.o_head_stride + c8;
+  uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + row * a.o_row_stride + (int64_t)h * a.o_head_stride + c0;
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    Pack8 o;
+    struct alignas(2 * PE) {
+      uint32_t w[PE / 2];
+    } o;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o.w[k] = pack2<T>(acc[8 * p + 2 * k] * inv, acc[8 * p + 2 * k + 1] * inv);
-    if (p == 0 ? mine : mine2) *reinterpret_cast<Pack8 *>(op + 128 * p) = o;
+    for (int k = 0; k < PE / 2; ++k) o.w[k] = pack2<T>(acc[PE * p + 2 * k] * inv, acc[PE * p + 2 * k + 1] * inv);
+    if (c0 + p * 16 * PE < D) *reinterpret_cast<decltype(o) *>(op + p * 16 * PE) = o;
   }
   if (li == 0) a.softmax_lse[(int64_t)h * a.total_q + row] = empty ? INFINITY : (M + __builtin_amdgcn_logf(L)) * 0.6931471805599453f;
 }
@@ -452,11 +493,8 @@ __global__ __launch_bounds__(256) void max_i32_kernel(const int32_t *p, int64_t 
 
 static inline size_t fwd_align256(size_t x) { return (x + 255) & ~(size_t)255; }
 static inline int fwd_key_block(int lg_block_n) { return lg_block_n % 128 == 0 ? 128 : 64; }
-// partial slots per (row, head): the caller's bound counts key blocks of fwd_key_block keys, and head dimensions above 128
-// have blocks of 64 (K and V of 128 keys would not leave room for a second workgroup on the unit)
-static inline int64_t fwd_partial_cap(const fmoba_attn_fwd_args &a) {
-  return (int64_t)a.max_visits_per_row * (a.head_dim > 128 ? fwd_key_block(a.lg_block_n) / 64 : 1);
-}
+// partial slots per (row, head)
+static inline int64_t fwd_partial_cap(const fmoba_attn_fwd_args &a) { return a.max_visits_per_row; }
 
 // the row-block form (attn_fwd_rows.hip)
 bool fwd_rows_feasible(const fmoba_attn_fwd_args &a);
@@ -472,12 +510,12 @@ static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   if (a.fwd_mode == 1) return false;
   if (!fwd_rows_feasible(a)) return false;
   if (a.fwd_mode == 2 || fwd_few_rows(a)) return true;
-  // Head dimensions above 128: a visit costs the column form a third of what the (row, 64 keys) step costs the row-block form
-  // (2 x 4096 tokens, 8 heads of 256, 8 of 128-key chunks: 1023 -> 275 us), so it serves dense patterns too,
-  // up to the size of the partial results that a call may ask for.
+  // Head dimensions above 128: the column form is the faster one at every density that was measured (columns against rows:
+  // 2 x 4096 tokens, 8 heads of 256, top-k 8 of 128-key chunks 269 against 976 us, top-k 32 of 64-key chunks 731 against 976;
+  // 16384 tokens, top-k 32 of 64-key chunks 1793 against 6918), up to the size of the partial results that a call may ask for.
   if (a.head_dim > 128) {
     const int64_t partials = (int64_t)a.total_q * a.heads * fwd_partial_cap(a);
-    return partials >= ((int64_t)1 << 31) || partials * (a.head_dim * 2 + 16) > kWidePartialBytes;
+    return partials >= ((int64_t)1 << 31) || partials * (int64_t)(a.head_dim * fwd_part_size(a.head_dim) + 16) > kWidePartialBytes;
   }
   const int64_t chunks_per_seq = std::max<int64_t>(1, ceil_div64(ceil_div64(std::max(a.total_k, 1), a.batch), a.lg_block_n));
   const int64_t chunks_per_row = std::max<int64_t>(1, (int64_t)a.max_visits_per_row * fwd_key_block(a.lg_block_n) / a.lg_block_n);
@@ -516,7 +554,7 @@ static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStre
     set_error("attn_fwd: too many (sequence, head, key block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws, grp);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * FwdColSmem<HD, KB>::NW), smem, s, a, ws, grp);
   return 0;
 }
 template <typename T>
@@ -527,7 +565,7 @@ static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hi
     const int kb = fwd_key_block(a.lg_block_n);
     int rc;
     if (a.head_dim > 128)
-      rc = launch_fwd_col<T, 256, 64>(a, ws, s);
+      rc = kb == 128 ? launch_fwd_col<T, 256, 128>(a, ws, s) : launch_fwd_col<T, 256, 64>(a, ws, s);
     else if (a.head_dim <= 64)
       rc = kb == 128 ? launch_fwd_col<T, 64, 128>(a, ws, s) : launch_fwd_col<T, 64, 64>(a, ws, s);
     else
@@ -537,7 +575,7 @@ static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hi
   if (phases & FMOBA_FWD_COMBINE) {
     const int capl = combine_order_entries(ws.cap);
     const size_t smem = (size_t)16 * capl * 4;
-    auto kern = a.head_dim > 128 ? attn_fwd_combine_kernel<T, 2> : attn_fwd_combine_kernel<T, 1>;
+    auto kern = a.head_dim > 128 ? attn_fwd_combine_kernel<T, float, 4> : attn_fwd_combine_kernel<T, uint16_t, 1>;
     if (smem > 32 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
       set_error("attn_fwd: a row with up to %d visits needs %zu bytes of LDS for the order of its partial results", ws.cap, smem);
       return 2;
@@ -555,7 +593,7 @@ static size_t fwd_cols_workspace_bytes(const fmoba_attn_fwd_args &a) {
   using namespace fmoba;
   if (a.max_visits_per_row <= 0) return 256;
   const size_t rows = (size_t)a.total_q * a.heads, cap = (size_t)fwd_partial_cap(a);
-  return fwd_align256((rows + 1) * 4) + fwd_align256(rows * cap * 16) + fwd_align256(rows * cap * a.head_dim * 2) + 256;
+  return fwd_align256((rows + 1) * 4) + fwd_align256(rows * cap * 16) + fwd_align256(rows * cap * a.head_dim * fwd_part_size(a.head_dim)) + 256;
 }
 
 extern "C" size_t fmoba_attn_fwd_workspace_bytes(const fmoba_attn_fwd_args *a) {
@@ -653,7 +691,7 @@ extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phase
   p += fwd_align256((rows + 1) * 4);
   ws.hdr = reinterpret_cast<float4 *>(p);
   p += fwd_align256(rows * ws.cap * 16);
-  ws.part = reinterpret_cast<uint16_t *>(p);
+  ws.part = reinterpret_cast<void *>(p);
   int rc = a->dtype == FMOBA_DTYPE_BF16 ? run_fwd<bf16_t>(*a, ws, phases, s) : run_fwd<f16_t>(*a, ws, phases, s);
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("attn_fwd");

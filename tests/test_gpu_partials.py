@@ -1,0 +1,34 @@
+"""Partial results of the column passes: their precision and their range against exact sums in 64 bits."""
+import pytest
+import torch
+
+import flash_moba
+from flash_moba import flash_moba_hip as hip
+
+pytestmark = pytest.mark.gpu
+
+# half a unit in the last place of the output, relative to the value, and the 32-bit sums under it
+_HALF_ULP = {torch.bfloat16: 2.0 ** -8 * (1 + 2 ** -6), torch.float16: 2.0 ** -11 * (1 + 2 ** -6)}
+
+
+def _uniform_rows(L, H, D, dtype, size, seed=0):
+    """Equal scores (q = 0): every probability is exactly 1 before it is normalised, and row i of a causal call that sees all
+    chunks is the mean of v[: i + 1]."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q = torch.zeros((L, H, D), device="cuda", dtype=dtype)
+    k = torch.randn((L, H, D), generator=g, device="cuda").to(dtype)
+    v = (size * (1 + 0.5 * torch.rand((L, H, D), generator=g, device="cuda"))).to(dtype)
+    exact = v.double().cumsum(0) / torch.arange(1, L + 1, device="cuda", dtype=torch.float64)[:, None, None]
+    return q, k, v, torch.tensor([0, L], dtype=torch.int32, device="cuda"), exact
+
+
+# above head dimension 128 the sums of a row are fp32 from end to end: a result is rounded once
+@pytest.mark.parametrize("dtype,size", [(torch.bfloat16, 1.0), (torch.float16, 1.0), (torch.float16, 2000.0)])
+@pytest.mark.parametrize("D", [136, 192, 256])
+@pytest.mark.parametrize("chunk", [64, 128])
+def test_wide_heads_round_once(dtype, size, D, chunk):
+    L = 900
+    q, k, v, cu, exact = _uniform_rows(L, 2, D, dtype, size, D)
+    out = flash_moba.flash_moba_varlen_func(q, k, v, cu, cu, L, L, chunk, 15, causal=True)
+    assert hip.last_fwd_row_blocks() == 0
+    assert ((out.double() - exact).abs() <= _HALF_ULP[dtype] * exact).all()
