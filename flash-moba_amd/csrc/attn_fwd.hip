@@ -28,11 +28,12 @@
 
 namespace fmoba {
 
-// row-block form when a row selects at least 10/50 (64-key blocks) resp. 10/24 (128-key blocks) of the chunks it may see:
-// measured break-even points, the same for 8192 to 32768 tokens, heads of 64 and 128, grouped or not (128-key blocks, columns
-// against rows: 16384 tokens, 16 over 4 heads, 0.30 of the chunks 719 against 1051 us, 0.45 1041 against 1073; 4 x 4096 tokens
-// 0.31 250 against 291, 0.44 312 against 295; 64-key blocks: 32768 tokens 0.20 4128 against 4200)
-constexpr int kFwdRowsDensity64 = 50, kFwdRowsDensity128 = 24;
+// row-block form when a row selects at least 10/50 (64-key blocks) resp. 10/27 (128-key blocks) of the chunks it may see:
+// break-even points measured at 8192 to 32768 tokens (columns against rows: 64-key blocks, 32768 tokens 0.20 of the chunks 4128
+// against 4200 us; 128-key blocks, 4 x 4096 tokens 0.31 250 against 291, 0.44 312 against 295).  With grouped heads the
+// columns are level with 128-key blocks only at 0.45 (16384 tokens, 16 over 4 heads, 0.30 719 against 1051 us, 0.45 1041 against 1073); the
+// line stays at 10/27 for them too, as rows that the row-block form adds up in fp32 are not moved to 16-bit partial rows.
+constexpr int kFwdRowsDensity64 = 50, kFwdRowsDensity128 = 27;
 constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 
 struct FwdWs {
@@ -505,7 +506,7 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s);
 // Which form runs.  The row-block form multiplies every row of a 128-row block with every chunk that
 // any of its rows selected, the column form only the selected pairs but pays a partial result per
 // visit: the first wins while a row selects more than about a fifth of the chunks it may see (64-key blocks) or
-// more than about two fifths of them (128-key blocks, whose visits cost the column form less per key).
+// more than about three eighths of them (128-key blocks, whose visits cost the column form less per key).
 static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   if (a.fwd_mode == 1) return false;
   if (!fwd_rows_feasible(a)) return false;
@@ -520,10 +521,7 @@ static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   const int64_t chunks_per_seq = std::max<int64_t>(1, ceil_div64(ceil_div64(std::max(a.total_k, 1), a.batch), a.lg_block_n));
   const int64_t chunks_per_row = std::max<int64_t>(1, (int64_t)a.max_visits_per_row * fwd_key_block(a.lg_block_n) / a.lg_block_n);
   const int64_t seen = a.is_causal ? (chunks_per_seq + 1) / 2 : chunks_per_seq;
-  if (fwd_key_block(a.lg_block_n) != 128) return chunks_per_row * kFwdRowsDensity64 >= seen * 10;
-  // (from 10/27 on: no more partial results than a call may ask for, as above)
-  const bool large = (int64_t)a.total_q * a.heads * fwd_partial_cap(a) * (a.head_dim * 2 + 16) > kWidePartialBytes;
-  return chunks_per_row * (large ? 27 : kFwdRowsDensity128) >= seen * 10;
+  return chunks_per_row * (fwd_key_block(a.lg_block_n) == 128 ? kFwdRowsDensity128 : kFwdRowsDensity64) >= seen * 10;
 }
 
 // Query heads per workgroup.  All heads of a group share the block's K and V and a workgroup's first loads, which is most of the

@@ -1,0 +1,25 @@
+"""Which form a call runs (host rules of the library), at the lines the rules draw."""
+import ctypes
+
+import pytest
+
+from flash_moba import flash_moba_hip as H
+
+
+def fwd_args(lens, chunk, topk, heads=4, D=128, causal=1):
+    f = H.AttnFwdArgs()
+    f.total_q = f.total_k = sum(lens)
+    f.heads = f.heads_k = heads
+    f.head_dim, f.batch, f.lg_block_n, f.is_causal = D, len(lens), chunk, causal
+    f.max_seqlen_q = f.max_seqlen_k = max(lens)
+    f.max_cols = -(-max(lens) // chunk)
+    f.max_visits_per_row = topk * (chunk // H.fwd_key_block(chunk))
+    return f
+
+
+# a row whose visits were added up in fp32 is not handed to 16-bit partial rows for speed: 128-key blocks stay on row blocks
+# from 10/27 of the visible chunks on, 64-key blocks from 10/50
+@pytest.mark.parametrize("chunk,topk,rows", [(128, 23, 0), (128, 24, 1), (128, 26, 1), (256, 11, 0), (256, 12, 1), (64, 25, 0), (64, 26, 1)])
+def test_forward_lines(chunk, topk, rows):
+    f = fwd_args([16384], chunk, topk)
+    assert H.load_library().fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == rows
