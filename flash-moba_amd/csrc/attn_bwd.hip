@@ -1670,14 +1670,13 @@ static inline bool bwd_wide_blocks(const fmoba_attn_bwd_args &a) { return a.head
 
 // Which form of the dQ computation a call uses.  The row-stationary form works on (256-row block, key block) steps
 // and is the faster one while a step has enough rows; with many chunks per sequence a step has one or two rows and
-// only the per-visit partials scale.  Measured, dK/dV and dQ together, partials against dS tiles:
-//  - 128-key blocks at head dimensions 65 to 128 (a visit leaves one partial per 128 keys): even where a row selects 3/8 of
-//    the chunks it may see (32768 tokens, 0.30 of them 5130 against 5433 us, 0.45 7371 against 7048);
-//  - 64-key blocks at head dimension 128: later with more chunks, hence the constant (4 x 4096 tokens even below 0.06; 8192 at 0.20;
-//    32768 tokens at 0.165, with 0.12 3142 against 3560 us; 16384 tokens, 16 over 4 heads, at 0.35);
-//  - head dimensions up to 64: 0.25 of the chunks at 16384 and 32768 tokens (0.12: 1999 against 2497 us), 0.45 at 8192.
-// Partials take twice the memory of dS tiles: beyond 1/10 (64-key blocks) only up to kPartialBytes of them.
-constexpr int64_t kPartialBytes = (int64_t)16 << 30;
+// only the per-visit partials scale.
+//  - 128-key blocks at head dimensions 65 to 128 (a visit leaves one partial per 128 keys): partials below 0.37 of the chunks a
+//    row may see (dK/dV and dQ together, partials against dS tiles: 32768 tokens, 0.30 of them 5130 against 5433 us, 0.45 7371 against 7048);
+//  - 64-key blocks, and head dimensions up to 64: below a tenth.  That line is one of precision, not of time: dS tiles add a row's
+//    visits up in fp32, a partial row is rounded to 16 bits (error of dQ against 64 bits, 8192 tokens, 0.12 of the chunks: 2.40e-3
+//    with dS tiles, 2.93e-3 with partials), and calls that have had the fp32 sums keep them although partials are the faster form
+//    further up (32768 tokens, 0.12 of the chunks, heads of 128 3142 against 3560 us, heads of 64 1999 against 2497).
 static int bwd_dq_partials(const fmoba_attn_bwd_args &a) {
   if (a.head_dim > 128) return 0;  // head dimensions above 128: dS tiles and the row-block pass only
   if (a.dq_mode == 1) return 0;
@@ -1685,10 +1684,7 @@ static int bwd_dq_partials(const fmoba_attn_bwd_args &a) {
   const double chunks_per_seq = (double)a.total_k / a.batch / a.lg_block_n;
   const double chunks_per_row = (double)a.max_visits_per_row * 64.0 / a.lg_block_n;
   const double seen = a.is_causal ? 0.5 * chunks_per_seq : chunks_per_seq;
-  if (bwd_wide_blocks(a)) return chunks_per_row < 0.37 * seen;
-  if (chunks_per_row < 0.10 * seen) return 1;
-  if ((int64_t)a.total_q * a.heads * std::max(a.max_visits_per_row, 1) * a.head_dim * 2 > kPartialBytes) return 0;
-  return a.head_dim > 64 ? chunks_per_row < 0.18 * seen - 4.0 : chunks_per_row < 0.22 * seen;
+  return chunks_per_row < (bwd_wide_blocks(a) ? 0.37 : 0.10) * seen;
 }
 // Heads of dK / dV the call is best made with: heads / this many query heads are added up by one workgroup, in fp32, instead
 // of in memory afterwards (24571 tokens, 32 over 8 heads: 1225 us and two sums of 48 us -> 1118 us).  All heads of a group, unless that

@@ -23,3 +23,16 @@ def fwd_args(lens, chunk, topk, heads=4, D=128, causal=1):
 def test_forward_lines(chunk, topk, rows):
     f = fwd_args([16384], chunk, topk)
     assert H.load_library().fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == rows
+
+
+# the same for dQ: fp32 sums over dS tiles from a tenth of the visible chunks on with 64-key blocks and with heads up to 64,
+# from 0.37 on with 128-key blocks
+@pytest.mark.parametrize("D,chunk,topk,partials", [(128, 64, 12, 1), (128, 64, 13, 0), (128, 64, 18, 0), (64, 64, 12, 1), (64, 64, 13, 0), (64, 64, 28, 0),
+                                                   (64, 128, 6, 1), (64, 128, 7, 0), (96, 128, 23, 1), (128, 128, 23, 1), (128, 128, 24, 0), (256, 64, 1, 0)])
+def test_dq_lines(D, chunk, topk, partials):
+    a = H.AttnBwdArgs()
+    a.total_q = a.total_k = a.max_seqlen_q = a.max_seqlen_k = 16384
+    a.heads = a.heads_k = 4
+    a.head_dim, a.batch, a.lg_block_n, a.is_causal = D, 1, chunk, 1
+    a.max_visits_per_row = topk * (chunk // 64)
+    assert H.load_library().fmoba_attn_bwd_uses_partials(ctypes.byref(a)) == partials
