@@ -10,9 +10,9 @@
 //                             the accumulators straight into the operand registers of
 //                             O^T = V^T P^T (V^T through transposing LDS reads).  Every visit of
 //                             a (row, key block) pair leaves a PARTIAL result: the block-local
-//                             maximum m, the sum l of exp2(s - m) and the unnormalised output row
-//                             (16-bit; fp32 above head dimension 128), in a slot that the row hands
-//                             out from a counter.
+//                             maximum m, the sum l of exp2(s - m) and the output row (bf16 or fp32:
+//                             unnormalised; fp16: divided by l), in a slot that the row hands out from
+//                             a counter.
 //   attn_fwd_combine_kernel : sixteen lanes per (row, head) merge the row's partials in ascending
 //                             key-block order (sorted by block id, so the result does not depend
 //                             on which slot a visit happened to get): out, log-sum-exp.
@@ -40,13 +40,20 @@ constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 struct FwdWs {
   int32_t *cnt;      // [total_q * heads] visits handed out per (row, head)
   float4 *hdr;       // [total_q * heads * cap] {m (log2 domain), l, key block id, -}
-  void *part;        // [total_q * heads * cap][head_dim] unnormalised partial outputs (fwd_part_size bytes each)
+  void *part;        // [total_q * heads * cap][head_dim] partial outputs (fwd_part_size bytes per element)
   int32_t cap;
 };
 
 // Bytes per element of a partial row: the 16-bit type of the call, fp32 at head dimensions above 128.  There this form serves
 // dense patterns too, whose rows the row-block form adds up in fp32 from end to end, and the two agree in precision.
 constexpr size_t fwd_part_size(int head_dim) { return head_dim > 128 ? 4 : 2; }
+
+// fp16 partial rows are divided by their sum of probabilities first: as they leave the products they are up to 64 or 128 times
+// the values, beyond the range of the type from values of about 500 on.
+// (8192 tokens, heads of 128, top-k 8 of 128-key chunks: error of the output against 64 bits 3.33e-4 -> 3.16e-4, 175 us with and
+// without; 32768 tokens, 32 heads, top-k 16 3040 -> 3054 us, the runs of one side differ by 16.)
+template <typename T, int HD>
+constexpr bool kFwdNormalisedParts = std::is_same_v<T, f16_t> && fwd_part_size(HD) == 2;
 
 template <int HD, int KB>
 struct FwdColSmem {
@@ -239,6 +246,8 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
             pf[kt][s2].w[w] = pack2<T>(p0, p1);
           }
       l = sum_xor32_f(l);
+      constexpr bool NORM = kFwdNormalisedParts<T, HD>;
+      const float inv = NORM && l > 0.f ? 1.f / l : 0.f;
       constexpr bool F32 = fwd_part_size(HD) == 4;
       // a tile's partial rows, 128 bytes of every row at a time: 64 features in 16 bits, 32 features in fp32
       constexpr int HELD = F32 ? NDT / KT : NDT;  // feature tiles that are kept until the next tile's loads are in
@@ -317,6 +326,10 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
             flush(y, dt);
           }
         } else {
+          if constexpr (NORM) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[i] *= inv;
+          }
           // four features per lane and group of eight: the two halves of the wave exchange, so that a lane stores eight
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
@@ -342,8 +355,9 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
 
 // One 16-lane group per (row, head), four per wave, sixteen per block of 256: a row's chain of dependent steps (count,
 // headers, order, rows) is mostly waiting, so a wave runs four of them side by side.  Lane li of a group owns the
-// 16-byte pieces li, li + 16, .. (NP of them) of the row, whose elements are of type E.
-template <typename T, typename E, int NP>
+// 16-byte pieces li, li + 16, .. (NP of them) of the row, whose elements are of type E
+// (NORM: divided by the visit's sum of probabilities).
+template <typename T, typename E, int NP, bool NORM>
 __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_args a, FwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
   __shared__ float sWgt[16][16], sWl[16][16];
@@ -398,7 +412,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
     const float wj = (li < cntb) ? __builtin_amdgcn_exp2f(mj - Mu) : 0.f;
     wave_lds_fence();
     if (li < cntb) {
-      sWgt[sg][li] = wj;
+      sWgt[sg][li] = NORM ? wj * lj : wj;
       sWl[sg][li] = wj * lj;
     }
     wave_lds_fence();
@@ -574,7 +588,7 @@ static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hi
   if (phases & FMOBA_FWD_COMBINE) {
     const int capl = combine_order_entries(ws.cap);
     const size_t smem = (size_t)16 * capl * 4;
-    auto kern = a.head_dim > 128 ? attn_fwd_combine_kernel<T, float, 4> : attn_fwd_combine_kernel<T, uint16_t, 1>;
+    auto kern = a.head_dim > 128 ? attn_fwd_combine_kernel<T, float, 4, false> : attn_fwd_combine_kernel<T, uint16_t, 1, kFwdNormalisedParts<T, 128>>;
     if (smem > 32 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
       set_error("attn_fwd: a row with up to %d visits needs %zu bytes of LDS for the order of its partial results", ws.cap, smem);
       return 2;

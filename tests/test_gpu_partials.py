@@ -32,3 +32,20 @@ def test_wide_heads_round_once(dtype, size, D, chunk):
     out = flash_moba.flash_moba_varlen_func(q, k, v, cu, cu, L, L, chunk, 15, causal=True)
     assert hip.last_fwd_row_blocks() == 0
     assert ((out.double() - exact).abs() <= _HALF_ULP[dtype] * exact).all()
+
+
+# fp16 rows of the column form: up to 128 equal probabilities times values of 2000 are beyond the type, the results are not
+@pytest.mark.parametrize("D", [40, 64, 128])
+@pytest.mark.parametrize("chunk", [64, 128])
+@pytest.mark.parametrize("size", [2.0 ** -13, 1.0, 2000.0, 40000.0])
+def test_fp16_column_rows_keep_to_their_range(D, chunk, size):
+    L = 900
+    q, k, v, cu, exact = _uniform_rows(L, 2, D, torch.float16, size, D)
+    co, cn, ind = flash_moba.flash_topk_varlen_func(q, k, cu, cu, L, L, 15, chunk, causal=True)
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, co, cn, ind, cu, cu, None, None, None, L, L, 0.0, 1.0, False, True, 0.0, False, 128, chunk, None,
+                                         _fwd_mode=1)
+    # a partial row and the result are rounded once each; values below 2^-14 have a fixed step of 2^-24
+    tol = 2 * _HALF_ULP[torch.float16] * exact + 2.0 ** -24
+    assert ((out.double() - exact).abs() <= tol).all()
+    n = torch.arange(1, L + 1, device="cuda", dtype=torch.float64)
+    assert ((lse.double() - n.log()).abs() <= 1e-5).all()
