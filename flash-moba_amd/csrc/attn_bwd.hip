@@ -10,7 +10,7 @@
 //                            dQ^T_partial = K^T dS^T            (per visit of a (row, key block) pair)
 //                          dK/dV live in registers for the whole list and are written
 //                          once.  For dQ the kernel leaves either its dS tiles (16-bit, indexed by
-//                          row-list position) or, per visit, a dQ partial row (16-bit, unscaled) in a
+//                          row-list position) or, per visit, a dQ partial row (16-bit; fp16: scaled) in a
 //                          slot that the row hands out from a counter.
 //   attn_bwd_dkdv_partials_kernel : the same for the long calls, dQ partials at head dimension 128.
 //   attn_bwd_dq_kernel   : dQ from the dS tiles, one workgroup per 128 query rows, dQ in registers
@@ -57,10 +57,31 @@ struct BwdWs {
   int32_t dkv_heads;  // heads of dK / dV (of the kernels that sum query heads)
   int32_t *cnt;    // [total_q * heads] visits handed out per (row, head)
   int32_t *pid;    // [total_q * heads * cap] key block id of each partial
-  uint16_t *part;  // [total_q * heads * cap][head_dim] dQ partials (unscaled)
+  uint16_t *part;  // [total_q * heads * cap][head_dim] dQ partials (times dq_part_scale)
   int32_t cap;
   uint16_t *ds;    // dS tiles (row-stationary dQ form): [row list position / 32][key of the column / 8][position % 32][8 keys]
 };
+
+// Softmax scale of dQ in the partials form: fp16 partial rows carry it (as far as it makes them smaller), the sums of bf16 ones get it.
+// Without it the rows are sqrt(head_dim) times the gradient they add up to, and fp16 rows overflow where the gradient does not.
+// (8192 tokens, heads of 128, top-k 8 of 128-key chunks, error of dQ against 64 bits: 3.69e-4 -> 3.59e-4, with dout 100 times
+// smaller 3.75e-4 -> 3.70e-4; 1000 times smaller, where the gradient itself is mostly below the normal numbers of the type, 0.85e-3 ->
+// 1.09e-3.  dK/dV and dQ of 32768 tokens, 32 heads, top-k 16: 5060 us before and after.)
+template <typename T>
+__device__ __forceinline__ float dq_part_scale(float softmax_scale) {
+  return std::is_same_v<T, f16_t> ? fminf(softmax_scale, 1.f) : 1.f;
+}
+template <typename T>
+__device__ __forceinline__ float dq_sum_scale(float softmax_scale) {
+  return std::is_same_v<T, f16_t> ? fmaxf(softmax_scale, 1.f) : softmax_scale;
+}
+template <typename T>
+__device__ __forceinline__ uint2 pack4_scaled(float x, float y, float z, float w, float scale) {
+  if constexpr (std::is_same_v<T, f16_t>)
+    return make_uint2(pack2<T>(x * scale, y * scale), pack2<T>(z * scale, w * scale));
+  else
+    return make_uint2(pack2<T>(x, y), pack2<T>(z, w));
+}
 
 // ------------------------------------------------------------------------------------
 // dK / dV.  One workgroup per (64 keys, query heads that share them, sequence) walks the row lists of its heads, 64
@@ -390,7 +411,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
 #pragma unroll
           for (int g = 0; g < 4; ++g)
             lds_write_vec<uint2>(ldsOut + (uint32_t)(frow * RB + fh * 8) + (((uint32_t)((kq * NDW + d) * 4 + g) ^ psw) * 16u),
-                                 make_uint2(pack2<T>(dq[d][4 * g], dq[d][4 * g + 1]), pack2<T>(dq[d][4 * g + 2], dq[d][4 * g + 3])));
+                                 pack4_scaled<T>(dq[d][4 * g], dq[d][4 * g + 1], dq[d][4 * g + 2], dq[d][4 * g + 3], dq_part_scale<T>(a.softmax_scale)));
         arrived();
         __syncthreads();  // the part rows are there; the next round's rows are, and this one's are no longer read
 #pragma unroll
@@ -888,7 +909,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
     };
     // dQ of the tile: both waves of a pair put dS^T of their 32 keys into one LDS tile [64 keys][32 rows]; after a
     // barrier each wave computes dQ^T = K^T dS^T over all 64 keys for ITS half of the features.  The
-    // half rows (16-bit, unscaled) go to the partial slot that the row handed out for this visit.
+    // half rows (16-bit) go to the partial slot that the row handed out for this visit.
     auto ds_write = [&](auto tsc) {
       constexpr int TS = decltype(tsc)::value;
       // tile slot TS of the pair, rows of all keys of the block
@@ -935,7 +956,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
 #pragma unroll
         for (int g = 0; g < 4; ++g)
           lds_write_vec<uint2>(bw + SO + (uint32_t)((d2 * 32 + 8 * g) * 2),
-                               make_uint2(pack2<T>(dqa[d2][4 * g], dqa[d2][4 * g + 1]), pack2<T>(dqa[d2][4 * g + 2], dqa[d2][4 * g + 3])));
+                               pack4_scaled<T>(dqa[d2][4 * g], dqa[d2][4 * g + 1], dqa[d2][4 * g + 2], dqa[d2][4 * g + 3], dq_part_scale<T>(a.softmax_scale)));
       wave_lds_fence();
       constexpr int LPR = NDH * 4;        // lanes per part row (16 bytes each)
       constexpr int RPP = 64 / LPR;       // rows per pass
@@ -1550,9 +1571,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
     for (; t < n; ++t) add(ld_stream16(part + (int64_t)sOrd[t] * D + c8));
   }
   if (valid && mine) {
+    const float scale = dq_sum_scale<T>(a.softmax_scale);
     Pack8 o;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o.w[k] = pack2<T>(acc[2 * k] * a.softmax_scale, acc[2 * k + 1] * a.softmax_scale);
+    for (int k = 0; k < 4; ++k) o.w[k] = pack2<T>(acc[2 * k] * scale, acc[2 * k + 1] * scale);
     *reinterpret_cast<Pack8 *>(reinterpret_cast<uint16_t *>(a.dq) + row * a.dq_row_stride + (int64_t)h * a.dq_head_stride + c8) = o;
   }
 }

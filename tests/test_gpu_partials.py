@@ -49,3 +49,31 @@ def test_fp16_column_rows_keep_to_their_range(D, chunk, size):
     assert ((out.double() - exact).abs() <= tol).all()
     n = torch.arange(1, L + 1, device="cuda", dtype=torch.float64)
     assert ((lse.double() - n.log()).abs() <= 1e-5).all()
+
+
+# fp16 partial rows of dQ: 64 keys of one sign add up to several times 65504 before the softmax scale, not after it
+@pytest.mark.parametrize("D,chunk", [(64, 64), (40, 128), (96, 64), (128, 64), (128, 128)])
+@pytest.mark.parametrize("scale", [None, 2.0])  # (a scale above one must not take range away either)
+def test_fp16_dq_partial_rows_keep_to_their_range(D, chunk, scale):
+    L, H = 300, 2
+    val = 2000.0 if scale is None else 100.0
+    scale = scale or D ** -0.5
+    g = torch.Generator(device="cuda").manual_seed(D)
+    s = (torch.randint(0, 2, (L, H, 1), generator=g, device="cuda") * 2 - 1).half()
+    q, k, v = torch.zeros((L, H, D), device="cuda").half(), (2 * s).expand(L, H, D).contiguous(), (val * s).expand(L, H, D).contiguous()
+    dout = torch.ones_like(q)
+    cu = torch.tensor([0, L], dtype=torch.int32, device="cuda")
+    co, cn, ind = flash_moba.flash_topk_varlen_func(q, k, cu, cu, L, L, 5, chunk, causal=True)
+    csc = (co, cn, ind, cu, cu)
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *csc, None, None, None, L, L, 0.0, scale, False, True, 0.0, False, 128, chunk, None)
+    dq, _, _, _ = hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, *csc, None, L, L, 0.0, scale, False, True, 0.0, False, 128, chunk, None,
+                                      _dq_mode=2)
+    # P = 1 / n over the row's n keys, m the mean sign: dq = scale * sum_j (dP_j - delta) K_j / n, dP_j = val D s_j, delta = val D m
+    n = torch.arange(1, L + 1, device="cuda", dtype=torch.float64)[:, None, None]
+    m = s.double().cumsum(0) / n
+    size = scale * val * D * 2
+    exact = (size * (1 - m * m)).expand(L, H, D)
+    assert exact.max() < 65504 and exact.max() > 0.9 * size
+    # Rows of fewer than 8 keys are left out: dS itself, 16-bit in every form, is up to val D 2 / n, beyond 65504 for them.
+    # Roundings of out (in delta), P, dS, up to five partial rows and the result, each 2^-11 of at most `size`
+    assert ((dq.double() - exact)[7:].abs() <= 9 * 2.0 ** -11 * size).all()
