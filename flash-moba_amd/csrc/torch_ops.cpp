@@ -26,6 +26,7 @@
 #include <cmath>
 #include <optional>
 #include <tuple>
+#include <utility>
 
 #include "../../include/flash_moba_hip.h"
 
@@ -155,7 +156,8 @@ fmoba_attn_fwd_args forward_args(const Shape &s, const Tensor &q, const Tensor &
 struct Result {
   Tensor out, lse;
 };
-thread_local int t_visits = 0, t_row_blocks = 0;  // what this thread's last forward ran (diagnostics)
+// what this thread's last forward ran, and its last backward if nobody has asked since (else -1): diagnostics
+thread_local int t_visits = 0, t_row_blocks = 0, t_partials = -1;
 
 Result forward(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const Pattern &p) {
   Result r;
@@ -228,6 +230,7 @@ struct Attention : public torch::autograd::Function<Attention> {
       const Tensor ws = bytes_like(q, n);
       a.workspace = ws.data_ptr(), a.workspace_bytes = n;
       check(fmoba_attn_bwd_grouped(&a, dkv_heads, 7, s.stream));
+      t_partials = fmoba_attn_bwd_uses_partials(&a);
       if (grouped) {
         at::sum_out(dk, dk_e.view({s.total_k, s.heads_k, dkv_heads / s.heads_k, s.dim}), at::IntArrayRef{2});
         at::sum_out(dv, dv_e.view({s.total_k, s.heads_k, dkv_heads / s.heads_k, s.dim}), at::IntArrayRef{2});
@@ -368,6 +371,7 @@ py::object attn_varlen(const py::handle &hq, const py::handle &hk, const py::han
 }
 
 py::tuple last_forward() { return py::make_tuple(t_visits, t_row_blocks); }
+int take_last_backward() { return std::exchange(t_partials, -1); }
 
 }  // namespace
 
@@ -377,4 +381,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("topk_varlen", &topk_varlen);
   m.def("attn_varlen", &attn_varlen);
   m.def("last_forward", &last_forward);
+  m.def("take_last_backward", &take_last_backward);
 }

@@ -362,7 +362,12 @@ def last_fwd_row_blocks():
 
 
 def last_bwd_partials():
-    """1 if the last backward of this thread formed dQ from per-visit partials, 0 for the row-block form."""
+    """1 if the last backward of this thread formed dQ from per-visit partials, 0 for the row-block form.  (The backward of
+    a call under autograd runs on the engine's thread.)"""
+    if _host is not None:
+        native = _host.take_last_backward()
+        if native >= 0:
+            _last.bwd_partials = native
     return int(getattr(_last, "bwd_partials", 0))
 
 
@@ -578,6 +583,8 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
             a.dk, a.dk_row_stride, a.dk_head_stride = dk_e.data_ptr(), dk_e.stride(0), dk_e.stride(1)
             a.dv, a.dv_row_stride, a.dv_head_stride = dv_e.data_ptr(), dv_e.stride(0), dv_e.stride(1)
         ws_bytes = lib.fmoba_attn_bwd_workspace_bytes(ctypes.byref(a))
+        if _host is not None:
+            _host.take_last_backward()  # (an earlier backward of the eager host path is no longer the last one)
         _last.bwd_partials = int(lib.fmoba_attn_bwd_uses_partials(ctypes.byref(a)))
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes

@@ -79,3 +79,21 @@ def test_dual_tensors_are_refused(which, two_step):
                 flash_moba.flash_moba_attn_varlen_func(*qkv, cu, cu, 200, 200, *pattern, lg_block_m=128, lg_block_n=64, causal=True)
             else:
                 flash_moba.flash_moba_varlen_func(*qkv, cu, cu, 200, 200, 64, 2)
+
+
+def test_the_form_of_the_last_backward_is_reported(monkeypatch):
+    def step(L, chunk, topk):
+        x = [torch.randn((L, 1, 128), device="cuda").to(torch.bfloat16).requires_grad_(True) for _ in range(3)]
+        cu = torch.tensor([0, L], dtype=torch.int32, device="cuda")
+        seen = []
+        x[0].register_hook(lambda g: seen.append(hip.last_bwd_partials()))  # (on the engine's thread, as the backward)
+        flash_moba.flash_moba_varlen_func(*x, cu, cu, L, L, chunk, topk).sum().backward()
+        return seen
+
+    with monkeypatch.context() as m:
+        m.setattr(hip, "host_module", lambda: _NoHost())
+        assert step(8192, 128, 4) == [1] and step(512, 64, 4) == [0]
+    assert step(8192, 128, 4) == [1] and step(512, 64, 4) == [0]
+    with monkeypatch.context() as m:
+        m.setattr(hip, "host_module", lambda: _NoHost())
+        assert step(8192, 128, 4) == [1] and step(512, 64, 4) == [0]
