@@ -180,7 +180,7 @@ struct Attention : public torch::autograd::Function<Attention> {
   // the pattern and the results of the forward pass are made by the caller, below autograd; this records them
   static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu_q, const Tensor &cu_k,
                         const Pattern &p, const Result &r, int64_t max_q, int64_t max_k, int64_t chunk, bool causal, double scale, int64_t bwd_visits,
-                        int64_t dq_mode, bool deterministic) {
+                        bool deterministic) {
     ctx->save_for_backward({q, k, v, r.out, r.lse, cu_q, cu_k, p.col_offsets, p.col_nnz, p.indices});
     ctx->saved_data["max_q"] = max_q;
     ctx->saved_data["max_k"] = max_k;
@@ -188,7 +188,6 @@ struct Attention : public torch::autograd::Function<Attention> {
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["visits"] = bwd_visits;
-    ctx->saved_data["dq_mode"] = dq_mode;
     ctx->saved_data["deterministic"] = deterministic;
     return r.out;
   }
@@ -197,7 +196,7 @@ struct Attention : public torch::autograd::Function<Attention> {
     const variable_list t = ctx->get_saved_variables();
     const Tensor &q = t[0], &k = t[1], &v = t[2], &out = t[3], &lse = t[4], &cu_q = t[5], &cu_k = t[6], &co = t[7], &cn = t[8], &ind = t[9];
     auto num = [&](const char *name) { return ctx->saved_data[name].toInt(); };
-    variable_list res(15);  // one per argument of forward
+    variable_list res(14);  // one per argument of forward
     {
       at::AutoDispatchBelowADInplaceOrView below;
       const c10::DeviceGuard guard(q.device());
@@ -212,7 +211,7 @@ struct Attention : public torch::autograd::Function<Attention> {
       a.batch = s.batch, a.total_q = s.total_q, a.total_k = s.total_k, a.heads = s.heads, a.heads_k = s.heads_k, a.head_dim = s.dim;
       a.max_seqlen_q = s.max_q, a.max_seqlen_k = s.max_k, a.max_cols = co.size(2), a.lg_block_m = 128, a.lg_block_n = s.chunk;
       a.is_causal = s.causal && s.max_q != 1, a.dtype = s.dtype, a.deterministic = ctx->saved_data["deterministic"].toBool();
-      a.max_visits_per_row = num("visits"), a.dq_mode = num("dq_mode"), a.softmax_scale = static_cast<float>(ctx->saved_data["scale"].toDouble());
+      a.max_visits_per_row = num("visits"), a.softmax_scale = static_cast<float>(ctx->saved_data["scale"].toDouble());
       // heads of a group that the library does not add up itself are summed below (flash_moba_api.cpp:842-845)
       const int32_t dkv_heads = fmoba_attn_bwd_dkv_heads(&a);
       const bool grouped = dkv_heads != s.heads_k;
@@ -278,7 +277,7 @@ py::object moba_varlen(const py::handle &hq, const py::handle &hk, const py::han
       a.selection_bits = p.selection;
       r = forward(s, a, q, p);
     }
-    out = grad ? Attention::apply(q, k, v, cu_q, cu_k, p, r, max_q, max_k, chunk, causal, scale, visits * (kb / 64), 0, false) : r.out;
+    out = grad ? Attention::apply(q, k, v, cu_q, cu_k, p, r, max_q, max_k, chunk, causal, scale, visits * (kb / 64), false) : r.out;
   }
   return py::reinterpret_steal<py::object>(THPVariable_Wrap(out));
 }
@@ -312,6 +311,8 @@ int64_t count_visits(const fmoba_attn_fwd_args &a, const Tensor &q, void *stream
   return std::max<int64_t>(1, counts.select(0, rows).item<int32_t>());
 }
 
+constexpr size_t kUncountedBytes = size_t(8) << 30;
+
 // flash_moba_attn_varlen_func over a pattern of the caller's own
 py::object attn_varlen(const py::handle &hq, const py::handle &hk, const py::handle &hv, const py::handle &hcq, const py::handle &hck, int64_t max_q,
                        int64_t max_k, const py::handle &hco, const py::handle &hcn, const py::handle &hind, int64_t lg_m, int64_t lg_n,
@@ -335,24 +336,26 @@ py::object attn_varlen(const py::handle &hq, const py::handle &hk, const py::han
   const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
   const double scale = softmax_scale ? *softmax_scale : std::pow(static_cast<double>(s.dim), -0.5);
   const int kb = fmoba_attn_fwd_key_block(lg_n);
-  // The forms are chosen by the mean number of chunks a row selects (at most list entries per row and head); a bound for
-  // every row, which takes a pass over the lists and a read-back, is needed only by the forms that size partial results
-  // by it.
-  const int64_t mean = std::max<int64_t>(1, (p.indices.numel() + s.total_q * s.heads - 1) / (s.total_q * s.heads));
-  int64_t visits = std::min<int64_t>(mean, s.max_cols) * (lg_n / kb), dq_mode = 0;
+  // The largest number of visits of a row takes a pass over the lists and a read-back (12037 tokens, 16 heads of 96, 8 of 64-key
+  // chunks, forward and backward: a fifth of the call).  It is left out where it cannot change anything: the rules of both forms
+  // turn to row blocks and dS tiles as rows get denser, so if the mean (at most list entries per row and head) says so, the
+  // maximum does too; and these forms need no bound.  List storage that is larger than the lists raises the mean: dS tiles
+  // are sized by the storage, hence the limit on them.
+  const int64_t rows = s.total_q * s.heads, mean = std::max<int64_t>(1, (p.indices.numel() + rows - 1) / rows);
+  int64_t visits = std::min<int64_t>(mean, s.max_cols) * (lg_n / kb);
   fmoba_attn_fwd_args a = forward_args(s, q, k, v, cu_q, cu_k, visits, scale, nullptr);
   a.col_offsets = p.col_offsets.data_ptr<int64_t>(), a.col_nnz = p.col_nnz.data_ptr<int32_t>(), a.row_indices = p.indices.data_ptr<int32_t>();
-  a.fwd_mode = fmoba_attn_fwd_uses_row_blocks(&a) ? 2 : 1;
+  const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+  bool count = !fmoba_attn_fwd_uses_row_blocks(&a);
   if (grad) {
     fmoba_attn_bwd_args b{};
     b.batch = s.batch, b.total_q = s.total_q, b.total_k = s.total_k, b.heads = s.heads, b.heads_k = s.heads_k, b.head_dim = s.dim;
     b.max_seqlen_q = s.max_q, b.max_seqlen_k = s.max_k, b.max_cols = s.max_cols, b.lg_block_n = lg_n, b.is_causal = a.is_causal;
-    b.max_visits_per_row = visits * (kb / 64);
-    dq_mode = fmoba_attn_bwd_uses_partials(&b) ? 2 : 1;
+    b.max_visits_per_row = visits * (kb / 64), b.num_row_indices = p.indices.numel();
+    count = count || fmoba_attn_bwd_uses_partials(&b) || (!capturing && fmoba_attn_bwd_workspace_bytes(&b) > kUncountedBytes);
   }
-  const bool count = a.fwd_mode == 1 || dq_mode == 2;
   // (nothing can be read back while a graph is captured)
-  if (count && c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return none();
+  if (count && capturing) return none();
   Tensor out;
   {
     py::gil_scoped_release nogil;
@@ -365,7 +368,7 @@ py::object attn_varlen(const py::handle &hq, const py::handle &hk, const py::han
       if (count) a.max_visits_per_row = visits = count_visits(a, q, s.stream);
       r = forward(s, a, q, p);
     }
-    out = grad ? Attention::apply(q, k, v, cu_q, cu_k, p, r, max_q, max_k, lg_n, causal, scale, visits * (kb / 64), dq_mode, deterministic) : r.out;
+    out = grad ? Attention::apply(q, k, v, cu_q, cu_k, p, r, max_q, max_k, lg_n, causal, scale, visits * (kb / 64), deterministic) : r.out;
   }
   return py::reinterpret_steal<py::object>(THPVariable_Wrap(out));
 }

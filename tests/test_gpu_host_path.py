@@ -97,3 +97,49 @@ def test_the_form_of_the_last_backward_is_reported(monkeypatch):
     with monkeypatch.context() as m:
         m.setattr(hip, "host_module", lambda: _NoHost())
         assert step(8192, 128, 4) == [1] and step(512, 64, 4) == [0]
+
+
+def _csc(sel):
+    """(heads, rows, chunks) bool of one sequence -> col_offsets, col_nnz, indices."""
+    cn = sel.sum(1, dtype=torch.int32)
+    co = cn.flatten().cumsum(0).view_as(cn).long() - cn
+    return co[None].contiguous(), cn[None].contiguous(), sel.transpose(1, 2).nonzero()[:, 2].int().contiguous()
+
+
+# The form, and what is allocated for it, goes by the row with the most chunks: a global token among sparse rows (the forward goes
+# to row blocks, the partial rows of columns would be sized for every row by that one), rows of one density, and lists that lie in
+# storage of several times their length
+@pytest.mark.parametrize("D,L,chunk,others,dense,pad,rows_form", [
+    (64, 4096, 64, 1, 1, 1, 1), (128, 4096, 64, 1, 1, 1, 1), (96, 4096, 128, 1, 2, 1, 1), (128, 4096, 64, 1, 0, 1, 0), (128, 2048, 64, 12, 0, 1, 1),
+    (256, 2048, 64, 1, 1, 1, 0), (128, 4096, 64, 1, 0, 30, 1)])
+def test_the_densest_row_decides_the_form(monkeypatch, D, L, chunk, others, dense, pad, rows_form):
+    H, C = 2, L // chunk
+    g = torch.Generator(device="cuda").manual_seed(D + others)
+    own = (torch.arange(L, device="cuda") // chunk)[:, None]
+    c = torch.arange(C, device="cuda")[None]
+    sel = (c == own).repeat(H, 1, 1)
+    for j in range(others):
+        sel |= c == (torch.arange(L, device="cuda")[:, None] * 7 + 5 * j) % (own + 1)
+    sel[:, L - 1 - torch.arange(dense, device="cuda")] = True
+    sel &= c <= own
+    co, cn, ind = _csc(sel)
+    ind = torch.cat([ind, ind.new_zeros((pad - 1) * ind.numel())])
+    cu = torch.tensor([0, L], dtype=torch.int32, device="cuda")
+    q, k, v, dout = (torch.randn((L, H, D), generator=g, device="cuda").to(torch.bfloat16) for _ in range(4))
+
+    def call():
+        qg, kg, vg = (t.clone().requires_grad_(True) for t in (q, k, v))
+        out = flash_moba.flash_moba_attn_varlen_func(qg, kg, vg, cu, cu, L, L, co, cn, ind, lg_block_m=128, lg_block_n=chunk, causal=True)
+        res = [hip.last_fwd_row_blocks()]
+        return res, (out.detach(), *torch.autograd.grad(out, (qg, kg, vg), dout))
+
+    form, got = call()
+    with monkeypatch.context() as m:
+        m.setattr(hip, "host_module", lambda: _NoHost())
+        _, want = call()
+    assert form == [rows_form]
+    for x, y in zip(got, want):
+        if pad == 1:
+            assert torch.equal(x, y)
+        else:  # (another form of the same sums: a partial result or two of a row are rounded to bf16 in one of them)
+            assert (x.float() - y.float()).norm() <= 2.0 ** -7 * y.float().norm()
