@@ -509,8 +509,17 @@ __global__ __launch_bounds__(256) void max_i32_kernel(const int32_t *p, int64_t 
 
 static inline size_t fwd_align256(size_t x) { return (x + 255) & ~(size_t)255; }
 static inline int fwd_key_block(int lg_block_n) { return lg_block_n % 128 == 0 ? 128 : 64; }
-// partial slots per (row, head)
-static inline int64_t fwd_partial_cap(const fmoba_attn_fwd_args &a) { return a.max_visits_per_row; }
+// partial slots per (row, head): above head dimension 128, where dense patterns come here too, no more than a sequence has key blocks
+// (top-k times the chunk can be far beyond the keys of a short sequence)
+static inline int64_t fwd_partial_cap(const fmoba_attn_fwd_args &a) {
+  const int64_t visits = a.max_visits_per_row;
+  return a.head_dim > 128 ? std::min(visits, std::max<int64_t>(1, ceil_div64(a.max_seqlen_k, fwd_key_block(a.lg_block_n)))) : visits;
+}
+// the combine keeps the order of sixteen rows' partial results in LDS, beside two 16 x 16 tables
+constexpr int kCombineStaticLds = 2 * 16 * 16 * 4;
+static inline bool fwd_combine_fits(const fmoba_attn_fwd_args &a) {
+  return (fwd_partial_cap(a) + 15) / 16 * 16 * 64 + kCombineStaticLds <= 160 * 1024;
+}
 
 // the row-block form (attn_fwd_rows.hip)
 bool fwd_rows_feasible(const fmoba_attn_fwd_args &a);
@@ -528,10 +537,11 @@ static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   if (a.fwd_mode == 2 || fwd_few_rows(a)) return true;
   // Head dimensions above 128: the column form is the faster one at every density that was measured (columns against rows:
   // 2 x 4096 tokens, 8 heads of 256, top-k 8 of 128-key chunks 269 against 976 us, top-k 32 of 64-key chunks 731 against 976;
-  // 16384 tokens, top-k 32 of 64-key chunks 1793 against 6918), up to the size of the partial results that a call may ask for.
+  // 16384 tokens, top-k 32 of 64-key chunks 1793 against 6918), up to the size of the partial results that a call may ask for
+  // and to what the combine has room for.
   if (a.head_dim > 128) {
     const int64_t partials = (int64_t)a.total_q * a.heads * fwd_partial_cap(a);
-    return partials >= ((int64_t)1 << 31) || partials * (int64_t)(a.head_dim * fwd_part_size(a.head_dim) + 16) > kWidePartialBytes;
+    return !fwd_combine_fits(a) || partials >= ((int64_t)1 << 31) || partials * (int64_t)(a.head_dim * fwd_part_size(a.head_dim) + 16) > kWidePartialBytes;
   }
   const int64_t chunks_per_seq = std::max<int64_t>(1, ceil_div64(ceil_div64(std::max(a.total_k, 1), a.batch), a.lg_block_n));
   const int64_t chunks_per_row = std::max<int64_t>(1, (int64_t)a.max_visits_per_row * fwd_key_block(a.lg_block_n) / a.lg_block_n);

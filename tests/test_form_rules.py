@@ -36,3 +36,19 @@ def test_dq_lines(D, chunk, topk, partials):
     a.head_dim, a.batch, a.lg_block_n, a.is_causal = D, 1, chunk, 1
     a.max_visits_per_row = topk * (chunk // 64)
     assert H.load_library().fmoba_attn_bwd_uses_partials(ctypes.byref(a)) == partials
+
+
+# above head dimension 128 the partial results of a row are bounded by the key blocks of a sequence, whatever top-k times the chunk
+# is, and calls whose rows still have more of them than the combine can order go to row blocks
+def test_wide_heads_partial_results_are_bounded_by_the_sequence():
+    lib = H.load_library()
+    f = fwd_args([512], 4096, 64, heads=2, D=256)
+    assert lib.fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == 0
+    assert lib.fmoba_attn_fwd_workspace_bytes(ctypes.byref(f)) < 512 * 2 * 4 * (4 * 256 + 16) + 8192
+    f = fwd_args([512], 64 * 129, 64, heads=2, D=256)
+    f.total_k = f.max_seqlen_k = 200000
+    f.max_cols = 25
+    assert lib.fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == 1
+    f.total_k = f.max_seqlen_k = 160000
+    f.max_cols = 20
+    assert lib.fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == 0

@@ -77,3 +77,11 @@ def test_fp16_dq_partial_rows_keep_to_their_range(D, chunk, scale):
     # Rows of fewer than 8 keys are left out: dS itself, 16-bit in every form, is up to val D 2 / n, beyond 65504 for them.
     # Roundings of out (in delta), P, dS, up to five partial rows and the result, each 2^-11 of at most `size`
     assert ((dq.double() - exact)[7:].abs() <= 9 * 2.0 ** -11 * size).all()
+
+
+@pytest.mark.parametrize("D", [136, 256])
+@pytest.mark.parametrize("chunk", [8192, 64 * 129])
+def test_wide_heads_with_chunks_far_longer_than_the_sequence(D, chunk):
+    q, k, v, cu, exact = _uniform_rows(500, 2, D, torch.bfloat16, 1.0, D)
+    out = flash_moba.flash_moba_varlen_func(q, k, v, cu, cu, 500, 500, chunk, 64, causal=True)
+    assert ((out.double() - exact).abs() <= _HALF_ULP[torch.bfloat16] * exact).all()
