@@ -193,8 +193,22 @@ struct Attention : public torch::autograd::Function<Attention> {
   }
 
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
-    const variable_list t = ctx->get_saved_variables();
+    variable_list t = ctx->get_saved_variables();
     const Tensor &q = t[0], &k = t[1], &v = t[2], &out = t[3], &lse = t[4], &cu_q = t[5], &cu_k = t[6], &co = t[7], &cn = t[8], &ind = t[9];
+    // What was saved may have been through saved-tensor hooks: nothing of it is taken on trust, as its addresses go to kernels.
+    TORCH_CHECK(q.defined() && q.is_cuda(), "flash_moba: a saved tensor is not on the GPU");
+    const at::Device dev = q.device();
+    const at::ScalarType dt = q.scalar_type();
+    for (int i = 0; i < 4; ++i) {
+      TORCH_CHECK(t[i].defined() && t[i].device() == dev && t[i].scalar_type() == dt && t[i].dim() == 3, "flash_moba: q, k, v or out was saved and came back as another tensor");
+      if (!is_rows(t[i], dt, dev)) t[i] = t[i].contiguous();
+    }
+    TORCH_CHECK(out.sizes() == q.sizes() && v.sizes() == k.sizes(), "flash_moba: q, k, v or out was saved and came back in another shape");
+    const int64_t nb = cu_q.defined() ? cu_q.numel() - 1 : 0;
+    auto is = [&](const Tensor &x, at::ScalarType type) { return x.defined() && x.device() == dev && x.scalar_type() == type && x.is_contiguous(); };
+    TORCH_CHECK(is(lse, at::kFloat) && lse.dim() == 2 && lse.size(0) == q.size(1) && lse.size(1) == q.size(0) && is(cu_q, at::kInt) && is(cu_k, at::kInt) &&
+                    is(co, at::kLong) && is(cn, at::kInt) && is(ind, at::kInt) && co.dim() == 3 && co.sizes() == cn.sizes() && co.size(0) == nb && co.size(1) == q.size(1),
+                "flash_moba: the pattern, the offsets or the log-sum-exp was saved and came back as another tensor");
     auto num = [&](const char *name) { return ctx->saved_data[name].toInt(); };
     variable_list res(14);  // one per argument of forward
     {
@@ -204,8 +218,8 @@ struct Attention : public torch::autograd::Function<Attention> {
       TORCH_CHECK(common_form(s, q, k, cu_q, cu_k, num("max_q"), num("max_k"), num("chunk"), ctx->saved_data["causal"].toBool()), "flash_moba: saved tensors changed");
       s.stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
       Tensor dout = grads[0];
-      TORCH_CHECK(dout.defined(), "flash_moba: no gradient");
-      if (!is_rows(dout, q.scalar_type(), q.device())) dout = dout.to(q.scalar_type()).contiguous();
+      TORCH_CHECK(dout.defined() && dout.sizes() == q.sizes() && dout.device() == dev, "flash_moba: no gradient of the shape of the output");
+      if (!is_rows(dout, dt, dev)) dout = dout.to(dt).contiguous();
       Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
       fmoba_attn_bwd_args a{};
       a.batch = s.batch, a.total_q = s.total_q, a.total_k = s.total_k, a.heads = s.heads, a.heads_k = s.heads_k, a.head_dim = s.dim;

@@ -143,3 +143,38 @@ def test_the_densest_row_decides_the_form(monkeypatch, D, L, chunk, others, dens
             assert torch.equal(x, y)
         else:  # (another form of the same sums: a partial result or two of a row are rounded to bf16 in one of them)
             assert (x.float() - y.float()).norm() <= 2.0 ** -7 * y.float().norm()
+
+
+def _step_with_hooks(pack, unpack, seed=5, make=None):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = [torch.randn((700, 4, 64), generator=g, device="cuda").to(torch.bfloat16) for _ in range(4)]
+    q, k, v = (t.clone().requires_grad_(True) for t in x[:3])
+    cu = torch.tensor([0, 300, 700], dtype=torch.int32, device="cuda")
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        out = flash_moba.flash_moba_varlen_func(q, k, v, cu, cu, 400, 400, 64, 3)
+    return (out.detach(), *torch.autograd.grad(out, (q, k, v), x[3]))
+
+
+def _spread(t):
+    """The same values with twice the distance between rows, at an address that is no multiple of 16."""
+    if t.dim() != 3 or t.dtype != torch.bfloat16:
+        return t
+    buf = torch.empty((t.shape[0], 2 * t.shape[1], t.shape[2] + 4), dtype=t.dtype, device=t.device)
+    return buf[:, ::2, 4:].copy_(t)
+
+
+# tensors that come back from saved-tensor hooks: anywhere in memory and with any strides they give the same gradients,
+# on the CPU, in another type or in another shape they are refused (their addresses would go to kernels)
+def test_saved_tensor_hooks():
+    want = _step_with_hooks(lambda t: t, lambda t: t)
+    for pack, unpack in ((lambda t: t.cpu(), lambda t: t.cuda()), (lambda t: t, _spread), (lambda t: t.clone(), lambda t: t)):
+        assert all(torch.equal(x, y) for x, y in zip(_step_with_hooks(pack, unpack), want))
+    with torch.autograd.graph.save_on_cpu():
+        assert all(torch.equal(x, y) for x, y in zip(_step_with_hooks(lambda t: t, lambda t: t), want))
+
+
+@pytest.mark.parametrize("unpack", [lambda t: t.cpu(), lambda t: t.float() if t.is_floating_point() else t, lambda t: t.long(), lambda t: t[:-1],
+                                    lambda t: t.cpu() if t.dim() == 2 else t, lambda t: t[:, :1] if t.dtype == torch.int64 else t])
+def test_saved_tensors_that_come_back_as_others_are_refused(unpack):
+    with pytest.raises(RuntimeError):
+        _step_with_hooks(lambda t: t, unpack)
