@@ -54,3 +54,35 @@ def test_attention_of_a_few_rows(lens_q, lens_k, chunk, topk, H, Hk, D, dtype):
     assert torch.equal(out, out2)
     assert_close("out", out, cols.float().cpu(), 2e-2, 1e-2)
     assert_close("lse", lse2, lse.float().cpu(), 2e-3, 1e-3)
+
+
+# scores that are infinite or not a number: a candidate needs a score above -inf, +inf comes first, ties go to the higher chunk
+@pytest.mark.parametrize("lens_k,chunk,topk", [([2048, 700], 64, 5), ([64 * 257 + 3, 64 * 40], 64, 33), ([5000, 1500], 2, 16), ([2048, 900], 64, 64)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D", [64, 256])
+def test_gate_with_infinite_scores_and_without_numbers(lens_k, chunk, topk, causal, D):
+    lens_q, H, Hk = [3, 8], 4, 2
+    q, k, _, cuq, cuk = (t.cuda() for t in _case(lens_q, lens_k, H, Hk, D, torch.bfloat16, topk, integer=True))
+    km, cu_km, _ = flash_topk_mean_pool(k, cuk, max(lens_k), chunk)
+    g = torch.Generator(device="cuda").manual_seed(topk)
+    km.copy_(torch.randint(-2, 3, km.shape, generator=g, device="cuda"))
+    q[:, :, 0] = torch.where(torch.rand(q.shape[:2], generator=g, device="cuda") < 0.5, 1.0, -1.0).to(q.dtype)
+    kind = torch.randint(0, 8, km.shape[:2], generator=g, device="cuda")
+    for i, special in enumerate((float("inf"), float("-inf"), float("nan"))):
+        km[:, :, 0] = torch.where(kind == i, special, km[:, :, 0].float()).to(km.dtype)
+    q[1] = float("nan")  # (a row without a score at all)
+    words = hip.moba_fused_topk(q, km, cuq, cuk, cu_km, 8, max(lens_k), topk, chunk, causal, return_raw=False, return_selection=True)[5].cpu()
+    C = -(-max(lens_k) // chunk)
+    got = (words[:, torch.arange(C) // 32, :] >> (torch.arange(C) % 32)[None, :, None]) & 1  # heads, chunks, rows
+    kpos = cu_km.cpu().tolist()
+    row = 0
+    for b, (nq, nk) in enumerate(zip(lens_q, lens_k)):
+        for i in range(nq):
+            pos = i + nk - nq
+            n = pos // chunk if causal else kpos[b + 1] - kpos[b]
+            for h in range(H):
+                score = (km[kpos[b]:kpos[b] + n, h // (H // Hk)].double().cpu() @ q[row, h].double().cpu()).tolist()
+                order = sorted((c for c in range(n) if score[c] > float("-inf")), key=lambda c: (-score[c], -c))
+                want = set(order[:topk - 1] + [pos // chunk] if causal else order[:topk])
+                assert set(got[h, :, row].nonzero().flatten().tolist()) == want, (b, i, h)
+            row += 1

@@ -178,3 +178,59 @@ def test_saved_tensor_hooks():
 def test_saved_tensors_that_come_back_as_others_are_refused(unpack):
     with pytest.raises(RuntimeError):
         _step_with_hooks(lambda t: t, unpack)
+
+
+def _layouts(name, q, k, v, dout):
+    """The same values as views: slices of one projection, head-major storage, rows at twice their distance, one row for all."""
+    T, H, D = q.shape
+    if name == "packed":
+        q, k, v = torch.stack((q, k, v), 1).unbind(1)
+        dout = torch.stack((dout, dout), 1)[:, 1]
+    elif name == "head_major":
+        q, k, v, dout = (t.transpose(0, 1).contiguous().transpose(0, 1) for t in (q, k, v, dout))
+    elif name == "spread":
+        q, k, v, dout = (torch.cat((t, t), 2)[:, :, D:] for t in (q, k, v, dout))
+    elif name == "expanded":  # (a gradient of stride 0, as a sum leaves it)
+        dout = dout[:1, :, :1].expand(T, H, D)
+    return q, k, v, dout
+
+
+# strides of every kind give the bits of the packed call, natively and through the ops, forward and backward; and so does a call on
+# another stream than the inputs were made on
+@pytest.mark.parametrize("layout", ["packed", "head_major", "spread", "expanded"])
+@pytest.mark.parametrize("L,H,D,chunk,topk", [(900, 4, 64, 64, 3), (8192, 2, 128, 128, 4), (700, 2, 256, 64, 3)])
+@pytest.mark.parametrize("stream", [False, True])
+def test_strided_inputs(monkeypatch, layout, L, H, D, chunk, topk, stream):
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    x = [torch.randn((L, H, D), generator=g, device="cuda").to(torch.bfloat16) for _ in range(4)]
+    if layout == "expanded":
+        x[3] = x[3][:1, :, :1].expand(L, H, D).contiguous()
+    cu = torch.tensor([0, L // 3, L], dtype=torch.int32, device="cuda")
+    where = (cu, cu, L - L // 3, L - L // 3)
+
+    def step(q, k, v, dout):
+        q, k, v = (t.detach().requires_grad_(True) for t in (q, k, v))
+        out = flash_moba.flash_moba_varlen_func(q, k, v, *where, chunk, topk, causal=True)
+        pattern = flash_moba.flash_topk_varlen_func(q, k, *where, topk, chunk, causal=True)
+        out2 = flash_moba.flash_moba_attn_varlen_func(q, k, v, *where, *pattern, lg_block_m=128, lg_block_n=chunk, causal=True)
+        return (out.detach(), *torch.autograd.grad(out, (q, k, v), dout), out2.detach(), *torch.autograd.grad(out2, (q, k, v), dout))
+
+    want = step(*x)
+    views = _layouts(layout, *x)
+    s = torch.cuda.Stream() if stream else torch.cuda.current_stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        got = _both(monkeypatch, lambda: step(*views))
+    torch.cuda.current_stream().wait_stream(s)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_inputs_off_16_bytes_stay_refused(monkeypatch):
+    x = [torch.randn((300, 2, 64), device="cuda").to(torch.bfloat16) for _ in range(3)]
+    cu = torch.tensor([0, 300], dtype=torch.int32, device="cuda")
+    for host in (hip.host_module(), _NoHost()):
+        monkeypatch.setattr(hip, "host_module", lambda: host)
+        for i in range(3):
+            y = [_spread(t) if i == j else t for j, t in enumerate(x)]
+            with pytest.raises(RuntimeError, match="aligned"):
+                flash_moba.flash_moba_varlen_func(*y, cu, cu, 300, 300, 64, 2)

@@ -85,3 +85,27 @@ def test_wide_heads_with_chunks_far_longer_than_the_sequence(D, chunk):
     q, k, v, cu, exact = _uniform_rows(500, 2, D, torch.bfloat16, 1.0, D)
     out = flash_moba.flash_moba_varlen_func(q, k, v, cu, cu, 500, 500, chunk, 64, causal=True)
     assert ((out.double() - exact).abs() <= _HALF_ULP[torch.bfloat16] * exact).all()
+
+
+# both widths of a key block above head dimension 128 (eight waves for 128 keys, four for 64) against the row-block form: lists shorter
+# than a tile and than a wave each, uneven tails, heads of a group in one workgroup
+@pytest.mark.parametrize("D,dtype", [(136, torch.bfloat16), (192, torch.float16), (256, torch.bfloat16)])
+@pytest.mark.parametrize("chunk,topk", [(64, 3), (128, 2), (128, 6), (192, 2), (256, 2)])
+@pytest.mark.parametrize("H,Hk", [(2, 2), (6, 2), (8, 1)])
+def test_wide_columns_against_row_blocks(D, dtype, chunk, topk, H, Hk):
+    lens = [1, 0, 127, 129, 33, 1200]
+    T, L = sum(lens), max(lens)
+    g = torch.Generator(device="cuda").manual_seed(D + chunk + H)
+    q, k, v = (torch.randn((T, h, D), generator=g, device="cuda").to(dtype) for h in (H, Hk, Hk))
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device="cuda")
+    co, cn, ind = flash_moba.flash_topk_varlen_func(q, k, cu, cu, L, L, topk, chunk, causal=True)
+    run = lambda form: hip.moba_varlen_fwd(q, k, v, None, co, cn, ind, cu, cu, None, None, None, L, L, 0.0, D ** -0.5, False, True, 0.0, False, 128, chunk,
+                                           None, _fwd_mode=form)[:2]
+    (out, lse), (want, want_lse) = run(1), run(2)
+    # probabilities (relative to different maxima) and results are rounded to 16 bits in both
+    step = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert (out.float() - want.float()).norm() <= step * want.float().norm()
+    assert (out.float() - want.float()).abs().max() <= 4 * step * v.float().abs().max()
+    assert (lse - want_lse).abs().max() <= 1e-5 * want_lse.abs().max()
+    again = run(1)
+    assert torch.equal(again[0], out) and torch.equal(again[1], lse)
