@@ -3,7 +3,8 @@
 //   bwd_prep_kernel      : delta[row] = sum_d dO*O (fp32).
 //   attn_bwd_dkdv_kernel : COLUMN-stationary.  One workgroup per (64-key block, query heads that share it,
 //                          sequence) keeps K and V of the block in registers and walks the block's
-//                          ascending row lists in rounds of 64 gathered rows:
+//                          ascending row lists in rounds of 64 gathered rows (head dimensions up to
+//                          128; above: attn_bwd_wide.hip):
 //                            S = Q K^T, dP = dO V^T
 //                            P = exp2(S*scale*log2e - LSE*log2e), dS = P o (dP - delta)
 //                            dV^T += dO^T P, dK^T += Q^T dS     (transposing LDS reads)
@@ -13,8 +14,8 @@
 //                          row-list position) or, per visit, a dQ partial row (16-bit; fp16: scaled) in a
 //                          slot that the row hands out from a counter.
 //   attn_bwd_dkdv_partials_kernel : the same for the long calls, dQ partials at head dimension 128.
-//   attn_bwd_dq_kernel   : dQ from the dS tiles, one workgroup per 128 query rows, dQ in registers
-//                          (patterns in which a 128-row block meets a dozen rows or more per step).
+//   attn_bwd_dq_kernel   : dQ from the dS tiles, one workgroup per 256 query rows, dQ in registers
+//                          (patterns in which a row block meets a dozen rows or more per step).
 //   attn_bwd_dq_combine_kernel : dQ from the partials, sixteen lanes per (row, head) add them in ascending
 //                          key-block order and scales.  Work and traffic are proportional to
 //                          the number of visits, whatever the number of chunks per sequence.
@@ -1317,9 +1318,9 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[rt][dt][i] = 0.f;
-  // Which rows a wave owns: the waves w and w + 4 share a SIMD, and under the causal rule the later rows of the block
-  // take part in more steps (the first wave's rows sit out the block's last seven key blocks, the last wave's none), so
-  // a SIMD gets the rows w and 7 - w: the four SIMDs then have the same number of products to do.
+  // Which rows a wave owns.  With eight waves w and w + 4 share a SIMD, and under the causal rule the later rows of the block
+  // take part in more steps, so a SIMD gets the row tiles w and 7 - w: the four SIMDs then have the same number of products
+  // to do.  With four waves each has a SIMD of its own (and shares it with a wave of another workgroup): tiles in order.
   const int wtile = wave < 4 ? wave : 11 - wave;
   int myrow[RT];
 #pragma unroll

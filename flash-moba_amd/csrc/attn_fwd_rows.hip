@@ -7,10 +7,11 @@
 // part in the matrix products of a step, and the rows that did not select the chunk are masked out
 // of the softmax (their probabilities are exact zeros).  The running maximum, the running sum and
 // the output accumulators stay in registers for the whole walk, so nothing but Q, K, V and the
-// output moves.  Two kernels: attn_fwd_rows_kernel (256 rows, eight compute waves that fetch the
-// K/V tiles straight into LDS themselves; head dimensions up to 128 and up to 512 chunks per
-// sequence) and attn_fwd_rows_loader_kernel (128 rows, four compute and four loader waves; every
-// other shape, head dimension 256 included).
+// output moves.  Two kernels of 128 rows per workgroup: attn_fwd_rows_kernel (four compute waves, or two
+// sets of four, that fetch the K/V tiles straight into LDS themselves; head dimensions up to 128 and up to
+// 512 chunks per sequence) and attn_fwd_rows_loader_kernel (four compute and four loader waves; every
+// other shape, head dimension 256 included).  Calls with at most eight query rows per sequence have a
+// kernel of their own (attn_fwd_few.hip).
 //
 // The selection of a row is one bit per chunk (a bitmap built from the CSC lists by
 // csc_bitmap_kernel); the chunks a workgroup walks are the OR of its rows' bitmaps.
@@ -539,9 +540,7 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
     return;
   }
 
-  // ---- feeding the rings: the waves 0..3 fetch the tiles, rows wave * 16 .. wave * 16 + 15 each.  They reach the
-  // barrier of a step well before the waves 4..7 (which run a step's last part one step late and meet them on the
-  // matrix cores at the end of the step), so the loads are theirs ---------------------------------------------------
+  // ---- feeding the rings: each of a set's four waves fetches rows wave * 16 .. wave * 16 + 15 of a tile ----------------
   const uint32_t ldsK = (uint32_t)(uintptr_t)smem + (uint32_t)(set * (int)SM::ring), ldsV = ldsK + (uint32_t)(2 * SM::tile);
   const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)k0 * a.k_row_stride + (int64_t)hk * a.k_head_stride;
   const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)k0 * a.v_row_stride + (int64_t)hk * a.v_head_stride;
@@ -633,9 +632,7 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
 
   // A step in three parts.  part0: masks, row maximum and the reference point of step t (vector arithmetic); part1:
   // S(t + 1) on the matrix cores under the exponentials of step t; part2: O^T += V^T P^T of step t (matrix cores).
-  // The waves 4..7 share their SIMDs with the waves 0..3 and run part2 one step late, before part0 and part1 of the
-  // next step: every step begins at a workgroup barrier, and two waves that walk the parts in the same order want the
-  // matrix cores, then the vector unit, at the same moments.
+  // The other wave of the SIMD belongs to another workgroup (or set) and is in whatever part it is in.
   Pack8 pf[2][2];      // P^T as the B operand of O^T += V^T P^T, straight from the accumulators
   Pack8 kf[KS];        // K operands of S(t + 1): read at the start of part0, their latency runs under its arithmetic
   Pack8 vt[2][2];      // V^T operands of the first feature tile of step t: read at the end of part1

@@ -536,11 +536,12 @@ __device__ __forceinline__ void static_for(F &&f) {
 // an L2 still holds a good part of a pair, the same order costs 13 %).
 // ------------------------------------------------------------------------------------
 constexpr long long kOnePairBytes = 64ll << 20;
-// longest_first takes the items of an XCD's pairs in turn instead, item 0 of every pair, then item 1, .. : the callers number
+// longest_first, with a multiple of 8 pairs, takes the items of an XCD's pairs in turn instead, item 0 of every pair, then item 1, .. : the callers number
 // the items of a pair from the longest down, so the launch begins with the longest of all pairs and its last round is made of
 // the shortest.  With a few rounds of workgroups, or sequences of different lengths, that is what decides the time: a
 // pair-by-pair launch ends with a whole pair's mixture, its long items among them.  It gives up what a pair's items find in the
-// L2 of each other, so it is for calls whose rows, all pairs together (row_bytes per row and head: what the kernel reads of
+// L2 of each other, and it needs pairs in multiples of 8 (an XCD's pairs; with another number of sequences times heads the items
+// of a pair stay consecutive whatever the size), so it is for calls whose rows, all pairs together (row_bytes per row and head: what the kernel reads of
 // them again and again), take no more than kLongestFirstBytes and come from the memory-side cache at worst.  The pairs of a turn
 // are rotated by one from turn to turn where their number is even: workgroups go round the shader engines, and without the
 // rotation an engine gets the same pairs, hence the same sequences, in every turn (8192 tokens in four sequences, 32 over 8

@@ -135,10 +135,12 @@ int fmoba_varlen_sort(const int64_t *seg_starts, const int64_t *seg_ends, int64_
  *   out (total_q, heads, head_dim) dtype, softmax_lse (heads, total_q) fp32.
  * Rows that see no key get out = 0, lse = +inf.
  * Two forms.  Row blocks (patterns in which a row selects a good part of the chunks it may see):
- * one workgroup per 256 (or 128) query rows walks every chunk any of its rows selected, with the running
- * softmax state in registers; `workspace` then holds one selection bit per (row, head, chunk).
+ * one workgroup per 128 query rows walks every chunk any of its rows selected, with the running
+ * softmax state in registers; `workspace` then holds one selection bit per (row, head, chunk).  Calls with at
+ * most eight query rows per sequence count as row blocks and run one workgroup per (row, head).
  * Columns (sparser patterns): every visit of a (query row, key block) pair leaves a
- * partial result in `workspace`, and a second launch merges the partials of each row.  A key
+ * partial result in `workspace` (a row of head_dim 16-bit values, fp32 above head dimension 128), and a second
+ * launch merges the partials of each row.  A key
  * block is fmoba_attn_fwd_key_block(lg_block_n) keys (128 if lg_block_n is a multiple of 128,
  * else 64).  max_visits_per_row bounds the number of visits of any (row, head): for a pattern
  * from the gating, topk * lg_block_n / key_block; for an arbitrary pattern,
@@ -155,7 +157,7 @@ typedef struct {
   const int32_t *cu_seqlens_q, *cu_seqlens_k;
   /* optional (may be NULL): the same pattern as one bit per (row, head, chunk), word
    * [(h * ceil(max_cols/32) + c/32) * total_q + global row] bit c%32 -- what fmoba_fused_topk leaves
-   * at the first 256-byte boundary of its workspace.  Only the row-block form reads it (and
+   * at the first 256-byte boundary of its workspace.  Only the row-block form, that of a few query rows included, reads it (and
    * then no list: col_offsets, col_nnz and row_indices may be NULL); without it that form derives the
    * bits from the lists first. */
   const uint32_t *selection_bits;
