@@ -340,8 +340,8 @@ def run_config(name, steps, warmup, args, dev, cpu_budget_s):
         # it writes one dQ partial row per visit instead
         if hip.last_bwd_partials():
             bwd_kb = 128 if (chunk % 128 == 0 and D > 64) else 64
-            name = "attn_bwd_dkdv_partials_kernel" if D > 64 else "attn_bwd_dkdv_kernel"
-            kernels[name] = (phase_ms["dkdv"], 10.0 * D * pairs, 6 * qkv_once + list_bytes, entries * (chunk // bwd_kb) * (D * 2 + 4))
+            dkdv = "attn_bwd_dkdv_partials_kernel" if D > 64 else "attn_bwd_dkdv_kernel"
+            kernels[dkdv] = (phase_ms["dkdv"], 10.0 * D * pairs, 6 * qkv_once + list_bytes, entries * (chunk // bwd_kb) * (D * 2 + 4))
         else:
             kernels["attn_bwd_dkdv_kernel"] = (phase_ms["dkdv"], 8.0 * D * pairs, 6 * qkv_once + list_bytes, entries * chunk * 2)
             kernels["attn_bwd_dq_kernel"] = (phase_ms["dq"], 2.0 * D * pairs, 2 * qkv_once + list_bytes, entries * chunk * 2)
