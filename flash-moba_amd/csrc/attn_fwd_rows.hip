@@ -401,7 +401,7 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 }
 
 // ------------------------------------------------------------------------------------
-// The same walk without loader waves, for head dimensions up to 128: four waves of 32 rows and 256 registers, two
+// The same walk without loader waves, for head dimensions up to 128: four (two) waves of 32 rows and 256 registers, two
 // workgroups per compute unit, so that the matrix products of one run under the softmax arithmetic of the other whatever
 // their steps wait for.  K and V tiles go from global memory straight into LDS (every wave issues a quarter of a tile's
 // loads, one step ahead, rings of two stages each) in rows of exactly HD elements, swizzled instead of padded (piece c of row
@@ -413,38 +413,38 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // ahead), half of the tile loads but one barrier for all: 65536 tokens in eight sequences, top-k 32 of 64-key chunks 3.08 ms
 // against 2.87 here, 2 x 4096 tokens 247 against 205 us, 12037 tokens in five sequences 290 against 253, 8191 tokens of short
 // documents with heads of 64 51 against 40 (two workgroups cover each other's first loads, and 128 rows are less padding).
-// SPLIT = 2: a second set of four waves takes every other step of the same rows, with rings of its own; the two results of a
-// row meet in LDS at the end.
+// RW: waves of a set, which share its tiles.  SPLIT = 2: a second set of waves takes every other step of the same rows, with
+// rings of its own; the two results of a row meet in LDS at the end.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
 constexpr int kRowsWords = 16;  // selection words per row that the workgroup keeps in LDS (512 chunks)
 
-template <int HD, int SPLIT>
+template <int HD, int RW, int SPLIT>
 struct FwdRowsDirectSmem {
-  static constexpr int ROWS = 128;  // rows of a workgroup: 32 for each of four waves
+  static constexpr int ROWS = 32 * RW;  // rows of a workgroup: 32 for each wave of a set
   static constexpr int LDO = HD + 8;   // elements, per-wave output tile [32 rows][LDO]
   static constexpr size_t tile = (size_t)64 * HD * 2;       // one 64-key tile of K or V
-  static constexpr size_t ring = 4 * tile;                    // K, K, V, V: the rings of one set of four waves
+  static constexpr size_t ring = 4 * tile;                    // K, K, V, V: the rings of one set of waves
   static constexpr size_t oStep = SPLIT * ring;               // int[step_cap]: key block | chunk << 16
-  // behind the steps, sized by the call: uint32[nw] union, int[8], uint32[nw][ROWS] the rows' selection words
-  static size_t bytes(int step_cap, int nw) { return oStep + ((size_t)step_cap + nw + 8 + (size_t)nw * ROWS) * 4; }
-  static_assert((size_t)4 * 32 * LDO * 2 <= ring && (size_t)4 * HD * 128 <= ring, "output tiles must fit the K/V rings");
+  static constexpr int UPW = ROWS / 64;                       // unions of 64 rows' selection words per word
+  // behind the steps, sized by the call: uint32[nw][UPW] unions, uint32[nw][ROWS] the rows' selection words
+  static size_t bytes(int step_cap, int nw) { return oStep + ((size_t)step_cap + (size_t)nw * (UPW + ROWS)) * 4; }
+  static_assert((size_t)RW * 32 * LDO * 2 <= ring && (size_t)RW * HD * 128 <= ring && SPLIT * RW * 512 <= ring, "output tiles must fit the K/V rings");
 };
 
-template <typename T, int HD, int SPLIT>
-__global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap) {
-  typedef FwdRowsDirectSmem<HD, SPLIT> SM;
+template <typename T, int HD, int RW, int SPLIT>
+__global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap) {
+  typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
   constexpr int kRows = SM::ROWS;
   constexpr int KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
-  constexpr int NTHR = SPLIT * 256;
+  constexpr int NTHR = SPLIT * RW * 64;
   constexpr int RB = HD * 2;            // bytes of a tile row
   constexpr int RPI = 64 / VPR;         // tile rows per direct-to-LDS instruction (64 lanes x 16 bytes)
-  constexpr int NI = 64 / RPI / 4;      // such instructions per tile and feeding wave
-  static_assert(NI >= 1, "four waves share the loads of a tile");
+  constexpr int NI = 64 / RPI / RW;      // such instructions per tile and feeding wave
+  static_assert(NI >= 1, "the waves of a set share the loads of a tile");
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   int *sStep = reinterpret_cast<int *>(smem + SM::oStep);
   uint32_t *sUnion = reinterpret_cast<uint32_t *>(sStep + step_cap);
-  int *sOff = reinterpret_cast<int *>(sUnion + nw);
-  uint32_t *sBits = reinterpret_cast<uint32_t *>(sOff + 8);
+  uint32_t *sBits = sUnion + nw * SM::UPW;
 
   const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
   const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
   const int D = a.head_dim;
   const int hk = h / (a.heads / a.heads_k);
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
-  const int wave = wave_all & 3, set = wave_all >> 2;  // rows 32 wave .., steps set, set + SPLIT, ..
+  const int wave = wave_all % RW, set = wave_all / RW;  // rows 32 wave .., steps set, set + SPLIT, ..
   const bool causal = a.is_causal != 0;
   const int Bn = a.lg_block_n, sub = Bn >> 6;
   const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
@@ -481,50 +481,51 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
   const int kend = min(Lk, causal ? rlast + off + 1 : Lk);  // keys [0, kend) are visible to some row
   const int nchunk = kend > 0 ? (kend + Bn - 1) / Bn : 0;
   const int nwu = min((nchunk + 31) >> 5, nw);
-  for (int w = tid; w < nwu; w += NTHR) sUnion[w] = 0u;
-  __syncthreads();
   {
+    constexpr int UPW = SM::UPW;
     const int nrow = rlast - r0 + 1;
     const uint32_t *bp = bm + (int64_t)h * nw * a.total_q + q0 + r0;
     // (the words stay in LDS for the walk: a load from global memory inside the step loop would make the compiler
     // wait for every outstanding load of the wave, the tile loads included, at every step)
-    for (int i = tid; i < nrow * nwu; i += NTHR) {
-      const int w = i / nrow, row = i - w * nrow;
-      const uint32_t x = bp[(int64_t)w * a.total_q + row];
-      sBits[w * kRows + row] = x;
-      if (x) atomicOr(&sUnion[w], x);
+    for (int it = wave_all; it < nwu * UPW; it += NTHR / 64) {  // one word of 64 rows per wave
+      const int w = it / UPW, rw = (it % UPW) * 64 + lane;
+      const uint32_t x = rw < nrow ? bp[(int64_t)w * a.total_q + rw] : 0u;
+      sBits[w * kRows + rw] = x;
+      const uint32_t u = or_wave(x);
+      if (lane == 0) sUnion[it] = u;
     }
   }
   __syncthreads();
-  // one thread per chunk: a chunk of the union contributes its 64-key blocks that hold a visible key; a scan over the
-  // workgroup gives every chunk the place of its first step
-  int nstep_all = 0;
+  // One thread per chunk: a chunk of the union contributes its 64-key blocks that hold a visible key.  All but the last visible
+  // chunk have all of theirs, so a chunk's first step is the number of chunks of the union before it times the blocks of one: no
+  // scan over the workgroup, and no atomics for the unions (1024 tokens, 8 heads of 64: 14.7 -> 14.3 us).
   const int nchunk_u = min(nchunk, nwu * 32);
-  for (int c0 = 0; c0 < nchunk_u; c0 += NTHR) {
-    const int c = c0 + tid;
-    int cnt = 0;
-    if (c < nchunk_u && ((sUnion[c >> 5] >> (c & 31)) & 1u)) cnt = min(sub, (kend - c * Bn + 63) >> 6);
-    int incl = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int up = __shfl_up(incl, o, 64);
-      incl += lane >= o ? up : 0;
+  int nstep_all = 0;
+  if (nchunk_u > 0) {
+    auto word = [&](int w) {
+      uint32_t u = sUnion[w * SM::UPW];
+      if constexpr (SM::UPW == 2) u |= sUnion[w * 2 + 1];
+      return u;
+    };
+    for (int c = tid; c < nchunk_u; c += NTHR) {
+      int before = 0;
+      for (int w = 0; w < (c >> 5); ++w) before += __popc(word(w));
+      const uint32_t u = word(c >> 5);
+      if ((u >> (c & 31)) & 1u) {
+        int pos = (before + __popc(u & ((1u << (c & 31)) - 1u))) * sub;
+        const int cnt = min(sub, (kend - c * Bn + 63) >> 6);
+        for (int jb = 0; jb < cnt; ++jb, ++pos)
+          if (pos < step_cap) sStep[pos] = (c * sub + jb) | (c << 16);
+      }
     }
-    if (lane == 63) sOff[wave_all] = incl;
-    __syncthreads();
-    int before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < NTHR / 64; ++w) {
-      const int v = sOff[w];
-      before += w < wave_all ? v : 0;
-      total += v;
-    }
-    int pos = nstep_all + before + incl - cnt;
-    for (int jb = 0; jb < cnt; ++jb, ++pos)
-      if (pos < step_cap) sStep[pos] = (c * sub + jb) | (c << 16);
-    nstep_all += total;
-    __syncthreads();
+    const int last = nchunk_u - 1;
+    const uint32_t ul = word(last >> 5) & (0xffffffffu >> (31 - (last & 31)));
+    int nsel = __popc(ul);
+    for (int w = 0; w < (last >> 5); ++w) nsel += __popc(word(w));
+    nstep_all = nsel * sub - (((ul >> (last & 31)) & 1u) ? sub - min(sub, (kend - last * Bn + 63) >> 6) : 0);
+    nstep_all = __builtin_amdgcn_readfirstlane(nstep_all);
   }
+  __syncthreads();
   const int nstep_wg = min(nstep_all, step_cap);
   const int nstep = (nstep_wg - set + SPLIT - 1) / SPLIT, nturn = (nstep_wg + SPLIT - 1) / SPLIT;  // this set's steps, the turns of the loop
   auto entry = [&](int t) { return sStep[min(t * SPLIT + set, nstep_wg - 1)]; };
@@ -552,7 +553,7 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
     const int rl = lane / VPR, p = lane - rl * VPR;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int tr = (wave & 3) * (64 / 4) + i * RPI + rl;
+      const int tr = wave * (64 / RW) + i * RPI + rl;
       const uint32_t e = (uint32_t)min((p ^ tile_swz<HD>(tr)) * 8, D - 8);
       lofK[i] = ((uint32_t)tr * (uint32_t)a.k_row_stride + e) * 2u;
       lofV[i] = ((uint32_t)tr * (uint32_t)a.v_row_stride + e) * 2u;
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
   }
   auto feed = [&](const uint16_t *g, uint32_t row_stride, const uint32_t(&lof)[NI], uint32_t lds_ring, int stage, int t) {
     const int key0 = __builtin_amdgcn_readfirstlane((entry(t) & 0xffff) << 6);
-    const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + wave * (64 / 4) * RB);
+    const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + wave * (64 / RW) * RB);
     if (key0 + 64 <= Lk) {
       const uint16_t *base = g + (uint64_t)(uint32_t)key0 * row_stride;
 #pragma unroll
@@ -569,7 +570,7 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
       const int rl = lane / VPR, p = lane - rl * VPR;
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        const int tr = wave * (64 / 4) + i * RPI + rl;  // row of the tile
+        const int tr = wave * (64 / RW) + i * RPI + rl;  // row of the tile
         const uint32_t e = (uint32_t)min((p ^ tile_swz<HD>(tr)) * 8, D - 8);
         const uint32_t key = (uint32_t)min(key0 + tr, Lk - 1);
         global_to_lds16(g + ((uint64_t)key * row_stride + e), dst + (uint32_t)(i * RPI * RB));
@@ -765,31 +766,34 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
     if (t + 1 < nturn) step(C1{}, t + 1);
   }
   // (every wave is done with the rings and nothing is in flight: they now hold the sets' sums, then the output tiles)
-  if constexpr (SPLIT == 2) {
-    float *sO = reinterpret_cast<float *>(smem + SM::ring);                                // [wave][HD / 2 registers][64 lanes], in the second set's rings
-    float *sMl = reinterpret_cast<float *>(smem);                                          // [wave][2][64]
-    if (set == 1) {
+  if constexpr (SPLIT > 1) {
+    auto sums_of = [&](int st) { return reinterpret_cast<float *>(smem + st * SM::ring) + (size_t)wave * (HD / 2) * 64 + lane; };  // [wave][HD / 2 registers][64 lanes], in the set's rings
+    auto ml_of = [&](int st) { return reinterpret_cast<float *>(smem) + (st * RW + wave) * 128 + lane; };                            // [set][wave][2][64]
+    if (set > 0) {
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sO[(wave * (HD / 2) + dt * 16 + i) * 64 + lane] = o[dt][i];
-      sMl[(wave * 2) * 64 + lane] = m_run;
-      sMl[(wave * 2 + 1) * 64 + lane] = l_run;
+        for (int i = 0; i < 16; ++i) sums_of(set)[(dt * 16 + i) * 64] = o[dt][i];
+      ml_of(set)[0] = m_run;
+      ml_of(set)[64] = l_run;
     }
     __syncthreads();
     if (set == 0) {
-      const float m1 = sMl[(wave * 2) * 64 + lane], l1 = sMl[(wave * 2 + 1) * 64 + lane];
-      const float mn = fmaxf(m_run, m1), mref = mn == -INFINITY ? 0.f : mn;
-      const float f0 = __builtin_amdgcn_exp2f((m_run - mref) * scale_log2), f1 = __builtin_amdgcn_exp2f((m1 - mref) * scale_log2);
-      m_run = mn;
-      l_run = l_run * f0 + l1 * f1;
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
+      for (int st = 1; st < SPLIT; ++st) {
+        const float m1 = ml_of(st)[0], l1 = ml_of(st)[64];
+        const float mn = fmaxf(m_run, m1), mref = mn == -INFINITY ? 0.f : mn;
+        const float f0 = __builtin_amdgcn_exp2f((m_run - mref) * scale_log2), f1 = __builtin_amdgcn_exp2f((m1 - mref) * scale_log2);
+        m_run = mn;
+        l_run = l_run * f0 + l1 * f1;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * f0 + sO[(wave * (HD / 2) + dt * 16 + i) * 64 + lane] * f1;
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * f0 + sums_of(st)[(dt * 16 + i) * 64] * f1;
+      }
     }
-    __syncthreads();  // (the output tiles lie where m and l of the second set did)
-    if (set == 1) return;
+    __syncthreads();  // (the output tiles lie where m and l of the other sets did)
+    if (set > 0) return;
   }
 
   const float l_tot = sum_xor32_f(l_run);
@@ -817,10 +821,10 @@ __global__ __launch_bounds__(SPLIT * 256, 2) void attn_fwd_rows_kernel(fmoba_att
   }
 }
 
-template <typename T, int HD, int SPLIT>
+template <typename T, int HD, int RW, int SPLIT>
 static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
-  typedef FwdRowsDirectSmem<HD, SPLIT> SM;
-  auto kern = attn_fwd_rows_kernel<T, HD, SPLIT>;
+  typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
+  auto kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT>;
   const int step_cap = ceil_div(a.max_seqlen_k, 64);  // (at most kRowsStepCap: fwd_rows_feasible)
   const size_t smem = SM::bytes(step_cap, nw);
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
@@ -832,16 +836,27 @@ static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, i
     set_error("attn_fwd: too many (sequence, head, row block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * 256), smem, s, a, bm, nw, step_cap);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap);
   return 0;
 }
-// Two sets of waves where the launch leaves compute units idle anyway (at most one workgroup for each of the 256): the walk
-// of a row block is half as long (3072 tokens, 8 heads of 64: 38 -> 30 us).  Otherwise a second workgroup beside the first
-// serves a unit better (8191 tokens of short documents: 40 us with one set, 64 with two).
+// Which workgroup, by the 128-row blocks of the call and the mean length of its sequences:
+// - two waves of 32 rows and two sets of them where 128-row blocks come to about one per compute unit (two at head dimensions up
+//   to 64, where two such workgroups fit a unit): the walks are half as long and there are twice as many of them.  Against one
+//   set of four waves (two sets of four, which served half of these calls before, lie between): heads of 64, 2048 tokens, 16 heads
+//   38.4 -> 26.0 us, 4096 tokens 76 -> 66, 8192 tokens 206 -> 214 (beyond the line), c1 of two sequences, 8 heads 37 -> 25; heads of
+//   128, 2048 tokens, 16 heads 50 -> 43, 2500 tokens 63 -> 66.
+// - two waves and one set at head dimensions up to 64 for short sequences, whose workgroups spend half of their time on the way
+//   to the first step: 64 rows are less padding and twice as many workgroups wait side by side.  8191 tokens of documents of 341
+//   on average 34.8 -> 31.2 us, of 540 50 -> 43, of 1483 93.3 -> 89.7; one sequence of 8192 tokens 206 -> 206, 16384 765 -> 811.  (At
+//   head dimension 128 the rings leave room for two workgroups of either kind, and the small ones have half of the waves: 73 -> 99.)
+// - four waves and one set otherwise.
 template <typename T, int HD>
 static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
   const int64_t blocks = (int64_t)a.heads * (a.total_q / 128 + a.batch);
-  return blocks <= 256 ? launch_rows_split<T, HD, 2>(a, bm, nw, s) : launch_rows_split<T, HD, 1>(a, bm, nw, s);
+  if (blocks <= (HD > 64 ? 288 : 544)) return launch_rows_split<T, HD, 2, 2>(a, bm, nw, s);
+  if constexpr (HD <= 64)
+    if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1>(a, bm, nw, s);
+  return launch_rows_split<T, HD, 4, 1>(a, bm, nw, s);
 }
 
 template <typename T, int HD>

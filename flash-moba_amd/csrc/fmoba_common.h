@@ -445,6 +445,19 @@ __device__ __forceinline__ float sum_rows4_f(float v) {
   return sum_xor32_f(__uint_as_float(p.a) + __uint_as_float(p.b));
 }
 
+// bitwise or over the wave, result everywhere: four rotations within rows of 16 lanes, then the two exchanges above
+__device__ __forceinline__ uint32_t or_wave(uint32_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xf, 0xf, false);
+  x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xf, 0xf, false);
+  x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xf, 0xf, false);
+  x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, false);
+#endif
+  const UPair p = swap16(x);
+  const UPair q = swap32(p.a | p.b);
+  return q.a | q.b;
+}
+
 // Monotone map float -> uint32 (larger float => larger key); every non-NaN value,
 // including -inf, maps to a key >= 0x007fffff > 0.
 __device__ __forceinline__ uint32_t float_order_key(float f) {
