@@ -98,6 +98,8 @@ __device__ __forceinline__ uint2 pack4_scaled(float x, float y, float z, float w
 // for the partials form at head dimension 128, attn_bwd_dkdv_partials_kernel): 8191 tokens of short documents, heads of 64
 // 100 -> 49 us; 12037 tokens, heads of 96 227 -> 177 us; 2 x 4096 tokens 223 -> 214 us; 65536-token batch 2.94 -> 2.65 ms.
 // One workgroup of eight waves per 128 keys (half of the gathers, three buffers): 256 us where two of 64 keys take 214.
+// Head dimensions 65 to 96: tiles of 96 features against 128 before, 12037 tokens, 16 heads of 96 180 -> 159 us, 2 x 4096 tokens,
+// heads of 80 202 -> 164.
 // ------------------------------------------------------------------------------------
 template <int HD, bool DQP>
 struct DkdvSmem {
@@ -120,8 +122,11 @@ struct DkdvSmem {
 template <typename T, int HD, bool DQP>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
   typedef DkdvSmem<HD, DQP> SM;
-  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, NDW = NDT / 2, LDR = SM::LDR, PRB = SM::PRB;
+  constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR, PRB = SM::PRB;
   constexpr int NKEY = 64;   // keys of the workgroup
+  // tiles of dV or dK that a wave adds up: half of the features and all keys, or all three feature tiles and half of the keys
+  constexpr int NDW = NDT % 2 == 0 ? NDT / 2 : NDT, NKW = NDT % 2 == 0 ? 2 : 1;
+  static_assert(!DQP || NDT % 2 == 0, "the partials form divides the features");
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   const int gh = ws.dkv_heads, gs = a.heads / gh;  // heads of dK / dV, query heads that are added up in one
@@ -146,14 +151,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   const int D = a.head_dim;
   const int hk = h0 / (a.heads / a.heads_k);
   const int kq = wave & 1, rt = wave >> 1;   // S and dP: this wave's 32 keys and 32 rows
-  const int sel = wave >> 1, fw = wave & 1;  // sums: dV (0) or dK (1), half fw of the features, all keys
+  const int sel = wave >> 1, fw = wave & 1;  // sums: dV (0) or dK (1), half fw of the features or of the keys
+  const int d0 = NKW == 2 ? fw * NDW : 0, kk0 = NKW == 2 ? 0 : fw;  // first feature tile, first key tile
   const bool causal = a.is_causal != 0;
   const float scale_log2 = a.softmax_scale * kLog2e;
   const uint32_t lds = (uint32_t)(uintptr_t)smem, ldsQ = lds + (uint32_t)SM::oQ, ldsdO = lds + (uint32_t)SM::odO, ldsP = lds + (uint32_t)SM::oP, ldsdS = lds + (uint32_t)SM::odS;
   constexpr uint32_t TILE = (uint32_t)SM::tile;
-  constexpr int RPI = 64 / VPR;              // tile rows per load instruction
-  constexpr int NI = 16 / RPI;               // load instructions per wave, operand and round: 16 rows
-  const int rl = lane / VPR, pc = lane % VPR;
+  constexpr int NI = VPR / 4;                // load instructions per wave, operand and round: 16 rows
 
   // K and V of the block pass through the tiles on their way to registers
   {
@@ -161,7 +165,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
     const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int key = (wave * NI + i) * RPI + rl;
+      const int v = (wave * NI + i) * 64 + lane, key = v / VPR, pc = v - key * VPR;
       const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
       const int64_t kc = min(key, Lk - 1 - key0);
       global_to_lds16(kg + kc * a.k_row_stride + e, ldsQ + (uint32_t)((wave * NI + i) * 1024));
@@ -206,16 +210,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride;
   const uint16_t *dog = reinterpret_cast<const uint16_t *>(a.dout) + (int64_t)q0 * a.do_row_stride;
 
-  f32x16 acc[NDW][2];  // register i of tile [d][kk] <-> feature (fw * NDW + d) * 32 + acc_row(i, hh), key kk * 32 + lane % 32
+  f32x16 acc[NDW][NKW];  // register i of tile [d][kk] <-> feature (d0 + d) * 32 + acc_row(i, hh), key (kk0 + kk) * 32 + lane % 32
 #pragma unroll
   for (int d = 0; d < NDW; ++d)
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int kk = 0; kk < NKW; ++kk)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[d][kk][i] = 0.f;
 
   const int myrow = rt * 32 + (lane & 31);  // this lane's row of a round
-  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
+  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + ((tile_frag_piece<HD>(hh, 0) ^ tile_swz<HD>(lane & 31)) * 16));
   const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
   const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
   auto entry_at = [&](const Round &w) { return a.row_indices + w.pos + min(myrow, w.n - 1); };
@@ -231,9 +235,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   Pack8 kf[KS], vf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    kf[ks] = lds_read16(((ldsQ + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
-    vf[ks] = lds_read16(((ldsdO + (uint32_t)(kq * 32 * RB) + rowoff) ^ (uint32_t)(ks * 16)));
-    if (D < HD && (hh * KS + ks) * 8 >= D) kf[ks] = vf[ks] = zero_pack8();
+    kf[ks] = lds_read16(tile_frag_addr<HD>(ldsQ + (uint32_t)(kq * 32 * RB) + rowoff, ks));
+    vf[ks] = lds_read16(tile_frag_addr<HD>(ldsdO + (uint32_t)(kq * 32 * RB) + rowoff, ks));
+    if (D < HD && tile_frag_piece<HD>(hh, ks) * 8 >= D) kf[ks] = vf[ks] = zero_pack8();
   }
   // partials form: K^T of this wave's features, the A operand of dQ^T = K^T dS^T (keys 16 s4 + 8 hh .. + 7)
   Pack8 ktf[DQP ? NDW : 1][4];
@@ -256,14 +260,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
     // rows of a round (ids `rid`): Q and dO into the buffer, 16 rows per wave, of its own 32
     int ft = tid;  // thread index for the code around the products, re-made opaque in every round: what is derived from it is not kept in registers
     auto feed = [&](int rid, const Round &w, uint32_t buf) {
-      const int fl = ft & 63, rl = fl / VPR, pc = fl % VPR;
+      const int fl = ft & 63;
       const uint16_t *qh = qg + (int64_t)w.h * a.q_head_stride, *doh = dog + (int64_t)w.h * a.do_head_stride;
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        const int tr = kq * 16 + i * RPI + rl;  // row of the tile of 32
+        const int v = i * 64 + fl, r16 = v / VPR, pc = v - r16 * VPR, tr = kq * 16 + r16;  // row of the tile of 32, piece
         const uint32_t src = (uint32_t)__shfl(rid, tr, 64) & 0x7fffffffu;
         const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
-        const uint32_t dst = buf + (uint32_t)((rt * 32 + kq * 16 + i * RPI) * RB);
+        const uint32_t dst = buf + (uint32_t)((rt * 32 + kq * 16) * RB + i * 1024);
         global_to_lds16(qh + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
         global_to_lds16(doh + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
       }
@@ -319,8 +323,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
         constexpr int B = decltype(bc)::value;
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-          qf[B & 1][u] = lds_read16(aq ^ (uint32_t)((B * NB + u) * 16));
-          df[B & 1][u] = lds_read16(ad ^ (uint32_t)((B * NB + u) * 16));
+          qf[B & 1][u] = lds_read16(tile_frag_addr<HD>(aq, B * NB + u));
+          df[B & 1][u] = lds_read16(tile_frag_addr<HD>(ad, B * NB + u));
         }
       };
       rd(std::integral_constant<int, 0>{});
@@ -355,19 +359,18 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
       __syncthreads();  // P and dS of the round are in LDS
       // dV^T[f][key] += dO^T[f][row] P[row][key], dK^T[f][key] += Q^T[f][row] dS[row][key]
       const uint32_t tx = (sel ? ldsQ : ldsdO) + buf + troff, px = (sel ? ldsdS : ldsP) + pread;
-      Pack8 pb[2][2], xa[2][NDW];
+      Pack8 pb[2][NKW], xa[2][NDW];
       auto rd2 = [&](auto sc) {
         constexpr int S4 = decltype(sc)::value;
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const uint32_t po = (px ^ (uint32_t)(kk * 64)) + (uint32_t)(S4 * 16 * PRB);
+        for (int kk = 0; kk < NKW; ++kk) {
+          const uint32_t po = (px ^ (uint32_t)((kk0 + kk) * 64)) + (uint32_t)(S4 * 16 * PRB);
           pb[S4 & 1][kk] = lds_tr8(po, po + 8 * PRB);
         }
 #pragma unroll
         for (int d = 0; d < NDW; ++d) {
-          const uint32_t dt = (uint32_t)(fw * NDW + d), xlo = dt * 64u, xhi = ((dt * 4u) ^ (uint32_t)TileSwz<HD>::kRow8) * 16u;
-          const uint32_t olo = (uint32_t)(S4 * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
-          xa[S4 & 1][d] = lds_tr8((tx ^ xlo) + olo, (tx ^ xhi) + ohi);
+          const uint32_t o = (uint32_t)(S4 * 16 * RB);
+          xa[S4 & 1][d] = lds_tr8(tile_tr_addr<HD>(tx, d0 + d) + o, tile_tr_addr8<HD>(tx, d0 + d) + o);
         }
       };
       rd2(std::integral_constant<int, 0>{});
@@ -378,7 +381,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
 #pragma unroll
         for (int d = 0; d < NDW; ++d)
 #pragma unroll
-          for (int kk = 0; kk < 2; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
+          for (int kk = 0; kk < NKW; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
         __builtin_amdgcn_sched_barrier(0);
       });
       if constexpr (DQP) {
@@ -447,10 +450,10 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
 #pragma unroll
   for (int d = 0; d < NDW; ++d)
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int kk = 0; kk < NKW; ++kk)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<f32x4 *>(red + (size_t)(sel * NKEY + kk * 32 + (lane & 31)) * LDR + (fw * NDW + d) * 32 + 8 * g + 4 * hh) =
+        *reinterpret_cast<f32x4 *>(red + (size_t)(sel * NKEY + (kk0 + kk) * 32 + (lane & 31)) * LDR + (d0 + d) * 32 + 8 * g + 4 * hh) =
             f32x4{acc[d][kk][4 * g], acc[d][kk][4 * g + 1], acc[d][kk][4 * g + 2], acc[d][kk][4 * g + 3]};
   __syncthreads();
   uint16_t *dkg = reinterpret_cast<uint16_t *>(a.dk) + (int64_t)(k0 + key0) * a.dk_row_stride + (int64_t)hg * a.dk_head_stride;
@@ -1158,7 +1161,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
 // groups of two steps; one workgroup of eight such waves per unit (groups of four steps, 512 rows) read half of the K tiles
 // but met at one barrier and left no unit a second walk: 65536 tokens in eight sequences, top-k 32 of 64-key chunks
 // 1634 -> 1556 us, 24571 tokens, 32 over 8 heads 691 -> 624, 12037 tokens, heads of 96 182 -> 124 (with the order of the items
-// below), 2 x 4096 tokens 143 -> 125.  Up to 64: eight waves of one tile (with two tiles in four waves 4096 tokens 58 -> 67 us).
+// below; tiles of 96 features instead of 128: 129 -> 115), 2 x 4096 tokens 143 -> 125.  Up to 64: eight waves of one tile (with two tiles in four waves 4096 tokens 58 -> 67 us).
 // Above 128: eight waves of one tile, one workgroup per unit (its K tiles take 128 KB).
 // ------------------------------------------------------------------------------------
 constexpr int kDqColBatch = 256;
@@ -1220,9 +1223,8 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
   constexpr int LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
   constexpr int RB = HD * 2;                       // bytes of a K tile row
   constexpr uint32_t TB = (uint32_t)SM::tileBytes;
-  constexpr int RPI = 64 / VPR;                    // K rows per load instruction
-  constexpr int NKI = 64 / RPI / NW;         // K load instructions per wave and tile
-  static_assert(NKI >= 1 && NKI * RPI * NW == 64, "the waves share a K tile evenly");
+  constexpr int NKI = VPR / NW;              // K load instructions per wave and tile
+  static_assert(NKI >= 1 && NKI * NW == VPR, "the waves share a K tile evenly");
   constexpr int NS = SM::NS, G = SM::G;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   int *sPos = reinterpret_cast<int *>(smem + SM::oTag);
@@ -1326,13 +1328,12 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) myrow[rt] = (wtile * RT + rt) * 32 + (lane & 31);
 
-  // K tile loads of this wave: instruction i brings tile rows (wave * NKI + i) * RPI .. + RPI - 1, lane -> row rl, piece p;
-  // piece c of tile row r is stored at piece c ^ tile_swz<HD>(r)
-  const int krl = lane / VPR, kpp = lane - krl * VPR;
+  // K tile loads of this wave: lane l of instruction i brings number (wave * NKI + i) * 64 + l of the tile's pieces as they lie
+  // in LDS; piece c of tile row r is stored at piece c ^ tile_swz<HD>(r)
   uint32_t ksrc[NKI];  // element offset of this lane's piece inside a tile that exists completely
 #pragma unroll
   for (int i = 0; i < NKI; ++i) {
-    const int r = (wave * NKI + i) * RPI + krl;
+    const int v = (wave * NKI + i) * 64 + lane, r = v / VPR, kpp = v - r * VPR;
     ksrc[i] = (uint32_t)(r * (int)a.k_row_stride + min((kpp ^ tile_swz<HD>(r)) * 8, D - 8));
   }
   // K^T operands (transposing reads): lane l (i = l % 16) supplies the address of key 8 hh + i / 4 (+ 4 for the
@@ -1375,7 +1376,7 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
       } else {  // keys past the end of the sequence: the last key's data, which meets dS = 0
 #pragma unroll
         for (int i = 0; i < NKI; ++i) {
-          const int r = (wave * NKI + i) * RPI + krl;
+          const int v = (wave * NKI + i) * 64 + lane, r = v / VPR, kpp = v - r * VPR;
           const int key = min(key0 + r, Lk - 1), e = min((kpp ^ tile_swz<HD>(r)) * 8, D - 8);
           global_to_lds16(kp + (int64_t)key * a.k_row_stride + e, dst + (uint32_t)i * 1024u);
         }
@@ -1433,11 +1434,10 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
       // K^T operands half a feature tile (two products per row tile) ahead of their use
       Pack8 kf[2][2];
       auto kread = [&](int u, Pack8 (&dst)[2]) {  // unit u: feature tile u / 2, keys 32 (u % 2) .. + 31
-        const uint32_t x = (uint32_t)((u >> 1) * 64);
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
           const uint32_t o = (uint32_t)(16 * (2 * (u & 1) + s2) * RB);
-          dst[s2] = lds_tr8((alo ^ x) + o, (ahi ^ x) + o);
+          dst[s2] = lds_tr8(tile_tr_addr<HD>(alo, u >> 1) + o, tile_tr_addr<HD>(ahi, u >> 1) + o);
         }
       };
       kread(0, kf[0]);
@@ -1752,7 +1752,7 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
       hipLaunchKernelGGL(zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, (int64_t)a.total_q * a.heads);
       rc = a.head_dim <= 64 ? launch_dkdv<T, 64, true>(a, ws, s) : (bwd_wide_blocks(a) ? launch_dkdv_partials<T, 128, 2>(a, ws, s) : launch_dkdv_partials<T, 128, 1>(a, ws, s));
     } else {
-      rc = a.head_dim <= 64 ? launch_dkdv<T, 64, false>(a, ws, s) : launch_dkdv<T, 128, false>(a, ws, s);
+      rc = a.head_dim <= 64 ? launch_dkdv<T, 64, false>(a, ws, s) : a.head_dim <= 96 ? launch_dkdv<T, 96, false>(a, ws, s) : launch_dkdv<T, 128, false>(a, ws, s);
     }
     if (rc) return rc;
   }
@@ -1768,7 +1768,7 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
       }
       hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 15) / 16)), dim3(256), smem, s, a, ws, capl);
     } else {
-      int rc = a.head_dim <= 64 ? launch_dq<T, 64, 1, 8>(a, ws.ds, s) : launch_dq<T, 128, 2, 4>(a, ws.ds, s);
+      int rc = a.head_dim <= 64 ? launch_dq<T, 64, 1, 8>(a, ws.ds, s) : a.head_dim <= 96 ? launch_dq<T, 96, 2, 4>(a, ws.ds, s) : launch_dq<T, 128, 2, 4>(a, ws.ds, s);
       if (rc) return rc;
     }
   }

@@ -413,6 +413,8 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // ahead), half of the tile loads but one barrier for all: 65536 tokens in eight sequences, top-k 32 of 64-key chunks 3.08 ms
 // against 2.87 here, 2 x 4096 tokens 247 against 205 us, 12037 tokens in five sequences 290 against 253, 8191 tokens of short
 // documents with heads of 64 51 against 40 (two workgroups cover each other's first loads, and 128 rows are less padding).
+// Head dimensions 65 to 96 have tiles of 96 features (rows of 192 bytes): a quarter of the products of 128-feature tiles less
+// (12037 tokens, 16 heads of 96, top-k 8 of 64-key chunks 208 -> 176 us; 2048 tokens, 8 heads 41 -> 29).
 // RW: waves of a set, which share its tiles.  SPLIT = 2: a second set of waves takes every other step of the same rows, with
 // rings of its own; the two results of a row meet in LDS at the end.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
@@ -438,9 +440,8 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   constexpr int KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
   constexpr int NTHR = SPLIT * RW * 64;
   constexpr int RB = HD * 2;            // bytes of a tile row
-  constexpr int RPI = 64 / VPR;         // tile rows per direct-to-LDS instruction (64 lanes x 16 bytes)
-  constexpr int NI = 64 / RPI / RW;      // such instructions per tile and feeding wave
-  static_assert(NI >= 1, "the waves of a set share the loads of a tile");
+  constexpr int NI = VPR / RW;          // direct-to-LDS instructions (64 lanes x 16 bytes) per tile and feeding wave
+  static_assert(NI >= 1 && NI * RW == VPR, "the waves of a set share the loads of a tile");
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   int *sStep = reinterpret_cast<int *>(smem + SM::oStep);
   uint32_t *sUnion = reinterpret_cast<uint32_t *>(sStep + step_cap);
@@ -471,7 +472,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + min(row, Lq - 1)) * a.q_row_stride + (int64_t)h * a.q_head_stride;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const int e = (hh * KS + ks) * 8;
+      const int e = tile_frag_piece<HD>(hh, ks) * 8;
       qb[ks] = (valid && e < D) ? ld_global16(qg + e) : zero_pack8();
     }
   }
@@ -545,15 +546,14 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   const uint32_t ldsK = (uint32_t)(uintptr_t)smem + (uint32_t)(set * (int)SM::ring), ldsV = ldsK + (uint32_t)(2 * SM::tile);
   const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)k0 * a.k_row_stride + (int64_t)hk * a.k_head_stride;
   const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)k0 * a.v_row_stride + (int64_t)hk * a.v_head_stride;
-  // A lane's piece of row tr = wave * 16 + i * RPI + lane / VPR of a tile: its byte offset from the tile's first key, for K
+  // A lane's piece in load i, number (wave * NI + i) * 64 + lane of the tile: its byte offset from the tile's first key, for K
   // and for V.  A tile whose 64 keys all exist is fetched from a wave-uniform base plus these offsets (no vector
   // instruction per load); the last tile of a sequence clamps the keys per lane.
   uint32_t lofK[NI], lofV[NI];
   {
-    const int rl = lane / VPR, p = lane - rl * VPR;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int tr = wave * (64 / RW) + i * RPI + rl;
+      const int v = (wave * NI + i) * 64 + lane, tr = v / VPR, p = v - tr * VPR;
       const uint32_t e = (uint32_t)min((p ^ tile_swz<HD>(tr)) * 8, D - 8);
       lofK[i] = ((uint32_t)tr * (uint32_t)a.k_row_stride + e) * 2u;
       lofV[i] = ((uint32_t)tr * (uint32_t)a.v_row_stride + e) * 2u;
@@ -561,19 +561,18 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   }
   auto feed = [&](const uint16_t *g, uint32_t row_stride, const uint32_t(&lof)[NI], uint32_t lds_ring, int stage, int t) {
     const int key0 = __builtin_amdgcn_readfirstlane((entry(t) & 0xffff) << 6);
-    const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + wave * (64 / RW) * RB);
+    const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + wave * NI * 1024);
     if (key0 + 64 <= Lk) {
       const uint16_t *base = g + (uint64_t)(uint32_t)key0 * row_stride;
 #pragma unroll
-      for (int i = 0; i < NI; ++i) global_to_lds16_sbase(lof[i], base, dst + (uint32_t)(i * RPI * RB));
+      for (int i = 0; i < NI; ++i) global_to_lds16_sbase(lof[i], base, dst + (uint32_t)(i * 1024));
     } else {
-      const int rl = lane / VPR, p = lane - rl * VPR;
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        const int tr = wave * (64 / RW) + i * RPI + rl;  // row of the tile
+        const int v = (wave * NI + i) * 64 + lane, tr = v / VPR, p = v - tr * VPR;  // row of the tile, piece
         const uint32_t e = (uint32_t)min((p ^ tile_swz<HD>(tr)) * 8, D - 8);
         const uint32_t key = (uint32_t)min(key0 + tr, Lk - 1);
-        global_to_lds16(g + ((uint64_t)key * row_stride + e), dst + (uint32_t)(i * RPI * RB));
+        global_to_lds16(g + ((uint64_t)key * row_stride + e), dst + (uint32_t)(i * 1024));
       }
     }
   };
@@ -600,7 +599,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   // byte offsets of this lane's pieces inside a tile: row reads (key lane % 32 of a 32-key half, pieces hh * KS ..) and
   // transposing reads (key (lane % 16) / 4 + 4 hh, feature tile 0); every other operand is an exclusive-or on the piece
   // bits plus a constant
-  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
+  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + ((tile_frag_piece<HD>(hh, 0) ^ tile_swz<HD>(lane & 31)) * 16));
   const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
   const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
   auto opaque = [](uint32_t &x) {
@@ -610,11 +609,10 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     (void)x;
 #endif
   };
-  auto k_frag = [&](uint32_t ak, int kt, int ks) { return lds_read16((ak ^ (uint32_t)(ks * 16)) + (uint32_t)(kt * 32 * RB)); };
+  auto k_frag = [&](uint32_t ak, int kt, int ks) { return lds_read16(tile_frag_addr<HD>(ak, ks) + (uint32_t)(kt * 32 * RB)); };
   auto v_frag = [&](uint32_t tv, int dt, int kt, int s2) {
-    const uint32_t xlo = (uint32_t)(dt * 4 * 16), xhi = (uint32_t)(((dt * 4) ^ TileSwz<HD>::kRow8) * 16);
-    const uint32_t olo = (uint32_t)((kt * 32 + 16 * s2) * RB), ohi = olo + (uint32_t)(8 * RB);
-    return lds_tr8((tv ^ xlo) + olo, (tv ^ xhi) + ohi);
+    const uint32_t o = (uint32_t)((kt * 32 + 16 * s2) * RB);
+    return lds_tr8(tile_tr_addr<HD>(tv, dt) + o, tile_tr_addr8<HD>(tv, dt) + o);
   };
   // S of the first step, not overlapped with anything
   auto s_plain = [&](uint32_t ak, f32x16(&sn)[2]) {
@@ -917,6 +915,8 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
     if (a.head_dim <= 64)
       rc = direct ? (bf ? launch_rows<bf16_t, 64>(a, bm, nw, s) : launch_rows<f16_t, 64>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 64>(a, bm, nw, s) : launch_rows_loader<f16_t, 64>(a, bm, nw, s));
+    else if (direct && a.head_dim <= 96)
+      rc = bf ? launch_rows<bf16_t, 96>(a, bm, nw, s) : launch_rows<f16_t, 96>(a, bm, nw, s);
     else if (a.head_dim <= 128)
       rc = direct ? (bf ? launch_rows<bf16_t, 128>(a, bm, nw, s) : launch_rows<f16_t, 128>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 128>(a, bm, nw, s) : launch_rows_loader<f16_t, 128>(a, bm, nw, s));

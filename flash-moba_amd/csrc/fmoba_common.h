@@ -621,7 +621,9 @@ __device__ __forceinline__ Pack8 zero_pack8() {
 // piece c of tile row r is stored at piece c ^ tile_swz<HD>(r)
 template <int HD>
 __device__ __forceinline__ int tile_swz(int r) {
-  if constexpr (HD > 64)
+  if constexpr (HD == 96)
+    return (r >> 2) & 3;  // 12 pieces per row: the rows of four begin in different quarters of a sweep by themselves
+  else if constexpr (HD > 64)
     return ((r & 3) << 2) | ((r >> 2) & 3);  // 16 pieces per row, one row per sweep of the banks
   else
     return (((r >> 1) & 1) << 2) | ((r >> 2) & 1);  // 8 pieces per row, two rows per sweep
@@ -630,6 +632,23 @@ template <int HD>
 struct TileSwz {
   static constexpr int kRow8 = HD > 64 ? 2 : 0;  // tile_swz(r + 8) ^ tile_swz(r)
 };
+// Operands of 32x32x16 products over the features of a row: the piece that half hh of the wave takes in k-step ks (any order does
+// that both operands share), and its address from that of step 0, which holds row * HD * 2 + (tile_frag_piece(hh, 0) ^
+// tile_swz(row)) * 16.  Rows of a power of two bytes leave the piece bits free for an exclusive-or; rows of 192 bytes only two of them.
+template <int HD>
+__device__ __forceinline__ constexpr int tile_frag_piece(int hh, int ks) { return HD == 96 ? 2 * ks + hh : hh * (HD / 16) + ks; }
+template <int HD>
+__device__ __forceinline__ uint32_t tile_frag_addr(uint32_t at0, int ks) {
+  return HD == 96 ? (at0 ^ (uint32_t)((ks & 1) * 32)) + (uint32_t)((ks >> 1) * 64) : at0 ^ (uint32_t)(ks * 16);
+}
+// Transposing reads: address of feature tile dt (32 features) from that of tile 0, and of the row eight further down
+template <int HD>
+__device__ __forceinline__ uint32_t tile_tr_addr(uint32_t at0, int dt) { return HD == 96 ? at0 + (uint32_t)(dt * 64) : at0 ^ (uint32_t)(dt * 64); }
+template <int HD>
+__device__ __forceinline__ uint32_t tile_tr_addr8(uint32_t at0, int dt) {
+  constexpr uint32_t x8 = (uint32_t)(TileSwz<HD>::kRow8 * 16);
+  return (HD == 96 ? (at0 ^ x8) + (uint32_t)(dt * 64) : at0 ^ ((uint32_t)(dt * 64) ^ x8)) + (uint32_t)(8 * HD * 2);
+}
 
 // (read as ONE vector: as a struct of four words the read is split and put together again by what the compiler knows
 // of the address bits, and where it knows nothing -- an address that comes out of an assembly statement, or round a

@@ -11,14 +11,15 @@ pytestmark = pytest.mark.gpu
 
 # Two sets over 64 rows: walks of one step, of odd and even numbers of steps (a set without a step among them), lengths at the edges
 # of 64 rows, chunks of one, two and four key blocks, the last of them cut short.  One set over 64 rows: many short sequences of
-# narrow heads.  One set over 128 rows: both widths, more than one word of selection bits per row
+# narrow heads.  One set over 128 rows: every width, more than one word of selection bits per row
 SMALL = [1, 63, 64, 65, 0, 127, 129, 193]
 DOCS = [1, 64, 65, 300] * 10
 
 
 @pytest.mark.parametrize("lens,H,Hk,D,chunk,topk", [
     (SMALL, 2, 2, 64, 64, 2), (SMALL, 4, 1, 128, 64, 3), (SMALL, 2, 1, 40, 128, 2), ([385, 700], 2, 2, 96, 256, 2), ([2100], 2, 2, 64, 64, 12),
-    (DOCS, 16, 16, 64, 64, 2), (DOCS, 16, 4, 32, 128, 2), ([2300], 32, 8, 64, 64, 12), ([2300], 16, 16, 128, 64, 12)])
+    (DOCS, 16, 16, 64, 64, 2), (DOCS, 16, 4, 32, 128, 2), ([2300], 32, 8, 64, 64, 12), ([2300], 16, 16, 128, 64, 12),
+    ([2300], 16, 16, 80, 64, 12)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_row_block_workgroups(lens, H, Hk, D, chunk, topk, dtype):
     g = torch.Generator(device="cuda").manual_seed(sum(lens) + D)
