@@ -1208,13 +1208,6 @@ __device__ __forceinline__ DqItem dq_decode_item(int id, int npairs, int nsb_max
   return w;
 }
 
-template <int N>
-__device__ __forceinline__ void wait_loads_but() {  // until at most N of the wave's vector memory loads are outstanding
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-#endif
-}
-
 // RT: 32-row tiles per wave (with two, every K^T operand read from LDS feeds two MFMAs).  NW: waves.
 template <typename T, int HD, int RT, int NW>
 __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, int nsb_max) {

@@ -72,12 +72,13 @@ struct FwdColSmem {
 // small workgroups that share a unit and serve all heads of a group.  The kernel this one replaces had one workgroup of
 // 512-register waves per unit and head and walked 128 rows between barriers: on those two shapes 2.32 -> 2.17 ms and
 // 530 -> 162 us, 8192 tokens with top-k 8 148 -> 132 us, 262144 tokens 9.99 -> 9.12 ms, and one row per sequence against
-// 16 sequences of up to 32768 keys 651 -> 113 us.
+// 16 sequences of up to 32768 keys 651 -> 113 us.  Since then, with the Q rows in runs of 64 bytes, the row ids ahead of the block and
+// no registers spilled: 2.08 -> 1.94 ms, 164 -> 154 us, 114 -> 109 us, 9.35 -> 8.53 ms, and 2 x 4096 tokens, 8 heads of 256, 175 -> 158 us.
 // Head dimensions above 128: an fp32 partial row per 128 keys is as many bytes as a 16-bit one per 64, and 128 keys are what one
 // workgroup of eight waves finds room for (2 x 4096 tokens, 8 heads of 256, top-k 8 of 128-key chunks, forward: 16-bit rows
 // per 64 keys 273 us, fp32 rows per 64 keys 450, per 128 keys 269).  Chunks that 128 does not divide pay for the wider rows:
 // top-k 16 of 64-key chunks 259 -> 439 us.
-template <typename T, int HD, int KB>
+template <typename T, int HD, int KB, bool FULL>  // FULL: the head dimension is HD
 __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp) {
   typedef FwdColSmem<HD, KB> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, KT = KB / 32, RB = HD * 2, NW = SM::NW;
@@ -88,268 +89,291 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
   const int key0 = nb * KB;
   const int c = key0 / a.lg_block_n;
+  // lane j: the list of head h0 + j (at most 64 of them: fwd_col_heads), asked for together with the sequence's bounds: neither needs
+  // the other
+  int nnz = 0;
+  int64_t lbase = 0;
+  if (c < a.max_cols && lane < grp) {
+    const int64_t ci = ((int64_t)b * a.heads + h0 + lane) * a.max_cols + c;
+    nnz = a.col_nnz[ci];
+    lbase = a.col_offsets[ci];
+  }
   const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   if (key0 >= Lk || c >= a.max_cols) return;
   const int off = Lk - Lq;
-  const int D = a.head_dim;
+  const int D = FULL ? HD : a.head_dim;
   const bool causal = a.is_causal != 0;
   const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
   const uint32_t ldsK = (uint32_t)(uintptr_t)smem, ldsV = ldsK + (uint32_t)SM::tile, ldsOut = ldsK + (uint32_t)(SM::oOut + wave * 4096);
 
-  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((hh * KS) ^ tile_swz<HD>(lane & 31)) * 16));
+  // k-step ks takes piece 4 (ks / 2) + ks % 2 + 2 hh of a row (the order in which Q arrives, see fetch)
+  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + (((2 * hh) ^ tile_swz<HD>(lane & 31)) * 16));
   const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
   const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
-  bool loaded = false;
-
-  for (int g0 = 0; g0 < grp; g0 += 64) {  // (a turn per 64 heads of the group)
-    // lane j: the list of head g0 + j of the group
-    int nnz = 0;
-    int64_t lbase = 0;
-    if (g0 + lane < grp) {
-      const int64_t ci = ((int64_t)b * a.heads + h0 + g0 + lane) * a.max_cols + c;
-      nnz = a.col_nnz[ci];
-      lbase = a.col_offsets[ci];
-    }
-    int incl = (nnz + 31) >> 5;  // tiles of the lists up to this one
+  int incl = (nnz + 31) >> 5;  // tiles of the lists up to this one
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int up = __shfl_up(incl, o, 64);
-      incl += lane >= o ? up : 0;
-    }
-    const int ntile = __builtin_amdgcn_readlane(incl, 63);
-    if (ntile == 0) continue;
-    if (!loaded) {
-      constexpr int RPI = 64 / VPR, NI = KB / RPI / NW;
-      const int rl = lane / VPR, pc = lane % VPR;
-      const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
-      const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int up = __shfl_up(incl, o, 64);
+    incl += lane >= o ? up : 0;
+  }
+  const int ntile = __builtin_amdgcn_readlane(incl, 63);
+  if (ntile == 0) return;
+  // The wave's tiles: tile t + 2 NW is picked (its row ids are asked for) and the rows of tile t + NW are fetched while tile t
+  // is worked on, and all of these loads are awaited at one place, before the stores of tile t: one counter covers
+  // loads and stores alike, and a load issued after the stores would be waited for together with them.
+  int g = 0, rem = 0, ridn = 0;
+  Pack8 qb[KS];
+  int slot = 0;
+  // (no branch around the loads: where two paths join, the compiler copies what was loaded, and waits for it there)
+  auto pick = [&](auto async, int t) {
+    t = min(t, ntile - 1);
+    g = __popcll(__ballot(incl <= t));
+    const int first = t - (g ? __builtin_amdgcn_readlane(incl, g - 1) : 0);
+    const int n = __builtin_amdgcn_readlane(nnz, g);
+    const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)lbase, g), bhi = __builtin_amdgcn_readlane((uint32_t)(lbase >> 32), g);
+    const int32_t *list = a.row_indices + (int64_t)(((uint64_t)bhi << 32) | blo) + first * 32;
+    rem = n - first * 32;
+    const int32_t *p = list + min(lane & 31, rem - 1);
+    if constexpr (decltype(async)::value)
+      ridn = load_async(p);
+    else
+      ridn = *p;
+  };
+  int rid = -1, hcur = 0;
+  auto fetch = [&](int t) {  // Q rows and partial slots of the picked tile
+    rid = tile_row_code(ridn, (lane & 31) < rem, Lq);
+    hcur = h0 + g;
+    // Four lanes fetch 64 bytes of a row together: load 2 j brings pieces 4 j .. 4 j + 3 of the tile's first sixteen rows, load 2 j + 1 those
+    // of the other sixteen, and an exchange of 16-lane rows then gives every lane pieces of its own row.  (A lane that fetched its own
+    // row's pieces touched a line of its own in every load, 64 lines a load where it is sixteen now: 32768 tokens, 32 heads, top-k 16
+    // 2089 -> 1924 us, 262144 tokens 9200 -> 8561.)
+    const UPair rr = swap16((uint32_t)rid & 0x7fffffffu);
+    const uint16_t *qh = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride + (int64_t)hcur * a.q_head_stride;
+    const uint16_t *qa = qh + (uint64_t)rr.a * (uint32_t)a.q_row_stride, *qo = qh + (uint64_t)rr.b * (uint32_t)a.q_row_stride;
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int key = (wave * NI + i) * RPI + rl;
-        const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
-        const int64_t kc = min(key, Lk - 1 - key0);
-        global_to_lds16(kg + kc * a.k_row_stride + e, ldsK + (uint32_t)((wave * NI + i) * 1024));
-        global_to_lds16(vg + kc * a.v_row_stride + e, ldsV + (uint32_t)((wave * NI + i) * 1024));
-      }
+    for (int j = 0; j < KS / 2; ++j) {
+      const int e = min((4 * j + (lane >> 4)) * 8, D - 8);  // (features past D: zeroed in arrived())
+      qb[2 * j] = ld_global16(qa + e);
+      qb[2 * j + 1] = ld_global16(qo + e);
     }
-    // The wave's tiles: tile t + 2 NW is picked (its row ids are asked for) and the rows of tile t + NW are fetched while tile t
-    // is worked on, and all of these loads are awaited at one place, before the stores of tile t: one counter covers
-    // loads and stores alike, and a load issued after the stores would be waited for together with them.
-    int g = 0, rem = 0, ridn = 0;
-    Pack8 qb[KS];
-    int slot = 0;
-    // (no branch around the loads: where two paths join, the compiler copies what was loaded, and waits for it there)
-    auto pick = [&](int t) {
-      t = min(t, ntile - 1);
-      g = __popcll(__ballot(incl <= t));
-      const int first = t - (g ? __builtin_amdgcn_readlane(incl, g - 1) : 0);
-      const int n = __builtin_amdgcn_readlane(nnz, g);
-      const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)lbase, g), bhi = __builtin_amdgcn_readlane((uint32_t)(lbase >> 32), g);
-      const int32_t *list = a.row_indices + (int64_t)(((uint64_t)bhi << 32) | blo) + first * 32;
-      rem = n - first * 32;
-      ridn = list[min(lane & 31, rem - 1)];
-    };
-    int rid = -1, hcur = 0;
-    auto fetch = [&](int t) {  // Q rows and partial slots of the picked tile
-      rid = tile_row_code(ridn, (lane & 31) < rem, Lq);
-      hcur = h0 + g0 + g;
-      const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + (rid & 0x7fffffff)) * a.q_row_stride + (int64_t)hcur * a.q_head_stride;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) qb[ks] = ld_global16(qp + min((hh * KS + ks) * 8, D - 8));  // (features past D: zeroed in arrived())
-      slot = take_slot(ws.cnt + ((int64_t)(q0 + (rid & 0x7fffffff)) * a.heads + hcur), __ballot(rid >= 0 && hh == 0 && t < ntile));
-    };
-    auto arrived = [&]() {
-      wait_all_loads();
+    slot = take_slot(ws.cnt + ((int64_t)(q0 + (rid & 0x7fffffff)) * a.heads + hcur), __ballot(rid >= 0 && hh == 0 && t < ntile));
+  };
+  auto arrived = [&]() {
+    wait_all_loads();
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
-      asm volatile("" : "+v"(slot), "+v"(ridn));
-#endif
-      if (D < HD) {
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
+    asm volatile("" : "+v"(slot), "+v"(ridn));
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+    for (int j = 0; j < KS / 2; ++j)
 #pragma unroll
-          for (int w = 0; w < 4; ++w) qb[ks].w[w] = (hh * KS + ks) * 8 < D ? qb[ks].w[w] : 0u;
+      for (int w = 0; w < 4; ++w) {
+        auto x = __builtin_amdgcn_permlane16_swap(qb[2 * j].w[w], qb[2 * j + 1].w[w], false, false);
+        qb[2 * j].w[w] = x[0];
+        qb[2 * j + 1].w[w] = x[1];
       }
-    };
-    pick(wave);
-    fetch(wave);
-    pick(wave + NW);
-    arrived();
-    if (!loaded) {
-      wait_all_loads();
-      __syncthreads();
-      loaded = true;
+#endif
+    if (D < HD) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) qb[ks].w[w] = (4 * (ks >> 1) + (ks & 1) + 2 * hh) * 8 < D ? qb[ks].w[w] : 0u;
     }
-    for (int t = wave; t < ntile; t += NW) {
-      const int r = rid, h = hcur;
-      const int s0 = __shfl(slot, lane & 31, 64);
-      const int pidx = (r >= 0 && s0 < ws.cap) ? ((q0 + r) * a.heads + h) * ws.cap + s0 : -1;
-      // keys beyond lim are masked
-      const int lim = r < 0 ? -1 : min(causal ? r + off : 0x7fffffff, Lk - 1) - key0;
-      f32x16 st[KT];
+  };
+  // The row ids of the first tile before the block's K and V, and waited for without them: the counter of a wave's loads counts in
+  // order, and the Q rows are the longest chain of a workgroup with few tiles (column bounds, row ids, rows: parts of prompts of 1024 rows
+  // against 9000 to 33000 keys 160 -> 154 us).
+  pick(std::true_type{}, wave);
+  constexpr int RPI = 64 / VPR, NI = KB / RPI / NW;
+  {
+    const int rl = lane / VPR, pc = lane % VPR;
+    const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)(k0 + key0) * a.k_row_stride + (int64_t)hk * a.k_head_stride;
+    const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)(k0 + key0) * a.v_row_stride + (int64_t)hk * a.v_head_stride;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int key = (wave * NI + i) * RPI + rl;
+      const int e = min((pc ^ tile_swz<HD>(key)) * 8, D - 8);
+      const int64_t kc = min(key, Lk - 1 - key0);
+      global_to_lds16(kg + kc * a.k_row_stride + e, ldsK + (uint32_t)((wave * NI + i) * 1024));
+      global_to_lds16(vg + kc * a.v_row_stride + e, ldsV + (uint32_t)((wave * NI + i) * 1024));
+    }
+  }
+  wait_loads_but<2 * NI>();
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(ridn));
+#endif
+  fetch(wave);
+  pick(std::false_type{}, wave + NW);
+  arrived();
+  __syncthreads();
+  for (int t = wave; t < ntile; t += NW) {
+    const int r = rid, h = hcur;
+    const int s0 = __shfl(slot, lane & 31, 64);
+    const int pidx = (r >= 0 && s0 < ws.cap) ? ((q0 + r) * a.heads + h) * ws.cap + s0 : -1;
+    // keys beyond lim are masked
+    const int lim = r < 0 ? -1 : min(causal ? r + off : 0x7fffffff, Lk - 1) - key0;
+    f32x16 st[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) st[kt][i] = 0.f;
+    uint32_t ak = ldsK + rowoff;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(ak));
+#endif
+    // (the K operands of a k-step are read while the step before it is on the matrix cores; the fences keep the compiler
+    // from moving every read next to its product)
+    Pack8 kf[2][KT];
+    auto k_read = [&](auto kc) {
+      constexpr int ks = decltype(kc)::value;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) kf[ks & 1][kt] = lds_read16((ak ^ (uint32_t)((4 * (ks >> 1) + (ks & 1)) * 16)) + (uint32_t)(kt * 32 * RB));
+    };
+    k_read(std::integral_constant<int, 0>{});
+    static_for<KS>([&](auto kc) {
+      constexpr int ks = decltype(kc)::value;
+      if constexpr (ks + 1 < KS) k_read(std::integral_constant<int, ks + 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) st[kt] = mfma32<T>(kf[ks & 1][kt], qb[ks], st[kt]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    fetch(t + NW);
+    pick(std::false_type{}, t + 2 * NW);
+    if (!__all(lim >= KB - 1)) {
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) st[kt][i] = 0.f;
-      uint32_t ak = ldsK + rowoff;
-#if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(ak));
-#endif
-      // (the K operands of a k-step are read while the step before it is on the matrix cores; the fences keep the compiler
-      // from moving every read next to its product)
-      Pack8 kf[2][KT];
-      auto k_read = [&](auto kc) {
-        constexpr int ks = decltype(kc)::value;
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) kf[ks & 1][kt] = lds_read16((ak ^ (uint32_t)(ks * 16)) + (uint32_t)(kt * 32 * RB));
-      };
-      k_read(std::integral_constant<int, 0>{});
-      static_for<KS>([&](auto kc) {
-        constexpr int ks = decltype(kc)::value;
-        if constexpr (ks + 1 < KS) k_read(std::integral_constant<int, ks + 1>{});
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) st[kt] = mfma32<T>(kf[ks & 1][kt], qb[ks], st[kt]);
-        __builtin_amdgcn_sched_barrier(0);
-      });
-      fetch(t + NW);
-      pick(t + 2 * NW);
-      if (!__all(lim >= KB - 1)) {
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int jrel = kt * 32 + 8 * (i >> 2) + (i & 3) + 4 * hh;
-            st[kt][i] = jrel <= lim ? st[kt][i] : -INFINITY;
-          }
-      }
-      float m = -INFINITY;
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) m = fmaxf(m, st[kt][i]);
-      m = max_xor32_f(m) * scale_log2;
-      const float m_use = m == -INFINITY ? 0.f : m;
-      float l = 0.f;
-      Pack8 pf[KT][2];
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const float p0 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w], scale_log2, -m_use));
-            const float p1 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w + 1], scale_log2, -m_use));
-            l += p0 + p1;
-            pf[kt][s2].w[w] = pack2<T>(p0, p1);
-          }
-      l = sum_xor32_f(l);
-      constexpr bool NORM = kFwdNormalisedParts<T, HD>;
-      const float inv = NORM && l > 0.f ? 1.f / l : 0.f;
-      constexpr bool F32 = fwd_part_size(HD) == 4;
-      // a tile's partial rows, 128 bytes of every row at a time: 64 features in 16 bits, 32 features in fp32
-      constexpr int HELD = F32 ? NDT / KT : NDT;  // feature tiles that are kept until the next tile's loads are in
-      Pack8 x[F32 ? HELD : NDT / 2][4];
-      uint32_t tv = ldsV + troff;
-#if defined(__HIP_DEVICE_COMPILE__)
-      asm volatile("" : "+v"(tv));
-#endif
-      // V^T operands: those of the next KT products are read while KT products run
-      Pack8 vt[2][KT];
-      auto v_read = [&](auto hc) {  // half hc & 1 of feature tile hc / 2
-        constexpr int hb = decltype(hc)::value, dt = hb >> 1;
-        const uint32_t xlo = (uint32_t)(dt * 4 * 16), xhi = (uint32_t)(((dt * 4) ^ TileSwz<HD>::kRow8) * 16);
-#pragma unroll
-        for (int u = 0; u < KT; ++u) {
-          const int q = (hb & 1) * KT + u;  // key tile q / 2, half q & 1
-          const uint32_t olo = (uint32_t)(q * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
-          vt[hb & 1][u] = lds_tr8((tv ^ xlo) + olo, (tv ^ xhi) + ohi);
+        for (int i = 0; i < 16; ++i) {
+          const int jrel = kt * 32 + 8 * (i >> 2) + (i & 3) + 4 * hh;
+          st[kt][i] = jrel <= lim ? st[kt][i] : -INFINITY;
         }
-      };
-      v_read(std::integral_constant<int, 0>{});
-      // Rows leave through LDS, 128 bytes of each at a time, so that eight lanes store the 128 bytes of a row together: stored
-      // from where the products leave them (16 bytes per lane, 32 per row and instruction) every line went to memory
-      // in pieces, and the kernel took nearly twice as long (275 against 146 us at 8192 tokens).  Piece p of row r lies at piece p ^ (r & 7).
-      auto flush = [&](const Pack8(&piece)[4], int part) {
+    }
+    float m = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) lds_write_vec<u32x4_t>(ldsOut + (uint32_t)((lane & 31) * 128 + (((2 * e + hh) ^ (lane & 7)) * 16)), pack8_vec(piece[e]));
-        wave_lds_fence();
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) m = fmaxf(m, st[kt][i]);
+    m = max_xor32_f(m) * scale_log2;
+    const float m_use = m == -INFINITY ? 0.f : m;
+    float l = 0.f;
+    Pack8 pf[KT][2];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w], scale_log2, -m_use));
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + 2 * w + 1], scale_log2, -m_use));
+          l += p0 + p1;
+          pf[kt][s2].w[w] = pack2<T>(p0, p1);
+        }
+    l = sum_xor32_f(l);
+    constexpr bool NORM = kFwdNormalisedParts<T, HD>;
+    const float inv = NORM && l > 0.f ? 1.f / l : 0.f;
+    constexpr bool F32 = fwd_part_size(HD) == 4;
+    // a tile's partial rows, 128 bytes of every row at a time: 64 features in 16 bits, 32 features in fp32
+    constexpr int HELD = F32 ? NDT / KT : NDT;  // feature tiles that are kept until the next tile's loads are in
+    Pack8 x[F32 ? HELD : NDT / 2][4];
+    uint32_t tv = ldsV + troff;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(tv));
+#endif
+    // V^T operands: those of the next KT products are read while KT products run
+    Pack8 vt[2][KT];
+    auto v_read = [&](auto hc) {  // half hc & 1 of feature tile hc / 2
+      constexpr int hb = decltype(hc)::value, dt = hb >> 1;
+      const uint32_t xlo = (uint32_t)(dt * 4 * 16), xhi = (uint32_t)(((dt * 4) ^ TileSwz<HD>::kRow8) * 16);
+#pragma unroll
+      for (int u = 0; u < KT; ++u) {
+        const int q = (hb & 1) * KT + u;  // key tile q / 2, half q & 1
+        const uint32_t olo = (uint32_t)(q * 16 * RB), ohi = olo + (uint32_t)(8 * RB);
+        vt[hb & 1][u] = lds_tr8((tv ^ xlo) + olo, (tv ^ xhi) + ohi);
+      }
+    };
+    v_read(std::integral_constant<int, 0>{});
+    // Rows leave through LDS, 128 bytes of each at a time, so that eight lanes store the 128 bytes of a row together: stored
+    // from where the products leave them (16 bytes per lane, 32 per row and instruction) every line went to memory
+    // in pieces, and the kernel took nearly twice as long (275 against 146 us at 8192 tokens).  Piece p of row r lies at piece p ^ (r & 7).
+    auto flush = [&](const Pack8(&piece)[4], int part) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) lds_write_vec<u32x4_t>(ldsOut + (uint32_t)((lane & 31) * 128 + (((2 * e + hh) ^ (lane & 7)) * 16)), pack8_vec(piece[e]));
+      wave_lds_fence();
+      Pack8 y[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) y[k] = lds_read16(ldsOut + (uint32_t)((8 * k + (lane >> 3)) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) * 16)));
+      wave_lds_fence();
+      typedef std::conditional_t<F32, float, uint16_t> E;
+      const int f = (part * 8 + (lane & 7)) * (int)(16 / sizeof(E));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int p2 = __shfl(pidx, 8 * k + (lane >> 3), 64);
+        if (p2 >= 0 && f < D) st_stream16(reinterpret_cast<E *>(ws.part) + ((uint64_t)(uint32_t)p2 * (uint32_t)D + (uint32_t)f), y[k]);
+      }
+    };
+    // once the next tile's loads are in, what is held of this one leaves
+    auto flush_held = [&]() {
+      arrived();
+      if (pidx >= 0 && hh == 0) st_stream16(ws.hdr + pidx, Pack8{{__float_as_uint(m), __float_as_uint(l), (uint32_t)nb, 0u}});
+      // (the header past the caches, as the rows: written the ordinary way it cost 6 to 8 % of the kernel)
+#pragma unroll
+      for (int part = 0; part < (int)(sizeof(x) / sizeof(x[0])); ++part) flush(x[part], part);
+    };
+    f32x16 o;
+    static_for<2 * NDT>([&](auto hc) {
+      constexpr int hb = decltype(hc)::value, dt = hb >> 1;
+      if constexpr (hb + 1 < 2 * NDT) v_read(std::integral_constant<int, hb + 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr ((hb & 1) == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] = 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < KT; ++u) {
+        const int q = (hb & 1) * KT + u;
+        o = mfma32<T>(vt[hb & 1][u], pf[q >> 1][q & 1], o);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr ((hb & 1) == 0) return;
+      if constexpr (F32) {
         Pack8 y[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) y[k] = lds_read16(ldsOut + (uint32_t)((8 * k + (lane >> 3)) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) * 16)));
-        wave_lds_fence();
-        typedef std::conditional_t<F32, float, uint16_t> E;
-        const int f = (part * 8 + (lane & 7)) * (int)(16 / sizeof(E));
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int p2 = __shfl(pidx, 8 * k + (lane >> 3), 64);
-          if (p2 >= 0 && f < D) st_stream16(reinterpret_cast<E *>(ws.part) + ((uint64_t)(uint32_t)p2 * (uint32_t)D + (uint32_t)f), y[k]);
-        }
-      };
-      // once the next tile's loads are in, what is held of this one leaves
-      auto flush_held = [&]() {
-        arrived();
-        if (pidx >= 0 && hh == 0) st_stream16(ws.hdr + pidx, Pack8{{__float_as_uint(m), __float_as_uint(l), (uint32_t)nb, 0u}});
-        // (the header past the caches, as the rows: written the ordinary way it cost 6 to 8 % of the kernel)
+          for (int w = 0; w < 4; ++w) y[e].w[w] = __float_as_uint(o[4 * e + w]);
+        if constexpr (dt < HELD) {
 #pragma unroll
-        for (int part = 0; part < (int)(sizeof(x) / sizeof(x[0])); ++part) flush(x[part], part);
-      };
-      f32x16 o;
-      static_for<2 * NDT>([&](auto hc) {
-        constexpr int hb = decltype(hc)::value, dt = hb >> 1;
-        if constexpr (hb + 1 < 2 * NDT) v_read(std::integral_constant<int, hb + 1>{});
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr ((hb & 1) == 0) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[i] = 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < KT; ++u) {
-          const int q = (hb & 1) * KT + u;
-          o = mfma32<T>(vt[hb & 1][u], pf[q >> 1][q & 1], o);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr ((hb & 1) == 0) return;
-        if constexpr (F32) {
-          Pack8 y[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) y[e].w[w] = __float_as_uint(o[4 * e + w]);
-          if constexpr (dt < HELD) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[dt][e] = y[e];
-            if constexpr (dt == HELD - 1) flush_held();
-          } else {
-            flush(y, dt);
-          }
+          for (int e = 0; e < 4; ++e) x[dt][e] = y[e];
+          if constexpr (dt == HELD - 1) flush_held();
         } else {
-          if constexpr (NORM) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o[i] *= inv;
-          }
-          // four features per lane and group of eight: the two halves of the wave exchange, so that a lane stores eight
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-#pragma unroll
-            for (int w = 0; w < 2; ++w) {
-              const uint32_t ev = pack2<T>(o[8 * j + 2 * w], o[8 * j + 2 * w + 1]), od = pack2<T>(o[8 * j + 4 + 2 * w], o[8 * j + 4 + 2 * w + 1]);
-              Pack8 &y = x[dt >> 1][2 * (dt & 1) + j];
-#if defined(__HIP_DEVICE_COMPILE__)
-              auto sw = __builtin_amdgcn_permlane32_swap(ev, od, false, false);
-              y.w[w] = sw[0];
-              y.w[2 + w] = sw[1];
-#else
-              y.w[w] = ev, y.w[2 + w] = od;
-#endif
-            }
-          }
-          if constexpr (dt == NDT - 1) flush_held();
+          flush(y, dt);
         }
-      });
-    }
+      } else {
+        if constexpr (NORM) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[i] *= inv;
+        }
+        // four features per lane and group of eight: the two halves of the wave exchange, so that a lane stores eight
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const uint32_t ev = pack2<T>(o[8 * j + 2 * w], o[8 * j + 2 * w + 1]), od = pack2<T>(o[8 * j + 4 + 2 * w], o[8 * j + 4 + 2 * w + 1]);
+            Pack8 &y = x[dt >> 1][2 * (dt & 1) + j];
+#if defined(__HIP_DEVICE_COMPILE__)
+            auto sw = __builtin_amdgcn_permlane32_swap(ev, od, false, false);
+            y.w[w] = sw[0];
+            y.w[2 + w] = sw[1];
+#else
+            y.w[w] = ev, y.w[2 + w] = od;
+#endif
+          }
+        }
+        if constexpr (dt == NDT - 1) flush_held();
+      }
+    });
   }
 }
 
@@ -559,13 +583,14 @@ static int fwd_col_heads(const fmoba_attn_fwd_args &a, int kb) {
   const int64_t blocks = (int64_t)a.total_k / kb + a.batch;
   const int64_t tiles = (int64_t)a.total_q * fwd_partial_cap(a) / 32 / blocks;  // of one head's lists, on average
   int best = grp;
-  for (int gs = grp - 1; gs >= 1 && blocks * (a.heads / best) < 1536 && tiles * gs >= 8; --gs)
+  while (best > 64 || grp % best != 0) --best;  // (a lane of the kernel's waves per list)
+  for (int gs = best - 1; gs >= 1 && blocks * (a.heads / best) < 1536 && tiles * gs >= 8; --gs)
     if (grp % gs == 0) best = gs;
   return best;
 }
 template <typename T, int HD, int KB>
 static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStream_t s) {
-  auto kern = attn_fwd_col_kernel<T, HD, KB>;
+  auto kern = a.head_dim == HD ? attn_fwd_col_kernel<T, HD, KB, true> : attn_fwd_col_kernel<T, HD, KB, false>;
   const size_t smem = FwdColSmem<HD, KB>::bytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
