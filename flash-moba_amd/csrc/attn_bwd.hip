@@ -60,8 +60,24 @@ struct BwdWs {
   int32_t *pid;    // [total_q * heads * cap] key block id of each partial
   uint16_t *part;  // [total_q * heads * cap][head_dim] dQ partials (times dq_part_scale)
   int32_t cap;
+  int32_t *tab;    // dS form: first list position of every column in every block of kDqRows query rows (RunTable)
   uint16_t *ds;    // dS tiles (row-stationary dQ form): [row list position / 32][key of the column / 8][position % 32][8 keys]
 };
+
+// Where the lists of the columns enter the row blocks of the dQ pass: [head][column][row block, and one past the last], the columns
+// of sequence b from number cu_seqlens_k[b] / Bn + b on (which leaves every sequence room for its own).  The delta pass looks the places
+// up, a wave per column, in front of its rows; found by every workgroup of the dQ pass for its own row block, two searches of
+// a dozen dependent loads per column, they were a quarter of that pass on short sequences.  Delta and dQ pass, and the clearing of the
+// padded delta that was a launch of its own: 8191 tokens of short documents 43.4 -> 36.6 us, 24571 tokens, 32 over 8 heads 728 -> 697,
+// 65536 tokens in eight sequences 1675 -> 1656 (12 M probes take 25 us of the delta pass and 40 out of the dQ pass).
+constexpr int kDqRows = 256;
+struct RunTable {
+  int cols, blocks;  // columns of all sequences, row blocks + 1
+  __host__ __device__ __forceinline__ int64_t at(int h, int col) const { return ((int64_t)h * cols + col) * blocks; }
+};
+static inline RunTable bwd_run_table(const fmoba_attn_bwd_args &a) {
+  return RunTable{a.total_k / a.lg_block_n + a.batch, ceil_div(a.max_seqlen_q, kDqRows) + 1};
+}
 
 // Softmax scale of dQ in the partials form: fp16 partial rows carry it (as far as it makes them smaller), the sums of bf16 ones get it.
 // Without it the rows are sqrt(head_dim) times the gradient they add up to, and fp16 rows overflow where the gradient does not.
@@ -1210,7 +1226,7 @@ __device__ __forceinline__ DqItem dq_decode_item(int id, int npairs, int nsb_max
 
 // RT: 32-row tiles per wave (with two, every K^T operand read from LDS feeds two MFMAs).  NW: waves.
 template <typename T, int HD, int RT, int NW>
-__global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, int nsb_max) {
+__global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int nsb_max) {
   typedef DqSmem<HD, RT, NW> SM;
   constexpr int ROWS = SM::ROWS;  // query rows of the workgroup
   constexpr int LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
@@ -1252,6 +1268,8 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
   if (causal) ncols = last_rowpos < 0 ? 0 : min(ncols, last_rowpos / Bn + 1);
   const int64_t bh = (int64_t)b * a.heads + h;
   const int64_t *coff = a.col_offsets + bh * a.max_cols;
+  static_assert(ROWS == kDqRows, "the row blocks of the table");
+  const int32_t *runs = tab + rt_.at(h, k0 / Bn + b) + sb;  // of column 0; column c: rt_.blocks further on each
   const uint16_t *kp = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)k0 * a.k_row_stride + (int64_t)hk * a.k_head_stride;
   const int cols_per_batch = min(kDqColBatch, kDqMaxSteps / nsub);
 
@@ -1266,10 +1284,9 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
       int64_t base = 0;
       if (nnz > 0) {
         base = coff[c];
-        const int32_t *list = a.row_indices + base;
-        lo = lower_bound_i32(list, nnz, m0);
-        const int hi = lo + lower_bound_i32(list + lo, nnz - lo, m0 + ROWS);
-        cnt = min(hi - lo, ROWS);
+        const int32_t *run = runs + (int64_t)c * rt_.blocks;
+        lo = min(max(run[0], 0), nnz);
+        cnt = min(min(max(run[1], lo), nnz) - lo, ROWS);
       }
       sLo[c - cb] = lo;
       sCnt[c - cb] = cnt;
@@ -1577,12 +1594,54 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
 // LPR lanes cooperate on one row (LPR = power of two >= head_dim / 8).
 constexpr int kPrepRows = 4;  // rows per thread: eight 16-byte loads in flight (with one row a thread had two, 4.7 TB/s)
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int LPR) {
+__global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int LPR, int32_t *tab, RunTable rt, int ztab) {
   const int rows_per_pass = 256 / LPR;
-  const int h = blockIdx.y, b = blockIdx.z;
+  if ((int)blockIdx.z < ztab) {  // four columns of the run table, before everything else: a chain of loads that the rows cover
+    const int lane = threadIdx.x & 63, Bn = a.lg_block_n, h = blockIdx.y;
+    const int64_t col = ((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (col >= rt.cols) return;
+    // the sequence: the last one whose columns begin at or before this one
+    int lo = 0, hi = a.batch;  // columns of sequence lo begin at or before it, those of hi do not
+    while (hi - lo > 1) {
+      const int step = (hi - lo + 63) >> 6, q = lo + lane * step;
+      const int below = max(1, (int)__popcll(__ballot(q < hi && a.cu_seqlens_k[q] / Bn + q <= col)));
+      lo += (below - 1) * step;
+      hi = min(lo + step, hi);
+    }
+    const int c = (int)col - (a.cu_seqlens_k[lo] / Bn + lo);
+    if (c < 0 || c >= a.max_cols || c * Bn >= a.cu_seqlens_k[lo + 1] - a.cu_seqlens_k[lo]) return;
+    const int64_t ci = ((int64_t)lo * a.heads + h) * a.max_cols + c;
+    const int nnz = a.col_nnz[ci];
+    const int32_t *list = a.row_indices + a.col_offsets[ci];
+    // G lanes per boundary: a step of the search narrows it G + 1 times (short sequences have few boundaries and wait for the steps)
+    int G = 64;
+    while (G > 1 && G * rt.blocks > 64) G >>= 1;
+    const int li = lane % G;
+    const unsigned long long mine = (G == 64 ? ~0ull : (1ull << G) - 1) << (lane - li);
+    for (int rb0 = 0; rb0 < rt.blocks; rb0 += 64 / G) {
+      const int rb = rb0 + lane / G, v = rb * kDqRows;
+      int l = 0, r = nnz;
+      while (__any(l < r)) {
+        const int step = (r - l + G) / (G + 1), q = l + (li + 1) * step - 1;
+        const int below = __popcll(__ballot(l < r && q < r && list[q] < v) & mine);
+        l += below * step;
+        r = below < G ? min(l + step - 1, r) : r;
+      }
+      if (li == 0 && rb < rt.blocks) tab[rt.at(h, (int)col) + rb] = l;
+    }
+    return;
+  }
+  const int h = blockIdx.y, b = blockIdx.z - ztab;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+  if (blockIdx.x == 0) {  // what lies between the sequences of the padded layout is zero
+    float *dh = a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch);
+    const int64_t end = b == a.batch - 1 ? (int64_t)a.total_q + 128 * (int64_t)a.batch : (int64_t)q0 + Lq + 128 * (int64_t)(b + 1);
+    for (int64_t i = (int64_t)q0 + Lq + 128 * (int64_t)b + threadIdx.x; i < end; i += 256) dh[i] = 0.f;
+    if (b == 0)
+      for (int i = threadIdx.x; i < q0; i += 256) dh[i] = 0.f;
+  }
   const int r0 = blockIdx.x * rows_per_pass * kPrepRows + threadIdx.x / LPR;
-  if (blockIdx.x * rows_per_pass * kPrepRows >= Lq) return;
+  if ((int)(blockIdx.x * rows_per_pass * kPrepRows) >= Lq) return;
   const int sub = threadIdx.x % LPR;
   const int e = sub * 8;
   const int D = a.head_dim;
@@ -1661,7 +1720,7 @@ static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, h
 }
 
 template <typename T, int HD, int RT, int NW>
-static int launch_dq(const fmoba_attn_bwd_args &a, const uint16_t *ws, hipStream_t s) {
+static int launch_dq(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   auto kern = attn_bwd_dq_kernel<T, HD, RT, NW>;
   const size_t smem = DqSmem<HD, RT, NW>::bytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
@@ -1674,7 +1733,7 @@ static int launch_dq(const fmoba_attn_bwd_args &a, const uint16_t *ws, hipStream
     set_error("attn_bwd: too many (sequence, head, superblock) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * NW), smem, s, a, ws, nsb_max);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * NW), smem, s, a, ws.ds, ws.tab, bwd_run_table(a), nsb_max);
   return 0;
 }
 
@@ -1728,15 +1787,22 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
   if (phases & FMOBA_BWD_PREP) {
     int lpr = 1;
     while (lpr * 8 < a.head_dim) lpr <<= 1;
-    const int rows_per_block = 256 / lpr;
-    hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(ceil_div(a.max_seqlen_q, rows_per_block * kPrepRows), a.heads, a.batch), dim3(256), 0, s, a, lpr);
+    const int nx = ceil_div(a.max_seqlen_q, 256 / lpr * kPrepRows);
+    const RunTable rt = bwd_run_table(a);
+    const int ztab = partials ? 0 : (int)ceil_div64(ceil_div(rt.cols, 4), nx);
+    if (a.batch + ztab <= 65535) {
+      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lpr, ws.tab, rt, ztab);
+    } else {  // (more planes than a launch has)
+      if (ztab > 0) hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(ceil_div(rt.cols, 4), a.heads, 1), dim3(256), 0, s, a, lpr, ws.tab, rt, 1);
+      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch), dim3(256), 0, s, a, lpr, ws.tab, rt, 0);
+    }
   }
   if (a.head_dim > 128) {
     // the plain feature-split dK/dV kernel (attn_bwd_wide.hip), then the row-block dQ pass over its dS tiles
     if (phases & FMOBA_BWD_DKDV)
       if (int rc = run_bwd_dkdv_wide(a, ws.ds, s)) return rc;
     if (phases & FMOBA_BWD_DQ)
-      if (int rc = launch_dq<T, 256, 1, 8>(a, ws.ds, s)) return rc;
+      if (int rc = launch_dq<T, 256, 1, 8>(a, ws, s)) return rc;
     return 0;
   }
   if (phases & FMOBA_BWD_DKDV) {
@@ -1761,7 +1827,7 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
       }
       hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 15) / 16)), dim3(256), smem, s, a, ws, capl);
     } else {
-      int rc = a.head_dim <= 64 ? launch_dq<T, 64, 1, 8>(a, ws.ds, s) : a.head_dim <= 96 ? launch_dq<T, 96, 2, 4>(a, ws.ds, s) : launch_dq<T, 128, 2, 4>(a, ws.ds, s);
+      int rc = a.head_dim <= 64 ? launch_dq<T, 64, 1, 8>(a, ws, s) : a.head_dim <= 96 ? launch_dq<T, 96, 2, 4>(a, ws, s) : launch_dq<T, 128, 2, 4>(a, ws, s);
       if (rc) return rc;
     }
   }
@@ -1786,7 +1852,10 @@ extern "C" int32_t fmoba_attn_bwd_dkv_heads(const fmoba_attn_bwd_args *a) {
 extern "C" size_t fmoba_attn_bwd_workspace_bytes(const fmoba_attn_bwd_args *a) {
   using namespace fmoba;
   if (a == nullptr || a->total_q <= 0 || a->heads <= 0 || a->head_dim <= 0 || a->batch <= 0 || a->lg_block_n <= 0) return 256;
-  if (!bwd_dq_partials(*a)) return ds_workspace_tiles(a->num_row_indices) * (size_t)a->lg_block_n * 64 + 256;
+  if (!bwd_dq_partials(*a)) {
+    const RunTable rt = bwd_run_table(*a);
+    return ds_workspace_tiles(a->num_row_indices) * (size_t)a->lg_block_n * 64 + bwd_align256((size_t)rt.at(a->heads, 0) * 4) + 256;
+  }
   const size_t rows = (size_t)a->total_q * a->heads, cap = (size_t)bwd_partial_cap(*a);
   // one spare partial row / block id at the end takes the writes of absent rows
   return bwd_align256(rows * 4) + bwd_align256((rows * cap + 1) * 4) + bwd_align256((rows * cap + 1) * a->head_dim * 2) + 256;
@@ -1839,10 +1908,10 @@ extern "C" int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_
     return 0;
   }
   FMOBA_REQUIRE(a->dout && a->q && a->out && a->softmax_lse && a->dq && a->softmax_d, "attn_bwd: null pointer");
-  if (phases & FMOBA_BWD_PREP)
-    hipLaunchKernelGGL(zero_f32_kernel, dim3(256), dim3(256), 0, s, a->softmax_d, (int64_t)a->heads * ((int64_t)a->total_q + 128 * (int64_t)a->batch));
   if (a->total_k == 0 || a->max_seqlen_k == 0 || a->max_cols == 0) {
     // no keys: dq = 0
+    if (phases & FMOBA_BWD_PREP)
+      hipLaunchKernelGGL(zero_f32_kernel, dim3(256), dim3(256), 0, s, a->softmax_d, (int64_t)a->heads * ((int64_t)a->total_q + 128 * (int64_t)a->batch));
     hipLaunchKernelGGL(zero_rows_kernel, dim3(1024), dim3(256), 0, s, a->dq, (int64_t)a->total_q, a->dq_row_stride, a->heads, a->dq_head_stride, a->head_dim);
     FMOBA_LAUNCH_CHECK("attn_bwd(no keys)");
     return 0;
@@ -1860,7 +1929,8 @@ extern "C" int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_
   // (the dK/dV pass keeps the place of a visit's dQ partial as a 32-bit index of partial rows)
   FMOBA_REQUIRE(!fmoba::bwd_dq_partials(*a) || rows * (size_t)ws.cap + 1 < ((size_t)1 << 31),
                 "attn_bwd: %zu rows x heads with up to %d dQ partials each are more partial rows than the partials form addresses", rows, ws.cap);
-  ws.ds = reinterpret_cast<uint16_t *>(wp);
+  ws.tab = reinterpret_cast<int32_t *>(wp);
+  ws.ds = reinterpret_cast<uint16_t *>(wp + bwd_align256((size_t)bwd_run_table(*a).at(a->heads, 0) * 4));
   ws.cnt = reinterpret_cast<int32_t *>(wp);
   wp += bwd_align256(rows * 4);
   ws.pid = reinterpret_cast<int32_t *>(wp);

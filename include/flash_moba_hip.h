@@ -252,7 +252,8 @@ int32_t fmoba_attn_bwd_uses_partials(const fmoba_attn_bwd_args *a);
 size_t fmoba_attn_bwd_workspace_bytes(const fmoba_attn_bwd_args *a);
 int fmoba_attn_bwd(const fmoba_attn_bwd_args *a, void *stream);
 /* The same call split into its three launches so that each can be timed on its own:
- * phases is a bit mask, 1 = dot(dO, O) (flash_bwd_launch_template.h:70-74), 2 = the
+ * phases is a bit mask, 1 = dot(dO, O) (flash_bwd_launch_template.h:70-74) and, in the workspace that
+ * the phases of a call share, where the column lists enter the row blocks of the dQ pass, 2 = the
  * column-stationary dK/dV kernel, which also fills the workspace (:76-96), 4 = the dQ pass
  * in either form (stands where the reference converts its fp32 dQ accumulator, :98-104).  fmoba_attn_bwd(a, s) == fmoba_attn_bwd_phases(a, 7, s). */
 #define FMOBA_BWD_PREP 1

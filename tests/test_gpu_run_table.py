@@ -1,0 +1,45 @@
+"""Where the column lists enter the row blocks of the dQ pass, and the padded layout of softmax_d: both come from the delta pass."""
+import numpy as np
+import pytest
+import torch
+
+import flash_moba
+from flash_moba import flash_moba_hip as hip
+from gpu_utils import assert_close
+
+pytestmark = pytest.mark.gpu
+
+MANY = [0, 1, 63, 64, 65, 255, 256, 257, 300, 513]
+
+
+# rows at the edges of 256-row blocks; more sequences than one step of the search for a column's sequence takes (64 and 64 * 64 are its
+# steps), empty ones among them; queries that are the last rows of longer sequences; more boundaries than a wave has lanes
+@pytest.mark.parametrize("lens_q,lens_k,D,chunk,topk", [
+    (MANY * 13, MANY * 13, 32, 64, 3), ([1] * 4200, [1] * 4200, 32, 64, 2), ([255, 0, 257], [900, 70, 257], 64, 128, 2),
+    ([100, 513], [1100, 600], 96, 64, 4), ([17000], [17000], 32, 256, 8), ([300], [300], 128, 64, 3)])
+def test_dq_over_row_blocks_agrees_with_partial_rows(lens_q, lens_k, D, chunk, topk):
+    H = 2
+    g = torch.Generator(device="cuda").manual_seed(sum(lens_q) + D)
+    mk = lambda n: torch.randn((n, H, D), generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v, dout = mk(sum(lens_q)), mk(sum(lens_k)), mk(sum(lens_k)), mk(sum(lens_q))
+    cq, ck = (torch.tensor([0] + list(np.cumsum(x)), dtype=torch.int32, device="cuda") for x in (lens_q, lens_k))
+    mq, mkk, scale = max(lens_q), max(lens_k), D ** -0.5
+    causal = mq > 1  # (as the attention entry points have it)
+    csc = flash_moba.flash_topk_varlen_func(q, k, cq, ck, mq, mkk, topk, chunk, causal=causal)
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *csc, cq, ck, None, None, None, mq, mkk, 0.0, scale, False, causal, 0.0, False, 128, chunk, None)
+    run = lambda mode: hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, *csc, cq, ck, None, mq, mkk, 0.0, scale, False, causal, 0.0, False,
+                                           128, chunk, None, _dq_mode=mode)
+    dq, dk, dv, sd = run(1)
+    want = run(2)
+    # (the bounds of the other attention tests: 16-bit results of sums of 16-bit factors, and 16-bit partial rows on one side)
+    for name, x, y in zip(("dq", "dk", "dv"), (dq, dk, dv), want):
+        assert_close(name, x, y, 2e-2, 1e-2)
+    assert torch.equal(sd, want[3])
+    delta = (out.float() * dout.float()).sum(-1).T
+    layout, pad = torch.zeros_like(sd), torch.ones(sd.shape[1], dtype=torch.bool, device="cuda")
+    for b, (s, n) in enumerate(zip(np.cumsum([0] + lens_q), lens_q)):
+        layout[:, s + 128 * b:s + 128 * b + n] = delta[:, s:s + n]
+        pad[s + 128 * b:s + 128 * b + n] = False
+    # (fp32 sums of D products in another order: a few 2^-24 of the sum of their magnitudes, which is below D here)
+    assert (sd - layout).abs().max() < 1e-5 * D
+    assert (sd[:, pad] == 0).all()
