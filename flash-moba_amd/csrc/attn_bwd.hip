@@ -60,6 +60,8 @@ struct BwdWs {
   int32_t *pid;    // [total_q * heads * cap] key block id of each partial
   uint16_t *part;  // [total_q * heads * cap][head_dim] dQ partials (times dq_part_scale)
   int32_t cap;
+  const uint32_t *visits;  // as in the forward pass (null: slots from the counters)
+  int32_t row_mask;        // of list entries: kListRowMask for ranked lists, else -1
   int32_t *tab;    // dS form: first list position of every column in every block of kDqRows query rows (RunTable)
   uint16_t *ds;    // dS tiles (row-stationary dQ form): [row list position / 32][key of the column / 8][position % 32][8 keys]
 };
@@ -135,7 +137,8 @@ struct DkdvSmem {
   static_assert(bytes <= 160 * 1024 && (size_t)64 * HD * 2 <= NBUF * tile, "LDS of one compute unit; K and V pass through the tiles");
 };
 
-template <typename T, int HD, bool DQP>
+// RANKED (partials form): part rows go to the place of the block among the row's, which the rank of the list entry gives
+template <typename T, int HD, bool DQP, bool RANKED>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
   typedef DkdvSmem<HD, DQP> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR, PRB = SM::PRB;
@@ -195,7 +198,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
     for (int g = 0; g < gs; ++g) {
       const int n = __builtin_amdgcn_readlane(nnz, g);
       const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)lbase, g), bhi = __builtin_amdgcn_readlane((uint32_t)(lbase >> 32), g);
-      const int st = n > 0 ? lower_bound_wave_i32(a.row_indices + (int64_t)(((uint64_t)bhi << 32) | blo), n, key0 - off) : 0;
+      const int st = n > 0 ? lower_bound_wave_i32(a.row_indices + (int64_t)(((uint64_t)bhi << 32) | blo), n, key0 - off, ws.row_mask) : 0;
       start = lane == g ? st : start;
     }
   }
@@ -239,7 +242,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
   const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
   auto entry_at = [&](const Round &w) { return a.row_indices + w.pos + min(myrow, w.n - 1); };
-  auto code = [&](int raw, const Round &w) { return tile_row_code(raw, myrow < w.n, Lq); };
+  const int nsub = Bn / NKEY, jsub = koff / NKEY;  // key blocks of the column, this one's number
+  auto code = [&](int raw, const Round &w) { return tile_row_code(raw & ws.row_mask, myrow < w.n, Lq); };
   Round w0{}, w1{};  // the round at hand and the one after it
   int raw0 = 0, raw_nx = 0;
   if (nround > 0) {
@@ -295,11 +299,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
     int *sSlot = reinterpret_cast<int *>(smem + SM::oSlot);
     const int trash = a.total_q * a.heads * ws.cap;  // a spare part row: takes what absent rows and visits beyond the caller's bound write
     // LSE, delta and (partials form, handed out by the waves of key quarter 0) the part row of a round's rows
-    auto scalars = [&](int rid, const Round &w, bool counted) {
+    auto scalars = [&](int rid, int rank, const Round &w, bool counted) {
       const int rc = rid & 0x7fffffff;
       lse = a.softmax_lse[(int64_t)w.h * a.total_q + q0 + rc];
       del = a.softmax_d[(int64_t)w.h * dstride + q0 + 128 * b + rc];
-      if constexpr (DQP) slot = take_slot(ws.cnt + ((int64_t)(q0 + rc) * a.heads + w.h), __ballot(rid >= 0 && hh == 0 && kq == 0 && counted));
+      if constexpr (DQP && RANKED)
+        slot = rank * nsub + jsub;
+      else if constexpr (DQP)
+        slot = take_slot(ws.cnt + ((int64_t)(q0 + rc) * a.heads + w.h), __ballot(rid >= 0 && hh == 0 && kq == 0 && counted));
     };
     auto arrived = [&]() {
       wait_all_loads();
@@ -307,7 +314,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
       asm volatile("" : "+v"(lse), "+v"(del), "+v"(raw_nx), "+v"(slot));
 #endif
     };
-    scalars(rid0, w0, true);
+    int rank1 = raw_nx >> kListRowBits;  // (of ranked lists)
+    scalars(rid0, raw0 >> kListRowBits, w0, true);
     arrived();
     __syncthreads();
     uint32_t buf = 0u;
@@ -326,7 +334,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
       }
       // the next round's rows and scalars, the row ids of the one after it
       if (r + 1 < nround) feed(rid1, w1, buf ^ TILE);
-      scalars(rid1, w1, r + 1 < nround);
+      scalars(rid1, rank1, w1, r + 1 < nround);
       raw_nx = *entry_at(w2);
       // S^T and dP^T: lane -> row, register i -> key kq * 32 + acc_row(i, hh)
       f32x16 s, dp;
@@ -440,7 +448,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
           const uint32_t p = (uint32_t)sSlot[(r & 1) * 64 + row];
           const Pack8 x = lds_read16(ldsOut + (uint32_t)(row * RB) + (((uint32_t)pcs ^ (uint32_t)(row & 7)) * 16u));
           if (pcs * 8 < D) st_stream16(ws.part + ((uint64_t)p * (uint32_t)D + (uint32_t)(pcs * 8)), x);
-          if (pcs == 0) ws.pid[p] = nb;
+          if (!RANKED && pcs == 0) ws.pid[p] = nb;
         }
       } else {
         arrived();
@@ -455,7 +463,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
         __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
       }
       w0 = w1, rid0 = rid1;
-      w1 = w2, rid1 = code(raw_nx, w2);
+      w1 = w2, rid1 = code(raw_nx, w2), rank1 = raw_nx >> kListRowBits;
       buf ^= TILE;
     }
     __syncthreads();  // (the last part rows have left LDS)
@@ -510,7 +518,7 @@ __device__ __forceinline__ uint32_t mul24_u32(uint32_t a, uint32_t b) {
 // leaves one dQ partial instead of two.
 // NEAR: the host has checked that a gathered row's place in q and dout is a 32-bit byte offset from the sequence's first
 // row that one 24-bit multiply makes (launch_dkdv); otherwise the loads take 64-bit addresses per lane.
-template <typename T, int HD, int KB, bool NEAR>
+template <typename T, int HD, int KB, bool NEAR, bool RANKED>
 __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
   typedef BwdSmem<HD> SM;
   constexpr int KS = HD / 16, LDQ = SM::LDQ, LDS_ = SM::LDS_, NDT = HD / 32, VPR = HD / 8, LDR = SM::LDR;
@@ -583,23 +591,27 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
   // began at the head of the list (it does unless rows of the list lie before the block); otherwise they are
   // fetched again.
   int spec01[2] = {0, 0};
+  const int nsub = Bn / NKEY, jsub = (key0 - c * Bn) / NKEY;  // key blocks of the column, this one's number
   if (tid < kBwdRoundRows && nnz > 0) {
 #pragma unroll
     for (int sr = 0; sr < 2; ++sr) spec01[sr] = a.row_indices[lbase + min(sr * kBwdRoundRows + tid, nnz - 1)];
   }
   int start = 0;
   // rows r with r + off < key0 see no key of this block
-  if (causal && nnz > 0) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off);
+  constexpr int row_mask = RANKED ? kListRowMask : -1;
+  if (causal && nnz > 0) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off, row_mask);
   const int32_t *list = a.row_indices + lbase + start;
   const int n = nnz - start;               // rows of the list that the block walks
   const int nround = (n + kBwdRoundRows - 1) / kBwdRoundRows;
   int rid01[2] = {-1, -1};         // threads 0..127: row ids of rounds 0 and 1
+  int rank01[2] = {0, 0};
   if (tid < kBwdRoundRows && n > 0) {
 #pragma unroll
     for (int sr = 0; sr < 2; ++sr) {
       const int j = sr * kBwdRoundRows + tid;
       const int r = start == 0 ? spec01[sr] : list[min(j, n - 1)];
-      rid01[sr] = tile_row_code(r, j < n, Lq);
+      rid01[sr] = tile_row_code(r & row_mask, j < n, Lq);
+      rank01[sr] = r >> kListRowBits;
     }
   }
 
@@ -664,6 +676,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
     // per-row scalars: the row id of round s+2 (it has to be in LDS one round before the tile loads that use it),
     // and LSE, delta and the dQ-partial slot of round s+1.
     const uint32_t ldsQ = (uint32_t)(uintptr_t)(smem + SM::oQ), ldsdO = (uint32_t)(uintptr_t)(smem + SM::odO);
+    int v_rank = rank01[1];  // RANKED: the rank of the entry of v_rid
     int n_rid = -1, v_rid = rid01[1], m_rid = -1, m_slot = 0;  // v_rid: the checked row id that was stored last = the one of the next round
     float m_lse = 0.f, m_del = 0.f;
     int ft = tid;  // thread index for the feeding code, re-made opaque in every round (see below)
@@ -675,18 +688,22 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
     auto rid_store = [&](int sr) {
       if (tid < kBwdRoundRows) {
         const int j = sr * kBwdRoundRows + ft;
-        v_rid = tile_row_code(n_rid, j < n, Lq);
+        v_rid = tile_row_code(n_rid & row_mask, j < n, Lq);
+        v_rank = n_rid >> kListRowBits;
         sRid[(sr & 1) * kBwdRoundRows + ft] = v_rid;
       }
     };
-    auto meta_issue = [&](int rid) {  // rid: this thread's row of the round after the current one
+    auto meta_issue = [&](int rid, int rank) {  // rid: this thread's row of the round after the current one
       if (tid < kBwdRoundRows) {
         m_rid = rid;
         const int rc = max(m_rid, 0);
         m_lse = lseg[rc];
         m_del = delg[rc];
         // every visit of a (row, key block) pair takes one dQ-partial slot of the row
-        if (m_rid >= 0) m_slot = atomicAdd(cntg + (int64_t)m_rid * a.heads, 1);
+        if constexpr (RANKED)
+          m_slot = rank * nsub + jsub;
+        else if (m_rid >= 0)
+          m_slot = atomicAdd(cntg + (int64_t)m_rid * a.heads, 1);
       }
     };
     const int64_t trash = (int64_t)a.total_q * a.heads * ws.cap;  // spare row: takes the writes of absent rows, no branch
@@ -769,7 +786,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
       sRid[kBwdRoundRows + tid] = rid01[1];
     }
     __syncthreads();  // K, V are in registers; the row ids of rounds 0 and 1 are in LDS
-    meta_issue(rid01[0]);
+    meta_issue(rid01[0], rank01[0]);
     tile_issue(0);
     meta_store(0);
     wait_all_loads();
@@ -996,7 +1013,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
           st_stream16(ws.part + ((uint64_t)pidx[k] * (uint32_t)D + (uint32_t)(kq * (NDH * 32) + col)), x);
         }
       }
-      if (kq == 0 && col == 0) {
+      if (!RANKED && kq == 0 && col == 0) {
 #pragma unroll
         for (int k = 0; k < 32 / RPP; ++k) ws.pid[pidx[k]] = nb;
       }
@@ -1092,7 +1109,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
       asm volatile("" : "+v"(ft));
 #endif
       rid_issue(r + 2);
-      meta_issue(v_rid);
+      meta_issue(v_rid, v_rank);
       if constexpr (kSpreadLoads)
         tile_rows(r + 1);
       else
@@ -1226,7 +1243,7 @@ __device__ __forceinline__ DqItem dq_decode_item(int id, int npairs, int nsb_max
 
 // RT: 32-row tiles per wave (with two, every K^T operand read from LDS feeds two MFMAs).  NW: waves.
 template <typename T, int HD, int RT, int NW>
-__global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int nsb_max) {
+__global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int row_mask, int nsb_max) {
   typedef DqSmem<HD, RT, NW> SM;
   constexpr int ROWS = SM::ROWS;  // query rows of the workgroup
   constexpr int LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
@@ -1365,7 +1382,7 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
       const int4 info = sInfo[min(step, nsteps - 1)];
       const int n = __builtin_amdgcn_readfirstlane(info.y) & 0xffff;
       const int64_t pos0 = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane(info.z) | ((int64_t)__builtin_amdgcn_readfirstlane(info.w) << 32);
-      return a.row_indices[pos0 + min(tid & (ROWS - 1), n - 1)];
+      return a.row_indices[pos0 + min(tid & (ROWS - 1), n - 1)] & row_mask;
     };
     auto put_pos = [&](int step, int rr) {  // thread t tells row rr, the t-th of the step's run, where it is
       if (step < nsteps && tid < ROWS) {
@@ -1536,7 +1553,7 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
 // sixteen per block of 256: a row's chain of dependent steps (count, ids, order, rows) is mostly waiting, so a wave
 // runs four of them side by side.  Lane li of a group owns the 16-byte piece li of the row.
 // ------------------------------------------------------------------------------------
-template <typename T>
+template <typename T, bool RANKED>
 __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd_args a, BwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, grp = lane >> 4, li = lane & 15;
@@ -1549,7 +1566,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
   const int64_t row = rh / a.heads;
   const int h = (int)(rh - row * a.heads);
   const int D = a.head_dim;
-  const int nall = valid ? ws.cnt[rh] : 0;
+  const int nall = !valid ? 0 : RANKED ? (int)(ws.visits[(int64_t)h * a.total_q + row] >> 16) : ws.cnt[rh];
   const int n = min(nall, ws.cap);
   if (nall > ws.cap && li == 0 && a.visits_overflow != nullptr) atomicMax(a.visits_overflow, nall);  // visits were dropped
   int nmax = max(n, __shfl_xor(n, 16, 64));
@@ -1562,7 +1579,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
   // ranks over the whole row: the order of the sum does not depend on which slot a visit got
-  group_rank_order(pid, 1, n, nmax, sOrd, lane);
+  if constexpr (!RANKED) group_rank_order(pid, 1, n, nmax, sOrd, lane);
   if (mine) {
     auto add = [&](const Pack8 &x) {
 #pragma unroll
@@ -1575,11 +1592,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
     for (; t + 4 <= n; t += 4) {  // independent loads, four in flight
       Pack8 x[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) x[u] = ld_stream16(part + (int64_t)sOrd[t + u] * D + c8);
+      for (int u = 0; u < 4; ++u) x[u] = ld_stream16(part + (int64_t)(RANKED ? t + u : sOrd[t + u]) * D + c8);
 #pragma unroll
       for (int u = 0; u < 4; ++u) add(x[u]);
     }
-    for (; t < n; ++t) add(ld_stream16(part + (int64_t)sOrd[t] * D + c8));
+    for (; t < n; ++t) add(ld_stream16(part + (int64_t)(RANKED ? t : sOrd[t]) * D + c8));
   }
   if (valid && mine) {
     const float scale = dq_sum_scale<T>(a.softmax_scale);
@@ -1594,7 +1611,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
 // LPR lanes cooperate on one row (LPR = power of two >= head_dim / 8).
 constexpr int kPrepRows = 4;  // rows per thread: eight 16-byte loads in flight (with one row a thread had two, 4.7 TB/s)
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int LPR, int32_t *tab, RunTable rt, int ztab) {
+__global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int LPR, int32_t *tab, RunTable rt, int row_mask, int ztab) {
   const int rows_per_pass = 256 / LPR;
   if ((int)blockIdx.z < ztab) {  // four columns of the run table, before everything else: a chain of loads that the rows cover
     const int lane = threadIdx.x & 63, Bn = a.lg_block_n, h = blockIdx.y;
@@ -1623,7 +1640,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
       int l = 0, r = nnz;
       while (__any(l < r)) {
         const int step = (r - l + G) / (G + 1), q = l + (li + 1) * step - 1;
-        const int below = __popcll(__ballot(l < r && q < r && list[q] < v) & mine);
+        const int below = __popcll(__ballot(l < r && q < r && (list[q] & row_mask) < v) & mine);
         l += below * step;
         r = below < G ? min(l + step - 1, r) : r;
       }
@@ -1707,7 +1724,9 @@ static int launch_dkdv_kernel(K kern, size_t smem, int heads, int keys, const fm
 }
 template <typename T, int HD, bool DQP>
 static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
-  return launch_dkdv_kernel(attn_bwd_dkdv_kernel<T, HD, DQP>, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
+  if constexpr (DQP)
+    if (ws.visits != nullptr) return launch_dkdv_kernel(attn_bwd_dkdv_kernel<T, HD, DQP, true>, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
+  return launch_dkdv_kernel(attn_bwd_dkdv_kernel<T, HD, DQP, false>, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
 }
 // NEAR: every row of a sequence's q and dout lies within 2 GB of the sequence's first row and is less than 2^24 rows
 // and 2^22 elements per row away, so a gathered row's place is a 32-bit offset made by one 24-bit multiply.
@@ -1715,8 +1734,9 @@ template <typename T, int HD, int KB>
 static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   const bool near_rows = a.max_seqlen_q < (1 << 24) && a.q_row_stride < (1 << 22) && a.do_row_stride < (1 << 22) &&
                          (int64_t)a.max_seqlen_q * a.q_row_stride < (int64_t)0x7fff0000 && (int64_t)a.max_seqlen_q * a.do_row_stride < (int64_t)0x7fff0000;
-  return near_rows ? launch_dkdv_kernel(attn_bwd_dkdv_partials_kernel<T, HD, KB, true>, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s)
-                   : launch_dkdv_kernel(attn_bwd_dkdv_partials_kernel<T, HD, KB, false>, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s);
+  auto kern = ws.visits != nullptr ? (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, true>)
+                                  : (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, false> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, false>);
+  return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s);
 }
 
 template <typename T, int HD, int RT, int NW>
@@ -1733,12 +1753,12 @@ static int launch_dq(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t 
     set_error("attn_bwd: too many (sequence, head, superblock) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * NW), smem, s, a, ws.ds, ws.tab, bwd_run_table(a), nsb_max);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * NW), smem, s, a, ws.ds, ws.tab, bwd_run_table(a), ws.row_mask, nsb_max);
   return 0;
 }
 
 // head dimensions above 128 (attn_bwd_wide.hip)
-int run_bwd_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, hipStream_t s);
+int run_bwd_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, int row_mask, hipStream_t s);
 
 // columns of a multiple of 128 keys: one workgroup (and one dQ partial per visit) per 128 keys
 static inline bool bwd_wide_blocks(const fmoba_attn_bwd_args &a) { return a.head_dim > 64 && a.lg_block_n % 128 == 0; }
@@ -1791,16 +1811,16 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
     const RunTable rt = bwd_run_table(a);
     const int ztab = partials ? 0 : (int)ceil_div64(ceil_div(rt.cols, 4), nx);
     if (a.batch + ztab <= 65535) {
-      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lpr, ws.tab, rt, ztab);
+      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lpr, ws.tab, rt, ws.row_mask, ztab);
     } else {  // (more planes than a launch has)
-      if (ztab > 0) hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(ceil_div(rt.cols, 4), a.heads, 1), dim3(256), 0, s, a, lpr, ws.tab, rt, 1);
-      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch), dim3(256), 0, s, a, lpr, ws.tab, rt, 0);
+      if (ztab > 0) hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(ceil_div(rt.cols, 4), a.heads, 1), dim3(256), 0, s, a, lpr, ws.tab, rt, ws.row_mask, 1);
+      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch), dim3(256), 0, s, a, lpr, ws.tab, rt, ws.row_mask, 0);
     }
   }
   if (a.head_dim > 128) {
     // the plain feature-split dK/dV kernel (attn_bwd_wide.hip), then the row-block dQ pass over its dS tiles
     if (phases & FMOBA_BWD_DKDV)
-      if (int rc = run_bwd_dkdv_wide(a, ws.ds, s)) return rc;
+      if (int rc = run_bwd_dkdv_wide(a, ws.ds, ws.row_mask, s)) return rc;
     if (phases & FMOBA_BWD_DQ)
       if (int rc = launch_dq<T, 256, 1, 8>(a, ws, s)) return rc;
     return 0;
@@ -1808,7 +1828,7 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
   if (phases & FMOBA_BWD_DKDV) {
     int rc;
     if (partials) {
-      hipLaunchKernelGGL(zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, (int64_t)a.total_q * a.heads);
+      if (ws.visits == nullptr) hipLaunchKernelGGL(zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, (int64_t)a.total_q * a.heads);
       rc = a.head_dim <= 64 ? launch_dkdv<T, 64, true>(a, ws, s) : (bwd_wide_blocks(a) ? launch_dkdv_partials<T, 128, 2>(a, ws, s) : launch_dkdv_partials<T, 128, 1>(a, ws, s));
     } else {
       rc = a.head_dim <= 64 ? launch_dkdv<T, 64, false>(a, ws, s) : a.head_dim <= 96 ? launch_dkdv<T, 96, false>(a, ws, s) : launch_dkdv<T, 128, false>(a, ws, s);
@@ -1819,8 +1839,8 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
     if (partials) {
       const int64_t rows = (int64_t)a.total_q * a.heads;
       const int capl = combine_order_entries(ws.cap);
-      const size_t smem = (size_t)16 * capl * 4;
-      auto kern = attn_bwd_dq_combine_kernel<T>;
+      const size_t smem = ws.visits != nullptr ? 0 : (size_t)16 * capl * 4;
+      auto kern = ws.visits != nullptr ? attn_bwd_dq_combine_kernel<T, true> : attn_bwd_dq_combine_kernel<T, false>;
       if (smem > 32 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
         set_error("attn_bwd: a row with up to %d visits needs %zu bytes of LDS for the order of its partial results", ws.cap, smem);
         return 2;
@@ -1866,6 +1886,10 @@ extern "C" int fmoba_attn_bwd(const fmoba_attn_bwd_args *a, void *stream) { retu
 extern "C" int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phases, void *stream) { return fmoba_attn_bwd_grouped(a, a ? a->heads : 0, phases, stream); }
 
 extern "C" int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_heads, int32_t phases, void *stream) {
+  return fmoba_attn_bwd_ranked(a, nullptr, dkv_heads, phases, stream);
+}
+
+extern "C" int fmoba_attn_bwd_ranked(const fmoba_attn_bwd_args *a, const uint32_t *visits, int32_t dkv_heads, int32_t phases, void *stream) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "attn_bwd: null args");
   FMOBA_REQUIRE(phases > 0 && phases <= 7, "attn_bwd: phases must be a mask of bits 1, 2, 4");
@@ -1926,6 +1950,8 @@ extern "C" int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_
   BwdWs ws;
   ws.dkv_heads = dkv_heads;
   ws.cap = bwd_partial_cap(*a);
+  ws.visits = visits;
+  ws.row_mask = visits != nullptr ? kListRowMask : -1;
   // (the dK/dV pass keeps the place of a visit's dQ partial as a 32-bit index of partial rows)
   FMOBA_REQUIRE(!fmoba::bwd_dq_partials(*a) || rows * (size_t)ws.cap + 1 < ((size_t)1 << 31),
                 "attn_bwd: %zu rows x heads with up to %d dQ partials each are more partial rows than the partials form addresses", rows, ws.cap);

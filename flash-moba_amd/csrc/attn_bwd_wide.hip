@@ -31,7 +31,7 @@ struct BwdWideSmem {
 };
 
 template <typename T>
-__global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws) {
+__global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws, int row_mask) {
   typedef BwdWideSmem SM;
   constexpr int HD = SM::HD, KS = HD / 16, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR;
   constexpr float kLog2e = 1.4426950408889634f;
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
     }
   }
   int start = 0;
-  if (causal && nnz > 0 && Bn > 64) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off);  // earlier rows see no key of the block
+  if (causal && nnz > 0 && Bn > 64) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off, row_mask);  // earlier rows see no key of the block
   const int32_t *list = a.row_indices + lbase + start;
   const int n = nnz - start;
   const int nround = (n + 63) >> 6;
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
   }
   __syncthreads();
   if (nround > 0) {
-    auto code = [&](int raw, int r) { return tile_row_code(raw, r * 64 + myrow < n, Lq); };
+    auto code = [&](int raw, int r) { return tile_row_code(raw & row_mask, r * 64 + myrow < n, Lq); };
     auto feed = [&](int rid, uint32_t buf) {  // eight rows per wave, of its own 32
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
 }
 
 template <typename T>
-static int launch_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, hipStream_t s) {
+static int launch_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, int row_mask, hipStream_t s) {
   auto kern = attn_bwd_dkdv_wide_kernel<T>;
   const size_t smem = BwdWideSmem::bytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
@@ -274,13 +274,13 @@ static int launch_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, hipSt
     set_error("attn_bwd: too many (sequence, head, key block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(512), smem, s, a, ds_ws);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(512), smem, s, a, ds_ws, row_mask);
   return 0;
 }
 
 // dK / dV and the dS tiles for head dimensions above 128 (ds_ws: the dS workspace, laid out by ds_piece_offset)
-int run_bwd_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, hipStream_t s) {
-  return a.dtype == FMOBA_DTYPE_BF16 ? launch_dkdv_wide<bf16_t>(a, ds_ws, s) : launch_dkdv_wide<f16_t>(a, ds_ws, s);
+int run_bwd_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, int row_mask, hipStream_t s) {
+  return a.dtype == FMOBA_DTYPE_BF16 ? launch_dkdv_wide<bf16_t>(a, ds_ws, row_mask, s) : launch_dkdv_wide<f16_t>(a, ds_ws, row_mask, s);
 }
 
 }  // namespace fmoba

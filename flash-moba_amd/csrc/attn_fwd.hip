@@ -39,9 +39,10 @@ constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 
 struct FwdWs {
   int32_t *cnt;      // [total_q * heads] visits handed out per (row, head)
-  float4 *hdr;       // [total_q * heads * cap] {m (log2 domain), l, key block id, -}
+  float4 *hdr;       // [total_q * heads * cap] {m (log2 domain), l, key block id, -}; ranked: float2 {m, l}
   void *part;        // [total_q * heads * cap][head_dim] partial outputs (fwd_part_size bytes per element)
   int32_t cap;
+  const uint32_t *visits;  // per (head, row), with ranked lists: the form whose slots are in key-block order (null: the other one)
 };
 
 // Bytes per element of a partial row: the 16-bit type of the call, fp32 at head dimensions above 128.  There this form serves
@@ -78,12 +79,17 @@ struct FwdColSmem {
 // workgroup of eight waves finds room for (2 x 4096 tokens, 8 heads of 256, top-k 8 of 128-key chunks, forward: 16-bit rows
 // per 64 keys 273 us, fp32 rows per 64 keys 450, per 128 keys 269).  Chunks that 128 does not divide pay for the wider rows:
 // top-k 16 of 64-key chunks 259 -> 439 us.
-template <typename T, int HD, int KB, bool FULL>  // FULL: the head dimension is HD
+// FULL: the head dimension is HD.  RANKED: a visit's slot is the place of its key block among the row's, made of the list entry's rank;
+// otherwise the row hands out slots from a counter.  The counters (a returning atomic on a line of its own per visit) and the ids
+// that the combine then needs to find the order are a tenth of the kernel (32 heads, top-k 16 of 128-key chunks, 32768 tokens: 1950 -> 1766 us,
+// 16 heads, 262144 tokens: 8.55 -> 7.43 ms), and the launch that clears them 5.5 us.
+template <typename T, int HD, int KB, bool FULL, bool RANKED>
 __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp) {
   typedef FwdColSmem<HD, KB> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, KT = KB / 32, RB = HD * 2, NW = SM::NW;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * (a.heads / grp), (a.max_seqlen_k + KB - 1) / KB, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
+  const bool one_pair = (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes;
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * (a.heads / grp), (a.max_seqlen_k + KB - 1) / KB, one_pair,
                                       longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 2));
   const int ngrp = a.heads / grp, nb = item.idx, b = item.pair / ngrp, h0 = (item.pair - b * ngrp) * grp, hk = h0 / (a.heads / a.heads_k);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
@@ -125,6 +131,7 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
   int g = 0, rem = 0, ridn = 0;
   Pack8 qb[KS];
   int slot = 0;
+  const int sub = a.lg_block_n / KB, jb = (key0 - c * a.lg_block_n) / KB;  // key blocks of a column, this one's number
   // (no branch around the loads: where two paths join, the compiler copies what was loaded, and waits for it there)
   auto pick = [&](auto async, int t) {
     t = min(t, ntile - 1);
@@ -132,9 +139,9 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
     const int first = t - (g ? __builtin_amdgcn_readlane(incl, g - 1) : 0);
     const int n = __builtin_amdgcn_readlane(nnz, g);
     const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)lbase, g), bhi = __builtin_amdgcn_readlane((uint32_t)(lbase >> 32), g);
-    const int32_t *list = a.row_indices + (int64_t)(((uint64_t)bhi << 32) | blo) + first * 32;
+    const int64_t at = (int64_t)(((uint64_t)bhi << 32) | blo) + first * 32;
     rem = n - first * 32;
-    const int32_t *p = list + min(lane & 31, rem - 1);
+    const int32_t *p = a.row_indices + at + min(lane & 31, rem - 1);
     if constexpr (decltype(async)::value)
       ridn = load_async(p);
     else
@@ -142,7 +149,7 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
   };
   int rid = -1, hcur = 0;
   auto fetch = [&](int t) {  // Q rows and partial slots of the picked tile
-    rid = tile_row_code(ridn, (lane & 31) < rem, Lq);
+    rid = tile_row_code(RANKED ? ridn & kListRowMask : ridn, (lane & 31) < rem, Lq);
     hcur = h0 + g;
     // Four lanes fetch 64 bytes of a row together: load 2 j brings pieces 4 j .. 4 j + 3 of the tile's first sixteen rows, load 2 j + 1 those
     // of the other sixteen, and an exchange of 16-lane rows then gives every lane pieces of its own row.  (A lane that fetched its own
@@ -157,7 +164,10 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
       qb[2 * j] = ld_global16(qa + e);
       qb[2 * j + 1] = ld_global16(qo + e);
     }
-    slot = take_slot(ws.cnt + ((int64_t)(q0 + (rid & 0x7fffffff)) * a.heads + hcur), __ballot(rid >= 0 && hh == 0 && t < ntile));
+    if constexpr (RANKED)
+      slot = (ridn >> kListRowBits) * sub + jb;
+    else
+      slot = take_slot(ws.cnt + ((int64_t)(q0 + (rid & 0x7fffffff)) * a.heads + hcur), __ballot(rid >= 0 && hh == 0 && t < ntile));
   };
   auto arrived = [&]() {
     wait_all_loads();
@@ -209,7 +219,7 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
   __syncthreads();
   for (int t = wave; t < ntile; t += NW) {
     const int r = rid, h = hcur;
-    const int s0 = __shfl(slot, lane & 31, 64);
+    const int s0 = RANKED ? slot : __shfl(slot, lane & 31, 64);
     const int pidx = (r >= 0 && s0 < ws.cap) ? ((q0 + r) * a.heads + h) * ws.cap + s0 : -1;
     // keys beyond lim are masked
     const int lim = r < 0 ? -1 : min(causal ? r + off : 0x7fffffff, Lk - 1) - key0;
@@ -316,7 +326,17 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
     // once the next tile's loads are in, what is held of this one leaves
     auto flush_held = [&]() {
       arrived();
-      if (pidx >= 0 && hh == 0) st_stream16(ws.hdr + pidx, Pack8{{__float_as_uint(m), __float_as_uint(l), (uint32_t)nb, 0u}});
+      if (pidx >= 0 && hh == 0) {
+        // The headers of a row share a line.  Where a pair's blocks run on one XCD its L2 collects them (32768 tokens 1975 -> 1789 us, 8192
+        // tokens 106 -> 103); where all XCDs work on one pair they go past the caches (262144 tokens 8.04 -> 7.51 ms).
+        if constexpr (RANKED) {
+          if (one_pair)
+            st_stream8(reinterpret_cast<float2 *>(ws.hdr) + pidx, __float_as_uint(m), __float_as_uint(l));
+          else
+            reinterpret_cast<float2 *>(ws.hdr)[pidx] = make_float2(m, l);
+        } else
+          st_stream16(ws.hdr + pidx, Pack8{{__float_as_uint(m), __float_as_uint(l), (uint32_t)nb, 0u}});
+      }
       // (the header past the caches, as the rows: written the ordinary way it cost 6 to 8 % of the kernel)
 #pragma unroll
       for (int part = 0; part < (int)(sizeof(x) / sizeof(x[0])); ++part) flush(x[part], part);
@@ -381,7 +401,8 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
 // headers, order, rows) is mostly waiting, so a wave runs four of them side by side.  Lane li of a group owns the
 // 16-byte pieces li, li + 16, .. (NP of them) of the row, whose elements are of type E
 // (NORM: divided by the visit's sum of probabilities).
-template <typename T, typename E, int NP, bool NORM>
+// RANKED: the slots are in key-block order and none of the first `visits` is empty.
+template <typename T, typename E, int NP, bool NORM, bool RANKED>
 __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_args a, FwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
   __shared__ float sWgt[16][16], sWl[16][16];
@@ -395,7 +416,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   const int64_t row = rh / a.heads;
   const int h = (int)(rh - row * a.heads);
   const int D = a.head_dim;
-  const int nall = valid ? ws.cnt[rh] : 0;
+  const int nall = !valid ? 0 : RANKED ? (int)(ws.visits[(int64_t)h * a.total_q + row] & 0xffffu) : ws.cnt[rh];
   const int n = min(nall, ws.cap);
   if (nall > ws.cap && li == 0 && a.visits_overflow != nullptr) atomicMax(a.visits_overflow, nall);  // visits were dropped
   int nmax = max(n, __shfl_xor(n, 16, 64));
@@ -408,20 +429,23 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   for (int i = 0; i < PE * NP; ++i) acc[i] = 0.f;
   float L = 0.f, M = -INFINITY;
   const float4 *hdr = ws.hdr + rh * ws.cap;
+  const float2 *hdr2 = reinterpret_cast<const float2 *>(ws.hdr) + rh * ws.cap;
   const E *part = reinterpret_cast<const E *>(ws.part) + rh * ws.cap * D;
   // The slot a visit got is arbitrary (a counter handed it out), the sum must not depend on it: every partial gets
   // its rank in ascending key-block order over the WHOLE row (equal ids, a malformed pattern, are ordered by slot),
   // and the partials are merged in rank order, 16 at a time.
-  group_rank_order(reinterpret_cast<const int *>(hdr) + 2, 4, n, nmax, sOrd, lane);
+  if constexpr (!RANKED) group_rank_order(reinterpret_cast<const int *>(hdr) + 2, 4, n, nmax, sOrd, lane);
   for (int base = 0; base < nmax; base += 16) {
     const int cntb = min(16, max(n - base, 0));
     float mj = -INFINITY, lj = 0.f;
-    int slot = 0;
     if (li < cntb) {
-      slot = sOrd[base + li];
-      const float4 x = hdr[slot];
-      mj = x.x;
-      lj = x.y;
+      if constexpr (RANKED) {
+        const float2 x = hdr2[base + li];
+        mj = x.x, lj = x.y;
+      } else {
+        const float4 x = hdr[sOrd[base + li]];
+        mj = x.x, lj = x.y;
+      }
     }
     float mb = mj;
 #pragma unroll
@@ -467,7 +491,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
         float w[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          load(x[u], sOrd[base + t + u]);
+          load(x[u], RANKED ? base + t + u : sOrd[base + t + u]);
           w[u] = sWgt[sg][t + u];
         }
 #pragma unroll
@@ -475,7 +499,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
       }
       for (; t < cntb; ++t) {
         Pack8 x[NP];
-        load(x, sOrd[base + t]);
+        load(x, RANKED ? base + t : sOrd[base + t]);
         add(x, sWgt[sg][t]);
       }
     }
@@ -590,7 +614,9 @@ static int fwd_col_heads(const fmoba_attn_fwd_args &a, int kb) {
 }
 template <typename T, int HD, int KB>
 static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStream_t s) {
-  auto kern = a.head_dim == HD ? attn_fwd_col_kernel<T, HD, KB, true> : attn_fwd_col_kernel<T, HD, KB, false>;
+  const bool ranked = ws.visits != nullptr;
+  auto kern = a.head_dim == HD ? (ranked ? attn_fwd_col_kernel<T, HD, KB, true, true> : attn_fwd_col_kernel<T, HD, KB, true, false>)
+                               : (ranked ? attn_fwd_col_kernel<T, HD, KB, false, true> : attn_fwd_col_kernel<T, HD, KB, false, false>);
   const size_t smem = FwdColSmem<HD, KB>::bytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
@@ -609,7 +635,7 @@ template <typename T>
 static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hipStream_t s) {
   const int64_t rows = (int64_t)a.total_q * a.heads;
   if (phases & FMOBA_FWD_COLUMNS) {
-    hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, rows);
+    if (ws.visits == nullptr) hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, rows);
     const int kb = fwd_key_block(a.lg_block_n);
     int rc;
     if (a.head_dim > 128)
@@ -622,8 +648,11 @@ static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hi
   }
   if (phases & FMOBA_FWD_COMBINE) {
     const int capl = combine_order_entries(ws.cap);
-    const size_t smem = (size_t)16 * capl * 4;
-    auto kern = a.head_dim > 128 ? attn_fwd_combine_kernel<T, float, 4, false> : attn_fwd_combine_kernel<T, uint16_t, 1, kFwdNormalisedParts<T, 128>>;
+    const bool ranked = ws.visits != nullptr;
+    const size_t smem = ranked ? 0 : (size_t)16 * capl * 4;
+    constexpr bool NORM = kFwdNormalisedParts<T, 128>;
+    auto kern = a.head_dim > 128 ? (ranked ? attn_fwd_combine_kernel<T, float, 4, false, true> : attn_fwd_combine_kernel<T, float, 4, false, false>)
+                                 : (ranked ? attn_fwd_combine_kernel<T, uint16_t, 1, NORM, true> : attn_fwd_combine_kernel<T, uint16_t, 1, NORM, false>);
     if (smem > 32 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
       set_error("attn_fwd: a row with up to %d visits needs %zu bytes of LDS for the order of its partial results", ws.cap, smem);
       return 2;
@@ -693,7 +722,9 @@ extern "C" int fmoba_csc_max_row_visits(const fmoba_attn_fwd_args *a, int32_t *c
 
 extern "C" int fmoba_attn_fwd(const fmoba_attn_fwd_args *a, void *stream) { return fmoba_attn_fwd_phases(a, 3, stream); }
 
-extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phases, void *stream) {
+extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phases, void *stream) { return fmoba_attn_fwd_ranked(a, nullptr, phases, stream); }
+
+extern "C" int fmoba_attn_fwd_ranked(const fmoba_attn_fwd_args *a, const uint32_t *visits, int32_t phases, void *stream) {
   using namespace fmoba;
   if (int rc = fwd_check_common(a)) return rc;
   FMOBA_REQUIRE(phases > 0 && phases <= 3, "attn_fwd: phases must be a mask of bits 1, 2");
@@ -724,6 +755,7 @@ extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phase
   const size_t need = fmoba_attn_fwd_workspace_bytes(a);
   FMOBA_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= need, "attn_fwd: workspace too small (%zu < %zu)", a->workspace_bytes, need);
   if (fwd_use_rows(*a)) {
+    FMOBA_REQUIRE(visits == nullptr || a->selection_bits != nullptr, "attn_fwd: the row-block form reads plain lists or selection bits");
     if (int rc = run_fwd_rows(*a, phases, s)) return rc;
     FMOBA_LAUNCH_CHECK("attn_fwd");
     return 0;
@@ -740,6 +772,7 @@ extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phase
   ws.hdr = reinterpret_cast<float4 *>(p);
   p += fwd_align256(rows * ws.cap * 16);
   ws.part = reinterpret_cast<void *>(p);
+  ws.visits = visits;
   int rc = a->dtype == FMOBA_DTYPE_BF16 ? run_fwd<bf16_t>(*a, ws, phases, s) : run_fwd<f16_t>(*a, ws, phases, s);
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("attn_fwd");

@@ -469,28 +469,18 @@ __device__ __forceinline__ float order_key_float(uint32_t k) {
   return __uint_as_float(u);
 }
 
-// first position of an ascending list whose entry is not below v
-__device__ __forceinline__ int lower_bound_i32(const int32_t *p, int n, int v) {
-  int lo = 0, hi = n;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (p[mid] < v)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
+// Entries of a ranked list: row | rank << kListRowBits.  `mask` below: kListRowMask for these, -1 for plain lists
+constexpr int kListRowBits = 24, kListRowMask = (1 << kListRowBits) - 1;
 
-// The same search by a whole wave (every lane passes the same arguments and gets the same result): 64 probes per
+// First position of an ascending list whose row is not below v, by a whole wave (every lane passes the same arguments and gets the same result): 64 probes per
 // step, so a list of a few thousand entries takes two or three dependent loads instead of a dozen.
-__device__ __forceinline__ int lower_bound_wave_i32(const int32_t *p, int n, int v) {
+__device__ __forceinline__ int lower_bound_wave_i32(const int32_t *p, int n, int v, int mask) {
   const int lane = threadIdx.x & 63;
   int lo = 0, hi = n;
   while (lo < hi) {
     const int step = (hi - lo + 63) >> 6;
     const int q = lo + lane * step;
-    const bool below = q < hi && p[q] < v;
+    const bool below = q < hi && (p[q] & mask) < v;
     const int cnt = __popcll(__ballot(below));  // the probes are ascending: the first cnt of them are below v
     if (cnt == 0) break;
     const int q1 = lo + (cnt - 1) * step;       // last probe below v: the answer lies in (q1, q1 + step]
@@ -607,6 +597,12 @@ __device__ __forceinline__ void st_stream16(void *p, const Pack8 &v) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   u32x4 x = {v.w[0], v.w[1], v.w[2], v.w[3]};
   __builtin_nontemporal_store(x, reinterpret_cast<u32x4 *>(p));
+}
+// the same for 8 bytes
+__device__ __forceinline__ void st_stream8(void *p, uint32_t x, uint32_t y) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  u32x2 v = {x, y};
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x2 *>(p));
 }
 __device__ __forceinline__ Pack8 zero_pack8() {
   Pack8 r;

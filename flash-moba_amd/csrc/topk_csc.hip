@@ -24,6 +24,8 @@ struct TopkParams {
   uint32_t *sel;      // [heads][W][total_q] selection bits, word w covers chunks 32w..32w+31
   int32_t *segcnt;    // [batch][heads][nseg][max_cols], null if no lists are wanted
   int32_t W, nseg, max_cols, seg_rows;
+  fmoba_csc_ranks ranks;       // all null: not wanted
+  int32_t sub_fwd, sub_bwd;    // key blocks of the attention's forward and backward (partials) per chunk
 };
 
 // Rows per counting segment.  A wave of the fill kernel walks one segment of one 32-chunk word column, 64 rows at a
@@ -1546,12 +1548,50 @@ __global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
   }
 }
 
-// grid (heads, batch), block 256
+// grid (heads, batch, 1 + blocks of kRankRows rows if ranks are wanted), block 256
+constexpr int kRankRows = 1024;
 __global__ __launch_bounds__(256) void csc_scan_kernel(TopkParams p) {
   const fmoba_fused_topk_args &a = p.a;
   const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
   const int q0 = a.cu_seqlens_q[b];
   const int Lq = a.cu_seqlens_q[b + 1] - q0;
+  if (blockIdx.z > 0) {
+    // How many chunks a row selected below each word of its selection, and its visits: independent of the scan, whose few
+    // workgroups mostly wait (scan without and with them: 8192 tokens, 16 heads 6.0 and 6.8 us; 262144 tokens 122 and 250 us)
+    const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b], last = (Lk + a.chunk - 1) / a.chunk - 1;  // the sequence's last chunk
+    for (int k = 0; k < kRankRows; k += 256) {
+      const int r = (int)(blockIdx.z - 1) * kRankRows + k + tid;
+      if (r >= Lq) return;
+      const int rp = r + Lk - Lq, own = rp >= 0 ? rp / a.chunk : -1;
+      const int nw = a.is_causal ? (own < 0 ? 0 : min(p.W, (own >> 5) + 1)) : p.W;
+      const uint32_t *words = p.sel + (int64_t)h * p.W * a.total_q + q0 + r;
+      uint8_t *pre = p.ranks.prefix + (int64_t)h * p.W * a.total_q + q0 + r;
+      int n = 0, has_last = 0;
+      for (int w0 = 0; w0 < nw; w0 += 8) {
+        uint32_t x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = w0 + i < nw ? words[(int64_t)(w0 + i) * a.total_q] : 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if (w0 + i > 0 && w0 + i < nw) pre[(int64_t)(w0 + i) * a.total_q] = (uint8_t)n;
+          n += __popc(x[i]);
+          if (w0 + i == (last >> 5)) has_last = (x[i] >> (last & 31)) & 1;
+        }
+      }
+      // Forward: all key blocks of a selected chunk that exist.  Backward: under the causal rule those of the row's own chunk, its
+      // last one, that begin at or before the row.
+      auto blocks = [&](int sub, int keys) {
+        const int kb = a.chunk / sub;
+        return (keys + kb - 1) / kb;
+      };
+      const int nf = n * p.sub_fwd - has_last * (p.sub_fwd - blocks(p.sub_fwd, Lk - last * a.chunk));
+      const int nb = n == 0         ? 0
+                     : a.is_causal ? (n - 1) * p.sub_bwd + blocks(p.sub_bwd, rp - own * a.chunk + 1)
+                                   : n * p.sub_bwd - has_last * (p.sub_bwd - blocks(p.sub_bwd, Lk - last * a.chunk));
+      p.ranks.visits[(int64_t)h * a.total_q + q0 + r] = (uint32_t)nf | ((uint32_t)nb << 16);
+    }
+    return;
+  }
   const int nseg_b = (Lq + p.seg_rows - 1) / p.seg_rows;
   const int64_t bh = (int64_t)b * a.heads + h;
   int32_t *segc = p.segcnt + bh * p.nseg * p.max_cols;
@@ -1625,7 +1665,20 @@ __device__ __forceinline__ void store_i32_in_lanes(int32_t *base, uint32_t byte_
 #endif
 }
 
+// n + 1 in the lanes of `lanes`
+__device__ __forceinline__ uint32_t count_lanes(uint32_t n, unsigned long long lanes) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("v_addc_co_u32_e64 %0, vcc, 0, %0, %1" : "+v"(n) : "s"(lanes) : "vcc");
+#else
+  (void)lanes;
+#endif
+  return n;
+}
+
 // grid (nseg * W, heads, batch), block 64: one wave walks the rows of one segment of one 32-chunk word column
+// RANKED: with every row id its chunk's place among the chunks of the row, in the bits from kListRowBits on (in an array of their own,
+// a byte per entry, the ranks cost a second store per chunk and step: 262144 tokens 789 -> 1723 us, 874 this way)
+template <bool RANKED>
 __global__ __launch_bounds__(64) void csc_fill_kernel(TopkParams p) {
   const fmoba_fused_topk_args &a = p.a;
   // consecutive workgroups: consecutive segments of one word column, i.e. consecutive memory.  (With the word column
@@ -1661,9 +1714,11 @@ __global__ __launch_bounds__(64) void csc_fill_kernel(TopkParams p) {
       rel = (uint32_t)(a.col_offsets[bh * p.max_cols + c] - first) + (uint32_t)p.segcnt[(bh * p.nseg + seg) * p.max_cols + c];
   }
   const uint32_t *words = p.sel + ((int64_t)h * p.W + wc) * a.total_q + q0;
+  const uint8_t *pre = RANKED ? p.ranks.prefix + ((int64_t)h * p.W + wc) * a.total_q + q0 : nullptr;
   for (int rb = rb0; rb < r1; rb += 64) {
     const int r = rb + lane;
     const uint32_t w = (r < r1) ? words[r] : 0u;
+    uint32_t nth = RANKED && wc > 0 && r < r1 ? pre[r] : 0u;  // chunks that the row selected so far
     // the chunks that some row of the step selects (a scalar, so that the others cost no vector instruction)
     const uint32_t present = __builtin_amdgcn_readfirstlane(__ockl_wfred_or_u32(w));
     if (present == 0u) continue;
@@ -1673,7 +1728,12 @@ __global__ __launch_bounds__(64) void csc_fill_kernel(TopkParams p) {
         const unsigned long long m = __ballot((w & (1u << j)) != 0u);
         const uint32_t at = __builtin_amdgcn_readlane(rel, j);
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        store_i32_in_lanes(lists, (at + rank) << 2, r, m);
+        if constexpr (RANKED) {
+          store_i32_in_lanes(lists, (at + rank) << 2, (int)((nth << kListRowBits) | (uint32_t)r), m);
+          nth = count_lanes(nth, m);
+        } else {
+          store_i32_in_lanes(lists, (at + rank) << 2, r, m);
+        }
         rel = write_lane<j>(rel, at + (uint32_t)__popcll(m));
       }
     });
@@ -1898,7 +1958,7 @@ int mean_pool_with_offsets(const fmoba_mean_pool_args *a, int32_t *clear, int64_
 // The call behind the entry points: everything of `a` except its workspace fields, which come as arguments.  `pool`: the
 // pooling pass that comes first and clears the segment counts; null: the chunk means are there already.
 static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_t workspace_bytes, const fmoba_mean_pool_args *pool, bool lists,
-                          void *stream) {
+                          const fmoba_csc_ranks *ranks, void *stream) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "fused_topk: null args");
   FMOBA_REQUIRE(a->dtype == FMOBA_DTYPE_F16 || a->dtype == FMOBA_DTYPE_BF16, "FlashMoBA only supports fp16 and bf16 data types");
@@ -1947,6 +2007,15 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   p.W = ceil_div(max_cols, 32);
   p.seg_rows = csc_seg_rows(a->batch, a->heads, a->max_seqlen_q, p.W);
   p.nseg = ceil_div(a->max_seqlen_q > 0 ? a->max_seqlen_q : 1, p.seg_rows);
+  p.ranks = ranks != nullptr ? *ranks : fmoba_csc_ranks{nullptr, nullptr};
+  p.sub_fwd = p.sub_bwd = 1;
+  if (ranks != nullptr) {
+    FMOBA_REQUIRE(ranks->visits && (ranks->prefix || p.W == 1), "pool_and_gate_ranked: null pointer");
+    FMOBA_REQUIRE(a->chunk % 64 == 0, "pool_and_gate_ranked: the attention takes chunks of a multiple of 64 keys");
+    p.sub_fwd = a->chunk % 128 == 0 ? a->chunk / 128 : a->chunk / 64;                       // (fmoba_attn_fwd_key_block)
+    p.sub_bwd = a->chunk % 128 == 0 && a->head_dim > 64 ? a->chunk / 128 : a->chunk / 64;
+    FMOBA_REQUIRE((int64_t)a->topk * p.sub_bwd < 65536, "pool_and_gate_ranked: more than 65535 visits per row");
+  }
   const size_t sel_bytes = align256((size_t)a->heads * p.W * a->total_q * 4);
   const size_t seg_bytes = align256((size_t)a->batch * a->heads * p.nseg * max_cols * 4);
   FMOBA_REQUIRE(workspace != nullptr && workspace_bytes >= sel_bytes + seg_bytes, "fused_topk: workspace too small (%zu < %zu)",
@@ -1983,9 +2052,9 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("topk_gate_kernel");
   if (!lists) return 0;
-  hipLaunchKernelGGL(csc_scan_kernel, dim3(a->heads, a->batch), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(csc_scan_kernel, dim3(a->heads, a->batch, 1 + (ranks ? ceil_div(a->max_seqlen_q, kRankRows) : 0)), dim3(256), 0, s, p);
   FMOBA_LAUNCH_CHECK("csc_scan_kernel");
-  hipLaunchKernelGGL(csc_fill_kernel, dim3(p.nseg * p.W, a->heads, a->batch), dim3(64), 0, s, p);
+  hipLaunchKernelGGL(ranks ? csc_fill_kernel<true> : csc_fill_kernel<false>, dim3(p.nseg * p.W, a->heads, a->batch), dim3(64), 0, s, p);
   FMOBA_LAUNCH_CHECK("csc_fill_kernel");
   if (a->raw_indices) {
     const size_t smem = (size_t)(max_cols + 64) * 4;
@@ -2001,10 +2070,10 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
 
 extern "C" int fmoba_fused_topk(const fmoba_fused_topk_args *a, void *stream) {
   FMOBA_REQUIRE(a != nullptr, "fused_topk: null args");
-  return fused_topk_run(a, a->workspace, a->workspace_bytes, nullptr, true, stream);
+  return fused_topk_run(a, a->workspace, a->workspace_bytes, nullptr, true, nullptr, stream);
 }
 
-extern "C" int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, int32_t want_lists, void *stream) {
+static int pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, bool want_lists, const fmoba_csc_ranks *r, void *stream) {
   FMOBA_REQUIRE(m != nullptr && g != nullptr, "pool_and_gate: null args");
   FMOBA_REQUIRE(m->km == g->km && m->cu_seqlens_km == g->cu_seqlens_km && m->cu_seqlens_k == g->cu_seqlens_k && m->batch == g->batch &&
                     m->heads_k == g->heads_k && m->head_dim == g->head_dim && m->chunk == g->chunk && m->dtype == g->dtype,
@@ -2012,7 +2081,16 @@ extern "C" int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fu
   FMOBA_REQUIRE(g->total_q > 0 && g->max_seqlen_q > 0 && g->max_seqlen_k > 0, "pool_and_gate: empty problem");
   FMOBA_REQUIRE(m->max_chunks == fmoba::ceil_div(g->max_seqlen_k, g->chunk), "pool_and_gate: max_chunks is ceil(max_seqlen_k / chunk)");
   FMOBA_REQUIRE(want_lists || g->raw_indices == nullptr, "pool_and_gate: the ordered lists come with the column lists only");
-  return fused_topk_run(g, g->workspace, g->workspace_bytes, m, want_lists != 0, stream);
+  return fused_topk_run(g, g->workspace, g->workspace_bytes, m, want_lists, r, stream);
+}
+
+extern "C" int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, int32_t want_lists, void *stream) {
+  return pool_and_gate(m, g, want_lists != 0, nullptr, stream);
+}
+
+extern "C" int fmoba_pool_and_gate_ranked(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, const fmoba_csc_ranks *r, void *stream) {
+  FMOBA_REQUIRE(r != nullptr, "pool_and_gate_ranked: null ranks");
+  return pool_and_gate(m, g, true, r, stream);
 }
 
 // ------------------------------------------------------------------------------------
@@ -2048,5 +2126,5 @@ extern "C" int fmoba_fused_topk_static(const fmoba_fused_topk_args *a, void *str
     }
     ptr = g_scratch_ptr[dev];
   }
-  return fused_topk_run(a, ptr, (size_t)FMOBA_STATIC_SCRATCH_BYTES, nullptr, true, stream);
+  return fused_topk_run(a, ptr, (size_t)FMOBA_STATIC_SCRATCH_BYTES, nullptr, true, nullptr, stream);
 }

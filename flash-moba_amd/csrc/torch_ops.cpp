@@ -104,11 +104,12 @@ size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
 struct Pattern {
   Tensor col_offsets, col_nnz, indices, scratch;
+  Tensor visits;                        // defined: the lists are ranked (gated patterns whose attention leaves partial results per visit)
   const uint32_t *selection = nullptr;  // in `scratch`
 };
 
-// chunk means, gating and (with `lists`) the column lists
-Pattern gate(const Shape &s, const Tensor &q, const Tensor &k, const Tensor &cu_q, const Tensor &cu_k, int64_t topk, bool lists) {
+// chunk means, gating and (with `lists`) the column lists, ranked if wanted
+Pattern gate(const Shape &s, const Tensor &q, const Tensor &k, const Tensor &cu_q, const Tensor &cu_k, int64_t topk, bool lists, bool ranked = false) {
   Pattern p;
   const auto i32 = q.options().dtype(at::kInt);
   if (lists) {
@@ -120,10 +121,12 @@ Pattern gate(const Shape &s, const Tensor &q, const Tensor &k, const Tensor &cu_
   const size_t gate_bytes = up256(fmoba_fused_topk_workspace_bytes(s.batch, s.total_q, s.heads, s.max_q, s.max_k, s.chunk));
   const size_t cu_bytes = up256((s.batch + 1) * 4);
   const size_t km_bytes = static_cast<size_t>(s.total_k / s.chunk + s.batch) * s.heads_k * s.dim * 2;
-  p.scratch = bytes_like(q, gate_bytes + cu_bytes + km_bytes + 256);
+  const size_t pre_bytes = ranked && s.max_cols > 32 ? up256(static_cast<size_t>(s.heads) * ((s.max_cols + 31) / 32) * s.total_q) : 0;
+  p.scratch = bytes_like(q, gate_bytes + cu_bytes + pre_bytes + km_bytes + 256);
+  if (ranked) p.visits = at::empty({s.heads, s.total_q}, i32);
   char *base = reinterpret_cast<char *>(up256(reinterpret_cast<size_t>(p.scratch.data_ptr())));
   fmoba_mean_pool_args m{};
-  m.k = k.data_ptr(), m.km = base + gate_bytes + cu_bytes;
+  m.k = k.data_ptr(), m.km = base + gate_bytes + cu_bytes + pre_bytes;
   m.cu_seqlens_k = cu_k.data_ptr<int32_t>(), m.cu_seqlens_km = reinterpret_cast<int32_t *>(base + gate_bytes);
   m.batch = s.batch, m.max_chunks = s.max_cols, m.heads_k = s.heads_k, m.head_dim = s.dim, m.chunk = s.chunk, m.dtype = s.dtype;
   m.k_row_stride = k.stride(0), m.k_head_stride = k.stride(1), m.km_row_stride = s.heads_k * s.dim, m.km_head_stride = s.dim;
@@ -134,7 +137,12 @@ Pattern gate(const Shape &s, const Tensor &q, const Tensor &k, const Tensor &cu_
   g.batch = s.batch, g.total_q = s.total_q, g.heads = s.heads, g.heads_k = s.heads_k, g.head_dim = s.dim;
   g.max_seqlen_q = s.max_q, g.max_seqlen_k = s.max_k, g.topk = topk, g.chunk = s.chunk, g.is_causal = s.causal, g.dtype = s.dtype;
   g.q_row_stride = q.stride(0), g.q_head_stride = q.stride(1), g.km_row_stride = m.km_row_stride, g.km_head_stride = m.km_head_stride;
-  check(fmoba_pool_and_gate(&m, &g, lists ? 1 : 0, s.stream));
+  if (ranked) {
+    const fmoba_csc_ranks r{reinterpret_cast<uint32_t *>(p.visits.data_ptr<int32_t>()), pre_bytes ? reinterpret_cast<uint8_t *>(base + gate_bytes + cu_bytes) : nullptr};
+    check(fmoba_pool_and_gate_ranked(&m, &g, &r, s.stream));
+  } else {
+    check(fmoba_pool_and_gate(&m, &g, lists ? 1 : 0, s.stream));
+  }
   p.selection = reinterpret_cast<const uint32_t *>(base);
   return p;
 }
@@ -156,6 +164,14 @@ fmoba_attn_fwd_args forward_args(const Shape &s, const Tensor &q, const Tensor &
 struct Result {
   Tensor out, lse;
 };
+const uint32_t *visit_ptr(const Tensor &t) { return t.defined() ? reinterpret_cast<const uint32_t *>(t.data_ptr<int32_t>()) : nullptr; }
+
+// what the form of dQ and its workspace depend on
+void backward_sizes(fmoba_attn_bwd_args &b, const Shape &s, int64_t visits64) {
+  b.batch = s.batch, b.total_q = s.total_q, b.total_k = s.total_k, b.heads = s.heads, b.heads_k = s.heads_k, b.head_dim = s.dim;
+  b.max_seqlen_q = s.max_q, b.max_seqlen_k = s.max_k, b.max_cols = s.max_cols, b.lg_block_n = s.chunk, b.is_causal = s.causal && s.max_q != 1;
+  b.max_visits_per_row = visits64;
+}
 // what this thread's last forward ran, and its last backward if nobody has asked since (else -1): diagnostics
 thread_local int t_visits = 0, t_row_blocks = 0, t_partials = -1;
 
@@ -171,7 +187,7 @@ Result forward(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const Pat
   const size_t n = fmoba_attn_fwd_workspace_bytes(&a);
   const Tensor ws = bytes_like(q, n);
   a.workspace = ws.data_ptr(), a.workspace_bytes = n;
-  check(fmoba_attn_fwd(&a, s.stream));
+  check(fmoba_attn_fwd_ranked(&a, visit_ptr(p.visits), 3, s.stream));
   return r;
 }
 
@@ -181,7 +197,7 @@ struct Attention : public torch::autograd::Function<Attention> {
   static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &cu_q, const Tensor &cu_k,
                         const Pattern &p, const Result &r, int64_t max_q, int64_t max_k, int64_t chunk, bool causal, double scale, int64_t bwd_visits,
                         bool deterministic) {
-    ctx->save_for_backward({q, k, v, r.out, r.lse, cu_q, cu_k, p.col_offsets, p.col_nnz, p.indices});
+    ctx->save_for_backward({q, k, v, r.out, r.lse, cu_q, cu_k, p.col_offsets, p.col_nnz, p.indices, p.visits});
     ctx->saved_data["max_q"] = max_q;
     ctx->saved_data["max_k"] = max_k;
     ctx->saved_data["chunk"] = chunk;
@@ -209,6 +225,8 @@ struct Attention : public torch::autograd::Function<Attention> {
     TORCH_CHECK(is(lse, at::kFloat) && lse.dim() == 2 && lse.size(0) == q.size(1) && lse.size(1) == q.size(0) && is(cu_q, at::kInt) && is(cu_k, at::kInt) &&
                     is(co, at::kLong) && is(cn, at::kInt) && is(ind, at::kInt) && co.dim() == 3 && co.sizes() == cn.sizes() && co.size(0) == nb && co.size(1) == q.size(1),
                 "flash_moba: the pattern, the offsets or the log-sum-exp was saved and came back as another tensor");
+    const Tensor &visits = t[10];
+    TORCH_CHECK(!visits.defined() || (is(visits, at::kInt) && visits.numel() == lse.numel()), "flash_moba: the visits of the pattern were saved and came back as another tensor");
     auto num = [&](const char *name) { return ctx->saved_data[name].toInt(); };
     variable_list res(14);  // one per argument of forward
     {
@@ -242,7 +260,7 @@ struct Attention : public torch::autograd::Function<Attention> {
       const size_t n = fmoba_attn_bwd_workspace_bytes(&a);
       const Tensor ws = bytes_like(q, n);
       a.workspace = ws.data_ptr(), a.workspace_bytes = n;
-      check(fmoba_attn_bwd_grouped(&a, dkv_heads, 7, s.stream));
+      check(fmoba_attn_bwd_ranked(&a, visit_ptr(visits), dkv_heads, 7, s.stream));
       t_partials = fmoba_attn_bwd_uses_partials(&a);
       if (grouped) {
         at::sum_out(dk, dk_e.view({s.total_k, s.heads_k, dkv_heads / s.heads_k, s.dim}), at::IntArrayRef{2});
@@ -286,8 +304,13 @@ py::object moba_varlen(const py::handle &hq, const py::handle &hk, const py::han
       check_device(q.device().index());
       s.stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
       fmoba_attn_fwd_args a = forward_args(s, q, k, v, cu_q, cu_k, visits, scale, nullptr);
-      const bool lists = grad || !fmoba_attn_fwd_uses_row_blocks(&a);  // (the row-block form reads the selection bits alone)
-      p = gate(s, q, k, cu_q, cu_k, topk, lists);
+      const bool columns = !fmoba_attn_fwd_uses_row_blocks(&a), lists = grad || columns;  // (the row-block form reads the selection bits alone)
+      // Ranks for the forms that leave a partial result per visit.  (One query row per sequence: the attention then drops the
+      // causal rule that the gating keeps, and the visits of a row are others.  65536 visits: more than a row's count holds.)
+      fmoba_attn_bwd_args b{};
+      backward_sizes(b, s, visits * (kb / 64));
+      const bool ranked = max_q > 1 && visits * (kb / 64) < 65536 && (columns || (grad && fmoba_attn_bwd_uses_partials(&b)));
+      p = gate(s, q, k, cu_q, cu_k, topk, lists, ranked);
       a.selection_bits = p.selection;
       r = forward(s, a, q, p);
     }
@@ -363,9 +386,8 @@ py::object attn_varlen(const py::handle &hq, const py::handle &hk, const py::han
   bool count = !fmoba_attn_fwd_uses_row_blocks(&a);
   if (grad) {
     fmoba_attn_bwd_args b{};
-    b.batch = s.batch, b.total_q = s.total_q, b.total_k = s.total_k, b.heads = s.heads, b.heads_k = s.heads_k, b.head_dim = s.dim;
-    b.max_seqlen_q = s.max_q, b.max_seqlen_k = s.max_k, b.max_cols = s.max_cols, b.lg_block_n = lg_n, b.is_causal = a.is_causal;
-    b.max_visits_per_row = visits * (kb / 64), b.num_row_indices = p.indices.numel();
+    backward_sizes(b, s, visits * (kb / 64));
+    b.num_row_indices = p.indices.numel();
     count = count || fmoba_attn_bwd_uses_partials(&b) || (!capturing && fmoba_attn_bwd_workspace_bytes(&b) > kUncountedBytes);
   }
   // (nothing can be read back while a graph is captured)

@@ -83,6 +83,10 @@ class AttnBwdArgs(ctypes.Structure):
                 ("dv_row_stride", c_i64), ("dv_head_stride", c_i64), ("visits_overflow", c_vp)]
 
 
+class CscRanks(ctypes.Structure):
+    _fields_ = [("visits", c_vp), ("prefix", c_vp)]
+
+
 EXPORTS = {
     "fmoba_version": (c_i32, []),
     "fmoba_last_error": (ctypes.c_char_p, []),
@@ -101,6 +105,9 @@ EXPORTS = {
     "fmoba_csc_max_row_visits": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp, c_vp, c_vp]),
     "fmoba_attn_fwd": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp]),
     "fmoba_attn_fwd_phases": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_i32, c_vp]),
+    "fmoba_attn_fwd_ranked": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp, c_i32, c_vp]),
+    "fmoba_attn_bwd_ranked": (c_i32, [ctypes.POINTER(AttnBwdArgs), c_vp, c_i32, c_i32, c_vp]),
+    "fmoba_pool_and_gate_ranked": (c_i32, [ctypes.POINTER(MeanPoolArgs), ctypes.POINTER(FusedTopkArgs), ctypes.POINTER(CscRanks), c_vp]),
     "fmoba_attn_bwd_grouped": (c_i32, [ctypes.POINTER(AttnBwdArgs), c_i32, c_i32, c_vp]),
     "fmoba_attn_bwd_dkv_heads": (c_i32, [ctypes.POINTER(AttnBwdArgs)]),
     "fmoba_attn_bwd_workspace_bytes": (c_sz, [ctypes.POINTER(AttnBwdArgs)]),

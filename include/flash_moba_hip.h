@@ -101,6 +101,17 @@ int fmoba_fused_topk(const fmoba_fused_topk_args *a, void *stream);
  * for callers whose attention form reads nothing else.  g->km and g->cu_seqlens_km must be m->km and m->cu_seqlens_km;
  * max_seqlen_k of g must be positive. */
 int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, int32_t want_lists, void *stream);
+/* The lists with the place of every entry among the chunks of its row: an entry is row | rank << 24, rank = number of chunks with a
+ * lower index that the row selected (top-k is at most 64, max_seqlen_q below 2^24).  visits[h * total_q + t] = visits of row t of
+ * head h in key blocks of the attention, forward in the low 16 bits, backward (partials form) in the high 16 bits; prefix: scratch of
+ * heads * ceil(max_seqlen_k / chunk / 32) * total_q bytes (may be NULL if that is one word per row).  With them the attention passes
+ * put a visit's partial result where it belongs, instead of handing out places from a counter per row and sorting them when they are
+ * added up.  Such lists are for the _ranked entry points alone.  No counterpart in the reference. */
+typedef struct {
+  uint32_t *visits;
+  uint8_t *prefix;
+} fmoba_csc_ranks;
+int fmoba_pool_and_gate_ranked(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, const fmoba_csc_ranks *r, void *stream);
 /* The same call without a workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
  * reference, whose host code allocates on every call.  `workspace` / `workspace_bytes` of `a` are
@@ -195,6 +206,9 @@ int fmoba_attn_fwd(const fmoba_attn_fwd_args *a, void *stream);
 #define FMOBA_FWD_COLUMNS 1
 #define FMOBA_FWD_COMBINE 2
 int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phases, void *stream);
+/* The same over the lists and visits of fmoba_pool_and_gate_ranked (is_causal has to be the gating's): the column form then
+ * needs no counters and sorts nothing.  The result is the same to the last bit.  visits = NULL: plain lists. */
+int fmoba_attn_fwd_ranked(const fmoba_attn_fwd_args *a, const uint32_t *visits, int32_t phases, void *stream);
 
 /* ------------------------------------------------------------------------------------
  * Sparse attention backward.
@@ -265,6 +279,8 @@ int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phases, void *st
  * caller sums what is left of a group. */
 int32_t fmoba_attn_bwd_dkv_heads(const fmoba_attn_bwd_args *a);
 int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_heads, int32_t phases, void *stream);
+/* The same over the lists and visits of fmoba_pool_and_gate_ranked, as fmoba_attn_fwd_ranked. */
+int fmoba_attn_bwd_ranked(const fmoba_attn_bwd_args *a, const uint32_t *visits, int32_t dkv_heads, int32_t phases, void *stream);
 
 #ifdef __cplusplus
 }
