@@ -66,8 +66,8 @@ __device__ __forceinline__ int count4_gt(int n, float x0, float x1, float x2, fl
 #endif
 }
 
-// n + (x >= y) in two halves: four compares into four scalar register pairs first, then an add with carry per flag
-// where the count is needed (a vector instruction that reads a scalar register written by the one before it has to
+// x >= y in two halves: four compares into four scalar register pairs first, then an add with carry per flag
+// where it is needed (a vector instruction that reads a scalar register written by the one before it has to
 // wait two slots: with the compares of four scores ahead of their adds nothing waits; left alone, the compiler
 // materialises every flag as 0 / 1 first).  Volatile, so that the compares stay ahead of the adds.
 struct Flags4 {
@@ -90,15 +90,6 @@ __device__ __forceinline__ Flags4 flags4_ge(float x0, float x1, float x2, float 
 #endif
   return f;
 }
-__device__ __forceinline__ int count_flag(int n, unsigned long long flag) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_addc_co_u32_e64 %0, vcc, 0, %0, %1" : "+v"(n) : "s"(flag) : "vcc");
-  return n;
-#else
-  return n + (int)(flag & 1);
-#endif
-}
-
 // the same with x > y
 __device__ __forceinline__ Flags4 flags4_gt(float x0, float x1, float x2, float x3, float y) {
   Flags4 f;
@@ -871,29 +862,37 @@ __global__ __launch_bounds__(256, CAP < kBigCap ? 2 : 1) void topk_gate_big_kern
 // ------------------------------------------------------------------------------------
 // The grouped gate for at most 16 running winners per row (top-k up to 17 causal, 16 otherwise): the common case of
 // long sequences.  Same total order and result as topk_gate_big_kernel; what differs is where things live:
-//  * a row's winners stay in REGISTERS across the groups: eight doubles per lane of the row's lane pair, each lane's
-//    share sorted, so that the weakest is at hand and a new winner goes in with one pass of minimum / maximum;
-//  * the chunk means of the next group are fetched into registers while the current group is worked on;
-//  * the scores of a later group that reach the row's weakest winner ("entrants") are compacted into one list per
-//    row in LDS -- the lane with chunks 0..3 of every eight fills it from the bottom, its partner from the top, so
-//    that no counter is shared; every score is stored at the lane's next slot and the slot advances only for an
-//    entrant, so there are no branches and no address selects -- and each then replaces the weakest winner if it
-//    beats it.  More than 16 entrants in some row of a wave, the first group, and rows whose list is not full yet
-//    take the bisection over this group's scores and the winners.
+//  * a row's winners stay in REGISTERS across the groups, sorted: the eight weakest of its sixteen places in the lane with
+//    chunks 0..3 of every eight, the eight strongest in its partner.  A new winner is offered to the strong half, which
+//    passes on what it gives up, and goes in with one pass of minimum / maximum: no compare, no choice between the lanes
+//    (shares sorted per lane needed both: which lane holds the weakest was two exchanges and six selects per winner);
+//  * the chunk means of the next group are fetched into the LDS tile while the current group is worked on;
+//  * the scores of a group lie in LDS, a row of 64 floats, and a mask of 64 bits per row says which of them reach the row's
+//    weakest winner ("entrants", two instructions per score): the row takes them from the lowest bit up.  (A list of entrants
+//    with their chunks, built score by score, cost five instructions and two LDS stores per score.)
+//  * the first group has no winners yet: a few probes find a score that at least K' and, as a rule, no more than K' + kGateSlack
+//    of the group reach, and those are its entrants.  The order does the rest, ties and all.
+// 262144 tokens, 16 heads, top-k 16 of 128-key chunks 3859 -> 2921 us; 1024-row parts of prompts with 9000 to 33000 keys, 32
+// heads, top-k 8 51 -> 29 us (before: winners shared out by lane, lists of entrants, the whole cut of the first group searched).  Bound by
+// the vector instructions, most of them the pass of a new winner.
 // ------------------------------------------------------------------------------------
-// A winner is ONE double: order key of its score * 65536 + chunk (exact: below 2^48), so that the order "score
+// A winner is ONE double between 1 and 2: order key of its score and chunk are 48 bits of its fraction, so that the order "score
 // descending, chunk descending" is the order of the doubles and minimum / maximum are single instructions.
-constexpr double kChunkSpan = 65536.0;  // chunk indices stay below it (checked on the host before the launch)
-constexpr double kSlotFiller = INFINITY;  // unused slot of a complete list: above every winner, never the weakest
-constexpr double kSlotEmpty = -1.0;       // unused slot of a list that is still filling: below every winner
+constexpr double kSlotFiller = INFINITY;  // place beyond the K'-th: above every winner
+constexpr double kSlotEmpty = 0.5;        // place of a winner still to come: below every winner
+constexpr uint32_t kNoEntrant = 0x3fd00000u;  // upper word of a double below kSlotEmpty
 
-__device__ __forceinline__ double winner_word(float score, int chunk) {
-  // (x + 0 turns -0 into +0: the order keys must agree with the float compares of the bisection)
-  return fma((double)float_order_key(score + 0.f), kChunkSpan, (double)chunk);
+__device__ __forceinline__ double double_of(uint32_t hi, uint32_t lo) { return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo)); }
+// the winner of a score and its chunk, or a double below all places
+__device__ __forceinline__ double winner_word(float score, int chunk, bool has) {
+  // (x + 0 turns -0 into +0: the order keys must agree with the float compares of the search)
+  const uint32_t u = __float_as_uint(score + 0.f);
+  const uint32_t key = u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);  // (float_order_key, an instruction less)
+  return double_of(has ? 0x3ff00000u | (key >> 16) : kNoEntrant, (key << 16) | (uint32_t)chunk);
 }
-__device__ __forceinline__ bool winner_real(double w) { return w >= 0.0 && w < (double)INFINITY; }
-__device__ __forceinline__ uint32_t winner_key(double w) { return (uint32_t)(w * (1.0 / kChunkSpan)); }  // (truncates)
-__device__ __forceinline__ int winner_chunk(double w) { return (int)fma(-(double)winner_key(w), kChunkSpan, w); }
+__device__ __forceinline__ bool winner_real(double w) { return w >= 1.0 && w < (double)INFINITY; }
+__device__ __forceinline__ uint32_t winner_key(double w) { return (uint32_t)((uint64_t)__double_as_longlong(w) >> 16); }
+__device__ __forceinline__ int winner_chunk(double w) { return (int)((uint32_t)__double_as_longlong(w) & 0xffffu); }
 // minimum and maximum of two winners as one instruction each (fmin / fmax first bring every operand that comes round a
 // loop into canonical form, one more instruction per operand and turn; winners are never NaN)
 __device__ __forceinline__ double min_winner(double a, double b) {
@@ -914,63 +913,53 @@ __device__ __forceinline__ double max_winner(double a, double b) {
   return a > b ? a : b;
 #endif
 }
-// score and chunk of a list entry (the chunk lies TO_CHUNK bytes after the score), requested here and awaited there: the
-// compiler waits for an LDS read of its own where it issues it when the address comes round a loop.  Nothing else of
-// the wave may be on its way from LDS between the two calls, and the values may only be used after the second.
-template <int TO_CHUNK>
-__device__ __forceinline__ void entrant_request(uint32_t lds_addr, float &score, int &chunk) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %2 offset:%3" : "=&v"(score), "=&v"(chunk) : "v"(lds_addr), "n"(TO_CHUNK));
-#else
-  score = 0.f;
-  chunk = (int)lds_addr;
-#endif
-}
-__device__ __forceinline__ void entrant_await(float &score, int &chunk) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(score), "+v"(chunk));
-#endif
-}
-__device__ __forceinline__ double shfl_xor32_d(double v) {
+// in lanes 0..31 the word of lane + 32, in the others +infinity
+__device__ __forceinline__ double upper_half_or_inf(double v) {
   const uint64_t u = (uint64_t)__double_as_longlong(v);
-  const uint64_t o = ((uint64_t)(uint32_t)shfl_xor32_i((int)(u >> 32)) << 32) | (uint32_t)shfl_xor32_i((int)(uint32_t)u);
-  return __longlong_as_double((long long)o);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, 0u, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), 0x7ff00000u, false, false);
+  return double_of(hi[1], lo[1]);
+#else
+  return v;
+#endif
+}
+// a float in LDS, requested here and awaited there: the compiler waits for an LDS read of its own where it issues it when the
+// address comes round a loop.  Nothing else of the wave may be on its way from LDS between the two calls, and the value may
+// only be used after the second.
+__device__ __forceinline__ void entrant_request(uint32_t lds_addr, float &score) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("ds_read_b32 %0, %1" : "=v"(score) : "v"(lds_addr));
+#else
+  score = (float)lds_addr;
+#endif
+}
+__device__ __forceinline__ void entrant_await(float &score) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(score));
+#endif
 }
 
-// a * b + c on 24-bit operands, one instruction (the compiler picks a 64-bit multiply-add for this address pattern)
-__device__ __forceinline__ uint32_t mad24_u32(int a, int b, uint32_t c) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t d;
-  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
-  return d;
-#else
-  return (uint32_t)(a * b) + c;
-#endif
+constexpr int kStreamGroup = 64;            // chunks per group: the bits of a row's mask
+constexpr int kStreamRowBytes = 64 * 4 + 16;  // a row's scores in LDS (16 bytes more: eight rows apart in banks)
+constexpr int kGateSlack = 3;               // (1, 3, 5 too many: 262144 tokens 2970, 2921, 2912 us, 32768 tokens 260, 250, 254)
+template <int HD>
+static constexpr size_t gate_stream_smem() {
+  return (size_t)kStreamGroup * HD * 2 + (size_t)kGateRows * kStreamRowBytes;  // tile and scores; later the selection words of a pass
 }
-constexpr int kStreamListMargin = 64;  // words on either side of a wave's lists
-constexpr int kStreamListStride = 19;  // words from one row's list (18 slots) to the next
-constexpr int kStreamListWords = 4 * (32 * kStreamListStride + 2 * kStreamListMargin) + 256;
-template <typename T, int HD, int NT>
-__global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void topk_gate_stream_kernel(TopkParams p) {
-  constexpr int CAP = 16, PL = 8;
+template <typename T, int HD>
+__global__ __launch_bounds__(256, HD > 128 ? 2 : 3) void topk_gate_stream_kernel(TopkParams p) {
+  constexpr int PL = 8;                   // winners' places per lane
   constexpr int KS = HD / 16;
-  constexpr int GC = NT * 32;             // chunks per group
+  constexpr int GC = kStreamGroup, NT = GC / 32;
   constexpr int VPR = HD / 8;             // 16-byte pieces of a row of chunk means
   constexpr int RPI = 64 / VPR;           // tile rows one load instruction brings (64 lanes x 16 bytes)
   constexpr int NV = GC / RPI / 4;        // load instructions per wave and tile
   static_assert(NV >= 1 && NV * RPI * 4 == GC, "the four waves share a tile evenly");
   constexpr int RB = HD * 2;              // bytes of a tile row: exactly HD elements, swizzled instead of padded
-  constexpr int LS = CAP + 2;                 // slots of a row's list: 16 entries and the two lanes' next slots
-  // words of an entrant array: per wave the lists of its 32 rows between two margins, then a trash word per thread.
-  // A lane with more entrants than its row's list holds writes on into the lists of the wave's other rows and, from
-  // the first and the last row, into a margin (at most 63 - 17 slots beyond the list): such a wave takes the bisection
-  // and rebuilds its lists, and no other wave's list is touched, so the slot needs no clamp.
-  constexpr int EW = kStreamListWords;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint32_t *sSel = reinterpret_cast<uint32_t *>(smem);  // [word columns of a pass][128], reuses the tile and the lists after the last group
-  float *sEv = reinterpret_cast<float *>(smem + (size_t)GC * RB);  // [EW] scores of the entrants
-  constexpr size_t head = (size_t)GC * RB + (size_t)2 * EW * 4;
-  int *sHist = reinterpret_cast<int *>(smem + head);                   // [32 chunks per word column of a pass]
+  // after the last group the words and counts of WP word columns at a time: [WP][128], [WP][32]
+  uint32_t *sSel = reinterpret_cast<uint32_t *>(smem);
 
   const fmoba_fused_topk_args &a = p.a;
   const int mb = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
@@ -1036,15 +1025,10 @@ __global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void topk_gate_stream_kernel(
   // this lane's operand row of a 32-chunk tile: row lane % 32, pieces hh * KS ..
   const uint32_t a_row = ldsTile + (uint32_t)((lane & 31) * RB);
   const int a_swz = tile_swz<HD>(lane & 31);
-  double win[PL];  // this lane's share of the row's winners, ascending (win[0] is the weakest the lane holds)
+  double win[PL];  // places hh * PL .. of the row's winners, ascending
 #pragma unroll
-  for (int j = 0; j < PL; ++j) win[j] = kSlotEmpty;
-  int m_prev = 0;    // winners the row holds
-  // (lists kStreamListStride = 19 words apart: with 18, an even number, rows l and l + 16 share a bank and every
-  // store of the 32 lanes of a half wave takes two turns)
-  float *const my_list_v = sEv + wave * (32 * kStreamListStride + 2 * kStreamListMargin) + kStreamListMargin + (lane & 31) * kStreamListStride;
-  float *const my_trash = sEv + 4 * (32 * kStreamListStride + 2 * kStreamListMargin) + tid;
-  constexpr int kToIdx = EW;  // from a score of the entrant arrays to its chunk, in words
+  for (int j = 0; j < PL; ++j) win[j] = hh * PL + j < kp ? kSlotEmpty : kSlotFiller;
+  const uint32_t row_b = ldsTile + (uint32_t)(GC * RB + rs * kStreamRowBytes);  // the row's scores
 
   if (ngroups > 0) tile_issue(0);
 #pragma nounroll
@@ -1100,165 +1084,31 @@ __global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void topk_gate_stream_kernel(
     __syncthreads();  // everyone has read the tile: the next group's chunk means may land in it
     if (g + 1 < ngroups) tile_issue(g + 1);
 
-    // ---- later groups: streaming update ---------------------------------------------------------
-    // A row that still has candidates in this group had at least GC of them in the first one, so it already holds
-    // kp winners.  Only the new scores that reach its weakest winner can enter (a new chunk has a higher index than
-    // every earlier one, so an equal score wins the tie).
-    // In the groups right after the first a row expects about kp ln((g + 1) / g) entrants (every position of a random
-    // stream enters with probability kp / position), which for the second group of a row with sixteen winners is more
-    // than a list takes for some row of nearly every wave: such groups are streamed tile by tile.
-    bool streamed = false;
-    if (g > 0 && __all(m_prev == kp || nc <= c0)) {
-      const int part_tiles = (kp > 10 * g) ? 1 : NT;
-      streamed = true;
-#pragma nounroll
-      for (int t0 = 0; t0 < n_tiles; t0 += part_tiles) {
-        const int t1 = t0 + part_tiles;
-        const double weakest = fmin(win[0], shfl_xor32_d(win[0]));
-        // (a row without winners, or one whose list is not full because it has no candidates left, admits nothing)
-        const float pmin = winner_real(weakest) ? order_key_float(winner_key(weakest)) : INFINITY;
-        // slot c of the lane with chunks 0..3 is entry c, of its partner entry LS - 1 - c; beyond the list both stay
-        // on the row's last slot
-        const uint32_t slot0 = (uint32_t)(uintptr_t)(my_list_v + (hh ? LS - 1 : 0));
-        const int slot_step = hh ? -4 : 4;  // bytes
-        int cbase = c0 + 4 * hh;
-        asm volatile("" : "+v"(cbase));  // (one register: the compiler would add its scalar and vector parts per position)
-        int cnt = 0;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          if (t >= t0 && t < t1 && t < n_tiles) {
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-              const Flags4 ge = flags4_ge(sc[t][4 * i4], sc[t][4 * i4 + 1], sc[t][4 * i4 + 2], sc[t][4 * i4 + 3], pmin);
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                const int i = 4 * i4 + j;
-                const uint32_t d = mad24_u32(cnt, slot_step, slot0);
-                lds_write_vec<float>(d, sc[t][i]);
-                lds_write_vec<int>(d + (uint32_t)kToIdx * 4u, cbase + t * 32 + 8 * (i >> 2) + (i & 3));
-                cnt = count_flag(cnt, ge.m[j]);
-              }
-            }
-          }
-        const int cnt_o = shfl_xor32_i(cnt);
-        const int ne_row = cnt + cnt_o;
-        if (!__all(ne_row <= CAP)) {
-          // the search below takes over; tiles whose entrants have gone into the winners leave the competition
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            if (t < t0) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) sc[t][i] = -INFINITY;
-            }
-          streamed = false;
-          break;
-        }
-        wave_lds_fence();
-        const int ne_lo = hh ? cnt_o : cnt;  // entrants that came from the bottom of the list
-        auto stream = [&](auto plc) {
-          constexpr int PLX = decltype(plc)::value;
-          // (entrant e + 1 is on its way from the list while entrant e goes up the entries)
-          auto slot_of = [&](int e) { return e < ne_row ? (e < ne_lo ? e : LS - 1 - (e - ne_lo)) : 0; };
-          const uint32_t list_b = (uint32_t)(uintptr_t)my_list_v;
-          float xv;
-          int xc;
-          entrant_request<kToIdx * 4>(list_b + 4u * (uint32_t)slot_of(0), xv, xc);
-          entrant_await(xv, xc);
-#pragma nounroll
-          for (int e = 0; __any(e < ne_row); ++e) {
-            const bool has = e < ne_row;
-            const double x = winner_word(xv, xc);
-            float xv_next;
-            int xc_next;
-            entrant_request<kToIdx * 4>(list_b + 4u * (uint32_t)slot_of(e + 1), xv_next, xc_next);
-            // the row's weakest winner is the lower of the two lanes' first entries; the lane that holds it drops it
-            // and passes the entrant up its sorted entries (a lane that keeps its entries passes its own first entry)
-            const double vo = shfl_xor32_d(win[0]);
-            const bool rep = has & (win[0] <= vo) & (x > win[0]);
-            const double xs = rep ? x : win[0];
-            double nw[PLX];
-            nw[0] = min_winner(xs, win[1]);
-#pragma unroll
-            for (int j = 1; j + 1 < PLX; ++j) nw[j] = min_winner(max_winner(win[j], xs), win[j + 1]);
-            nw[PLX - 1] = max_winner(win[PLX - 1], xs);
-#pragma unroll
-            for (int j = 0; j < PLX; ++j) win[j] = nw[j];
-            entrant_await(xv_next, xc_next);
-            xv = xv_next;
-            xc = xc_next;
-          }
-        };
-        // (a lane holds at most (kp + 1) / 2 winners; the fillers above them never move)
-        if (kp <= PL)
-          stream(std::integral_constant<int, PL / 2>{});
-        else
-          stream(std::integral_constant<int, PL>{});
-        wave_lds_fence();  // (the list takes the next entrants)
-      }
-    }
-    if (streamed) continue;
-
-    // ---- first group, lists that are filling, too many entrants: bisection over scores and winners ------------
-    float pv[PL];
-    int pi[PL];
-    float vmin = INFINITY, vmax = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < PL; ++j) {
-      const bool ok = winner_real(win[j]);
-      pv[j] = ok ? order_key_float(winner_key(win[j])) : -INFINITY;
-      pi[j] = ok ? winner_chunk(win[j]) : -1;
-      vmin = fminf(vmin, ok ? pv[j] : INFINITY);
-      vmax = fmaxf(vmax, pv[j]);
-    }
-    // A full list bounds the search from below: its kp winners all reach its weakest one, so the new threshold cannot
-    // lie below that score (if nothing enters, the search closes on it and the tie rule keeps the list as it is).
-    const float floor_v = (m_prev == kp && kp > 0) ? min_xor32_f(vmin) : -INFINITY;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      if (t < n_tiles) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const bool cand = c0 + t * 32 + acc_row(i, hh) < nc;
-          vmin = fminf(vmin, cand ? sc[t][i] : INFINITY);
-          vmax = fmaxf(vmax, sc[t][i]);
-        }
-      }
-    vmin = min_xor32_f(vmin);
-    vmax = max_xor32_f(vmax);
-    const int ntot = m_prev + max(0, min(nc - c0, GC));  // candidates that compete in this group
-    const bool need = (ntot > kp) && (kp > 0);
-
-    auto count_gt = [&](float probe) {
-      int cnt = 0;
+    // scores from `bound` on are the group's entrants
+    float bound;
+    if (g == 0) {
+      // No winners yet: bisection between the smallest and the largest score (as in topk_gate_kernel: first the range of values,
+      // then the range of order keys) until no more than kGateSlack scores too many lie above the lower end.  The lower end
+      // always has at least K' above it, or all there are; scores of minus infinity and NaN are never among them.
+      float vmin = INFINITY, vmax = -INFINITY;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
 #pragma unroll
-          for (int i = 0; i < 16; i += 4) cnt = count4_gt(cnt, sc[t][i], sc[t][i + 1], sc[t][i + 2], sc[t][i + 3], probe);
+        for (int i = 0; i < 16; ++i) {
+          vmin = fminf(vmin, sc[t][i] == -INFINITY ? INFINITY : sc[t][i]);  // (no candidates, or never chosen)
+          vmax = fmaxf(vmax, sc[t][i]);
         }
-      static_assert(PL % 4 == 0, "the winners are counted four at a time");
-#pragma unroll
-      for (int j = 0; j < PL; j += 4) cnt = count4_gt(cnt, pv[j], pv[j + 1], pv[j + 2], pv[j + 3], probe);
-      return sum_xor32_i(cnt);
-    };
-    float tau = -INFINITY, tau_eq = INFINITY;
-    int n_eq = 0;
-    uint32_t iota = 0u;
-    {
-      uint32_t lo_k = float_order_key(fmaxf(vmin, floor_v)) - 1u;
+      vmin = min_xor32_f(vmin);
+      vmax = max_xor32_f(vmax);
+      const int ntot = max(0, min(nc - c0, GC));
+      bool open = ntot > kp + kGateSlack && kp > 0 && vmin < vmax;
+      const uint32_t lowest = float_order_key(-INFINITY);
+      uint32_t lo_k = open ? max(float_order_key(vmin) - 1u, lowest) : lowest;
+      if (lo_k == 0x7fffffffu) lo_k -= 1u;  // (-0 is not below a vmin of +0)
       uint32_t hi_k = float_order_key(vmax);
-      int c_hi = 0;
-      bool open = need;
 #pragma nounroll
       for (int iter = 0;; ++iter) {
-        if (open && hi_k - lo_k <= 1u) {
-          tau = order_key_float(hi_k);
-          if (tau != -INFINITY) {
-            tau_eq = tau;
-            n_eq = kp - c_hi;
-          }
-          open = false;
-        }
+        open = open && hi_k - lo_k > 1u;
         if (!__any(open)) break;
         uint32_t pk = lo_k + ((hi_k - lo_k) >> 1);
         if (iter < 12) {
@@ -1267,120 +1117,93 @@ __global__ __launch_bounds__(256, NT <= 2 ? 3 : 2) void topk_gate_stream_kernel(
           if (mk > lo_k && mk < hi_k) pk = mk;
         }
         const float probe = order_key_float(pk);
-        const int cnt = count_gt(probe);
+        int cnt = 0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; i += 4) cnt = count4_gt(cnt, sc[t][i], sc[t][i + 1], sc[t][i + 2], sc[t][i + 3], probe);
+        cnt = sum_xor32_i(cnt);
         if (open) {
-          if (cnt == kp) {
-            tau = probe;
-            open = false;
-          } else if (cnt > kp) {
+          if (cnt >= kp) {
             lo_k = pk;
+            open = cnt > kp + kGateSlack;
           } else {
             hi_k = pk;
-            c_hi = cnt;
           }
         }
       }
-      const bool tie = n_eq > 0;
-      if (__any(tie)) {
-        auto count_eq_ge = [&](uint32_t trial) {
-          int cnt = 0;
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            if (t < n_tiles) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) {
-                const uint32_t c = (uint32_t)(c0 + t * 32 + acc_row(i, hh));
-                cnt += ((sc[t][i] == tau_eq) & (c >= trial)) ? 1 : 0;
-              }
-            }
-#pragma unroll
-          for (int j = 0; j < PL; ++j) cnt += ((pv[j] == tau_eq) & ((uint32_t)pi[j] >= trial) & (pi[j] >= 0)) ? 1 : 0;
-          return sum_xor32_i(cnt);
-        };
-        const int ceq = count_eq_ge(0u);
-        const bool split = tie && ceq > n_eq;
-        if (__any(split)) {
-          uint32_t i_acc = 0u;
-#pragma nounroll
-          for (int bit = 23; bit >= 0; --bit) {
-            const uint32_t trial = i_acc | (1u << bit);
-            const int cnt = count_eq_ge(trial);
-            if (cnt >= n_eq) i_acc = trial;
-          }
-          if (split) iota = i_acc;
-        }
+      // (the next float above lo, which after -0 is the smallest positive number)
+      bound = kp > 0 ? order_key_float(lo_k + (lo_k == 0x7fffffffu ? 2u : 1u)) : INFINITY;
+    } else {
+      // Scores that reach the row's weakest winner (a new chunk has a higher index than every earlier one, so an equal score
+      // wins the tie); every finite score while places are empty; none if the row keeps none
+      double weakest = win[0];
+      {
+        const uint64_t u = (uint64_t)__double_as_longlong(weakest);
+        weakest = double_of(swap32((uint32_t)(u >> 32)).a, swap32((uint32_t)u).a);
       }
+      bound = winner_real(weakest) ? order_key_float(winner_key(weakest)) : weakest < 1.0 ? order_key_float(float_order_key(-INFINITY) + 1u) : INFINITY;
     }
 
-    // the winners of this round go through the row's LDS list (densely: the partner lane starts where this one ends)
-    // and come back as alternate entries per lane
-    int nwin = 0;
-    if (kp > 0) {
+    // the scores to LDS, the row's mask of entrants (both lanes of the row hold it)
+    uint64_t mask = 0;
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
+    for (int t = 0; t < NT; ++t) {
+      uint32_t m16 = 0u;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const uint32_t c = (uint32_t)(c0 + t * 32 + acc_row(i, hh));
-            const float x = sc[t][i];
-            nwin += ((x > tau) | ((x == tau_eq) & (c >= iota))) ? 1 : 0;
-          }
-        }
+      for (int i4 = 3; i4 >= 0; --i4) {
+        const Flags4 f = flags4_ge(sc[t][4 * i4 + 3], sc[t][4 * i4 + 2], sc[t][4 * i4 + 1], sc[t][4 * i4], bound);
 #pragma unroll
-      for (int j = 0; j < PL; ++j) nwin += ((pi[j] >= 0) & ((pv[j] > tau) | ((pv[j] == tau_eq) & ((uint32_t)pi[j] >= iota)))) ? 1 : 0;
-    }
-    const int nwin_o = shfl_xor32_i(nwin);
-    const int m_new = min(nwin + nwin_o, CAP);
-    int slot = hh ? nwin_o : 0;
-    if (__any(nwin > 0)) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const uint32_t c = (uint32_t)(c0 + t * 32 + acc_row(i, hh));
-            const float x = sc[t][i];
-            const bool w = (kp > 0) & ((x > tau) | ((x == tau_eq) & (c >= iota))) & (slot < CAP);
-            float *d = w ? my_list_v + slot : my_trash;
-            d[0] = x;
-            reinterpret_cast<int *>(d)[kToIdx] = (int)c;
-            slot += w ? 1 : 0;
-          }
-        }
-#pragma unroll
-      for (int j = 0; j < PL; ++j) {
-        const bool w = (kp > 0) & (pi[j] >= 0) & ((pv[j] > tau) | ((pv[j] == tau_eq) & ((uint32_t)pi[j] >= iota))) & (slot < CAP);
-        float *d = w ? my_list_v + slot : my_trash;
-        d[0] = pv[j];
-        reinterpret_cast<int *>(d)[kToIdx] = pi[j];
-        slot += w ? 1 : 0;
+        for (int j = 0; j < 4; ++j) m16 = shift_in_flag(m16, f.m[j]);
+        const f32x4 quad = {sc[t][4 * i4], sc[t][4 * i4 + 1], sc[t][4 * i4 + 2], sc[t][4 * i4 + 3]};
+        lds_write_vec<f32x4>(row_b + (uint32_t)((t * 32 + 8 * i4) * 4 + 16 * hh), quad);
       }
+      // the four nibbles of the flags move to the places of the lane's chunks (4 hh + 8 g .. + 3)
+      const uint32_t w = ((m16 & 0xfu) | ((m16 & 0xf0u) << 4) | ((m16 & 0xf00u) << 8) | ((m16 & 0xf000u) << 12)) << (4 * hh);
+      const UPair wp = swap32(w);
+      mask |= (uint64_t)(wp.a | wp.b) << (32 * t);
     }
     wave_lds_fence();
+
+    auto stream = [&](auto two) {
+      // (entrant e + 1 is on its way from LDS while entrant e goes up the winners)
+      float xv;
+      auto next_bit = [&]() { return (int)__builtin_ctzll(mask | (1ull << 63)); };
+      int xc = next_bit();
+      bool has = mask != 0;
+      entrant_request(row_b + 4u * (uint32_t)xc, xv);
+      mask &= mask - 1;
+      entrant_await(xv);
+#pragma nounroll
+      while (__any(has)) {
+        double x = winner_word(xv, c0 + xc, has);
+        has = mask != 0;
+        xc = next_bit();
+        float xv_next;
+        entrant_request(row_b + 4u * (uint32_t)xc, xv_next);
+        mask &= mask - 1;
+        if constexpr (decltype(two)::value) x = min_winner(x, upper_half_or_inf(win[0]));  // what the strong half does not keep
 #pragma unroll
-    for (int j = 0; j < PL; ++j) {
-      const int e = 2 * j + hh;
-      const bool ok = e < m_new;
-      const double x = winner_word(my_list_v[ok ? e : 0], reinterpret_cast<const int *>(my_list_v)[kToIdx + (ok ? e : 0)]);
-      win[j] = ok ? x : (m_new == kp ? kSlotFiller : kSlotEmpty);
-    }
-    wave_lds_fence();  // (the list takes this row's entrants next)
-    // each lane's share in ascending order (odd-even transposition: this path runs once or twice per row)
-#pragma unroll
-    for (int rnd = 0; rnd < PL; ++rnd)
-#pragma unroll
-      for (int j = rnd & 1; j + 1 < PL; j += 2) {
-        const double lo = fmin(win[j], win[j + 1]), hi = fmax(win[j], win[j + 1]);
-        win[j] = lo;
-        win[j + 1] = hi;
+        for (int j = 0; j + 1 < PL; ++j) win[j] = min_winner(max_winner(win[j], x), win[j + 1]);
+        win[PL - 1] = max_winner(win[PL - 1], x);
+        entrant_await(xv_next);
+        xv = xv_next;
       }
-    m_prev = m_new;
+    };
+    // (up to eight winners have their places in the weak half alone)
+    if (kp <= PL)
+      stream(std::integral_constant<bool, false>{});
+    else
+      stream(std::integral_constant<bool, true>{});
+    wave_lds_fence();  // (the row takes the next group's scores)
   }
   __syncthreads();
 
   // selection words and per-chunk counts of the block, assembled in LDS and written out in passes of WP word columns
   // (what the tile and the lists hold), so that a sequence may have any number of chunks
-  const int WP = min(p.W, (int)(head / (kGateRows * 4)));
+  constexpr int kPassWords = (int)(gate_stream_smem<HD>() / ((kGateRows + 32) * 4));
+  const int WP = min(p.W, kPassWords);
+  int *sHist = reinterpret_cast<int *>(sSel + WP * kGateRows);
   const int seg = m0 / p.seg_rows;
   for (int w0 = 0; w0 < p.W; w0 += WP) {
     const int wn = min(WP, p.W - w0);
@@ -1860,12 +1683,6 @@ static int launch_gate(const TopkParams &p, dim3 grid, hipStream_t s) {
   hipLaunchKernelGGL(kern, grid, dim3(256), smem, s, p);
   return 0;
 }
-template <typename T, int HD>
-static int launch_gate_nt(const TopkParams &p, dim3 grid, hipStream_t s) {
-  if (p.W <= 2) return launch_gate<T, HD, 2>(p, grid, s);
-  if (p.W <= 4) return launch_gate<T, HD, 4>(p, grid, s);
-  return launch_gate<T, HD, 8>(p, grid, s);
-}
 template <int HD, int NT, int CAP>
 static constexpr size_t gate_big_smem() {
   const size_t tile = (size_t)NT * 32 * (HD + 16) * 2;  // chunk means of a group; later the selection words of a pass
@@ -1886,15 +1703,12 @@ static int launch_gate_big(const TopkParams &p, dim3 grid, hipStream_t s) {
   hipLaunchKernelGGL(kern, grid, dim3(256), smem, s, p);
   return 0;
 }
-template <int HD, int NT>
-static constexpr size_t gate_stream_smem() {
-  const size_t head = (size_t)NT * 32 * HD * 2 + (size_t)2 * kStreamListWords * 4;  // tile and lists; later the selection words of a pass
-  return head + head / (kGateRows * 4) * 32 * 4;
-}
-template <typename T, int HD, int NT>
+// chunks that a row keeps besides its own
+static int gate_winners(const TopkParams &p) { return p.a.is_causal ? p.a.topk - 1 : p.a.topk; }
+template <typename T, int HD>
 static int launch_gate_stream(const TopkParams &p, dim3 grid, hipStream_t s) {
-  const size_t smem = gate_stream_smem<HD, NT>();
-  auto kern = topk_gate_stream_kernel<T, HD, NT>;
+  const size_t smem = gate_stream_smem<HD>();
+  auto kern = topk_gate_stream_kernel<T, HD>;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("fused_topk: cannot reserve %zu bytes of LDS", smem);
     return 2;
@@ -1906,19 +1720,19 @@ template <typename T>
 static int launch_gate_big_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
   // up to 16 running winners per row: the kernel that keeps them in registers, in groups of 64 chunks (three workgroups
   // per compute unit; with groups of 128 and two workgroups it took 6.4 ms instead of 5.1 at 262144 tokens)
-  const int kp = p.a.is_causal ? p.a.topk - 1 : p.a.topk;
+  const int kp = gate_winners(p);
   if (p.a.head_dim <= 64) {
     if (kp > kBigCap) return launch_gate_big<T, 64, 4, kBigCapMax>(p, grid, s);
-    if (kp <= 16) return launch_gate_stream<T, 64, 2>(p, grid, s);
+    if (kp <= 16) return launch_gate_stream<T, 64>(p, grid, s);
     return launch_gate_big<T, 64, 8, kBigCap>(p, grid, s);
   }
   if (p.a.head_dim <= 128) {
     if (kp > kBigCap) return launch_gate_big<T, 128, 4, kBigCapMax>(p, grid, s);
-    if (kp <= 16) return launch_gate_stream<T, 128, 2>(p, grid, s);
+    if (kp <= 16) return launch_gate_stream<T, 128>(p, grid, s);
     return launch_gate_big<T, 128, 8, kBigCap>(p, grid, s);
   }
   if (kp > kBigCap) return launch_gate_big<T, 256, 2, kBigCapMax>(p, grid, s);
-  if (kp <= 16) return launch_gate_stream<T, 256, 2>(p, grid, s);
+  if (kp <= 16) return launch_gate_stream<T, 256>(p, grid, s);
   return launch_gate_big<T, 256, 4, kBigCap>(p, grid, s);
 }
 template <typename T, int HD, int NJ>
@@ -1943,6 +1757,15 @@ static int launch_gate_few_hd(const TopkParams &p, hipStream_t s) {
   if (p.a.head_dim <= 64) return launch_gate_few<T, 64>(p, s);
   if (p.a.head_dim <= 128) return launch_gate_few<T, 128>(p, s);
   return launch_gate_few<T, 256>(p, s);
+}
+template <typename T, int HD>
+static int launch_gate_nt(const TopkParams &p, dim3 grid, hipStream_t s) {
+  if (p.W <= 2) return launch_gate<T, HD, 2>(p, grid, s);
+  if (p.W <= 4) return launch_gate<T, HD, 4>(p, grid, s);
+  // more than 128 chunks and no more than 16 winners: in groups.  (32768 tokens, 32 heads, top-k 16 of 128-key chunks 306 -> 250 us; with up to
+  // 128 chunks all scores in registers are the faster form: 21000 tokens in two sequences, top-k 12 55 against 64 us, 16384 tokens, top-k 8 41 against 43.)
+  if (gate_winners(p) <= 16) return launch_gate_stream<T, HD>(p, grid, s);
+  return launch_gate<T, HD, 8>(p, grid, s);
 }
 template <typename T>
 static int launch_gate_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
