@@ -469,12 +469,8 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   // this lane's query row as the B operand of S^T = K Q^T: asked for first, on its way while the steps are counted
   Pack8 qb[KS];
   {
-    const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + min(row, Lq - 1)) * a.q_row_stride + (int64_t)h * a.q_head_stride;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int e = tile_frag_piece<HD>(hh, ks) * 8;
-      qb[ks] = (valid && e < D) ? ld_global16(qg + e) : zero_pack8();
-    }
+    const uint16_t *qg = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)q0 * a.q_row_stride + (int64_t)h * a.q_head_stride;
+    q_rows_load<HD>(qb, qg, a.q_row_stride, r0 + wave * 32, Lq, lane, D);
   }
 
   // ---- the steps of this row block -------------------------------------------------------------
@@ -584,6 +580,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
 #endif
+  q_rows_arrange<HD>(qb, hh, D);
   wait_all_loads();
   feed_k(0);
   feed_k(1);

@@ -637,6 +637,68 @@ template <int HD>
 __device__ __forceinline__ uint32_t tile_frag_addr(uint32_t at0, int ks) {
   return HD == 96 ? (at0 ^ (uint32_t)((ks & 1) * 32)) + (uint32_t)((ks >> 1) * 64) : at0 ^ (uint32_t)(ks * 16);
 }
+// The 32 consecutive query rows of a wave as B operands, q[ks] = piece tile_frag_piece(hh, ks) of row lane % 32, in two parts: the loads
+// and, once they have arrived, the exchange.  Four lanes fetch 64 bytes of a row together: lane group g = lane / 16 brings one of four
+// adjacent pieces of row lane % 16 (q[2 i]) and of row 16 + lane % 16 (q[2 i + 1]), sixteen lines a load.  (Lanes that fetch their own row's
+// pieces touch 64 lines a load: gate of 24571 tokens, 32 heads 68.6 -> 62.2 us, of 2 x 4096, 16 heads 22.1 -> 19.4.)
+// row: sequence's first row that the wave takes; rows from `rows` on are copies of the last.
+template <int HD>
+__device__ __forceinline__ void q_rows_load(Pack8 (&q)[HD / 16], const uint16_t *base, int64_t row_stride, int row, int rows, int lane, int D) {
+  const int g = lane >> 4;
+  const int gp = HD == 96 ? ((g & 1) << 1) | (g >> 1) : g;  // (one exchange is enough: its order of the pieces suits the other)
+  const uint16_t *even = base + (int64_t)min(row + (lane & 15), rows - 1) * row_stride, *odd = base + (int64_t)min(row + 16 + (lane & 15), rows - 1) * row_stride;
+#pragma unroll
+  for (int i = 0; i < HD / 32; ++i) {
+    const int e = min((4 * i + gp) * 8, D - 8);  // (features past D: zeroed by the exchange)
+    q[2 * i] = ld_global16(even + e);
+    q[2 * i + 1] = ld_global16(odd + e);
+  }
+}
+template <int HD>
+__device__ __forceinline__ void q_rows_arrange(Pack8 (&q)[HD / 16], int hh, int D) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int KS = HD / 16;
+  auto swap = [](auto wide, uint32_t &x, uint32_t &y) {
+    if constexpr (decltype(wide)::value) {
+      const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+      x = r[0], y = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+      x = r[0], y = r[1];
+    }
+  };
+  std::integral_constant<bool, true> halves;
+  std::integral_constant<bool, false> rows16;
+  Pack8 out[KS];
+  if constexpr (HD == 96) {
+#pragma unroll
+    for (int i = 0; i < KS; i += 2) {
+      out[i] = q[i], out[i + 1] = q[i + 1];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) swap(rows16, out[i].w[w], out[i + 1].w[w]);
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < KS / 4; ++t) {  // pieces 4 t .. 4 t + 3 for the lower half of the wave, those KS further on for the upper
+      Pack8 x0 = q[2 * t], x1 = q[2 * t + 1], y0 = q[2 * (t + KS / 4)], y1 = q[2 * (t + KS / 4) + 1];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        swap(halves, x0.w[w], y0.w[w]);
+        swap(halves, x1.w[w], y1.w[w]);
+        swap(rows16, x0.w[w], x1.w[w]);
+        swap(rows16, y0.w[w], y1.w[w]);
+      }
+      out[4 * t] = x0, out[4 * t + 1] = x1, out[4 * t + 2] = y0, out[4 * t + 3] = y1;
+    }
+  }
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) q[ks].w[w] = D == HD || tile_frag_piece<HD>(hh, ks) * 8 < D ? out[ks].w[w] : 0u;
+#else
+  (void)q, (void)hh, (void)D;
+#endif
+}
 // Transposing reads: address of feature tile dt (32 features) from that of tile 0, and of the row eight further down
 template <int HD>
 __device__ __forceinline__ uint32_t tile_tr_addr(uint32_t at0, int dt) { return HD == 96 ? at0 + (uint32_t)(dt * 64) : at0 ^ (uint32_t)(dt * 64); }

@@ -61,3 +61,19 @@ def test_selection_of_exact_scores(kind, C, topk, D, causal):
             if causal:
                 want[r, own] = True
         assert (got == want).all(), np.argwhere(got != want)[:4]
+
+
+def test_more_row_blocks_than_the_second_dimension_of_a_grid():
+    L, chunk = 65536 * 128 + 5, 65536
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn((L, 1, 8), generator=g, device="cuda").to(torch.bfloat16)
+    cu = torch.tensor([0, L], dtype=torch.int32, device="cuda")
+    co, cn, ind = flash_moba.flash_topk_varlen_func(x, x, cu, cu, L, L, 2, chunk, causal=True)
+    off, nnz = co.flatten().tolist(), cn.flatten().tolist()
+    rows = torch.zeros(L, dtype=torch.int32, device="cuda")
+    for c in range(len(nnz)):
+        e = ind[off[c]:off[c] + nnz[c]].long()
+        own = torch.arange(c * chunk, min(L, (c + 1) * chunk), device="cuda")
+        assert torch.equal(e[:own.numel()], own) and (e[1:] > e[:-1]).all()
+        rows.index_add_(0, e, torch.ones_like(e, dtype=torch.int32))
+    assert (rows[:chunk] == 1).all() and (rows[chunk:] == 2).all()
