@@ -744,6 +744,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     opaque(ak0);
     s_plain(ak0, st[0]);
   }
+  __syncthreads();  // every wave has read K(0): K(2) takes its place
   auto step = [&](auto par, int t) {
     // K(t + 1) and V(t) are in LDS (the wait before the last barrier); the readers of K(t) and V(t - 1) are done
     feed_k(t + 2);

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import flash_moba
+from flash_moba import flash_moba_hip as hip
 from gpu_utils import assert_close
 from test_gpu_item_order import _reference
 
@@ -33,3 +34,16 @@ def test_row_block_workgroups(lens, H, Hk, D, chunk, topk, dtype):
     want = _reference(q, k, v, torch.zeros_like(q), cu, *pattern, chunk)[0]
     # (the bound of the other attention tests)
     assert_close("out", out, want, 2e-2, 1e-2)
+
+
+def test_row_blocks_repeat_to_the_last_bit():
+    """Workgroups whose waves drift apart (two to a unit, thousands of them): nothing may land in a tile that a wave still reads."""
+    lens, H, D, chunk, topk = [13632, 9600, 5376, 2752], 16, 128, 64, 32
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v = (torch.randn((sum(lens), H, D), generator=g, device="cuda").to(torch.bfloat16) for _ in range(3))
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device="cuda")
+    run = lambda: flash_moba.flash_moba_varlen_func(q, k, v, cu, cu, max(lens), max(lens), chunk, topk, causal=True)
+    with torch.no_grad():
+        first = run()
+        assert hip.last_fwd_row_blocks()
+        assert all(torch.equal(run(), first) for _ in range(200))
