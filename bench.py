@@ -104,18 +104,18 @@ def time_events(fn, iters, warmup=1):
 # same counter reads for a plain 1 GiB copy (the summaries of those runs are kept under profiles/, one per workload).
 # Counter runs cannot be made from inside this script, so the figures are the committed measurement.
 MEASURED_TRAFFIC_BYTES = {
-    ("headline", "attn_fwd_rows_kernel"): 1.431e9,
-    ("headline", "attn_bwd_dkdv_kernel"): 7.395e9,
-    ("headline", "attn_bwd_dq_kernel"): 5.902e9,
-    ("c2", "attn_fwd_col_kernel"): 4.816e8,
-    ("c3", "attn_fwd_col_kernel"): 8.155e9,
-    ("c3", "attn_bwd_dkdv_partials_kernel"): 1.303e10,
-    ("c5", "attn_fwd_col_kernel"): 3.996e10,
-    ("c5", "attn_bwd_dkdv_partials_kernel"): 6.704e10,
-    ("sweep16k", "attn_fwd_col_kernel"): 2.303e9,
-    ("sweep16k", "attn_bwd_dkdv_partials_kernel"): 2.961e9,
-    ("sweep64k", "attn_fwd_col_kernel"): 9.459e9,
-    ("sweep64k", "attn_bwd_dkdv_partials_kernel"): 1.559e10,
+    ("headline", "attn_fwd_rows_kernel"): 1.420e9,
+    ("headline", "attn_bwd_dkdv_kernel"): 7.411e9,
+    ("headline", "attn_bwd_dq_kernel"): 5.590e9,
+    ("c2", "attn_fwd_col_kernel"): 4.772e8,
+    ("c3", "attn_fwd_col_kernel"): 8.160e9,
+    ("c3", "attn_bwd_dkdv_partials_kernel"): 1.306e10,
+    ("c5", "attn_fwd_col_kernel"): 3.979e10,
+    ("c5", "attn_bwd_dkdv_partials_kernel"): 6.702e10,
+    ("sweep16k", "attn_fwd_col_kernel"): 2.277e9,
+    ("sweep16k", "attn_bwd_dkdv_partials_kernel"): 2.963e9,
+    ("sweep64k", "attn_fwd_col_kernel"): 9.408e9,
+    ("sweep64k", "attn_bwd_dkdv_partials_kernel"): 1.557e10,
 }
 
 

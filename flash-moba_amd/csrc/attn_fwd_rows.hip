@@ -7,14 +7,14 @@
 // part in the matrix products of a step, and the rows that did not select the chunk are masked out
 // of the softmax (their probabilities are exact zeros).  The running maximum, the running sum and
 // the output accumulators stay in registers for the whole walk, so nothing but Q, K, V and the
-// output moves.  Two kernels of 128 rows per workgroup: attn_fwd_rows_kernel (four compute waves, or two
-// sets of four, that fetch the K/V tiles straight into LDS themselves; head dimensions up to 128 and up to
-// 512 chunks per sequence) and attn_fwd_rows_loader_kernel (four compute and four loader waves; every
+// output moves.  Two kernels: attn_fwd_rows_kernel (128 rows and four waves per workgroup, or 64 rows and one or
+// two sets of two, that fetch the K/V tiles straight into LDS themselves; head dimensions up to 128 and up to
+// 512 chunks per sequence) and attn_fwd_rows_loader_kernel (128 rows, four compute and four loader waves; every
 // other shape, head dimension 256 included).  Calls with at most eight query rows per sequence have a
 // kernel of their own (attn_fwd_few.hip).
 //
-// The selection of a row is one bit per chunk (a bitmap built from the CSC lists by
-// csc_bitmap_kernel); the chunks a workgroup walks are the OR of its rows' bitmaps.
+// The selection of a row is one bit per chunk (the gating's own, or a bitmap built from the CSC lists by
+// csc_bitmap_lds_kernel); the chunks a workgroup walks are the OR of its rows' bitmaps.
 #include "fmoba_common.h"
 
 #include <type_traits>
