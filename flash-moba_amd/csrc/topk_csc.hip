@@ -1394,6 +1394,16 @@ __global__ __launch_bounds__(256) void csc_scan_kernel(TopkParams p) {
     // How many chunks a row selected below each word of its selection, and its visits: independent of the scan, whose few
     // workgroups mostly wait (scan without and with them: 8192 tokens, 16 heads 6.0 and 6.8 us; 262144 tokens 122 and 250 us)
     const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b], last = (Lk + a.chunk - 1) / a.chunk - 1;  // the sequence's last chunk
+    // rows before the first sequence and after the last one (a buffer longer than its batch) have no visits: the combine kernels
+    // look at every row
+    {
+      uint32_t *vh = p.ranks.visits + (int64_t)h * a.total_q;
+      const int64_t first = (int64_t)(blockIdx.z - 1) * 256 + tid, step = (int64_t)(gridDim.z - 1) * 256;
+      if (b == 0)
+        for (int64_t i = first; i < q0; i += step) vh[i] = 0u;
+      if (b == a.batch - 1)
+        for (int64_t i = (int64_t)q0 + Lq + first; i < a.total_q; i += step) vh[i] = 0u;
+    }
     for (int k = 0; k < kRankRows; k += 256) {
       const int r = (int)(blockIdx.z - 1) * kRankRows + k + tid;
       if (r >= Lq) return;

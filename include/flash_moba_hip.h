@@ -103,7 +103,7 @@ int fmoba_fused_topk(const fmoba_fused_topk_args *a, void *stream);
 int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, int32_t want_lists, void *stream);
 /* The lists with the place of every entry among the chunks of its row: an entry is row | rank << 24, rank = number of chunks with a
  * lower index that the row selected (top-k is at most 64, max_seqlen_q below 2^24).  visits[h * total_q + t] = visits of row t of
- * head h in key blocks of the attention, forward in the low 16 bits, backward (partials form) in the high 16 bits; prefix: scratch of
+ * head h in key blocks of the attention, forward in the low 16 bits, backward (partials form) in the high 16 bits, 0 for rows of no sequence; prefix: scratch of
  * heads * ceil(max_seqlen_k / chunk / 32) * total_q bytes (may be NULL if that is one word per row).  With them the attention passes
  * put a visit's partial result where it belongs, instead of handing out places from a counter per row and sorting them when they are
  * added up.  Such lists are for the _ranked entry points alone.  No counterpart in the reference. */

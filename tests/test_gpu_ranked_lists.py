@@ -42,6 +42,40 @@ def test_ranked_lists_give_the_bits_of_counted_places(monkeypatch, lens_q, lens_
     _both(monkeypatch, run)
 
 
+# A buffer longer than its batch, at both ends: rows that belong to no sequence come out as with plain lists, whatever the memory of the
+# call held before (NaN here).  One word of selection per row and several, partial rows in 16 bits and in fp32, row blocks with
+# partial rows of dQ; more such rows than a block of the scan has threads
+@pytest.mark.parametrize("lens_q,lens_k,before,after,H,D,chunk,topk,rows,partials", [
+    ([4100, 300], [4100, 300], 3, 700, 2, 128, 128, 2, 0, 1), ([9000], [9000], 300, 1, 2, 64, 128, 2, 0, 1), ([2100], [2100], 0, 3000, 2, 256, 128, 4, 0, 0),
+    ([5, 3], [7000, 9100], 2, 9, 2, 128, 128, 4, 1, 1)])
+def test_rows_of_no_sequence_are_zero(monkeypatch, lens_q, lens_k, before, after, H, D, chunk, topk, rows, partials):
+    g = torch.Generator(device="cuda").manual_seed(D)
+    nq = sum(lens_q) + before + after
+    mk = lambda n: torch.randn((n, H, D), generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v, dout = mk(nq), mk(sum(lens_k)), mk(sum(lens_k)), mk(nq)
+    cq = before + torch.tensor([0] + list(np.cumsum(lens_q)), dtype=torch.int32, device="cuda")
+    ck = torch.tensor([0] + list(np.cumsum(lens_k)), dtype=torch.int32, device="cuda")
+
+    def run():
+        qg, kg, vg = (t.clone().requires_grad_(True) for t in (q, k, v))
+        seen = []
+        qg.register_hook(lambda _: seen.append(hip.last_bwd_partials()))
+        nan = [torch.full((n >> 2,), 0x7fc07fc0, dtype=torch.int32, device="cuda") for n in [1 << 19] * 32 + [1 << 24] * 16 + [1 << 28]]
+        del nan
+        out = flash_moba.flash_moba_varlen_func(qg, kg, vg, cq, ck, max(lens_q), max(lens_k), chunk, topk, causal=True)
+        assert hip.last_fwd_row_blocks() == rows
+        nan = [torch.full((n >> 2,), 0x7fc07fc0, dtype=torch.int32, device="cuda") for n in [1 << 19] * 32 + [1 << 24] * 16 + [1 << 28]]
+        del nan
+        out.backward(dout)
+        assert seen == [partials]
+        own = slice(before, nq - after)
+        for t in ([] if rows else [out.detach()]) + ([qg.grad] if partials else []):  # (the other forms leave such rows alone)
+            assert not torch.cat([t[:before], t[nq - after:]]).any()
+        return [t.view(torch.int16) for t in (out.detach()[own], qg.grad[own], kg.grad, vg.grad)]
+
+    _both(monkeypatch, run)
+
+
 def test_ranked_lists_hold_the_rows_of_plain_ones():
     """Row | rank << 24, as the entry point documents it, and the visits of every row."""
     import ctypes
