@@ -71,7 +71,8 @@ struct BwdWs {
 // up, a wave per column, in front of its rows; found by every workgroup of the dQ pass for its own row block, two searches of
 // a dozen dependent loads per column, they were a quarter of that pass on short sequences.  Delta and dQ pass, and the clearing of the
 // padded delta that was a launch of its own: 8191 tokens of short documents 43.4 -> 36.6 us, 24571 tokens, 32 over 8 heads 728 -> 697,
-// 65536 tokens in eight sequences 1675 -> 1656 (12 M probes take 25 us of the delta pass and 40 out of the dQ pass).
+// 65536 tokens in eight sequences 1675 -> 1656 (its places take 25 us of the delta pass; with those looked up that no row block reads, past a
+// sequence's end or before a column's first row, 27, and beside 256 sequences of 512 tokens one of 65536 took 842 us instead of 788).
 constexpr int kDqRows = 256;
 struct RunTable {
   int cols, blocks;  // columns of all sequences, row blocks + 1
@@ -1608,13 +1609,19 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
 }
 
 // grid (ceil(max_seqlen_q / rows_per_block), heads, batch), block 256.
-// LPR lanes cooperate on one row (LPR = power of two >= head_dim / 8).
+// LPR = 2^lg_lpr lanes cooperate on one row (LPR >= head_dim / 8).
 constexpr int kPrepRows = 4;  // rows per thread: eight 16-byte loads in flight (with one row a thread had two, 4.7 TB/s)
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int LPR, int32_t *tab, RunTable rt, int row_mask, int ztab) {
-  const int rows_per_pass = 256 / LPR;
-  if ((int)blockIdx.z < ztab) {  // four columns of the run table, before everything else: a chain of loads that the rows cover
-    const int lane = threadIdx.x & 63, Bn = a.lg_block_n, h = blockIdx.y;
+__global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int lg_lpr, int32_t *tab, RunTable rt, int row_mask, int ztab) {
+  const int LPR = 1 << lg_lpr, rows_per_pass = 256 >> lg_lpr;
+  // Uneven batches have up to millions of blocks past their sequence's end, each of which lives as long as its chain of loads: they leave
+  // before anything else (65536 tokens and 256 sequences of 512: 764 -> 526 us)
+  const int h = blockIdx.y, b = (int)blockIdx.z - ztab;
+  const int q0 = a.cu_seqlens_q[max(b, 0)], Lq = a.cu_seqlens_q[max(b, 0) + 1] - q0;
+  const int first = (int)blockIdx.x * rows_per_pass * kPrepRows;
+  if (b >= 0 && blockIdx.x > 0 && first >= Lq) return;
+  if (b < 0) {  // four columns of the run table, before everything else: a chain of loads that the rows cover
+    const int lane = threadIdx.x & 63, Bn = a.lg_block_n;
     const int64_t col = ((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (col >= rt.cols) return;
     // the sequence: the last one whose columns begin at or before this one
@@ -1625,17 +1632,22 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
       lo += (below - 1) * step;
       hi = min(lo + step, hi);
     }
-    const int c = (int)col - (a.cu_seqlens_k[lo] / Bn + lo);
-    if (c < 0 || c >= a.max_cols || c * Bn >= a.cu_seqlens_k[lo + 1] - a.cu_seqlens_k[lo]) return;
+    const int c = (int)col - (a.cu_seqlens_k[lo] / Bn + lo), Lk = a.cu_seqlens_k[lo + 1] - a.cu_seqlens_k[lo];
+    if (c < 0 || c >= a.max_cols || c * Bn >= Lk) return;
     const int64_t ci = ((int64_t)lo * a.heads + h) * a.max_cols + c;
     const int nnz = a.col_nnz[ci];
     const int32_t *list = a.row_indices + a.col_offsets[ci];
+    // The boundaries that the dQ pass reads: from the first row block that sees the column to the end of the sequence
+    const int rows = a.cu_seqlens_q[lo + 1] - a.cu_seqlens_q[lo];
+    const int first_row = a.is_causal ? max(c * Bn - (Lk - rows), 0) : 0;
+    if (first_row >= rows) return;
+    const int rb_first = first_row / kDqRows, rb_end = min((rows + kDqRows - 1) / kDqRows + 1, rt.blocks);
     // G lanes per boundary: a step of the search narrows it G + 1 times (short sequences have few boundaries and wait for the steps)
     int G = 64;
-    while (G > 1 && G * rt.blocks > 64) G >>= 1;
+    while (G > 1 && G * (rb_end - rb_first) > 64) G >>= 1;
     const int li = lane % G;
     const unsigned long long mine = (G == 64 ? ~0ull : (1ull << G) - 1) << (lane - li);
-    for (int rb0 = 0; rb0 < rt.blocks; rb0 += 64 / G) {
+    for (int rb0 = rb_first; rb0 < rb_end; rb0 += 64 / G) {
       const int rb = rb0 + lane / G, v = rb * kDqRows;
       int l = 0, r = nnz;
       while (__any(l < r)) {
@@ -1644,12 +1656,10 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
         l += below * step;
         r = below < G ? min(l + step - 1, r) : r;
       }
-      if (li == 0 && rb < rt.blocks) tab[rt.at(h, (int)col) + rb] = l;
+      if (li == 0 && rb < rb_end) tab[rt.at(h, (int)col) + rb] = l;
     }
     return;
   }
-  const int h = blockIdx.y, b = blockIdx.z - ztab;
-  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   if (blockIdx.x == 0) {  // what lies between the sequences of the padded layout is zero
     float *dh = a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch);
     const int64_t end = b == a.batch - 1 ? (int64_t)a.total_q + 128 * (int64_t)a.batch : (int64_t)q0 + Lq + 128 * (int64_t)(b + 1);
@@ -1657,9 +1667,8 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
     if (b == 0)
       for (int i = threadIdx.x; i < q0; i += 256) dh[i] = 0.f;
   }
-  const int r0 = blockIdx.x * rows_per_pass * kPrepRows + threadIdx.x / LPR;
-  if ((int)(blockIdx.x * rows_per_pass * kPrepRows) >= Lq) return;
-  const int sub = threadIdx.x % LPR;
+  if (first >= Lq) return;
+  const int r0 = first + (threadIdx.x >> lg_lpr), sub = threadIdx.x & (LPR - 1);
   const int e = sub * 8;
   const int D = a.head_dim;
   Pack8 o[kPrepRows], g[kPrepRows];
@@ -1805,16 +1814,16 @@ template <typename T>
 static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hipStream_t s) {
   const bool partials = bwd_dq_partials(a);
   if (phases & FMOBA_BWD_PREP) {
-    int lpr = 1;
-    while (lpr * 8 < a.head_dim) lpr <<= 1;
-    const int nx = ceil_div(a.max_seqlen_q, 256 / lpr * kPrepRows);
+    int lg_lpr = 0;
+    while ((8 << lg_lpr) < a.head_dim) ++lg_lpr;
+    const int nx = ceil_div(a.max_seqlen_q, (256 >> lg_lpr) * kPrepRows);
     const RunTable rt = bwd_run_table(a);
     const int ztab = partials ? 0 : (int)ceil_div64(ceil_div(rt.cols, 4), nx);
     if (a.batch + ztab <= 65535) {
-      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lpr, ws.tab, rt, ws.row_mask, ztab);
+      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, ztab);
     } else {  // (more planes than a launch has)
-      if (ztab > 0) hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(ceil_div(rt.cols, 4), a.heads, 1), dim3(256), 0, s, a, lpr, ws.tab, rt, ws.row_mask, 1);
-      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch), dim3(256), 0, s, a, lpr, ws.tab, rt, ws.row_mask, 0);
+      if (ztab > 0) hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(ceil_div(rt.cols, 4), a.heads, 1), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, 1);
+      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, 0);
     }
   }
   if (a.head_dim > 128) {

@@ -43,3 +43,26 @@ def test_dq_over_row_blocks_agrees_with_partial_rows(lens_q, lens_k, D, chunk, t
     # (fp32 sums of D products in another order: a few 2^-24 of the sum of their magnitudes, which is below D here)
     assert (sd - layout).abs().max() < 1e-5 * D
     assert (sd[:, pad] == 0).all()
+
+
+# The places are looked up from the first row block that sees a column to the end of its sequence: one sequence far longer than the others,
+# columns that begin inside a row block, queries that are the last rows (columns before the first row, after the last), and the plain rule
+@pytest.mark.parametrize("lens_q,lens_k,chunk,topk", [([5000] + [70] * 9, [5000] + [70] * 9, 64, 4), ([700, 3], [1500, 2000], 64, 3), ([900], [400], 192, 2)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_places_between_a_columns_first_row_and_the_end(lens_q, lens_k, chunk, topk, causal):
+    H, D = 2, 64
+    g = torch.Generator(device="cuda").manual_seed(sum(lens_q) + chunk)
+    mk = lambda n: torch.randn((n, H, D), generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v, dout = mk(sum(lens_q)), mk(sum(lens_k)), mk(sum(lens_k)), mk(sum(lens_q))
+    cq, ck = (torch.tensor([0] + list(np.cumsum(x)), dtype=torch.int32, device="cuda") for x in (lens_q, lens_k))
+    mq, mkk, scale = max(lens_q), max(lens_k), D ** -0.5
+    csc = flash_moba.flash_topk_varlen_func(q, k, cq, ck, mq, mkk, topk, chunk, causal=causal)
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *csc, cq, ck, None, None, None, mq, mkk, 0.0, scale, False, causal, 0.0, False, 128, chunk, None)
+    res = []
+    for mode in (1, 2):
+        held = [torch.full((1 << 17,), -1, dtype=torch.int32, device="cuda") for _ in range(64)]  # (what the workspace may hold before)
+        del held
+        res.append(hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, *csc, cq, ck, None, mq, mkk, 0.0, scale, False, causal, 0.0, False,
+                                       128, chunk, None, _dq_mode=mode))
+    for name, x, y in zip(("dq", "dk", "dv"), *res):  # (bounds as above)
+        assert_close(name, x, y, 2e-2, 1e-2)
