@@ -133,7 +133,7 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
   int slot = 0;
   const int sub = a.lg_block_n / KB, jb = (key0 - c * a.lg_block_n) / KB;  // key blocks of a column, this one's number
   // (no branch around the loads: where two paths join, the compiler copies what was loaded, and waits for it there)
-  auto pick = [&](auto async, int t) {
+  auto pick = [&](auto to_lds, int t) {
     t = min(t, ntile - 1);
     g = __popcll(__ballot(incl <= t));
     const int first = t - (g ? __builtin_amdgcn_readlane(incl, g - 1) : 0);
@@ -142,8 +142,8 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
     const int64_t at = (int64_t)(((uint64_t)bhi << 32) | blo) + first * 32;
     rem = n - first * 32;
     const int32_t *p = a.row_indices + at + min(lane & 31, rem - 1);
-    if constexpr (decltype(async)::value)
-      ridn = load_async(p);
+    if constexpr (decltype(to_lds)::value)
+      global_to_lds4(p, ldsOut);
     else
       ridn = *p;
   };
@@ -193,7 +193,7 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
   };
   // The row ids of the first tile before the block's K and V, and waited for without them: the counter of a wave's loads counts in
   // order, and the Q rows are the longest chain of a workgroup with few tiles (column bounds, row ids, rows: parts of prompts of 1024 rows
-  // against 9000 to 33000 keys 160 -> 154 us).
+  // against 9000 to 33000 keys 160 -> 154 us).  They come by way of the wave's part of LDS for the partial rows.
   pick(std::true_type{}, wave);
   constexpr int RPI = 64 / VPR, NI = KB / RPI / NW;
   {
@@ -210,9 +210,7 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
     }
   }
   wait_loads_but<2 * NI>();
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("" : "+v"(ridn));
-#endif
+  ridn = lds_read_vec<int>(ldsOut + (uint32_t)(lane * 4));
   fetch(wave);
   pick(std::false_type{}, wave + NW);
   arrived();

@@ -772,6 +772,15 @@ __device__ __forceinline__ void global_to_lds16_sbase(uint32_t lane_byte_off, co
   (void)lane_byte_off, (void)uniform_base, (void)lds_base;
 #endif
 }
+// 64 lanes x 4 bytes to LDS bytes [lds_base, lds_base + 256), in the same way.  For a value that other loads are issued behind and that is wanted
+// before them: in a register it would be one that the compiler may copy or spill before it has arrived.
+__device__ __forceinline__ void global_to_lds4(const void *g, uint32_t lds_base) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_base) : "memory");
+#else
+  (void)g, (void)lds_base;
+#endif
+}
 template <int N>
 __device__ __forceinline__ void wait_loads_but() {  // until at most N of the wave's vector memory loads are outstanding
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -792,16 +801,6 @@ __device__ __forceinline__ void wait_all_loads() {
 __host__ __device__ __forceinline__ int64_t ds_piece_offset(int64_t p, int kg, int kgs) { return ((((p >> 5) * kgs + kg) << 5) + (p & 31)) << 3; }
 static inline size_t ds_workspace_tiles(int64_t positions) { return (size_t)((positions > 0 ? positions : 0) + 31) / 32 + 1; }
 
-// a 32-bit load that the compiler does not wait for; the caller does, before the value is used
-__device__ __forceinline__ int load_async(const int32_t *p) {
-  int x = 0;
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("global_load_dword %0, %1, off" : "=v"(x) : "v"(p) : "memory");
-#else
-  (void)p;
-#endif
-  return x;
-}
 // *p += 1 in the lanes of `lanes`; the old value arrives with the wave's other loads (the caller waits), what the other
 // lanes get is undefined
 __device__ __forceinline__ int take_slot(int32_t *p, unsigned long long lanes) {
