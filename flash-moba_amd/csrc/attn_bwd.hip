@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
       if constexpr (DQP && RANKED)
         slot = rank * nsub + jsub;
       else if constexpr (DQP)
-        slot = take_slot(ws.cnt + ((int64_t)(q0 + rc) * a.heads + w.h), __ballot(rid >= 0 && hh == 0 && kq == 0 && counted));
+        slot = take_slot(ws.cnt + ((int64_t)(q0 + rc) * a.heads + w.h), rid >= 0 && hh == 0 && kq == 0 && counted);
     };
     auto arrived = [&]() {
       wait_all_loads();

@@ -167,7 +167,7 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
     if constexpr (RANKED)
       slot = (ridn >> kListRowBits) * sub + jb;
     else
-      slot = take_slot(ws.cnt + ((int64_t)(q0 + (rid & 0x7fffffff)) * a.heads + hcur), __ballot(rid >= 0 && hh == 0 && t < ntile));
+      slot = take_slot(ws.cnt + ((int64_t)(q0 + (rid & 0x7fffffff)) * a.heads + hcur), rid >= 0 && hh == 0 && t < ntile);
   };
   auto arrived = [&]() {
     wait_all_loads();

@@ -801,22 +801,11 @@ __device__ __forceinline__ void wait_all_loads() {
 __host__ __device__ __forceinline__ int64_t ds_piece_offset(int64_t p, int kg, int kgs) { return ((((p >> 5) * kgs + kg) << 5) + (p & 31)) << 3; }
 static inline size_t ds_workspace_tiles(int64_t positions) { return (size_t)((positions > 0 ? positions : 0) + 31) / 32 + 1; }
 
-// *p += 1 in the lanes of `lanes`; the old value arrives with the wave's other loads (the caller waits), what the other
-// lanes get is undefined
-__device__ __forceinline__ int take_slot(int32_t *p, unsigned long long lanes) {
+// *p += 1 where `mine`; the old value there, 0 in the other lanes.  (An ordinary branch: the compiler leaves the result where the atomic
+// puts it and waits for it at its first use.)
+__device__ __forceinline__ int take_slot(int32_t *p, bool mine) {
   int old = 0;
-#if defined(__HIP_DEVICE_COMPILE__)
-  unsigned long long saved;
-  asm volatile("s_mov_b64 %1, exec\n\t"
-               "s_mov_b64 exec, %2\n\t"
-               "global_atomic_add %0, %3, %4, off sc0\n\t"
-               "s_mov_b64 exec, %1"
-               : "=&v"(old), "=&s"(saved)
-               : "s"(lanes), "v"(p), "v"(1)
-               : "memory");
-#else
-  (void)p, (void)lanes;
-#endif
+  if (mine) old = __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return old;
 }
 

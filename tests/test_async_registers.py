@@ -8,6 +8,7 @@ import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flash-moba_amd", "csrc")
 FAMILIES = {  # an instruction that writes a register later, the counter that says when
+    "atomic": (r"(global|flat|buffer)_atomic_\w+[^\\]* (sc0|glc)", "vmcnt"),
     "load": (r"(global|flat|buffer|scratch)_load_(?!lds)", "vmcnt"),
 }
 
