@@ -907,7 +907,7 @@ __device__ __forceinline__ double winner_word(float score, int chunk, bool has) 
 __device__ __forceinline__ bool winner_real(double w) { return w >= 1.0 && w < (double)INFINITY; }
 __device__ __forceinline__ uint32_t winner_key(double w) { return (uint32_t)((uint64_t)__double_as_longlong(w) >> 16); }
 __device__ __forceinline__ int winner_chunk(double w) { return (int)((uint32_t)__double_as_longlong(w) & 0xffffu); }
-// minimum and maximum of two winners as one instruction each (fmin / fmax first bring every operand that comes round a
+// the lesser of two winners as one instruction (fmin first brings every operand that comes round a
 // loop into canonical form, one more instruction per operand and turn; winners are never NaN)
 __device__ __forceinline__ double min_winner(double a, double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -916,15 +916,6 @@ __device__ __forceinline__ double min_winner(double a, double b) {
   return d;
 #else
   return a < b ? a : b;
-#endif
-}
-__device__ __forceinline__ double max_winner(double a, double b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  double d;
-  asm("v_max_f64 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
-  return d;
-#else
-  return a > b ? a : b;
 #endif
 }
 // in lanes 0..31 the word of lane + 32, in the others +infinity
@@ -938,20 +929,39 @@ __device__ __forceinline__ double upper_half_or_inf(double v) {
   return v;
 #endif
 }
-// a float in LDS, requested here and awaited there: the compiler waits for an LDS read of its own where it issues it when the
-// address comes round a loop.  Nothing else of the wave may be on its way from LDS between the two calls, and the value may
-// only be used after the second.
-__device__ __forceinline__ void entrant_request(uint32_t lds_addr, float &score) {
+// A winner word x goes up the ascending places w, all but the largest of eight and x stay: and while it does, the float at lds_addr is on
+// its way, which is the result.  One statement from the request to the wait: the compiler waits for an LDS read of its own where it issues it when
+// the address comes round a loop, and a register whose value has yet to arrive must not be one that it may copy or spill.  (Nothing
+// else of the wave may be on its way from LDS.)
+__device__ __forceinline__ float insert_winner(double (&w)[8], double x, uint32_t lds_addr) {
+  float score;
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("ds_read_b32 %0, %1" : "=v"(score) : "v"(lds_addr));
+  double t;
+  asm volatile("ds_read_b32 %0, %10\n\t"
+               "v_max_f64 %9, %1, %11\n\t"
+               "v_min_f64 %1, %9, %2\n\t"
+               "v_max_f64 %9, %2, %11\n\t"
+               "v_min_f64 %2, %9, %3\n\t"
+               "v_max_f64 %9, %3, %11\n\t"
+               "v_min_f64 %3, %9, %4\n\t"
+               "v_max_f64 %9, %4, %11\n\t"
+               "v_min_f64 %4, %9, %5\n\t"
+               "v_max_f64 %9, %5, %11\n\t"
+               "v_min_f64 %5, %9, %6\n\t"
+               "v_max_f64 %9, %6, %11\n\t"
+               "v_min_f64 %6, %9, %7\n\t"
+               "v_max_f64 %9, %7, %11\n\t"
+               "v_min_f64 %7, %9, %8\n\t"
+               "v_max_f64 %8, %8, %11\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(score), "+&v"(w[0]), "+&v"(w[1]), "+&v"(w[2]), "+&v"(w[3]), "+&v"(w[4]), "+&v"(w[5]), "+&v"(w[6]), "+&v"(w[7]), "=&v"(t)
+               : "v"(lds_addr), "v"(x)
+               : "memory");
 #else
+  w[7] = x;
   score = (float)lds_addr;
 #endif
-}
-__device__ __forceinline__ void entrant_await(float &score) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(score));
-#endif
+  return score;
 }
 
 constexpr int kStreamGroup = 64;            // chunks per group: the bits of a row's mask
@@ -1036,6 +1046,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 2 : 3) void topk_gate_stream_kernel
   // this lane's operand row of a 32-chunk tile: row lane % 32, pieces hh * KS ..
   const uint32_t a_row = ldsTile + (uint32_t)((lane & 31) * RB);
   const int a_swz = tile_swz<HD>(lane & 31);
+  static_assert(PL == 8, "insert_winner");
   double win[PL];  // places hh * PL .. of the row's winners, ascending
 #pragma unroll
   for (int j = 0; j < PL; ++j) win[j] = hh * PL + j < kp ? kSlotEmpty : kSlotFiller;
@@ -1179,27 +1190,19 @@ __global__ __launch_bounds__(256, HD > 128 ? 2 : 3) void topk_gate_stream_kernel
 
     auto stream = [&](auto two) {
       // (entrant e + 1 is on its way from LDS while entrant e goes up the winners)
-      float xv;
       auto next_bit = [&]() { return (int)__builtin_ctzll(mask | (1ull << 63)); };
       int xc = next_bit();
       bool has = mask != 0;
-      entrant_request(row_b + 4u * (uint32_t)xc, xv);
+      float xv = lds_read_vec<float>(row_b + 4u * (uint32_t)xc);
       mask &= mask - 1;
-      entrant_await(xv);
 #pragma nounroll
       while (__any(has)) {
         double x = winner_word(xv, c0 + xc, has);
         has = mask != 0;
         xc = next_bit();
-        float xv_next;
-        entrant_request(row_b + 4u * (uint32_t)xc, xv_next);
         mask &= mask - 1;
         if constexpr (decltype(two)::value) x = min_winner(x, upper_half_or_inf(win[0]));  // what the strong half does not keep
-#pragma unroll
-        for (int j = 0; j + 1 < PL; ++j) win[j] = min_winner(max_winner(win[j], x), win[j + 1]);
-        win[PL - 1] = max_winner(win[PL - 1], x);
-        entrant_await(xv_next);
-        xv = xv_next;
+        xv = insert_winner(win, x, row_b + 4u * (uint32_t)xc);
       }
     };
     // (up to eight winners have their places in the weak half alone)

@@ -1,4 +1,4 @@
-"""Loads whose result is a register are the compiler's to wait for.  An assembly statement that issues one and leaves the wait to a later
+"""Loads and atomics whose result is a register are the compiler's to wait for.  An assembly statement that issues one and leaves the wait to a later
 statement gives the compiler a register that it takes for written: it may copy or spill the old value in between, silently."""
 import glob
 import os
@@ -9,6 +9,7 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flash-moba_amd", "csrc")
 FAMILIES = {  # an instruction that writes a register later, the counter that says when
     "atomic": (r"(global|flat|buffer)_atomic_\w+[^\\]* (sc0|glc)", "vmcnt"),
+    "lds": (r"ds_(read|bpermute|permute|swizzle|\w+_rtn)", "lgkmcnt"),
     "load": (r"(global|flat|buffer|scratch)_load_(?!lds)", "vmcnt"),
 }
 
