@@ -1386,14 +1386,18 @@ __global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
   }
 }
 
-// grid (heads, batch, 1 + blocks of kRankRows rows if ranks are wanted), block 256
+// grid (heads, batch, 1 + blocks of kRankRows rows if ranks are wanted), block 256.
+// RANKS: with the blocks of the ranks, a kernel of its own: in one with both, the scan of plain lists was 4073 instructions with 36 scalars
+// spilled, 571 and none without (8192 tokens, 16 heads 5.4 -> 4.9 us, 32768 tokens, 32 heads 13.3 -> 12.6).  The ranks' loops stay
+// unrolled, spilled scalars and all: rolled up they keep fewer loads in flight (262144 tokens 254 -> 264 us).
 constexpr int kRankRows = 1024;
+template <bool RANKS>
 __global__ __launch_bounds__(256) void csc_scan_kernel(TopkParams p) {
   const fmoba_fused_topk_args &a = p.a;
   const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
   const int q0 = a.cu_seqlens_q[b];
   const int Lq = a.cu_seqlens_q[b + 1] - q0;
-  if (blockIdx.z > 0) {
+  if (RANKS && blockIdx.z > 0) {
     // How many chunks a row selected below each word of its selection, and its visits: independent of the scan, whose few
     // workgroups mostly wait (scan without and with them: 8192 tokens, 16 heads 6.0 and 6.8 us; 262144 tokens 122 and 250 us)
     const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b], last = (Lk + a.chunk - 1) / a.chunk - 1;  // the sequence's last chunk
@@ -1877,7 +1881,7 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
     // no query rows: every column is empty, offsets are the (constant) region bases
     const int64_t n = (int64_t)a->batch * a->heads * max_cols;
     hipLaunchKernelGGL(fill_i32_kernel, dim3(256), dim3(256), 0, s, p.segcnt, (int64_t)(seg_bytes / 4), 0);
-    hipLaunchKernelGGL(csc_scan_kernel, dim3(a->heads, a->batch), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(csc_scan_kernel<false>, dim3(a->heads, a->batch), dim3(256), 0, s, p);
     (void)n;
     FMOBA_LAUNCH_CHECK("fused_topk(no rows)");
     return 0;
@@ -1902,7 +1906,10 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("topk_gate_kernel");
   if (!lists) return 0;
-  hipLaunchKernelGGL(csc_scan_kernel, dim3(a->heads, a->batch, 1 + (ranks ? ceil_div(a->max_seqlen_q, kRankRows) : 0)), dim3(256), 0, s, p);
+  if (ranks)
+    hipLaunchKernelGGL(csc_scan_kernel<true>, dim3(a->heads, a->batch, 1 + ceil_div(a->max_seqlen_q, kRankRows)), dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL(csc_scan_kernel<false>, dim3(a->heads, a->batch), dim3(256), 0, s, p);
   FMOBA_LAUNCH_CHECK("csc_scan_kernel");
   hipLaunchKernelGGL(ranks ? csc_fill_kernel<true> : csc_fill_kernel<false>, dim3(p.nseg * p.W, a->heads, a->batch), dim3(64), 0, s, p);
   FMOBA_LAUNCH_CHECK("csc_fill_kernel");
