@@ -399,7 +399,10 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
 // headers, order, rows) is mostly waiting, so a wave runs four of them side by side.  Lane li of a group owns the
 // 16-byte pieces li, li + 16, .. (NP of them) of the row, whose elements are of type E
 // (NORM: divided by the visit's sum of probabilities).
-// RANKED: the slots are in key-block order and none of the first `visits` is empty.
+// RANKED: the slots are in key-block order and none of the first `visits` is empty.  The addresses of a row's partials are then known
+// together, which the compiler spends registers on: five waves per SIMD instead of seven with 16-bit rows, two instead of three with fp32
+// ones.  It is no loss, and no launch bound asks for more: held to 72 and 168 registers the kernel spills and takes 814 us instead of
+// 800 (32768 tokens, 32 heads, top-k 16; 262144 tokens 3430 and 3385) and 108 instead of 89 (2 x 4096 tokens of 256-wide heads, top-k 8).
 template <typename T, typename E, int NP, bool NORM, bool RANKED>
 __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_args a, FwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
