@@ -257,6 +257,8 @@ def run_config(name, steps, warmup, args, dev, cpu_budget_s):
         co, cn, ind, _, _, selection = hip.moba_fused_topk(q.detach(), km0, cu, cu, cu_km0, max_len, max_len, topk, chunk, True,
                                                            return_raw=False, return_selection=True)
         del km0
+    plain = (co, cn, ind)
+    row_visits = None
     pairs = count_pairs(seqlens, cn, chunk, H)
     fwd_flops = 4.0 * D * pairs
     bwd_flops = 2.5 * fwd_flops
@@ -279,11 +281,26 @@ def run_config(name, steps, warmup, args, dev, cpu_budget_s):
     def fwd(**kw):
         return hip.moba_varlen_fwd(qd, kd, vd, None, co, cn, ind, cu, cu, None, None, None, max_len, max_len, 0.0, scale,
                                    False, True, 0.0, False, lg_m, chunk, None, _fwd_mode=args.fwd_mode, _max_visits=visits,
-                                   _selection=selection, **kw)
+                                   _selection=selection, _visits=row_visits, **kw)
 
     fwd_phase_ms = {}
-    fwd()
+    out, lse, _, _ = fwd()
     row_blocks = bool(hip.last_fwd_row_blocks())  # which of the two forward forms the library picks for this shape
+    partials = False
+    if backward:
+        dq, dk, dv = torch.empty_like(qd), torch.empty_like(kd), torch.empty_like(vd)
+        bwd_visits = visits * (hip.fwd_key_block(chunk) // 64)
+
+        def bwd(**kw):
+            return hip.moba_varlen_bwd(dout, qd, kd, vd, out, lse, dq, dk, dv, co, cn, ind, cu, cu, None, max_len, max_len, 0.0,
+                                       scale, False, True, 0.0, False, lg_m, chunk, None, None, _dq_mode=args.dq_mode,
+                                       _max_visits=bwd_visits, _visits=row_visits, **kw)
+
+        bwd()
+        partials = bool(hip.last_bwd_partials())
+    ranked = not row_blocks or partials  # forms with partial results per visit: the timed steps run them over ranked lists, and so does what follows
+    if ranked:
+        co, cn, ind, selection, row_visits = hip.pool_and_gate_ranked(qd, kd, cu, cu, max_len, max_len, topk, chunk, True)
     fwd_names = ("selection_bits", "row_blocks") if row_blocks else ("columns", "combine")
 
     def run_fwd_phases(run):
@@ -299,8 +316,11 @@ def run_config(name, steps, warmup, args, dev, cpu_budget_s):
         "mean_pool": {"ms": t_pool, "GBps": pool_bytes / t_pool / 1e6, "frac_hbm": pool_bytes / t_pool / 1e6 / PEAK_HBM_GBS},
         "topk_csc": {"ms": t_gate, "GBps": gate_bytes / t_gate / 1e6, "frac_hbm": gate_bytes / t_gate / 1e6 / PEAK_HBM_GBS},
         "attn_fwd": {"ms": t_fwd, "TFLOPs": fwd_flops / t_fwd / 1e9, "frac_mfma": fwd_flops / t_fwd / 1e9 / PEAK_BF16_TFLOPS,
-                     "phases_ms": fwd_phase_ms},
+                     "phases_ms": fwd_phase_ms, "lists": "ranked" if ranked else "plain"},
     }
+    if ranked:  # pooling, gate and ranked lists as the timed steps run them (topk_csc: the public gating function, plain lists)
+        t_ranked = time_events(lambda: hip.pool_and_gate_ranked(qd, kd, cu, cu, max_len, max_len, topk, chunk, True), it)
+        stages["pool_and_gate_ranked"] = {"ms": t_ranked}
     # Compulsory HBM bytes of a launch: the tensors it has to read and write, once each (q, k, v, out, dout, dq, dk, dv of
     # T*H*D*2 bytes, the selection bits or the CSC lists); rows that a kernel gathers again per visit count once.  What a
     # form of a kernel writes or reads per list entry on top of that (partial results, dS tiles) is the implementation's
@@ -314,22 +334,14 @@ def run_config(name, steps, warmup, args, dev, cpu_budget_s):
     if row_blocks:
         kernels = {"attn_fwd_rows_kernel": (fwd_phase_ms["row_blocks"], fwd_flops, 4 * qkv_once + T * H * ((maxC + 31) // 32) * 4, 0)}
     else:
-        kernels = {"attn_fwd_col_kernel": (fwd_phase_ms["columns"], fwd_flops, 3 * qkv_once + list_bytes, fwd_visits * (D * 2 + 16))}
+        kernels = {"attn_fwd_col_kernel": (fwd_phase_ms["columns"], fwd_flops, 3 * qkv_once + list_bytes, fwd_visits * (D * 2 + 8))}
     if backward:
-        dq, dk, dv = torch.empty_like(qd), torch.empty_like(kd), torch.empty_like(vd)
         phase_ms = {}
 
         def run_phases(run):
             run(7)  # make the buffers consistent first
             for name, mask in (("prep", 1), ("dkdv", 2), ("dq", 4)):
                 phase_ms[name] = time_events(lambda: run(mask), it)
-
-        bwd_visits = visits * (hip.fwd_key_block(chunk) // 64)
-
-        def bwd(**kw):
-            return hip.moba_varlen_bwd(dout, qd, kd, vd, out, lse, dq, dk, dv, co, cn, ind, cu, cu, None, max_len, max_len, 0.0,
-                                       scale, False, True, 0.0, False, lg_m, chunk, None, None, _dq_mode=args.dq_mode,
-                                       _max_visits=bwd_visits, **kw)
 
         bwd(_phases=run_phases)
         t_bwd = time_events(bwd, it)
@@ -341,12 +353,12 @@ def run_config(name, steps, warmup, args, dev, cpu_budget_s):
         if hip.last_bwd_partials():
             bwd_kb = 128 if (chunk % 128 == 0 and D > 64) else 64
             dkdv = "attn_bwd_dkdv_partials_kernel" if D > 64 else "attn_bwd_dkdv_kernel"
-            kernels[dkdv] = (phase_ms["dkdv"], 10.0 * D * pairs, 6 * qkv_once + list_bytes, entries * (chunk // bwd_kb) * (D * 2 + 4))
+            kernels[dkdv] = (phase_ms["dkdv"], 10.0 * D * pairs, 6 * qkv_once + list_bytes, entries * (chunk // bwd_kb) * D * 2)
         else:
             kernels["attn_bwd_dkdv_kernel"] = (phase_ms["dkdv"], 8.0 * D * pairs, 6 * qkv_once + list_bytes, entries * chunk * 2)
             kernels["attn_bwd_dq_kernel"] = (phase_ms["dq"], 2.0 * D * pairs, 2 * qkv_once + list_bytes, entries * chunk * 2)
     # sort alone, on the CSC the gating produced (already sorted input; same traffic)
-    t_sort = time_events(lambda: torch.ops.flash_moba._varlen_sort(co, cn, ind), it)
+    t_sort = time_events(lambda: torch.ops.flash_moba._varlen_sort(*plain), it)
     sort_bytes = 2 * int(cn.sum().item()) * 4 + 2 * cn.numel() * 8
     stages["varlen_sort"] = {"ms": t_sort, "GBps": sort_bytes / t_sort / 1e6, "frac_hbm": sort_bytes / t_sort / 1e6 / PEAK_HBM_GBS}
 
@@ -405,6 +417,8 @@ def stage_summary(r):
            "mean_pool_ms": round(st["mean_pool"]["ms"], 4), "mean_pool_frac_hbm": round(st["mean_pool"]["frac_hbm"], 4),
            "topk_csc_ms": round(st["topk_csc"]["ms"], 4), "topk_csc_frac_hbm": round(st["topk_csc"]["frac_hbm"], 4),
            "attn_fwd_ms": round(st["attn_fwd"]["ms"], 4), "attn_fwd_frac_mfma": round(st["attn_fwd"]["frac_mfma"], 4)}
+    if "pool_and_gate_ranked" in st:
+        out["pool_and_gate_ranked_ms"] = round(st["pool_and_gate_ranked"]["ms"], 4)
     for k, v in st["attn_fwd"]["phases_ms"].items():
         out["fwd_" + k + "_ms"] = round(v, 4)
     if "attn_bwd" in st:

@@ -294,6 +294,44 @@ def moba_fused_topk(q: torch.Tensor, km: torch.Tensor, cu_seqlens_q: torch.Tenso
     return res
 
 
+def pool_and_gate_ranked(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, topk, chunk, is_causal):
+    """Chunk means, gating and ranked lists as the gated path makes them for an attention with partial results per visit
+    (fmoba_pool_and_gate_ranked): [col_offsets, col_nnz, lists, selection words, visits of the rows].  Such lists are for moba_varlen_fwd /
+    moba_varlen_bwd with _visits alone."""
+    _require(q.is_cuda and k.is_cuda and q.dim() == 3 and k.dim() == 3 and q.stride(-1) == 1 and k.stride(-1) == 1 and q.dtype == k.dtype,
+             "q and k must be (total, heads, head_size) tensors of one dtype on CUDA with contiguous last dimension")
+    batch = cu_seqlens_q.numel() - 1
+    _require(batch > 0 and max_seqlen_q > 0 and max_seqlen_k > 0 and chunk > 0 and 1 <= topk <= 64, "sizes must be positive, topk at most 64")
+    _check_cu("cu_seqlens_q", cu_seqlens_q, batch)
+    _check_cu("cu_seqlens_k", cu_seqlens_k, batch)
+    total_q, heads, d = q.shape
+    total_k, heads_k = k.shape[0], k.shape[1]
+    _require(k.shape[2] == d and d <= 256 and d % 8 == 0 and heads % heads_k == 0, "heads or head sizes of q and k do not fit")
+    max_cols = (max_seqlen_k + chunk - 1) // chunk
+    words = (max_cols + 31) // 32
+    with _device_guard(q):
+        lib, dev = load_library(), q.device
+        col_offsets = torch.empty((batch, heads, max_cols), dtype=torch.int64, device=dev)
+        col_nnz = torch.empty((batch, heads, max_cols), dtype=torch.int32, device=dev)
+        lists = torch.empty((total_q * heads * topk,), dtype=torch.int32, device=dev)
+        visits = torch.empty((heads, total_q), dtype=torch.int32, device=dev)
+        prefix = torch.empty((heads * words * total_q,), dtype=torch.uint8, device=dev)
+        km = torch.empty((total_k // chunk + batch, heads_k, d), dtype=k.dtype, device=dev)
+        cu_km = torch.empty((batch + 1,), dtype=torch.int32, device=dev)
+        ws_bytes = lib.fmoba_fused_topk_workspace_bytes(batch, total_q, heads, max_seqlen_q, max_seqlen_k, chunk)
+        ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+        m = MeanPoolArgs(k.data_ptr(), km.data_ptr(), cu_seqlens_k.data_ptr(), cu_km.data_ptr(), batch, max_cols, heads_k, d, int(chunk), _dt(k),
+                         k.stride(0), k.stride(1), km.stride(0), km.stride(1))
+        a = FusedTopkArgs(q.data_ptr(), km.data_ptr(), cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), cu_km.data_ptr(),
+                          col_offsets.data_ptr(), col_nnz.data_ptr(), lists.data_ptr(), None, None, ws.data_ptr(), ws_bytes,
+                          batch, total_q, heads, heads_k, d, int(max_seqlen_q), int(max_seqlen_k), int(topk), int(chunk), int(bool(is_causal)), _dt(q),
+                          q.stride(0), q.stride(1), km.stride(0), km.stride(1))
+        r = CscRanks(visits.data_ptr(), prefix.data_ptr())
+        _check(lib.fmoba_pool_and_gate_ranked(ctypes.byref(m), ctypes.byref(a), ctypes.byref(r), _stream()))
+        off = (-ws.data_ptr()) % 256
+        return [col_offsets, col_nnz, lists, ws[off:off + heads * words * total_q * 4].view(torch.int32).view(heads, words, total_q), visits]
+
+
 # --------------------------------------------------------------------------------------
 # varlen_sort
 # --------------------------------------------------------------------------------------
@@ -398,6 +436,16 @@ def _count_visits(lib, q, moba_col_offsets, moba_col_nnz, moba_row_indices, cu_s
     return max(1, int(counts[total_q * heads].item()))
 
 
+def _row_visits(visits, max_visits, heads, total_q, device):
+    """Address of the visits of ranked lists; None: plain lists."""
+    if visits is None:
+        return None
+    _require(visits.dtype == torch.int32 and visits.device == device and visits.is_contiguous() and tuple(visits.shape) == (heads, total_q),
+             "the visits of ranked lists must be a contiguous int32 tensor of shape (num_heads, total_q) on q's device")
+    _require(max_visits is not None and int(max_visits) >= 1, "ranked lists cannot be counted: their bound has to be given")
+    return visits.data_ptr()
+
+
 def count_max_visits(q, moba_col_offsets, moba_col_nnz, moba_row_indices, cu_seqlens_q, cu_seqlens_k, total_k, heads_k,
                      max_seqlen_q, max_seqlen_k, n_lg_block_dim) -> int:
     """Largest number of (row, forward key block) visits of any (row, head) of a CSC pattern: the bound the attention
@@ -420,14 +468,15 @@ def count_max_visits(q, moba_col_offsets, moba_col_nnz, moba_row_indices, cu_seq
 def moba_varlen_fwd(q, k, v, out_, moba_col_offsets, moba_col_nnz, moba_row_indices, cu_seqlens_q, cu_seqlens_k,
                     seqused_k, leftpad_k, alibi_slopes, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale,
                     zero_tensors, is_causal, softcap, return_softmax, m_lg_block_dim, n_lg_block_dim, gen=None, _phases=None,
-                    _fwd_mode=0, _max_visits=None, _selection=None, _overflow=None):
+                    _fwd_mode=0, _max_visits=None, _selection=None, _overflow=None, _visits=None):
     """Returns [out, softmax_lse (H, total_q) fp32, p (empty), rng_state (2,) int64].
 
     Beyond the reference's arguments: _max_visits, a bound on the (row, forward key block) visits of any (row, head)
     -- a gated pattern has top-k * lg_block_n / fwd_key_block(lg_block_n); None or a value below 1 makes the call count
     them from the pattern (one device-to-host read) -- and _selection, the int32 selection words of the gating call that
     produced exactly this pattern (moba_fused_topk(return_selection=True)); _overflow, a zeroed int32 tensor of one
-    element that a form with per-visit partial results raises to the visit count of a row that exceeds the bound."""
+    element that a form with per-visit partial results raises to the visit count of a row that exceeds the bound; _visits, the
+    visits of the rows of ranked lists (pool_and_gate_ranked), which the three list tensors then have to be."""
     dtype = q.dtype
     _require(dtype in (torch.float16, torch.bfloat16), "FlashMoBA only support fp16 and bf16 data type")
     _require(k.dtype == dtype, "query and key must have the same dtype")
@@ -473,6 +522,7 @@ def moba_varlen_fwd(q, k, v, out_, moba_col_offsets, moba_col_nnz, moba_row_indi
                      and tuple(_selection.shape) == (heads, (max_cols + 31) // 32, total_q),
                      "selection bits must be a contiguous int32 tensor of shape (num_heads, ceil(max_lg_col_num / 32), total_q) on q's device")
             sel_ptr = _selection.data_ptr()
+        row_visits = _row_visits(_visits, _max_visits, heads, total_q, q.device)
 
         def args(ws_ptr, ws_bytes, visits):
             return AttnFwdArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
@@ -497,9 +547,9 @@ def moba_varlen_fwd(q, k, v, out_, moba_col_offsets, moba_col_nnz, moba_row_indi
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=q.device)
         a = args(ws.data_ptr(), ws_bytes, visits)
         if _phases is None:
-            _check(lib.fmoba_attn_fwd(ctypes.byref(a), _stream()))
+            _check(lib.fmoba_attn_fwd_ranked(ctypes.byref(a), row_visits, 3, _stream()))
         else:  # measurement hook: callable(run) receives run(mask) launching the chosen phases
-            _phases(lambda mask: _check(lib.fmoba_attn_fwd_phases(ctypes.byref(a), mask, _stream())))
+            _phases(lambda mask: _check(lib.fmoba_attn_fwd_ranked(ctypes.byref(a), row_visits, mask, _stream())))
     return [out, lse, p, rng_state]
 
 
@@ -509,12 +559,12 @@ def moba_varlen_fwd(q, k, v, out_, moba_col_offsets, moba_col_nnz, moba_row_indi
 def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_offsets, moba_col_nnz, moba_row_indices,
                     cu_seqlens_q, cu_seqlens_k, alibi_slopes, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale,
                     zero_tensors, is_causal, softcap, deterministic, m_lg_block_dim, n_lg_block_dim, gen=None,
-                    rng_state=None, _phases=None, _dq_mode=0, _max_visits=None, _overflow=None):
+                    rng_state=None, _phases=None, _dq_mode=0, _max_visits=None, _overflow=None, _visits=None):
     """Returns [dq, dk, dv, softmax_d (H, total_q + 128*batch) fp32].
 
     Beyond the reference's arguments: _max_visits, a bound on the visits of any (row, head) in 64-KEY blocks (a gated
     pattern has top-k * lg_block_n / 64); None or a value below 1 makes the call count them from the pattern (one
-    device-to-host read)."""
+    device-to-host read) -- and _visits, as for the forward."""
     dtype = q.dtype
     _require(dtype in (torch.float16, torch.bfloat16), "FlashMoBA only support fp16 and bf16 data type")
     _require(k.dtype == dtype, "query and key must have the same dtype")
@@ -563,6 +613,7 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
         dv = _grad(dv_, v, "dv", (total_k, heads_k, d))
         dev = q.device
         softmax_d = torch.empty((heads, total_q + 128 * batch), dtype=torch.float32, device=dev)
+        row_visits = _row_visits(_visits, _max_visits, heads, total_q, dev)
         lib = load_library()
         visits = _max_visits
         if visits is None or int(visits) < 1:
@@ -596,9 +647,9 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
         ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes
         if _phases is None:
-            _check(lib.fmoba_attn_bwd_grouped(ctypes.byref(a), dkv_heads, 7, _stream()))
+            _check(lib.fmoba_attn_bwd_ranked(ctypes.byref(a), row_visits, dkv_heads, 7, _stream()))
         else:  # measurement hook: callable(run) receives run(mask) launching the chosen phases
-            _phases(lambda mask: _check(lib.fmoba_attn_bwd_grouped(ctypes.byref(a), dkv_heads, mask, _stream())))
+            _phases(lambda mask: _check(lib.fmoba_attn_bwd_ranked(ctypes.byref(a), row_visits, dkv_heads, mask, _stream())))
         if dkv_heads != heads_k:
             grp = dkv_heads // heads_k
             torch.sum(dk_e.view(total_k, heads_k, grp, d), dim=2, out=dk)

@@ -106,3 +106,30 @@ def test_ranked_lists_hold_the_rows_of_plain_ones():
             seen[e & 0xffffff] += 1
         got = visits[h].cpu().numpy()
         assert (got & 0xffff == seen).all() and (got >> 16 == seen).all()
+
+
+@pytest.mark.parametrize("lens,H,Hk,D,chunk,topk,rows,partials", [([4100, 3000], 4, 2, 128, 128, 3, 0, 1), ([9000], 2, 2, 64, 64, 5, 0, 1), ([2100], 2, 1, 256, 128, 4, 0, 0), ([700], 2, 2, 128, 64, 6, 1, 0)])
+def test_attention_over_ranked_lists_by_hand(lens, H, Hk, D, chunk, topk, rows, partials):
+    """pool_and_gate_ranked, then moba_varlen_fwd / _bwd with the visits: the bits of plain lists."""
+    g = torch.Generator(device="cuda").manual_seed(sum(lens))
+    mk = lambda h: torch.randn((sum(lens), h, D), generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v, dout = mk(H), mk(Hk), mk(Hk), mk(H)
+    cu, n, scale = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device="cuda"), max(lens), D ** -0.5
+    plain = list(flash_moba.flash_topk_varlen_func(q, k, cu, cu, n, n, topk, chunk, causal=True))
+    *ranked, selection, visits = hip.pool_and_gate_ranked(q, k, cu, cu, n, n, topk, chunk, True)
+    kb = hip.fwd_key_block(chunk)
+    bound = topk * (chunk // kb)
+    res = []
+    for lists, kw in ((plain, {}), (ranked, {"_visits": visits})):
+        sel = {"_selection": selection} if rows else {}  # (row blocks over ranked lists read the selection words)
+        out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *lists, cu, cu, None, None, None, n, n, 0.0, scale, False, True, 0.0, False, 128, chunk, None,
+                                             _max_visits=bound, **sel, **kw)
+        assert hip.last_fwd_row_blocks() == rows
+        grads = hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, *lists, cu, cu, None, n, n, 0.0, scale, False, True, 0.0, False, 128, chunk, None,
+                                    _max_visits=bound * (kb // 64), **kw)
+        assert hip.last_bwd_partials() == partials
+        res.append([t.view(torch.int16) for t in (out, *grads[:3])])
+    for name, a, b in zip(("out", "dq", "dk", "dv"), *res):
+        assert torch.equal(a, b), name
+    with pytest.raises(RuntimeError, match="bound"):
+        hip.moba_varlen_fwd(q, k, v, None, *ranked, cu, cu, None, None, None, n, n, 0.0, scale, False, True, 0.0, False, 128, chunk, None, _visits=visits)
