@@ -102,20 +102,20 @@ def time_events(fn, iters, warmup=1):
 
 # HBM-side bytes per launch, per workload: rocprofv3 FETCH_SIZE + WRITE_SIZE per dispatch, each scaled by what the
 # same counter reads for a plain 1 GiB copy (the summaries of those runs are kept under profiles/, one per workload).
-# Counter runs cannot be made from inside this script, so the figures are the committed measurement.
+# Counter runs cannot be made from inside this script, so the figures are the committed measurement (ranked lists where the step has them).
 MEASURED_TRAFFIC_BYTES = {
-    ("headline", "attn_fwd_rows_kernel"): 1.420e9,
-    ("headline", "attn_bwd_dkdv_kernel"): 7.411e9,
-    ("headline", "attn_bwd_dq_kernel"): 5.590e9,
-    ("c2", "attn_fwd_col_kernel"): 4.772e8,
-    ("c3", "attn_fwd_col_kernel"): 8.160e9,
-    ("c3", "attn_bwd_dkdv_partials_kernel"): 1.306e10,
-    ("c5", "attn_fwd_col_kernel"): 3.979e10,
-    ("c5", "attn_bwd_dkdv_partials_kernel"): 6.702e10,
-    ("sweep16k", "attn_fwd_col_kernel"): 2.277e9,
-    ("sweep16k", "attn_bwd_dkdv_partials_kernel"): 2.963e9,
-    ("sweep64k", "attn_fwd_col_kernel"): 9.408e9,
-    ("sweep64k", "attn_bwd_dkdv_partials_kernel"): 1.557e10,
+    ("headline", "attn_fwd_rows_kernel"): 1.415e9,
+    ("headline", "attn_bwd_dkdv_kernel"): 7.422e9,
+    ("headline", "attn_bwd_dq_kernel"): 5.639e9,
+    ("c2", "attn_fwd_col_kernel"): 4.320e8,
+    ("c3", "attn_fwd_col_kernel"): 7.551e9,
+    ("c3", "attn_bwd_dkdv_partials_kernel"): 1.172e10,
+    ("c5", "attn_fwd_col_kernel"): 3.719e10,
+    ("c5", "attn_bwd_dkdv_partials_kernel"): 6.140e10,
+    ("sweep16k", "attn_fwd_col_kernel"): 2.132e9,
+    ("sweep16k", "attn_bwd_dkdv_partials_kernel"): 2.557e9,
+    ("sweep64k", "attn_fwd_col_kernel"): 8.810e9,
+    ("sweep64k", "attn_bwd_dkdv_partials_kernel"): 1.406e10,
 }
 
 

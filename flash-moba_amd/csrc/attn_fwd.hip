@@ -11,11 +11,13 @@
 //                             O^T = V^T P^T (V^T through transposing LDS reads).  Every visit of
 //                             a (row, key block) pair leaves a PARTIAL result: the block-local
 //                             maximum m, the sum l of exp2(s - m) and the output row (bf16 or fp32:
-//                             unnormalised; fp16: divided by l), in a slot that the row hands out from
-//                             a counter.
+//                             unnormalised; fp16: divided by l).  Over ranked lists (the gated path)
+//                             its slot is that of the key block among the row's, made of the list
+//                             entry's rank; over plain lists the row hands it out from a counter.
 //   attn_fwd_combine_kernel : sixteen lanes per (row, head) merge the row's partials in ascending
-//                             key-block order (sorted by block id, so the result does not depend
-//                             on which slot a visit happened to get): out, log-sum-exp.
+//                             key-block order: that of the slots over ranked lists, else found by
+//                             sorting the block ids, so the result does not depend on which slot a
+//                             visit happened to get.  Out, log-sum-exp.
 //
 // Work and traffic are proportional to the number of (row, key block) visits whatever the number of
 // chunks per sequence; a row-stationary formulation degenerates when every 128-row block touches

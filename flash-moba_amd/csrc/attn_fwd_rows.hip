@@ -577,7 +577,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     return;
   }
 
-  // ---- feeding the rings: each of a set's four waves fetches rows wave * 16 .. wave * 16 + 15 of a tile ----------------
+  // ---- feeding the rings: each wave of a set (two or four) fetches an equal run of a tile's 16-byte pieces, NI loads of 64 ----
   const uint32_t ldsK = (uint32_t)(uintptr_t)smem + (uint32_t)(set * (int)SM::ring), ldsV = ldsK + (uint32_t)(2 * SM::tile);
   const uint16_t *kg = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)k0 * a.k_row_stride + (int64_t)hk * a.k_head_stride;
   const uint16_t *vg = reinterpret_cast<const uint16_t *>(a.v) + (int64_t)k0 * a.v_row_stride + (int64_t)hk * a.v_head_stride;
