@@ -17,13 +17,19 @@ LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libflash_moba_hip.so")
 HOST_MODULE = "flash_moba_host"  # the eager host path (csrc/torch_ops.cpp), a Python extension beside the library
 HOST_LIB = os.path.join(LIBDIR, HOST_MODULE + ".so")
-SOURCES = ["fmoba_host.hip", "mean_pool.hip", "topk_csc.hip", "varlen_sort.hip", "attn_fwd.hip", "attn_fwd_rows.hip", "attn_fwd_few.hip", "attn_bwd.hip", "attn_bwd_wide.hip"]
+SOURCES = ["fmoba_host.hip", "mean_pool.hip", "topk_csc.hip", "varlen_sort.hip", "attn_fwd.hip", "attn_fwd_rows.hip", "attn_fwd_rows_wide.hip", "attn_fwd_few.hip", "attn_bwd.hip", "attn_bwd_wide.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # keep packed-fp32 VALU ops out of the generated code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
+
+
+# The compiler's choice between ordinary and accumulation registers for the results of matrix products, for kernels of 512 registers whose
+# results vector instructions read: left to itself it takes accumulation registers for all of them and copies (attn_fwd_rows_wide.hip: 600 copies
+# in the loop of 64 products, 60 with the flag).
+FILE_FLAGS = {"attn_fwd_rows_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def hipcc() -> str:
@@ -35,7 +41,7 @@ def hipcc() -> str:
 
 def _compile(src: str, objdir: str) -> str:
     obj = os.path.join(objdir, src.replace(".hip", ".o"))
-    cmd = [hipcc()] + FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [hipcc()] + FLAGS + FILE_FLAGS.get(src, []) + ["-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, r.stdout, r.stderr))

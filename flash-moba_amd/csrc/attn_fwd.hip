@@ -37,6 +37,11 @@ namespace fmoba {
 // line stays at 10/27 for them too, as rows that the row-block form adds up in fp32 are not moved to 16-bit partial rows
 // (8192 tokens, 0.41 of the chunks: error of the output against 64 bits 2.17e-3 in row blocks, 2.63e-3 in columns).
 constexpr int kFwdRowsDensity64 = 50, kFwdRowsDensity128 = 27;
+// The same above head dimension 128 (fp32 partial rows in the column form; whole prefill, 8 heads of 256, columns against rows): 64-key blocks,
+// 2 x 4096 tokens 0.12 of the chunks 170 against 178 us, 0.24 249 against 181, 16384 tokens 0.12 897 against 1168, 0.25 1691 against 1220; 128-key
+// blocks, 2 x 4096 tokens 0.24 176 against 188, 0.48 252 against 190, 8 x 2048 tokens 0.38 481 against 451, 16384 tokens 0.25 874 against 1169, 0.5 1552
+// against 1200.  From one 128-row block per compute unit on: fewer of them leave units idle for the length of a walk.
+constexpr int kFwdRowsDensityWide64 = 57, kFwdRowsDensityWide128 = 28, kFwdRowsWideBlocks = 256;
 constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 
 struct FwdWs {
@@ -574,6 +579,7 @@ static inline bool fwd_combine_fits(const fmoba_attn_fwd_args &a) {
 
 // the row-block form (attn_fwd_rows.hip)
 bool fwd_rows_feasible(const fmoba_attn_fwd_args &a);
+bool fwd_rows_direct(const fmoba_attn_fwd_args &a);  // without loader waves
 bool fwd_few_rows(const fmoba_attn_fwd_args &a);  // its variant for calls with a handful of rows (attn_fwd_few.hip)
 size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a);
 int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s);
@@ -586,18 +592,16 @@ static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   if (a.fwd_mode == 1) return false;
   if (!fwd_rows_feasible(a)) return false;
   if (a.fwd_mode == 2 || fwd_few_rows(a)) return true;
-  // Head dimensions above 128: the column form is the faster one at every density that was measured (columns against rows:
-  // 2 x 4096 tokens, 8 heads of 256, top-k 8 of 128-key chunks 269 against 976 us, top-k 32 of 64-key chunks 731 against 976;
-  // 16384 tokens, top-k 32 of 64-key chunks 1793 against 6918), up to the size of the partial results that a call may ask for
-  // and to what the combine has room for.
+  const int64_t chunks_per_seq = std::max<int64_t>(1, ceil_div64(ceil_div64(std::max(a.total_k, 1), a.batch), a.lg_block_n));
+  const int64_t seen = a.is_causal ? (chunks_per_seq + 1) / 2 : chunks_per_seq;
+  const int64_t chunks_per_row = std::max<int64_t>(1, (int64_t)a.max_visits_per_row * fwd_key_block(a.lg_block_n) / a.lg_block_n);
+  const bool wide_keys = fwd_key_block(a.lg_block_n) == 128;
   if (a.head_dim > 128) {
     const int64_t partials = (int64_t)a.total_q * a.heads * fwd_partial_cap(a);
-    return !fwd_combine_fits(a) || partials >= ((int64_t)1 << 31) || partials * (int64_t)(a.head_dim * fwd_part_size(a.head_dim) + 16) > kWidePartialBytes;
+    if (!fwd_combine_fits(a) || partials >= ((int64_t)1 << 31) || partials * (int64_t)(a.head_dim * fwd_part_size(a.head_dim) + 16) > kWidePartialBytes) return true;
+    return fwd_rows_direct(a) && (int64_t)a.heads * (a.total_q / 128 + a.batch) >= kFwdRowsWideBlocks && chunks_per_row * (wide_keys ? kFwdRowsDensityWide128 : kFwdRowsDensityWide64) >= seen * 10;
   }
-  const int64_t chunks_per_seq = std::max<int64_t>(1, ceil_div64(ceil_div64(std::max(a.total_k, 1), a.batch), a.lg_block_n));
-  const int64_t chunks_per_row = std::max<int64_t>(1, (int64_t)a.max_visits_per_row * fwd_key_block(a.lg_block_n) / a.lg_block_n);
-  const int64_t seen = a.is_causal ? (chunks_per_seq + 1) / 2 : chunks_per_seq;
-  return chunks_per_row * (fwd_key_block(a.lg_block_n) == 128 ? kFwdRowsDensity128 : kFwdRowsDensity64) >= seen * 10;
+  return chunks_per_row * (wide_keys ? kFwdRowsDensity128 : kFwdRowsDensity64) >= seen * 10;
 }
 
 // Query heads per workgroup.  All heads of a group share the block's K and V and a workgroup's first loads, which is most of the

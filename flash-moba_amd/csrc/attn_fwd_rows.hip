@@ -9,21 +9,18 @@
 // the output accumulators stay in registers for the whole walk, so nothing but Q, K, V and the
 // output moves.  Two kernels: attn_fwd_rows_kernel (128 rows and four waves per workgroup, or 64 rows and one or
 // two sets of two, that fetch the K/V tiles straight into LDS themselves; head dimensions up to 128 and up to
-// 512 chunks per sequence) and attn_fwd_rows_loader_kernel (128 rows, four compute and four loader waves; every
-// other shape, head dimension 256 included).  Calls with at most eight query rows per sequence have a
+// 512 chunks per sequence) and attn_fwd_rows_loader_kernel (128 rows, four compute and four loader waves; longer
+// sequences).  Head dimensions above 128 have a loop of their own in attn_fwd_rows_wide.hip.  Calls with at most eight query rows per sequence have a
 // kernel of their own (attn_fwd_few.hip).
 //
 // The selection of a row is one bit per chunk (the gating's own, or a bitmap built from the CSC lists by
 // csc_bitmap_lds_kernel); the chunks a workgroup walks are the OR of its rows' bitmaps.
-#include "fmoba_common.h"
+#include "attn_fwd_rows.h"
 
 #include <type_traits>
 #include <utility>
 
 namespace fmoba {
-
-constexpr int kRowsStepCap = 4096;  // 64-key steps of one row block (its step list lives in LDS)
-constexpr int kRowsWordCap = 128;   // bitmap words per row (32 chunks each)
 
 template <int HD>
 struct FwdRowsSmem {
@@ -457,21 +454,6 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // RW: waves of a set, which share its tiles.  SPLIT = 2: a second set of waves takes every other step of the same rows, with
 // rings of its own; the two results of a row meet in LDS at the end.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
-constexpr int kRowsWords = 16;  // selection words per row that the workgroup keeps in LDS (512 chunks)
-
-template <int HD, int RW, int SPLIT>
-struct FwdRowsDirectSmem {
-  static constexpr int ROWS = 32 * RW;  // rows of a workgroup: 32 for each wave of a set
-  static constexpr int LDO = HD + 8;   // elements, per-wave output tile [32 rows][LDO]
-  static constexpr size_t tile = (size_t)64 * HD * 2;       // one 64-key tile of K or V
-  static constexpr size_t ring = 4 * tile;                    // K, K, V, V: the rings of one set of waves
-  static constexpr size_t oStep = SPLIT * ring;               // int[step_cap]: key block | chunk << 16
-  static constexpr int UPW = ROWS / 64;                       // unions of 64 rows' selection words per word
-  // behind the steps, sized by the call: uint32[nw][UPW] unions, uint32[nw][ROWS] the rows' selection words
-  static size_t bytes(int step_cap, int nw) { return oStep + ((size_t)step_cap + (size_t)nw * (UPW + ROWS)) * 4; }
-  static_assert((size_t)RW * 32 * LDO * 2 <= ring && (size_t)RW * HD * 128 <= ring && SPLIT * RW * 512 <= ring, "output tiles must fit the K/V rings");
-};
-
 template <typename T, int HD, int RW, int SPLIT>
 __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap) {
   typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
@@ -500,7 +482,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
   const int wave = wave_all % RW, set = wave_all / RW;  // rows 32 wave .., steps set, set + SPLIT, ..
   const bool causal = a.is_causal != 0;
-  const int Bn = a.lg_block_n, sub = Bn >> 6;
+  const int Bn = a.lg_block_n;
   const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
 
   const int row = r0 + wave * 32 + (lane & 31);
@@ -515,53 +497,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   // ---- the steps of this row block -------------------------------------------------------------
   const int rlast = min(r0 + kRows - 1, Lq - 1);
   const int kend = min(Lk, causal ? rlast + off + 1 : Lk);  // keys [0, kend) are visible to some row
-  const int nchunk = kend > 0 ? (kend + Bn - 1) / Bn : 0;
-  const int nwu = min((nchunk + 31) >> 5, nw);
-  {
-    constexpr int UPW = SM::UPW;
-    const int nrow = rlast - r0 + 1;
-    const uint32_t *bp = bm + (int64_t)h * nw * a.total_q + q0 + r0;
-    // (the words stay in LDS for the walk: a load from global memory inside the step loop would make the compiler
-    // wait for every outstanding load of the wave, the tile loads included, at every step)
-    for (int it = wave_all; it < nwu * UPW; it += NTHR / 64) {  // one word of 64 rows per wave
-      const int w = it / UPW, rw = (it % UPW) * 64 + lane;
-      const uint32_t x = rw < nrow ? bp[(int64_t)w * a.total_q + rw] : 0u;
-      sBits[w * kRows + rw] = x;
-      const uint32_t u = or_wave(x);
-      if (lane == 0) sUnion[it] = u;
-    }
-  }
-  __syncthreads();
-  // One thread per chunk: a chunk of the union contributes its 64-key blocks that hold a visible key.  All but the last visible
-  // chunk have all of theirs, so a chunk's first step is the number of chunks of the union before it times the blocks of one: no
-  // scan over the workgroup, and no atomics for the unions (1024 tokens, 8 heads of 64: 14.7 -> 14.3 us).
-  const int nchunk_u = min(nchunk, nwu * 32);
-  int nstep_all = 0;
-  if (nchunk_u > 0) {
-    auto word = [&](int w) {
-      uint32_t u = sUnion[w * SM::UPW];
-      if constexpr (SM::UPW == 2) u |= sUnion[w * 2 + 1];
-      return u;
-    };
-    for (int c = tid; c < nchunk_u; c += NTHR) {
-      int before = 0;
-      for (int w = 0; w < (c >> 5); ++w) before += __popc(word(w));
-      const uint32_t u = word(c >> 5);
-      if ((u >> (c & 31)) & 1u) {
-        int pos = (before + __popc(u & ((1u << (c & 31)) - 1u))) * sub;
-        const int cnt = min(sub, (kend - c * Bn + 63) >> 6);
-        for (int jb = 0; jb < cnt; ++jb, ++pos)
-          if (pos < step_cap) sStep[pos] = (c * sub + jb) | (c << 16);
-      }
-    }
-    const int last = nchunk_u - 1;
-    const uint32_t ul = word(last >> 5) & (0xffffffffu >> (31 - (last & 31)));
-    int nsel = __popc(ul);
-    for (int w = 0; w < (last >> 5); ++w) nsel += __popc(word(w));
-    nstep_all = nsel * sub - (((ul >> (last & 31)) & 1u) ? sub - min(sub, (kend - last * Bn + 63) >> 6) : 0);
-    nstep_all = __builtin_amdgcn_readfirstlane(nstep_all);
-  }
-  __syncthreads();
+  const int nstep_all = row_block_steps<kRows, NTHR>(bm + (int64_t)h * nw * a.total_q + q0 + r0, a.total_q, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
   const int nstep_wg = min(nstep_all, step_cap);
   const int nstep = (nstep_wg - set + SPLIT - 1) / SPLIT, nturn = (nstep_wg + SPLIT - 1) / SPLIT;  // this set's steps, the turns of the loop
   auto entry = [&](int t) { return sStep[min(t * SPLIT + set, nstep_wg - 1)]; };
@@ -911,6 +847,8 @@ static int launch_rows_loader(const fmoba_attn_fwd_args &a, const uint32_t *bm, 
   return 0;
 }
 
+// head dimensions above 128 (attn_fwd_rows_wide.hip)
+int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s);
 // a call with a handful of rows (attn_fwd_few.hip)
 bool fwd_few_rows(const fmoba_attn_fwd_args &a);
 void run_fwd_few(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s);
@@ -919,6 +857,9 @@ bool fwd_rows_feasible(const fmoba_attn_fwd_args &a) {
   return a.head_dim <= 256 && ceil_div(a.max_cols, 32) <= kRowsWordCap && ceil_div(a.max_seqlen_k, 64) <= kRowsStepCap &&
          a.max_cols < 32768 && a.lg_block_n % 64 == 0;
 }
+
+// the rows' selection words fit the workgroup's LDS (512 chunks per sequence): the kernels without loader waves
+bool fwd_rows_direct(const fmoba_attn_fwd_args &a) { return ceil_div(a.max_cols, 32) <= kRowsWords; }
 
 size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a) {
   if (a.selection_bits != nullptr) return 256;
@@ -952,9 +893,8 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
   if (phases & 2) {
     const bool bf = a.dtype == FMOBA_DTYPE_BF16;
     int rc;
-    // without loader waves when the rows' selection words fit the workgroup's LDS (up to 512 chunks per sequence)
-    // (and the rows of a tile lie within 32-bit byte offsets of its first key)
-    const bool direct = nw <= kRowsWords && a.k_row_stride < ((int64_t)1 << 24) && a.v_row_stride < ((int64_t)1 << 24);
+    // (the rows of a tile lie within 32-bit byte offsets of its first key)
+    const bool direct = fwd_rows_direct(a) && a.k_row_stride < ((int64_t)1 << 24) && a.v_row_stride < ((int64_t)1 << 24);
     if (a.head_dim <= 64)
       rc = direct ? (bf ? launch_rows<bf16_t, 64>(a, bm, nw, s) : launch_rows<f16_t, 64>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 64>(a, bm, nw, s) : launch_rows_loader<f16_t, 64>(a, bm, nw, s));
@@ -964,7 +904,7 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
       rc = direct ? (bf ? launch_rows<bf16_t, 128>(a, bm, nw, s) : launch_rows<f16_t, 128>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 128>(a, bm, nw, s) : launch_rows_loader<f16_t, 128>(a, bm, nw, s));
     else
-      rc = bf ? launch_rows_loader<bf16_t, 256>(a, bm, nw, s) : launch_rows_loader<f16_t, 256>(a, bm, nw, s);
+      rc = direct ? launch_rows_wide(a, bm, nw, s) : (bf ? launch_rows_loader<bf16_t, 256>(a, bm, nw, s) : launch_rows_loader<f16_t, 256>(a, bm, nw, s));
     if (rc) return rc;
   }
   return 0;

@@ -1,0 +1,104 @@
+"""Row-block forward of head dimensions above 128: edges of its tiles, its rule, its precision beside the column form's."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import flash_moba
+from flash_moba import flash_moba_hip as hip
+from gpu_utils import assert_close
+from test_form_rules import fwd_args
+from test_gpu_item_order import _reference
+
+
+# 0.36 of the visible chunks with 128-key blocks (0.18 with 64-key ones), from one block of 128 rows per compute unit on
+@pytest.mark.parametrize("lens,chunk,topk,heads,rows", [([16384], 128, 22, 4, 0), ([16384], 128, 23, 4, 1), ([16384], 64, 22, 4, 0), ([16384], 64, 23, 4, 1),
+                                                        ([4096, 4096], 128, 8, 3, 0), ([4096, 4096], 128, 8, 4, 1)])
+def test_wide_forward_lines(lens, chunk, topk, heads, rows):
+    f = fwd_args(lens, chunk, topk, heads=heads, D=256)
+    assert hip.load_library().fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == rows
+
+
+def _inputs(lens, H, Hk, D, dtype, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q, k, v = (torch.randn((sum(lens), h, D), generator=g, device="cuda").to(dtype) for h in (H, Hk, Hk))
+    cu = [0] + [int(x) for x in np.cumsum(lens)]
+    return q, k, v, cu, torch.tensor(cu, dtype=torch.int32, device="cuda")
+
+
+def _forward(q, k, v, cu, lens, pattern, chunk, mode):
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *pattern, cu, cu, None, None, None, max(lens), max(lens), 0.0, q.shape[2] ** -0.5, False, True, 0.0,
+                                         False, 128, chunk, None, _fwd_mode=mode)
+    return out, lse
+
+
+# walks of one step and of two, rows and keys at the edges of 32, 64 and 128, a last chunk cut short, feature pieces that do not exist,
+# key heads that are shared, more than one word of selection bits
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,H,Hk,D,chunk,topk", [
+    ([1, 31, 32, 33, 0, 63, 64, 65], 2, 2, 256, 64, 2), ([127, 128, 129, 193, 257], 4, 1, 136, 64, 3), ([385, 700], 2, 1, 192, 256, 2),
+    ([2300], 2, 2, 256, 64, 20), ([513, 1100], 2, 2, 248, 128, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_row_blocks(lens, H, Hk, D, chunk, topk, dtype):
+    q, k, v, cu, cud = _inputs(lens, H, Hk, D, dtype, sum(lens) + D)
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cud, cud, max(lens), max(lens), topk, chunk, causal=True)
+    out, lse = _forward(q, k, v, cud, lens, pattern, chunk, 2)
+    # (the bound of the other attention tests)
+    assert_close("out", out, _reference(q, k, v, torch.zeros_like(q), cu, *pattern, chunk)[0], 2e-2, 1e-2)
+    # the column form's sums of the same scores are fp32 too: the two differ by the order of some 2500 of them
+    assert (lse - _forward(q, k, v, cud, lens, pattern, chunk, 1)[1]).abs().nan_to_num(0.0).max() <= 1e-4
+
+
+# equal scores: every probability is a power of two, a row the mean of its values, rounded once
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_row_blocks_round_once(dtype):
+    L, D, chunk = 900, 256, 64
+    q, k, v, _, cud = _inputs([L], 2, 2, D, dtype, 3)
+    q, v = torch.zeros_like(q), v.abs() + 0.5
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cud, cud, L, L, 15, chunk, causal=True)
+    out, _ = _forward(q, k, v, cud, [L], pattern, chunk, 2)
+    exact = v.double().cumsum(0) / torch.arange(1, L + 1, device="cuda", dtype=torch.float64)[:, None, None]
+    half_ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * (1 + 2 ** -6)  # and the 32-bit sums under it
+    assert ((out.double() - exact).abs() <= half_ulp * exact).all()
+
+
+# scores that grow by up to 2^10 from block to block and fall again, scores of -inf, and rows whose unselected chunks hold infinite ones
+@pytest.mark.gpu
+def test_wide_row_blocks_extreme_scores():
+    L, D, chunk = 640, 256, 64
+    q, k, v, cu, cud = _inputs([L], 1, 1, D, torch.bfloat16, 5)
+    size = torch.tensor([1.0, 30.0, 0.01, 120.0, 5.0, 60.0, 0.5, 90.0, 2.0, 1.0], device="cuda").repeat_interleave(chunk)
+    k = (k.float() * size[:, None, None]).to(k.dtype)
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cud, cud, L, L, 10, chunk, causal=True)
+    rows, _ = _forward(q, k, v, cud, [L], pattern, chunk, 2)
+    want = _reference(q, k, v, torch.zeros_like(q), cu, *pattern, chunk)[0]
+    assert_close("out", rows, want, 2e-2, 1e-2)
+    q = q.abs() + 0.1
+    k[3 * chunk:4 * chunk] = float("-inf")  # selected by rows that have no more than their own chunk and this one alone
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cud, cud, L, L, 3, chunk, causal=True)
+    rows, rows_lse = _forward(q, k, v, cud, [L], pattern, chunk, 2)
+    cols, cols_lse = _forward(q, k, v, cud, [L], pattern, chunk, 1)
+    assert torch.equal(rows.isnan(), cols.isnan()) and torch.equal(rows_lse.isinf(), cols_lse.isinf())
+    assert_close("out", rows.nan_to_num(0.0), cols.nan_to_num(0.0), 2e-2, 1e-2)
+    k[3 * chunk:4 * chunk] = float("inf")
+    pattern = [t.clone() for t in pattern]  # rows of a pattern that leaves those keys out
+    pattern[1][0, 0, 3] = 0
+    rows, _ = _forward(q, k, v, cud, [L], pattern, chunk, 2)
+    cols, _ = _forward(q, k, v, cud, [L], pattern, chunk, 1)
+    assert_close("out", rows, cols, 2e-2, 1e-2)
+
+
+# The largest probability of a block is a power of two, which 16 bits hold exactly, as in the column form, whose blocks are as long or
+# longer: the error against 32-bit attention is no larger (1 % for the sample)
+@pytest.mark.gpu
+@pytest.mark.parametrize("chunk,topk", [(64, 8), (128, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_row_blocks_are_as_precise_as_columns(chunk, topk, dtype):
+    lens = [2048]
+    q, k, v, cu, cud = _inputs(lens, 4, 4, 256, dtype, 7)
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cud, cud, 2048, 2048, topk, chunk, causal=True)
+    want = _reference(q, k, v, torch.zeros_like(q), cu, *pattern, chunk)[0]
+    err = [float((_forward(q, k, v, cud, lens, pattern, chunk, m)[0].float() - want).norm()) for m in (2, 1)]
+    assert err[0] <= err[1] * 1.01
