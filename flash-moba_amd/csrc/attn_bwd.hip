@@ -138,8 +138,21 @@ struct DkdvSmem {
   static_assert(bytes <= 160 * 1024 && (size_t)64 * HD * 2 <= NBUF * tile, "LDS of one compute unit; K and V pass through the tiles");
 };
 
+// a * b of two values below 2^24, b the same in every lane: one full-rate instruction (a 32-bit multiply takes four
+// times as long)
+__device__ __forceinline__ uint32_t mul24_u32(uint32_t a, uint32_t b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t d;
+  asm("v_mul_u32_u24 %0, %1, %2" : "=v"(d) : "v"(a), "s"(b));
+  return d;
+#else
+  return a * b;
+#endif
+}
+
 // RANKED (partials form): part rows go to the place of the block among the row's, which the rank of the list entry gives
-template <typename T, int HD, bool DQP, bool RANKED>
+// NEAR: a gathered row's place is a 32-bit byte offset from the sequence's first row that one 24-bit multiply makes (rows_near).
+template <typename T, int HD, bool DQP, bool RANKED, bool NEAR>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
   typedef DkdvSmem<HD, DQP> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR, PRB = SM::PRB;
@@ -280,21 +293,39 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   if (nround > 0) {
     // rows of a round (ids `rid`): Q and dO into the buffer, 16 rows per wave, of its own 32
     int ft = tid;  // thread index for the code around the products, re-made opaque in every round: what is derived from it is not kept in registers
-    auto feed = [&](int rid, const Round &w, uint32_t buf) {
-      const int fl = ft & 63;
-      const uint16_t *qh = qg + (int64_t)w.h * a.q_head_stride, *doh = dog + (int64_t)w.h * a.do_head_stride;
+    // What a round's head has of its own: changes when the walk goes on to the next head of the group.
+    struct Head {
+      int h;
+      const uint16_t *q, *dout;
+      const float *lse, *del;
+    };
+    auto head_at = [&](int h) {
+      return Head{h, qg + (int64_t)h * a.q_head_stride, dog + (int64_t)h * a.do_head_stride, a.softmax_lse + (int64_t)h * a.total_q + q0,
+                  a.softmax_d + (int64_t)h * dstride + q0 + 128 * b};
+    };
+    Head hd = head_at(w0.h);
+    uint32_t fsrc[NI];  // the rows this lane fetches pieces of
+    auto feed_rows = [&](int rid) {  // (all exchanges at once: one wait for them)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int v = i * 64 + fl, r16 = v / VPR, pc = v - r16 * VPR, tr = kq * 16 + r16;  // row of the tile of 32, piece
-        const uint32_t src = (uint32_t)__shfl(rid, tr, 64) & 0x7fffffffu;
-        const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
-        const uint32_t dst = buf + (uint32_t)((rt * 32 + kq * 16) * RB + i * 1024);
-        global_to_lds16(qh + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
-        global_to_lds16(doh + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
+      for (int i = 0; i < NI; ++i) fsrc[i] = (uint32_t)__shfl(rid, kq * 16 + (i * 64 + (ft & 63)) / VPR, 64);
+    };
+    auto feed = [&](auto ic, uint32_t buf) {  // load ic of Q and of dO
+      constexpr int I = decltype(ic)::value;
+      const int v = I * 64 + (ft & 63), r16 = v / VPR, pc = v - r16 * VPR, tr = kq * 16 + r16;  // row of the tile of 32, piece
+      const uint32_t src = fsrc[I] & 0x7fffffffu;
+      const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
+      const uint32_t dst = buf + (uint32_t)((rt * 32 + kq * 16) * RB + I * 1024);
+      if constexpr (NEAR) {
+        global_to_lds16_sbase(mul24_u32(src, (uint32_t)a.q_row_stride * 2u) + e * 2u, hd.q, ldsQ + dst);
+        global_to_lds16_sbase(mul24_u32(src, (uint32_t)a.do_row_stride * 2u) + e * 2u, hd.dout, ldsdO + dst);
+      } else {
+        global_to_lds16(hd.q + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
+        global_to_lds16(hd.dout + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
       }
     };
     int rid0 = code(raw0, w0), rid1 = code(raw_nx, w1);
-    feed(rid0, w0, 0);
+    feed_rows(rid0);
+    static_for<NI>([&](auto ic) { feed(ic, 0u); });
     float lse = 0.f, del = 0.f;
     int slot = 0;
     int *sSlot = reinterpret_cast<int *>(smem + SM::oSlot);
@@ -302,8 +333,13 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
     // LSE, delta and (partials form, handed out by the waves of key quarter 0) the part row of a round's rows
     auto scalars = [&](int rid, int rank, const Round &w, bool counted) {
       const int rc = rid & 0x7fffffff;
-      lse = a.softmax_lse[(int64_t)w.h * a.total_q + q0 + rc];
-      del = a.softmax_d[(int64_t)w.h * dstride + q0 + 128 * b + rc];
+      if constexpr (NEAR) {  // (offsets of 32 bits)
+        lse = *reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(hd.lse) + (uint32_t)rc * 4u);
+        del = *reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(hd.del) + (uint32_t)rc * 4u);
+      } else {
+        lse = hd.lse[rc];
+        del = hd.del[rc];
+      }
       if constexpr (DQP && RANKED)
         slot = rank * nsub + jsub;
       else if constexpr (DQP)
@@ -333,8 +369,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
       if constexpr (DQP) {
         if (kq == 0 && fh == 0) sSlot[(r & 1) * 64 + frow] = (rid0 >= 0 && slot < ws.cap) ? ((q0 + rid0) * a.heads + w0.h) * ws.cap + slot : trash;
       }
-      // the next round's rows and scalars, the row ids of the one after it
-      if (r + 1 < nround) feed(rid1, w1, buf ^ TILE);
+      // The next round's rows and scalars, the row ids of the one after it.  The rows are asked for between the products of S and dP, a
+      // load of Q and one of dO after every four, by 32-bit offsets.  Before the products, one after the other with an exchange, a wait for it and a
+      // 64-bit product each, and with the head's addresses made anew every round: 65536 tokens in eight sequences, training step 7543
+      // us against 7430 now, 24571 tokens, 32 over 8 heads 2782 -> 2720, 12037 tokens, heads of 96 479 -> 473, 2 x 4096 tokens 482 -> 477.
+      if (w1.h != hd.h) hd = head_at(w1.h);
+      feed_rows(rid1);
       scalars(rid1, rank1, w1, r + 1 < nround);
       raw_nx = *entry_at(w2);
       // S^T and dP^T: lane -> row, register i -> key kq * 32 + acc_row(i, hh)
@@ -361,6 +401,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
         for (int u = 0; u < NB; ++u) {
           s = mfma32<T>(kf[B * NB + u], qf[B & 1][u], s);
           dp = mfma32<T>(vf[B * NB + u], df[B & 1][u], dp);
+        }
+        if constexpr (B < NI) {
+          if (r + 1 < nround) feed(bc, buf ^ TILE);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
@@ -452,14 +495,19 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
           if (!RANKED && pcs == 0) ws.pid[p] = nb;
         }
       } else {
-        arrived();
         // dS of row `lane`, key groups 2 wave and 2 wave + 1: consecutive lanes write consecutive pieces of the dS tile
         Pack8 x[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) x[u] = lds_read16(ldsdS + (uint32_t)(lane * PRB) + (((uint32_t)(2 * wave + u) ^ (uint32_t)(lane & 7)) * 16u));
+        arrived();
         if (lane < w0.n) {
+          // ds_piece_offset(w0.pos + lane, koff / 8 + 2 wave, Bn / 8) in two parts: what the round has in common, and the lane's own
+          // (at most two tiles further on)
+          const uint32_t kgs = (uint32_t)Bn >> 3, t = ((uint32_t)w0.pos & 31u) + (uint32_t)lane;
+          uint16_t *base = ws.ds + (((w0.pos >> 5) * (int64_t)kgs + (koff >> 3) + 2 * wave) << 8);
+          uint8_t *dst = reinterpret_cast<uint8_t *>(base) + ((mul24_u32(t >> 5, kgs) << 9) + ((t & 31u) << 4));
 #pragma unroll
-          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(ws.ds + ds_piece_offset(w0.pos + lane, (koff >> 3) + 2 * wave + u, Bn >> 3)) = x[u];
+          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(dst + 512 * u) = x[u];
         }
         __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
       }
@@ -496,18 +544,6 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
     *reinterpret_cast<Pack8 *>(dvg + (int64_t)key * a.dv_row_stride + e) = ov;
     *reinterpret_cast<Pack8 *>(dkg + (int64_t)key * a.dk_row_stride + e) = ok;
   }
-}
-
-// a * b of two values below 2^24, b the same in every lane: one full-rate instruction (a 32-bit multiply takes four
-// times as long)
-__device__ __forceinline__ uint32_t mul24_u32(uint32_t a, uint32_t b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t d;
-  asm("v_mul_u32_u24 %0, %1, %2" : "=v"(d) : "v"(a), "s"(b));
-  return d;
-#else
-  return a * b;
-#endif
 }
 
 // dK / dV and dQ partials at head dimension 128 (the long calls).  Four waves of 512 registers, one per SIMD, all of which
@@ -1731,18 +1767,23 @@ static int launch_dkdv_kernel(K kern, size_t smem, int heads, int keys, const fm
   hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws);
   return 0;
 }
+// Every row of a sequence's q and dout lies within 2^31 elements of the sequence's first row and is less than 2^24 rows
+// and 2^22 elements per row away, so a gathered row's place is a 32-bit offset made by one 24-bit multiply.
+static bool rows_near(const fmoba_attn_bwd_args &a) {
+  return a.max_seqlen_q < (1 << 24) && a.q_row_stride < (1 << 22) && a.do_row_stride < (1 << 22) &&
+         (int64_t)a.max_seqlen_q * a.q_row_stride < (int64_t)0x7fff0000 && (int64_t)a.max_seqlen_q * a.do_row_stride < (int64_t)0x7fff0000;
+}
 template <typename T, int HD, bool DQP>
 static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
+  const bool near_rows = rows_near(a);
+  auto kern = near_rows ? attn_bwd_dkdv_kernel<T, HD, DQP, false, true> : attn_bwd_dkdv_kernel<T, HD, DQP, false, false>;
   if constexpr (DQP)
-    if (ws.visits != nullptr) return launch_dkdv_kernel(attn_bwd_dkdv_kernel<T, HD, DQP, true>, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
-  return launch_dkdv_kernel(attn_bwd_dkdv_kernel<T, HD, DQP, false>, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
+    if (ws.visits != nullptr) kern = near_rows ? attn_bwd_dkdv_kernel<T, HD, DQP, true, true> : attn_bwd_dkdv_kernel<T, HD, DQP, true, false>;
+  return launch_dkdv_kernel(kern, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
 }
-// NEAR: every row of a sequence's q and dout lies within 2 GB of the sequence's first row and is less than 2^24 rows
-// and 2^22 elements per row away, so a gathered row's place is a 32-bit offset made by one 24-bit multiply.
 template <typename T, int HD, int KB>
 static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
-  const bool near_rows = a.max_seqlen_q < (1 << 24) && a.q_row_stride < (1 << 22) && a.do_row_stride < (1 << 22) &&
-                         (int64_t)a.max_seqlen_q * a.q_row_stride < (int64_t)0x7fff0000 && (int64_t)a.max_seqlen_q * a.do_row_stride < (int64_t)0x7fff0000;
+  const bool near_rows = rows_near(a);
   auto kern = ws.visits != nullptr ? (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, true>)
                                   : (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, false> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, false>);
   return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s);

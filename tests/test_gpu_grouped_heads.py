@@ -53,3 +53,25 @@ def test_groups_add_up(lens_q, lens_k, chunk, topk, causal, H, Hk, counts, D, dq
         for name, got, ref in (("dk", dk2, dk), ("dv", dv2, dv)):  # (every term of the sum was rounded to 16 bits, and so are partial sums)
             worst = (got.float() - ref.sum(2)).abs() - 2.0 ** -7 * ref.abs().sum(2)
             assert worst.max().item() < 1e-3, f"{name}: {worst.max().item()}"
+
+
+# rows of q and dout that 32-bit byte offsets do not reach (2^22 elements apart), in a walk over several heads: the bits of the packed tensors
+@pytest.mark.parametrize("D,dq_mode", [(128, 1), (96, 1), (64, 1), (64, 2)])
+def test_groups_of_rows_far_apart(D, dq_mode, monkeypatch):
+    L, H, chunk = 150, 4, 64
+    g = torch.Generator().manual_seed(D)
+    mk = lambda h: torch.randn((L, h, D), generator=g).to(torch.bfloat16).cuda()
+    q, k, v, dout, cu = mk(H), mk(1), mk(1), mk(H), torch.tensor([0, L], dtype=torch.int32).cuda()
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cu, cu, L, L, 2, chunk, causal=True)
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *pattern, cu, cu, None, None, None, L, L, 0.0, D ** -0.5, False, True, 0.0, False, 128, chunk, None)
+    lib = hip.load_library()
+    monkeypatch.setattr(hip, "load_library", lambda: _Library(lib, 1))
+
+    def far(t):
+        view = torch.empty((L, 1 << 22), dtype=t.dtype, device="cuda")[:, :H * D].view(L, H, D)
+        return view.copy_(t)
+
+    grads = lambda q, dout: hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, *pattern, cu, cu, None, L, L, 0.0, D ** -0.5,
+                                                False, True, 0.0, False, 128, chunk, _dq_mode=dq_mode)[:3]
+    for near, apart in zip(grads(q, dout), grads(far(q), far(dout))):
+        assert torch.equal(near, apart)
