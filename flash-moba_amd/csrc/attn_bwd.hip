@@ -1278,6 +1278,24 @@ __device__ __forceinline__ DqItem dq_decode_item(int id, int npairs, int nsb_max
   return w;
 }
 
+// A buffer of (almost) 2^32 bytes from a wave-uniform address on, and 16 bytes of it at a byte offset per lane plus a constant: zeros from offset
+// kRowBufferBytes on, without an access.
+constexpr uint32_t kRowBufferBytes = 0xfffff000u;
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __amdgpu_buffer_rsrc_t RowBuffer;
+__device__ __forceinline__ RowBuffer row_buffer(const uint16_t *p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(p), 0, (int)kRowBufferBytes, 0x00020000);
+}
+__device__ __forceinline__ Pack8 row_buffer_load16(RowBuffer b, uint32_t lane_bytes, int offset) {
+  const auto x = __builtin_amdgcn_raw_buffer_load_b128(b, (int)lane_bytes + offset, 0, 0);
+  return Pack8{{x[0], x[1], x[2], x[3]}};
+}
+#else
+typedef const uint16_t *RowBuffer;
+__device__ __forceinline__ RowBuffer row_buffer(const uint16_t *p) { return p; }
+__device__ __forceinline__ Pack8 row_buffer_load16(RowBuffer, uint32_t, int) { return Pack8{{0u, 0u, 0u, 0u}}; }
+#endif
+
 // RT: 32-row tiles per wave (with two, every K^T operand read from LDS feeds two MFMAs).  NW: waves.
 template <typename T, int HD, int RT, int NW>
 __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int row_mask, int nsb_max) {
@@ -1415,23 +1433,38 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
   for (int cb = 0; cb < ncols; cb += cols_per_batch) {
     const int nsteps = prepare_batch(cb, min(ncols, cb + cols_per_batch));
     if (nsteps == 0) continue;
+    // The records of 64 steps from step wbase on, one per lane: what a step of the walk needs of them comes into scalar registers by a
+    // lane read.  (Read from LDS where they are needed they were nine dependent LDS reads per group of two steps, and rows that are absent
+    // were fetched from a place that exists and cleared before the products, a vector instruction per register.  Training steps without and
+    // with the two: 65536 tokens in eight sequences 7393 -> 7311 us, 24571 tokens, 32 over 8 heads 2684 -> 2650, 12037 tokens, heads of 96
+    // 474 -> 469, 2 x 4096 tokens, 8 heads of 256 509 -> 504, 8191 tokens of short documents 128.0 -> 126.7.)
+    int4 rec = sInfo[min(lane, nsteps - 1)];
+    int wbase = 0;
+    struct Step {
+      int key0, n, kb;  // first key, rows of the run, the 64-key block's number inside its column
+      int64_t pos0;     // list position of the run
+    };
+    auto at = [&](int step) {
+      const int l = min(step, nsteps - 1) - wbase;
+      const int ny = __builtin_amdgcn_readlane(rec.y, l);
+      return Step{__builtin_amdgcn_readlane(rec.x, l), ny & 0xffff, ny >> 16,
+                  (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(rec.w, l) << 32) | (uint32_t)__builtin_amdgcn_readlane(rec.z, l))};
+    };
     auto row_id = [&](int step) {  // row of list position tid of the step (clamped)
-      const int4 info = sInfo[min(step, nsteps - 1)];
-      const int n = __builtin_amdgcn_readfirstlane(info.y) & 0xffff;
-      const int64_t pos0 = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane(info.z) | ((int64_t)__builtin_amdgcn_readfirstlane(info.w) << 32);
-      return a.row_indices[pos0 + min(tid & (ROWS - 1), n - 1)] & row_mask;
+      const Step st = at(step);
+      const uint32_t o = (uint32_t)min(tid & (ROWS - 1), st.n - 1) * 4u;
+      return *reinterpret_cast<const int32_t *>(reinterpret_cast<const uint8_t *>(a.row_indices + st.pos0) + o) & row_mask;
     };
     auto put_pos = [&](int step, int rr) {  // thread t tells row rr, the t-th of the step's run, where it is
       if (step < nsteps && tid < ROWS) {
-        const int4 info = sInfo[step];
-        const int key0 = info.x, n = info.y & 0xffff;
-        const int first_rel = causal ? key0 - off - m0 : -0x40000000;  // rows before it see no key of the block
+        const Step st = at(step);
+        const int first_rel = causal ? st.key0 - off - m0 : -0x40000000;  // rows before it see no key of the block
         const int rel = rr - m0;
-        if ((tid < n) & ((uint32_t)rel < (uint32_t)rows_sb) & (rel >= first_rel)) sPos[(step % NS) * ROWS + rel] = ((tag_base + step + 1) << 10) | tid;
+        if ((tid < st.n) & ((uint32_t)rel < (uint32_t)rows_sb) & (rel >= first_rel)) sPos[(step % NS) * ROWS + rel] = ((tag_base + step + 1) << 10) | tid;
       }
     };
     auto k_issue = [&](int step) {  // this wave's share of the K tile of `step`
-      const int key0 = __builtin_amdgcn_readfirstlane(sInfo[min(step, nsteps - 1)].x);
+      const int key0 = at(step).key0;
       const uint32_t dst = ldsK + (uint32_t)__builtin_amdgcn_readfirstlane(step % NS) * TB + (uint32_t)(wave * NKI) * 1024u;
       if (key0 + 64 <= Lk) {
         const uint16_t *kb0 = kp + (int64_t)key0 * a.k_row_stride;
@@ -1446,32 +1479,30 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
         }
       }
     };
-    // fetch this lane's dS rows of `step` into ring entry R (unconditional: an absent row reads a piece near its neighbours')
-    auto fetch = [&](auto rc, int step) {
-      constexpr int R = decltype(rc)::value;
-      const int sc_ = min(step, nsteps - 1);
-      // (all LDS reads first: one wait)
-      const int4 info = sInfo[sc_];
-      int v[RT];
+    // where this lane's rows are in the run of `step`
+    auto row_pos = [&](int step, int (&v)[RT]) {
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) v[rt] = sPos[(sc_ % NS) * ROWS + myrow[rt]];
-      const int ny = __builtin_amdgcn_readfirstlane(info.y);
-      const int n = ny & 0xffff, kb = ny >> 16;
-      const int64_t pos0 = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane(info.z) | ((int64_t)__builtin_amdgcn_readfirstlane(info.w) << 32);
+      for (int rt = 0; rt < RT; ++rt) v[rt] = sPos[(min(step, nsteps - 1) % NS) * ROWS + myrow[rt]];
+    };
+    // Fetch this lane's dS rows of `step` (v: row_pos) into ring entry R.  A row that is absent reads past the end of the buffer that the
+    // loads name, which gives zeros without an access: nothing to clear before the products.
+    auto fetch = [&](auto rc, int step, const int (&v)[RT]) {
+      constexpr int R = decltype(rc)::value;
+      const Step st = at(step);
+      const int tag = tag_base + min(step, nsteps - 1) + 1;
       // ds_piece_offset(pos0 + j, 8 kb + hh + 2 s4, Bn / 8) in two parts: what the step's run has in common (the tile of
       // its first position and the block's first piece: scalar arithmetic, 64 bits) and the lane's own part (at most
-      // 17 tiles further on: 32 bits, no wide multiply among the vector instructions)
-      const uint32_t kgs = (uint32_t)Bn >> 3, r0s = (uint32_t)pos0 & 31u;
-      const uint16_t *base = ds_ws + (((pos0 >> 5) * (int64_t)kgs + 8 * kb) << 8);
+      // 9 tiles further on: 32 bits, no wide multiply among the vector instructions)
+      const uint32_t kgs = (uint32_t)Bn >> 3, r0s = (uint32_t)st.pos0 & 31u;
+      const RowBuffer buf = row_buffer(ds_ws + (((st.pos0 >> 5) * (int64_t)kgs + 8 * st.kb) << 8));
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        const bool pres = (step < nsteps) & ((v[rt] >> 10) == tag_base + sc_ + 1);
-        const uint32_t j = pres ? (uint32_t)(v[rt] & 1023) : mul24_u32((uint32_t)myrow[rt], (uint32_t)n) / (uint32_t)ROWS;
-        const uint32_t t = r0s + j;
+        const bool pres = (step < nsteps) & ((v[rt] >> 10) == tag);
+        const uint32_t t = r0s + (uint32_t)(v[rt] & 1023);
         const uint32_t lane_bytes = ((mul24_u32(t >> 5, kgs) + (uint32_t)hh) << 9) + ((t & 31u) << 4);
-        const uint16_t *rp = reinterpret_cast<const uint16_t *>(reinterpret_cast<const uint8_t *>(base) + lane_bytes);
+        const uint32_t at_bytes = pres ? lane_bytes : kRowBufferBytes;
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) df[R][rt][s4] = ld_global16(rp + 512 * s4);
+        for (int s4 = 0; s4 < 4; ++s4) df[R][rt][s4] = row_buffer_load16(buf, at_bytes, 1024 * s4);
         dfp[R][rt] = pres;
       }
     };
@@ -1486,13 +1517,6 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
         between();
         return;
       }
-      Pack8 dz[RT][4];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4)
-#pragma unroll
-          for (int w = 0; w < 4; ++w) dz[rt][s4].w[w] = dfp[R][rt] ? df[R][rt][s4].w[w] : 0u;
       const uint32_t stage = ldsK + (uint32_t)__builtin_amdgcn_readfirstlane(step % NS) * TB;
       const uint32_t alo = tlo + stage, ahi = thi + stage;
       // K^T operands half a feature tile (two products per row tile) ahead of their use
@@ -1511,7 +1535,7 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
-          for (int rt = 0; rt < RT; ++rt) acc[rt][u >> 1] = mfma32<T>(kf[u & 1][s2], dz[rt][2 * (u & 1) + s2], acc[rt][u >> 1]);
+          for (int rt = 0; rt < RT; ++rt) acc[rt][u >> 1] = mfma32<T>(kf[u & 1][s2], df[R][rt][2 * (u & 1) + s2], acc[rt][u >> 1]);
         if (u == 0) between();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -1529,13 +1553,21 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
 #pragma unroll
     for (int g = 0; g < G; ++g) k_issue(g);
     __syncthreads();
-    fetch(std::integral_constant<int, 0>{}, 0);
+    {
+      int v[RT];
+      row_pos(0, v);
+      fetch(std::integral_constant<int, 0>{}, 0, v);
+    }
     wait_all_loads();
     // group of steps s0 .. s0 + G - 1: positions of steps s0 + G + 1 .. s0 + 2 G into LDS, row ids of the G steps after
     // those, then per step the dS rows of the next step and the products of this one; the K tile loads of the next
     // group are issued among the products of the group's first step
     const int nsteps_pad = (nsteps + G - 1) / G * G;
     for (int s0 = 0; s0 < nsteps_pad; s0 += G) {
+      if ((s0 & 31) == 0) {
+        wbase = s0;
+        rec = sInfo[min(s0 + lane, nsteps - 1)];
+      }
       __syncthreads();  // the K tiles of this group and the positions up to step s0 + G are in LDS; everyone is done with the group before
 #pragma unroll
       for (int g = 0; g < G; ++g) put_pos(s0 + G + 1 + g, rid[g]);
@@ -1544,7 +1576,9 @@ __global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bw
       static_for<G>([&](auto e) {
         constexpr int E = decltype(e)::value;
         const int s = s0 + E;
-        fetch(std::integral_constant<int, (E + 1) & 1>{}, s + 1);
+        int pos[RT];
+        row_pos(s + 1, pos);
+        fetch(std::integral_constant<int, (E + 1) & 1>{}, s + 1, pos);
         compute(std::integral_constant<int, E & 1>{}, s, [&]() {
           if constexpr (E == 0) {
 #pragma unroll

@@ -6,6 +6,7 @@ import torch
 import flash_moba
 from flash_moba import flash_moba_hip as hip
 from gpu_utils import assert_close
+from test_gpu_item_order import _reference
 
 pytestmark = pytest.mark.gpu
 
@@ -66,3 +67,19 @@ def test_places_between_a_columns_first_row_and_the_end(lens_q, lens_k, chunk, t
                                        128, chunk, None, _dq_mode=mode))
     for name, x, y in zip(("dq", "dk", "dv"), *res):  # (bounds as above)
         assert_close(name, x, y, 2e-2, 1e-2)
+
+
+# Walks of the dQ pass around 32 and 64 steps and past 64 (its records come 64 at a time, every 32 steps), of several batches of columns
+# (256 of them, 512 steps), with rows that are in few of the steps or, past the first 64, in none
+@pytest.mark.parametrize("L,chunk,topk", [(31 * 64, 64, 3), (32 * 64 + 1, 64, 3), (64 * 64, 64, 2), (65 * 64 + 7, 128, 1), (4200, 192, 2), (16700, 64, 2)])
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+def test_dq_over_long_walks(L, chunk, topk, D):
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    mk = lambda h: torch.randn((L, h, D), generator=g, device="cuda").to(torch.bfloat16)
+    q, k, v, dout, cu = mk(1), mk(1), mk(1), mk(1), torch.tensor([0, L], dtype=torch.int32, device="cuda")
+    csc = flash_moba.flash_topk_varlen_func(q, k, cu, cu, L, L, topk, chunk, causal=True)
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *csc, cu, cu, None, None, None, L, L, 0.0, D ** -0.5, False, True, 0.0, False, 128, chunk, None)
+    dq, dk, dv, _ = hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, *csc, cu, cu, None, L, L, 0.0, D ** -0.5, False, True, 0.0, False,
+                                        128, chunk, None, _dq_mode=1)
+    for name, x, y in zip(("dq", "dk", "dv"), (dq, dk, dv), _reference(q, k, v, dout, [0, L], *csc, chunk)[1:]):
+        assert_close(name, x, y, 2e-2, 1e-2)  # (the bounds of the other attention tests)
