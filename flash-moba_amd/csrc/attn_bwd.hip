@@ -138,18 +138,6 @@ struct DkdvSmem {
   static_assert(bytes <= 160 * 1024 && (size_t)64 * HD * 2 <= NBUF * tile, "LDS of one compute unit; K and V pass through the tiles");
 };
 
-// a * b of two values below 2^24, b the same in every lane: one full-rate instruction (a 32-bit multiply takes four
-// times as long)
-__device__ __forceinline__ uint32_t mul24_u32(uint32_t a, uint32_t b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t d;
-  asm("v_mul_u32_u24 %0, %1, %2" : "=v"(d) : "v"(a), "s"(b));
-  return d;
-#else
-  return a * b;
-#endif
-}
-
 // RANKED (partials form): part rows go to the place of the block among the row's, which the rank of the list entry gives
 // NEAR: a gathered row's place is a 32-bit byte offset from the sequence's first row that one 24-bit multiply makes (rows_near).
 template <typename T, int HD, bool DQP, bool RANKED, bool NEAR>
@@ -501,13 +489,9 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
         for (int u = 0; u < 2; ++u) x[u] = lds_read16(ldsdS + (uint32_t)(lane * PRB) + (((uint32_t)(2 * wave + u) ^ (uint32_t)(lane & 7)) * 16u));
         arrived();
         if (lane < w0.n) {
-          // ds_piece_offset(w0.pos + lane, koff / 8 + 2 wave, Bn / 8) in two parts: what the round has in common, and the lane's own
-          // (at most two tiles further on)
-          const uint32_t kgs = (uint32_t)Bn >> 3, t = ((uint32_t)w0.pos & 31u) + (uint32_t)lane;
-          uint16_t *base = ws.ds + (((w0.pos >> 5) * (int64_t)kgs + (koff >> 3) + 2 * wave) << 8);
-          uint8_t *dst = reinterpret_cast<uint8_t *>(base) + ((mul24_u32(t >> 5, kgs) << 9) + ((t & 31u) << 4));
+          uint16_t *dst = ds_piece(ws.ds, w0.pos, lane, (koff >> 3) + 2 * wave, Bn >> 3);
 #pragma unroll
-          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(dst + 512 * u) = x[u];
+          for (int u = 0; u < 2; ++u) *reinterpret_cast<Pack8 *>(dst + 256 * u) = x[u];
         }
         __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
       }
@@ -1800,12 +1784,6 @@ static int launch_dkdv_kernel(K kern, size_t smem, int heads, int keys, const fm
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws);
   return 0;
-}
-// Every row of a sequence's q and dout lies within 2^31 elements of the sequence's first row and is less than 2^24 rows
-// and 2^22 elements per row away, so a gathered row's place is a 32-bit offset made by one 24-bit multiply.
-static bool rows_near(const fmoba_attn_bwd_args &a) {
-  return a.max_seqlen_q < (1 << 24) && a.q_row_stride < (1 << 22) && a.do_row_stride < (1 << 22) &&
-         (int64_t)a.max_seqlen_q * a.q_row_stride < (int64_t)0x7fff0000 && (int64_t)a.max_seqlen_q * a.do_row_stride < (int64_t)0x7fff0000;
 }
 template <typename T, int HD, bool DQP>
 static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {

@@ -30,7 +30,8 @@ struct BwdWideSmem {
   static_assert(bytes <= 160 * 1024, "LDS of one compute unit");
 };
 
-template <typename T>
+// NEAR: as in attn_bwd_dkdv_kernel (attn_bwd.hip)
+template <typename T, bool NEAR>
 __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws, int row_mask) {
   typedef BwdWideSmem SM;
   constexpr int HD = SM::HD, KS = HD / 16, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR;
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
     }
   }
   int start = 0;
-  if (causal && nnz > 0 && Bn > 64) start = lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off, row_mask);  // earlier rows see no key of the block
+  if (causal && nnz > 0 && Bn > 64) start = __builtin_amdgcn_readfirstlane(lower_bound_wave_i32(a.row_indices + lbase, nnz, key0 - off, row_mask));  // earlier rows see no key of the block
   const int32_t *list = a.row_indices + lbase + start;
   const int n = nnz - start;
   const int nround = (n + 63) >> 6;
@@ -113,19 +114,28 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
   __syncthreads();
   if (nround > 0) {
     auto code = [&](int raw, int r) { return tile_row_code(raw & row_mask, r * 64 + myrow < n, Lq); };
-    auto feed = [&](int rid, uint32_t buf) {  // eight rows per wave, of its own 32
+    uint32_t fsrc[4];  // the rows this lane fetches pieces of: eight per wave, of its own 32
+    auto feed_rows = [&](int rid) {  // (all exchanges at once: one wait for them)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int tr = (wave >> 1) * 8 + i * RPI + rl;
-        const uint32_t src = (uint32_t)__shfl(rid, tr, 64) & 0x7fffffffu;
-        const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
-        const uint32_t dst = buf + (uint32_t)((rt * 32 + (wave >> 1) * 8 + i * RPI) * RB);
+      for (int i = 0; i < 4; ++i) fsrc[i] = (uint32_t)__shfl(rid, (wave >> 1) * 8 + i * RPI + rl, 64);
+    };
+    auto feed = [&](auto ic, uint32_t buf) {  // load ic of Q and of dO
+      constexpr int I = decltype(ic)::value;
+      const int tr = (wave >> 1) * 8 + I * RPI + rl;
+      const uint32_t src = fsrc[I] & 0x7fffffffu;
+      const uint32_t e = (uint32_t)min((pc ^ tile_swz<HD>(tr)) * 8, D - 8);
+      const uint32_t dst = buf + (uint32_t)((rt * 32 + (wave >> 1) * 8 + I * RPI) * RB);
+      if constexpr (NEAR) {
+        global_to_lds16_sbase(mul24_u32(src, (uint32_t)a.q_row_stride * 2u) + e * 2u, qg, ldsQ + dst);
+        global_to_lds16_sbase(mul24_u32(src, (uint32_t)a.do_row_stride * 2u) + e * 2u, dog, ldsdO + dst);
+      } else {
         global_to_lds16(qg + ((uint64_t)src * (uint32_t)a.q_row_stride + e), ldsQ + dst);
         global_to_lds16(dog + ((uint64_t)src * (uint32_t)a.do_row_stride + e), ldsdO + dst);
       }
     };
     int rid = code(rid_nx, 0);
-    feed(rid, 0);
+    feed_rows(rid);
+    static_for<4>([&](auto ic) { feed(ic, 0u); });
     float scl = sclg[rid & 0x7fffffff];
     rid_nx = list[min(64 + myrow, n - 1)];
     auto arrived = [&]() {
@@ -143,7 +153,8 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
       const int rcur = rid;
       const float x0 = is_s ? (rcur >= 0 ? scl * kLog2e : INFINITY) : scl;
       rid = code(rid_nx, r + 1);
-      if (r + 1 < nround) feed(rid, buf ^ TILE);
+      // (the rows by 32-bit offsets and between the products, as in attn_bwd_dkdv_kernel: 2 x 4096 tokens, 8 heads of 256, training step 506 -> 487 us)
+      feed_rows(rid);
       scl = sclg[rid & 0x7fffffff];
       rid_nx = list[min((r + 2) * 64 + myrow, n - 1)];
       // S^T or dP^T: lane -> row, register i -> key 32 kq + acc_row(i, hh)
@@ -165,6 +176,8 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < NB; ++u) s = mfma32<T>(kf[B * NB + u], qf[B & 1][u], s);
+        static_assert(KS / NB == 4, "a load of Q and one of dO after every batch of products");
+        if (r + 1 < nround) feed(bc, buf ^ TILE);
         __builtin_amdgcn_sched_barrier(0);
       });
       const uint32_t at = pw + ((uint32_t)(kq * 4) ^ psw) * 16u;
@@ -222,12 +235,11 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
           for (int kk = 0; kk < 2; ++kk) acc[d][kk] = mfma32<T>(xa[S4 & 1][d], pb[S4 & 1][kk], acc[d][kk]);
         __builtin_amdgcn_sched_barrier(0);
       });
-      arrived();
       // dS of row `lane`, key group `wave`: consecutive lanes write consecutive pieces of the dS tile
       {
-        const int p = r * 64 + lane;
         const Pack8 x = lds_read16(ldsdS + (uint32_t)(lane * 128) + (((uint32_t)wave ^ (uint32_t)(lane & 7)) * 16u));
-        if (p < n) *reinterpret_cast<Pack8 *>(ds_ws + ds_piece_offset(lbase + start + p, (koff >> 3) + wave, Bn >> 3)) = x;
+        arrived();
+        if (r * 64 + lane < n) *reinterpret_cast<Pack8 *>(ds_piece(ds_ws, lbase + start + r * 64, lane, (koff >> 3) + wave, Bn >> 3)) = x;
       }
       __syncthreads();  // the next round's rows are in LDS, this one's are no longer read
     }
@@ -263,7 +275,7 @@ __global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_b
 
 template <typename T>
 static int launch_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, int row_mask, hipStream_t s) {
-  auto kern = attn_bwd_dkdv_wide_kernel<T>;
+  auto kern = rows_near(a) ? attn_bwd_dkdv_wide_kernel<T, true> : attn_bwd_dkdv_wide_kernel<T, false>;
   const size_t smem = BwdWideSmem::bytes;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);

@@ -772,6 +772,17 @@ __device__ __forceinline__ void global_to_lds16_sbase(uint32_t lane_byte_off, co
   (void)lane_byte_off, (void)uniform_base, (void)lds_base;
 #endif
 }
+// a * b of two values below 2^24, b the same in every lane: one full-rate instruction (a 32-bit multiply takes four
+// times as long)
+__device__ __forceinline__ uint32_t mul24_u32(uint32_t a, uint32_t b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t d;
+  asm("v_mul_u32_u24 %0, %1, %2" : "=v"(d) : "v"(a), "s"(b));
+  return d;
+#else
+  return a * b;
+#endif
+}
 // 64 lanes x 4 bytes to LDS bytes [lds_base, lds_base + 256), in the same way.  For a value that other loads are issued behind and that is wanted
 // before them: in a register it would be one that the compiler may copy or spill before it has arrived.
 __device__ __forceinline__ void global_to_lds4(const void *g, uint32_t lds_base) {
@@ -799,6 +810,13 @@ __device__ __forceinline__ void wait_all_loads() {
 // brings a run of positions into LDS one contiguous kilobyte (two key groups of a tile) per load instruction.
 // Returns the element offset of piece (position p, key group kg); kgs = key groups per entry (column width / 8).
 __host__ __device__ __forceinline__ int64_t ds_piece_offset(int64_t p, int kg, int kgs) { return ((((p >> 5) * kgs + kg) << 5) + (p & 31)) << 3; }
+// The same place in two parts: what the lanes have in common (position p0, 64-bit scalar arithmetic) and the lane's own (position p0 + j,
+// 0 <= j < 64: at most two tiles further on, 32 bits).
+__device__ __forceinline__ uint16_t *ds_piece(uint16_t *ds, int64_t p0, int j, int kg, int kgs) {
+  const uint32_t t = ((uint32_t)p0 & 31u) + (uint32_t)j;
+  uint16_t *base = ds + (((p0 >> 5) * (int64_t)kgs + kg) << 8);
+  return reinterpret_cast<uint16_t *>(reinterpret_cast<uint8_t *>(base) + ((mul24_u32(t >> 5, (uint32_t)kgs) << 9) + ((t & 31u) << 4)));
+}
 static inline size_t ds_workspace_tiles(int64_t positions) { return (size_t)((positions > 0 ? positions : 0) + 31) / 32 + 1; }
 
 // *p += 1 where `mine`; the old value there, 0 in the other lanes.  (An ordinary branch: the compiler leaves the result where the atomic
@@ -819,5 +837,11 @@ __device__ __forceinline__ int tile_row_code(int r, bool present, int rows) {
   return (present & exists) ? src : (int)((uint32_t)src | 0x80000000u);
 }
 
+// Every row of a sequence's q and dout lies within 2^31 elements of the sequence's first row and is less than 2^24 rows
+// and 2^22 elements per row away, so a gathered row's place is a 32-bit offset made by one 24-bit multiply.
+static inline bool rows_near(const fmoba_attn_bwd_args &a) {
+  return a.max_seqlen_q < (1 << 24) && a.q_row_stride < (1 << 22) && a.do_row_stride < (1 << 22) &&
+         (int64_t)a.max_seqlen_q * a.q_row_stride < (int64_t)0x7fff0000 && (int64_t)a.max_seqlen_q * a.do_row_stride < (int64_t)0x7fff0000;
+}
 
 }  // namespace fmoba

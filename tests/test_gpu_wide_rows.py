@@ -102,3 +102,19 @@ def test_wide_row_blocks_are_as_precise_as_columns(chunk, topk, dtype):
     want = _reference(q, k, v, torch.zeros_like(q), cu, *pattern, chunk)[0]
     err = [float((_forward(q, k, v, cud, lens, pattern, chunk, m)[0].float() - want).norm()) for m in (2, 1)]
     assert err[0] <= err[1] * 1.01
+
+
+# rows of q and dout that 32-bit byte offsets do not reach (2^22 elements apart): the bits of the packed tensors
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,chunk", [(256, 64), (192, 128)])
+def test_wide_backward_with_rows_far_apart(D, chunk):
+    lens = [150, 70]
+    q, k, v, _, cu = _inputs(lens, 2, 2, D, torch.bfloat16, D)
+    dout = _inputs(lens, 2, 2, D, torch.bfloat16, D + 1)[0]
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cu, cu, 150, 150, 2, chunk, causal=True)
+    out, lse = _forward(q, k, v, cu, lens, pattern, chunk, 0)
+    far = lambda t: torch.empty((220, 1 << 22), dtype=t.dtype, device="cuda")[:, :2 * D].view(220, 2, D).copy_(t)
+    grads = lambda q, dout: hip.moba_varlen_bwd(dout, q, k, v, out, lse, None, None, None, *pattern, cu, cu, None, 150, 150, 0.0, D ** -0.5, False, True, 0.0,
+                                                False, 128, chunk, None)[:3]
+    for near, apart in zip(grads(q, dout), grads(far(q), far(dout))):
+        assert torch.equal(near, apart)
