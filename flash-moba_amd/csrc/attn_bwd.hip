@@ -882,7 +882,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
     // -inf elsewhere (the products then leave -inf there and the exponential gives 0), and only in rounds that have
     // such pairs at all (`masked`, the same for the whole wave): the rows of a list come in ascending order, so
     // from the first row that sees every key of the block on, S starts from nothing and no comparison is made.
-    auto mm_a = [&](auto pc, auto pp, auto tsc, auto gc, bool masked, auto &&after_step) {
+    auto mm_a = [&](auto pc, auto pp, auto tsc, auto gc, bool masked, auto &&after_step, auto &&after_product) {
       constexpr int TS = decltype(tsc)::value, G = decltype(gc)::value;
       static_for<KC>([&](auto tc) {
         constexpr int t = decltype(tc)::value;
@@ -902,12 +902,15 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
           } else {
             mfma32_b_acc<T, true>(s[TS], qa[G & 1][t], kb[G * KC + t]);
           }
+          after_product(std::integral_constant<int, 2 * t>{});
           mfma32_b_acc<T, true>(dp[TS], doa[G & 1][t], vb[G * KC + t]);
         } else {
           mfma32_b_acc<T, false>(s[TS], qa[G & 1][t], kb[G * KC + t]);
+          after_product(std::integral_constant<int, 2 * t>{});
           mfma32_b_acc<T, false>(dp[TS], doa[G & 1][t], vb[G * KC + t]);
         }
         after_step(std::integral_constant<int, G * KC + t>{});
+        after_product(std::integral_constant<int, 2 * t + 1>{});
       });
       if constexpr (G == 3) mfma_results_ready(s[TS], dp[TS]);
     };
@@ -925,20 +928,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
         qt[G & 1][t] = lds_tr8((tQ ^ xlo) + olo, (tQ ^ xhi) + ohi);
       }
     };
-    auto mm_b = [&](auto tsc, auto gc) {
+    auto mm_b = [&](auto tsc, auto gc, auto &&after_product) {
       constexpr int TS = decltype(tsc)::value, G = decltype(gc)::value;
       // dV^T[d][key] += dO^T[d][row] P[row][key];  dK^T[d][key] += Q^T[d][row] dS[row][key]
-#pragma unroll
-      for (int t = 0; t < BC; ++t) {
-        const int pi = G * BC + t, dt = pi >> 1, s2 = pi & 1;
-        static_for<NDT>([&](auto dc) {
-          constexpr int DT = decltype(dc)::value;
-          if (DT == dt) {
-            mfma32_c_acc<T, 2 * DT>(dv[DT], dot[G & 1][t], pf[TS][s2]);
-            mfma32_c_acc<T, 2 * DT + 1>(dk[DT], qt[G & 1][t], dsf[TS][s2]);
-          }
-        });
-      }
+      static_for<BC>([&](auto tc) {
+        constexpr int t = decltype(tc)::value, pi = G * BC + t, DT = pi >> 1, s2 = pi & 1;
+        mfma32_c_acc<T, 2 * DT>(dv[DT], dot[G & 1][t], pf[TS][s2]);
+        after_product(std::integral_constant<int, 2 * t>{});
+        mfma32_c_acc<T, 2 * DT + 1>(dk[DT], qt[G & 1][t], dsf[TS][s2]);
+        after_product(std::integral_constant<int, 2 * t + 1>{});
+      });
     };
     auto ld_s = [&](auto pc, auto pp, auto tsc, auto gc) {
       constexpr int TS = decltype(pc)::value * 4 + decltype(pp)::value * 2 + decltype(tsc)::value, G = decltype(gc)::value;
@@ -949,21 +948,26 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
       lse4[G & 1] = lds_read_vec<f32x4>(smx0 + O + (uint32_t)(SM::oLse - SM::oRow));
       del4[G & 1] = lds_read_vec<f32x4>(smx0 + O + (uint32_t)(SM::oDelta - SM::oRow));
     };
-    auto smx = [&](auto tsc, auto gc) {
-      constexpr int TS = decltype(tsc)::value, G = decltype(gc)::value;
-      float pr[4], ds[4];
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int i = 4 * G + jj;
-        const float x = fmaf(s[TS][i], scale_log2, -lse4[G & 1][jj]);  // (-inf for a masked pair, see mm_a)
-        pr[jj] = __builtin_amdgcn_exp2f(x);
-        ds[jj] = pr[jj] * (dp[TS][i] - del4[G & 1][jj]);
-      }
+    // The softmax of a chunk's four rows in four parts, one behind each of the chunk's four products: a wave issues in order, so what is to
+    // run under a product has to stand right behind it.
+    static_assert(KC == 2 && BC == 2, "four products per chunk");
+    float pr[4], ds[4];
+    auto smx = [&](auto tsc, auto gc, auto ic) {
+      constexpr int TS = decltype(tsc)::value, G = decltype(gc)::value, I = decltype(ic)::value;
+      pr[I] = __builtin_amdgcn_exp2f(fmaf(s[TS][4 * G + I], scale_log2, -lse4[G & 1][I]));  // (-inf for a masked pair, see mm_a)
+      auto grad = [&](int jj) { ds[jj] = pr[jj] * (dp[TS][4 * G + jj] - del4[G & 1][jj]); };
       // operand register s2 = G/2 holds rows 16*s2 + 8*(w/2) + 4*hh + ..: words 2*(G%2), 2*(G%2)+1
-      pf[TS][G >> 1].w[2 * (G & 1)] = pack2<T>(pr[0], pr[1]);
-      pf[TS][G >> 1].w[2 * (G & 1) + 1] = pack2<T>(pr[2], pr[3]);
-      dsf[TS][G >> 1].w[2 * (G & 1)] = pack2<T>(ds[0], ds[1]);
-      dsf[TS][G >> 1].w[2 * (G & 1) + 1] = pack2<T>(ds[2], ds[3]);
+      auto pack = [&](int w) {
+        pf[TS][G >> 1].w[2 * (G & 1) + w] = pack2<T>(pr[2 * w], pr[2 * w + 1]);
+        dsf[TS][G >> 1].w[2 * (G & 1) + w] = pack2<T>(ds[2 * w], ds[2 * w + 1]);
+      };
+      if constexpr (I > 0) grad(I - 1);
+      if constexpr (I == 2) pack(0);
+      if constexpr (I == 3) {
+        grad(3);
+        pack(1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     };
     // dQ of the tile: both waves of a pair put dS^T of their 32 keys into one LDS tile [64 keys][32 rows]; after a
     // barrier each wave computes dQ^T = K^T dS^T over all 64 keys for ITS half of the features.  The
@@ -1058,7 +1062,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
         }
         mm_a(pc, pp, C0{}, gc, masked, [&](auto ic) {
           if constexpr (kSpreadLoads && decltype(pp)::value == 0) tile_issue_q(ic);
-        });
+        }, [](auto) {});
         fence();
       });
       // S, dP of the second tile between the softmax rows of the first
@@ -1073,8 +1077,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
         }
         mm_a(pc, pp, C1{}, gc, masked, [&](auto ic) {
           if constexpr (kSpreadLoads && decltype(pp)::value == 0) tile_issue_do(ic);
-        });
-        smx(C0{}, gc);
+        }, [&](auto ic) { smx(C0{}, gc, ic); });
         fence();
       });
       // dV, dK of the first tile between the softmax rows of the second
@@ -1090,8 +1093,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
         } else {
           ld_b(pc, pp, C1{}, C0{});
         }
-        mm_b(C0{}, gc);
-        smx(C1{}, gc);
+        mm_b(C0{}, gc, [&](auto ic) { smx(C1{}, gc, ic); });
         fence();
       });
       // dV, dK of the second tile; dQ of the first one runs between them: by now all key
@@ -1103,7 +1105,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
       static_for<4>([&](auto gc) {
         constexpr int G = decltype(gc)::value;
         if constexpr (G < 3) ld_b(pc, pp, C1{}, std::integral_constant<int, G + 1>{});
-        mm_b(C1{}, gc);
+        mm_b(C1{}, gc, [](auto) {});
         dq_mma(gc);
         fence();
       });
