@@ -556,6 +556,65 @@ __global__ __launch_bounds__(256) void csc_row_visits_kernel(fmoba_attn_fwd_args
     if (r >= 0 && r < Lq) atomicAdd(&cnt[(int64_t)(q0 + r) * a.heads + h], nblk);
   }
 }
+// The same with the counts of a range of rows of one (sequence, head) in LDS: no atomics in memory, the maximum on the way out.  Every workgroup
+// reads all lists of the pair (in any order) and counts what falls into its rows; a wave takes 512 entries of two lists at a time.
+// grid (row ranges, heads, batch); `range` rows in LDS, `max_out` cleared before.
+__global__ __launch_bounds__(1024) void csc_row_visits_lds_kernel(fmoba_attn_fwd_args a, int32_t *cnt, int32_t *max_out, int kb, int range) {
+  extern __shared__ int32_t visits[];
+  constexpr int kCols = 512;
+  __shared__ int64_t first[kCols];
+  __shared__ int32_t len[kCols], blocks[kCols];
+  const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+  const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b];
+  const int64_t bh = (int64_t)b * a.heads + h;
+  const int ncols = min(a.max_cols, (Lk + a.lg_block_n - 1) / a.lg_block_n);
+  for (int r0 = blockIdx.x * range; r0 < Lq; r0 += gridDim.x * range) {
+    const int rows = min(range, Lq - r0);
+    for (int i = tid; i < rows; i += blockDim.x) visits[i] = 0;
+    for (int c0 = 0; c0 < ncols; c0 += kCols) {
+      const int nc = min(kCols, ncols - c0);
+      __syncthreads();
+      for (int i = tid; i < nc; i += blockDim.x) {
+        const int key_lo = (c0 + i) * a.lg_block_n, key_hi = min(Lk, key_lo + a.lg_block_n);
+        first[i] = a.col_offsets[bh * a.max_cols + c0 + i];
+        len[i] = a.col_nnz[bh * a.max_cols + c0 + i];
+        blocks[i] = (key_hi - key_lo + kb - 1) / kb;  // key blocks of the column that exist in the sequence
+      }
+      __syncthreads();
+      for (int c = 2 * wave; c < nc; c += 2 * waves) {
+        const bool two = c + 1 < nc;
+        const int32_t *list[2] = {a.row_indices + first[c], a.row_indices + first[two ? c + 1 : c]};
+        const int n[2] = {len[c], two ? len[c + 1] : 0};
+        for (int p = 0; p < max(n[0], n[1]); p += 512) {
+          int r[2][8];
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) r[u][i] = p + i * 64 + lane < n[u] ? list[u][p + i * 64 + lane] - r0 : -1;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int add = blocks[u && two ? c + 1 : c];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              if ((uint32_t)r[u][i] < (uint32_t)rows) atomicAdd(&visits[r[u][i]], add);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    int m = 0;
+    for (int i = tid; i < rows; i += blockDim.x) {
+      const int v = visits[i];
+      cnt[(int64_t)(q0 + r0 + i) * a.heads + h] = v;
+      m = max(m, v);
+    }
+    for (int o = 32; o >= 1; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+    if (lane == 0 && m > 0) atomicMax(max_out, m);
+    __syncthreads();  // (the next range takes the places)
+  }
+}
 __global__ __launch_bounds__(256) void max_i32_kernel(const int32_t *p, int64_t n, int32_t *out) {
   int m = 0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) m = max(m, p[i]);
@@ -720,8 +779,22 @@ extern "C" int fmoba_csc_max_row_visits(const fmoba_attn_fwd_args *a, int32_t *c
   hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(1), dim3(64), 0, s, max_out, (int64_t)1);
   if (rows > 0 && a->max_cols > 0 && a->total_k > 0) {
     FMOBA_REQUIRE(a->col_offsets && a->col_nnz && a->row_indices, "csc_max_row_visits: null CSC pointer");
-    hipLaunchKernelGGL(csc_row_visits_kernel, dim3(a->max_cols, a->heads, a->batch), dim3(256), 0, s, *a, counts, fwd_key_block(a->lg_block_n));
-    hipLaunchKernelGGL(max_i32_kernel, dim3(256), dim3(256), 0, s, counts, rows, max_out);
+    // Counts in LDS from eight (sequence, head) pairs on: a workgroup reads all lists of its pair, at about a quarter of the rate at which the
+    // whole chip does atomics in memory, so few pairs are better counted there (32768 tokens, one head, top-k 16 of 128-key chunks 25 us,
+    // 90 in LDS; 8 heads, 8192 tokens 28 and 26; 54437 tokens, 32 heads, top-k 27 of 64-key chunks 1715 and 332; 262144 tokens, 16 heads 2527
+    // and 1911).  Row ranges: enough of them for a workgroup per compute unit, 1024 to 32768 rows.
+    const int64_t pairs = (int64_t)a->batch * a->heads;
+    const int per = ceil_div(a->max_seqlen_q, (int)std::max<int64_t>(1, 256 / pairs));
+    const int range = std::min(32768, std::max(1024, (per + 255) & ~255)), nrange = std::max(1, ceil_div(a->max_seqlen_q, range));
+    const size_t smem = (size_t)range * 4;
+    auto kern = csc_row_visits_lds_kernel;
+    if (pairs >= 8 &&
+        (smem <= 32 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess)) {
+      hipLaunchKernelGGL(kern, dim3(nrange, a->heads, a->batch), dim3(1024), smem, s, *a, counts, max_out, fwd_key_block(a->lg_block_n), range);
+    } else {
+      hipLaunchKernelGGL(csc_row_visits_kernel, dim3(a->max_cols, a->heads, a->batch), dim3(256), 0, s, *a, counts, fwd_key_block(a->lg_block_n));
+      hipLaunchKernelGGL(max_i32_kernel, dim3(256), dim3(256), 0, s, counts, rows, max_out);
+    }
   }
   FMOBA_LAUNCH_CHECK("csc_max_row_visits");
   return 0;
