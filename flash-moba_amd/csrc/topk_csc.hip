@@ -463,421 +463,13 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
 }
 
 // ------------------------------------------------------------------------------------
-// The same gate for sequences with more key chunks than one register tile set holds
-// (NT*32).  Chunks are scored in groups of NT*32; after every group the row keeps the
-// K' best (score, chunk) pairs seen so far in LDS, and the next group competes against
-// them.  The total order (score descending, chunk index descending) is strict, so the
-// running winners after the last group are exactly the global top-K'.  Selection words
-// and counts are then assembled in LDS and written out like the small kernel's.
-// ------------------------------------------------------------------------------------
-constexpr int kBigCap = 32;   // running winners per row (K' = scored chunks kept) of the common variants
-constexpr int kBigCapMax = 64;  // ... of the variant for top-k above 33: moba_topk goes up to 64 at any sequence length
-
-// CAP: entries of a row's list of running winners (16, kBigCap or kBigCapMax).  With 16 and groups of 128 chunks the
-// kernel needs half the LDS and fewer registers, and two workgroups share a compute unit.  With 64 a row has ONE list
-// (two would not fit the LDS): every group then takes the general path, which has read the whole list into registers
-// before it writes the winners back; the streaming update of the smaller variants needs the second list for its entrants.
-template <typename T, int HD, int NT, int CAP>
-__global__ __launch_bounds__(256, CAP < kBigCap ? 2 : 1) void topk_gate_big_kernel(TopkParams p) {
-  constexpr bool TWO_LISTS = CAP <= kBigCap;
-  constexpr int NLIST = TWO_LISTS ? 2 : 1;
-  constexpr int KS = HD / 16;
-  constexpr int LD = HD + 16;
-  constexpr int GC = NT * 32;        // chunks per group
-  constexpr int PL = CAP / 2;    // previous winners held per lane (two lanes per row)
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  uint16_t *sKm = reinterpret_cast<uint16_t *>(smem);
-  uint32_t *sSel = reinterpret_cast<uint32_t *>(smem);  // [word columns of a pass][128], reuses the chunk-mean tile after the last group
-  float *sVal = reinterpret_cast<float *>(smem + (size_t)GC * LD * 2);   // [NLIST][128][CAP]
-  int *sIdx = reinterpret_cast<int *>(sVal + NLIST * kGateRows * CAP);   // [NLIST][128][CAP]
-  int *sCnt = sIdx + NLIST * kGateRows * CAP;                            // [2][128]
-  int *sHist = sCnt + 2 * kGateRows;                                     // [32 chunks per word column the tile holds as selection words]
-  int *sTrash = sHist + (size_t)GC * LD * 2 / (kGateRows * 4) * 32;      // [256]: takes the stores of lanes that have nothing to store
-
-  const fmoba_fused_topk_args &a = p.a;
-  const GateItem item = gate_item(p);
-  const int mb = item.mb, h = item.h, b = blockIdx.z;
-  const int q0 = a.cu_seqlens_q[b];
-  const int Lq = a.cu_seqlens_q[b + 1] - q0;
-  const int m0 = mb * kGateRows;
-  if (m0 >= Lq) return;
-  const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b];
-  const int km0 = a.cu_seqlens_km[b];
-  const int Cb = min(a.cu_seqlens_km[b + 1] - km0, p.max_cols);
-  const int off = Lk - Lq;
-  const int B = a.chunk;
-  const int D = a.head_dim;
-  const int hk = h / (a.heads / a.heads_k);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hh = lane >> 5;
-  const int rs = wave * 32 + (lane & 31);  // row slot inside the block
-
-  int nsc;  // chunks [0, nsc) can be candidates of some row of this block
-  if (a.is_causal) {
-    const int rmax = min(m0 + kGateRows - 1, Lq - 1) + off;
-    nsc = rmax < 0 ? 0 : min(Cb, rmax / B);
-  } else {
-    nsc = Cb;
-  }
-  const int ngroups = (nsc + GC - 1) / GC;
-
-  const int r = m0 + rs;
-  const bool valid = r < Lq;
-  Pack8 qf[KS];
-  {
-    const uint16_t *qp = reinterpret_cast<const uint16_t *>(a.q) + (int64_t)(q0 + (valid ? r : 0)) * a.q_row_stride + (int64_t)h * a.q_head_stride;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int e = (hh * KS + ks) * 8;
-      qf[ks] = (valid && e < D) ? ld_global16(qp + e) : zero_pack8();
-    }
-  }
-  const int rp = r + off;
-  int nc;  // candidate chunks of this row: chunks strictly before its own chunk
-  if (a.is_causal)
-    nc = (valid && rp >= 0) ? min(rp / B, Cb) : 0;
-  else
-    nc = valid ? Cb : 0;
-  const int kp = a.is_causal ? a.topk - 1 : a.topk;
-
-  if (tid < 2 * kGateRows) sCnt[tid] = 0;
-  int cur = 0;
-  const uint16_t *kmp = reinterpret_cast<const uint16_t *>(a.km) + (int64_t)hk * a.km_head_stride;
-#pragma nounroll
-  for (int g = 0; g < ngroups; ++g) {
-    const int c0 = g * GC;
-    const int gsc = min(GC, nsc - c0);
-    const int n_tiles = (gsc + 31) >> 5;
-    __syncthreads();  // the previous group's tile and lists are no longer read
-    {
-      const int vecs = HD / 8;
-      for (int v = tid; v < n_tiles * 32 * vecs; v += 256) {
-        const int c = v / vecs, e = (v - c * vecs) * 8;
-        Pack8 x = zero_pack8();
-        if (c < gsc && e < D) x = ld_global16(kmp + (int64_t)(km0 + c0 + c) * a.km_row_stride + e);
-        *reinterpret_cast<Pack8 *>(sKm + c * LD + e) = x;
-      }
-    }
-    const int nxt = cur ^ 1;
-    if (hh == 0) sCnt[nxt * kGateRows + rs] = 0;
-    __syncthreads();
-
-    // this group's scores and the winners so far
-    float sc[NT][16];
-    float pv[PL];
-    int pi[PL];
-    const int m_prev = sCnt[cur * kGateRows + rs];
-    float vmin = INFINITY, vmax = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < PL; ++j) {
-      const int e = 2 * j + hh;  // the two lanes of a row hold alternate entries of its list
-      const bool ok = e < m_prev;
-      pv[j] = ok ? sVal[((TWO_LISTS ? cur : 0) * kGateRows + rs) * CAP + e] : -INFINITY;
-      pi[j] = ok ? sIdx[((TWO_LISTS ? cur : 0) * kGateRows + rs) * CAP + e] : -1;
-      vmin = fminf(vmin, ok ? pv[j] : INFINITY);
-      vmax = fmaxf(vmax, pv[j]);
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (t < n_tiles) {
-        f32x16 acc;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const Pack8 af = *reinterpret_cast<const Pack8 *>(sKm + (t * 32 + (lane & 31)) * LD + (hh * KS + ks) * 8);
-          acc = mfma32<T>(af, qf[ks], acc);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int c = c0 + t * 32 + acc_row(i, hh);
-          const bool cand = c < nc;
-          const float x = acc[i];
-          sc[t][i] = cand ? x : -INFINITY;
-          vmin = fminf(vmin, cand ? x : INFINITY);
-          vmax = fmaxf(vmax, sc[t][i]);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sc[t][i] = -INFINITY;
-      }
-    }
-    // ---- later groups: streaming update ---------------------------------------------------------
-    // A row that still has candidates in this group had at least GC of them in the first one, so it already holds
-    // kp winners.  Only the new scores that reach its weakest winner can enter (a new chunk has a higher index than
-    // every earlier one, so an equal score wins the tie): they are put into the row's other list, then each takes
-    // the place of the weakest winner if it beats it.  That is the top kp of the union, in the same total order
-    // (score descending, chunk descending) as the bisection below, which stays for the first group and for rows
-    // with more entrants than a list holds.
-    if (TWO_LISTS && g > 0 && __all(m_prev == kp || nc <= c0)) {
-      float pmin = INFINITY;
-#pragma unroll
-      for (int j = 0; j < PL; ++j) pmin = fminf(pmin, pi[j] >= 0 ? pv[j] : INFINITY);
-      pmin = min_xor32_f(pmin);
-      int ne = 0;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) ne += (sc[t][i] >= pmin) ? 1 : 0;
-        }
-      int slot = 0;
-      if (ne > 0) slot = atomicAdd(&sCnt[nxt * kGateRows + rs], ne);
-      wave_lds_fence();
-      const int ne_row = sCnt[nxt * kGateRows + rs];
-      wave_lds_fence();
-      if (__all(ne_row <= CAP)) {
-        float *ev = sVal + (size_t)(nxt * kGateRows + rs) * CAP;
-        int *ei = sIdx + (size_t)(nxt * kGateRows + rs) * CAP;
-        // (no branches: a lane without an entrant at this position stores to its trash word)
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          if (t < n_tiles) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const bool w = sc[t][i] >= pmin;
-              *(w ? ev + slot : reinterpret_cast<float *>(sTrash + tid)) = sc[t][i];
-              *(w ? ei + slot : sTrash + tid) = c0 + t * 32 + acc_row(i, hh);
-              slot += w ? 1 : 0;
-            }
-          }
-        wave_lds_fence();
-        // (with at most 16 winners a lane holds at most 8 of them: the short variant of the loop)
-        auto stream = [&](auto plc) {
-          constexpr int PLX = decltype(plc)::value;
-#pragma nounroll
-          for (int e = 0; __any(e < ne_row); ++e) {
-            const bool has = e < ne_row;
-            const float x = has ? ev[e] : -INFINITY;
-            const int c = has ? ei[e] : -1;
-            // the weakest winner of this lane's half of the list, then of the row
-            float vw = INFINITY;
-            int cw = 0x7fffffff, jw = -1;
-#pragma unroll
-            for (int j = 0; j < PLX; ++j) {
-              const bool better = (pi[j] >= 0) & ((pv[j] < vw) | ((pv[j] == vw) & (pi[j] < cw)));
-              vw = better ? pv[j] : vw;
-              cw = better ? pi[j] : cw;
-              jw = better ? j : jw;
-            }
-            const float vo = shfl_xor32_f(vw);
-            const int co = shfl_xor32_i(cw);
-            const bool mine = (jw >= 0) & ((vw < vo) | ((vw == vo) & (cw < co)));
-            const float vr = mine ? vw : vo;
-            const int cr = mine ? cw : co;
-            const bool beats = has & ((x > vr) | ((x == vr) & (c > cr)));
-            const int jr = (beats & mine) ? jw : -1;
-#pragma unroll
-            for (int j = 0; j < PLX; ++j) {
-              pv[j] = j == jr ? x : pv[j];
-              pi[j] = j == jr ? c : pi[j];
-            }
-          }
-        };
-        if (kp <= PL)
-          stream(std::integral_constant<int, PL / 2>{});
-        else
-          stream(std::integral_constant<int, PL>{});
-        // the updated winners go back to where they came from; the list keeps its length
-#pragma unroll
-        for (int j = 0; j < PL; ++j) {
-          const int e = 2 * j + hh;  // the two lanes of a row hold alternate entries of its list
-          if (e < m_prev) {
-            sVal[(cur * kGateRows + rs) * CAP + e] = pv[j];
-            sIdx[(cur * kGateRows + rs) * CAP + e] = pi[j];
-          }
-        }
-        continue;
-      }
-      // more entrants than a list holds: the general path below recounts from scratch
-      if (hh == 0) sCnt[nxt * kGateRows + rs] = 0;
-      wave_lds_fence();
-    }
-    vmin = min_xor32_f(vmin);
-    vmax = max_xor32_f(vmax);
-    const int ntot = m_prev + max(0, min(nc - c0, GC));  // candidates that compete in this group
-    const bool need = (ntot > kp) && (kp > 0);
-
-    auto count_gt = [&](float probe) {
-      int cnt = 0;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; i += 4) cnt = count4_gt(cnt, sc[t][i], sc[t][i + 1], sc[t][i + 2], sc[t][i + 3], probe);
-        }
-      static_assert(PL % 4 == 0, "the winners are counted four at a time");
-#pragma unroll
-      for (int j = 0; j < PL; j += 4) cnt = count4_gt(cnt, pv[j], pv[j + 1], pv[j + 2], pv[j + 3], probe);
-      return sum_xor32_i(cnt);
-    };
-    float tau = -INFINITY, tau_eq = INFINITY;
-    int n_eq = 0;
-    uint32_t iota = 0u;
-    {
-      uint32_t lo_k = float_order_key(vmin) - 1u;
-      uint32_t hi_k = float_order_key(vmax);
-      int c_hi = 0;
-      bool open = need;
-#pragma nounroll
-      for (int iter = 0;; ++iter) {
-        if (open && hi_k - lo_k <= 1u) {
-          tau = order_key_float(hi_k);
-          if (tau != -INFINITY) {
-            tau_eq = tau;
-            n_eq = kp - c_hi;
-          }
-          open = false;
-        }
-        if (!__any(open)) break;
-        uint32_t pk = lo_k + ((hi_k - lo_k) >> 1);
-        if (iter < 12) {
-          const float mf = 0.5f * order_key_float(lo_k + 1u) + 0.5f * order_key_float(hi_k);
-          const uint32_t mk = float_order_key(mf);
-          if (mk > lo_k && mk < hi_k) pk = mk;
-        }
-        const float probe = order_key_float(pk);
-        const int cnt = count_gt(probe);
-        if (open) {
-          if (cnt == kp) {
-            tau = probe;
-            open = false;
-          } else if (cnt > kp) {
-            lo_k = pk;
-          } else {
-            hi_k = pk;
-            c_hi = cnt;
-          }
-        }
-      }
-      const bool tie = n_eq > 0;
-      if (__any(tie)) {
-        auto count_eq_ge = [&](uint32_t trial) {
-          int cnt = 0;
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            if (t < n_tiles) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) {
-                const uint32_t c = (uint32_t)(c0 + t * 32 + acc_row(i, hh));
-                cnt += ((sc[t][i] == tau_eq) & (c >= trial)) ? 1 : 0;
-              }
-            }
-#pragma unroll
-          for (int j = 0; j < PL; ++j) cnt += ((pv[j] == tau_eq) & ((uint32_t)pi[j] >= trial) & (pi[j] >= 0)) ? 1 : 0;
-          return sum_xor32_i(cnt);
-        };
-        const int ceq = count_eq_ge(0u);
-        const bool split = tie && ceq > n_eq;
-        if (__any(split)) {
-          uint32_t i_acc = 0u;
-#pragma nounroll
-          for (int bit = 23; bit >= 0; --bit) {
-            const uint32_t trial = i_acc | (1u << bit);
-            const int cnt = count_eq_ge(trial);
-            if (cnt >= n_eq) i_acc = trial;
-          }
-          if (split) iota = i_acc;
-        }
-      }
-    }
-
-    // winners of this round -> the other list: count per lane, reserve slots once, then store
-    int nwin = 0;
-    if (kp > 0) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const uint32_t c = (uint32_t)(c0 + t * 32 + acc_row(i, hh));
-            const float x = sc[t][i];
-            nwin += ((x > tau) | ((x == tau_eq) & (c >= iota))) ? 1 : 0;
-          }
-        }
-#pragma unroll
-      for (int j = 0; j < PL; ++j) nwin += ((pi[j] >= 0) & ((pv[j] > tau) | ((pv[j] == tau_eq) & ((uint32_t)pi[j] >= iota)))) ? 1 : 0;
-    }
-    int slot = 0;
-    if (nwin > 0) slot = atomicAdd(&sCnt[nxt * kGateRows + rs], nwin);
-    float *ov = sVal + (size_t)((TWO_LISTS ? nxt : 0) * kGateRows + rs) * CAP;
-    int *oi = sIdx + (size_t)((TWO_LISTS ? nxt : 0) * kGateRows + rs) * CAP;
-    if (!TWO_LISTS) wave_lds_fence();  // (one list: both lanes of the row have read it into registers)
-    if (__any(nwin > 0)) {  // (no branches inside: a lane without a winner at a position stores to its trash word)
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const uint32_t c = (uint32_t)(c0 + t * 32 + acc_row(i, hh));
-            const float x = sc[t][i];
-            const bool w = (kp > 0) & ((x > tau) | ((x == tau_eq) & (c >= iota))) & (slot < CAP);
-            *(w ? ov + slot : reinterpret_cast<float *>(sTrash + tid)) = x;
-            *(w ? oi + slot : sTrash + tid) = (int)c;
-            slot += w ? 1 : 0;
-          }
-        }
-#pragma unroll
-      for (int j = 0; j < PL; ++j) {
-        const bool w = (kp > 0) & (pi[j] >= 0) & ((pv[j] > tau) | ((pv[j] == tau_eq) & ((uint32_t)pi[j] >= iota))) & (slot < CAP);
-        *(w ? ov + slot : reinterpret_cast<float *>(sTrash + tid)) = pv[j];
-        *(w ? oi + slot : sTrash + tid) = pi[j];
-        slot += w ? 1 : 0;
-      }
-    }
-    cur = nxt;
-  }
-  __syncthreads();
-
-  // selection words and per-chunk counts of the block, assembled in LDS and written out in passes of WP word columns
-  // (what the chunk-mean tile holds), so that a sequence may have any number of chunks
-  const int WP = min(p.W, (int)((size_t)GC * LD * 2 / (kGateRows * 4)));
-  const int m_fin = valid ? min(sCnt[cur * kGateRows + rs], CAP) : 0;
-  const int seg = m0 / p.seg_rows;
-  for (int w0 = 0; w0 < p.W; w0 += WP) {
-    const int wn = min(WP, p.W - w0);
-    __syncthreads();  // the pass before has been written out
-    for (int v = tid; v < wn * kGateRows; v += 256) sSel[v] = 0u;
-    for (int c = tid; c < wn * 32; c += 256) sHist[c] = 0;
-    __syncthreads();
-    if (valid) {
-#pragma unroll
-      for (int j = 0; j < PL; ++j) {
-        const int e = 2 * j + hh;  // the two lanes of a row hold alternate entries of its list
-        if (e < m_fin) {
-          const int c = sIdx[((TWO_LISTS ? cur : 0) * kGateRows + rs) * CAP + e];
-          const int cw = (c >> 5) - w0;
-          if ((uint32_t)cw < (uint32_t)wn) {
-            atomicOr(&sSel[cw * kGateRows + rs], 1u << (c & 31));
-            atomicAdd(&sHist[c - 32 * w0], 1);
-          }
-        }
-      }
-      if (hh == 0 && a.is_causal && rp >= 0) {
-        const int c = rp / B;  // the own chunk is always selected
-        const int cw = (c >> 5) - w0;
-        if (c < p.max_cols && (uint32_t)cw < (uint32_t)wn) {
-          atomicOr(&sSel[cw * kGateRows + rs], 1u << (c & 31));
-          atomicAdd(&sHist[c - 32 * w0], 1);
-        }
-      }
-    }
-    __syncthreads();
-    for (int v = tid; v < wn * kGateRows; v += 256) {
-      const int t = v / kGateRows, slot_r = v - t * kGateRows;
-      if (m0 + slot_r < Lq) p.sel[((int64_t)h * p.W + w0 + t) * a.total_q + q0 + m0 + slot_r] = sSel[v];
-    }
-    for (int c = tid; c < wn * 32; c += 256) {
-      const int v = sHist[c];
-      if (v && p.segcnt != nullptr) atomicAdd(&p.segcnt[(((int64_t)b * a.heads + h) * p.nseg + seg) * p.max_cols + 32 * w0 + c], v);
-    }
-  }
-}
-
-// ------------------------------------------------------------------------------------
-// The grouped gate for at most 16 running winners per row (top-k up to 17 causal, 16 otherwise): the common case of
-// long sequences.  Same total order and result as topk_gate_big_kernel; what differs is where things live:
-//  * a row's winners stay in REGISTERS across the groups, sorted: the eight weakest of its sixteen places in the lane with
-//    chunks 0..3 of every eight, the eight strongest in its partner.  A new winner is offered to the strong half, which
+// The same gate for sequences with more key chunks than one set of register tiles holds, and for few winners among more than 128.  Chunks are
+// scored in groups of 64; every row keeps the K' best (score, chunk) pairs seen so far, and the next group competes against
+// them.  The total order (score descending, chunk index descending) is strict, so the running winners after the last group are
+// exactly the global top-K'.  PL places per lane, two lanes per row: 8, 16 or 32 for top-k up to 17, 33 and 64 (one more than the places
+// where the own chunk takes no place).
+//  * a row's winners stay in REGISTERS across the groups, sorted: the weaker half of its places in the lane with
+//    chunks 0..3 of every eight, the stronger half in its partner.  A new winner is offered to the strong half, which
 //    passes on what it gives up, and goes in with one pass of minimum / maximum: no compare, no choice between the lanes
 //    (shares sorted per lane needed both: which lane holds the weakest was two exchanges and six selects per winner);
 //  * the chunk means of the next group are fetched into the LDS tile while the current group is worked on;
@@ -888,7 +480,9 @@ __global__ __launch_bounds__(256, CAP < kBigCap ? 2 : 1) void topk_gate_big_kern
 //    of the group reach, and those are its entrants.  The order does the rest, ties and all.
 // 262144 tokens, 16 heads, top-k 16 of 128-key chunks 3859 -> 2921 us; 1024-row parts of prompts with 9000 to 33000 keys, 32
 // heads, top-k 8 51 -> 29 us (before: winners shared out by lane, lists of entrants, the whole cut of the first group searched).  Bound by
-// the vector instructions (87 % of the clocks at 262144 tokens), most of them the pass of a new winner.
+// the vector instructions (87 % of the clocks at 262144 tokens), most of them the pass of a new winner.  Above 16 winners: 126187 tokens, 16 heads, top-k
+// 28 of 64-key chunks, gating and lists 9514 -> 2340 us, 54437 tokens, 32 heads, top-k 27 2603 -> 1007, 40000 tokens, 16 heads, top-k 50 1748 -> 846 (before: winners in two lists in LDS, an entrant looked for the weakest
+// of all, one workgroup per compute unit).
 // ------------------------------------------------------------------------------------
 // A winner is ONE double between 1 and 2: order key of its score and chunk are 48 bits of its fraction, so that the order "score
 // descending, chunk descending" is the order of the doubles and minimum / maximum are single instructions.
@@ -918,6 +512,15 @@ __device__ __forceinline__ double min_winner(double a, double b) {
   return a < b ? a : b;
 #endif
 }
+__device__ __forceinline__ double max_winner(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double d;
+  asm("v_max_f64 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+  return d;
+#else
+  return a > b ? a : b;
+#endif
+}
 // in lanes 0..31 the word of lane + 32, in the others +infinity
 __device__ __forceinline__ double upper_half_or_inf(double v) {
   const uint64_t u = (uint64_t)__double_as_longlong(v);
@@ -929,12 +532,16 @@ __device__ __forceinline__ double upper_half_or_inf(double v) {
   return v;
 #endif
 }
-// A winner word x goes up the ascending places w, all but the largest of eight and x stay: and while it does, the float at lds_addr is on
+// A winner word x goes up the ascending places w, all but the smallest of them and x stay: and while it goes up the last eight, the float at lds_addr is on
 // its way, which is the result.  One statement from the request to the wait: the compiler waits for an LDS read of its own where it issues it when
 // the address comes round a loop, and a register whose value has yet to arrive must not be one that it may copy or spill.  (Nothing
 // else of the wave may be on its way from LDS.)
-__device__ __forceinline__ float insert_winner(double (&w)[8], double x, uint32_t lds_addr) {
+template <int PL>
+__device__ __forceinline__ float insert_winner(double (&places)[PL], double x, uint32_t lds_addr) {
   float score;
+#pragma unroll
+  for (int j = 0; j < PL - 8; ++j) places[j] = min_winner(max_winner(places[j], x), places[j + 1]);
+  double *w = places + PL - 8;
 #if defined(__HIP_DEVICE_COMPILE__)
   double t;
   asm volatile("ds_read_b32 %0, %10\n\t"
@@ -971,9 +578,8 @@ template <int HD>
 static constexpr size_t gate_stream_smem() {
   return (size_t)kStreamGroup * HD * 2 + (size_t)kGateRows * kStreamRowBytes;  // tile and scores; later the selection words of a pass
 }
-template <typename T, int HD>
-__global__ __launch_bounds__(256, HD > 128 ? 2 : 3) void topk_gate_stream_kernel(TopkParams p) {
-  constexpr int PL = 8;                   // winners' places per lane
+template <typename T, int HD, int PL>  // PL: winners' places per lane
+__global__ __launch_bounds__(256, HD > 128 || PL > 16 ? 2 : 3) void topk_gate_stream_kernel(TopkParams p) {
   constexpr int KS = HD / 16;
   constexpr int GC = kStreamGroup, NT = GC / 32;
   constexpr int VPR = HD / 8;             // 16-byte pieces of a row of chunk means
@@ -1046,7 +652,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 2 : 3) void topk_gate_stream_kernel
   // this lane's operand row of a 32-chunk tile: row lane % 32, pieces hh * KS ..
   const uint32_t a_row = ldsTile + (uint32_t)((lane & 31) * RB);
   const int a_swz = tile_swz<HD>(lane & 31);
-  static_assert(PL == 8, "insert_winner");
+  static_assert(PL % 8 == 0, "insert_winner");
   double win[PL];  // places hh * PL .. of the row's winners, ascending
 #pragma unroll
   for (int j = 0; j < PL; ++j) win[j] = hh * PL + j < kp ? kSlotEmpty : kSlotFiller;
@@ -1205,7 +811,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 2 : 3) void topk_gate_stream_kernel
         xv = insert_winner(win, x, row_b + 4u * (uint32_t)xc);
       }
     };
-    // (up to eight winners have their places in the weak half alone)
+    // (winners that have their places in the weak half alone)
     if (kp <= PL)
       stream(std::integral_constant<bool, false>{});
     else
@@ -1712,32 +1318,15 @@ static int launch_gate(const TopkParams &p, dim3 grid, hipStream_t s) {
   hipLaunchKernelGGL(kern, grid, dim3(256), smem, s, p);
   return 0;
 }
-template <int HD, int NT, int CAP>
-static constexpr size_t gate_big_smem() {
-  const size_t tile = (size_t)NT * 32 * (HD + 16) * 2;  // chunk means of a group; later the selection words of a pass
-  const size_t hist = tile / (kGateRows * 4) * 32 * 4;   // counts of the chunks of a pass
-  return tile + (size_t)(CAP <= kBigCap ? 2 : 1) * kGateRows * CAP * 8 + (size_t)2 * kGateRows * 4 + hist + 256 * 4;
-}
 // chunk indices are 16-bit fields of the running winners (topk_gate_stream_kernel) and the forward's step lists
 constexpr int kMaxChunksPerSequence = 65535;
-template <typename T, int HD, int NT, int CAP>
-static int launch_gate_big(const TopkParams &p, dim3 grid, hipStream_t s) {
-  const size_t smem = gate_big_smem<HD, NT, CAP>();
-  static_assert(gate_big_smem<HD, NT, CAP>() <= 160 * 1024, "LDS of one compute unit");
-  auto kern = topk_gate_big_kernel<T, HD, NT, CAP>;
-  if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
-    set_error("fused_topk: cannot reserve %zu bytes of LDS", smem);
-    return 2;
-  }
-  hipLaunchKernelGGL(kern, grid, dim3(256), smem, s, p);
-  return 0;
-}
 // chunks that a row keeps besides its own
 static int gate_winners(const TopkParams &p) { return p.a.is_causal ? p.a.topk - 1 : p.a.topk; }
 template <typename T, int HD>
 static int launch_gate_stream(const TopkParams &p, dim3 grid, hipStream_t s) {
   const size_t smem = gate_stream_smem<HD>();
-  auto kern = topk_gate_stream_kernel<T, HD>;
+  const int kp = gate_winners(p);
+  auto kern = kp <= 16 ? topk_gate_stream_kernel<T, HD, 8> : kp <= 32 ? topk_gate_stream_kernel<T, HD, 16> : topk_gate_stream_kernel<T, HD, 32>;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("fused_topk: cannot reserve %zu bytes of LDS", smem);
     return 2;
@@ -1746,23 +1335,11 @@ static int launch_gate_stream(const TopkParams &p, dim3 grid, hipStream_t s) {
   return 0;
 }
 template <typename T>
-static int launch_gate_big_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
-  // up to 16 running winners per row: the kernel that keeps them in registers, in groups of 64 chunks (three workgroups
-  // per compute unit; with groups of 128 and two workgroups it took 6.4 ms instead of 5.1 at 262144 tokens)
-  const int kp = gate_winners(p);
-  if (p.a.head_dim <= 64) {
-    if (kp > kBigCap) return launch_gate_big<T, 64, 4, kBigCapMax>(p, grid, s);
-    if (kp <= 16) return launch_gate_stream<T, 64>(p, grid, s);
-    return launch_gate_big<T, 64, 8, kBigCap>(p, grid, s);
-  }
-  if (p.a.head_dim <= 128) {
-    if (kp > kBigCap) return launch_gate_big<T, 128, 4, kBigCapMax>(p, grid, s);
-    if (kp <= 16) return launch_gate_stream<T, 128>(p, grid, s);
-    return launch_gate_big<T, 128, 8, kBigCap>(p, grid, s);
-  }
-  if (kp > kBigCap) return launch_gate_big<T, 256, 2, kBigCapMax>(p, grid, s);
-  if (kp <= 16) return launch_gate_stream<T, 256>(p, grid, s);
-  return launch_gate_big<T, 256, 4, kBigCap>(p, grid, s);
+static int launch_gate_stream_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
+  // (groups of 64 chunks, three workgroups per compute unit; with groups of 128 and two workgroups 6.4 ms instead of 5.1 at 262144 tokens)
+  if (p.a.head_dim <= 64) return launch_gate_stream<T, 64>(p, grid, s);
+  if (p.a.head_dim <= 128) return launch_gate_stream<T, 128>(p, grid, s);
+  return launch_gate_stream<T, 256>(p, grid, s);
 }
 template <typename T, int HD, int NJ>
 static int launch_gate_few_nj(const TopkParams &p, hipStream_t s) {
@@ -1900,7 +1477,7 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   if (a->max_seqlen_q <= kFewGateRows && max_cols <= kFewGateChunks)
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_few_hd<bf16_t>(p, s) : launch_gate_few_hd<f16_t>(p, s);
   else if (big)
-    rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_big_hd<bf16_t>(p, ggrid, s) : launch_gate_big_hd<f16_t>(p, ggrid, s);
+    rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_stream_hd<bf16_t>(p, ggrid, s) : launch_gate_stream_hd<f16_t>(p, ggrid, s);
   else
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_hd<bf16_t>(p, ggrid, s) : launch_gate_hd<f16_t>(p, ggrid, s);
   if (rc) return rc;

@@ -77,3 +77,13 @@ def test_more_row_blocks_than_the_second_dimension_of_a_grid():
         assert torch.equal(e[:own.numel()], own) and (e[1:] > e[:-1]).all()
         rows.index_add_(0, e, torch.ones_like(e, dtype=torch.int32))
     assert (rows[:chunk] == 1).all() and (rows[chunk:] == 2).all()
+
+
+# the same with 16 and 32 places per lane: the first count beyond those of 8 and 16, the weak half full and one more, all places; fewer chunks
+# than winners in the first group, and than winners at all in most rows
+@pytest.mark.parametrize("kind", ["random", "levels", "equal", "ascending", "descending"])
+@pytest.mark.parametrize("C,topk,D,causal", [
+    (257, 18, 128, True), (300, 17, 64, False), (321, 33, 128, True), (260, 32, 256, False), (400, 34, 64, True), (290, 33, 128, False),
+    (333, 64, 128, True), (520, 64, 40, False), (280, 64, 256, True), (257, 33, 64, True)])
+def test_selection_of_exact_scores_with_many_winners(kind, C, topk, D, causal):
+    test_selection_of_exact_scores(kind, C, topk, D, causal)
