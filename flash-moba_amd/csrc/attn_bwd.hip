@@ -58,7 +58,7 @@ struct BwdWs {
   int32_t dkv_heads;  // heads of dK / dV (of the kernels that sum query heads)
   int32_t *cnt;    // [total_q * heads] visits handed out per (row, head)
   int32_t *pid;    // [total_q * heads * cap] key block id of each partial
-  uint16_t *part;  // [total_q * heads * cap][head_dim] dQ partials (times dq_part_scale)
+  uint16_t *part;  // [total_q * heads * cap][part_row_elems] dQ partials (times dq_part_scale)
   int32_t cap;
   const uint32_t *visits;  // as in the forward pass (null: slots from the counters)
   int32_t row_mask;        // of list entries: kListRowMask for ranked lists, else -1
@@ -170,6 +170,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   const int off = Lk - Lq;
   const int D = a.head_dim;
+  const int PD = part_row_elems(D, 2);
+  (void)PD;
   const int hk = h0 / (a.heads / a.heads_k);
   const int kq = wave & 1, rt = wave >> 1;   // S and dP: this wave's 32 keys and 32 rows
   const int sel = wave >> 1, fw = wave & 1;  // sums: dV (0) or dK (1), half fw of the features or of the keys
@@ -479,7 +481,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
           const int v = v0 + ft, row = v / VPR, pcs = v - row * VPR;
           const uint32_t p = (uint32_t)sSlot[(r & 1) * 64 + row];
           const Pack8 x = lds_read16(ldsOut + (uint32_t)(row * RB) + (((uint32_t)pcs ^ (uint32_t)(row & 7)) * 16u));
-          if (pcs * 8 < D) st_stream16(ws.part + ((uint64_t)p * (uint32_t)D + (uint32_t)(pcs * 8)), x);
+          if (pcs * 8 < PD) st_stream16(ws.part + ((uint64_t)p * (uint32_t)PD + (uint32_t)(pcs * 8)), x);
           if (!RANKED && pcs == 0) ws.pid[p] = nb;
         }
       } else {
@@ -577,7 +579,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
   if (key0 >= Lk) return;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   const int off = Lk - Lq;
-  const int D = a.head_dim;
+  const int D = a.head_dim, PD = part_row_elems(a.head_dim, 2);
   const int hk = h / (a.heads / a.heads_k);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hh = lane >> 5;
   const int kq = KB == 1 ? (wave & 1) : wave;  // this wave's 32 keys of the block, and its share of the dQ features
@@ -1026,16 +1028,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
       uint32_t bs = (uint32_t)(uintptr_t)(smem + SM::oRow) + (uint32_t)((px * 64 + lane / LPR) * 4);
       uint32_t bx = (uint32_t)(uintptr_t)sdQ0 + (uint32_t)(((lane / LPR) * LDH + col) * 2);
       opaque(bs, bx);
-      // (one test around all rows of the tile rather than one per store: a lane either has features of the head
-      // dimension in its piece or it has not)
+      // (one test around all rows of the tile rather than one per store: a lane either has a piece of the part
+      // row or it has not)
       uint32_t pidx[32 / RPP];
 #pragma unroll
       for (int k = 0; k < 32 / RPP; ++k) pidx[k] = (uint32_t)lds_read_vec<int>(bs + (uint32_t)(TS * 32 + k * RPP) * 4 + (uint32_t)(SM::oSlot - SM::oRow));
-      if (kq * (NDH * 32) + col < D) {
+      if (kq * (NDH * 32) + col < PD) {
 #pragma unroll
         for (int k = 0; k < 32 / RPP; ++k) {
           const Pack8 x = lds_read16(bx + SO + (uint32_t)(k * RPP * LDH * 2));
-          st_stream16(ws.part + ((uint64_t)pidx[k] * (uint32_t)D + (uint32_t)(kq * (NDH * 32) + col)), x);
+          st_stream16(ws.part + ((uint64_t)pidx[k] * (uint32_t)PD + (uint32_t)(kq * (NDH * 32) + col)), x);
         }
       }
       if (!RANKED && kq == 0 && col == 0) {
@@ -1631,7 +1633,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
   const int c8 = li * 8;
   const bool mine = c8 < D;
   const int32_t *pid = ws.pid + rh * ws.cap;
-  const uint16_t *part = ws.part + rh * ws.cap * D;
+  const int PD = part_row_elems(D, 2);
+  const uint16_t *part = ws.part + rh * ws.cap * PD;
   float acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
@@ -1649,11 +1652,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
     for (; t + 4 <= n; t += 4) {  // independent loads, four in flight
       Pack8 x[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) x[u] = ld_stream16(part + (int64_t)(RANKED ? t + u : sOrd[t + u]) * D + c8);
+      for (int u = 0; u < 4; ++u) x[u] = ld_stream16(part + (int64_t)(RANKED ? t + u : sOrd[t + u]) * PD + c8);
 #pragma unroll
       for (int u = 0; u < 4; ++u) add(x[u]);
     }
-    for (; t < n; ++t) add(ld_stream16(part + (int64_t)(RANKED ? t : sOrd[t]) * D + c8));
+    for (; t < n; ++t) add(ld_stream16(part + (int64_t)(RANKED ? t : sOrd[t]) * PD + c8));
   }
   if (valid && mine) {
     const float scale = dq_sum_scale<T>(a.softmax_scale);
@@ -1942,7 +1945,7 @@ extern "C" size_t fmoba_attn_bwd_workspace_bytes(const fmoba_attn_bwd_args *a) {
   }
   const size_t rows = (size_t)a->total_q * a->heads, cap = (size_t)bwd_partial_cap(*a);
   // one spare partial row / block id at the end takes the writes of absent rows
-  return bwd_align256(rows * 4) + bwd_align256((rows * cap + 1) * 4) + bwd_align256((rows * cap + 1) * a->head_dim * 2) + 256;
+  return bwd_align256(rows * 4) + bwd_align256((rows * cap + 1) * 4) + bwd_align256((rows * cap + 1) * part_row_elems(a->head_dim, 2) * 2) + 256;
 }
 
 extern "C" int fmoba_attn_bwd(const fmoba_attn_bwd_args *a, void *stream) { return fmoba_attn_bwd_phases(a, 7, stream); }

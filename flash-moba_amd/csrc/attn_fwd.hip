@@ -47,7 +47,7 @@ constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 struct FwdWs {
   int32_t *cnt;      // [total_q * heads] visits handed out per (row, head)
   float4 *hdr;       // [total_q * heads * cap] {m (log2 domain), l, key block id, -}; ranked: float2 {m, l}
-  void *part;        // [total_q * heads * cap][head_dim] partial outputs (fwd_part_size bytes per element)
+  void *part;        // [total_q * heads * cap][part_row_elems] partial outputs (fwd_part_size bytes per element)
   int32_t cap;
   const uint32_t *visits;  // per (head, row), with ranked lists: the form whose slots are in key-block order (null: the other one)
 };
@@ -321,11 +321,11 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
       for (int k = 0; k < 4; ++k) y[k] = lds_read16(ldsOut + (uint32_t)((8 * k + (lane >> 3)) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) * 16)));
       wave_lds_fence();
       typedef std::conditional_t<F32, float, uint16_t> E;
-      const int f = (part * 8 + (lane & 7)) * (int)(16 / sizeof(E));
+      const int f = (part * 8 + (lane & 7)) * (int)(16 / sizeof(E)), PD = part_row_elems(D, (int)sizeof(E));
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int p2 = __shfl(pidx, 8 * k + (lane >> 3), 64);
-        if (p2 >= 0 && f < D) st_stream16(reinterpret_cast<E *>(ws.part) + ((uint64_t)(uint32_t)p2 * (uint32_t)D + (uint32_t)f), y[k]);
+        if (p2 >= 0 && f < PD) st_stream16(reinterpret_cast<E *>(ws.part) + ((uint64_t)(uint32_t)p2 * (uint32_t)PD + (uint32_t)f), y[k]);
       }
     };
     // once the next tile's loads are in, what is held of this one leaves
@@ -438,7 +438,8 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   float L = 0.f, M = -INFINITY;
   const float4 *hdr = ws.hdr + rh * ws.cap;
   const float2 *hdr2 = reinterpret_cast<const float2 *>(ws.hdr) + rh * ws.cap;
-  const E *part = reinterpret_cast<const E *>(ws.part) + rh * ws.cap * D;
+  const int PD = part_row_elems(D, (int)sizeof(E));
+  const E *part = reinterpret_cast<const E *>(ws.part) + rh * ws.cap * PD;
   // The slot a visit got is arbitrary (a counter handed it out), the sum must not depend on it: every partial gets
   // its rank in ascending key-block order over the WHOLE row (equal ids, a malformed pattern, are ordered by slot),
   // and the partials are merged in rank order, 16 at a time.
@@ -489,7 +490,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
           }
       };
       auto load = [&](Pack8(&x)[NP], int slot) {
-        const E *row = part + (int64_t)slot * D + c0;
+        const E *row = part + (int64_t)slot * PD + c0;
 #pragma unroll
         for (int p = 0; p < NP; ++p) x[p] = ld_stream16(c0 + p * 16 * PE < D ? row + p * 16 * PE : row);
       };
@@ -736,7 +737,7 @@ static size_t fwd_cols_workspace_bytes(const fmoba_attn_fwd_args &a) {
   using namespace fmoba;
   if (a.max_visits_per_row <= 0) return 256;
   const size_t rows = (size_t)a.total_q * a.heads, cap = (size_t)fwd_partial_cap(a);
-  return fwd_align256((rows + 1) * 4) + fwd_align256(rows * cap * 16) + fwd_align256(rows * cap * a.head_dim * fwd_part_size(a.head_dim)) + 256;
+  return fwd_align256((rows + 1) * 4) + fwd_align256(rows * cap * 16) + fwd_align256(rows * cap * part_row_elems(a.head_dim, (int)fwd_part_size(a.head_dim)) * fwd_part_size(a.head_dim)) + 256;
 }
 
 extern "C" size_t fmoba_attn_fwd_workspace_bytes(const fmoba_attn_fwd_args *a) {
