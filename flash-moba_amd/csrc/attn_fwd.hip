@@ -535,8 +535,9 @@ __global__ void fwd_empty_kernel(void *out, float *lse, int64_t n_out_words, int
   for (int64_t i = i0; i < n_lse; i += st) lse[i] = INFINITY;
 }
 
-__global__ void fwd_zero_i32_kernel(int32_t *p, int64_t n) {
+__global__ void fwd_zero_i32_kernel(int32_t *p, int64_t n, int32_t *one_more) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0;
+  if (one_more != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *one_more = 0;
 }
 
 // visits per (row, head) of a pattern: grid over list entries is not possible without the segment of each
@@ -564,13 +565,14 @@ __global__ __launch_bounds__(1024) void csc_row_visits_lds_kernel(fmoba_attn_fwd
   extern __shared__ int32_t visits[];
   constexpr int kCols = 512;
   __shared__ int64_t first[kCols];
-  __shared__ int32_t len[kCols], blocks[kCols];
+  __shared__ int32_t len[kCols], blocks[kCols], most;
   const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b];
   const int64_t bh = (int64_t)b * a.heads + h;
   const int ncols = min(a.max_cols, (Lk + a.lg_block_n - 1) / a.lg_block_n);
+  if (tid == 0) most = 0;
   for (int r0 = blockIdx.x * range; r0 < Lq; r0 += gridDim.x * range) {
     const int rows = min(range, Lq - r0);
     for (int i = tid; i < rows; i += blockDim.x) visits[i] = 0;
@@ -612,15 +614,23 @@ __global__ __launch_bounds__(1024) void csc_row_visits_lds_kernel(fmoba_attn_fwd
       m = max(m, v);
     }
     for (int o = 32; o >= 1; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
-    if (lane == 0 && m > 0) atomicMax(max_out, m);
+    if (lane == 0 && m > 0) atomicMax(&most, m);
     __syncthreads();  // (the next range takes the places)
   }
+  __syncthreads();
+  if (tid == 0 && most > 0) atomicMax(max_out, most);  // (one per workgroup: atomics on one address go one after the other, some 15 ns each)
 }
 __global__ __launch_bounds__(256) void max_i32_kernel(const int32_t *p, int64_t n, int32_t *out) {
   int m = 0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) m = max(m, p[i]);
   for (int o = 32; o >= 1; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0 && m > 0) atomicMax(out, m);
+  __shared__ int most[4];
+  if ((threadIdx.x & 63) == 0) most[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    m = max(max(most[0], most[1]), max(most[2], most[3]));
+    if (m > 0) atomicMax(out, m);
+  }
 }
 
 static inline size_t fwd_align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -702,7 +712,7 @@ template <typename T>
 static int run_fwd(const fmoba_attn_fwd_args &a, const FwdWs &ws, int phases, hipStream_t s) {
   const int64_t rows = (int64_t)a.total_q * a.heads;
   if (phases & FMOBA_FWD_COLUMNS) {
-    if (ws.visits == nullptr) hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, rows);
+    if (ws.visits == nullptr) hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(512), dim3(256), 0, s, ws.cnt, rows, (int32_t *)nullptr);
     const int kb = fwd_key_block(a.lg_block_n);
     int rc;
     if (a.head_dim > 128)
@@ -776,14 +786,13 @@ extern "C" int fmoba_csc_max_row_visits(const fmoba_attn_fwd_args *a, int32_t *c
   FMOBA_REQUIRE(counts && max_out, "csc_max_row_visits: null output pointer");
   hipStream_t s = (hipStream_t)stream;
   const int64_t rows = (int64_t)a->total_q * a->heads;
-  hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(256), dim3(256), 0, s, counts, rows);
-  hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(1), dim3(64), 0, s, max_out, (int64_t)1);
+  hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(256), dim3(256), 0, s, counts, rows, max_out);
   if (rows > 0 && a->max_cols > 0 && a->total_k > 0) {
     FMOBA_REQUIRE(a->col_offsets && a->col_nnz && a->row_indices, "csc_max_row_visits: null CSC pointer");
     // Counts in LDS from eight (sequence, head) pairs on: a workgroup reads all lists of its pair, at about a quarter of the rate at which the
-    // whole chip does atomics in memory, so few pairs are better counted there (32768 tokens, one head, top-k 16 of 128-key chunks 25 us,
-    // 90 in LDS; 8 heads, 8192 tokens 28 and 26; 54437 tokens, 32 heads, top-k 27 of 64-key chunks 1715 and 332; 262144 tokens, 16 heads 2527
-    // and 1911).  Row ranges: enough of them for a workgroup per compute unit, 1024 to 32768 rows.
+    // whole chip does atomics in memory, so few pairs are better counted there (32768 tokens, one head, top-k 16 of 128-key chunks 19 us,
+    // 90 in LDS; 8 heads, 8192 tokens 28 and 17; 54437 tokens, 32 heads, top-k 27 of 64-key chunks 1715 and 332; 262144 tokens, 16 heads 2527
+    // and 1923).  Row ranges: enough of them for a workgroup per compute unit, 1024 to 32768 rows.
     const int64_t pairs = (int64_t)a->batch * a->heads;
     const int per = ceil_div(a->max_seqlen_q, (int)std::max<int64_t>(1, 256 / pairs));
     const int range = std::min(32768, std::max(1024, (per + 255) & ~255)), nrange = std::max(1, ceil_div(a->max_seqlen_q, range));
