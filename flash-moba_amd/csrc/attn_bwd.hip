@@ -1286,7 +1286,7 @@ __device__ __forceinline__ Pack8 row_buffer_load16(RowBuffer, uint32_t, int) { r
 
 // RT: 32-row tiles per wave (with two, every K^T operand read from LDS feeds two MFMAs).  NW: waves.
 template <typename T, int HD, int RT, int NW>
-__global__ __launch_bounds__(64 * NW, (HD > 128 || RT > 1) ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int row_mask, int nsb_max) {
+__global__ __launch_bounds__(64 * NW, HD > 64 ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int row_mask, int nsb_max) {
   typedef DqSmem<HD, RT, NW> SM;
   constexpr int ROWS = SM::ROWS;  // query rows of the workgroup
   constexpr int LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
@@ -1914,7 +1914,14 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
       }
       hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 15) / 16)), dim3(256), smem, s, a, ws, capl);
     } else {
-      int rc = a.head_dim <= 64 ? launch_dq<T, 64, 1, 8>(a, ws, s) : a.head_dim <= 96 ? launch_dq<T, 96, 2, 4>(a, ws, s) : launch_dq<T, 128, 2, 4>(a, ws, s);
+      // Head dimensions 97 to 128: eight waves of one tile instead of four of two for few and long walks, each of which then has a unit (or
+      // most of one) for itself and takes half the time for a step.  Training steps, four waves and eight: one sequence of 1531 tokens, 8 heads
+      // 124.7 -> 120.6 us, 5000 tokens, 16 heads (320 row blocks) 356 -> 342, 8000 tokens, 8 heads 532 -> 518; 8192 tokens, 16 heads (512) 866 ->
+      // 893; six sequences of 1010 (384 blocks of four to a sequence) 206 -> 209.
+      const bool few = (int64_t)a.heads * ((a.total_q + (kDqRows - 1) * (int64_t)a.batch) / kDqRows) <= 400 && a.total_q >= 1500 * (int64_t)a.batch;
+      int rc = a.head_dim <= 64   ? launch_dq<T, 64, 1, 8>(a, ws, s)
+               : a.head_dim <= 96 ? (launch_dq<T, 96, 2, 4>(a, ws, s))
+                                  : (few ? launch_dq<T, 128, 1, 8>(a, ws, s) : launch_dq<T, 128, 2, 4>(a, ws, s));
       if (rc) return rc;
     }
   }
