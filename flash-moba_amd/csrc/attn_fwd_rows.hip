@@ -453,8 +453,8 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // (12037 tokens, 16 heads of 96, top-k 8 of 64-key chunks 208 -> 176 us; 2048 tokens, 8 heads 41 -> 29).
 // With the products at a higher priority than the rest of a step, whole training steps: 65536 tokens in eight sequences 7681 -> 7549 us, 2 x 4096 tokens,
 // top-k 8 of 128-key chunks 496 -> 484, 12037 tokens, 16 heads of 96 484 -> 481, 8191 tokens of short documents the same.
-// RW: waves of a set, which share its tiles.  SPLIT = 2: a second set of waves takes every other step of the same rows, with
-// rings of its own; the two results of a row meet in LDS at the end.  Which of them: launch_rows.
+// RW: waves of a set, which share its tiles.  SPLIT = 2 (4): two (four) sets of waves take turns at the steps of the same rows, with
+// rings of their own; the results of a row meet in LDS at the end.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
 template <typename T, int HD, int RW, int SPLIT>
 __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap) {
@@ -827,6 +827,11 @@ static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, i
   hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap);
   return 0;
 }
+// Workgroups of 64 rows up to which four sets share a walk (head dimensions up to 64): one for every compute unit.  Their rings leave a unit
+// room for one such workgroup; two sets, of which two workgroups fit, take the calls above.  Forward: 2048 tokens, 8 heads (256 of them) 31.8 -> 30.2 us,
+// 4096 tokens, 4 heads (256) 49.2 -> 45.3, 400 rows against 6000 keys, 8 heads (56) 64.7 -> 56.6, 632 rows against 24924 keys, 8 heads (88) 200 -> 164; 3072
+// tokens in two sequences, 8 heads (384) 33.8 -> 37.4.
+constexpr int kRowsFourSets = 256;
 // Which workgroup, by the 128-row blocks of the call and the mean length of its sequences:
 // - two waves of 32 rows and two sets of them where 128-row blocks come to about one per compute unit (two at head dimensions up
 //   to 64, where two such workgroups fit a unit): the walks are half as long and there are twice as many of them.  Against one
@@ -841,6 +846,8 @@ static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, i
 template <typename T, int HD>
 static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
   const int64_t blocks = (int64_t)a.heads * (a.total_q / 128 + a.batch);
+  if constexpr (HD <= 64)
+    if (a.heads * (((int64_t)a.total_q + 63 * a.batch) / 64) <= kRowsFourSets) return launch_rows_split<T, HD, 2, 4>(a, bm, nw, s);
   if (blocks <= (HD > 64 ? 288 : 544)) return launch_rows_split<T, HD, 2, 2>(a, bm, nw, s);
   if constexpr (HD <= 64)
     if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1>(a, bm, nw, s);

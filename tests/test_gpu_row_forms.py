@@ -47,3 +47,13 @@ def test_row_blocks_repeat_to_the_last_bit():
         first = run()
         assert hip.last_fwd_row_blocks()
         assert all(torch.equal(run(), first) for _ in range(200))
+
+
+# Four sets over 64 rows (up to 256 workgroups): walks of fewer steps than sets, of one more, of every remainder, queries that are the last rows of
+# longer sequences' worth of steps; two sets on the other side of the line
+@pytest.mark.parametrize("lens,H,Hk,D,chunk,topk", [
+    ([63, 64, 128, 129, 192, 193, 256, 257, 320, 321, 385], 2, 1, 64, 64, 3), ([449, 513, 577], 4, 4, 48, 64, 9), ([4096], 4, 2, 64, 128, 6),
+    ([900], 1, 1, 16, 256, 2), ([700, 1, 640, 330], 16, 8, 64, 64, 4), ([1024, 2048], 8, 8, 32, 128, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_row_block_workgroups_of_four_sets(lens, H, Hk, D, chunk, topk, dtype):
+    test_row_block_workgroups(lens, H, Hk, D, chunk, topk, dtype)
