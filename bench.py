@@ -104,9 +104,9 @@ def time_events(fn, iters, warmup=1):
 # same counter reads for a plain 1 GiB copy (the summaries of those runs are kept under profiles/, one per workload).
 # Counter runs cannot be made from inside this script, so the figures are the committed measurement (ranked lists where the step has them).
 MEASURED_TRAFFIC_BYTES = {
-    ("headline", "attn_fwd_rows_kernel"): 1.415e9,
-    ("headline", "attn_bwd_dkdv_kernel"): 7.422e9,
-    ("headline", "attn_bwd_dq_kernel"): 5.639e9,
+    ("headline", "attn_fwd_rows_kernel"): 1.249e9,
+    ("headline", "attn_bwd_dkdv_kernel"): 7.353e9,
+    ("headline", "attn_bwd_dq_kernel"): 5.785e9,
     ("c2", "attn_fwd_col_kernel"): 4.320e8,
     ("c3", "attn_fwd_col_kernel"): 7.551e9,
     ("c3", "attn_bwd_dkdv_partials_kernel"): 1.172e10,
