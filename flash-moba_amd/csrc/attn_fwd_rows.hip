@@ -7,8 +7,8 @@
 // part in the matrix products of a step, and the rows that did not select the chunk are masked out
 // of the softmax (their probabilities are exact zeros).  The running maximum, the running sum and
 // the output accumulators stay in registers for the whole walk, so nothing but Q, K, V and the
-// output moves.  Two kernels: attn_fwd_rows_kernel (128 rows and four waves per workgroup, or 64 rows and one or
-// two sets of two, that fetch the K/V tiles straight into LDS themselves; head dimensions up to 128 and up to
+// output moves.  Two kernels: attn_fwd_rows_kernel (128 rows and four waves per workgroup, or 64 rows and one, two or
+// four sets of two, that fetch the K/V tiles straight into LDS themselves; head dimensions up to 128 and up to
 // 512 chunks per sequence) and attn_fwd_rows_loader_kernel (128 rows, four compute and four loader waves; longer
 // sequences).  Head dimensions above 128 have a loop of their own in attn_fwd_rows_wide.hip.  Calls with at most eight query rows per sequence have a
 // kernel of their own (attn_fwd_few.hip).

@@ -17,7 +17,7 @@ struct PoolExtra {
 // grid (max_chunks, batch, ceil(vecs / 64)), block 256 = 4 waves.
 // A wave owns 64 consecutive 16-byte vectors of the (heads_k*head_dim) axis; the four
 // waves of the block split the rows of the chunk and reduce through LDS.
-template <typename T>
+template <typename T, bool MANY>
 __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x) {
   const int c = blockIdx.x, b = blockIdx.y;
   const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1];
@@ -57,9 +57,11 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
     const uint16_t *base = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)head * a.k_head_stride + d0;
     int r = wave;
     // Sixteen independent 16-byte loads in flight per lane, added up in the order of the loop of four below: with four, a chunk of 256 rows is
-    // sixteen memory latencies one after the other (forward of 3334 tokens, 8 heads, 256-key chunks 65.8 -> 62.0 us, decode of 16 sequences of
-    // 512 to 32768 keys, 8 key heads 98.6 -> 95.6, 3072 tokens, 8 heads of 64, 128-key chunks 34.1 -> 33.4; chunks of 64 rows gain nothing).
-    for (; a.chunk > 64 && r + 60 < n; r += 64) {
+    // sixteen memory latencies one after the other.  For rows of up to 2 KB (forward of 3334 tokens, 8 heads, 256-key chunks 65.8 -> 62.0 us, decode of
+    // 43 sequences of up to 59161 keys, 2 key heads of 64 102.9 -> 95.5, of 16 sequences, 8 key heads of 128 119.2 -> 118.6, 3072 tokens, 8 heads of 64, 128-key
+    // chunks 34.2 -> 33.5); wider rows read fewer pages of memory at a time with four (decode of 8 sequences of 30000 keys, 32 key heads, 256-key
+    // chunks 370 us, 392 with sixteen), and chunks of 64 rows gain nothing.
+    for (; MANY && r + 60 < n; r += 64) {
       Pack8 p[16];
 #pragma unroll
       for (int j = 0; j < 16; ++j) p[j] = ld_global16(base + (int64_t)(row0 + r + 4 * j) * a.k_row_stride);
@@ -169,10 +171,10 @@ static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &
   dim3 grid(a->max_chunks, a->batch, ceil_div(nvec, 64));
   FMOBA_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "mean_pool: batch or heads*dim too large for the launch grid");
   hipStream_t s = (hipStream_t)stream;
-  if (a->dtype == FMOBA_DTYPE_BF16)
-    hipLaunchKernelGGL(mean_pool_kernel<bf16_t>, grid, dim3(256), 0, s, *a, extra);
-  else
-    hipLaunchKernelGGL(mean_pool_kernel<f16_t>, grid, dim3(256), 0, s, *a, extra);
+  const bool many = a->chunk > 64 && nvec <= 128;  // (the reasons stand at its loop)
+  auto kern = a->dtype == FMOBA_DTYPE_BF16 ? (many ? mean_pool_kernel<bf16_t, true> : mean_pool_kernel<bf16_t, false>)
+                                          : (many ? mean_pool_kernel<f16_t, true> : mean_pool_kernel<f16_t, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, *a, extra);
   FMOBA_LAUNCH_CHECK("mean_pool");
   return 0;
 }
