@@ -20,9 +20,13 @@ __device__ __forceinline__ uint32_t mad24_u32(uint32_t a, uint32_t b, uint32_t c
 // nothing runs under the softmax unless it stands there, so a step is two runs of 32 products: S of the next step, with the rescaling
 // of O between them, and V^T P of this one, with the softmax of the next step between them.  Each run has the tile loads of a later step
 // between its products, one per four (eight in a row at its start: 181 -> 171 us below).
-// O is rescaled in every step, by a factor between 2^-1/2 and 2^1/2 as a rule: that keeps a block's reference point at its maximum less
-// a whole number, so that its largest probability is exact in 16 bits (error of the output against 64 bits, 2 x 4096 tokens, 8 heads, top-k 8 of
-// 128-key chunks: bf16 2.007e-3, fp16 2.507e-4; the column form, whose blocks have their maximum for reference, 2.046e-3 and 2.556e-4).
+// O is rescaled in every step, by a factor between 1/2 and 2 as a rule: that keeps a block's reference point at its maximum less
+// a whole number, so that its largest probability is exact in 16 bits, and the whole number is chosen by the largest score of the walk so far: the
+// reference point lies at most 1/2 above that score and 8 1/2 below it, however long the walk is.  (Chosen by the reference point before, it would go
+// up to 1/2 further in every step: wrong fp16 results from 64 steps on, NaN in either type within a few hundred.)
+// Error of the output against 64 bits, rows here and columns, whose blocks have their own maximum for reference: 2 x 4096 tokens, 8 heads, top-k 8 of
+// 128-key chunks bf16 2.010e-3 and 2.047e-3, fp16 2.507e-4 and 2.554e-4; rows that see 64 steps 2.105e-3 and 2.106e-3, 2.632e-4 and 2.632e-4, 512 steps
+// 2.108e-3 and 2.166e-3, 2.623e-4 and 2.694e-4, 2048 steps 2.094e-3 and 2.157e-3, 2.629e-4 and 2.699e-4.
 // What bounds it: matrix products at the power limit (1.0 PFLOP/s executed at 16384 tokens; without the tile loads it would be 15 % faster, without
 // the rescaling or the exponentials 3 to 5 %).  The same call: columns 134 us and their combine 89 -> 171 us, training step 612 -> 530.
 template <typename T>
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
   f32x16 st[2];       // S^T: register i of tile kt <-> key kt*32 + acc_row(i, hh), this lane's row
   Pack8 pf[2][2], pn[2][2];  // P^T of step t and of step t + 1, as the B operand of O^T += V^T P^T
-  float ref = -INFINITY, l_run = 0.f, alpha = 1.f;
+  float ref = -INFINITY, top = -INFINITY, l_run = 0.f, alpha = 1.f;  // reference point and largest score of the walk so far (log2)
   const uint32_t rowoff = (uint32_t)((lane & 31) * RB + ((tile_frag_piece<HD>(hh, 0) ^ tile_swz<HD>(lane & 31)) * 16));
   const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
   const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
@@ -195,12 +199,13 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
 #pragma unroll
       for (int i = 0; i < 8; ++i) mloc = fmaxf(mloc, st[s / 2][(s & 1) * 8 + i]);
     } else if constexpr (s == 4) {
-      // The reference point of the exponentials is the block's maximum less a whole number: the largest p of the block is a
-      // power of two, which the 16-bit P holds exactly.
+      // The reference point of the exponentials is the block's maximum less a whole number (the largest p of the block is a
+      // power of two, which the 16-bit P holds exactly) and within 1/2 of the walk's maximum so far, or below it by up to 8 1/2.
       const float x = max_xor32_f(mloc) * scale_log2;
       const bool seen = active && x > -INFINITY;
-      const float k = x - ref > 8.f ? 0.f : rintf(x - ref);
+      const float k = x - top > 8.f ? 0.f : rintf(x - top);
       const float r = seen ? x - k : ref;
+      top = seen ? fmaxf(top, x) : top;
       alpha = r == ref ? 1.f : __builtin_amdgcn_exp2f(ref - r);
       neg = seen ? -r : -INFINITY;
       ref = r;
