@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
   // ---- the softmax of step t in slices: 0..3 row maximum, 4 reference point, 5..20 two exponentials each ----
   float mloc = 0.f, neg = 0.f, lsum = 0.f;
   bool active = false;
-  uint32_t keep = 0u;  // nothing of a row that skips the step, whatever the scores are
+  uint32_t keep = 0u;  // nothing of a row that skips the step, whatever the scores are (one that takes part hands on its NaN scores)
   auto mask = [&](int key0, int c, uint32_t word) {
     active = valid && ((word >> (c & 31)) & 1u) != 0u && lim >= key0;
     const int lim_rel = active ? lim - key0 : -1;
@@ -207,10 +207,10 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
       const float r = seen ? x - k : ref;
       top = seen ? fmaxf(top, x) : top;
       alpha = r == ref ? 1.f : __builtin_amdgcn_exp2f(ref - r);
-      neg = seen ? -r : -INFINITY;
+      neg = seen ? -r : 0.f;  // (0: all scores are minus infinity or NaN)
       ref = r;
       lsum = 0.f;
-      keep = seen ? 0xffffffffu : 0u;
+      keep = active ? 0xffffffffu : 0u;
     } else if constexpr (s < 21) {
       constexpr int j = s - 5, kt = j / 8, w = j % 8;
       const float p0 = __builtin_amdgcn_exp2f(fmaf(st[kt][2 * w], scale_log2, neg));

@@ -118,3 +118,22 @@ def test_wide_backward_with_rows_far_apart(D, chunk):
                                                 False, 128, chunk, None)[:3]
     for near, apart in zip(grads(q, dout), grads(far(q), far(dout))):
         assert torch.equal(near, apart)
+
+
+# infinities and NaN in Q and K: the same elements of out and lse are NaN and infinite as in the column form, the others agree
+@pytest.mark.gpu
+@pytest.mark.parametrize("which,at,value", [("q", 300, float("nan")), ("q", 300, float("inf")), ("k", 200, float("nan")), ("k", 200, float("inf")),
+                                            ("k", 200, float("-inf")), ("k", slice(192, 256), float("nan"))])
+@pytest.mark.parametrize("D", [256, 136])
+def test_wide_row_blocks_non_finite_scores(which, at, value, D):
+    L, chunk = 700, 64
+    q, k, v, cu, cud = _inputs([L], 2, 1, D, torch.bfloat16, 11)
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cud, cud, L, L, 4, chunk, causal=True)
+    {"q": q, "k": k}[which][at, 0] = value
+    _assert_same_places(_forward(q, k, v, cud, [L], pattern, chunk, 2), _forward(q, k, v, cud, [L], pattern, chunk, 1))
+
+
+def _assert_same_places(got, want):
+    for x, y in zip(got, want):
+        assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.isposinf(), y.isposinf()) and torch.equal(x.isneginf(), y.isneginf())
+        assert_close("row blocks", x.nan_to_num(0.0, 0.0, 0.0), y.nan_to_num(0.0, 0.0, 0.0), 2e-2, 1e-2)  # (the bounds of the other attention tests)
