@@ -38,6 +38,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
   int *sStep = reinterpret_cast<int *>(smem + SM::oStep);
   uint32_t *sUnion = reinterpret_cast<uint32_t *>(sStep + step_cap);
   uint32_t *sBits = sUnion + nw * SM::UPW;
+  int *sAgain = reinterpret_cast<int *>(sBits + nw * kRows);  // per wave: a sum is not finite
 
   const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
   const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
@@ -116,20 +117,11 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
 #endif
   }
   wait_all_loads();
-  const int e0 = __builtin_amdgcn_readfirstlane(entry_at(0));
-  int e1 = __builtin_amdgcn_readfirstlane(entry_at(1)), e2 = __builtin_amdgcn_readfirstlane(entry_at(2)), e3 = __builtin_amdgcn_readfirstlane(entry_at(3));  // of steps t + 1, t + 2, t + 3
-  feed(tile_k(0, e0));
-  feed(tile_k(1, e1));
-  feed(tile_v(0, e0));
 
   f32x16 o[NDT];  // O^T: register i of feature tile dt <-> feature dt*32 + acc_row(i, hh), this lane's row
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
   f32x16 st[2];       // S^T: register i of tile kt <-> key kt*32 + acc_row(i, hh), this lane's row
   Pack8 pf[2][2], pn[2][2];  // P^T of step t and of step t + 1, as the B operand of O^T += V^T P^T
-  float ref = -INFINITY, top = -INFINITY, l_run = 0.f, alpha = 1.f;  // reference point and largest score of the walk so far (log2)
+  float ref, top, l_run, alpha;  // reference point and largest score of the walk so far (log2)
   const uint32_t rowoff = (uint32_t)((lane & 31) * RB + ((tile_frag_piece<HD>(hh, 0) ^ tile_swz<HD>(lane & 31)) * 16));
   const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
   const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
@@ -141,7 +133,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
 #endif
   };
   // ---- S^T of step t, the sums of the walk scaled by alpha meanwhile ----
-  auto scores = [&](auto scaled, int t, const Tile &x) {
+  auto scores = [&](auto scaled, int t, const Tile &x) __attribute__((always_inline)) {
     uint32_t ak = ldsK + (uint32_t)((t & 1) * (int)SM::tile) + rowoff;
     opaque(ak);
     constexpr int AHEAD = 6;
@@ -192,7 +184,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
         }
     }
   };
-  auto soft = [&](auto sc) {
+  auto soft = [&](auto sc) __attribute__((always_inline)) {
     constexpr int s = decltype(sc)::value;
     if constexpr (s < 4) {
       if constexpr (s == 0) mloc = -INFINITY;
@@ -220,14 +212,16 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
       if constexpr (j == 15) l_run = keep ? l_run * alpha + lsum : l_run;
     }
   };
+  uint32_t took = 0u;  // keep of step t
   auto next = [&]() {
+    took = keep;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) pf[kt][s2] = pn[kt][s2];
   };
   // ---- O^T += V^T P^T of step t, the softmax of step t + 1 meanwhile ----
-  auto sums = [&](int t, const Tile &x) {
+  auto sums = [&](auto apart, int t, const Tile &x) __attribute__((always_inline)) {
     uint32_t tv = ldsV + (uint32_t)((t & 1) * (int)SM::tile) + troff;
     opaque(tv);
     Pack8 vt[2][4];
@@ -240,9 +234,19 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
     for (int m = 0; m < AHEAD; ++m) read(m);
     static_for<4>([&](auto sl) { soft(sl); });
     __builtin_amdgcn_sched_barrier(0);
+    f32x16 with;
     static_for<4 * NDT>([&](auto mc) {
       constexpr int m = decltype(mc)::value, dt = m >> 2, u = m & 3;
-      o[dt] = mfma32<T>(vt[dt & 1][u], pf[u >> 1][u & 1], o[dt]);
+      if constexpr (decltype(apart)::value) {
+        if constexpr (u == 0) with = o[dt];
+        with = mfma32<T>(vt[dt & 1][u], pf[u >> 1][u & 1], with);
+        if constexpr (u == 3) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[dt][i] = took ? with[i] : o[dt][i];
+        }
+      } else {
+        o[dt] = mfma32<T>(vt[dt & 1][u], pf[u >> 1][u & 1], o[dt]);
+      }
       if constexpr (m + AHEAD < 4 * NDT) read(m + AHEAD);
       if constexpr (m == 0) soft(std::integral_constant<int, 4>{});
       if constexpr (m % 4 == 3) load_piece(x, m / 4);
@@ -253,33 +257,59 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
   };
 
   auto word_of = [&](int s) { return sBits[((s >> 16) >> 5) * kRows + wave * 32 + (lane & 31)]; };
-  wait_loads_but<2 * NI>();  // K(0)
-  __syncthreads();
-  scores(std::false_type{}, 0, Tile{});
-  mask((e0 & 0xffff) << 6, e0 >> 16, word_of(e0));
-  static_for<21>([&](auto sl) { soft(sl); });
-  next();
-  alpha = 1.f;
-  __syncthreads();  // every wave has read K(0)
-  feed(tile_k(2, e2));
-  int e_nx = entry_at(4);
-  // Two barriers per step: before S(t + 1) and before the products with V(t).  A tile of V is asked for behind the first, one of K behind the
-  // second (among the products of that part), each one and a half steps ahead of its use; 2 NI loads are younger than the ones that a
-  // barrier hands over.
-  for (int t = 0; t < nstep; ++t) {
-    wait_loads_but<2 * NI>();  // K(t + 1)
-    __syncthreads();           // and every wave is done with V(t - 1)
-    const uint32_t word = word_of(e1);
-    scores(std::true_type{}, t + 1, tile_v(t + 1, e1));
-    wait_loads_but<2 * NI>();  // V(t)
-    __syncthreads();           // and every wave is done with K(t + 1)
-    mask((e1 & 0xffff) << 6, e1 >> 16, t + 1 < nstep ? word : 0u);
-    sums(t, tile_k(t + 3, e3));
-    e1 = e2, e2 = e3, e3 = __builtin_amdgcn_readfirstlane(e_nx);
-    e_nx = entry_at(t + 5);
-  }
-  wait_all_loads();
-  __syncthreads();  // every wave is done with the rings and nothing is in flight: they now hold the output tiles
+  // A step's products take a row that skips it along with probabilities of zero, which leave NaN where V is infinite or NaN.  If
+  // the block has any sum that is not finite, it is walked a second time with the sums of rows that skip a step set aside: as in the column form,
+  // a row's output depends on the chunks that it selected alone.  (The look at the sums: training step of 2 x 4096 tokens, 8 heads 470.5 -> 472.7 us.)
+  auto walk = [&](auto apart) __attribute__((always_inline)) {
+    const int e0 = __builtin_amdgcn_readfirstlane(entry_at(0));
+    int e1 = __builtin_amdgcn_readfirstlane(entry_at(1)), e2 = __builtin_amdgcn_readfirstlane(entry_at(2)), e3 = __builtin_amdgcn_readfirstlane(entry_at(3));  // of steps t + 1, t + 2, t + 3
+    feed(tile_k(0, e0));
+    feed(tile_k(1, e1));
+    feed(tile_v(0, e0));
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+    ref = -INFINITY, top = -INFINITY, l_run = 0.f, alpha = 1.f;
+    wait_loads_but<2 * NI>();  // K(0)
+    __syncthreads();
+    scores(std::false_type{}, 0, Tile{});
+    mask((e0 & 0xffff) << 6, e0 >> 16, word_of(e0));
+    static_for<21>([&](auto sl) { soft(sl); });
+    next();
+    alpha = 1.f;
+    __syncthreads();  // every wave has read K(0)
+    feed(tile_k(2, e2));
+    int e_nx = entry_at(4);
+    // Two barriers per step: before S(t + 1) and before the products with V(t).  A tile of V is asked for behind the first, one of K behind the
+    // second (among the products of that part), each one and a half steps ahead of its use; 2 NI loads are younger than the ones that a
+    // barrier hands over.
+    for (int t = 0; t < nstep; ++t) {
+      wait_loads_but<2 * NI>();  // K(t + 1)
+      __syncthreads();           // and every wave is done with V(t - 1)
+      const uint32_t word = word_of(e1);
+      scores(std::true_type{}, t + 1, tile_v(t + 1, e1));
+      wait_loads_but<2 * NI>();  // V(t)
+      __syncthreads();           // and every wave is done with K(t + 1)
+      mask((e1 & 0xffff) << 6, e1 >> 16, t + 1 < nstep ? word : 0u);
+      sums(apart, t, tile_k(t + 3, e3));
+      e1 = e2, e2 = e3, e3 = __builtin_amdgcn_readfirstlane(e_nx);
+      e_nx = entry_at(t + 5);
+    }
+    if constexpr (!decltype(apart)::value) {
+      float x[4] = {0.f, 0.f, 0.f, 0.f};  // NaN if a sum is not finite
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i & 3] = fmaf(o[dt][i], 0.f, x[i & 3]);
+      const bool mine = __any(valid && (x[0] + x[1]) + (x[2] + x[3]) != 0.f);
+      if (lane == 0) sAgain[wave] = mine;
+    }
+    wait_all_loads();
+    __syncthreads();  // every wave is done with the rings and nothing is in flight: they now hold the output tiles
+  };
+  walk(std::false_type{});
+  if (__builtin_amdgcn_readfirstlane(sAgain[0] | sAgain[1] | sAgain[2] | sAgain[3]) != 0) walk(std::true_type{});
 
   const float l_tot = sum_xor32_f(l_run);
   const bool empty = !(l_tot > 0.f);
@@ -309,7 +339,7 @@ int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, h
   typedef FwdRowsDirectSmem<256, 4, 1> SM;
   auto kern = a.dtype == FMOBA_DTYPE_BF16 ? attn_fwd_rows_wide_kernel<bf16_t> : attn_fwd_rows_wide_kernel<f16_t>;
   const int step_cap = ceil_div(a.max_seqlen_k, 64);  // (at most kRowsStepCap: fwd_rows_feasible)
-  const size_t smem = SM::bytes(step_cap, nw);
+  const size_t smem = SM::bytes(step_cap, nw) + 16;  // (and the four words of sAgain)
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;

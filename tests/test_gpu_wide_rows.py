@@ -137,3 +137,27 @@ def _assert_same_places(got, want):
     for x, y in zip(got, want):
         assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.isposinf(), y.isposinf()) and torch.equal(x.isneginf(), y.isneginf())
         assert_close("row blocks", x.nan_to_num(0.0, 0.0, 0.0), y.nan_to_num(0.0, 0.0, 0.0), 2e-2, 1e-2)  # (the bounds of the other attention tests)
+
+
+# infinities and NaN in V: they reach the rows that selected their chunk, as in the column form, and no bit of the others; a head apart, pieces at the end of
+# the features, the last key of a sequence, a row block whose walk is one step
+@pytest.mark.gpu
+@pytest.mark.parametrize("at,feature,value", [(70, 3, float("inf")), (255, 100, float("nan")), (400, -1, float("-inf")), (699, 0, float("inf")), (720, 8, float("nan")),
+                                              (1, slice(None), float("inf"))])
+@pytest.mark.parametrize("D", [256, 136])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_row_blocks_non_finite_values(at, feature, value, D, dtype):
+    lens, chunk = [700, 40, 300], 64
+    q, k, v, cu, cud = _inputs(lens, 4, 2, D, dtype, 12)
+    pattern = flash_moba.flash_topk_varlen_func(q, k, cud, cud, max(lens), max(lens), 4, chunk, causal=True)
+    plain, _ = _forward(q, k, v, cud, lens, pattern, chunk, 2)
+    v[at, 1, feature] = value
+    rows, cols = (_forward(q, k, v, cud, lens, pattern, chunk, m) for m in (2, 1))
+    _assert_same_places(rows, cols)
+    b = 0 if at < 700 else 1
+    c = (at - cu[b]) // chunk
+    hit = torch.zeros(q.shape[:2], dtype=torch.bool, device="cuda")
+    for h in (2, 3):
+        lo, n = int(pattern[0][b, h, c]), int(pattern[1][b, h, c])
+        hit[cu[b] + pattern[2][lo:lo + n].long(), h] = True
+    assert hit.any() and not hit.all() and torch.equal(rows[0][~hit], plain[~hit])
