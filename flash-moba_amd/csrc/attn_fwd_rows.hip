@@ -882,8 +882,11 @@ bool fwd_rows_feasible(const fmoba_attn_fwd_args &a) {
          a.max_cols < 32768 && a.lg_block_n % 64 == 0;
 }
 
-// the rows' selection words fit the workgroup's LDS (512 chunks per sequence): the kernels without loader waves
-bool fwd_rows_direct(const fmoba_attn_fwd_args &a) { return ceil_div(a.max_cols, 32) <= kRowsWords; }
+// The kernels without loader waves: the rows' selection words fit the workgroup's LDS (512 chunks per sequence), the rows of a tile lie within 32-bit
+// byte offsets of its first key.
+bool fwd_rows_direct(const fmoba_attn_fwd_args &a) {
+  return ceil_div(a.max_cols, 32) <= kRowsWords && a.k_row_stride < ((int64_t)1 << 24) && a.v_row_stride < ((int64_t)1 << 24);
+}
 
 size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a) {
   if (a.selection_bits != nullptr) return 256;
@@ -917,8 +920,7 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
   if (phases & 2) {
     const bool bf = a.dtype == FMOBA_DTYPE_BF16;
     int rc;
-    // (the rows of a tile lie within 32-bit byte offsets of its first key)
-    const bool direct = fwd_rows_direct(a) && a.k_row_stride < ((int64_t)1 << 24) && a.v_row_stride < ((int64_t)1 << 24);
+    const bool direct = fwd_rows_direct(a);
     if (a.head_dim <= 64)
       rc = direct ? (bf ? launch_rows<bf16_t, 64>(a, bm, nw, s) : launch_rows<f16_t, 64>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 64>(a, bm, nw, s) : launch_rows_loader<f16_t, 64>(a, bm, nw, s));

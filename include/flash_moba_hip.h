@@ -190,8 +190,8 @@ typedef struct {
   int32_t *visits_overflow;
 } fmoba_attn_fwd_args;
 int32_t fmoba_attn_fwd_key_block(int32_t lg_block_n);
-/* Bytes of workspace for the call described by `a` (sizes, max_visits_per_row and fwd_mode are read,
- * pointers are not), and which form it will run (1 = row blocks, 0 = columns). */
+/* Bytes of workspace for the call described by `a` (sizes, the row strides of k and v, max_visits_per_row
+ * and fwd_mode are read, pointers are not), and which form it will run (1 = row blocks, 0 = columns). */
 size_t fmoba_attn_fwd_workspace_bytes(const fmoba_attn_fwd_args *a);
 int32_t fmoba_attn_fwd_uses_row_blocks(const fmoba_attn_fwd_args *a);
 /* counts (total_q * heads) int32 and max_out (1) int32 are device outputs: visits per (row, head) and

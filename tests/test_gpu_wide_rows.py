@@ -20,6 +20,15 @@ def test_wide_forward_lines(lens, chunk, topk, heads, rows):
     assert hip.load_library().fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == rows
 
 
+# keys or values further apart than the kernel's 32-bit offsets reach stay with the columns
+@pytest.mark.parametrize("field", ["k_row_stride", "v_row_stride"])
+def test_wide_forward_of_rows_far_apart(field):
+    f = fwd_args([16384], 64, 32, heads=4, D=256)
+    for stride, rows in ((1024, 1), ((1 << 24) - 8, 1), (1 << 24, 0), (1 << 26, 0)):
+        setattr(f, field, stride)
+        assert hip.load_library().fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == rows
+
+
 def _inputs(lens, H, Hk, D, dtype, seed):
     g = torch.Generator(device="cuda").manual_seed(seed)
     q, k, v = (torch.randn((sum(lens), h, D), generator=g, device="cuda").to(dtype) for h in (H, Hk, Hk))
