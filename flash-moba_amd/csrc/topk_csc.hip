@@ -811,8 +811,8 @@ __global__ __launch_bounds__(256, HD > 128 || PL > 16 ? 2 : 3) void topk_gate_st
         xv = insert_winner(win, x, row_b + 4u * (uint32_t)xc);
       }
     };
-    // (winners that have their places in the weak half alone)
-    if (kp <= PL)
+    // (up to eight winners have their places in the weak half alone; 16 and 32 places per lane serve more winners than that)
+    if (PL == 8 && kp <= PL)
       stream(std::integral_constant<bool, false>{});
     else
       stream(std::integral_constant<bool, true>{});
