@@ -780,6 +780,18 @@ static int fwd_check_common(const fmoba_attn_fwd_args *a) {
   return 0;
 }
 
+// Counts in LDS or by atomics in memory.  In LDS a workgroup reads all lists of its (sequence, head), some 2.4 entries per ns, so the longest sequence is the
+// call; the whole chip does 27 atomics per ns, up to 60 where the counters of few heads lie close together.  So LDS where a call is worth
+// many heads of its longest sequence.  Atomics and LDS, us: 262144 tokens, top-k 16 of 128-key chunks, 8 heads 1219 and 1497, 16 heads 2530 and 1925;
+// 90000 tokens, top-k 8, 10 heads 279 and 285, 12 heads 336 and 295; sequences of 20000, top-k 16, 4 x 4 heads 146 and 136, 8 x 2 heads 115 and 135, 16 x 2
+// heads 206 and 142, 32 x 1 head 142 and 144; one sequence of 200000 with seven of 2048, 1 head 118 and 1086, 16 heads of 150000 with three of 2000 767
+// and 504.  And where the longest lists are so short that their reading takes less than the two more launches: 8 heads of 1000 tokens.
+static bool csc_visits_in_lds(const fmoba_attn_fwd_args &a) {
+  const int64_t longest = std::max(1, a.max_seqlen_q), alike = (int64_t)a.heads * a.total_q / longest;
+  return alike >= std::max(12, 64 / a.heads) || (alike >= 8 && longest * a.max_cols <= 32768);
+}
+extern "C" int32_t fmoba_csc_row_visits_in_lds(const fmoba_attn_fwd_args *a) { return a != nullptr && a->heads > 0 && csc_visits_in_lds(*a) ? 1 : 0; }
+
 extern "C" int fmoba_csc_max_row_visits(const fmoba_attn_fwd_args *a, int32_t *counts, int32_t *max_out, void *stream) {
   using namespace fmoba;
   if (int rc = fwd_check_common(a)) return rc;
@@ -789,16 +801,13 @@ extern "C" int fmoba_csc_max_row_visits(const fmoba_attn_fwd_args *a, int32_t *c
   hipLaunchKernelGGL(fwd_zero_i32_kernel, dim3(256), dim3(256), 0, s, counts, rows, max_out);
   if (rows > 0 && a->max_cols > 0 && a->total_k > 0) {
     FMOBA_REQUIRE(a->col_offsets && a->col_nnz && a->row_indices, "csc_max_row_visits: null CSC pointer");
-    // Counts in LDS from eight (sequence, head) pairs on: a workgroup reads all lists of its pair, at about a quarter of the rate at which the
-    // whole chip does atomics in memory, so few pairs are better counted there (32768 tokens, one head, top-k 16 of 128-key chunks 19 us,
-    // 90 in LDS; 8 heads, 8192 tokens 28 and 17; 54437 tokens, 32 heads, top-k 27 of 64-key chunks 1715 and 332; 262144 tokens, 16 heads 2527
-    // and 1923).  Row ranges: enough of them for a workgroup per compute unit, 1024 to 32768 rows.
+    // Row ranges: enough of them for a workgroup per compute unit, 1024 to 32768 rows.
     const int64_t pairs = (int64_t)a->batch * a->heads;
     const int per = ceil_div(a->max_seqlen_q, (int)std::max<int64_t>(1, 256 / pairs));
     const int range = std::min(32768, std::max(1024, (per + 255) & ~255)), nrange = std::max(1, ceil_div(a->max_seqlen_q, range));
     const size_t smem = (size_t)range * 4;
     auto kern = csc_row_visits_lds_kernel;
-    if (pairs >= 8 &&
+    if (csc_visits_in_lds(*a) &&
         (smem <= 32 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess)) {
       hipLaunchKernelGGL(kern, dim3(nrange, a->heads, a->batch), dim3(1024), smem, s, *a, counts, max_out, fwd_key_block(a->lg_block_n), range);
     } else {

@@ -198,6 +198,8 @@ int32_t fmoba_attn_fwd_uses_row_blocks(const fmoba_attn_fwd_args *a);
  * their maximum for the pattern in `a` (q/k/v/out/workspace of `a` are not read).  No counterpart in the
  * reference, whose row-wise scratch needs no bound. */
 int fmoba_csc_max_row_visits(const fmoba_attn_fwd_args *a, int32_t *counts, int32_t *max_out, void *stream);
+/* 1 if the counts of that call are kept in LDS, 0 if by atomics in memory (sizes alone are read; same results). */
+int32_t fmoba_csc_row_visits_in_lds(const fmoba_attn_fwd_args *a);
 int fmoba_attn_fwd(const fmoba_attn_fwd_args *a, void *stream);
 /* The same call split into its two launches so that each can be timed on its own: phases is a bit
  * mask, 1 = the column pass (clears the visit counters first), 2 = the per-row combine; in the

@@ -52,3 +52,12 @@ def test_wide_heads_partial_results_are_bounded_by_the_sequence():
     f.total_k = f.max_seqlen_k = 160000
     f.max_cols = 20
     assert lib.fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == 0
+
+
+# visits of a pattern: in LDS for calls worth at least twelve heads of the longest sequence (more of them where a sequence has few), by atomics where one
+# workgroup would read most of the call's lists
+@pytest.mark.parametrize("lens,heads,lds", [([262144], 8, 0), ([262144], 11, 0), ([262144], 12, 1), ([200000] + [2048] * 7, 1, 0), ([150000] + [2000] * 7, 4, 0),
+                                            ([20000] * 63, 1, 0), ([20000] * 64, 1, 1), ([20000] * 15, 2, 0), ([20000] * 16, 2, 1), ([20000] * 4, 4, 1),
+                                            ([1024], 8, 1), ([1024], 7, 0), ([2304], 8, 0)])
+def test_visits_in_lds(lens, heads, lds):
+    assert H.load_library().fmoba_csc_row_visits_in_lds(ctypes.byref(fwd_args(lens, 128, 16, heads=heads))) == lds

@@ -10,11 +10,13 @@ from flash_moba import flash_moba_hip as hip
 pytestmark = pytest.mark.gpu
 
 
-# pairs on both sides of the line between the two kernels; ranges of rows that end inside a sequence, sequences of no rows, of one; more than
+# atomics in memory and (the last five) counts in LDS; ranges of rows that end inside a sequence, sequences of no rows, of one; more than
 # 512 columns; lists of more than 512 entries, unequal in pairs; columns whose last key block is cut short; rows of no sequence
 @pytest.mark.parametrize("lens_q,lens_k,heads,chunk,rest", [
     ([3000, 1, 0, 1025], [3000, 700, 64, 1025], 2, 64, 0), ([300, 90], [300, 90], 4, 192, 5), ([40000], [40000], 8, 64, 0),
-    ([1500, 1500], [1500, 1700], 3, 128, 3), ([700], [1000], 1, 128, 1)])
+    ([1500, 1500], [1500, 1700], 3, 128, 3), ([700], [1000], 1, 128, 1),
+    ([3000, 1, 0, 1025] * 2, [3000, 700, 64, 1025] * 2, 8, 64, 0), ([300, 90] * 8, [300, 90] * 8, 4, 192, 5), ([40000], [40000], 12, 64, 0),
+    ([1500, 1500] * 6, [1500, 1700] * 6, 3, 128, 3), ([300], [400], 8, 128, 1)])
 def test_counts(lens_q, lens_k, heads, chunk, rest):
     rng = np.random.default_rng(sum(lens_q) + chunk)
     cols = -(-max(lens_k) // chunk)
