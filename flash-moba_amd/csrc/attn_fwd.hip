@@ -654,6 +654,15 @@ bool fwd_few_rows(const fmoba_attn_fwd_args &a);  // its variant for calls with 
 size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a);
 int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s);
 
+// Mean length of the sequence that a row belongs to, of `batch` sequences of `total` rows whose longest has `longest` and the others as many as each other (the
+// least that it can be).
+static int64_t row_mean_length(int64_t total, int64_t longest, int64_t batch) {
+  longest = std::min(longest, total);
+  if (batch <= 1 || longest <= 0) return longest;
+  const double rest = (double)(total - longest);
+  return (int64_t)(((double)longest * (double)longest + rest * rest / (double)(batch - 1)) / (double)total);
+}
+
 // Which form runs.  The row-block form multiplies every row of a 128-row block with every chunk that
 // any of its rows selected, the column form only the selected pairs but pays a partial result per
 // visit: the first wins while a row selects more than about a fifth of the chunks it may see (64-key blocks) or
@@ -669,7 +678,12 @@ static bool fwd_use_rows(const fmoba_attn_fwd_args &a) {
   if (a.head_dim > 128) {
     const int64_t partials = (int64_t)a.total_q * a.heads * fwd_partial_cap(a);
     if (!fwd_combine_fits(a) || partials >= ((int64_t)1 << 31) || partials * (int64_t)(a.head_dim * fwd_part_size(a.head_dim) + 16) > kWidePartialBytes) return true;
-    return fwd_rows_direct(a) && (int64_t)a.heads * (a.total_q / 128 + a.batch) >= kFwdRowsWideBlocks && chunks_per_row * (wide_keys ? kFwdRowsDensityWide128 : kFwdRowsDensityWide64) >= seen * 10;
+    // (What a row may see goes by its own sequence's length, of which the longest is known, and by where its queries lie in it.  By the mean length and as
+    // if every call were a whole prompt, columns against rows: one sequence of 25592 tokens with five short ones, 8 heads, top-k 3 of 256-key chunks 1452
+    // against 2956 us, parts of prompts of 1451 rows against 11481 keys, 32 over 4 heads, top-k 7 of 64-key chunks 259 against 670.)
+    const int64_t kl = row_mean_length(a.total_k, a.max_seqlen_k, a.batch), ql = std::min(kl, row_mean_length(a.total_q, a.max_seqlen_q, a.batch));
+    const int64_t seen_wide = std::max<int64_t>(1, (a.is_causal ? kl - ql / 2 : kl) / a.lg_block_n);
+    return fwd_rows_direct(a) && (int64_t)a.heads * (a.total_q / 128 + a.batch) >= kFwdRowsWideBlocks && chunks_per_row * (wide_keys ? kFwdRowsDensityWide128 : kFwdRowsDensityWide64) >= seen_wide * 10;
   }
   return chunks_per_row * (wide_keys ? kFwdRowsDensity128 : kFwdRowsDensity64) >= seen * 10;
 }

@@ -20,6 +20,17 @@ def test_wide_forward_lines(lens, chunk, topk, heads, rows):
     assert hip.load_library().fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == rows
 
 
+# the density is that of the rows: most of them in the longest sequence of a batch, the last of their sequences in a part of a prompt
+@pytest.mark.parametrize("lens_q,lens_k,chunk,topk,heads,rows", [
+    ([637, 12295], None, 128, 13, 16, 0), ([6466, 6466], None, 128, 13, 16, 1), ([2789, 25592, 2556, 1271, 1642, 2226], None, 256, 3, 8, 0),
+    ([1451, 156, 137], [11481, 479, 1317], 64, 7, 32, 0), ([1024, 1024], [4096, 4096], 128, 9, 32, 0), ([1024, 1024], [4096, 4096], 128, 11, 32, 1)])
+def test_wide_forward_lines_of_uneven_calls(lens_q, lens_k, chunk, topk, heads, rows):
+    lens_k = lens_k or lens_q
+    f = fwd_args(lens_k, chunk, topk, heads=heads, D=256)
+    f.total_q, f.max_seqlen_q = sum(lens_q), max(lens_q)
+    assert hip.load_library().fmoba_attn_fwd_uses_row_blocks(ctypes.byref(f)) == rows
+
+
 # keys or values further apart than the kernel's 32-bit offsets reach stay with the columns
 @pytest.mark.parametrize("field", ["k_row_stride", "v_row_stride"])
 def test_wide_forward_of_rows_far_apart(field):
