@@ -827,11 +827,12 @@ static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, i
   hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap);
   return 0;
 }
-// Workgroups of 64 rows up to which four sets share a walk (head dimensions up to 64): one for every compute unit.  Their rings leave a unit
-// room for one such workgroup; two sets, of which two workgroups fit, take the calls above.  Forward: 2048 tokens, 8 heads (256 of them) 31.8 -> 30.2 us,
-// 4096 tokens, 4 heads (256) 49.2 -> 45.3, 400 rows against 6000 keys, 8 heads (56) 64.7 -> 56.6, 632 rows against 24924 keys, 8 heads (88) 200 -> 164; 3072
-// tokens in two sequences, 8 heads (384) 33.8 -> 37.4.
-constexpr int kRowsFourSets = 256;
+// Four sets share a walk (head dimensions up to 64) where the workgroups of 64 rows are no more than the compute units, as their rings leave a unit
+// room for one (two sets, of which two workgroups fit, take the calls above), and the longest walk is 16 steps or more: four sets take longer to start and to add
+// up.  Forward, two sets and four: 2048 tokens, 8 heads (256 workgroups) 31.8 -> 30.2 us, 4096 tokens, 4 heads (256) 49.2 -> 45.3, 400 rows against 6000 keys,
+// 8 heads (56) 64.7 -> 56.6, 632 rows against 24924 keys, 8 heads (88) 200 -> 164; 3072 tokens in two sequences, 8 heads (384) 33.8 -> 37.4.  Two sequences, 4
+// heads, top-k 3 of 64-key chunks: of 1024 tokens 24.7 -> 24.2, 896 23.5 -> 23.8, 640 21.3 -> 22.5, 128 14.9 -> 16.5.
+constexpr int kRowsFourSets = 256, kRowsFourSetsKeys = 1024;
 // Which workgroup, by the 128-row blocks of the call and the mean length of its sequences:
 // - two waves of 32 rows and two sets of them where 128-row blocks come to about one per compute unit (two at head dimensions up
 //   to 64, where two such workgroups fit a unit): the walks are half as long and there are twice as many of them.  Against one
@@ -843,12 +844,16 @@ constexpr int kRowsFourSets = 256;
 //   on average 34.8 -> 31.2 us, of 540 50 -> 43, of 1483 93.3 -> 89.7; one sequence of 8192 tokens 206 -> 206, 16384 765 -> 811.  (At
 //   head dimension 128 the rings leave room for two workgroups of either kind, and the small ones have half of the waves: 73 -> 99.)
 // - four waves and one set otherwise.
+static int rows_sets(const fmoba_attn_fwd_args &a) {
+  if (a.head_dim <= 64 && a.max_seqlen_k >= kRowsFourSetsKeys && a.heads * (((int64_t)a.total_q + 63 * a.batch) / 64) <= kRowsFourSets) return 4;
+  return (int64_t)a.heads * (a.total_q / 128 + a.batch) <= (a.head_dim > 64 ? 288 : 544) ? 2 : 1;
+}
 template <typename T, int HD>
 static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
-  const int64_t blocks = (int64_t)a.heads * (a.total_q / 128 + a.batch);
+  const int sets = rows_sets(a);
   if constexpr (HD <= 64)
-    if (a.heads * (((int64_t)a.total_q + 63 * a.batch) / 64) <= kRowsFourSets) return launch_rows_split<T, HD, 2, 4>(a, bm, nw, s);
-  if (blocks <= (HD > 64 ? 288 : 544)) return launch_rows_split<T, HD, 2, 2>(a, bm, nw, s);
+    if (sets == 4) return launch_rows_split<T, HD, 2, 4>(a, bm, nw, s);
+  if (sets == 2) return launch_rows_split<T, HD, 2, 2>(a, bm, nw, s);
   if constexpr (HD <= 64)
     if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1>(a, bm, nw, s);
   return launch_rows_split<T, HD, 4, 1>(a, bm, nw, s);
@@ -937,3 +942,5 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
 }
 
 }  // namespace fmoba
+
+extern "C" int32_t fmoba_attn_fwd_row_sets(const fmoba_attn_fwd_args *a) { return a != nullptr && a->head_dim > 0 && a->head_dim <= 128 && fmoba::fwd_rows_direct(*a) ? fmoba::rows_sets(*a) : 1; }

@@ -61,3 +61,10 @@ def test_wide_heads_partial_results_are_bounded_by_the_sequence():
                                             ([1024], 8, 1), ([1024], 7, 0), ([2304], 8, 0)])
 def test_visits_in_lds(lens, heads, lds):
     assert H.load_library().fmoba_csc_row_visits_in_lds(ctypes.byref(fwd_args(lens, 128, 16, heads=heads))) == lds
+
+
+# four sets of waves share a walk of 16 steps and more in calls of few row blocks of narrow heads: not the short ones, which they only make longer
+@pytest.mark.parametrize("lens,heads,D,sets", [([64] * 2, 4, 64, 2), ([896] * 2, 4, 64, 2), ([1023], 8, 64, 2), ([1024], 8, 64, 4), ([1024] * 2, 8, 64, 2), ([2048], 8, 64, 4),
+                                               ([2112], 8, 64, 2), ([1024], 8, 72, 2), ([8192], 8, 32, 2), ([8832], 8, 64, 1), ([4480], 8, 128, 2), ([4736], 8, 128, 1)])
+def test_sets_of_a_walk(lens, heads, D, sets):
+    assert H.load_library().fmoba_attn_fwd_row_sets(ctypes.byref(fwd_args(lens, 64, 16, heads=heads, D=D))) == sets

@@ -49,11 +49,41 @@ def test_row_blocks_repeat_to_the_last_bit():
         assert all(torch.equal(run(), first) for _ in range(200))
 
 
-# Four sets over 64 rows (up to 256 workgroups): walks of fewer steps than sets, of one more, of every remainder, queries that are the last rows of
-# longer sequences' worth of steps; two sets on the other side of the line
+# Up to 256 workgroups of 64 rows, with a sequence of 1024 keys and more (four sets) and without one (two)
 @pytest.mark.parametrize("lens,H,Hk,D,chunk,topk", [
     ([63, 64, 128, 129, 192, 193, 256, 257, 320, 321, 385], 2, 1, 64, 64, 3), ([449, 513, 577], 4, 4, 48, 64, 9), ([4096], 4, 2, 64, 128, 6),
     ([900], 1, 1, 16, 256, 2), ([700, 1, 640, 330], 16, 8, 64, 64, 4), ([1024, 2048], 8, 8, 32, 128, 4)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_row_block_workgroups_of_four_sets(lens, H, Hk, D, chunk, topk, dtype):
     test_row_block_workgroups(lens, H, Hk, D, chunk, topk, dtype)
+
+
+# Four sets over 64 rows: walks of fewer steps than sets, of one more, of every remainder beside a long one; queries that are the last rows of longer
+# sequences, with more than 32 and 64 turns per set (a set's entries are read 64 turns at a time, every 32); a last chunk cut short
+@pytest.mark.parametrize("lens_q,lens_k,H,Hk,D,chunk,topk", [
+    ([63, 64, 128, 129, 192, 193, 256, 257, 320, 321, 385, 1100], None, 2, 1, 64, 64, 9), ([449, 513, 1077], None, 4, 4, 48, 64, 9), ([2100], None, 1, 1, 16, 256, 4),
+    ([100, 1, 64], [8300, 70, 1500], 2, 2, 64, 64, 40), ([130], [18000], 2, 1, 32, 128, 60), ([65, 300], [1025, 300], 8, 8, 64, 128, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal", [True, False])
+def test_row_block_workgroups_of_four_sets_over_long_walks(lens_q, lens_k, H, Hk, D, chunk, topk, dtype, causal):
+    lens_k = lens_k or lens_q
+    g = torch.Generator(device="cuda").manual_seed(sum(lens_k) + D)
+    mk = lambda n, h: torch.randn((n, h, D), generator=g, device="cuda").to(dtype)
+    q, k, v = mk(sum(lens_q), H), mk(sum(lens_k), Hk), mk(sum(lens_k), Hk)
+    cu_q, cu_k = ([0] + [int(x) for x in np.cumsum(lens)] for lens in (lens_q, lens_k))
+    args = (*(torch.tensor(x, dtype=torch.int32, device="cuda") for x in (cu_q, cu_k)), max(lens_q), max(lens_k))
+    out = flash_moba.flash_moba_varlen_func(q, k, v, *args, chunk, topk, causal=causal)
+    assert hip.last_fwd_row_blocks()
+    off, nnz, rows = flash_moba.flash_topk_varlen_func(q, k, *args, topk, chunk, causal=causal)
+    want = torch.zeros_like(q, dtype=torch.float32)
+    for b, (n, m) in enumerate(zip(lens_q, lens_k)):
+        for h in range(H):
+            seen = torch.zeros(n, m, dtype=torch.bool, device="cuda")
+            for c in range(-(-m // chunk)):
+                lo = int(off[b, h, c])
+                seen[rows[lo:lo + int(nnz[b, h, c])].long(), c * chunk:(c + 1) * chunk] = True
+            if causal:
+                seen &= torch.arange(m, device="cuda")[None] <= torch.arange(m - n, m, device="cuda")[:, None]
+            s = q[cu_q[b]:cu_q[b + 1], h].float() @ k[cu_k[b]:cu_k[b + 1], h // (H // Hk)].float().T * D ** -0.5
+            want[cu_q[b]:cu_q[b + 1], h] = torch.softmax(s.masked_fill(~seen, float("-inf")), -1).nan_to_num(0.0) @ v[cu_k[b]:cu_k[b + 1], h // (H // Hk)].float()
+    assert_close("out", out, want, 2e-2, 1e-2)  # (the bound of the other attention tests)
