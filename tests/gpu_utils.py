@@ -96,3 +96,27 @@ def dense_ref_one_head(q, k, v, dout, km, chunk, topk, row_block=2048, sel_overr
     out = torch.cat(outs)
     dq, dk, dv = torch.autograd.grad(out, (qf, kf, vf), dout.float())
     return out.detach(), dq, dk, dv, sel, gate
+
+
+def pattern_forward(q, k, v, cu_q, cu_k, off, nnz, rows, chunk, causal):
+    """out (fp32) and lse of attention over the lists of a pattern, in fp32, a head at a time; queries are the last rows of their sequence.  Rows that see
+    nothing: 0 and +inf."""
+    H, D, grp = q.shape[1], q.shape[2], q.shape[1] // k.shape[1]
+    off, nnz = off.cpu(), nnz.cpu()
+    out, lse = torch.zeros_like(q, dtype=torch.float32), torch.full((H, q.shape[0]), float("inf"), device=q.device)
+    for b in range(len(cu_q) - 1):
+        n, m = cu_q[b + 1] - cu_q[b], cu_k[b + 1] - cu_k[b]
+        visible = torch.ones(n, m, dtype=torch.bool, device=q.device)
+        if causal:
+            visible = torch.arange(m, device=q.device)[None] <= torch.arange(m - n, m, device=q.device)[:, None]
+        for h in range(H):
+            seen = torch.zeros_like(visible)
+            for c in range(-(-m // chunk)):
+                lo = int(off[b, h, c])
+                seen[rows[lo:lo + int(nnz[b, h, c])].long(), c * chunk:(c + 1) * chunk] = True
+            s = q[cu_q[b]:cu_q[b + 1], h].float() @ k[cu_k[b]:cu_k[b + 1], h // grp].float().T * D ** -0.5
+            s = s.masked_fill(~(seen & visible), float("-inf"))
+            out[cu_q[b]:cu_q[b + 1], h] = torch.softmax(s, -1).nan_to_num(0.0) @ v[cu_k[b]:cu_k[b + 1], h // grp].float()
+            x = torch.logsumexp(s, -1)
+            lse[h, cu_q[b]:cu_q[b + 1]] = torch.where(x == float("-inf"), float("inf"), x)
+    return out, lse

@@ -5,7 +5,7 @@ import torch
 
 import flash_moba
 from flash_moba import flash_moba_hip as hip
-from gpu_utils import assert_close
+from gpu_utils import assert_close, pattern_forward
 from test_gpu_item_order import _reference
 
 pytestmark = pytest.mark.gpu
@@ -74,16 +74,6 @@ def test_row_block_workgroups_of_four_sets_over_long_walks(lens_q, lens_k, H, Hk
     args = (*(torch.tensor(x, dtype=torch.int32, device="cuda") for x in (cu_q, cu_k)), max(lens_q), max(lens_k))
     out = flash_moba.flash_moba_varlen_func(q, k, v, *args, chunk, topk, causal=causal)
     assert hip.last_fwd_row_blocks()
-    off, nnz, rows = flash_moba.flash_topk_varlen_func(q, k, *args, topk, chunk, causal=causal)
-    want = torch.zeros_like(q, dtype=torch.float32)
-    for b, (n, m) in enumerate(zip(lens_q, lens_k)):
-        for h in range(H):
-            seen = torch.zeros(n, m, dtype=torch.bool, device="cuda")
-            for c in range(-(-m // chunk)):
-                lo = int(off[b, h, c])
-                seen[rows[lo:lo + int(nnz[b, h, c])].long(), c * chunk:(c + 1) * chunk] = True
-            if causal:
-                seen &= torch.arange(m, device="cuda")[None] <= torch.arange(m - n, m, device="cuda")[:, None]
-            s = q[cu_q[b]:cu_q[b + 1], h].float() @ k[cu_k[b]:cu_k[b + 1], h // (H // Hk)].float().T * D ** -0.5
-            want[cu_q[b]:cu_q[b + 1], h] = torch.softmax(s.masked_fill(~seen, float("-inf")), -1).nan_to_num(0.0) @ v[cu_k[b]:cu_k[b + 1], h // (H // Hk)].float()
-    assert_close("out", out, want, 2e-2, 1e-2)  # (the bound of the other attention tests)
+    pattern = flash_moba.flash_topk_varlen_func(q, k, *args, topk, chunk, causal=causal)
+    # (the bound of the other attention tests)
+    assert_close("out", out, pattern_forward(q, k, v, cu_q, cu_k, *pattern, chunk, causal)[0], 2e-2, 1e-2)

@@ -7,7 +7,7 @@ import torch
 
 import flash_moba
 from flash_moba import flash_moba_hip as hip
-from gpu_utils import assert_close
+from gpu_utils import assert_close, pattern_forward
 from test_form_rules import fwd_args
 from test_gpu_item_order import _reference
 
@@ -181,3 +181,25 @@ def test_wide_row_blocks_non_finite_values(at, feature, value, D, dtype):
         lo, n = int(pattern[0][b, h, c]), int(pattern[1][b, h, c])
         hit[cu[b] + pattern[2][lo:lo + n].long(), h] = True
     assert hit.any() and not hit.all() and torch.equal(rows[0][~hit], plain[~hit])
+
+
+# later parts of prompts, more queries than keys (the first rows see nothing: out 0, lse +inf, whole blocks of them), no causal limit; a last chunk cut short
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens_q,lens_k", [([200, 1, 130], [1000, 65, 131]), ([700, 300, 40], [150, 300, 1]), ([129, 257], [2100, 64])])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D,chunk", [(256, 64), (192, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_row_blocks_of_unequal_lengths(lens_q, lens_k, causal, D, chunk, dtype):
+    g = torch.Generator(device="cuda").manual_seed(sum(lens_k) + D)
+    q, k, v = (torch.randn((sum(n), h, D), generator=g, device="cuda").to(dtype) for n, h in ((lens_q, 4), (lens_k, 2), (lens_k, 2)))
+    cu_q, cu_k = ([0] + [int(x) for x in np.cumsum(lens)] for lens in (lens_q, lens_k))
+    where = (*(torch.tensor(x, dtype=torch.int32, device="cuda") for x in (cu_q, cu_k)), max(lens_q), max(lens_k))
+    pattern = flash_moba.flash_topk_varlen_func(q, k, *where, 6, chunk, causal=causal)
+    out, lse, _, _ = hip.moba_varlen_fwd(q, k, v, None, *pattern, *where[:2], None, None, None, *where[2:], 0.0, D ** -0.5, False, causal, 0.0, False, 128, chunk, None,
+                                         _fwd_mode=2)
+    assert hip.last_fwd_row_blocks()
+    want, want_lse = pattern_forward(q, k, v, cu_q, cu_k, *pattern, chunk, causal)
+    assert_close("out", out, want, 2e-2, 1e-2)  # (the bound of the other attention tests)
+    assert torch.equal(lse.isinf(), want_lse.isinf()) and torch.equal(out[(want_lse.T == float("inf"))], torch.zeros_like(out[(want_lse.T == float("inf"))]))
+    # (256 products and 1100 probabilities per sum in 32 bits, in another order; scores of up to 2^3 in magnitude)
+    assert (lse - want_lse).nan_to_num(0.0).abs().max() <= 1e-3
