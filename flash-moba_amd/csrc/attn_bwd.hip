@@ -1216,7 +1216,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
 //
 // What bounds it: the misses a unit can have in flight (dS pieces of 64 to 512 bytes at scattered places), and in calls of few
 // workgroups the longest walk.  Head dimensions 65 to 128: four waves with two row tiles each, two workgroups per unit and
-// groups of two steps; one workgroup of eight such waves per unit (groups of four steps, 512 rows) read half of the K tiles
+// groups of two steps; from 97 on eight waves of one tile where the walks are few and long (run_bwd draws the line).  One workgroup of eight
+// waves of two tiles per unit (groups of four steps, 512 rows) read half of the K tiles
 // but met at one barrier and left no unit a second walk: 65536 tokens in eight sequences, top-k 32 of 64-key chunks
 // 1634 -> 1556 us, 24571 tokens, 32 over 8 heads 691 -> 624, 12037 tokens, heads of 96 182 -> 124 (with the order of the items
 // below; tiles of 96 features instead of 128: 129 -> 115), 2 x 4096 tokens 143 -> 125.  Up to 64: eight waves of one tile (with two tiles in four waves 4096 tokens 58 -> 67 us).

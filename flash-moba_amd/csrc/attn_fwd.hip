@@ -42,6 +42,8 @@ constexpr int kFwdRowsDensity64 = 50, kFwdRowsDensity128 = 27;
 // blocks, 2 x 4096 tokens 0.24 176 against 188, 0.48 252 against 190, 8 x 2048 tokens 0.38 481 against 451, 16384 tokens 0.25 874 against 1169, 0.5 1552
 // against 1200.  From one 128-row block per compute unit on: fewer of them leave units idle for the length of a walk.
 constexpr int kFwdRowsDensityWide64 = 57, kFwdRowsDensityWide128 = 28, kFwdRowsWideBlocks = 256;
+// Partial results of wide heads that a call may ask for, counted without the padding of part_row_elems (up to 6 % more is allocated), as the line lay
+// before rows were padded: no call changes its form by it.
 constexpr int64_t kWidePartialBytes = (int64_t)16 << 30;
 
 struct FwdWs {

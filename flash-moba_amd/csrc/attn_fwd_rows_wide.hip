@@ -4,17 +4,6 @@
 
 namespace fmoba {
 
-// a * b + c for a and b below 2^24: a full-rate instruction
-__device__ __forceinline__ uint32_t mad24_u32(uint32_t a, uint32_t b, uint32_t c) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t d;
-  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(b), "v"(c));
-  return d;
-#else
-  return a * b + c;
-#endif
-}
-
 // 128 rows per workgroup, four waves of 32 rows and 512 registers, one workgroup per compute unit: a wave's 256 features of O^T are half of the
 // ordinary registers, its Q rows lie in accumulation registers, and the rings of two K and two V tiles take 128 KB.  With one wave per SIMD
 // nothing runs under the softmax unless it stands there, so a step is two runs of 32 products: S of the next step, with the rescaling

@@ -783,6 +783,16 @@ __device__ __forceinline__ uint32_t mul24_u32(uint32_t a, uint32_t b) {
   return a * b;
 #endif
 }
+// a * b + c likewise (a and b below 2^24, b the same in every lane)
+__device__ __forceinline__ uint32_t mad24_u32(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t d;
+  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(b), "v"(c));
+  return d;
+#else
+  return a * b + c;
+#endif
+}
 // 64 lanes x 4 bytes to LDS bytes [lds_base, lds_base + 256), in the same way.  For a value that other loads are issued behind and that is wanted
 // before them: in a register it would be one that the compiler may copy or spill before it has arrived.
 __device__ __forceinline__ void global_to_lds4(const void *g, uint32_t lds_base) {
@@ -804,7 +814,8 @@ __device__ __forceinline__ void wait_all_loads() {
 #endif
 }
 // Elements of a partial row (of the forward's output or of dQ) of `dim` features of `size` bytes: whole 64-byte pieces, written to their end.  A store past the
-// caches that covers a part of such a piece makes the memory read it first: with rows of exactly `dim` features 7346 tokens, 32 heads of 80,
+// caches that covers a part of such a piece makes the memory read it first (and workspaces are larger by the padding: heads of 40 in 16 bits 1.6 times, of 8 four
+// times, of 136 in 32 bits 1.06 times): with rows of exactly `dim` features 7346 tokens, 32 heads of 80,
 // top-k 2 of 64-key chunks, backward 649 -> 265 us, 8192 tokens, 16 heads of 112, top-k 4 of 128-key chunks 381 -> 213.
 __host__ __device__ constexpr int part_row_elems(int dim, int size) { return (dim * size + 63) / 64 * 64 / size; }
 // The dS workspace of the backward (16-bit): tiles of 32 consecutive positions of the row-index array; inside a tile
