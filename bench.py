@@ -107,15 +107,15 @@ MEASURED_TRAFFIC_BYTES = {
     ("headline", "attn_fwd_rows_kernel"): 1.249e9,
     ("headline", "attn_bwd_dkdv_kernel"): 7.353e9,
     ("headline", "attn_bwd_dq_kernel"): 5.785e9,
-    ("c2", "attn_fwd_col_kernel"): 4.320e8,
-    ("c3", "attn_fwd_col_kernel"): 7.551e9,
-    ("c3", "attn_bwd_dkdv_partials_kernel"): 1.172e10,
-    ("c5", "attn_fwd_col_kernel"): 3.719e10,
-    ("c5", "attn_bwd_dkdv_partials_kernel"): 6.140e10,
-    ("sweep16k", "attn_fwd_col_kernel"): 2.132e9,
-    ("sweep16k", "attn_bwd_dkdv_partials_kernel"): 2.557e9,
-    ("sweep64k", "attn_fwd_col_kernel"): 8.810e9,
-    ("sweep64k", "attn_bwd_dkdv_partials_kernel"): 1.406e10,
+    ("c2", "attn_fwd_col_kernel"): 4.310e8,
+    ("c3", "attn_fwd_col_kernel"): 7.547e9,
+    ("c3", "attn_bwd_dkdv_partials_kernel"): 1.169e10,
+    ("c5", "attn_fwd_col_kernel"): 3.717e10,
+    ("c5", "attn_bwd_dkdv_partials_kernel"): 6.134e10,
+    ("sweep16k", "attn_fwd_col_kernel"): 2.131e9,
+    ("sweep16k", "attn_bwd_dkdv_partials_kernel"): 2.565e9,
+    ("sweep64k", "attn_fwd_col_kernel"): 8.825e9,
+    ("sweep64k", "attn_bwd_dkdv_partials_kernel"): 1.409e10,
 }
 
 
