@@ -5,7 +5,8 @@ import torch
 
 import flash_moba
 from flash_moba import flash_moba_hip as hip
-from gpu_utils import assert_close, pattern_forward
+from gpu_utils import assert_close
+from gpu_utils import pattern_forward
 from test_gpu_item_order import _reference
 
 pytestmark = pytest.mark.gpu

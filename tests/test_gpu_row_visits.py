@@ -10,13 +10,11 @@ from flash_moba import flash_moba_hip as hip
 pytestmark = pytest.mark.gpu
 
 
-# atomics in memory and (the last five) counts in LDS; ranges of rows that end inside a sequence, sequences of no rows, of one; more than
+# Atomics in memory; ranges of rows that end inside a sequence, sequences of no rows, of one; more than
 # 512 columns; lists of more than 512 entries, unequal in pairs; columns whose last key block is cut short; rows of no sequence
 @pytest.mark.parametrize("lens_q,lens_k,heads,chunk,rest", [
     ([3000, 1, 0, 1025], [3000, 700, 64, 1025], 2, 64, 0), ([300, 90], [300, 90], 4, 192, 5), ([40000], [40000], 8, 64, 0),
-    ([1500, 1500], [1500, 1700], 3, 128, 3), ([700], [1000], 1, 128, 1),
-    ([3000, 1, 0, 1025] * 2, [3000, 700, 64, 1025] * 2, 8, 64, 0), ([300, 90] * 8, [300, 90] * 8, 4, 192, 5), ([40000], [40000], 12, 64, 0),
-    ([1500, 1500] * 6, [1500, 1700] * 6, 3, 128, 3), ([300], [400], 8, 128, 1)])
+    ([1500, 1500], [1500, 1700], 3, 128, 3), ([700], [1000], 1, 128, 1)])
 def test_counts(lens_q, lens_k, heads, chunk, rest):
     rng = np.random.default_rng(sum(lens_q) + chunk)
     cols = -(-max(lens_k) // chunk)
@@ -46,3 +44,14 @@ def test_counts(lens_q, lens_k, heads, chunk, rest):
                                                      torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     assert np.array_equal(counts[:-1].cpu().numpy().reshape(total, heads), want) and int(counts[-1]) == want.max()
+
+
+# the same counted in LDS: many pairs of the longest sequence's length, or lists that are short
+@pytest.mark.parametrize("lens_q,lens_k,heads,chunk,rest", [
+    ([3000, 1, 0, 1025] * 2, [3000, 700, 64, 1025] * 2, 8, 64, 0), ([300, 90] * 8, [300, 90] * 8, 4, 192, 5), ([40000], [40000], 12, 64, 0),
+    ([1500, 1500] * 6, [1500, 1700] * 6, 3, 128, 3), ([300], [400], 8, 128, 1)])
+def test_counts_in_lds(lens_q, lens_k, heads, chunk, rest):
+    f = hip.AttnFwdArgs()
+    f.heads, f.total_q, f.max_seqlen_q, f.max_cols = heads, sum(lens_q) + rest, max(lens_q), -(-max(lens_k) // chunk)
+    assert hip.load_library().fmoba_csc_row_visits_in_lds(ctypes.byref(f)) == 1
+    test_counts(lens_q, lens_k, heads, chunk, rest)

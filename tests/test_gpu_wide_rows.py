@@ -7,7 +7,8 @@ import torch
 
 import flash_moba
 from flash_moba import flash_moba_hip as hip
-from gpu_utils import assert_close, pattern_forward
+from gpu_utils import assert_close
+from gpu_utils import pattern_forward
 from test_form_rules import fwd_args
 from test_gpu_item_order import _reference
 
