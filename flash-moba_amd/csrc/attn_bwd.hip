@@ -127,7 +127,7 @@ struct DkdvSmem {
   static constexpr size_t tile = (size_t)64 * HD * 2;        // 64 gathered rows of Q or dO, swizzled (tile_swz)
   static constexpr size_t oQ = 0;                             // [NBUF]
   static constexpr size_t odO = oQ + NBUF * tile;             // [NBUF]
-  static constexpr size_t oP = odO + NBUF * tile;             // [64 rows][64 keys], piece p (8 keys) of row r at p ^ (r & 7)
+  static constexpr size_t oP = odO + NBUF * tile;             // [64 rows][64 keys], piece p (8 keys) of row r at p ^ tile_swz<64>(r)
   static constexpr size_t odS = oP + 64 * PRB;
   static constexpr size_t oOut = odS + 64 * PRB;              // partials form: [64 rows][HD], dQ part rows on their way out
   static constexpr size_t oSlot = oOut + (DQP ? (size_t)64 * HD * 2 : 0);  // int[2][64]: places of the part rows
@@ -352,8 +352,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
 #endif
       // places of this lane in the P and dS rows (and of its row in a round)
       const int fl = ft & 63, fh = fl >> 5, fli = fl & 15, frow = rt * 32 + (fl & 31), fr = (fli >> 2) + 4 * fh;
-      const uint32_t pw = (uint32_t)(frow * PRB + fh * 8), psw = (uint32_t)(frow & 7);
-      const uint32_t pread = (uint32_t)(fr * PRB + (((((fl >> 4) & 1) * 2 + ((fli & 3) >> 1)) ^ (fr & 7)) * 16) + (fli & 1) * 8);
+      const uint32_t pw = (uint32_t)(frow * PRB + fh * 8), psw = (uint32_t)tile_swz<64>(frow);
+      const uint32_t pread = (uint32_t)(fr * PRB + (((((fl >> 4) & 1) * 2 + ((fli & 3) >> 1)) ^ tile_swz<64>(fr)) * 16) + (fli & 1) * 8);
       const Round w2 = round_at(r + 2);
       const float lse2 = rid0 >= 0 ? lse * kLog2e : INFINITY, delta = del;
       if constexpr (DQP) {
@@ -422,8 +422,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
         constexpr int S4 = decltype(sc)::value;
 #pragma unroll
         for (int kk = 0; kk < NKW; ++kk) {
-          const uint32_t po = (px ^ (uint32_t)((kk0 + kk) * 64)) + (uint32_t)(S4 * 16 * PRB);
-          pb[S4 & 1][kk] = lds_tr8(po, po + 8 * PRB);
+          const uint32_t o = (uint32_t)(S4 * 16 * PRB);
+          pb[S4 & 1][kk] = lds_tr8(tile_tr_addr<64>(px, kk0 + kk) + o, tile_tr_addr8<64>(px, kk0 + kk) + o);
         }
 #pragma unroll
         for (int d = 0; d < NDW; ++d) {
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
             for (int d = 0; d < NDW; ++d) dq[d] = mfma32<T>(ktf[d][2 * S + u], sf[S & 1][u], dq[d]);
           __builtin_amdgcn_sched_barrier(0);
         });
-        // rows through LDS, so that a row's 16-byte pieces leave together (piece p of row r at p ^ (r & 7))
+        // rows through LDS, so that a row's 16-byte pieces leave together (piece p of row r at p ^ tile_swz<64>(r))
         const uint32_t ldsOut = lds + (uint32_t)SM::oOut;
 #pragma unroll
         for (int d = 0; d < NDW; ++d)
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
         for (int v0 = 0; v0 < 64 * VPR; v0 += 256) {
           const int v = v0 + ft, row = v / VPR, pcs = v - row * VPR;
           const uint32_t p = (uint32_t)sSlot[(r & 1) * 64 + row];
-          const Pack8 x = lds_read16(ldsOut + (uint32_t)(row * RB) + (((uint32_t)pcs ^ (uint32_t)(row & 7)) * 16u));
+          const Pack8 x = lds_read16(ldsOut + (uint32_t)(row * RB) + (((uint32_t)pcs ^ (uint32_t)tile_swz<64>(row)) * 16u));
           if (pcs * 8 < PD) st_stream16(ws.part + ((uint64_t)p * (uint32_t)PD + (uint32_t)(pcs * 8)), x);
           if (!RANKED && pcs == 0) ws.pid[p] = nb;
         }
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
         // dS of row `lane`, key groups 2 wave and 2 wave + 1: consecutive lanes write consecutive pieces of the dS tile
         Pack8 x[2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) x[u] = lds_read16(ldsdS + (uint32_t)(lane * PRB) + (((uint32_t)(2 * wave + u) ^ (uint32_t)(lane & 7)) * 16u));
+        for (int u = 0; u < 2; ++u) x[u] = lds_read16(ldsdS + (uint32_t)(lane * PRB) + (((uint32_t)(2 * wave + u) ^ (uint32_t)tile_swz<64>(lane)) * 16u));
         arrived();
         if (lane < w0.n) {
           uint16_t *dst = ds_piece(ws.ds, w0.pos, lane, (koff >> 3) + 2 * wave, Bn >> 3);

@@ -615,6 +615,11 @@ __device__ __forceinline__ Pack8 zero_pack8() {
 // instruction writes 64 lanes x 16 bytes to consecutive addresses), swizzled instead of padded
 // ------------------------------------------------------------------------------------
 // piece c of tile row r is stored at piece c ^ tile_swz<HD>(r)
+// The LDS delivers 256 bytes a clock where sixteen lanes of a 16-byte read, or 32 lanes of a transposing 8-byte read, meet 64 different banks
+// (64 lanes x 16 bytes: 4.2 clocks, one two-way meeting: 8).  Rows of 128 bytes lie two to a sweep of the banks, so eight pieces have to tell
+// the rows of a parity among sixteen apart (bits 1 to 3), and bit 1, which parts rows of a parity inside a transposing read's four, moves the
+// upper half of the pieces.  Told apart by bits 1 and 2 alone: row reads 8 clocks, the P and dS tiles of the dK/dV pass (piece ^ row % 8)
+// 8 and 4 instead of 4.2 and 2; 8191 tokens of short documents, heads of 64, training step 137.5 -> 136.4 us, 2 x 4096 tokens 475.9 -> 471.7.
 template <int HD>
 __device__ __forceinline__ int tile_swz(int r) {
   if constexpr (HD == 96)
@@ -622,11 +627,11 @@ __device__ __forceinline__ int tile_swz(int r) {
   else if constexpr (HD > 64)
     return ((r & 3) << 2) | ((r >> 2) & 3);  // 16 pieces per row, one row per sweep of the banks
   else
-    return (((r >> 1) & 1) << 2) | ((r >> 2) & 1);  // 8 pieces per row, two rows per sweep
+    return (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 1) | ((r >> 2) & 1);  // 8 pieces per row, two rows per sweep
 }
 template <int HD>
 struct TileSwz {
-  static constexpr int kRow8 = HD > 64 ? 2 : 0;  // tile_swz(r + 8) ^ tile_swz(r)
+  static constexpr int kRow8 = 2;  // tile_swz(r + 8) ^ tile_swz(r)
 };
 // Operands of 32x32x16 products over the features of a row: the piece that half hh of the wave takes in k-step ks (any order does
 // that both operands share), and its address from that of step 0, which holds row * HD * 2 + (tile_frag_piece(hh, 0) ^
