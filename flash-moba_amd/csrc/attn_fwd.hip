@@ -835,6 +835,20 @@ extern "C" int fmoba_csc_max_row_visits(const fmoba_attn_fwd_args *a, int32_t *c
   return 0;
 }
 
+// the tensors and strides of a call that has keys
+static int fwd_check_tensors(const fmoba_attn_fwd_args *a) {
+  using namespace fmoba;
+  FMOBA_REQUIRE(a->k && a->v, "attn_fwd: null k/v pointer");
+  const int64_t st[] = {a->q_row_stride, a->q_head_stride, a->k_row_stride, a->k_head_stride,
+                        a->v_row_stride, a->v_head_stride, a->o_row_stride, a->o_head_stride};
+  for (int64_t x : st) FMOBA_REQUIRE(x % 8 == 0, "attn_fwd: strides must be multiples of 8 elements");
+  FMOBA_REQUIRE(a->q_row_stride < ((int64_t)1 << 31), "attn_fwd: q_row_stride must be below 2^31 elements");
+  FMOBA_REQUIRE(((uintptr_t)a->q % 16) == 0 && ((uintptr_t)a->k % 16) == 0 && ((uintptr_t)a->v % 16) == 0 && ((uintptr_t)a->out % 16) == 0,
+                "attn_fwd: q, k, v and out must be 16-byte aligned");
+  FMOBA_REQUIRE(a->max_visits_per_row > 0, "attn_fwd: max_visits_per_row must be positive");
+  return 0;
+}
+
 extern "C" int fmoba_attn_fwd(const fmoba_attn_fwd_args *a, void *stream) { return fmoba_attn_fwd_phases(a, 3, stream); }
 
 extern "C" int fmoba_attn_fwd_phases(const fmoba_attn_fwd_args *a, int32_t phases, void *stream) { return fmoba_attn_fwd_ranked(a, nullptr, phases, stream); }
@@ -855,15 +869,8 @@ extern "C" int fmoba_attn_fwd_ranked(const fmoba_attn_fwd_args *a, const uint32_
     FMOBA_LAUNCH_CHECK("attn_fwd(empty)");
     return 0;
   }
-  FMOBA_REQUIRE(a->k && a->v, "attn_fwd: null k/v pointer");
   FMOBA_REQUIRE((a->col_offsets && a->col_nnz && a->row_indices) || (a->selection_bits && fwd_use_rows(*a)), "attn_fwd: null CSC pointer");
-  const int64_t st[] = {a->q_row_stride, a->q_head_stride, a->k_row_stride, a->k_head_stride,
-                        a->v_row_stride, a->v_head_stride, a->o_row_stride, a->o_head_stride};
-  for (int64_t x : st) FMOBA_REQUIRE(x % 8 == 0, "attn_fwd: strides must be multiples of 8 elements");
-  FMOBA_REQUIRE(a->q_row_stride < ((int64_t)1 << 31), "attn_fwd: q_row_stride must be below 2^31 elements");
-  FMOBA_REQUIRE(((uintptr_t)a->q % 16) == 0 && ((uintptr_t)a->k % 16) == 0 && ((uintptr_t)a->v % 16) == 0 && ((uintptr_t)a->out % 16) == 0,
-                "attn_fwd: q, k, v and out must be 16-byte aligned");
-  FMOBA_REQUIRE(a->max_visits_per_row > 0, "attn_fwd: max_visits_per_row must be positive");
+  if (int rc = fwd_check_tensors(a)) return rc;
   FMOBA_REQUIRE(a->fwd_mode >= 0 && a->fwd_mode <= 2, "attn_fwd: fwd_mode must be 0 (automatic), 1 (columns) or 2 (row blocks)");
   FMOBA_REQUIRE(a->fwd_mode != 2 || fwd_rows_feasible(*a), "attn_fwd: the row-block form does not take this shape (more than %d chunks or %d keys per sequence)",
                 32 * 128, 64 * 4096);
@@ -891,5 +898,40 @@ extern "C" int fmoba_attn_fwd_ranked(const fmoba_attn_fwd_args *a, const uint32_
   int rc = a->dtype == FMOBA_DTYPE_BF16 ? run_fwd<bf16_t>(*a, ws, phases, s) : run_fwd<f16_t>(*a, ws, phases, s);
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("attn_fwd");
+  return 0;
+}
+
+namespace fmoba {
+bool pool_scores_feasible(int head_dim, int group, int rows, int batch);                                       // mean_pool.hip
+int mean_pool_with_scores(const fmoba_mean_pool_args *a, const FewGate &few, void *stream);
+void run_fwd_few_scored(const fmoba_attn_fwd_args &a, const FewGate &few, hipStream_t s);                      // attn_fwd_few.hip
+}  // namespace fmoba
+
+extern "C" size_t fmoba_attn_fwd_gated_few_bytes(const fmoba_attn_fwd_args *a) {
+  using namespace fmoba;
+  if (a == nullptr || a->total_q <= 0 || a->total_k <= 0 || a->heads <= 0 || a->heads_k <= 0 || a->batch <= 0 || a->max_seqlen_q <= 0 || a->lg_block_n <= 0) return 0;
+  if (a->fwd_mode != 0 || !fwd_rows_feasible(*a) || !fwd_few_rows(*a) || !pool_scores_feasible(a->head_dim, a->heads / a->heads_k, a->max_seqlen_q, a->batch)) return 0;
+  return fwd_align256((size_t)(a->total_k / a->lg_block_n + a->batch) * a->heads * a->max_seqlen_q * 4);
+}
+
+extern "C" int fmoba_attn_fwd_gated_few(const fmoba_mean_pool_args *m, const fmoba_attn_fwd_args *a, int32_t topk, int32_t gate_is_causal, float *scores, void *stream) {
+  using namespace fmoba;
+  if (int rc = fwd_check_common(a)) return rc;
+  FMOBA_REQUIRE(m != nullptr && scores != nullptr && m->cu_seqlens_km != nullptr, "attn_fwd_gated_few: null pointer");
+  FMOBA_REQUIRE(fmoba_attn_fwd_gated_few_bytes(a) > 0, "attn_fwd_gated_few: not a call of this form (fmoba_attn_fwd_gated_few_bytes tells)");
+  FMOBA_REQUIRE(topk >= 1 && topk <= 64, "moba_topk must be in [1, 64]");
+  FMOBA_REQUIRE(m->k == a->k && m->cu_seqlens_k == a->cu_seqlens_k && m->batch == a->batch && m->heads_k == a->heads_k && m->head_dim == a->head_dim &&
+                    m->chunk == a->lg_block_n && m->dtype == a->dtype && m->k_row_stride == a->k_row_stride && m->k_head_stride == a->k_head_stride,
+                "attn_fwd_gated_few: the two argument structs describe different problems");
+  FMOBA_REQUIRE(m->max_chunks == a->max_cols && a->max_cols == ceil_div(a->max_seqlen_k, a->lg_block_n), "attn_fwd_gated_few: max_cols is ceil(max_seqlen_k / lg_block_n)");
+  FMOBA_REQUIRE(a->q && a->out && a->softmax_lse, "attn_fwd: null q/out/lse pointer");
+  if (int rc = fwd_check_tensors(a)) return rc;
+  FewGate few;
+  few.q = reinterpret_cast<const uint16_t *>(a->q), few.cu_seqlens_q = a->cu_seqlens_q, few.cu_seqlens_km = m->cu_seqlens_km, few.scores = scores;
+  few.q_row_stride = a->q_row_stride, few.q_head_stride = a->q_head_stride;
+  few.heads = a->heads, few.group = a->heads / a->heads_k, few.rows = a->max_seqlen_q, few.topk = topk, few.is_causal = gate_is_causal;
+  if (int rc = mean_pool_with_scores(m, few, stream)) return rc;
+  run_fwd_few_scored(*a, few, (hipStream_t)stream);
+  FMOBA_LAUNCH_CHECK("attn_fwd_gated_few");
   return 0;
 }

@@ -1,19 +1,21 @@
 // Sparse attention forward for calls with a handful of query rows (decode steps): one workgroup per (query row, head)
 // streams the keys and values of the chunks the row selected, eight waves side by side, and merges their results in
-// LDS.  Reads the selection bits alone, leaves no partial result in memory and needs no second launch.
+// LDS.  Reads the selection bits, or picks the chunks itself from the scores that the pooling pass left (which spares the gate's launch),
+// leaves no partial result in memory and needs no second launch.
 //
 // Bound by memory: with one row per sequence nothing is shared, every selected chunk is read once.  Each wave has a
 // whole unit of 64 keys in flight (K and V, 32 KB at head dimension 128), one 16-byte piece per lane and load, LPR
 // consecutive lanes on the same key, so every load instruction reads whole lines.  There is nothing for the matrix cores:
 // a product with one row uses 1/32 of them, and the vector arithmetic (about 600 instructions per unit) hides under the
 // loads.  16 requests against 512 to 32768 keys, 32 over 8 heads of 128, top-k 8 of 128-key chunks: 44 us, where the
-// column form takes 113 us, its combine 6 and the lists it walks another 10.
+// column form takes 113 us, its combine 6 and the lists it walks another 10.  (Held to 128 registers, for two workgroups per unit, it spills: 105.9 ->
+// 107.0 us for the whole call, 8 requests, heads of 256 27.6 -> 30.0.)
 #include "fmoba_common.h"
 
 namespace fmoba {
 
 constexpr int kFewWaves = 8;
-constexpr int kFewMaxCols = 4096;  // chunks per sequence (the row's list of chunks lies in LDS)
+constexpr int kFewMaxCols = kFewChunks;  // (the row's list of chunks lies in LDS)
 
 // sum over the LPR consecutive lanes that share a key, in all of them
 template <int LPR>
@@ -40,12 +42,81 @@ __device__ __forceinline__ float sum_lpr(float x) {
   return x;
 }
 
-template <typename T, int HD>
-__global__ __launch_bounds__(64 * kFewWaves, 2) void attn_fwd_few_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw) {
+// The best kp of a row's nc scores and behind them chunk `self` (the row's own; below 0: none), ascending in `chunks`; returns how many.
+// One wave, a chunk per lane and place, a count is a ballot; the order is that of topk_gate_few_kernel (score descending, chunk
+// descending; a candidate needs a score above -inf), so is the selection.  The places are registers for up to 64 NJ chunks, NJ = 0: `keys` in LDS
+// (registers for 4096 chunks were 167 of them, and 72 scalars spilled, in every decode call).
+template <int NJ>
+__device__ __forceinline__ int pick_chunks(const float *scores, int64_t stride, int nc, int kp, int self, int lane, uint32_t *keys, int *chunks) {
+  // in the order of the scores; 0: no candidate
+  auto order = [&](int c, float x) { return c < nc && x + 0.f > -INFINITY ? float_order_key(x + 0.f) : 0u; };  // (-0 is +0)
+  constexpr int GRP = NJ > 0 ? NJ : 8;  // places at a time
+  const int ngrp = NJ > 0 ? 1 : (nc + GRP * 64 - 1) / (GRP * 64);
+  uint32_t key[GRP];
+  for (int g = 0; g < ngrp; ++g) {
+    float x[GRP];
+#pragma unroll
+    for (int j = 0; j < GRP; ++j) {
+      const int c = (g * GRP + j) * 64 + lane;
+      x[j] = c < nc ? scores[(int64_t)c * stride] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < GRP; ++j) {
+      key[j] = order((g * GRP + j) * 64 + lane, x[j]);
+      if constexpr (NJ == 0) keys[(g * GRP + j) * 64 + lane] = key[j];
+    }
+  }
+  auto place = [&](int g, int j) { return NJ > 0 ? key[j] : keys[(g * GRP + j) * 64 + lane]; };  // (its own lane wrote it)
+  auto count_ge = [&](uint32_t v) {
+    int n = 0;
+    for (int g = 0; g < ngrp; ++g)
+#pragma unroll
+      for (int j = 0; j < GRP; ++j) n += __popcll(__ballot(place(g, j) >= v));
+    return n;
+  };
+  // the largest cut with at least kp keys at or above it, or one with exactly kp (1: all of them, if there are no more)
+  uint32_t cut = 1u;
+  const int all = kp > 0 ? count_ge(1u) : 0;
+  if (all > kp) {
+    cut = 0u;
+    for (int bit = 31; bit >= 0; --bit) {
+      const uint32_t trial = cut | (1u << bit);
+      const int n = count_ge(trial);
+      if (n >= kp) cut = trial;
+      if (n == kp) break;
+    }
+  }
+  int excess = all > kp ? count_ge(cut) - kp : 0;  // of the keys equal to the cut, the lowest chunks go
+  int total = 0;
+  for (int g = 0; g < (all > 0 ? ngrp : 0); ++g)
+#pragma unroll
+    for (int j = 0; j < GRP; ++j) {
+      const uint32_t k = place(g, j);
+      unsigned long long eq = __ballot(k == cut);
+      const unsigned long long gt = __ballot(k > cut);
+      while (excess > 0 && eq != 0ull) {
+        eq &= eq - 1ull;
+        --excess;
+      }
+      const unsigned long long m = gt | eq;
+      if ((m >> lane) & 1ull) chunks[total + __popcll(m & ((1ull << lane) - 1ull))] = (g * GRP + j) * 64 + lane;
+      total += __popcll(m);
+    }
+  if (self >= 0) {
+    if (lane == 0) chunks[total] = self;
+    ++total;
+  }
+  return total;
+}
+
+// SCORED: the row's chunks come from the scores that the pooling pass left (FewGate), else from the gate's selection bits.
+template <typename T, int HD, bool SCORED>
+__global__ __launch_bounds__(64 * kFewWaves, 2) void attn_fwd_few_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, FewGate few) {
   constexpr int LPR = HD / 8, KPI = 64 / LPR;  // lanes per key, keys per load instruction
   constexpr int NIN = HD == 64 ? 8 : 16;       // load instructions per unit and operand
   constexpr int BK = NIN * KPI;                // keys per unit
-  __shared__ int sChunk[kFewMaxCols];
+  __shared__ int sChunk[SCORED ? 128 : kFewMaxCols];       // (top-k is at most 64)
+  __shared__ uint32_t sKeys[SCORED ? kFewMaxCols : 1];
   __shared__ int sCount;
   __shared__ float sAcc[kFewWaves][HD], sM[kFewWaves], sL[kFewWaves];
   const int h = blockIdx.x, t = blockIdx.y;
@@ -62,7 +133,18 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void attn_fwd_few_kernel(fmoba_a
   const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
 
   // ---- the chunks of the row ----
-  if (wave == 0) {
+  if constexpr (SCORED) {
+    if (wave == 0) {
+      const int row = t - q0, rp = row + Lk - Lq;  // rp: the row's place among the keys
+      const int own = few.is_causal && rp >= 0 ? rp / Bn : -1, self = row < few.rows && own < a.max_cols ? own : -1;
+      const int nc = row >= few.rows ? 0 : min(few.is_causal ? max(own, 0) : (Lk + Bn - 1) / Bn, a.max_cols);
+      const int kp = few.is_causal ? few.topk - 1 : few.topk;
+      const int64_t stride = (int64_t)few.heads * few.rows;
+      const float *sc = few.scores + ((int64_t)few.cu_seqlens_km[b] * few.heads + h) * few.rows + row;
+      const int total = nc <= 256 ? pick_chunks<4>(sc, stride, nc, kp, self, lane, sKeys, sChunk) : pick_chunks<0>(sc, stride, nc, kp, self, lane, sKeys, sChunk);
+      if (lane == 0) sCount = total;
+    }
+  } else if (wave == 0) {
     const int nwu = min(((kend + Bn - 1) / Bn + 31) >> 5, nw);
     int total = 0;
     for (int w0 = 0; w0 < nwu; w0 += 64) {
@@ -185,21 +267,27 @@ bool fwd_few_rows(const fmoba_attn_fwd_args &a) {
   return (int64_t)a.total_q * a.heads * per_row <= 4 * (int64_t)a.total_k * a.heads_k;
 }
 
-template <typename T>
-static void launch_few(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
+template <typename T, bool SCORED>
+static void launch_few(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, const FewGate &few, hipStream_t s) {
   const dim3 grid(a.heads, a.total_q), block(64 * kFewWaves);
   if (a.head_dim <= 64)
-    hipLaunchKernelGGL((attn_fwd_few_kernel<T, 64>), grid, block, 0, s, a, bm, nw);
+    hipLaunchKernelGGL((attn_fwd_few_kernel<T, 64, SCORED>), grid, block, 0, s, a, bm, nw, few);
   else if (a.head_dim <= 128)
-    hipLaunchKernelGGL((attn_fwd_few_kernel<T, 128>), grid, block, 0, s, a, bm, nw);
+    hipLaunchKernelGGL((attn_fwd_few_kernel<T, 128, SCORED>), grid, block, 0, s, a, bm, nw, few);
   else
-    hipLaunchKernelGGL((attn_fwd_few_kernel<T, 256>), grid, block, 0, s, a, bm, nw);
+    hipLaunchKernelGGL((attn_fwd_few_kernel<T, 256, SCORED>), grid, block, 0, s, a, bm, nw, few);
 }
 void run_fwd_few(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
   if (a.dtype == FMOBA_DTYPE_BF16)
-    launch_few<bf16_t>(a, bm, nw, s);
+    launch_few<bf16_t, false>(a, bm, nw, FewGate{}, s);
   else
-    launch_few<f16_t>(a, bm, nw, s);
+    launch_few<f16_t, false>(a, bm, nw, FewGate{}, s);
+}
+void run_fwd_few_scored(const fmoba_attn_fwd_args &a, const FewGate &few, hipStream_t s) {
+  if (a.dtype == FMOBA_DTYPE_BF16)
+    launch_few<bf16_t, true>(a, nullptr, 0, few, s);
+  else
+    launch_few<f16_t, true>(a, nullptr, 0, few, s);
 }
 
 }  // namespace fmoba

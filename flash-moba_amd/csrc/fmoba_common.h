@@ -864,4 +864,16 @@ static inline bool rows_near(const fmoba_attn_bwd_args &a) {
          (int64_t)a.max_seqlen_q * a.q_row_stride < (int64_t)0x7fff0000 && (int64_t)a.max_seqlen_q * a.do_row_stride < (int64_t)0x7fff0000;
 }
 
+// The gate of a call with a few query rows per sequence, shared out between its two launches: the pooling pass scores every chunk it has the mean of,
+// the attention picks a row's chunks from the scores (mean_pool.hip, attn_fwd_few.hip).
+struct FewGate {
+  const uint16_t *q;
+  const int32_t *cu_seqlens_q, *cu_seqlens_km;
+  float *scores;  // [pooled row][query head][row of the sequence, rows of them]
+  int64_t q_row_stride, q_head_stride;
+  int32_t heads, group, rows, topk, is_causal;  // group: query heads per key head; rows: the longest sequence's
+  int32_t block_heads;                          // key heads of a block of the pooling pass (set by its launch)
+};
+constexpr int kFewRows = 8, kFewChunks = 4096;  // query rows and chunks per sequence of such a call, at most
+
 }  // namespace fmoba

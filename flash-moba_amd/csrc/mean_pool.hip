@@ -17,8 +17,13 @@ struct PoolExtra {
 // grid (max_chunks, batch, ceil(vecs / 64)), block 256 = 4 waves.
 // A wave owns 64 consecutive 16-byte vectors of the (heads_k*head_dim) axis; the four
 // waves of the block split the rows of the chunk and reduce through LDS.
-template <typename T, bool MANY>
-__global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x) {
+// HD > 0 (head_dim padded to 64, 128 or 256; blocks of whole heads): the means go nowhere, the block scores the sequence's few query rows with
+// them while it has them.  Each wave takes key heads of the block; the query rows of a group's heads are the columns of one product (the one
+// of topk_gate_few_kernel: the same scores to the last bit).  What it costs hides under the other blocks' loads, the gate is no launch any more, and the
+// chunk of a lone row's own keys is not read.  Decode of 16 requests against 512 to 32768 keys, 32 over 8 heads of 128, top-k 8 of 128-key chunks 119 -> 106 us;
+// one request of 3000 keys 21.3 -> 16.6, of 60000 48.5 -> 36.5; 20 of 256 to 65536, 32 over 32 heads 740 -> 694.
+template <typename T, bool MANY, int HD>
+__global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x, FewGate few) {
   const int c = blockIdx.x, b = blockIdx.y;
   const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1];
   const int row0 = seq_start + c * a.chunk;
@@ -41,12 +46,21 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
     }
   }
   if (row0 >= seq_end) return;
+  int few_q0 = 0, few_rows = 0;
+  if constexpr (HD > 0) {  // the chunks that are candidates of the last row (with the causal rule those before its own)
+    few_q0 = few.cu_seqlens_q[b];
+    const int lq = few.cu_seqlens_q[b + 1] - few_q0;
+    few_rows = min(lq, few.rows);
+    const int rmax = few_rows - 1 + (seq_end - seq_start) - lq;
+    if (few_rows <= 0 || (few.is_causal && (rmax < 0 || c >= rmax / a.chunk))) return;
+  }
   const int n = min(a.chunk, seq_end - row0);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int vecs_per_head = a.head_dim >> 3;
   const int nvec = a.heads_k * vecs_per_head;
-  const int vec = blockIdx.z * 64 + lane;
-  const bool active = vec < nvec;
+  const int block_heads = HD > 0 ? few.block_heads : 0;
+  const int vec = HD > 0 ? blockIdx.z * block_heads * vecs_per_head + lane : blockIdx.z * 64 + lane;
+  const bool active = vec < nvec && (HD == 0 || lane < block_heads * vecs_per_head);
   const int head = active ? vec / vecs_per_head : 0;
   const int d0 = active ? (vec - head * vecs_per_head) * 8 : 0;
 
@@ -55,7 +69,7 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
   if (active) {
     const uint16_t *base = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)head * a.k_head_stride + d0;
-    int r = wave;
+    int r = wave;  // row of the chunk
     // Sixteen independent 16-byte loads in flight per lane, added up in the order of the loop of four below: with four, a chunk of 256 rows is
     // sixteen memory latencies one after the other.  For rows of up to 2 KB (forward of 3334 tokens, 8 heads, 256-key chunks 65.8 -> 62.0 us, decode of
     // 43 sequences of up to 59161 keys, 2 key heads of 64 102.9 -> 95.5, of 16 sequences, 8 key heads of 128 119.2 -> 118.6, 3072 tokens, 8 heads of 64, 128-key
@@ -98,10 +112,24 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
       for (int i = 0; i < 8; ++i) acc[i] += f0[i];
     }
   }
+  // the query rows of this wave's first key head: on their way during the reduction
+  constexpr int KS = HD > 0 ? HD / 16 : 1;
+  const int r = lane & 31, hh = lane >> 5;
+  Pack8 qf[KS];
+  auto load_q = [&](int hk) {
+    const int g = r / few.rows, row = r - g * few.rows;
+    const bool mine = g < few.group && row < few_rows && hk < a.heads_k;
+    const uint16_t *qp = few.q + (int64_t)(few_q0 + (mine ? row : 0)) * few.q_row_stride + (int64_t)(mine ? hk * few.group + g : 0) * few.q_head_stride;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = mine && hh * KS + ks < vecs_per_head ? ld_global16(qp + (hh * KS + ks) * 8) : zero_pack8();
+  };
+  if constexpr (HD > 0) load_q(blockIdx.z * block_heads + wave);
   __shared__ float red[4][64][9];
 #pragma unroll
   for (int i = 0; i < 8; ++i) red[wave][lane][i] = acc[i];
   __syncthreads();
+  __shared__ Pack8 mean[64];
+  __shared__ int pooled_row;
   if (wave == 0 && active) {
     const float nf = (float)n;
     float s[8];
@@ -111,8 +139,27 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
 #pragma unroll
     for (int i = 0; i < 4; ++i) o.w[i] = pack2<T>(s[2 * i], s[2 * i + 1]);
     const int out_row = (offsets ? before : a.cu_seqlens_km[b]) + c;
-    uint16_t *dst = reinterpret_cast<uint16_t *>(a.km) + (int64_t)out_row * a.km_row_stride + (int64_t)head * a.km_head_stride + d0;
-    *reinterpret_cast<Pack8 *>(dst) = o;
+    if constexpr (HD > 0) {
+      mean[lane] = o;
+      if (lane == 0) pooled_row = out_row;
+    } else {
+      uint16_t *dst = reinterpret_cast<uint16_t *>(a.km) + (int64_t)out_row * a.km_row_stride + (int64_t)head * a.km_head_stride + d0;
+      *reinterpret_cast<Pack8 *>(dst) = o;
+    }
+  }
+  if constexpr (HD > 0) {
+    __syncthreads();
+    for (int j = wave; j < block_heads; j += 4) {
+      const int hk = blockIdx.z * block_heads + j;
+      if (hk >= a.heads_k) break;
+      if (j != wave) load_q(hk);
+      f32x16 s;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s = mfma32<T>(mean[j * vecs_per_head + min(hh * KS + ks, vecs_per_head - 1)], qf[ks], s);  // (every row of the product is the chunk's)
+      if (hh == 0 && r < few.group * few.rows) few.scores[((int64_t)pooled_row * few.heads + (int64_t)hk * few.group) * few.rows + r] = s[0];
+    }
   }
 }
 
@@ -154,7 +201,7 @@ extern "C" int fmoba_chunk_offsets(const int32_t *cu_seqlens, int32_t *cu_seqlen
 }
 
 // `extra`: cu_km and clear_* of PoolExtra
-static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &extra, void *stream) {
+static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &extra, void *stream, const fmoba::FewGate *few = nullptr) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "mean_pool: null args");
   FMOBA_REQUIRE(a->dtype == FMOBA_DTYPE_F16 || a->dtype == FMOBA_DTYPE_BF16, "mean_pool: only fp16 and bf16 are supported");
@@ -172,9 +219,21 @@ static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &
   FMOBA_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "mean_pool: batch or heads*dim too large for the launch grid");
   hipStream_t s = (hipStream_t)stream;
   const bool many = a->chunk > 64 && nvec <= 128;  // (the reasons stand at its loop)
-  auto kern = a->dtype == FMOBA_DTYPE_BF16 ? (many ? mean_pool_kernel<bf16_t, true> : mean_pool_kernel<bf16_t, false>)
-                                          : (many ? mean_pool_kernel<f16_t, true> : mean_pool_kernel<f16_t, false>);
-  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, *a, extra);
+  const int hd = few == nullptr ? 0 : a->head_dim <= 64 ? 64 : a->head_dim <= 128 ? 128 : 256;
+  FewGate scored{};
+  if (few != nullptr) {
+    scored = *few;
+    scored.block_heads = 64 / (a->head_dim / 8);
+    grid.z = ceil_div(a->heads_k, scored.block_heads);
+  }
+  auto pick = [&](auto t) {
+    typedef decltype(t) T;
+    if (hd == 64) return many ? mean_pool_kernel<T, true, 64> : mean_pool_kernel<T, false, 64>;
+    if (hd == 128) return many ? mean_pool_kernel<T, true, 128> : mean_pool_kernel<T, false, 128>;
+    if (hd == 256) return many ? mean_pool_kernel<T, true, 256> : mean_pool_kernel<T, false, 256>;
+    return many ? mean_pool_kernel<T, true, 0> : mean_pool_kernel<T, false, 0>;
+  };
+  hipLaunchKernelGGL(a->dtype == FMOBA_DTYPE_BF16 ? pick(bf16_t()) : pick(f16_t()), grid, dim3(256), 0, s, *a, extra, scored);
   FMOBA_LAUNCH_CHECK("mean_pool");
   return 0;
 }
@@ -192,5 +251,11 @@ int mean_pool_with_offsets(const fmoba_mean_pool_args *a, int32_t *clear, int64_
     cu_km = nullptr;
   }
   return mean_pool_run(a, PoolExtra{cu_km, clear, clear_vec16}, stream);
+}
+
+// Whether the pooling pass can score the rows of a call: a product has 32 columns.
+bool pool_scores_feasible(int head_dim, int group, int rows, int batch) { return head_dim <= 256 && group * rows <= 32 && batch <= kPoolOffsetsBatch; }
+int mean_pool_with_scores(const fmoba_mean_pool_args *a, const FewGate &few, void *stream) {
+  return mean_pool_run(a, PoolExtra{const_cast<int32_t *>(a->cu_seqlens_km), nullptr, 0}, stream, &few);
 }
 }  // namespace fmoba

@@ -166,14 +166,35 @@ struct Result {
 };
 const uint32_t *visit_ptr(const Tensor &t) { return t.defined() ? reinterpret_cast<const uint32_t *>(t.data_ptr<int32_t>()) : nullptr; }
 
+// what this thread's last forward ran, and its last backward if nobody has asked since (else -1): diagnostics
+thread_local int t_visits = 0, t_row_blocks = 0, t_partials = -1;
+
+// gate and attention of a call with a few query rows per sequence
+Result forward_few(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const Tensor &k, int64_t topk, size_t score_bytes) {
+  Result r;
+  r.out = at::empty_like(q);
+  r.lse = at::empty({s.heads, s.total_q}, q.options().dtype(at::kFloat));
+  a.out = r.out.data_ptr(), a.softmax_lse = r.lse.data_ptr<float>();
+  a.o_row_stride = r.out.stride(0), a.o_head_stride = r.out.stride(1);
+  const size_t cu_bytes = up256((s.batch + 1) * 4);
+  const Tensor scratch = bytes_like(q, cu_bytes + score_bytes + 256);
+  char *base = reinterpret_cast<char *>(up256(reinterpret_cast<size_t>(scratch.data_ptr())));
+  fmoba_mean_pool_args m{};
+  m.k = a.k, m.km = base + cu_bytes;  // (not written)
+  m.cu_seqlens_k = a.cu_seqlens_k, m.cu_seqlens_km = reinterpret_cast<int32_t *>(base);
+  m.batch = s.batch, m.max_chunks = s.max_cols, m.heads_k = s.heads_k, m.head_dim = s.dim, m.chunk = s.chunk, m.dtype = s.dtype;
+  m.k_row_stride = k.stride(0), m.k_head_stride = k.stride(1), m.km_row_stride = s.heads_k * s.dim, m.km_head_stride = s.dim;
+  t_visits = a.max_visits_per_row, t_row_blocks = 1;
+  check(fmoba_attn_fwd_gated_few(&m, &a, topk, s.causal, reinterpret_cast<float *>(base + cu_bytes), s.stream));
+  return r;
+}
+
 // what the form of dQ and its workspace depend on
 void backward_sizes(fmoba_attn_bwd_args &b, const Shape &s, int64_t visits64) {
   b.batch = s.batch, b.total_q = s.total_q, b.total_k = s.total_k, b.heads = s.heads, b.heads_k = s.heads_k, b.head_dim = s.dim;
   b.max_seqlen_q = s.max_q, b.max_seqlen_k = s.max_k, b.max_cols = s.max_cols, b.lg_block_n = s.chunk, b.is_causal = s.causal && s.max_q != 1;
   b.max_visits_per_row = visits64;
 }
-// what this thread's last forward ran, and its last backward if nobody has asked since (else -1): diagnostics
-thread_local int t_visits = 0, t_row_blocks = 0, t_partials = -1;
 
 Result forward(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const Pattern &p) {
   Result r;
@@ -304,15 +325,20 @@ py::object moba_varlen(const py::handle &hq, const py::handle &hk, const py::han
       check_device(q.device().index());
       s.stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
       fmoba_attn_fwd_args a = forward_args(s, q, k, v, cu_q, cu_k, visits, scale, nullptr);
-      const bool columns = !fmoba_attn_fwd_uses_row_blocks(&a), lists = grad || columns;  // (the row-block form reads the selection bits alone)
-      // Ranks for the forms that leave a partial result per visit.  (One query row per sequence: the attention then drops the
-      // causal rule that the gating keeps, and the visits of a row are others.  65536 visits: more than a row's count holds.)
-      fmoba_attn_bwd_args b{};
-      backward_sizes(b, s, visits * (kb / 64));
-      const bool ranked = max_q > 1 && visits * (kb / 64) < 65536 && (columns || (grad && fmoba_attn_bwd_uses_partials(&b)));
-      p = gate(s, q, k, cu_q, cu_k, topk, lists, ranked);
-      a.selection_bits = p.selection;
-      r = forward(s, a, q, p);
+      const size_t few = grad ? 0 : fmoba_attn_fwd_gated_few_bytes(&a);
+      if (few > 0) {
+        r = forward_few(s, a, q, k, topk, few);
+      } else {
+        const bool columns = !fmoba_attn_fwd_uses_row_blocks(&a), lists = grad || columns;  // (the row-block form reads the selection bits alone)
+        // Ranks for the forms that leave a partial result per visit.  (One query row per sequence: the attention then drops the
+        // causal rule that the gating keeps, and the visits of a row are others.  65536 visits: more than a row's count holds.)
+        fmoba_attn_bwd_args b{};
+        backward_sizes(b, s, visits * (kb / 64));
+        const bool ranked = max_q > 1 && visits * (kb / 64) < 65536 && (columns || (grad && fmoba_attn_bwd_uses_partials(&b)));
+        p = gate(s, q, k, cu_q, cu_k, topk, lists, ranked);
+        a.selection_bits = p.selection;
+        r = forward(s, a, q, p);
+      }
     }
     out = grad ? Attention::apply(q, k, v, cu_q, cu_k, p, r, max_q, max_k, chunk, causal, scale, visits * (kb / 64), false) : r.out;
   }

@@ -6,6 +6,7 @@ import torch
 import flash_moba
 from flash_moba import flash_moba_hip as hip
 from flash_moba.mean_pool import flash_topk_mean_pool
+from test_gpu_host_path import _both
 from gpu_utils import assert_close
 from oracle import moba_oracle as O
 
@@ -86,3 +87,31 @@ def test_gate_with_infinite_scores_and_without_numbers(lens_k, chunk, topk, caus
                 want = set(order[:topk - 1] + [pos // chunk] if causal else order[:topk])
                 assert set(got[h, :, row].nonzero().flatten().tolist()) == want, (b, i, h)
             row += 1
+
+
+# Scores from the pooling pass and the choice in front of the attention, against the gate and the attention over its selection bits.  Chunks at and past
+# a lane's registers (256, 1024), products full of rows (4 heads x 8 rows), ties, keys that are infinite or not a number, more key heads than a block has.
+@pytest.mark.parametrize("lens_q,lens_k,chunk,topk", [
+    ([1], [5], 64, 3), ([1, 1, 0, 1], [64 * 65, 64, 100, 129], 64, 1), ([8, 3], [64 * 65 + 1, 700], 64, 7), ([1, 2], [64 * 257, 64 * 256], 64, 33),
+    ([1, 1], [64 * 1024, 64 * 1025 + 9], 64, 64), ([2], [1], 128, 5), ([4, 1], [128 * 300, 128 * 7], 128, 16)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("kind", ["normal", "ties", "special"])
+@pytest.mark.parametrize("H,Hk,D,dtype", [(8, 2, 128, torch.bfloat16), (10, 10, 64, torch.float16), (12, 3, 256, torch.bfloat16), (12, 6, 96, torch.float16),
+                                          (6, 6, 40, torch.bfloat16)])
+def test_scores_from_the_pooling_pass(monkeypatch, lens_q, lens_k, chunk, topk, causal, kind, H, Hk, D, dtype):
+    q, k, v, cuq, cuk = (t.cuda() for t in _case(lens_q, lens_k, H, Hk, D, dtype, D + topk, kind == "ties"))
+    if kind == "special":
+        g = torch.Generator(device="cuda").manual_seed(topk)
+        at = torch.randint(0, 300, k.shape[:2], generator=g, device="cuda")
+        for i, x in enumerate((float("inf"), float("-inf"), float("nan"))):
+            k[:, :, 0] = torch.where(at == i, x, k[:, :, 0].float()).to(dtype)
+    out = lambda: (flash_moba.flash_moba_varlen_func(q, k, v, cuq, cuk, max(lens_q), max(lens_k), chunk, topk, causal=causal).view(torch.int16),)
+    _both(monkeypatch, out)
+
+
+@pytest.mark.parametrize("heads,heads_k,dim,rows,takes", [(32, 8, 128, 1, True), (32, 8, 128, 8, True), (32, 4, 128, 8, False), (8, 8, 96, 1, True), (8, 8, 256, 8, True)])
+def test_which_calls_the_pooling_pass_scores(heads, heads_k, dim, rows, takes):
+    f = hip.AttnFwdArgs()
+    f.batch, f.total_q, f.total_k, f.heads, f.heads_k, f.head_dim = 4, 4 * rows, 4 << 16, heads, heads_k, dim
+    f.max_seqlen_q, f.max_seqlen_k, f.max_cols, f.lg_block_n, f.is_causal, f.max_visits_per_row = rows, 1 << 16, 512, 128, 1, 8
+    assert (hip.load_library().fmoba_attn_fwd_gated_few_bytes(f) > 0) == takes
