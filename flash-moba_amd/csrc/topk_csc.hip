@@ -992,6 +992,56 @@ __global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
   }
 }
 
+// How many chunks a row selected below each word of its selection (PREFIX), and its visits, for rows first, first + step, .. of `rows` rows of sequence b from `row0` on;
+// with them, shared out among `nblk` blocks, the rows before the first sequence and after the last one (a buffer longer than its batch), which have no visits: the combine
+// kernels look at every row.
+template <bool PREFIX>
+__device__ __forceinline__ void rank_rows(const TopkParams &p, int h, int b, int blk, int nblk, int row0, int rows) {
+  const fmoba_fused_topk_args &a = p.a;
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+  const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b], last = (Lk + a.chunk - 1) / a.chunk - 1;  // the sequence's last chunk
+  {
+    uint32_t *vh = p.ranks.visits + (int64_t)h * a.total_q;
+    const int64_t first = (int64_t)blk * nthr + tid, step = (int64_t)nblk * nthr;
+    if (b == 0)
+      for (int64_t i = first; i < q0; i += step) vh[i] = 0u;
+    if (b == a.batch - 1)
+      for (int64_t i = (int64_t)q0 + Lq + first; i < a.total_q; i += step) vh[i] = 0u;
+  }
+  for (int k = 0; k < rows; k += nthr) {
+    const int r = row0 + k + tid;
+    if (r >= Lq) return;
+    const int rp = r + Lk - Lq, own = rp >= 0 ? rp / a.chunk : -1;
+    const int nw = a.is_causal ? (own < 0 ? 0 : min(p.W, (own >> 5) + 1)) : p.W;
+    const uint32_t *words = p.sel + (int64_t)h * p.W * a.total_q + q0 + r;
+    uint8_t *pre = PREFIX ? p.ranks.prefix + (int64_t)h * p.W * a.total_q + q0 + r : nullptr;
+    int n = 0, has_last = 0;
+    for (int w0 = 0; w0 < nw; w0 += 8) {
+      uint32_t x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = w0 + i < nw ? words[(int64_t)(w0 + i) * a.total_q] : 0u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (PREFIX && w0 + i > 0 && w0 + i < nw) pre[(int64_t)(w0 + i) * a.total_q] = (uint8_t)n;
+        n += __popc(x[i]);
+        if (w0 + i == (last >> 5)) has_last = (x[i] >> (last & 31)) & 1;
+      }
+    }
+    // Forward: all key blocks of a selected chunk that exist.  Backward: under the causal rule those of the row's own chunk, its
+    // last one, that begin at or before the row.
+    auto blocks = [&](int sub, int keys) {
+      const int kb = a.chunk / sub;
+      return (keys + kb - 1) / kb;
+    };
+    const int nf = n * p.sub_fwd - has_last * (p.sub_fwd - blocks(p.sub_fwd, Lk - last * a.chunk));
+    const int nb = n == 0         ? 0
+                   : a.is_causal ? (n - 1) * p.sub_bwd + blocks(p.sub_bwd, rp - own * a.chunk + 1)
+                                 : n * p.sub_bwd - has_last * (p.sub_bwd - blocks(p.sub_bwd, Lk - last * a.chunk));
+    p.ranks.visits[(int64_t)h * a.total_q + q0 + r] = (uint32_t)nf | ((uint32_t)nb << 16);
+  }
+}
+
 // grid (heads, batch, 1 + blocks of kRankRows rows if ranks are wanted), block 256.
 // RANKS: with the blocks of the ranks, a kernel of its own: in one with both, the scan of plain lists was 4073 instructions with 36 scalars
 // spilled, 571 and none without (8192 tokens, 16 heads 5.4 -> 4.9 us, 32768 tokens, 32 heads 13.3 -> 12.6).  The ranks' loops stay
@@ -1001,55 +1051,14 @@ template <bool RANKS>
 __global__ __launch_bounds__(256) void csc_scan_kernel(TopkParams p) {
   const fmoba_fused_topk_args &a = p.a;
   const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  const int q0 = a.cu_seqlens_q[b];
-  const int Lq = a.cu_seqlens_q[b + 1] - q0;
+  // (independent of the scan, whose few workgroups mostly wait: scan without and with the ranks, 8192 tokens, 16 heads 6.0 and 6.8 us; 262144 tokens 122 and
+  // 250 us)
   if (RANKS && blockIdx.z > 0) {
-    // How many chunks a row selected below each word of its selection, and its visits: independent of the scan, whose few
-    // workgroups mostly wait (scan without and with them: 8192 tokens, 16 heads 6.0 and 6.8 us; 262144 tokens 122 and 250 us)
-    const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b], last = (Lk + a.chunk - 1) / a.chunk - 1;  // the sequence's last chunk
-    // rows before the first sequence and after the last one (a buffer longer than its batch) have no visits: the combine kernels
-    // look at every row
-    {
-      uint32_t *vh = p.ranks.visits + (int64_t)h * a.total_q;
-      const int64_t first = (int64_t)(blockIdx.z - 1) * 256 + tid, step = (int64_t)(gridDim.z - 1) * 256;
-      if (b == 0)
-        for (int64_t i = first; i < q0; i += step) vh[i] = 0u;
-      if (b == a.batch - 1)
-        for (int64_t i = (int64_t)q0 + Lq + first; i < a.total_q; i += step) vh[i] = 0u;
-    }
-    for (int k = 0; k < kRankRows; k += 256) {
-      const int r = (int)(blockIdx.z - 1) * kRankRows + k + tid;
-      if (r >= Lq) return;
-      const int rp = r + Lk - Lq, own = rp >= 0 ? rp / a.chunk : -1;
-      const int nw = a.is_causal ? (own < 0 ? 0 : min(p.W, (own >> 5) + 1)) : p.W;
-      const uint32_t *words = p.sel + (int64_t)h * p.W * a.total_q + q0 + r;
-      uint8_t *pre = p.ranks.prefix + (int64_t)h * p.W * a.total_q + q0 + r;
-      int n = 0, has_last = 0;
-      for (int w0 = 0; w0 < nw; w0 += 8) {
-        uint32_t x[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = w0 + i < nw ? words[(int64_t)(w0 + i) * a.total_q] : 0u;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if (w0 + i > 0 && w0 + i < nw) pre[(int64_t)(w0 + i) * a.total_q] = (uint8_t)n;
-          n += __popc(x[i]);
-          if (w0 + i == (last >> 5)) has_last = (x[i] >> (last & 31)) & 1;
-        }
-      }
-      // Forward: all key blocks of a selected chunk that exist.  Backward: under the causal rule those of the row's own chunk, its
-      // last one, that begin at or before the row.
-      auto blocks = [&](int sub, int keys) {
-        const int kb = a.chunk / sub;
-        return (keys + kb - 1) / kb;
-      };
-      const int nf = n * p.sub_fwd - has_last * (p.sub_fwd - blocks(p.sub_fwd, Lk - last * a.chunk));
-      const int nb = n == 0         ? 0
-                     : a.is_causal ? (n - 1) * p.sub_bwd + blocks(p.sub_bwd, rp - own * a.chunk + 1)
-                                   : n * p.sub_bwd - has_last * (p.sub_bwd - blocks(p.sub_bwd, Lk - last * a.chunk));
-      p.ranks.visits[(int64_t)h * a.total_q + q0 + r] = (uint32_t)nf | ((uint32_t)nb << 16);
-    }
+    rank_rows<true>(p, h, b, blockIdx.z - 1, gridDim.z - 1, (int)(blockIdx.z - 1) * kRankRows, kRankRows);
     return;
   }
+  const int q0 = a.cu_seqlens_q[b];
+  const int Lq = a.cu_seqlens_q[b + 1] - q0;
   const int nseg_b = (Lq + p.seg_rows - 1) / p.seg_rows;
   const int64_t bh = (int64_t)b * a.heads + h;
   int32_t *segc = p.segcnt + bh * p.nseg * p.max_cols;
@@ -1133,6 +1142,30 @@ __device__ __forceinline__ uint32_t count_lanes(uint32_t n, unsigned long long l
   return n;
 }
 
+// Rows r (lane by lane) with words w of a word column: every row goes to the lists of the chunks it selected.  rel: lane j's is the place of the
+// next row of chunk j, counted from `lists`.
+template <bool RANKED>
+__device__ __forceinline__ void fill_step(int32_t *lists, uint32_t &rel, int r, uint32_t w, uint32_t nth) {
+  // the chunks that some row of the step selects (a scalar, so that the others cost no vector instruction)
+  const uint32_t present = __builtin_amdgcn_readfirstlane(__ockl_wfred_or_u32(w));
+  if (present == 0u) return;
+  static_for<32>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    if (present & (1u << j)) {
+      const unsigned long long m = __ballot((w & (1u << j)) != 0u);
+      const uint32_t at = __builtin_amdgcn_readlane(rel, j);
+      const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+      if constexpr (RANKED) {
+        store_i32_in_lanes(lists, (at + rank) << 2, (int)((nth << kListRowBits) | (uint32_t)r), m);
+        nth = count_lanes(nth, m);
+      } else {
+        store_i32_in_lanes(lists, (at + rank) << 2, r, m);
+      }
+      rel = write_lane<j>(rel, at + (uint32_t)__popcll(m));
+    }
+  });
+}
+
 // grid (nseg * W, heads, batch), block 64: one wave walks the rows of one segment of one 32-chunk word column
 // RANKED: with every row id its chunk's place among the chunks of the row, in the bits from kListRowBits on (in an array of their own,
 // a byte per entry, the ranks cost a second store per chunk and step: 262144 tokens 789 -> 1723 us, 874 this way)
@@ -1176,26 +1209,113 @@ __global__ __launch_bounds__(64) void csc_fill_kernel(TopkParams p) {
   for (int rb = rb0; rb < r1; rb += 64) {
     const int r = rb + lane;
     const uint32_t w = (r < r1) ? words[r] : 0u;
-    uint32_t nth = RANKED && wc > 0 && r < r1 ? pre[r] : 0u;  // chunks that the row selected so far
-    // the chunks that some row of the step selects (a scalar, so that the others cost no vector instruction)
-    const uint32_t present = __builtin_amdgcn_readfirstlane(__ockl_wfred_or_u32(w));
-    if (present == 0u) continue;
-    static_for<32>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      if (present & (1u << j)) {
-        const unsigned long long m = __ballot((w & (1u << j)) != 0u);
-        const uint32_t at = __builtin_amdgcn_readlane(rel, j);
-        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        if constexpr (RANKED) {
-          store_i32_in_lanes(lists, (at + rank) << 2, (int)((nth << kListRowBits) | (uint32_t)r), m);
-          nth = count_lanes(nth, m);
-        } else {
-          store_i32_in_lanes(lists, (at + rank) << 2, r, m);
-        }
-        rel = write_lane<j>(rel, at + (uint32_t)__popcll(m));
-      }
-    });
+    const uint32_t nth = RANKED && wc > 0 && r < r1 ? pre[r] : 0u;  // chunks that the row selected so far
+    fill_step<RANKED>(lists, rel, r, w, nth);
   }
+}
+
+// Scan and fill in one launch, for calls with few counts per (sequence, head): every workgroup adds up the counts it needs itself (no more than kListCounts of them,
+// each wave a quarter, all loads in flight at once), a segment's rows are asked for together with them, and with ranks the chunks of a row below the word column are
+// counted from its words, of which there are few.  grid (nseg * W, + nseg for the visits if ranks are wanted; heads, batch), a wave for each 64 rows of a segment.
+// What bounds it is a chain: launch, counts, 32 ballots and stores.  The scan before it was a launch and a chain of its own whose few workgroups left the chip
+// empty, and one wave per segment walks four times as far: 8192 tokens, 16 heads, ranked lists of 128-key chunks, scan and fill 17.6 us, one wave per segment 15.1, this 10.0 (four waves of
+// eight chunks each, which read the words below four times: 10.9, and 23 where this takes 19); parts of prompts of 1024 rows against 9000 to 33000 keys, 32 heads
+// 22.0 -> 19.4; 8191 tokens of short documents, plain lists 10.7 -> 4.8.  More counts, or longer segments (which calls of many waves have), go to the two launches: there the
+// scan is a small part of the time and the counts of a workgroup would be a large one.
+constexpr int kListCounts = 4096, kListWords = 16, kListSegRows = 256;
+template <bool RANKED>
+__global__ __launch_bounds__(256) void csc_lists_kernel(TopkParams p) {
+  const fmoba_fused_topk_args &a = p.a;
+  __shared__ int sBefore[4], sAll[4][32], sMine[4][32], sStep[4][32];
+  const int h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 31;
+  if (RANKED && (int)blockIdx.x >= p.nseg * p.W) {
+    const int blk = blockIdx.x - p.nseg * p.W;
+    rank_rows<false>(p, h, b, blk, p.nseg, blk * p.seg_rows, p.seg_rows);
+    return;
+  }
+  const int wc = blockIdx.x / p.nseg, seg = blockIdx.x - wc * p.nseg;
+  const int q0 = a.cu_seqlens_q[b];
+  const int Lq = a.cu_seqlens_q[b + 1] - q0;
+  const int r0 = seg * kListSegRows;
+  if (r0 >= Lq && seg > 0) return;
+  const int r1 = min(Lq, r0 + kListSegRows), nseg_b = (Lq + kListSegRows - 1) / kListSegRows;
+  // with the causal rule a row selects no chunk beyond its own: the rows before the word column's first chunk hold zeros
+  bool rows = r0 < r1;
+  if (a.is_causal) rows = rows && (int64_t)wc * 32 * a.chunk - ((int64_t)(a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b]) - Lq) < r1;
+  // (the first segment's workgroup tells where the lists of its word column are, those of the last word column clear what no list uses)
+  if (!rows && seg > 0 && wc < p.W - 1) return;
+  const int64_t bh = (int64_t)b * a.heads + h;
+  const int32_t *cnt = p.segcnt + bh * p.nseg * p.max_cols;
+  const int cols = p.max_cols, c = wc * 32 + j;
+  const int r = r0 + wave * 64 + lane;
+  const uint32_t *below = p.sel + (int64_t)h * p.W * a.total_q + q0 + r;
+  const uint32_t w = rows && r < r1 ? below[(int64_t)wc * a.total_q] : 0u;
+  uint32_t nth = 0u;
+  if constexpr (RANKED) {
+    for (int v0 = 0; v0 < (rows ? wc : 0); v0 += 8) {
+      uint32_t x[8];
+#pragma unroll
+      for (int v = 0; v < 8; ++v) x[v] = v0 + v < wc && r < r1 ? below[(int64_t)(v0 + v) * a.total_q] : 0u;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) nth += __popc(x[v]);
+    }
+  }
+  // counts of this column (lanes j and 32 + j: column j, two segments at a time), all of them and those of the segments before this one; and of the columns
+  // before the word column
+  int before = 0, all = 0, mine = 0;
+  for (int s0 = 0; s0 < nseg_b; s0 += 32) {
+    int y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int s = s0 + 8 * i + 2 * wave + (lane >> 5);
+      y[i] = c < cols && s < nseg_b ? cnt[s * cols + c] : 0;
+    }
+    for (int c0 = lane; c0 < wc * 32; c0 += 128) {
+      int x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int s = s0 + 4 * (i >> 1) + wave, c1 = c0 + 64 * (i & 1);
+        x[i] = c1 < wc * 32 && s < nseg_b ? cnt[s * cols + c1] : 0;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) before += x[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      all += y[i];
+      mine += s0 + 8 * i + 2 * wave + (lane >> 5) < seg ? y[i] : 0;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) before += __shfl_xor(before, o, 64);
+  all = sum_xor32_i(all);
+  mine = sum_xor32_i(mine);
+  const int step = sum_xor32_i(bit_column_count32(w, lane));  // rows of this wave in column j
+  if (lane < 32) sAll[wave][lane] = all, sMine[wave][lane] = mine, sStep[wave][lane] = step;
+  if (lane == 0) sBefore[wave] = before;
+  __syncthreads();
+  before = __builtin_amdgcn_readfirstlane((sBefore[0] + sBefore[1]) + (sBefore[2] + sBefore[3]));
+  all = (sAll[0][j] + sAll[1][j]) + (sAll[2][j] + sAll[3][j]);
+  mine = (sMine[0][j] + sMine[1][j]) + (sMine[2][j] + sMine[3][j]);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) mine += i < wave ? sStep[i][j] : 0;
+  int incl = all;
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) {
+    const int up = __shfl_up(incl, o, 32);
+    incl += j >= o ? up : 0;
+  }
+  const int64_t base = ((int64_t)q0 * a.heads + (int64_t)Lq * h) * a.topk;
+  if (seg == 0 && threadIdx.x < 32 && c < cols) {
+    a.col_nnz[bh * cols + c] = all;
+    a.col_offsets[bh * cols + c] = base + before + incl - all;
+  }
+  if (wc == p.W - 1) {
+    const int64_t end = base + (int64_t)Lq * a.topk;
+    for (int64_t i = base + before + __builtin_amdgcn_readlane(incl, 31) + seg * 256 + threadIdx.x; i < end; i += nseg_b * 256) a.flat_indices[i] = 0;
+  }
+  uint32_t rel = (uint32_t)(incl - all + mine);
+  if (rows) fill_step<RANKED>(a.flat_indices + base + before, rel, r, w, nth);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1483,12 +1603,16 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("topk_gate_kernel");
   if (!lists) return 0;
-  if (ranks)
-    hipLaunchKernelGGL(csc_scan_kernel<true>, dim3(a->heads, a->batch, 1 + ceil_div(a->max_seqlen_q, kRankRows)), dim3(256), 0, s, p);
-  else
-    hipLaunchKernelGGL(csc_scan_kernel<false>, dim3(a->heads, a->batch), dim3(256), 0, s, p);
-  FMOBA_LAUNCH_CHECK("csc_scan_kernel");
-  hipLaunchKernelGGL(ranks ? csc_fill_kernel<true> : csc_fill_kernel<false>, dim3(p.nseg * p.W, a->heads, a->batch), dim3(64), 0, s, p);
+  if ((int64_t)p.nseg * max_cols <= kListCounts && p.W <= kListWords && p.seg_rows == kListSegRows) {
+    hipLaunchKernelGGL(ranks ? csc_lists_kernel<true> : csc_lists_kernel<false>, dim3(p.nseg * p.W + (ranks ? p.nseg : 0), a->heads, a->batch), dim3(256), 0, s, p);
+  } else {
+    if (ranks)
+      hipLaunchKernelGGL(csc_scan_kernel<true>, dim3(a->heads, a->batch, 1 + ceil_div(a->max_seqlen_q, kRankRows)), dim3(256), 0, s, p);
+    else
+      hipLaunchKernelGGL(csc_scan_kernel<false>, dim3(a->heads, a->batch), dim3(256), 0, s, p);
+    FMOBA_LAUNCH_CHECK("csc_scan_kernel");
+    hipLaunchKernelGGL(ranks ? csc_fill_kernel<true> : csc_fill_kernel<false>, dim3(p.nseg * p.W, a->heads, a->batch), dim3(64), 0, s, p);
+  }
   FMOBA_LAUNCH_CHECK("csc_fill_kernel");
   if (a->raw_indices) {
     const size_t smem = (size_t)(max_cols + 64) * 4;
