@@ -902,10 +902,25 @@ extern "C" int fmoba_attn_fwd_ranked(const fmoba_attn_fwd_args *a, const uint32_
 }
 
 namespace fmoba {
+bool fwd_rows_gated(const fmoba_attn_fwd_args &a);  // attn_fwd_rows.hip
+// the checks of a forward call whose gate is part of it (topk_csc.hip)
+int fwd_check_gated(const fmoba_attn_fwd_args *a) {
+  if (int rc = fwd_check_common(a)) return rc;
+  FMOBA_REQUIRE(a->total_q > 0 && a->max_seqlen_q > 0 && a->total_k > 0 && a->max_seqlen_k > 0, "attn_fwd: empty problem");
+  FMOBA_REQUIRE(a->q && a->out && a->softmax_lse, "attn_fwd: null q/out/lse pointer");
+  if (int rc = fwd_check_tensors(a)) return rc;
+  FMOBA_REQUIRE(fmoba_attn_fwd_gates_rows(a) != 0, "attn_fwd_gated_rows: not a call of this form (fmoba_attn_fwd_gates_rows tells)");
+  return 0;
+}
 bool pool_scores_feasible(int head_dim, int group, int rows, int batch);                                       // mean_pool.hip
 int mean_pool_with_scores(const fmoba_mean_pool_args *a, const FewGate &few, void *stream);
 void run_fwd_few_scored(const fmoba_attn_fwd_args &a, const FewGate &few, hipStream_t s);                      // attn_fwd_few.hip
 }  // namespace fmoba
+
+extern "C" int32_t fmoba_attn_fwd_gates_rows(const fmoba_attn_fwd_args *a) {
+  using namespace fmoba;
+  return fmoba_attn_fwd_uses_row_blocks(a) && a->fwd_mode == 0 && fwd_rows_gated(*a) ? 1 : 0;
+}
 
 extern "C" size_t fmoba_attn_fwd_gated_few_bytes(const fmoba_attn_fwd_args *a) {
   using namespace fmoba;

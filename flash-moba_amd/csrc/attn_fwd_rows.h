@@ -23,11 +23,12 @@ struct FwdRowsDirectSmem {
   static_assert((size_t)RW * 32 * LDO * 2 <= ring && (size_t)RW * HD * 128 <= ring && SPLIT * RW * 512 <= ring, "output tiles must fit the K/V rings");
 };
 
+// IN_LDS: the rows' words are in sBits already, visible to every thread.
 // The steps of a row block: the selection words of its rows go to sBits (word w of row r at w * ROWS + r), the 64-key blocks of every chunk that
 // a row of it selected to sStep in ascending order (key block | chunk << 16).  `words` points to word 0 of the block's first row, `stride`
 // words lie between two words of a row, `nrow` rows exist, keys [0, kend) are visible to some row.  Returns the number of steps, of which at most step_cap are listed.
 // Every thread of the workgroup takes part; ends with the lists visible to all of them.
-template <int ROWS, int NTHR>
+template <int ROWS, int NTHR, bool IN_LDS = false>
 __device__ __forceinline__ int row_block_steps(const uint32_t *words, int64_t stride, int nrow, int kend, int Bn, int nw, int step_cap, int *sStep,
                                                uint32_t *sUnion, uint32_t *sBits) {
   constexpr int UPW = ROWS / 64;
@@ -38,8 +39,13 @@ __device__ __forceinline__ int row_block_steps(const uint32_t *words, int64_t st
   // wait for every outstanding load of the wave, the tile loads included, at every step)
   for (int it = wave; it < nwu * UPW; it += NTHR / 64) {  // one word of 64 rows per wave
     const int w = it / UPW, rw = (it % UPW) * 64 + lane;
-    const uint32_t x = rw < nrow ? words[w * stride + rw] : 0u;
-    sBits[w * ROWS + rw] = x;
+    uint32_t x;
+    if constexpr (IN_LDS) {
+      x = sBits[w * ROWS + rw];
+    } else {
+      x = rw < nrow ? words[w * stride + rw] : 0u;
+      sBits[w * ROWS + rw] = x;
+    }
     const uint32_t u = or_wave(x);
     if (lane == 0) sUnion[it] = u;
   }

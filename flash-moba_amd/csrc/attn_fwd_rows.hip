@@ -16,6 +16,7 @@
 // The selection of a row is one bit per chunk (the gating's own, or a bitmap built from the CSC lists by
 // csc_bitmap_lds_kernel); the chunks a workgroup walks are the OR of its rows' bitmaps.
 #include "attn_fwd_rows.h"
+#include "gate_select.h"
 
 #include <type_traits>
 #include <utility>
@@ -453,11 +454,16 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // (12037 tokens, 16 heads of 96, top-k 8 of 64-key chunks 208 -> 176 us; 2048 tokens, 8 heads 41 -> 29).
 // With the products at a higher priority than the rest of a step, whole training steps: 65536 tokens in eight sequences 7681 -> 7549 us, 2 x 4096 tokens,
 // top-k 8 of 128-key chunks 496 -> 484, 12037 tokens, 16 heads of 96 484 -> 481, 8191 tokens of short documents the same.
+// GATED: the rows choose their chunks here (up to kRowGateChunks of them), while Q is in registers anyway, and the words of the selection go to memory only if
+// column lists follow (with the counts these need).  The search for a row's cut is vector arithmetic of one wave beside the products of another workgroup's, where a gate
+// launch in front leaves the matrix cores idle, reads Q once more and is a launch.  Whole calls: forward of 1024 + 2048 tokens, 8 heads of 64 33.5 -> 30.1 us, 1024 tokens 23.8 -> 20.6, 2048
+// tokens, 16 heads of 128 53.2 -> 50.3, parts of prompts of 512 and 1000 rows against 4000 and 7000 keys, 32 over 8 heads 172 -> 166; training step of 8191 tokens of short documents 122.2 ->
+// 116.4, 5000 tokens, 8 heads of 112 216 -> 211, 8 x 4096 tokens, 32 over 8 heads, forward 1262 -> 1234; nothing from 24571 tokens of training on.
 // RW: waves of a set, which share its tiles.  SPLIT = 2 (4): two (four) sets of waves take turns at the steps of the same rows, with
 // rings of their own; the results of a row meet in LDS at the end.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
-template <typename T, int HD, int RW, int SPLIT>
-__global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap) {
+template <typename T, int HD, int RW, int SPLIT, bool GATED>
+__global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, RowGate gate) {
   typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
   constexpr int kRows = SM::ROWS;
   constexpr int KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
@@ -499,7 +505,14 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   // ---- the steps of this row block -------------------------------------------------------------
   const int rlast = min(r0 + kRows - 1, Lq - 1);
   const int kend = min(Lk, causal ? rlast + off + 1 : Lk);  // keys [0, kend) are visible to some row
-  const int nstep_all = row_block_steps<kRows, NTHR>(bm + (int64_t)h * nw * a.total_q + q0 + r0, a.total_q, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
+  int nstep_all;
+  if constexpr (GATED) {
+    static_assert(row_gate_lds<HD>() <= SM::ring, "the chunk means and the counts lie where the K/V rings will");
+    gate_row_block<T, HD, RW, SPLIT>(a, gate, smem, sBits, qb, b, h, hk, q0, r0, rlast, Lq, off, nw);
+    nstep_all = row_block_steps<kRows, NTHR, true>(nullptr, 0, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
+  } else {
+    nstep_all = row_block_steps<kRows, NTHR>(bm + (int64_t)h * nw * a.total_q + q0 + r0, a.total_q, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
+  }
   const int nstep_wg = min(nstep_all, step_cap);
   const int nstep = (nstep_wg - set + SPLIT - 1) / SPLIT, nturn = (nstep_wg + SPLIT - 1) / SPLIT;  // this set's steps, the turns of the loop
   // The entries of 64 turns from turn wbase on, one per lane: those of a step come into scalar registers by a lane read.  (Read from LDS in
@@ -561,12 +574,14 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   auto feed_v = [&](int t) { feed(vg, (uint32_t)a.v_row_stride, lofV, ldsV, t & 1, t); };
   const int lim = valid ? min(causal ? row + off : 0x7fffffff, Lk - 1) : -1;  // last visible key
   // (Q is in registers before the first tile loads are issued: from here on the wave counts its outstanding loads)
+  if constexpr (!GATED) {
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
 #endif
-  q_rows_arrange<HD>(qb, hh, D);
-  wait_all_loads();
+    q_rows_arrange<HD>(qb, hh, D);
+    wait_all_loads();
+  }
   entries_from(0);
   feed_k(0);
   feed_k(1);
@@ -810,9 +825,11 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
 }
 
 template <typename T, int HD, int RW, int SPLIT>
-static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
+static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, const RowGate *gate, hipStream_t s) {
   typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
-  auto kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT>;
+  auto kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT, false>;
+  if constexpr (HD != 96)
+    if (gate != nullptr) kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT, true>;
   const int step_cap = ceil_div(a.max_seqlen_k, 64);  // (at most kRowsStepCap: fwd_rows_feasible)
   const size_t smem = SM::bytes(step_cap, nw);
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
@@ -824,7 +841,7 @@ static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, i
     set_error("attn_fwd: too many (sequence, head, row block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap, gate != nullptr ? *gate : RowGate{});
   return 0;
 }
 // Four sets share a walk (head dimensions up to 64) where the workgroups of 64 rows are no more than the compute units, as their rings leave a unit
@@ -849,14 +866,14 @@ static int rows_sets(const fmoba_attn_fwd_args &a) {
   return (int64_t)a.heads * (a.total_q / 128 + a.batch) <= (a.head_dim > 64 ? 288 : 544) ? 2 : 1;
 }
 template <typename T, int HD>
-static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
+static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s, const RowGate *gate = nullptr) {
   const int sets = rows_sets(a);
   if constexpr (HD <= 64)
-    if (sets == 4) return launch_rows_split<T, HD, 2, 4>(a, bm, nw, s);
-  if (sets == 2) return launch_rows_split<T, HD, 2, 2>(a, bm, nw, s);
+    if (sets == 4) return launch_rows_split<T, HD, 2, 4>(a, bm, nw, gate, s);
+  if (sets == 2) return launch_rows_split<T, HD, 2, 2>(a, bm, nw, gate, s);
   if constexpr (HD <= 64)
-    if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1>(a, bm, nw, s);
-  return launch_rows_split<T, HD, 4, 1>(a, bm, nw, s);
+    if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1>(a, bm, nw, gate, s);
+  return launch_rows_split<T, HD, 4, 1>(a, bm, nw, gate, s);
 }
 
 template <typename T, int HD>
@@ -897,6 +914,19 @@ size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a) {
   if (a.selection_bits != nullptr) return 256;
   const size_t rows = (size_t)a.total_q * a.heads;
   return ((rows * (size_t)ceil_div(a.max_cols, 32) * 4 + 255) & ~(size_t)255) + 256;
+}
+
+// Calls whose rows can choose their chunks in attn_fwd_rows_kernel: the scores of a row are two tiles of products with the operands that Q already is (tiles of 96
+// features have them in another order), calls of a few rows have a gate of their own.
+bool fwd_rows_gated(const fmoba_attn_fwd_args &a) {
+  return a.selection_bits == nullptr && a.max_cols <= kRowGateChunks && a.max_seqlen_q > kFewRows && !fwd_few_rows(a) && fwd_rows_direct(a) &&
+         (a.head_dim <= 64 || (a.head_dim > 96 && a.head_dim <= 128));
+}
+int run_fwd_rows_gated(const fmoba_attn_fwd_args &a, const RowGate &gate, hipStream_t s) {
+  const int nw = ceil_div(a.max_cols, 32);
+  const bool bf = a.dtype == FMOBA_DTYPE_BF16;
+  if (a.head_dim <= 64) return bf ? launch_rows<bf16_t, 64>(a, nullptr, nw, s, &gate) : launch_rows<f16_t, 64>(a, nullptr, nw, s, &gate);
+  return bf ? launch_rows<bf16_t, 128>(a, nullptr, nw, s, &gate) : launch_rows<f16_t, 128>(a, nullptr, nw, s, &gate);
 }
 
 // bitmap build (phase 1) + the row-block pass (phase 2)

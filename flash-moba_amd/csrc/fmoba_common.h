@@ -874,6 +874,18 @@ struct FewGate {
   int32_t heads, group, rows, topk, is_causal;  // group: query heads per key head; rows: the longest sequence's
   int32_t block_heads;                          // key heads of a block of the pooling pass (set by its launch)
 };
+// What the row-block forward needs to choose its rows' chunks itself, in place of a gate launch before it (attn_fwd_rows.hip).
+struct RowGate {
+  const uint16_t *km;
+  const int32_t *cu_seqlens_km;
+  int64_t km_row_stride, km_head_stride;
+  int32_t topk;
+  // for the column lists that follow; null without them
+  uint32_t *sel;
+  int32_t *segcnt;
+  int32_t W, nseg, seg_rows;
+};
+constexpr int kRowGateChunks = 64;  // chunks per sequence that it takes, at most
 constexpr int kFewRows = 8, kFewChunks = 4096;  // query rows and chunks per sequence of such a call, at most
 
 }  // namespace fmoba

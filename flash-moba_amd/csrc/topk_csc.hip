@@ -9,7 +9,7 @@
 //                      the row-list buffer.
 //   csc_fill_kernel  : walks the bit columns in row order and writes each chunk's row list
 //                      ascending, so no sort pass is needed afterwards.
-#include "fmoba_common.h"
+#include "gate_select.h"
 
 #include <algorithm>
 #include <mutex>
@@ -56,81 +56,6 @@ struct GateItem {
 __device__ __forceinline__ GateItem gate_item(const TopkParams &p) {
   if (p.rows_in_x) return GateItem{(int)(gridDim.x - 1 - blockIdx.x), (int)blockIdx.y};
   return GateItem{(int)(gridDim.y - 1 - blockIdx.y), (int)blockIdx.x};
-}
-
-// n + (x0 > y) + (x1 > y) + (x2 > y) + (x3 > y): four compares into four scalar register pairs, then four adds with
-// carry, so that no add follows its compare at once (a vector instruction that reads a scalar register written by the
-// one before it has to wait; left alone, the compiler pairs every compare with its consumer and pads with idle slots)
-__device__ __forceinline__ int count4_gt(int n, float x0, float x1, float x2, float x3, float y) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  unsigned long long m0, m1, m2, m3;
-  asm("v_cmp_gt_f32_e64 %1, %5, %9\n\t"
-      "v_cmp_gt_f32_e64 %2, %6, %9\n\t"
-      "v_cmp_gt_f32_e64 %3, %7, %9\n\t"
-      "v_cmp_gt_f32_e64 %4, %8, %9\n\t"
-      "v_addc_co_u32_e64 %0, vcc, 0, %0, %1\n\t"
-      "v_addc_co_u32_e64 %0, vcc, 0, %0, %2\n\t"
-      "v_addc_co_u32_e64 %0, vcc, 0, %0, %3\n\t"
-      "v_addc_co_u32_e64 %0, vcc, 0, %0, %4"
-      : "+v"(n), "=&s"(m0), "=&s"(m1), "=&s"(m2), "=&s"(m3)
-      : "v"(x0), "v"(x1), "v"(x2), "v"(x3), "v"(y)
-      : "vcc");
-  return n;
-#else
-  return n + (x0 > y) + (x1 > y) + (x2 > y) + (x3 > y);
-#endif
-}
-
-// x >= y in two halves: four compares into four scalar register pairs first, then an add with carry per flag
-// where it is needed (a vector instruction that reads a scalar register written by the one before it has to
-// wait two slots: with the compares of four scores ahead of their adds nothing waits; left alone, the compiler
-// materialises every flag as 0 / 1 first).  Volatile, so that the compares stay ahead of the adds.
-struct Flags4 {
-  unsigned long long m[4];
-};
-__device__ __forceinline__ Flags4 flags4_ge(float x0, float x1, float x2, float x3, float y) {
-  Flags4 f;
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_cmp_ge_f32_e64 %0, %4, %8\n\t"
-               "v_cmp_ge_f32_e64 %1, %5, %8\n\t"
-               "v_cmp_ge_f32_e64 %2, %6, %8\n\t"
-               "v_cmp_ge_f32_e64 %3, %7, %8"
-               : "=&s"(f.m[0]), "=&s"(f.m[1]), "=&s"(f.m[2]), "=&s"(f.m[3])
-               : "v"(x0), "v"(x1), "v"(x2), "v"(x3), "v"(y));
-#else
-  f.m[0] = x0 >= y;
-  f.m[1] = x1 >= y;
-  f.m[2] = x2 >= y;
-  f.m[3] = x3 >= y;
-#endif
-  return f;
-}
-// the same with x > y
-__device__ __forceinline__ Flags4 flags4_gt(float x0, float x1, float x2, float x3, float y) {
-  Flags4 f;
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_cmp_gt_f32_e64 %0, %4, %8\n\t"
-               "v_cmp_gt_f32_e64 %1, %5, %8\n\t"
-               "v_cmp_gt_f32_e64 %2, %6, %8\n\t"
-               "v_cmp_gt_f32_e64 %3, %7, %8"
-               : "=&s"(f.m[0]), "=&s"(f.m[1]), "=&s"(f.m[2]), "=&s"(f.m[3])
-               : "v"(x0), "v"(x1), "v"(x2), "v"(x3), "v"(y));
-#else
-  f.m[0] = x0 > y;
-  f.m[1] = x1 > y;
-  f.m[2] = x2 > y;
-  f.m[3] = x3 > y;
-#endif
-  return f;
-}
-// (w << 1) | flag of the lane: one add with carry
-__device__ __forceinline__ uint32_t shift_in_flag(uint32_t w, unsigned long long flag) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_addc_co_u32_e64 %0, vcc, %0, %0, %1" : "+v"(w) : "s"(flag) : "vcc");
-  return w;
-#else
-  return (w << 1) | (uint32_t)(flag & 1);
-#endif
 }
 
 template <typename T, int HD, int NT>
@@ -199,9 +124,6 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
   __syncthreads();
   q_rows_arrange<HD>(qf, hh, D);
 
-  // scores: lane (query l%32) gets chunk t*32 + acc_row(i, hh) in register i of tile t;
-  // chunks that are not candidates of the row hold -inf
-  float sc[NT][16];
   const int rp = r + off;
   int nc;  // number of candidate chunks of this row: chunks strictly before its own chunk
   if (a.is_causal)
@@ -209,252 +131,18 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
   else
     nc = valid ? Cb : 0;
   nc = min(nc, nsc);
-  float vmin = INFINITY, vmax = -INFINITY;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    if (t < n_tiles) {
-      f32x16 acc;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const Pack8 af = lds_read16(ldsTile + (uint32_t)((t * 32 + (lane & 31)) * RB) + (uint32_t)(((hh * KS + ks) ^ tile_swz<HD>(lane & 31)) * 16));
-        acc = mfma32<T>(af, qf[ks], acc);
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int c = t * 32 + acc_row(i, hh);
-        const bool cand = c < nc;
-        const float x = acc[i];
-        sc[t][i] = cand ? x : -INFINITY;
-        vmin = fminf(vmin, cand ? x : INFINITY);
-        vmax = fmaxf(vmax, sc[t][i]);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sc[t][i] = -INFINITY;
-    }
-  }
-  vmin = min_xor32_f(vmin);
-  vmax = max_xor32_f(vmax);
-
-  // K' = number of scored chunks to keep (the own chunk takes one slot in causal mode).
-  // A row keeps every candidate x with x > tau, plus, among the candidates equal to tau_eq,
-  // those with chunk index >= iota.  tau is found by bisection between the row's smallest
-  // and largest score and the search stops as soon as exactly K' scores lie above the probe.
-  // The bracket is kept as order-preserving integer keys (lo_k, hi_k]; the first probes
-  // bisect the VALUE range (few steps for ordinary score distributions), later ones the key
-  // range (at most 32 more steps whatever the values).  If the bracket closes first, the
-  // scores inside it are all equal and tie across the cut: the highest chunk indices win.
   const int kp = a.is_causal ? a.topk - 1 : a.topk;
-  const bool need = (nc > kp) && (kp > 0);
-  float tau = -INFINITY;    // nc <= K': every candidate with a score above -inf
-  float tau_eq = INFINITY;  // no tie group by default
-  int n_eq = 0;
-  uint32_t iota = 0u;
-  uint32_t lo_k = float_order_key(vmin) - 1u;  // count(x > lo) = nc > K'
-  uint32_t hi_k = float_order_key(vmax);       // count(x > hi) = 0  < K'
-  int c_lo = nc, c_hi = 0;
-  bool open = need;
-  // A row whose bracket holds exactly one score too many, or one too few, needs no more probes: the cut lies right
-  // below the largest score of the bracket, or right at its smallest.  When every open row of the wave is in that state
-  // (about eight probes in, where the search of the slowest row takes twelve or thirteen), one pass over the scores
-  // finds that score for all of them, the largest of -x for the rows that want the smallest.  The cut it gives is
-  // exact unless the score occurs twice; such rows are found by their count below and searched to the end.
-  bool guessed = false;
-  auto bisect = [&](bool may_finish) {
-    for (int iter = 0;; ++iter) {
-      if (open && hi_k - lo_k <= 1u) {
-        // nothing representable strictly inside: every score in (lo, hi] equals hi
-        tau = order_key_float(hi_k);
-        if (tau != -INFINITY) {
-          tau_eq = tau;
-          n_eq = kp - c_hi;
-        }
-        open = false;
-      }
-      if (!__any(open)) break;
-      if (may_finish) {
-        const bool up = kp - c_hi == 1, dn = c_lo - kp == 1;
-        if (__all(!open || up || dn)) {
-          const bool want_min = open && !up;
-          const uint32_t flip = want_min ? 0x80000000u : 0u;
-          // (x > lo for a score x is x >= the next float above lo, which after -0 is the smallest positive number)
-          const uint32_t above_lo = lo_k + (lo_k == 0x7fffffffu ? 2u : 1u);
-          const float bound = want_min ? -order_key_float(above_lo) : order_key_float(hi_k);
-          float best = -INFINITY;
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            if (t < n_tiles) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) {
-                const float y = __uint_as_float(__float_as_uint(sc[t][i]) ^ flip);
-                best = fmaxf(best, y <= bound ? y : -INFINITY);
-              }
-            }
-          best = max_xor32_f(best);
-          if (open) {
-            const float v = __uint_as_float(__float_as_uint(best) ^ flip);
-            uint32_t below = float_order_key(v) - 1u;  // (the float below +0 that compares below it is not -0)
-            if (below == 0x7fffffffu) below -= 1u;
-            tau = up ? order_key_float(below) : v;
-            guessed = true;
-            open = false;
-          }
-          break;
-        }
-      }
-      uint32_t pk = lo_k + ((hi_k - lo_k) >> 1);
-      if (iter < 12) {
-        const float mf = 0.5f * order_key_float(lo_k + 1u) + 0.5f * order_key_float(hi_k);
-        const uint32_t mk = float_order_key(mf);
-        if (mk > lo_k && mk < hi_k) pk = mk;
-      }
-      const float probe = order_key_float(pk);
-      int cnt = 0;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; i += 4) cnt = count4_gt(cnt, sc[t][i], sc[t][i + 1], sc[t][i + 2], sc[t][i + 3], probe);
-        }
-      cnt = sum_xor32_i(cnt);
-      if (open) {
-        if (cnt == kp) {
-          tau = probe;
-          open = false;
-        } else if (cnt > kp) {
-          lo_k = pk;
-          c_lo = cnt;
-        } else {
-          hi_k = pk;
-          c_hi = cnt;
-        }
-      }
-    }
-  };
-  // K' = number of scored chunks to keep (the own chunk takes one slot in causal mode).
-  // A row keeps every candidate x with x > tau, plus, among the candidates equal to tau_eq,
-  // those with chunk index >= iota.  tau is found by bisection between the row's smallest
-  // and largest score and the search stops as soon as exactly K' scores lie above the probe.
-  // The bracket is kept as order-preserving integer keys (lo_k, hi_k]; the first probes
-  // bisect the VALUE range (few steps for ordinary score distributions), later ones the key
-  // range (at most 32 more steps whatever the values).  If the bracket closes first, the
-  // scores inside it are all equal and tie across the cut: the highest chunk indices win.
-  bisect(true);
-  bool any_tie = __any(n_eq > 0);  // some row of the wave has a tie across its cut
-  // Without a tie in the wave a score is selected iff it lies above tau: the flags of the lane's 16 scores of a tile,
-  // shifted in one by one (w + w + flag: one add with carry each), highest first.
-  uint32_t bits[NT];
-  auto flags_above_tau = [&]() {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      bits[t] = 0u;
-      if (t < n_tiles) {
-#pragma unroll
-        for (int i4 = 3; i4 >= 0; --i4) {
-          const Flags4 f = flags4_gt(sc[t][4 * i4 + 3], sc[t][4 * i4 + 2], sc[t][4 * i4 + 1], sc[t][4 * i4], tau);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) bits[t] = shift_in_flag(bits[t], f.m[j]);
-        }
-      }
-    }
-  };
-  if (!any_tie) flags_above_tau();
-  if (__any(guessed)) {
-    int above = 0;
-    if (!any_tie) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) above += __popc(bits[t]);
-    } else {
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if (t < n_tiles) {
-#pragma unroll
-          for (int i = 0; i < 16; i += 4) above = count4_gt(above, sc[t][i], sc[t][i + 1], sc[t][i + 2], sc[t][i + 3], tau);
-        }
-    }
-    above = sum_xor32_i(above);
-    const bool again = guessed && above != kp;
-    if (__any(again)) {
-      open = again;
-      bisect(false);
-      any_tie = __any(n_eq > 0);
-      if (!any_tie) flags_above_tau();
-    }
-  }
-  // a tie group keeps its n_eq highest chunk indices
-  if (any_tie) {
-    const bool tie = n_eq > 0;
-    int ceq = 0;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      if (t < n_tiles) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) ceq += (sc[t][i] == tau_eq) ? 1 : 0;
-      }
-    ceq = sum_xor32_i(ceq);
-    const bool split = tie && ceq > n_eq;
-    if (__any(split)) {
-      uint32_t i_acc = 0u;
-      constexpr int IB = (NT * 32 <= 64) ? 6 : (NT * 32 <= 128 ? 7 : 8);
-      for (int bit = IB - 1; bit >= 0; --bit) {
-        const uint32_t trial = i_acc | (1u << bit);
-        int cnt = 0;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          if (t < n_tiles) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const uint32_t c = (uint32_t)(t * 32 + acc_row(i, hh));
-              cnt += ((sc[t][i] == tau_eq) & (c >= trial)) ? 1 : 0;
-            }
-          }
-        cnt = sum_xor32_i(cnt);
-        if (cnt >= n_eq) i_acc = trial;
-      }
-      if (split) iota = i_acc;
-    }
-  }
-
-  // selection words (32 chunks each), own chunk forced in causal mode
-  const bool has_self = a.is_causal && valid && rp >= 0;
-  const int pself = has_self ? rp / B : -1;
+  const int own = a.is_causal && valid && rp >= 0 ? rp / B : -1;
   const int seg = m0 / p.seg_rows;
   uint32_t *selp = p.sel + (int64_t)h * p.W * a.total_q + q0 + r;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    if (t < p.W) {
-      uint32_t w = 0u;
-      if (t < n_tiles && kp > 0) {
-        if (!any_tie) {
-          // the four nibbles of the flags move to the places of the lane's chunks (4 hh + 8 g .. + 3)
-          const uint32_t b = bits[t];
-          w = ((b & 0xfu) | ((b & 0xf0u) << 4) | ((b & 0xf00u) << 8) | ((b & 0xf000u) << 12)) << (4 * hh);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const uint32_t c = (uint32_t)(t * 32 + acc_row(i, hh));
-            const float x = sc[t][i];
-            const bool s = (x > tau) | ((x == tau_eq) & (c >= iota));
-            w |= s ? (1u << ((8 * (i >> 2) + (i & 3)) + 4 * hh)) : 0u;
-          }
-        }
-      }
-      {
-        const UPair wp = swap32(w);
-        w = wp.a | wp.b;
-      }
-      if (has_self && (pself >> 5) == t) w |= 1u << (pself & 31);
-      if (!valid) w = 0u;
-      if (valid && hh == 0) selp[(int64_t)t * a.total_q] = w;
-      // per-chunk counts of this wave's 32 rows (both halves of the wave hold the rows' words)
-      if (p.segcnt != nullptr && __any(w != 0u)) {
-        const int mycnt = bit_column_count32(w, lane);
-        if (lane < 32 && mycnt) atomicAdd(&sHist[t * 32 + lane], mycnt);
-      }
+  gate_select<T, HD, NT>(ldsTile, qf, lane, n_tiles, nc, kp, own, valid, p.W, [&](int t, uint32_t w) {
+    if (valid && hh == 0) selp[(int64_t)t * a.total_q] = w;
+    // per-chunk counts of this wave's 32 rows (both halves of the wave hold the rows' words)
+    if (p.segcnt != nullptr && __any(w != 0u)) {
+      const int mycnt = bit_column_count32(w, lane);
+      if (lane < 32 && mycnt) atomicAdd(&sHist[t * 32 + lane], mycnt);
     }
-  }
+  });
   __syncthreads();
   for (int c = tid; c < p.W * 32 && c < p.max_cols; c += 256) {
     const int v = sHist[c];
@@ -1503,11 +1191,13 @@ static int launch_gate_hd(const TopkParams &p, dim3 grid, hipStream_t s) {
 
 namespace fmoba {
 int mean_pool_with_offsets(const fmoba_mean_pool_args *a, int32_t *clear, int64_t clear_vec16, void *stream);
+int fwd_check_gated(const fmoba_attn_fwd_args *a);                                                  // attn_fwd.hip
+int run_fwd_rows_gated(const fmoba_attn_fwd_args &a, const RowGate &gate, hipStream_t s);           // attn_fwd_rows.hip
 }
 // The call behind the entry points: everything of `a` except its workspace fields, which come as arguments.  `pool`: the
-// pooling pass that comes first and clears the segment counts; null: the chunk means are there already.
+// pooling pass that comes first and clears the segment counts; null: the chunk means are there already.  `attn`: the forward that takes the gate's place.
 static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_t workspace_bytes, const fmoba_mean_pool_args *pool, bool lists,
-                          const fmoba_csc_ranks *ranks, void *stream) {
+                          const fmoba_csc_ranks *ranks, void *stream, const fmoba_attn_fwd_args *attn = nullptr) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "fused_topk: null args");
   FMOBA_REQUIRE(a->dtype == FMOBA_DTYPE_F16 || a->dtype == FMOBA_DTYPE_BF16, "FlashMoBA only supports fp16 and bf16 data types");
@@ -1594,7 +1284,10 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   p.rows_in_x = row_blocks > kMaxGridY;
   const dim3 ggrid = p.rows_in_x ? dim3(row_blocks, a->heads, a->batch) : dim3(a->heads, row_blocks, a->batch);
   int rc;
-  if (a->max_seqlen_q <= kFewGateRows && max_cols <= kFewGateChunks)
+  if (attn != nullptr)
+    rc = run_fwd_rows_gated(*attn, RowGate{reinterpret_cast<const uint16_t *>(a->km), a->cu_seqlens_km, a->km_row_stride, a->km_head_stride, a->topk, lists ? p.sel : nullptr, p.segcnt, p.W,
+                                           p.nseg, p.seg_rows}, s);
+  else if (a->max_seqlen_q <= kFewGateRows && max_cols <= kFewGateChunks)
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_few_hd<bf16_t>(p, s) : launch_gate_few_hd<f16_t>(p, s);
   else if (big)
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_stream_hd<bf16_t>(p, ggrid, s) : launch_gate_stream_hd<f16_t>(p, ggrid, s);
@@ -1631,7 +1324,7 @@ extern "C" int fmoba_fused_topk(const fmoba_fused_topk_args *a, void *stream) {
   return fused_topk_run(a, a->workspace, a->workspace_bytes, nullptr, true, nullptr, stream);
 }
 
-static int pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, bool want_lists, const fmoba_csc_ranks *r, void *stream) {
+static int pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, bool want_lists, const fmoba_csc_ranks *r, void *stream, const fmoba_attn_fwd_args *attn = nullptr) {
   FMOBA_REQUIRE(m != nullptr && g != nullptr, "pool_and_gate: null args");
   FMOBA_REQUIRE(m->km == g->km && m->cu_seqlens_km == g->cu_seqlens_km && m->cu_seqlens_k == g->cu_seqlens_k && m->batch == g->batch &&
                     m->heads_k == g->heads_k && m->head_dim == g->head_dim && m->chunk == g->chunk && m->dtype == g->dtype,
@@ -1639,11 +1332,22 @@ static int pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_a
   FMOBA_REQUIRE(g->total_q > 0 && g->max_seqlen_q > 0 && g->max_seqlen_k > 0, "pool_and_gate: empty problem");
   FMOBA_REQUIRE(m->max_chunks == fmoba::ceil_div(g->max_seqlen_k, g->chunk), "pool_and_gate: max_chunks is ceil(max_seqlen_k / chunk)");
   FMOBA_REQUIRE(want_lists || g->raw_indices == nullptr, "pool_and_gate: the ordered lists come with the column lists only");
-  return fused_topk_run(g, g->workspace, g->workspace_bytes, m, want_lists, r, stream);
+  return fused_topk_run(g, g->workspace, g->workspace_bytes, m, want_lists, r, stream, attn);
 }
 
 extern "C" int fmoba_pool_and_gate(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, int32_t want_lists, void *stream) {
   return pool_and_gate(m, g, want_lists != 0, nullptr, stream);
+}
+
+extern "C" int fmoba_attn_fwd_gated_rows(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, const fmoba_attn_fwd_args *a, int32_t want_lists, void *stream) {
+  if (int rc = fmoba::fwd_check_gated(a)) return rc;
+  FMOBA_REQUIRE(m != nullptr && g != nullptr, "attn_fwd_gated_rows: null args");
+  FMOBA_REQUIRE(g->q == a->q && g->q_row_stride == a->q_row_stride && g->q_head_stride == a->q_head_stride && g->cu_seqlens_q == a->cu_seqlens_q && m->k == a->k &&
+                    g->cu_seqlens_k == a->cu_seqlens_k && g->batch == a->batch && g->total_q == a->total_q && g->heads == a->heads && g->heads_k == a->heads_k &&
+                    g->head_dim == a->head_dim && g->max_seqlen_q == a->max_seqlen_q && g->max_seqlen_k == a->max_seqlen_k && g->chunk == a->lg_block_n &&
+                    g->dtype == a->dtype && (g->is_causal != 0) == (a->is_causal != 0) && a->max_cols == fmoba::ceil_div(a->max_seqlen_k, a->lg_block_n),
+                "attn_fwd_gated_rows: the argument structs describe different problems");
+  return pool_and_gate(m, g, want_lists != 0, nullptr, stream, a);
 }
 
 extern "C" int fmoba_pool_and_gate_ranked(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, const fmoba_csc_ranks *r, void *stream) {

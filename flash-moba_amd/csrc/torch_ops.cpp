@@ -108,8 +108,9 @@ struct Pattern {
   const uint32_t *selection = nullptr;  // in `scratch`
 };
 
-// chunk means, gating and (with `lists`) the column lists, ranked if wanted
-Pattern gate(const Shape &s, const Tensor &q, const Tensor &k, const Tensor &cu_q, const Tensor &cu_k, int64_t topk, bool lists, bool ranked = false) {
+// chunk means, gating and (with `lists`) the column lists, ranked if wanted; `attn`: with the forward that takes the gate's place
+Pattern gate(const Shape &s, const Tensor &q, const Tensor &k, const Tensor &cu_q, const Tensor &cu_k, int64_t topk, bool lists, bool ranked = false,
+             const fmoba_attn_fwd_args *attn = nullptr) {
   Pattern p;
   const auto i32 = q.options().dtype(at::kInt);
   if (lists) {
@@ -137,7 +138,9 @@ Pattern gate(const Shape &s, const Tensor &q, const Tensor &k, const Tensor &cu_
   g.batch = s.batch, g.total_q = s.total_q, g.heads = s.heads, g.heads_k = s.heads_k, g.head_dim = s.dim;
   g.max_seqlen_q = s.max_q, g.max_seqlen_k = s.max_k, g.topk = topk, g.chunk = s.chunk, g.is_causal = s.causal, g.dtype = s.dtype;
   g.q_row_stride = q.stride(0), g.q_head_stride = q.stride(1), g.km_row_stride = m.km_row_stride, g.km_head_stride = m.km_head_stride;
-  if (ranked) {
+  if (attn != nullptr) {
+    check(fmoba_attn_fwd_gated_rows(&m, &g, attn, lists ? 1 : 0, s.stream));
+  } else if (ranked) {
     const fmoba_csc_ranks r{reinterpret_cast<uint32_t *>(p.visits.data_ptr<int32_t>()), pre_bytes ? reinterpret_cast<uint8_t *>(base + gate_bytes + cu_bytes) : nullptr};
     check(fmoba_pool_and_gate_ranked(&m, &g, &r, s.stream));
   } else {
@@ -166,16 +169,21 @@ struct Result {
 };
 const uint32_t *visit_ptr(const Tensor &t) { return t.defined() ? reinterpret_cast<const uint32_t *>(t.data_ptr<int32_t>()) : nullptr; }
 
-// what this thread's last forward ran, and its last backward if nobody has asked since (else -1): diagnostics
-thread_local int t_visits = 0, t_row_blocks = 0, t_partials = -1;
-
-// gate and attention of a call with a few query rows per sequence
-Result forward_few(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const Tensor &k, int64_t topk, size_t score_bytes) {
+// the tensors that a forward writes
+Result results(const Shape &s, fmoba_attn_fwd_args &a, const Tensor &q) {
   Result r;
   r.out = at::empty_like(q);
   r.lse = at::empty({s.heads, s.total_q}, q.options().dtype(at::kFloat));
   a.out = r.out.data_ptr(), a.softmax_lse = r.lse.data_ptr<float>();
   a.o_row_stride = r.out.stride(0), a.o_head_stride = r.out.stride(1);
+  return r;
+}
+// what this thread's last forward ran, and its last backward if nobody has asked since (else -1): diagnostics
+thread_local int t_visits = 0, t_row_blocks = 0, t_partials = -1;
+
+// gate and attention of a call with a few query rows per sequence
+Result forward_few(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const Tensor &k, int64_t topk, size_t score_bytes) {
+  const Result r = results(s, a, q);
   const size_t cu_bytes = up256((s.batch + 1) * 4);
   const Tensor scratch = bytes_like(q, cu_bytes + score_bytes + 256);
   char *base = reinterpret_cast<char *>(up256(reinterpret_cast<size_t>(scratch.data_ptr())));
@@ -197,11 +205,7 @@ void backward_sizes(fmoba_attn_bwd_args &b, const Shape &s, int64_t visits64) {
 }
 
 Result forward(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const Pattern &p) {
-  Result r;
-  r.out = at::empty_like(q);
-  r.lse = at::empty({s.heads, s.total_q}, q.options().dtype(at::kFloat));
-  a.out = r.out.data_ptr(), a.softmax_lse = r.lse.data_ptr<float>();
-  a.o_row_stride = r.out.stride(0), a.o_head_stride = r.out.stride(1);
+  const Result r = results(s, a, q);
   if (p.indices.defined()) a.col_offsets = p.col_offsets.data_ptr<int64_t>(), a.col_nnz = p.col_nnz.data_ptr<int32_t>(), a.row_indices = p.indices.data_ptr<int32_t>();
   t_visits = a.max_visits_per_row;
   t_row_blocks = fmoba_attn_fwd_uses_row_blocks(&a);
@@ -335,9 +339,15 @@ py::object moba_varlen(const py::handle &hq, const py::handle &hk, const py::han
         fmoba_attn_bwd_args b{};
         backward_sizes(b, s, visits * (kb / 64));
         const bool ranked = max_q > 1 && visits * (kb / 64) < 65536 && (columns || (grad && fmoba_attn_bwd_uses_partials(&b)));
-        p = gate(s, q, k, cu_q, cu_k, topk, lists, ranked);
-        a.selection_bits = p.selection;
-        r = forward(s, a, q, p);
+        if (!ranked && fmoba_attn_fwd_gates_rows(&a)) {
+          t_visits = a.max_visits_per_row, t_row_blocks = 1;
+          r = results(s, a, q);
+          p = gate(s, q, k, cu_q, cu_k, topk, lists, false, &a);
+        } else {
+          p = gate(s, q, k, cu_q, cu_k, topk, lists, ranked);
+          a.selection_bits = p.selection;
+          r = forward(s, a, q, p);
+        }
       }
     }
     out = grad ? Attention::apply(q, k, v, cu_q, cu_k, p, r, max_q, max_k, chunk, causal, scale, visits * (kb / 64), false) : r.out;

@@ -108,6 +108,8 @@ EXPORTS = {
     "fmoba_attn_fwd": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp]),
     "fmoba_attn_fwd_phases": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_i32, c_vp]),
     "fmoba_attn_fwd_ranked": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp, c_i32, c_vp]),
+    "fmoba_attn_fwd_gates_rows": (c_i32, [ctypes.POINTER(AttnFwdArgs)]),
+    "fmoba_attn_fwd_gated_rows": (c_i32, [ctypes.POINTER(MeanPoolArgs), ctypes.POINTER(FusedTopkArgs), ctypes.POINTER(AttnFwdArgs), c_i32, c_vp]),
     "fmoba_attn_fwd_gated_few_bytes": (c_sz, [ctypes.POINTER(AttnFwdArgs)]),
     "fmoba_attn_fwd_gated_few": (c_i32, [ctypes.POINTER(MeanPoolArgs), ctypes.POINTER(AttnFwdArgs), c_i32, c_i32, c_vp, c_vp]),
     "fmoba_attn_bwd_ranked": (c_i32, [ctypes.POINTER(AttnBwdArgs), c_vp, c_i32, c_i32, c_vp]),

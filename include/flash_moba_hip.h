@@ -220,6 +220,11 @@ int fmoba_attn_fwd_ranked(const fmoba_attn_fwd_args *a, const uint32_t *visits, 
  * read.  gate_is_causal: the gating's is_causal (that of `a` is the attention's).  No counterpart in the reference. */
 size_t fmoba_attn_fwd_gated_few_bytes(const fmoba_attn_fwd_args *a);
 int fmoba_attn_fwd_gated_few(const fmoba_mean_pool_args *m, const fmoba_attn_fwd_args *a, int32_t topk, int32_t gate_is_causal, float *scores, void *stream);
+/* The same for calls of more rows that take the row-block form over up to 64 chunks per sequence: the attention chooses its rows' chunks itself, between the
+ * pooling and (want_lists) the column lists of `g`.  fmoba_attn_fwd_gates_rows: 1 for calls of this form (sizes, strides and fwd_mode of `a` are read).  `m` and `g` as for
+ * fmoba_pool_and_gate, with a causal rule and top-k in `g`; no list, selection bits or workspace of `a` are read. */
+int32_t fmoba_attn_fwd_gates_rows(const fmoba_attn_fwd_args *a);
+int fmoba_attn_fwd_gated_rows(const fmoba_mean_pool_args *m, const fmoba_fused_topk_args *g, const fmoba_attn_fwd_args *a, int32_t want_lists, void *stream);
 
 /* ------------------------------------------------------------------------------------
  * Sparse attention backward.
