@@ -894,7 +894,7 @@ static int launch_rows_loader(const fmoba_attn_fwd_args &a, const uint32_t *bm, 
 }
 
 // head dimensions above 128 (attn_fwd_rows_wide.hip)
-int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s);
+int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, const RowGate *gate, hipStream_t s);
 // a call with a handful of rows (attn_fwd_few.hip)
 bool fwd_few_rows(const fmoba_attn_fwd_args &a);
 void run_fwd_few(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s);
@@ -920,12 +920,13 @@ size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a) {
 // features have them in another order), calls of a few rows have a gate of their own.
 bool fwd_rows_gated(const fmoba_attn_fwd_args &a) {
   return a.selection_bits == nullptr && a.max_cols <= kRowGateChunks && a.max_seqlen_q > kFewRows && !fwd_few_rows(a) && fwd_rows_direct(a) &&
-         (a.head_dim <= 64 || (a.head_dim > 96 && a.head_dim <= 128));
+         (a.head_dim <= 64 || a.head_dim > 96);
 }
 int run_fwd_rows_gated(const fmoba_attn_fwd_args &a, const RowGate &gate, hipStream_t s) {
   const int nw = ceil_div(a.max_cols, 32);
   const bool bf = a.dtype == FMOBA_DTYPE_BF16;
   if (a.head_dim <= 64) return bf ? launch_rows<bf16_t, 64>(a, nullptr, nw, s, &gate) : launch_rows<f16_t, 64>(a, nullptr, nw, s, &gate);
+  if (a.head_dim > 128) return launch_rows_wide(a, nullptr, nw, &gate, s);
   return bf ? launch_rows<bf16_t, 128>(a, nullptr, nw, s, &gate) : launch_rows<f16_t, 128>(a, nullptr, nw, s, &gate);
 }
 
@@ -965,7 +966,7 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
       rc = direct ? (bf ? launch_rows<bf16_t, 128>(a, bm, nw, s) : launch_rows<f16_t, 128>(a, bm, nw, s))
                  : (bf ? launch_rows_loader<bf16_t, 128>(a, bm, nw, s) : launch_rows_loader<f16_t, 128>(a, bm, nw, s));
     else
-      rc = direct ? launch_rows_wide(a, bm, nw, s) : (bf ? launch_rows_loader<bf16_t, 256>(a, bm, nw, s) : launch_rows_loader<f16_t, 256>(a, bm, nw, s));
+      rc = direct ? launch_rows_wide(a, bm, nw, nullptr, s) : (bf ? launch_rows_loader<bf16_t, 256>(a, bm, nw, s) : launch_rows_loader<f16_t, 256>(a, bm, nw, s));
     if (rc) return rc;
   }
   return 0;

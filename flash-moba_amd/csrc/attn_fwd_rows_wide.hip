@@ -1,6 +1,7 @@
 // Sparse attention forward in row blocks for head dimensions above 128 (up to 256): the walk of attn_fwd_rows.hip with a
 // loop of its own.
 #include "attn_fwd_rows.h"
+#include "gate_select.h"
 
 namespace fmoba {
 
@@ -17,9 +18,10 @@ namespace fmoba {
 // 128-key chunks bf16 2.010e-3 and 2.047e-3, fp16 2.507e-4 and 2.554e-4; rows that see 64 steps 2.105e-3 and 2.106e-3, 2.632e-4 and 2.632e-4, 512 steps
 // 2.108e-3 and 2.166e-3, 2.623e-4 and 2.694e-4, 2048 steps 2.094e-3 and 2.157e-3, 2.629e-4 and 2.699e-4.
 // What bounds it: matrix products at the power limit (1.0 PFLOP/s executed at 16384 tokens; without the tile loads it would be 15 % faster, without
-// the rescaling or the exponentials 3 to 5 %).  The same call: columns 134 us and their combine 89 -> 171 us, training step 612 -> 530.
-template <typename T>
-__global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap) {
+// the rescaling or the exponentials 3 to 5 %).  GATED as in attn_fwd_rows_kernel: forward of 2 x 4096 tokens, 8 heads, top-k 8 of 128-key chunks 178.7 -> 173.2 us, of 2048 tokens, 16 heads
+// 85.9 -> 80.4, 9000 tokens, 16 over 2 heads 343.6 -> 336.0.  The same call: columns 134 us and their combine 89 -> 171 us, training step 612 -> 530.
+template <typename T, bool GATED>
+__global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, RowGate gate) {
   constexpr int HD = 256, RW = 4;
   typedef FwdRowsDirectSmem<HD, RW, 1> SM;
   constexpr int kRows = SM::ROWS, KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, NI = VPR / RW;
@@ -52,7 +54,15 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
                   r0 + wave * 32, Lq, lane, D);
   const int rlast = min(r0 + kRows - 1, Lq - 1);
   const int kend = min(Lk, causal ? rlast + off + 1 : Lk);  // keys [0, kend) are visible to some row
-  const int nstep = min(row_block_steps<kRows, 256>(bm + (int64_t)h * nw * a.total_q + q0 + r0, a.total_q, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits), step_cap);
+  int nstep;
+  if constexpr (GATED) {
+    static_assert(row_gate_lds<HD>() <= SM::ring, "the chunk means and the counts lie where the K/V rings will");
+    gate_row_block<T, HD, RW, 1>(a, gate, smem, sBits, qb, b, h, hk, q0, r0, rlast, Lq, off, nw);
+    nstep = row_block_steps<kRows, 256, true>(nullptr, 0, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
+  } else {
+    nstep = row_block_steps<kRows, 256>(bm + (int64_t)h * nw * a.total_q + q0 + r0, a.total_q, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
+  }
+  nstep = min(nstep, step_cap);
   if (nstep == 0) {  // no visible selected key: out = 0, lse = +inf for the rows of this block
     if (valid) {
       uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + row) * a.o_row_stride + (int64_t)h * a.o_head_stride;
@@ -91,11 +101,13 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
   };
   const int lim = valid ? min(causal ? row + off : 0x7fffffff, Lk - 1) : -1;  // last visible key
   // (Q is in registers before the first tile loads are issued: from here on the wave counts its outstanding loads)
+  if constexpr (!GATED) {
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qb[ks].w[0]), "+v"(qb[ks].w[1]), "+v"(qb[ks].w[2]), "+v"(qb[ks].w[3]));
 #endif
-  q_rows_arrange<HD>(qb, hh, D);
+    q_rows_arrange<HD>(qb, hh, D);
+  }
   // (Q stays in accumulation registers, which the products read as well as the others)
   u32x4_t qa[KS];
 #pragma unroll
@@ -324,9 +336,10 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
   }
 }
 
-int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s) {
+int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, const RowGate *gate, hipStream_t s) {
   typedef FwdRowsDirectSmem<256, 4, 1> SM;
-  auto kern = a.dtype == FMOBA_DTYPE_BF16 ? attn_fwd_rows_wide_kernel<bf16_t> : attn_fwd_rows_wide_kernel<f16_t>;
+  auto kern = a.dtype == FMOBA_DTYPE_BF16 ? (gate != nullptr ? attn_fwd_rows_wide_kernel<bf16_t, true> : attn_fwd_rows_wide_kernel<bf16_t, false>)
+                                          : (gate != nullptr ? attn_fwd_rows_wide_kernel<f16_t, true> : attn_fwd_rows_wide_kernel<f16_t, false>);
   const int step_cap = ceil_div(a.max_seqlen_k, 64);  // (at most kRowsStepCap: fwd_rows_feasible)
   const size_t smem = SM::bytes(step_cap, nw) + 16;  // (and the four words of sAgain)
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
@@ -338,7 +351,7 @@ int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, h
     set_error("attn_fwd: too many (sequence, head, row block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, bm, nw, step_cap);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, bm, nw, step_cap, gate != nullptr ? *gate : RowGate{});
   return 0;
 }
 

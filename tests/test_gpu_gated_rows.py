@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("lens_q,lens_k,H,Hk,D,chunk,topk", [
     ([9], [9], 2, 2, 64, 64, 1), ([1024, 2048], [1024, 2048], 8, 8, 64, 128, 4), ([2048], [2048], 4, 2, 64, 64, 9), ([33, 0, 65, 300], [33, 7, 65, 300], 2, 1, 40, 64, 2),
     ([341] * 30, [341] * 30, 16, 16, 64, 64, 4), ([4096], [4096], 16, 16, 64, 64, 24), ([129, 2112], [129, 2112], 4, 4, 128, 64, 12), ([512, 90], [2049, 4000], 4, 4, 120, 64, 20),
-    ([4096, 100], [4096, 100], 16, 4, 128, 64, 30), ([700], [300], 2, 2, 128, 64, 3)])
+    ([4096, 100], [4096, 100], 16, 4, 128, 64, 30), ([700], [300], 2, 2, 128, 64, 3),
+    ([2048], [2048], 16, 4, 256, 64, 16), ([2000, 77], [2000, 77], 16, 16, 136, 64, 20)])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("kind", ["normal", "ties", "special"])
 @pytest.mark.parametrize("grad", [True, False])
@@ -39,7 +40,7 @@ def test_rows_that_choose_their_chunks(monkeypatch, lens_q, lens_k, H, Hk, D, ch
     _both(monkeypatch, run)
 
 
-@pytest.mark.parametrize("D,chunks,rows,takes", [(64, 64, 2048, 1), (64, 65, 2048, 0), (96, 20, 2048, 0), (128, 20, 2048, 1), (128, 20, 8, 0)])
+@pytest.mark.parametrize("D,chunks,rows,takes", [(64, 64, 2048, 1), (64, 65, 2048, 0), (96, 20, 2048, 0), (128, 20, 2048, 1), (256, 20, 2048, 1), (128, 20, 8, 0)])
 def test_which_calls_choose_their_chunks_in_the_forward(D, chunks, rows, takes):
     f = hip.AttnFwdArgs()
     f.batch, f.total_q, f.total_k, f.heads, f.heads_k, f.head_dim = 2, 2 * rows, 128 * chunks, 8, 8, D
