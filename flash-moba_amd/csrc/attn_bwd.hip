@@ -141,7 +141,7 @@ struct DkdvSmem {
 // RANKED (partials form): part rows go to the place of the block among the row's, which the rank of the list entry gives
 // NEAR: a gathered row's place is a 32-bit byte offset from the sequence's first row that one 24-bit multiply makes (rows_near).
 template <typename T, int HD, bool DQP, bool RANKED, bool NEAR>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
+__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
   typedef DkdvSmem<HD, DQP> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR, PRB = SM::PRB;
   constexpr int NKEY = 64;   // keys of the workgroup
@@ -151,9 +151,16 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   const int gh = ws.dkv_heads, gs = a.heads / gh;  // heads of dK / dV, query heads that are added up in one
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * gh, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
-                                      longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
-  const int nb = item.idx, b = item.pair / gh, hg = item.pair - b * gh, h0 = hg * gs;
+  int nb, b, hg;
+  if (order == kListedLongestFirst) {
+    const BlockItem item = listed_item<NKEY, false>(blockIdx.x, a.batch, gh, a.max_seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k);
+    if (item.b < 0) return;
+    nb = item.idx, b = item.b, hg = item.h;
+  } else {
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * gh, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes, order == kLongestFirst);
+    nb = item.idx, b = item.pair / gh, hg = item.pair - b * gh;
+  }
+  const int h0 = hg * gs;
   const int key0 = nb * NKEY;
   const int Bn = a.lg_block_n, c = key0 / Bn;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
@@ -542,7 +549,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
 // NEAR: the host has checked that a gathered row's place in q and dout is a 32-bit byte offset from the sequence's first
 // row that one 24-bit multiply makes (launch_dkdv); otherwise the loads take 64-bit addresses per lane.
 template <typename T, int HD, int KB, bool NEAR, bool RANKED>
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws) {
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
   typedef BwdSmem<HD> SM;
   constexpr int KS = HD / 16, LDQ = SM::LDQ, LDS_ = SM::LDS_, NDT = HD / 32, VPR = HD / 8, LDR = SM::LDR;
   constexpr int NKEY = 64 * KB;         // keys of the workgroup
@@ -559,8 +566,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
   float *sLse = reinterpret_cast<float *>(smem + SM::oLse);
   float *sDelta = reinterpret_cast<float *>(smem + SM::oDelta);
 
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
-                                      longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
+  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes, order == kLongestFirst);
   const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
   const int key0 = nb * NKEY;
   // One workgroup per compute unit: nothing covers the dependent loads before the first round, so their chain is kept
@@ -1287,7 +1293,7 @@ __device__ __forceinline__ Pack8 row_buffer_load16(RowBuffer, uint32_t, int) { r
 
 // RT: 32-row tiles per wave (with two, every K^T operand read from LDS feeds two MFMAs).  NW: waves.
 template <typename T, int HD, int RT, int NW>
-__global__ __launch_bounds__(64 * NW, HD > 64 ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int row_mask, int nsb_max) {
+__global__ __launch_bounds__(64 * NW, HD > 64 ? 2 : 4) void attn_bwd_dq_kernel(fmoba_attn_bwd_args a, const uint16_t *ds_ws, const int32_t *tab, RunTable rt_, int row_mask, int nsb_max, ItemOrder order) {
   typedef DqSmem<HD, RT, NW> SM;
   constexpr int ROWS = SM::ROWS;  // query rows of the workgroup
   constexpr int LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
@@ -1306,13 +1312,20 @@ __global__ __launch_bounds__(64 * NW, HD > 64 ? 2 : 4) void attn_bwd_dq_kernel(f
   int *sMisc = reinterpret_cast<int *>(smem + SM::oMisc);
   const uint32_t ldsK = (uint32_t)(uintptr_t)(smem + SM::oK);
 
-  const DqItem wi = dq_decode_item(blockIdx.x, a.heads * a.batch, nsb_max, longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 2));
-  if (wi.pair < 0) return;
-  const int b = wi.pair / a.heads, h = wi.pair - b * a.heads, sb = wi.sb;
-  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+  int b, h, sb, q0, Lq, k0, Lk;
+  if (order == kListedLongestFirst) {
+    const BlockItem item = listed_item<ROWS, true>(blockIdx.x, a.batch, a.heads, a.max_seqlen_q, a.cu_seqlens_q, a.cu_seqlens_k);
+    if (item.b < 0) return;
+    b = item.b, h = item.h, sb = item.idx, q0 = item.q0, Lq = item.Lq, k0 = item.k0, Lk = item.Lk;
+  } else {
+    const DqItem wi = dq_decode_item(blockIdx.x, a.heads * a.batch, nsb_max, order == kLongestFirst);
+    if (wi.pair < 0) return;
+    b = wi.pair / a.heads, h = wi.pair - b * a.heads, sb = wi.sb;
+    q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+    k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+  }
   const int m0 = sb * ROWS;
   if (m0 >= Lq) return;
-  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
   const int rows_sb = min(ROWS, Lq - m0);
   const int off = Lk - Lq;
   const int D = a.head_dim;
@@ -1778,33 +1791,35 @@ __global__ void zero_f32_kernel(float *p, int64_t n) {
 }
 
 template <typename K>
-static int launch_dkdv_kernel(K kern, size_t smem, int heads, int keys, const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
+static int launch_dkdv_kernel(K kern, size_t smem, int heads, int keys, ItemOrder order, const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * heads * ceil_div(a.max_seqlen_k, keys);
+  const int64_t items = heads * (order == kListedLongestFirst ? listed_blocks(a.total_k, a.batch, keys) : (int64_t)a.batch * ceil_div(a.max_seqlen_k, keys));
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_bwd: too many (sequence, head, key block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, ws, order);
   return 0;
 }
 template <typename T, int HD, bool DQP>
 static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
+  // (one pair at a time is for sequences far beyond those that go longest first)
+  const ItemOrder order = item_order(a.total_k, a.max_seqlen_k, a.batch, ws.dkv_heads, 64, longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4));
   const bool near_rows = rows_near(a);
   auto kern = near_rows ? attn_bwd_dkdv_kernel<T, HD, DQP, false, true> : attn_bwd_dkdv_kernel<T, HD, DQP, false, false>;
   if constexpr (DQP)
     if (ws.visits != nullptr) kern = near_rows ? attn_bwd_dkdv_kernel<T, HD, DQP, true, true> : attn_bwd_dkdv_kernel<T, HD, DQP, true, false>;
-  return launch_dkdv_kernel(kern, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, a, ws, s);
+  return launch_dkdv_kernel(kern, DkdvSmem<HD, DQP>::bytes, ws.dkv_heads, 64, order, a, ws, s);
 }
 template <typename T, int HD, int KB>
 static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   const bool near_rows = rows_near(a);
   auto kern = ws.visits != nullptr ? (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, true>)
                                   : (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, false> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, false>);
-  return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB, a, ws, s);
+  return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB, longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4) ? kLongestFirst : kPairOrder, a, ws, s);
 }
 
 template <typename T, int HD, int RT, int NW>
@@ -1816,12 +1831,13 @@ static int launch_dq(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t 
     return 2;
   }
   const int nsb_max = ceil_div(a.max_seqlen_q, DqSmem<HD, RT, NW>::ROWS);
-  const int64_t items = (int64_t)a.heads * a.batch * nsb_max;
+  const ItemOrder order = item_order(a.total_q, a.max_seqlen_q, a.batch, a.heads, DqSmem<HD, RT, NW>::ROWS, longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 2));
+  const int64_t items = a.heads * (order == kListedLongestFirst ? listed_blocks(a.total_q, a.batch, DqSmem<HD, RT, NW>::ROWS) : (int64_t)a.batch * nsb_max);
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_bwd: too many (sequence, head, superblock) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * NW), smem, s, a, ws.ds, ws.tab, bwd_run_table(a), ws.row_mask, nsb_max);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * NW), smem, s, a, ws.ds, ws.tab, bwd_run_table(a), ws.row_mask, nsb_max, order);
   return 0;
 }
 

@@ -11,6 +11,7 @@
 // K and V as LDS operands, 235 us now.  What bounds it: one operand from LDS per product, and the two exchanges.
 #include "fmoba_common.h"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -32,13 +33,20 @@ struct BwdWideSmem {
 
 // NEAR: as in attn_bwd_dkdv_kernel (attn_bwd.hip)
 template <typename T, bool NEAR>
-__global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws, int row_mask) {
+__global__ __launch_bounds__(512, 2) void attn_bwd_dkdv_wide_kernel(fmoba_attn_bwd_args a, uint16_t *ds_ws, int row_mask, ItemOrder order) {
   typedef BwdWideSmem SM;
   constexpr int HD = SM::HD, KS = HD / 16, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR;
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + 63) / 64, false, longest_items_first(max(a.total_q, a.total_k), a.heads, 1024));
-  const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
+  int nb, b, h;
+  if (order == kListedLongestFirst) {
+    const BlockItem item = listed_item<64, false>(blockIdx.x, a.batch, a.heads, a.max_seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k);
+    if (item.b < 0) return;
+    nb = item.idx, b = item.b, h = item.h;
+  } else {
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + 63) / 64, false, order == kLongestFirst);
+    nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
+  }
   const int key0 = nb * 64;
   const int Bn = a.lg_block_n, c = key0 / Bn;
   const int64_t bh = (int64_t)b * a.heads + h;
@@ -281,12 +289,13 @@ static int launch_dkdv_wide(const fmoba_attn_bwd_args &a, uint16_t *ds_ws, int r
     set_error("attn_bwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_k, 64);
+  const ItemOrder order = item_order(a.total_k, a.max_seqlen_k, a.batch, a.heads, 64, longest_items_first(std::max(a.total_q, a.total_k), a.heads, 1024));
+  const int64_t items = a.heads * (order == kListedLongestFirst ? listed_blocks(a.total_k, a.batch, 64) : (int64_t)a.batch * ceil_div(a.max_seqlen_k, 64));
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_bwd: too many (sequence, head, key block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(512), smem, s, a, ds_ws, row_mask);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(512), smem, s, a, ds_ws, row_mask, order);
   return 0;
 }
 

@@ -92,15 +92,33 @@ struct FwdColSmem {
 // otherwise the row hands out slots from a counter.  The counters (a returning atomic on a line of its own per visit) and the ids
 // that the combine then needs to find the order are a tenth of the kernel (32 heads, top-k 16 of 128-key chunks, 32768 tokens: 1950 -> 1766 us,
 // 16 heads, 262144 tokens: 8.55 -> 7.43 ms), and the launch that clears them 5.5 us.
+// The blocks that exist alone, by length or by pairs (one pair at a time is for sequences far beyond these).  Pair by pair only where they are at most half: the look-up is one more load in front
+// of the lists' bounds (parts of prompts against 9216, 33000 and 20000 keys, 0.63 of the blocks 241.5 -> 243.3 us; six of 300 rows against 3000 to 60000, 0.4 202.9 -> 195.2).
+static ItemOrder col_order(const fmoba_attn_fwd_args &a, int ngrp, int hd, int kb) {
+  const bool longest_first = longest_items_first(std::max(a.total_q, a.total_k), a.heads, hd * 2);
+  const bool listed = lists_blocks(a.total_k, a.max_seqlen_k, a.batch, ngrp, kb, true) && (int64_t)a.max_seqlen_q * hd * 4 < kOnePairBytes;
+  if (listed && longest_first) return kListedLongestFirst;
+  if (listed && (int64_t)a.batch * ceil_div(a.max_seqlen_k, kb) >= 2 * listed_blocks(a.total_k, a.batch, kb)) return kListedPairs;
+  return longest_first ? kLongestFirst : kPairOrder;
+}
 template <typename T, int HD, int KB, bool FULL, bool RANKED>
-__global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp) {
+__global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp, ItemOrder order) {
   typedef FwdColSmem<HD, KB> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, KT = KB / 32, RB = HD * 2, NW = SM::NW;
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   const bool one_pair = (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes;
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * (a.heads / grp), (a.max_seqlen_k + KB - 1) / KB, one_pair,
-                                      longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 2));
-  const int ngrp = a.heads / grp, nb = item.idx, b = item.pair / ngrp, h0 = (item.pair - b * ngrp) * grp, hk = h0 / (a.heads / a.heads_k);
+  const int ngrp = a.heads / grp;
+  int nb, b, h0;
+  if (order >= kListedLongestFirst) {
+    const BlockItem item = order == kListedPairs ? listed_pair_item<KB>(blockIdx.x, a.batch, ngrp, a.max_seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k)
+                                                 : listed_item<KB, false>(blockIdx.x, a.batch, ngrp, a.max_seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k);
+    if (item.b < 0) return;
+    nb = item.idx, b = item.b, h0 = item.h * grp;
+  } else {
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * ngrp, (a.max_seqlen_k + KB - 1) / KB, one_pair, order == kLongestFirst);
+    nb = item.idx, b = item.pair / ngrp, h0 = (item.pair - b * ngrp) * grp;
+  }
+  const int hk = h0 / (a.heads / a.heads_k);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
   const int key0 = nb * KB;
   const int c = key0 / a.lg_block_n;
@@ -708,6 +726,8 @@ static int fwd_col_heads(const fmoba_attn_fwd_args &a, int kb) {
 template <typename T, int HD, int KB>
 static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStream_t s) {
   const bool ranked = ws.visits != nullptr;
+  const int grp = fwd_col_heads(a, KB);
+  const ItemOrder order = col_order(a, a.heads / grp, HD, KB);
   auto kern = a.head_dim == HD ? (ranked ? attn_fwd_col_kernel<T, HD, KB, true, true> : attn_fwd_col_kernel<T, HD, KB, true, false>)
                                : (ranked ? attn_fwd_col_kernel<T, HD, KB, false, true> : attn_fwd_col_kernel<T, HD, KB, false, false>);
   const size_t smem = FwdColSmem<HD, KB>::bytes;
@@ -715,13 +735,12 @@ static int launch_fwd_col(const fmoba_attn_fwd_args &a, const FwdWs &ws, hipStre
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int grp = fwd_col_heads(a, KB);
-  const int64_t items = (int64_t)a.batch * (a.heads / grp) * ceil_div(a.max_seqlen_k, KB);
+  const int64_t items = (a.heads / grp) * (order >= kListedLongestFirst ? listed_blocks(a.total_k, a.batch, KB) : (int64_t)a.batch * ceil_div(a.max_seqlen_k, KB));
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_fwd: too many (sequence, head, key block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * FwdColSmem<HD, KB>::NW), smem, s, a, ws, grp);
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64 * FwdColSmem<HD, KB>::NW), smem, s, a, ws, grp, order);
   return 0;
 }
 template <typename T>

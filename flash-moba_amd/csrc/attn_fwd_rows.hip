@@ -18,6 +18,7 @@
 #include "attn_fwd_rows.h"
 #include "gate_select.h"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // rings of their own; the results of a row meet in LDS at the end.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
 template <typename T, int HD, int RW, int SPLIT, bool GATED>
-__global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, RowGate gate) {
+__global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, ItemOrder order, RowGate gate) {
   typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
   constexpr int kRows = SM::ROWS;
   constexpr int KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
@@ -476,14 +477,21 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   uint32_t *sUnion = reinterpret_cast<uint32_t *>(sStep + step_cap);
   uint32_t *sBits = sUnion + nw * SM::UPW;
 
-  const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
-  const int b = item.pair / a.heads, h = item.pair - b * a.heads;
-  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
-  const int rb = nrb - 1 - item.idx;  // the longest walks (last rows of a causal sequence) start first
+  // the longest walks (last rows of a causal sequence) start first
+  int b, h, rb, q0, Lq, k0, Lk;
+  if (order == kListedLongestFirst) {
+    const BlockItem item = listed_item<kRows, true>(blockIdx.x, a.batch, a.heads, a.max_seqlen_q, a.cu_seqlens_q, a.cu_seqlens_k);
+    if (item.b < 0) return;
+    b = item.b, h = item.h, rb = item.idx, q0 = item.q0, Lq = item.Lq, k0 = item.k0, Lk = item.Lk;
+  } else {
+    const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, order == kLongestFirst);
+    b = item.pair / a.heads, h = item.pair - b * a.heads, rb = nrb - 1 - item.idx;
+    q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+    k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+  }
   const int r0 = rb * kRows;
   if (r0 >= Lq) return;
-  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
   const int off = Lk - Lq;
   const int D = a.head_dim;
   const int hk = h / (a.heads / a.heads_k);
@@ -836,12 +844,13 @@ static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, i
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_q, SM::ROWS);
+  const ItemOrder order = item_order(a.total_q, a.max_seqlen_q, a.batch, a.heads, SM::ROWS, longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4));
+  const int64_t items = a.heads * (order == kListedLongestFirst ? listed_blocks(a.total_q, a.batch, SM::ROWS) : (int64_t)a.batch * ceil_div(a.max_seqlen_q, SM::ROWS));
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_fwd: too many (sequence, head, row block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap, gate != nullptr ? *gate : RowGate{});
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap, order, gate != nullptr ? *gate : RowGate{});
   return 0;
 }
 // Four sets share a walk (head dimensions up to 64) where the workgroups of 64 rows are no more than the compute units, as their rings leave a unit

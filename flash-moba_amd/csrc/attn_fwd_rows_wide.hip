@@ -3,6 +3,8 @@
 #include "attn_fwd_rows.h"
 #include "gate_select.h"
 
+#include <algorithm>
+
 namespace fmoba {
 
 // 128 rows per workgroup, four waves of 32 rows and 512 registers, one workgroup per compute unit: a wave's 256 features of O^T are half of the
@@ -21,7 +23,7 @@ namespace fmoba {
 // the rescaling or the exponentials 3 to 5 %).  GATED as in attn_fwd_rows_kernel: forward of 2 x 4096 tokens, 8 heads, top-k 8 of 128-key chunks 178.7 -> 173.2 us, of 2048 tokens, 16 heads
 // 85.9 -> 80.4, 9000 tokens, 16 over 2 heads 343.6 -> 336.0.  The same call: columns 134 us and their combine 89 -> 171 us, training step 612 -> 530.
 template <typename T, bool GATED>
-__global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, RowGate gate) {
+__global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, ItemOrder order, RowGate gate) {
   constexpr int HD = 256, RW = 4;
   typedef FwdRowsDirectSmem<HD, RW, 1> SM;
   constexpr int kRows = SM::ROWS, KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, NI = VPR / RW;
@@ -31,14 +33,21 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
   uint32_t *sBits = sUnion + nw * SM::UPW;
   int *sAgain = reinterpret_cast<int *>(sBits + nw * kRows);  // per wave: a sum is not finite
 
-  const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
-  const int b = item.pair / a.heads, h = item.pair - b * a.heads;
-  const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
-  const int rb = nrb - 1 - item.idx;  // the longest walks (last rows of a causal sequence) start first
+  // the longest walks (last rows of a causal sequence) start first
+  int b, h, rb, q0, Lq, k0, Lk;
+  if (order == kListedLongestFirst) {
+    const BlockItem item = listed_item<kRows, true>(blockIdx.x, a.batch, a.heads, a.max_seqlen_q, a.cu_seqlens_q, a.cu_seqlens_k);
+    if (item.b < 0) return;
+    b = item.b, h = item.h, rb = item.idx, q0 = item.q0, Lq = item.Lq, k0 = item.k0, Lk = item.Lk;
+  } else {
+    const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, order == kLongestFirst);
+    b = item.pair / a.heads, h = item.pair - b * a.heads, rb = nrb - 1 - item.idx;
+    q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
+    k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+  }
   const int r0 = rb * kRows;
   if (r0 >= Lq) return;
-  const int k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
   const int off = Lk - Lq;
   const int D = a.head_dim;
   const int hk = h / (a.heads / a.heads_k);
@@ -346,12 +355,13 @@ int launch_rows_wide(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, c
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
   }
-  const int64_t items = (int64_t)a.batch * a.heads * ceil_div(a.max_seqlen_q, SM::ROWS);
+  const ItemOrder order = item_order(a.total_q, a.max_seqlen_q, a.batch, a.heads, SM::ROWS, longest_items_first(std::max(a.total_q, a.total_k), a.heads, 256 * 4));
+  const int64_t items = a.heads * (order == kListedLongestFirst ? listed_blocks(a.total_q, a.batch, SM::ROWS) : (int64_t)a.batch * ceil_div(a.max_seqlen_q, SM::ROWS));
   if (items >= ((int64_t)1 << 31)) {
     set_error("attn_fwd: too many (sequence, head, row block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, bm, nw, step_cap, gate != nullptr ? *gate : RowGate{});
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(256), smem, s, a, bm, nw, step_cap, order, gate != nullptr ? *gate : RowGate{});
   return 0;
 }
 

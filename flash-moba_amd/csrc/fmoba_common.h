@@ -552,7 +552,7 @@ constexpr long long kOnePairBytes = 64ll << 20;
 // of 2 x 4096 211 -> 195, dK/dV of 8191 tokens of short documents 55 -> 44, column forward of 8192 tokens 134 -> 114.  Where the line
 // lies: 24576 tokens, 16 heads of 128 (201 MB) dK/dV 1031 -> 1061 us, 65536 tokens (537 MB) row-block forward 2787 -> 3203.
 constexpr long long kLongestFirstBytes = 128ll << 20;
-__device__ __forceinline__ bool longest_items_first(int64_t rows, int heads, int row_bytes) { return rows * heads * row_bytes <= kLongestFirstBytes; }
+__host__ __device__ __forceinline__ bool longest_items_first(int64_t rows, int heads, int row_bytes) { return rows * heads * row_bytes <= kLongestFirstBytes; }
 struct PairItem {
   int pair, idx;
 };
@@ -572,6 +572,94 @@ __device__ __forceinline__ PairItem xcd_pair_item(int id, int npairs, int nper, 
     w.pair = id / nper;
     w.idx = id - w.pair * nper;
   }
+  return w;
+}
+
+// Uneven batches: the blocks that exist alone, of all sequences and heads, from the longest walks to the shortest.  A grid for the longest sequence's blocks in every sequence is mostly
+// workgroups that find no block, each of which takes its place (and its LDS) for as long as its first loads take; here every workgroup looks its block up, some ten
+// instructions per sequence.  Whole calls: training steps of 3000 tokens in ten sequences, 16 over 4 heads of 256 (whose workgroups have a unit each) 190.8 -> 162.8 us, of 9000 in six, 8 heads
+// of 256 383 -> 362, of 4000 in eight, 32 heads of 80 185.4 -> 173.1, 16000 in sixteen, 16 heads of 64 326.3 -> 318.4, 30000 in thirty, 8 heads of 128 484.8 -> 479.9, 2000 in four, 8 heads of
+// 64 89.5 -> 88.1; forward of 30000 in eight, 16 heads of 128, by columns 434 -> 423.6; 8191 tokens in 24 documents the same (the look-up goes through all of them).
+// For calls whose items go longest first and whose heads are whole turns of the XCDs (a head's blocks then run on one), where it leaves out a fifth of the items or more.
+constexpr int kListedBatch = 32;
+__host__ __device__ __forceinline__ int64_t listed_blocks(int64_t total, int batch, int block) { return total / block + batch; }  // at least as many as there are
+__host__ __device__ __forceinline__ bool lists_blocks(int64_t total, int longest, int batch, int heads, int block, bool longest_first) {
+  const int nper = (longest + block - 1) / block;
+  return longest_first && batch >= 2 && batch <= kListedBatch && heads % 8 == 0 && nper <= 4096 && 4 * (int64_t)batch * nper >= 5 * listed_blocks(total, batch, block);
+}
+// The order of a launch's items, which its host side chooses (the rules take a workgroup a dozen dependent instructions before its first load).
+enum ItemOrder { kPairOrder, kLongestFirst, kListedLongestFirst, kListedPairs };
+__host__ __device__ __forceinline__ ItemOrder item_order(int64_t total, int longest, int batch, int heads, int block, bool longest_first) {
+  return lists_blocks(total, longest, batch, heads, block, longest_first) ? kListedLongestFirst : longest_first ? kLongestFirst : kPairOrder;
+}
+struct BlockItem {
+  int b, h, idx;       // b < 0: none
+  int q0, Lq, k0, Lk;  // the sequence's bounds
+};
+// item `id` of listed_blocks * heads: block idx of head h of sequence b.  Blocks of query rows come from the last ones (whose walks are the longest) to the first, blocks of keys (rows =
+// false; the first are seen by most rows) from the first to the last.
+template <int BLOCK, bool ROWS>
+__device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, int longest, const int32_t *cu_q, const int32_t *cu_k) {
+  const int lane = threadIdx.x & 63, nper = (longest + BLOCK - 1) / BLOCK;
+  int q_lo = 0, q_hi = 0, k_lo = 0, k_hi = 0;
+  if (lane < batch) q_lo = cu_q[lane], q_hi = cu_q[lane + 1], k_lo = cu_k[lane], k_hi = cu_k[lane + 1];
+  const int n = id / heads;
+  const int h = (id + 8 * n) % heads;  // (a head of the same XCD; not the same shader engine in every turn)
+  const int nb = min((max(ROWS ? q_hi - q_lo : k_hi - k_lo, 0) + BLOCK - 1) / BLOCK, nper);
+  // the blocks of number r and those before them in the order
+  auto upto = [&](int r) {
+    int sum = 0;
+    for (int b = 0; b < batch; b += 8)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {  // (no blocks from lane `batch` on)
+        const int x = __builtin_amdgcn_readlane(nb, b + i);
+        sum += ROWS ? max(x - r, 0) : min(x, r + 1);
+      }
+    return sum;
+  };
+  int base = 0;
+  if (nper > 64) {
+    const int step = (nper + 63) >> 6;
+    const unsigned long long more = __ballot(upto(ROWS ? lane * step : lane * step + step - 1) > n);
+    base = step * (ROWS ? max((int)__popcll(more) - 1, 0) : 64 - (int)__popcll(more));
+  }
+  const int at = upto(base + lane);
+  const unsigned long long more = __ballot(at > n);
+  const int l = ROWS ? (int)__popcll(more) - 1 : 64 - (int)__popcll(more);
+  BlockItem w{-1, h, base + l, 0, 0, 0, 0};
+  if (l < 0 || l > 63) return w;
+  const unsigned long long have = __ballot(nb > w.idx);
+  const int k = n - (__builtin_amdgcn_readlane(at, l) - (int)__popcll(have));  // which of the sequences that have such a block
+  const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0u));
+  const unsigned long long it = __ballot(nb > w.idx && rank == k);
+  if (it == 0ull) return w;
+  w.b = (int)__ffsll(it) - 1;
+  w.q0 = __builtin_amdgcn_readlane(q_lo, w.b), w.Lq = __builtin_amdgcn_readlane(q_hi, w.b) - w.q0;
+  w.k0 = __builtin_amdgcn_readlane(k_lo, w.b), w.Lk = __builtin_amdgcn_readlane(k_hi, w.b) - w.k0;
+  return w;
+}
+
+// The same blocks of keys pair by pair, each pair's on one XCD (the order of xcd_pair_item without longest_first).
+template <int BLOCK>
+__device__ __forceinline__ BlockItem listed_pair_item(int id, int batch, int heads, int longest, const int32_t *cu_q, const int32_t *cu_k) {
+  const int lane = threadIdx.x & 63, nper = (longest + BLOCK - 1) / BLOCK, np = heads >> 3;  // np: heads of an XCD
+  int q_lo = 0, q_hi = 0, k_lo = 0, k_hi = 0;
+  if (lane < batch) q_lo = cu_q[lane], q_hi = cu_q[lane + 1], k_lo = cu_k[lane], k_hi = cu_k[lane + 1];
+  const int nb = min((max(k_hi - k_lo, 0) + BLOCK - 1) / BLOCK, nper);
+  int upto = nb;  // blocks of a head of the sequences up to this lane's
+#pragma unroll
+  for (int o = 1; o < kListedBatch; o <<= 1) {
+    const int up = __shfl_up(upto, o, 64);
+    upto += lane >= o ? up : 0;
+  }
+  const int s = id >> 3;
+  BlockItem w{-1, 0, 0, 0, 0, 0, 0};
+  const int b = (int)__popcll(__ballot(lane < batch && upto * np <= s));
+  if (b >= batch) return w;
+  const int n = __builtin_amdgcn_readlane(nb, b), rest = s - (__builtin_amdgcn_readlane(upto, b) - n) * np, pl = rest / n;
+  w.b = b, w.h = pl * 8 + (id & 7), w.idx = rest - pl * n;
+  w.q0 = __builtin_amdgcn_readlane(q_lo, b), w.Lq = __builtin_amdgcn_readlane(q_hi, b) - w.q0;
+  w.k0 = __builtin_amdgcn_readlane(k_lo, b), w.Lk = __builtin_amdgcn_readlane(k_hi, b) - w.k0;
   return w;
 }
 
