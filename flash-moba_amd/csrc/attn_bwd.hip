@@ -566,8 +566,15 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
   float *sLse = reinterpret_cast<float *>(smem + SM::oLse);
   float *sDelta = reinterpret_cast<float *>(smem + SM::oDelta);
 
-  const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes, order == kLongestFirst);
-  const int nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
+  int nb, b, h;
+  if (order == kListedLongestFirst) {
+    const BlockItem item = listed_item<NKEY, false>(blockIdx.x, a.batch, a.heads, a.max_seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k);
+    if (item.b < 0) return;
+    nb = item.idx, b = item.b, h = item.h;
+  } else {
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes, order == kLongestFirst);
+    nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
+  }
   const int key0 = nb * NKEY;
   // One workgroup per compute unit: nothing covers the dependent loads before the first round, so their chain is kept
   // short.  Where the block's column list lies depends on nothing that is loaded: asked for together with the
@@ -1819,7 +1826,8 @@ static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, h
   const bool near_rows = rows_near(a);
   auto kern = ws.visits != nullptr ? (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, true>)
                                   : (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, false> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, false>);
-  return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB, longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4) ? kLongestFirst : kPairOrder, a, ws, s);
+  return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB,
+                            item_order(a.total_k, a.max_seqlen_k, a.batch, a.heads, 64 * KB, longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4)), a, ws, s);
 }
 
 template <typename T, int HD, int RT, int NW>

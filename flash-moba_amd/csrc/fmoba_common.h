@@ -577,9 +577,9 @@ __device__ __forceinline__ PairItem xcd_pair_item(int id, int npairs, int nper, 
 
 // Uneven batches: the blocks that exist alone, of all sequences and heads, from the longest walks to the shortest.  A grid for the longest sequence's blocks in every sequence is mostly
 // workgroups that find no block, each of which takes its place (and its LDS) for as long as its first loads take; here every workgroup looks its block up, some ten
-// instructions per sequence.  Whole calls: training steps of 3000 tokens in ten sequences, 16 over 4 heads of 256 (whose workgroups have a unit each) 190.8 -> 162.8 us, of 9000 in six, 8 heads
+// instructions per sequence.  Whole calls: training steps of 3000 tokens in ten sequences, 16 over 4 heads of 256 (whose workgroups have a unit each) 192 -> 167 us, of 9000 in six, 8 heads
 // of 256 383 -> 362, of 4000 in eight, 32 heads of 80 185.4 -> 173.1, 16000 in sixteen, 16 heads of 64 326.3 -> 318.4, 30000 in thirty, 8 heads of 128 484.8 -> 479.9, 2000 in four, 8 heads of
-// 64 89.5 -> 88.1; forward of 30000 in eight, 16 heads of 128, by columns 434 -> 423.6; 8191 tokens in 24 documents the same (the look-up goes through all of them).
+// 64 89.5 -> 88.1; forward of 30000 in eight, 16 heads of 128, by columns 434 -> 423.6; 8191 tokens in 24 documents the same (the look-up goes through all of them), 13400 in eight, 8 heads of 128 339 -> 344.
 // For calls whose items go longest first and whose heads are whole turns of the XCDs (a head's blocks then run on one), where it leaves out a fifth of the items or more.
 constexpr int kListedBatch = 32;
 __host__ __device__ __forceinline__ int64_t listed_blocks(int64_t total, int batch, int block) { return total / block + batch; }  // at least as many as there are
@@ -604,7 +604,7 @@ __device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, i
   int q_lo = 0, q_hi = 0, k_lo = 0, k_hi = 0;
   if (lane < batch) q_lo = cu_q[lane], q_hi = cu_q[lane + 1], k_lo = cu_k[lane], k_hi = cu_k[lane + 1];
   const int n = id / heads;
-  const int h = (id + 8 * n) % heads;  // (a head of the same XCD; not the same shader engine in every turn)
+  const int h = id - n * heads;
   const int nb = min((max(ROWS ? q_hi - q_lo : k_hi - k_lo, 0) + BLOCK - 1) / BLOCK, nper);
   // the blocks of number r and those before them in the order
   auto upto = [&](int r) {
@@ -629,7 +629,9 @@ __device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, i
   BlockItem w{-1, h, base + l, 0, 0, 0, 0};
   if (l < 0 || l > 63) return w;
   const unsigned long long have = __ballot(nb > w.idx);
-  const int k = n - (__builtin_amdgcn_readlane(at, l) - (int)__popcll(have));  // which of the sequences that have such a block
+  // Which of the sequences that have such a block: rotated by one from number to number, as in xcd_pair_item and for the same reason (30000 tokens in four sequences, 8 heads, dK/dV with partials:
+  // training step 804 us, 865 without).
+  const int some = (int)__popcll(have), k = (n - (__builtin_amdgcn_readlane(at, l) - some) + w.idx) % max(some, 1);
   const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0u));
   const unsigned long long it = __ballot(nb > w.idx && rank == k);
   if (it == 0ull) return w;
