@@ -686,7 +686,8 @@ __global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
 template <bool PREFIX>
 __device__ __forceinline__ void rank_rows(const TopkParams &p, int h, int b, int blk, int nblk, int row0, int rows) {
   const fmoba_fused_topk_args &a = p.a;
-  const int tid = threadIdx.x, nthr = blockDim.x;
+  constexpr int nthr = 256;
+  const int tid = threadIdx.x;
   const int q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
   const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b], last = (Lk + a.chunk - 1) / a.chunk - 1;  // the sequence's last chunk
   {
@@ -909,8 +910,10 @@ __global__ __launch_bounds__(64) void csc_fill_kernel(TopkParams p) {
 // empty, and one wave per segment walks four times as far: 8192 tokens, 16 heads, ranked lists of 128-key chunks, scan and fill 17.6 us, one wave per segment 15.1, this 10.0 (four waves of
 // eight chunks each, which read the words below four times: 10.9, and 23 where this takes 19); parts of prompts of 1024 rows against 9000 to 33000 keys, 32 heads
 // 22.0 -> 19.4; 8191 tokens of short documents, plain lists 10.7 -> 4.8.  More counts, or longer segments (which calls of many waves have), go to the two launches: there the
-// scan is a small part of the time and the counts of a workgroup would be a large one.
-constexpr int kListCounts = 4096, kListWords = 16, kListSegRows = 256;
+// scan is a small part of the time and the counts of a workgroup would be a large one.  So do calls of many workgroups, each of which counts for itself,
+// earlier where ranks are made beside the lists: ranked, 9856 of them 28.2 us against 21.4 and 5120 of them 22.7 against 18.7, while 3840 win (above); plain, 4800 of them
+// (12037 tokens, 16 heads) 11.8 against 18.0, and 11200 (24571 tokens, 32 heads) as long as the two launches.
+constexpr int kListCounts = 4096, kListWords = 16, kListSegRows = 256, kListGroups = 8192, kListRankedGroups = 4096;
 template <bool RANKED>
 __global__ __launch_bounds__(256) void csc_lists_kernel(TopkParams p) {
   const fmoba_fused_topk_args &a = p.a;
@@ -1296,7 +1299,8 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   if (rc) return rc;
   FMOBA_LAUNCH_CHECK("topk_gate_kernel");
   if (!lists) return 0;
-  if ((int64_t)p.nseg * max_cols <= kListCounts && p.W <= kListWords && p.seg_rows == kListSegRows) {
+  const int64_t list_groups = (int64_t)p.nseg * (p.W + (ranks ? 1 : 0)) * a->heads * a->batch;
+  if ((int64_t)p.nseg * max_cols <= kListCounts && p.W <= kListWords && p.seg_rows == kListSegRows && list_groups <= (ranks ? kListRankedGroups : kListGroups)) {
     hipLaunchKernelGGL(ranks ? csc_lists_kernel<true> : csc_lists_kernel<false>, dim3(p.nseg * p.W + (ranks ? p.nseg : 0), a->heads, a->batch), dim3(256), 0, s, p);
   } else {
     if (ranks)
