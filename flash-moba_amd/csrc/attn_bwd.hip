@@ -548,8 +548,10 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_ar
 // leaves one dQ partial instead of two.
 // NEAR: the host has checked that a gathered row's place in q and dout is a 32-bit byte offset from the sequence's first
 // row that one 24-bit multiply makes (launch_dkdv); otherwise the loads take 64-bit addresses per lane.
-template <typename T, int HD, int KB, bool NEAR, bool RANKED>
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
+// LISTED: the block is looked up (listed_item).  An instance of its own, for ranked lists with NEAR: with the look-up as a branch beside the other decoding every launch was
+// slower (256 and 237 registers either way; 32768 tokens, 32 heads: 3.77 ms against 3.54).
+template <typename T, int HD, int KB, bool NEAR, bool RANKED, bool LISTED>
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder) {
   typedef BwdSmem<HD> SM;
   constexpr int KS = HD / 16, LDQ = SM::LDQ, LDS_ = SM::LDS_, NDT = HD / 32, VPR = HD / 8, LDR = SM::LDR;
   constexpr int NKEY = 64 * KB;         // keys of the workgroup
@@ -567,12 +569,13 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
   float *sDelta = reinterpret_cast<float *>(smem + SM::oDelta);
 
   int nb, b, h;
-  if (order == kListedLongestFirst) {
+  if constexpr (LISTED) {
     const BlockItem item = listed_item<NKEY, false>(blockIdx.x, a.batch, a.heads, a.max_seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k);
     if (item.b < 0) return;
     nb = item.idx, b = item.b, h = item.h;
   } else {
-    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes, order == kLongestFirst);
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
+                                        longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
     nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
   }
   const int key0 = nb * NKEY;
@@ -1824,10 +1827,15 @@ static int launch_dkdv(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_
 template <typename T, int HD, int KB>
 static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   const bool near_rows = rows_near(a);
-  auto kern = ws.visits != nullptr ? (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, true>)
-                                  : (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, false> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, false>);
-  return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB,
-                            item_order(a.total_k, a.max_seqlen_k, a.batch, a.heads, 64 * KB, longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4)), a, ws, s);
+  const bool longest_first = longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4);
+  // Workgroups of one to a unit, whose empty ones come last: looking blocks up pays where two thirds of them are empty (30000 tokens in twelve sequences, 8 heads, 4.5 times as many as there
+  // are blocks: step 440 -> 427 us; 1.5 to 2.2 times as many: 12846, 5768, 4917 and 6469 tokens 783 -> 790, 15400 in eight 344.7 -> 347.2, 15004 in five and 8999 in eight, 16 heads, the same).
+  const bool listed = near_rows && ws.visits != nullptr && lists_blocks(a.total_k, a.max_seqlen_k, a.batch, a.heads, 64 * KB, longest_first) &&
+                      (int64_t)a.batch * ceil_div(a.max_seqlen_k, 64 * KB) >= 3 * listed_blocks(a.total_k, a.batch, 64 * KB);
+  auto kern = listed                  ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true, true>
+              : ws.visits != nullptr ? (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true, false> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, true, false>)
+                                     : (near_rows ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, false, false> : attn_bwd_dkdv_partials_kernel<T, HD, KB, false, false, false>);
+  return launch_dkdv_kernel(kern, BwdSmem<HD>::bytes, a.heads, 64 * KB, listed ? kListedLongestFirst : longest_first ? kLongestFirst : kPairOrder, a, ws, s);
 }
 
 template <typename T, int HD, int RT, int NW>

@@ -579,7 +579,7 @@ __device__ __forceinline__ PairItem xcd_pair_item(int id, int npairs, int nper, 
 // workgroups that find no block, each of which takes its place (and its LDS) for as long as its first loads take; here every workgroup looks its block up, some ten
 // instructions per sequence.  Whole calls: training steps of 3000 tokens in ten sequences, 16 over 4 heads of 256 (whose workgroups have a unit each) 192 -> 167 us, of 9000 in six, 8 heads
 // of 256 383 -> 362, of 4000 in eight, 32 heads of 80 185.4 -> 173.1, 16000 in sixteen, 16 heads of 64 326.3 -> 318.4, 30000 in thirty, 8 heads of 128 484.8 -> 479.9, 2000 in four, 8 heads of
-// 64 89.5 -> 88.1; forward of 30000 in eight, 16 heads of 128, by columns 434 -> 423.6; 8191 tokens in 24 documents the same (the look-up goes through all of them), 13400 in eight, 8 heads of 128 339 -> 344.
+// 64 89.5 -> 88.1; forward of 30000 in eight, 16 heads of 128, by columns 434 -> 423.6; 13400 in eight, 8 heads of 128 354 -> 337; 8191 tokens in 24 documents the same (the look-up goes through all of them).
 // For calls whose items go longest first and whose heads are whole turns of the XCDs (a head's blocks then run on one), where it leaves out a fifth of the items or more.
 constexpr int kListedBatch = 32;
 __host__ __device__ __forceinline__ int64_t listed_blocks(int64_t total, int batch, int block) { return total / block + batch; }  // at least as many as there are

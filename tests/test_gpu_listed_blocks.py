@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
     ([1300, 40], 8, 8, 64, 64, 4, 0), ([0, 700, 0, 64, 65, 1, 0], 16, 4, 128, 64, 3, 0), ([900] + [30 + i for i in range(31)], 8, 8, 64, 64, 3, 0),
     ([900] + [30 + i for i in range(32)], 8, 8, 64, 64, 3, 0), ([4097, 100, 5], 8, 8, 64, 64, 20, 0), ([4160, 64, 63], 8, 2, 64, 64, 3, 0), ([100, 3000, 129], 16, 16, 96, 128, 2, 0),
     ([100, 2600, 127, 300], 8, 8, 128, 128, 2, 0), ([1500, 256, 20, 257, 90], 16, 8, 256, 64, 8, 0), ([40, 2100, 200], 8, 8, 200, 64, 2, 0), ([500, 20, 30], 24, 8, 128, 64, 3, 5000),
-    ([8200, 33, 40], 8, 1, 64, 64, 2, 0)])
+    ([8200, 33, 40], 8, 1, 64, 64, 2, 0), ([60, 3000, 40, 20, 130], 8, 8, 128, 64, 2, 0), ([6500, 127, 40, 20], 16, 4, 128, 128, 2, 0)])
 def test_every_block_once(lens, H, Hk, D, chunk, topk, bound):
     g = torch.Generator(device="cuda").manual_seed(sum(lens) + D)
     mk = lambda h: torch.randn((sum(lens), h, D), generator=g, device="cuda").to(torch.bfloat16)
