@@ -140,8 +140,10 @@ struct DkdvSmem {
 
 // RANKED (partials form): part rows go to the place of the block among the row's, which the rank of the list entry gives
 // NEAR: a gathered row's place is a 32-bit byte offset from the sequence's first row that one 24-bit multiply makes (rows_near).
+// Three waves per SIMD for the dS form of heads up to 64, whose LDS takes three workgroups to a unit: the compiler's own choice for rows far apart was 182 registers (166 now) and two waves,
+// backward of 8191 tokens, 16 heads 248 us against 236, of 16384, 32 heads 1264 against 1223.
 template <typename T, int HD, bool DQP, bool RANKED, bool NEAR>
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
+__global__ __launch_bounds__(256, HD <= 64 && !DQP ? 3 : 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
   typedef DkdvSmem<HD, DQP> SM;
   constexpr int KS = HD / 16, NDT = HD / 32, VPR = HD / 8, RB = HD * 2, LDR = SM::LDR, PRB = SM::PRB;
   constexpr int NKEY = 64;   // keys of the workgroup
