@@ -281,6 +281,12 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
       constexpr int IB = (NT * 32 <= 64) ? 6 : (NT * 32 <= 128 ? 7 : 8);
       for (int bit = IB - 1; bit >= 0; --bit) {
         const uint32_t trial = i_acc | (1u << bit);
+        // (Made anew in every turn: the flags of 128 and 256 scores, the same in all of them, were kept in scalar registers beside the loop, which took them from the whole kernel: 79 and
+        // 223 scalars spilled, in a path that next to no row takes.  Gate of 32384 tokens, 16 heads, 256 chunks 138 -> 124 us for heads of 64 and 152 -> 138 of 128, 128 chunks 80 -> 75.5.)
+        float eq = tau_eq;
+#if defined(__HIP_DEVICE_COMPILE__)
+        if constexpr (NT > 2) asm volatile("" : "+v"(eq));
+#endif
         int cnt = 0;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
@@ -288,7 +294,7 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
               const uint32_t c = (uint32_t)(t * 32 + acc_row(i, hh));
-              cnt += ((sc[t][i] == tau_eq) & (c >= trial)) ? 1 : 0;
+              cnt += ((sc[t][i] == eq) & (c >= trial)) ? 1 : 0;
             }
           }
         cnt = sum_xor32_i(cnt);

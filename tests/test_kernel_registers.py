@@ -32,3 +32,10 @@ def test_dkdv_of_narrow_heads_keeps_three_waves_per_simd(dtype, near):
     # 512 registers per SIMD lane, given out in eights: three waves of at most 168
     for k in _matching("attn_bwd_dkdv_kernelI%sLi64ELb0ELb0ELb%dE" % (dtype, near)):
         assert k[".vgpr_count"] <= 168 and k[".vgpr_spill_count"] == 0
+
+
+@pytest.mark.parametrize("chunks", [64, 128, 256])
+def test_gate_spills_nothing(chunks):
+    for k in _matching("topk_gate_kernelI"):
+        if "ELi%dEEEv" % (chunks // 32) in k[".name"]:
+            assert (k[".sgpr_spill_count"], k[".vgpr_spill_count"], k[".private_segment_fixed_size"]) == (0, 0, 0), k[".name"]
