@@ -928,7 +928,7 @@ size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a) {
 // Calls whose rows can choose their chunks in attn_fwd_rows_kernel: the scores of a row are two tiles of products with the operands that Q already is (tiles of 96
 // features have them in another order), calls of a few rows have a gate of their own.
 bool fwd_rows_gated(const fmoba_attn_fwd_args &a) {
-  return a.selection_bits == nullptr && a.max_cols <= kRowGateChunks && a.max_seqlen_q > kFewRows && !fwd_few_rows(a) && fwd_rows_direct(a) &&
+  return a.max_cols <= kRowGateChunks && a.max_seqlen_q > kFewRows && !fwd_few_rows(a) && fwd_rows_direct(a) &&
          (a.head_dim <= 64 || a.head_dim > 96);
 }
 int run_fwd_rows_gated(const fmoba_attn_fwd_args &a, const RowGate &gate, hipStream_t s) {

@@ -68,3 +68,11 @@ def test_visits_in_lds(lens, heads, lds):
                                                ([2112], 8, 64, 2), ([1024], 8, 72, 2), ([8192], 8, 32, 2), ([8832], 8, 64, 1), ([4480], 8, 128, 2), ([4736], 8, 128, 1)])
 def test_sets_of_a_walk(lens, heads, D, sets):
     assert H.load_library().fmoba_attn_fwd_row_sets(ctypes.byref(fwd_args(lens, 64, 16, heads=heads, D=D))) == sets
+
+
+# the form that chooses its rows' chunks itself reads no selection bits: a struct that still holds some from another call is of the form as well
+@pytest.mark.parametrize("lens,D,gated", [([2048], 64, 1), ([4096], 128, 1), ([2048], 256, 1), ([2048], 96, 0), ([4160], 64, 0)])
+def test_gated_row_blocks_whatever_selection_bits(lens, D, gated):
+    f = fwd_args(lens, 64, 20, heads=16, D=D)
+    for f.selection_bits in (None, 4096):
+        assert H.load_library().fmoba_attn_fwd_gates_rows(ctypes.byref(f)) == gated
