@@ -200,7 +200,7 @@ extern "C" int fmoba_chunk_offsets(const int32_t *cu_seqlens, int32_t *cu_seqlen
   return 0;
 }
 
-// `extra`: cu_km and clear_* of PoolExtra
+// `extra`: cu_km and clear_* of PoolExtra.  `few`: scores in place of the means (km and its strides are not looked at)
 static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &extra, void *stream, const fmoba::FewGate *few = nullptr) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "mean_pool: null args");
@@ -210,10 +210,10 @@ static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &
   FMOBA_REQUIRE(a->head_dim > 0 && a->head_dim % 8 == 0, "mean_pool: head_dim must be a multiple of 8");
   FMOBA_REQUIRE(a->heads_k > 0, "mean_pool: heads_k must be positive");
   if (a->max_chunks <= 0) return 0;
-  FMOBA_REQUIRE(a->k && a->km && a->cu_seqlens_k && a->cu_seqlens_km, "mean_pool: null pointer");
-  FMOBA_REQUIRE(a->k_row_stride % 8 == 0 && a->k_head_stride % 8 == 0 && a->km_row_stride % 8 == 0 && a->km_head_stride % 8 == 0,
+  FMOBA_REQUIRE(a->k && (a->km || few != nullptr) && a->cu_seqlens_k && a->cu_seqlens_km, "mean_pool: null pointer");
+  FMOBA_REQUIRE(a->k_row_stride % 8 == 0 && a->k_head_stride % 8 == 0 && (few != nullptr || (a->km_row_stride % 8 == 0 && a->km_head_stride % 8 == 0)),
                 "mean_pool: strides must be multiples of 8 elements (16-byte vectors)");
-  FMOBA_REQUIRE(((uintptr_t)a->k % 16) == 0 && ((uintptr_t)a->km % 16) == 0, "mean_pool: k and km must be 16-byte aligned");
+  FMOBA_REQUIRE(((uintptr_t)a->k % 16) == 0 && (few != nullptr || ((uintptr_t)a->km % 16) == 0), "mean_pool: k and km must be 16-byte aligned");
   const int nvec = a->heads_k * (a->head_dim / 8);
   dim3 grid(a->max_chunks, a->batch, ceil_div(nvec, 64));
   FMOBA_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "mean_pool: batch or heads*dim too large for the launch grid");

@@ -188,10 +188,10 @@ Result forward_few(const Shape &s, fmoba_attn_fwd_args a, const Tensor &q, const
   const Tensor scratch = bytes_like(q, cu_bytes + score_bytes + 256);
   char *base = reinterpret_cast<char *>(up256(reinterpret_cast<size_t>(scratch.data_ptr())));
   fmoba_mean_pool_args m{};
-  m.k = a.k, m.km = base + cu_bytes;  // (not written)
+  m.k = a.k;
   m.cu_seqlens_k = a.cu_seqlens_k, m.cu_seqlens_km = reinterpret_cast<int32_t *>(base);
   m.batch = s.batch, m.max_chunks = s.max_cols, m.heads_k = s.heads_k, m.head_dim = s.dim, m.chunk = s.chunk, m.dtype = s.dtype;
-  m.k_row_stride = k.stride(0), m.k_head_stride = k.stride(1), m.km_row_stride = s.heads_k * s.dim, m.km_head_stride = s.dim;
+  m.k_row_stride = k.stride(0), m.k_head_stride = k.stride(1);
   t_visits = a.max_visits_per_row, t_row_blocks = 1;
   check(fmoba_attn_fwd_gated_few(&m, &a, topk, s.causal, reinterpret_cast<float *>(base + cu_bytes), s.stream));
   return r;

@@ -216,7 +216,7 @@ int fmoba_attn_fwd_ranked(const fmoba_attn_fwd_args *a, const uint32_t *visits, 
 /* Gate and attention of a call with a few query rows per sequence (decode steps) in two launches: the pooling pass leaves a score per (row, chunk) in
  * place of the chunk means, the attention picks a row's chunks from them.  The result is that of fmoba_pool_and_gate and fmoba_attn_fwd to the last bit.
  * fmoba_attn_fwd_gated_few_bytes: bytes of `scores` (sizes, strides and fwd_mode of `a` are read), 0 for calls that are not of this form.  `m` as for
- * fmoba_pool_and_gate: the same problem, cu_seqlens_km is written, m->km is not; no list, selection bits or workspace of `a` are
+ * fmoba_pool_and_gate: the same problem, cu_seqlens_km is written, m->km and its strides are not used; no list, selection bits or workspace of `a` are
  * read.  gate_is_causal: the gating's is_causal (that of `a` is the attention's).  No counterpart in the reference. */
 size_t fmoba_attn_fwd_gated_few_bytes(const fmoba_attn_fwd_args *a);
 int fmoba_attn_fwd_gated_few(const fmoba_mean_pool_args *m, const fmoba_attn_fwd_args *a, int32_t topk, int32_t gate_is_causal, float *scores, void *stream);

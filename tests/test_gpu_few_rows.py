@@ -115,3 +115,31 @@ def test_which_calls_the_pooling_pass_scores(heads, heads_k, dim, rows, takes):
     f.batch, f.total_q, f.total_k, f.heads, f.heads_k, f.head_dim = 4, 4 * rows, 4 << 16, heads, heads_k, dim
     f.max_seqlen_q, f.max_seqlen_k, f.max_cols, f.lg_block_n, f.is_causal, f.max_visits_per_row = rows, 1 << 16, 512, 128, 1, 8
     assert (hip.load_library().fmoba_attn_fwd_gated_few_bytes(f) > 0) == takes
+
+
+def _fwd_args(lens_q, lens_k, H, Hk, D, chunk, topk, causal=True):
+    """The sizes of a call of flash_moba_varlen_func."""
+    f = hip.AttnFwdArgs()
+    f.batch, f.total_q, f.total_k, f.heads, f.heads_k, f.head_dim = len(lens_q), sum(lens_q), sum(lens_k), H, Hk, D
+    f.max_seqlen_q, f.max_seqlen_k, f.max_cols, f.lg_block_m, f.lg_block_n = max(lens_q), max(lens_k), -(-max(lens_k) // chunk), 128, chunk
+    f.is_causal, f.max_visits_per_row = int(causal and max(lens_q) != 1), topk * (chunk // hip.fwd_key_block(chunk))
+    f.q_row_stride = f.o_row_stride = H * D
+    f.k_row_stride = f.v_row_stride = Hk * D
+    f.q_head_stride = f.k_head_stride = f.v_head_stride = f.o_head_stride = D
+    return f
+
+
+def test_the_entry_point_needs_no_place_for_chunk_means(monkeypatch):
+    lens_q, lens_k, H, Hk, D, chunk, topk = [1, 2], [5000, 900], 8, 2, 128, 64, 5
+    q, k, v, cuq, cuk = (t.cuda() for t in _case(lens_q, lens_k, H, Hk, D, torch.bfloat16, 5))
+    f, lib, stream = _fwd_args(lens_q, lens_k, H, Hk, D, chunk, topk), hip.load_library(), torch.cuda.current_stream().cuda_stream
+    f.dtype, f.softmax_scale = 1, D ** -0.5  # (bf16)
+    out, lse = torch.empty_like(q), torch.empty((H, sum(lens_q)), device="cuda")
+    scores = torch.empty(lib.fmoba_attn_fwd_gated_few_bytes(f), dtype=torch.uint8, device="cuda")
+    cu_km = torch.empty_like(cuk)
+    f.q, f.k, f.v, f.out, f.softmax_lse, f.cu_seqlens_q, f.cu_seqlens_k = (t.data_ptr() for t in (q, k, v, out, lse, cuq, cuk))
+    m = hip.MeanPoolArgs(k=f.k, cu_seqlens_k=f.cu_seqlens_k, cu_seqlens_km=cu_km.data_ptr(), batch=f.batch, max_chunks=f.max_cols, heads_k=Hk, head_dim=D, chunk=chunk,
+                         dtype=f.dtype, k_row_stride=f.k_row_stride, k_head_stride=D)
+    assert lib.fmoba_attn_fwd_gated_few(m, f, topk, 1, scores.data_ptr(), stream) == 0, lib.fmoba_last_error()
+    want = _both(monkeypatch, lambda: (flash_moba.flash_moba_varlen_func(q, k, v, cuq, cuk, max(lens_q), max(lens_k), chunk, topk, causal=True),))[0]
+    assert torch.equal(out, want)
