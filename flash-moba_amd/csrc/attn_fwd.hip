@@ -75,6 +75,16 @@ struct FwdColSmem {
   static_assert(bytes * (8 / NW) <= 160 * 1024, "eight waves per compute unit");
 };
 
+// The blocks that exist alone, by length or by pairs (one pair at a time is for sequences far beyond these).  Pair by pair only where they are at most half: the look-up is one more load in front
+// of the lists' bounds (parts of prompts against 9216, 33000 and 20000 keys, 0.63 of the blocks 241.5 -> 243.3 us; six of 300 rows against 3000 to 60000, 0.4 202.9 -> 195.2).
+static ItemOrder col_order(const fmoba_attn_fwd_args &a, int ngrp, int hd, int kb) {
+  const bool longest_first = longest_items_first(std::max(a.total_q, a.total_k), a.heads, hd * 2);
+  const bool listed = lists_blocks(a.total_k, a.max_seqlen_k, a.batch, ngrp, kb, true) && (int64_t)a.max_seqlen_q * hd * 4 < kOnePairBytes;
+  if (listed && longest_first) return kListedLongestFirst;
+  if (listed && (int64_t)a.batch * ceil_div(a.max_seqlen_k, kb) >= 2 * listed_blocks(a.total_k, a.batch, kb)) return kListedPairs;
+  return longest_first ? kLongestFirst : kPairOrder;
+}
+
 // Two workgroups per compute unit, two waves per SIMD, no barrier after the block's K and V have arrived.  What bounds it
 // depends on the lists.  Long ones (32768 tokens, 32 heads, top-k 16 of 256 chunks: 2000 rows per list): the partial
 // results on their way out and the gathered Q rows, together about 4 TB/s.  Short ones (a part of a prompt against the
@@ -92,15 +102,6 @@ struct FwdColSmem {
 // otherwise the row hands out slots from a counter.  The counters (a returning atomic on a line of its own per visit) and the ids
 // that the combine then needs to find the order are a tenth of the kernel (32 heads, top-k 16 of 128-key chunks, 32768 tokens: 1950 -> 1766 us,
 // 16 heads, 262144 tokens: 8.55 -> 7.43 ms), and the launch that clears them 5.5 us.
-// The blocks that exist alone, by length or by pairs (one pair at a time is for sequences far beyond these).  Pair by pair only where they are at most half: the look-up is one more load in front
-// of the lists' bounds (parts of prompts against 9216, 33000 and 20000 keys, 0.63 of the blocks 241.5 -> 243.3 us; six of 300 rows against 3000 to 60000, 0.4 202.9 -> 195.2).
-static ItemOrder col_order(const fmoba_attn_fwd_args &a, int ngrp, int hd, int kb) {
-  const bool longest_first = longest_items_first(std::max(a.total_q, a.total_k), a.heads, hd * 2);
-  const bool listed = lists_blocks(a.total_k, a.max_seqlen_k, a.batch, ngrp, kb, true) && (int64_t)a.max_seqlen_q * hd * 4 < kOnePairBytes;
-  if (listed && longest_first) return kListedLongestFirst;
-  if (listed && (int64_t)a.batch * ceil_div(a.max_seqlen_k, kb) >= 2 * listed_blocks(a.total_k, a.batch, kb)) return kListedPairs;
-  return longest_first ? kLongestFirst : kPairOrder;
-}
 template <typename T, int HD, int KB, bool FULL, bool RANKED>
 __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col_kernel(fmoba_attn_fwd_args a, FwdWs ws, int grp, ItemOrder order) {
   typedef FwdColSmem<HD, KB> SM;

@@ -15,7 +15,6 @@
 namespace fmoba {
 
 constexpr int kFewWaves = 8;
-constexpr int kFewMaxCols = kFewChunks;  // (the row's list of chunks lies in LDS)
 
 // sum over the LPR consecutive lanes that share a key, in all of them
 template <int LPR>
@@ -115,8 +114,8 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void attn_fwd_few_kernel(fmoba_a
   constexpr int LPR = HD / 8, KPI = 64 / LPR;  // lanes per key, keys per load instruction
   constexpr int NIN = HD == 64 ? 8 : 16;       // load instructions per unit and operand
   constexpr int BK = NIN * KPI;                // keys per unit
-  __shared__ int sChunk[SCORED ? 128 : kFewMaxCols];       // (top-k is at most 64)
-  __shared__ uint32_t sKeys[SCORED ? kFewMaxCols : 1];
+  __shared__ int sChunk[SCORED ? 128 : kFewChunks];        // (top-k is at most 64)
+  __shared__ uint32_t sKeys[SCORED ? kFewChunks : 1];
   __shared__ int sCount;
   __shared__ float sAcc[kFewWaves][HD], sM[kFewWaves], sL[kFewWaves];
   const int h = blockIdx.x, t = blockIdx.y;
@@ -260,7 +259,7 @@ __global__ __launch_bounds__(64 * kFewWaves, 2) void attn_fwd_few_kernel(fmoba_a
 // little: at most eight query rows per sequence, and no more to read than the keys and values of the call are (twice, if
 // a row's bound counts chunks it does not have).
 bool fwd_few_rows(const fmoba_attn_fwd_args &a) {
-  if (a.max_seqlen_q > 8 || a.max_cols > kFewMaxCols || a.max_cols < 1 || a.lg_block_n % 64 != 0 || a.total_q > 65535) return false;
+  if (a.max_seqlen_q > kFewRows || a.max_cols > kFewChunks || a.max_cols < 1 || a.lg_block_n % 64 != 0 || a.total_q > 65535) return false;
   const int64_t unit = a.lg_block_n % 128 == 0 ? 128 : 64;
   const int64_t chunk_rows = (int64_t)a.max_visits_per_row * unit;  // keys a row may select
   const int64_t per_row = chunk_rows < a.max_seqlen_k ? chunk_rows : a.max_seqlen_k;

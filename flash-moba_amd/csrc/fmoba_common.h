@@ -976,6 +976,7 @@ struct RowGate {
   int32_t W, nseg, seg_rows;
 };
 constexpr int kRowGateChunks = 64;  // chunks per sequence that it takes, at most
-constexpr int kFewRows = 8, kFewChunks = 4096;  // query rows and chunks per sequence of such a call, at most
+// Query rows and chunks per sequence of a call of a few rows, at most: for its gate, its attention and the two as one (topk_csc.hip, attn_fwd_few.hip), which the row-block form leaves them to.
+constexpr int kFewRows = 8, kFewChunks = 4096;
 
 }  // namespace fmoba

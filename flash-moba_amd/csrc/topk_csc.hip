@@ -9,6 +9,7 @@
 //                      the row-list buffer.
 //   csc_fill_kernel  : walks the bit columns in row order and writes each chunk's row list
 //                      ascending, so no sort pass is needed afterwards.
+//   csc_lists_kernel : the two in one launch, for calls with few counts per (sequence, head).
 #include "gate_select.h"
 
 #include <algorithm>
@@ -562,8 +563,6 @@ __global__ __launch_bounds__(256, HD > 128 || PL > 16 ? 2 : 3) void topk_gate_st
 // the same as above, so are the scores, and the order (score descending, chunk descending) is total: the same selection.
 // 20 -> 13.6 us there.
 // ------------------------------------------------------------------------------------
-constexpr int kFewGateRows = 8, kFewGateChunks = 4096;
-
 // NJ: chunks per lane of a row's wave
 template <typename T, int HD, int NJ>
 __global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
@@ -573,7 +572,7 @@ __global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
   const fmoba_fused_topk_args &a = p.a;
   const int h = blockIdx.x, b = blockIdx.y;
   const int q0 = a.cu_seqlens_q[b];
-  const int Lq = min(a.cu_seqlens_q[b + 1] - q0, a.max_seqlen_q);  // (at most kFewGateRows)
+  const int Lq = min(a.cu_seqlens_q[b + 1] - q0, a.max_seqlen_q);  // (at most kFewRows)
   if (Lq <= 0) return;
   const int Lk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b];
   const int km0 = a.cu_seqlens_km[b];
@@ -1154,7 +1153,7 @@ static int launch_gate_stream_hd(const TopkParams &p, dim3 grid, hipStream_t s) 
 }
 template <typename T, int HD, int NJ>
 static int launch_gate_few_nj(const TopkParams &p, hipStream_t s) {
-  const size_t smem = (size_t)std::min(p.a.max_seqlen_q, kFewGateRows) * NJ * 64 * 4;
+  const size_t smem = (size_t)std::min(p.a.max_seqlen_q, kFewRows) * NJ * 64 * 4;
   auto kern = topk_gate_few_kernel<T, HD, NJ>;
   if (smem > 32 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("fused_topk: cannot reserve %zu bytes of LDS", smem);
@@ -1290,18 +1289,19 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
   if (attn != nullptr)
     rc = run_fwd_rows_gated(*attn, RowGate{reinterpret_cast<const uint16_t *>(a->km), a->cu_seqlens_km, a->km_row_stride, a->km_head_stride, a->topk, lists ? p.sel : nullptr, p.segcnt, p.W,
                                            p.nseg, p.seg_rows}, s);
-  else if (a->max_seqlen_q <= kFewGateRows && max_cols <= kFewGateChunks)
+  else if (a->max_seqlen_q <= kFewRows && max_cols <= kFewChunks)
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_few_hd<bf16_t>(p, s) : launch_gate_few_hd<f16_t>(p, s);
   else if (big)
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_stream_hd<bf16_t>(p, ggrid, s) : launch_gate_stream_hd<f16_t>(p, ggrid, s);
   else
     rc = (a->dtype == FMOBA_DTYPE_BF16) ? launch_gate_hd<bf16_t>(p, ggrid, s) : launch_gate_hd<f16_t>(p, ggrid, s);
   if (rc) return rc;
-  FMOBA_LAUNCH_CHECK("topk_gate_kernel");
+  FMOBA_LAUNCH_CHECK(attn != nullptr ? "attn_fwd_rows_kernel (gated)" : "topk_gate_kernel");
   if (!lists) return 0;
   const int64_t list_groups = (int64_t)p.nseg * (p.W + (ranks ? 1 : 0)) * a->heads * a->batch;
   if ((int64_t)p.nseg * max_cols <= kListCounts && p.W <= kListWords && p.seg_rows == kListSegRows && list_groups <= (ranks ? kListRankedGroups : kListGroups)) {
     hipLaunchKernelGGL(ranks ? csc_lists_kernel<true> : csc_lists_kernel<false>, dim3(p.nseg * p.W + (ranks ? p.nseg : 0), a->heads, a->batch), dim3(256), 0, s, p);
+    FMOBA_LAUNCH_CHECK("csc_lists_kernel");
   } else {
     if (ranks)
       hipLaunchKernelGGL(csc_scan_kernel<true>, dim3(a->heads, a->batch, 1 + ceil_div(a->max_seqlen_q, kRankRows)), dim3(256), 0, s, p);
@@ -1309,8 +1309,8 @@ static int fused_topk_run(const fmoba_fused_topk_args *a, void *workspace, size_
       hipLaunchKernelGGL(csc_scan_kernel<false>, dim3(a->heads, a->batch), dim3(256), 0, s, p);
     FMOBA_LAUNCH_CHECK("csc_scan_kernel");
     hipLaunchKernelGGL(ranks ? csc_fill_kernel<true> : csc_fill_kernel<false>, dim3(p.nseg * p.W, a->heads, a->batch), dim3(64), 0, s, p);
+    FMOBA_LAUNCH_CHECK("csc_fill_kernel");
   }
-  FMOBA_LAUNCH_CHECK("csc_fill_kernel");
   if (a->raw_indices) {
     const size_t smem = (size_t)(max_cols + 64) * 4;
     dim3 rgrid(a->total_q, a->heads);
