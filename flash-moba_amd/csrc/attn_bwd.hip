@@ -553,7 +553,7 @@ __global__ __launch_bounds__(256, HD <= 64 && !DQP ? 3 : 2) void attn_bwd_dkdv_k
 // LISTED: the block is looked up (listed_item).  An instance of its own, for ranked lists with NEAR: with the look-up as a branch beside the other decoding every launch was
 // slower (256 and 237 registers either way; 32768 tokens, 32 heads: 3.77 ms against 3.54).
 template <typename T, int HD, int KB, bool NEAR, bool RANKED, bool LISTED>
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder) {
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
   typedef BwdSmem<HD> SM;
   constexpr int KS = HD / 16, LDQ = SM::LDQ, LDS_ = SM::LDS_, NDT = HD / 32, VPR = HD / 8, LDR = SM::LDR;
   constexpr int NKEY = 64 * KB;         // keys of the workgroup
@@ -576,13 +576,12 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
     if (item.b < 0) return;
     nb = item.idx, b = item.b, h = item.h;
   } else {
-    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes,
-                                        longest_items_first(max(a.total_q, a.total_k), a.heads, HD * 4));
+    const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, (a.max_seqlen_k + NKEY - 1) / NKEY, (int64_t)a.max_seqlen_q * HD * 4 >= kOnePairBytes, order == kLongestFirst);
     nb = item.idx, b = item.pair / a.heads, h = item.pair - b * a.heads;
   }
   const int key0 = nb * NKEY;
   // One workgroup per compute unit: nothing covers the dependent loads before the first round, so their chain is kept
-  // short.  Where the block's column list lies depends on nothing that is loaded: asked for together with the
+  // short.  Where the block's column list lies depends on nothing that is loaded (but for a block that is looked up): asked for together with the
   // sequence bounds.
   const int Bn = a.lg_block_n;
   const int c = key0 / Bn;
