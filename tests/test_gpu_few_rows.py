@@ -89,16 +89,31 @@ def test_gate_with_infinite_scores_and_without_numbers(lens_k, chunk, topk, caus
             row += 1
 
 
+def _fwd_args(lens_q, lens_k, H, Hk, D, chunk, topk, causal=True):
+    """The sizes of a call of flash_moba_varlen_func."""
+    f = hip.AttnFwdArgs()
+    f.batch, f.total_q, f.total_k, f.heads, f.heads_k, f.head_dim = len(lens_q), sum(lens_q), sum(lens_k), H, Hk, D
+    f.max_seqlen_q, f.max_seqlen_k, f.max_cols, f.lg_block_m, f.lg_block_n = max(lens_q), max(lens_k), -(-max(lens_k) // chunk), 128, chunk
+    f.is_causal, f.max_visits_per_row = int(causal and max(lens_q) != 1), topk * (chunk // hip.fwd_key_block(chunk))
+    f.q_row_stride = f.o_row_stride = H * D
+    f.k_row_stride = f.v_row_stride = Hk * D
+    f.q_head_stride = f.k_head_stride = f.v_head_stride = f.o_head_stride = D
+    return f
+
+
 # Scores from the pooling pass and the choice in front of the attention, against the gate and the attention over its selection bits.  Chunks at and past
 # a lane's registers (256, 1024), products full of rows (4 heads x 8 rows), ties, keys that are infinite or not a number, more key heads than a block has.
 @pytest.mark.parametrize("lens_q,lens_k,chunk,topk", [
-    ([1], [5], 64, 3), ([1, 1, 0, 1], [64 * 65, 64, 100, 129], 64, 1), ([8, 3], [64 * 65 + 1, 700], 64, 7), ([1, 2], [64 * 257, 64 * 256], 64, 33),
-    ([1, 1], [64 * 1024, 64 * 1025 + 9], 64, 64), ([2], [1], 128, 5), ([4, 1], [128 * 300, 128 * 7], 128, 16)])
+    ([1], [5], 64, 3), ([1, 1, 0, 1], [64 * 65, 64, 100, 129], 64, 1), ([8, 3], [64 * 65 + 1, 700], 64, 7), ([8, 3], [64 * 65 + 1, 900], 64, 7),
+    ([1, 2], [64 * 257, 64 * 256], 64, 33), ([1, 1], [64 * 1024, 64 * 1025 + 9], 64, 64), ([2], [1], 128, 5), ([4, 1], [128 * 300, 128 * 7], 128, 16)])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("kind", ["normal", "ties", "special"])
 @pytest.mark.parametrize("H,Hk,D,dtype", [(8, 2, 128, torch.bfloat16), (10, 10, 64, torch.float16), (12, 3, 256, torch.bfloat16), (12, 6, 96, torch.float16),
                                           (6, 6, 40, torch.bfloat16)])
 def test_scores_from_the_pooling_pass(monkeypatch, lens_q, lens_k, chunk, topk, causal, kind, H, Hk, D, dtype):
+    # (calls whose rows share too much to be read one by one keep the launch of the gate)
+    scored = hip.load_library().fmoba_attn_fwd_gated_few_bytes(_fwd_args(lens_q, lens_k, H, Hk, D, chunk, topk, causal)) > 0
+    assert scored == (H == Hk or (H, Hk) == (12, 6) or lens_k not in ([64 * 65 + 1, 700], [1]))
     q, k, v, cuq, cuk = (t.cuda() for t in _case(lens_q, lens_k, H, Hk, D, dtype, D + topk, kind == "ties"))
     if kind == "special":
         g = torch.Generator(device="cuda").manual_seed(topk)
@@ -115,18 +130,6 @@ def test_which_calls_the_pooling_pass_scores(heads, heads_k, dim, rows, takes):
     f.batch, f.total_q, f.total_k, f.heads, f.heads_k, f.head_dim = 4, 4 * rows, 4 << 16, heads, heads_k, dim
     f.max_seqlen_q, f.max_seqlen_k, f.max_cols, f.lg_block_n, f.is_causal, f.max_visits_per_row = rows, 1 << 16, 512, 128, 1, 8
     assert (hip.load_library().fmoba_attn_fwd_gated_few_bytes(f) > 0) == takes
-
-
-def _fwd_args(lens_q, lens_k, H, Hk, D, chunk, topk, causal=True):
-    """The sizes of a call of flash_moba_varlen_func."""
-    f = hip.AttnFwdArgs()
-    f.batch, f.total_q, f.total_k, f.heads, f.heads_k, f.head_dim = len(lens_q), sum(lens_q), sum(lens_k), H, Hk, D
-    f.max_seqlen_q, f.max_seqlen_k, f.max_cols, f.lg_block_m, f.lg_block_n = max(lens_q), max(lens_k), -(-max(lens_k) // chunk), 128, chunk
-    f.is_causal, f.max_visits_per_row = int(causal and max(lens_q) != 1), topk * (chunk // hip.fwd_key_block(chunk))
-    f.q_row_stride = f.o_row_stride = H * D
-    f.k_row_stride = f.v_row_stride = Hk * D
-    f.q_head_stride = f.k_head_stride = f.v_head_stride = f.o_head_stride = D
-    return f
 
 
 def test_the_entry_point_needs_no_place_for_chunk_means(monkeypatch):

@@ -5,6 +5,7 @@ import torch
 
 import flash_moba
 from flash_moba import flash_moba_hip as hip
+from test_gpu_few_rows import _fwd_args
 from test_gpu_host_path import _both
 
 pytestmark = pytest.mark.gpu
@@ -21,6 +22,13 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["normal", "ties", "special"])
 @pytest.mark.parametrize("grad", [True, False])
 def test_rows_that_choose_their_chunks(monkeypatch, lens_q, lens_k, H, Hk, D, chunk, topk, causal, kind, grad):
+    # (without a causal limit 4 of 16 chunks are few: by columns)
+    f, b = _fwd_args(lens_q, lens_k, H, Hk, D, chunk, topk, causal), hip.AttnBwdArgs()
+    for name in ("batch", "total_q", "total_k", "heads", "heads_k", "head_dim", "max_seqlen_q", "max_seqlen_k", "max_cols", "lg_block_n", "is_causal"):
+        setattr(b, name, getattr(f, name))
+    b.max_visits_per_row = topk * (chunk // 64)
+    assert hip.load_library().fmoba_attn_fwd_gates_rows(f) == (causal or lens_q != [1024, 2048])
+    assert not hip.load_library().fmoba_attn_bwd_uses_partials(b)  # (whose lists are ranked by a gate of its own)
     g = torch.Generator(device="cuda").manual_seed(sum(lens_q) + D)
     dtype = torch.float16 if H == 4 else torch.bfloat16
     draw = (lambda s: torch.randint(-2, 3, s, generator=g, device="cuda").float()) if kind == "ties" else (lambda s: torch.randn(s, generator=g, device="cuda"))

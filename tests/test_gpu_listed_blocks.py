@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import flash_moba
+from flash_moba import flash_moba_hip as hip
 from gpu_utils import assert_close
 from test_gpu_item_order import _reference
 
@@ -18,11 +19,18 @@ pytestmark = pytest.mark.gpu
     ([100, 2600, 127, 300], 8, 8, 128, 128, 2, 0), ([1500, 256, 20, 257, 90], 16, 8, 256, 64, 8, 0), ([40, 2100, 200], 8, 8, 200, 64, 2, 0), ([500, 20, 30], 24, 8, 128, 64, 3, 5000),
     ([8200, 33, 40], 8, 1, 64, 64, 2, 0), ([60, 3000, 40, 20, 130], 8, 8, 128, 64, 2, 0), ([6500, 127, 40, 20], 16, 4, 128, 128, 2, 0)])
 def test_every_block_once(lens, H, Hk, D, chunk, topk, bound):
+    _every_block_once(lens, H, Hk, D, chunk, topk, bound, torch.bfloat16)
+
+
+def _every_block_once(lens, H, Hk, D, chunk, topk, bound, dtype):
+    """Result and gradients against the pattern's in fp32; returns whether the backward left dQ in partials."""
     g = torch.Generator(device="cuda").manual_seed(sum(lens) + D)
-    mk = lambda h: torch.randn((sum(lens), h, D), generator=g, device="cuda").to(torch.bfloat16)
+    mk = lambda h: torch.randn((sum(lens), h, D), generator=g, device="cuda").to(dtype)
     q, k, v, dout = (x.requires_grad_(True) for x in (mk(H), mk(Hk), mk(Hk), mk(H)))
     cu = [0] + [int(x) for x in np.cumsum(lens)]
     cud, longest = torch.tensor(cu, dtype=torch.int32, device="cuda"), max(*lens, bound)
+    form = []
+    q.register_hook(lambda _: form.append(hip.last_bwd_partials()))  # (on the engine's thread, as the backward)
     out = flash_moba.flash_moba_varlen_func(q, k, v, cud, cud, longest, longest, chunk, topk, causal=True)
     got = (out.detach(), *torch.autograd.grad(out, (q, k, v), dout.detach()))
     pattern = flash_moba.flash_topk_varlen_func(q.detach(), k.detach(), cud, cud, longest, longest, topk, chunk, causal=True)
@@ -32,6 +40,17 @@ def test_every_block_once(lens, H, Hk, D, chunk, topk, bound):
         assert_close(name, x, y, 2e-2 * n, 1e-2)
     again = flash_moba.flash_moba_varlen_func(q.detach(), k.detach(), v.detach(), cud, cud, longest, longest, chunk, topk, causal=True)
     assert torch.equal(again, got[0])
+    return form[0]
+
+
+# dK/dV with partials, whose blocks are looked up where a plain grid has three times as many as there may be: blocks of 64 keys and of 128, empty sequences, a bound longer than every sequence
+@pytest.mark.parametrize("lens,H,Hk,chunk,topk,bound", [
+    ([5200, 100, 20, 40], 8, 8, 64, 1, 0), ([20, 0, 11000, 65], 8, 2, 64, 2, 0), ([6500, 127, 40, 20], 16, 4, 128, 2, 0), ([129, 7000, 0, 128], 8, 8, 128, 2, 9000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_block_of_a_backward_with_partials_once(lens, H, Hk, chunk, topk, bound, dtype):
+    keys = hip.fwd_key_block(chunk)  # (of a block of this pass too)
+    assert len(lens) * -(-max(*lens, bound) // keys) >= 3 * (sum(lens) // keys + len(lens))
+    assert _every_block_once(lens, H, Hk, 128, chunk, topk, bound, dtype) == 1
 
 
 # later parts of prompts, by columns: keys and queries of other lengths, blocks by pairs (many keys) and by length
