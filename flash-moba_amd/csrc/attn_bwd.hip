@@ -140,8 +140,8 @@ struct DkdvSmem {
 
 // RANKED (partials form): part rows go to the place of the block among the row's, which the rank of the list entry gives
 // NEAR: a gathered row's place is a 32-bit byte offset from the sequence's first row that one 24-bit multiply makes (rows_near).
-// Three waves per SIMD for the dS form of heads up to 64, whose LDS takes three workgroups to a unit: the compiler's own choice for rows far apart was 182 registers (166 now) and two waves,
-// backward of 8191 tokens, 16 heads 248 us against 236, of 16384, 32 heads 1264 against 1223.
+// Three waves per SIMD for the dS form of heads up to 64, whose LDS takes three workgroups to a unit: the compiler's own choice for rows far apart was 182
+// registers (166 now) and two waves, backward of 8191 tokens, 16 heads 248 us against 236, of 16384, 32 heads 1264 against 1223.
 template <typename T, int HD, bool DQP, bool RANKED, bool NEAR>
 __global__ __launch_bounds__(256, HD <= 64 && !DQP ? 3 : 2) void attn_bwd_dkdv_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
   typedef DkdvSmem<HD, DQP> SM;
@@ -550,8 +550,8 @@ __global__ __launch_bounds__(256, HD <= 64 && !DQP ? 3 : 2) void attn_bwd_dkdv_k
 // leaves one dQ partial instead of two.
 // NEAR: the host has checked that a gathered row's place in q and dout is a 32-bit byte offset from the sequence's first
 // row that one 24-bit multiply makes (launch_dkdv); otherwise the loads take 64-bit addresses per lane.
-// LISTED: the block is looked up (listed_item).  An instance of its own, for ranked lists with NEAR: with the look-up as a branch beside the other decoding every launch was
-// slower (256 and 237 registers either way; 32768 tokens, 32 heads: 3.77 ms against 3.54).
+// LISTED: the block is looked up (listed_item).  An instance of its own, for ranked lists with NEAR: with the look-up as a branch beside the other decoding
+// every launch was slower (256 and 237 registers either way; 32768 tokens, 32 heads: 3.77 ms against 3.54).
 template <typename T, int HD, int KB, bool NEAR, bool RANKED, bool LISTED>
 __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_bwd_args a, BwdWs ws, ItemOrder order) {
   typedef BwdSmem<HD> SM;
@@ -1237,8 +1237,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_partials_kernel(fmoba_attn_
 // waves of two tiles per unit (groups of four steps, 512 rows) read half of the K tiles
 // but met at one barrier and left no unit a second walk: 65536 tokens in eight sequences, top-k 32 of 64-key chunks
 // 1634 -> 1556 us, 24571 tokens, 32 over 8 heads 691 -> 624, 12037 tokens, heads of 96 182 -> 124 (with the order of the items
-// below; tiles of 96 features instead of 128: 129 -> 115), 2 x 4096 tokens 143 -> 125.  Up to 64: eight waves of one tile (with two tiles in four waves 4096 tokens 58 -> 67 us).
-// Above 128: eight waves of one tile, one workgroup per unit (its K tiles take 128 KB).
+// below; tiles of 96 features instead of 128: 129 -> 115), 2 x 4096 tokens 143 -> 125.  Up to 64: eight waves of one tile (with two tiles in four waves 4096
+// tokens 58 -> 67 us). Above 128: eight waves of one tile, one workgroup per unit (its K tiles take 128 KB).
 // ------------------------------------------------------------------------------------
 constexpr int kDqColBatch = 256;
 constexpr int kDqMaxSteps = 512;
@@ -1829,8 +1829,9 @@ template <typename T, int HD, int KB>
 static int launch_dkdv_partials(const fmoba_attn_bwd_args &a, const BwdWs &ws, hipStream_t s) {
   const bool near_rows = rows_near(a);
   const bool longest_first = longest_items_first(std::max(a.total_q, a.total_k), a.heads, HD * 4);
-  // Workgroups of one to a unit, whose empty ones come last: looking blocks up pays where two thirds of them are empty (30000 tokens in twelve sequences, 8 heads, 4.5 times as many as there
-  // are blocks: step 440 -> 427 us; 1.5 to 2.2 times as many: 12846, 5768, 4917 and 6469 tokens 783 -> 790, 15400 in eight 344.7 -> 347.2, 15004 in five and 8999 in eight, 16 heads, the same).
+  // Workgroups of one to a unit, whose empty ones come last: looking blocks up pays where two thirds of them are empty (30000 tokens in twelve sequences, 8
+  // heads, 4.5 times as many as there are blocks: step 440 -> 427 us; 1.5 to 2.2 times as many: 12846, 5768, 4917 and 6469 tokens 783 -> 790, 15400 in eight
+  // 344.7 -> 347.2, 15004 in five and 8999 in eight, 16 heads, the same).
   const bool listed = near_rows && ws.visits != nullptr && lists_blocks(a.total_k, a.max_seqlen_k, a.batch, a.heads, 64 * KB, longest_first) &&
                       (int64_t)a.batch * ceil_div(a.max_seqlen_k, 64 * KB) >= 3 * listed_blocks(a.total_k, a.batch, 64 * KB);
   auto kern = listed                  ? attn_bwd_dkdv_partials_kernel<T, HD, KB, true, true, true>

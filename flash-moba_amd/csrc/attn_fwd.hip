@@ -75,8 +75,9 @@ struct FwdColSmem {
   static_assert(bytes * (8 / NW) <= 160 * 1024, "eight waves per compute unit");
 };
 
-// The blocks that exist alone, by length or by pairs (one pair at a time is for sequences far beyond these).  Pair by pair only where they are at most half: the look-up is one more load in front
-// of the lists' bounds (parts of prompts against 9216, 33000 and 20000 keys, 0.63 of the blocks 241.5 -> 243.3 us; six of 300 rows against 3000 to 60000, 0.4 202.9 -> 195.2).
+// The blocks that exist alone, by length or by pairs (one pair at a time is for sequences far beyond these).  Pair by pair only where they are at most half:
+// the look-up is one more load in front of the lists' bounds (parts of prompts against 9216, 33000 and 20000 keys, 0.63 of the blocks 241.5 -> 243.3 us; six of
+// 300 rows against 3000 to 60000, 0.4 202.9 -> 195.2).
 static ItemOrder col_order(const fmoba_attn_fwd_args &a, int ngrp, int hd, int kb) {
   const bool longest_first = longest_items_first(std::max(a.total_q, a.total_k), a.heads, hd * 2);
   const bool listed = lists_blocks(a.total_k, a.max_seqlen_k, a.batch, ngrp, kb, true) && (int64_t)a.max_seqlen_q * hd * 4 < kOnePairBytes;

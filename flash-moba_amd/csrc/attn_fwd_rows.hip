@@ -457,9 +457,10 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // top-k 8 of 128-key chunks 496 -> 484, 12037 tokens, 16 heads of 96 484 -> 481, 8191 tokens of short documents the same.
 // GATED: the rows choose their chunks here (up to kRowGateChunks of them), while Q is in registers anyway, and the words of the selection go to memory only if
 // column lists follow (with the counts these need).  The search for a row's cut is vector arithmetic of one wave beside the products of another workgroup's, where a gate
-// launch in front leaves the matrix cores idle, reads Q once more and is a launch.  Whole calls: forward of 1024 + 2048 tokens, 8 heads of 64 33.5 -> 30.1 us, 1024 tokens 23.8 -> 20.6, 2048
-// tokens, 16 heads of 128 53.2 -> 50.3, parts of prompts of 512 and 1000 rows against 4000 and 7000 keys, 32 over 8 heads 172 -> 166; training step of 8191 tokens of short documents 122.2 ->
-// 116.4, 5000 tokens, 8 heads of 112 216 -> 211, 8 x 4096 tokens, 32 over 8 heads, forward 1262 -> 1234; nothing from 24571 tokens of training on.
+// launch in front leaves the matrix cores idle, reads Q once more and is a launch.  Whole calls: forward of 1024 + 2048 tokens, 8 heads of 64 33.5 -> 30.1 us,
+// 1024 tokens 23.8 -> 20.6, 2048 tokens, 16 heads of 128 53.2 -> 50.3, parts of prompts of 512 and 1000 rows against 4000 and 7000 keys, 32 over 8 heads 172 ->
+// 166; training step of 8191 tokens of short documents 122.2 -> 116.4, 5000 tokens, 8 heads of 112 216 -> 211, 8 x 4096 tokens, 32 over 8 heads, forward 1262
+// -> 1234; nothing from 24571 tokens of training on.  (One to six scalars of these instances are spilled, none without the choice.)
 // RW: waves of a set, which share its tiles.  SPLIT = 2 (4): two (four) sets of waves take turns at the steps of the same rows, with
 // rings of their own; the results of a row meet in LDS at the end.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
@@ -925,8 +926,9 @@ size_t fwd_rows_workspace_bytes(const fmoba_attn_fwd_args &a) {
   return ((rows * (size_t)ceil_div(a.max_cols, 32) * 4 + 255) & ~(size_t)255) + 256;
 }
 
-// Calls whose rows can choose their chunks in attn_fwd_rows_kernel: the scores of a row are two tiles of products with the operands that Q already is (tiles of 96
-// features have them in another order), calls of a few rows have a gate of their own.
+// Calls whose rows can choose their chunks in attn_fwd_rows_kernel: the scores of a row are two tiles of products with the operands that Q already is; calls of
+// a few rows have a gate of their own.  Heads of 72 to 96 keep the launch of the gate: in their tiles the operands' pieces lie in another order
+// (tile_frag_piece<96>), which gate_select has no instance for.
 bool fwd_rows_gated(const fmoba_attn_fwd_args &a) {
   return a.max_cols <= kRowGateChunks && a.max_seqlen_q > kFewRows && !fwd_few_rows(a) && fwd_rows_direct(a) &&
          (a.head_dim <= 64 || a.head_dim > 96);

@@ -20,8 +20,9 @@ namespace fmoba {
 // 128-key chunks bf16 2.010e-3 and 2.047e-3, fp16 2.507e-4 and 2.554e-4; rows that see 64 steps 2.105e-3 and 2.106e-3, 2.632e-4 and 2.632e-4, 512 steps
 // 2.108e-3 and 2.166e-3, 2.623e-4 and 2.694e-4, 2048 steps 2.094e-3 and 2.157e-3, 2.629e-4 and 2.699e-4.
 // What bounds it: matrix products at the power limit (1.0 PFLOP/s executed at 16384 tokens; without the tile loads it would be 15 % faster, without
-// the rescaling or the exponentials 3 to 5 %).  GATED as in attn_fwd_rows_kernel: forward of 2 x 4096 tokens, 8 heads, top-k 8 of 128-key chunks 178.7 -> 173.2 us, of 2048 tokens, 16 heads
-// 85.9 -> 80.4, 9000 tokens, 16 over 2 heads 343.6 -> 336.0.  The same call: columns 134 us and their combine 89 -> 171 us, training step 612 -> 530.
+// the rescaling or the exponentials 3 to 5 %).  GATED as in attn_fwd_rows_kernel: forward of 2 x 4096 tokens, 8 heads, top-k 8 of 128-key chunks 178.7 -> 173.2
+// us, of 2048 tokens, 16 heads 85.9 -> 80.4, 9000 tokens, 16 over 2 heads 343.6 -> 336.0.  The same call: columns 134 us and their combine 89 -> 171 us,
+// training step 612 -> 530.
 template <typename T, bool GATED>
 __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, ItemOrder order, RowGate gate) {
   constexpr int HD = 256, RW = 4;

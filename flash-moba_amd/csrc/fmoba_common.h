@@ -575,12 +575,14 @@ __device__ __forceinline__ PairItem xcd_pair_item(int id, int npairs, int nper, 
   return w;
 }
 
-// Uneven batches: the blocks that exist alone, of all sequences and heads, from the longest walks to the shortest.  A grid for the longest sequence's blocks in every sequence is mostly
-// workgroups that find no block, each of which takes its place (and its LDS) for as long as its first loads take; here every workgroup looks its block up, some ten
-// instructions per sequence.  Whole calls: training steps of 3000 tokens in ten sequences, 16 over 4 heads of 256 (whose workgroups have a unit each) 192 -> 167 us, of 9000 in six, 8 heads
-// of 256 383 -> 362, of 4000 in eight, 32 heads of 80 185.4 -> 173.1, 16000 in sixteen, 16 heads of 64 326.3 -> 318.4, 30000 in thirty, 8 heads of 128 484.8 -> 479.9, 2000 in four, 8 heads of
-// 64 89.5 -> 88.1; forward of 30000 in eight, 16 heads of 128, by columns 434 -> 423.6; 13400 in eight, 8 heads of 128 354 -> 337; 8191 tokens in 24 documents the same (the look-up goes through all of them).
-// For calls whose items go longest first and whose heads are whole turns of the XCDs (a head's blocks then run on one), where it leaves out a fifth of the items or more.
+// Uneven batches: the blocks that exist alone, of all sequences and heads, from the longest walks to the shortest.  A grid for the longest sequence's blocks in
+// every sequence is mostly workgroups that find no block, each of which takes its place (and its LDS) for as long as its first loads take; here every workgroup
+// looks its block up, some ten instructions per sequence.  Whole calls: training steps of 3000 tokens in ten sequences, 16 over 4 heads of 256 (whose
+// workgroups have a unit each) 192 -> 167 us, of 9000 in six, 8 heads of 256 383 -> 362, of 4000 in eight, 32 heads of 80 185.4 -> 173.1, 16000 in sixteen, 16
+// heads of 64 326.3 -> 318.4, 30000 in thirty, 8 heads of 128 484.8 -> 479.9, 2000 in four, 8 heads of 64 89.5 -> 88.1; forward of 30000 in eight, 16 heads of
+// 128, by columns 434 -> 423.6; 13400 in eight, 8 heads of 128 354 -> 337; 8191 tokens in 24 documents the same (the look-up goes through all of them). For
+// calls whose items go longest first and whose heads are whole turns of the XCDs (a head's blocks then run on one), where it leaves out a fifth of the items or
+// more.
 constexpr int kListedBatch = 32;
 __host__ __device__ __forceinline__ int64_t listed_blocks(int64_t total, int batch, int block) { return total / block + batch; }  // at least as many as there are
 __host__ __device__ __forceinline__ bool lists_blocks(int64_t total, int longest, int batch, int heads, int block, bool longest_first) {
@@ -596,8 +598,8 @@ struct BlockItem {
   int b, h, idx;       // b < 0: none
   int q0, Lq, k0, Lk;  // the sequence's bounds
 };
-// item `id` of listed_blocks * heads: block idx of head h of sequence b.  Blocks of query rows come from the last ones (whose walks are the longest) to the first, blocks of keys (rows =
-// false; the first are seen by most rows) from the first to the last.
+// item `id` of listed_blocks * heads: block idx of head h of sequence b.  Blocks of query rows come from the last ones (whose walks are the longest) to the
+// first, blocks of keys (rows = false; the first are seen by most rows) from the first to the last.
 template <int BLOCK, bool ROWS>
 __device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, int longest, const int32_t *cu_q, const int32_t *cu_k) {
   const int lane = threadIdx.x & 63, nper = (longest + BLOCK - 1) / BLOCK;
@@ -629,8 +631,8 @@ __device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, i
   BlockItem w{-1, h, base + l, 0, 0, 0, 0};
   if (l < 0 || l > 63) return w;
   const unsigned long long have = __ballot(nb > w.idx);
-  // Which of the sequences that have such a block: rotated by one from number to number, as in xcd_pair_item and for the same reason (30000 tokens in four sequences, 8 heads, dK/dV with partials:
-  // training step 804 us, 865 without).
+  // Which of the sequences that have such a block: rotated by one from number to number, as in xcd_pair_item and for the same reason (30000 tokens in four
+  // sequences, 8 heads, dK/dV with partials: training step 804 us, 865 without).
   const int some = (int)__popcll(have), k = (n - (__builtin_amdgcn_readlane(at, l) - some) + w.idx) % max(some, 1);
   const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0u));
   const unsigned long long it = __ballot(nb > w.idx && rank == k);
@@ -709,7 +711,8 @@ __device__ __forceinline__ Pack8 zero_pack8() {
 // (64 lanes x 16 bytes: 4.2 clocks, one two-way meeting: 8).  Rows of 128 bytes lie two to a sweep of the banks, so eight pieces have to tell
 // the rows of a parity among sixteen apart (bits 1 to 3), and bit 1, which parts rows of a parity inside a transposing read's four, moves the
 // upper half of the pieces.  Told apart by bits 1 and 2 alone: row reads 8 clocks, the P and dS tiles of the dK/dV pass (piece ^ row % 8)
-// 8 and 4 instead of 4.2 and 2; 8191 tokens of short documents, heads of 64, training step 137.5 -> 136.4 us, 2 x 4096 tokens 475.9 -> 471.7.
+// 8 and 4 instead of 4.2 and 2 (27 % of its LDS cycles were conflicts, 14 % are); training steps of 8191 tokens of short documents, heads of 64 135.7 -> 135.0 us, of
+// 2 x 4096 tokens 459.7 -> 456.9, of 65536 tokens 7139 -> 7095.  It takes two addresses per transposed piece where a constant did for the second one.
 template <int HD>
 __device__ __forceinline__ int tile_swz(int r) {
   if constexpr (HD == 96)
@@ -976,7 +979,8 @@ struct RowGate {
   int32_t W, nseg, seg_rows;
 };
 constexpr int kRowGateChunks = 64;  // chunks per sequence that it takes, at most
-// Query rows and chunks per sequence of a call of a few rows, at most: for its gate, its attention and the two as one (topk_csc.hip, attn_fwd_few.hip), which the row-block form leaves them to.
+// Query rows and chunks per sequence of a call of a few rows, at most: for its gate, its attention and the two as one (topk_csc.hip, attn_fwd_few.hip), which
+// the row-block form leaves them to.
 constexpr int kFewRows = 8, kFewChunks = 4096;
 
 }  // namespace fmoba

@@ -281,8 +281,9 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
       constexpr int IB = (NT * 32 <= 64) ? 6 : (NT * 32 <= 128 ? 7 : 8);
       for (int bit = IB - 1; bit >= 0; --bit) {
         const uint32_t trial = i_acc | (1u << bit);
-        // (Made anew in every turn: the flags of 128 and 256 scores, the same in all of them, were kept in scalar registers beside the loop, which took them from the whole kernel: 79 and
-        // 223 scalars spilled, in a path that next to no row takes.  Gate of 32384 tokens, 16 heads, 256 chunks 138 -> 124 us for heads of 64 and 152 -> 138 of 128, 128 chunks 80 -> 75.5.)
+        // (Made anew in every turn: the flags of 128 and 256 scores, the same in all of them, were kept in scalar registers beside the loop, which took them
+        // from the whole kernel: 79 and 223 scalars spilled, in a path that next to no row takes.  Gate of 32384 tokens, 16 heads, 256 chunks 138 -> 124 us for
+        // heads of 64 and 152 -> 138 of 128, 128 chunks 80 -> 75.5.)
         float eq = tau_eq;
 #if defined(__HIP_DEVICE_COMPILE__)
         if constexpr (NT > 2) asm volatile("" : "+v"(eq));
@@ -335,9 +336,9 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
   }
 }
 
-// The gate of a row block, by the workgroup that is about to walk its keys (SPLIT sets of RW waves of 32 rows each; the first set chooses): candidates of some row of the block, their
-// means into LDS, scores, choice, as topk_gate_kernel does it.  Q is asked for and not awaited when it begins, arranged when it ends.  The rows' words go to sBits (word w of row r at w *
-// 32 RW + r), and if column lists follow to memory with their counts.  Takes row_gate_lds bytes of `smem`.
+// The gate of a row block, by the workgroup that is about to walk its keys (SPLIT sets of RW waves of 32 rows each; the first set chooses): candidates of some
+// row of the block, their means into LDS, scores, choice, as topk_gate_kernel does it.  Q is asked for and not awaited when it begins, arranged when it ends.
+// The rows' words go to sBits (word w of row r at w * 32 RW + r), and if column lists follow to memory with their counts.  Takes row_gate_lds bytes of `smem`.
 template <int HD>
 constexpr size_t row_gate_lds() { return (size_t)kRowGateChunks * HD * 2 + kRowGateChunks * 4; }
 template <typename T, int HD, int RW, int SPLIT>

@@ -21,7 +21,9 @@ struct PoolExtra {
 // them while it has them.  Each wave takes key heads of the block; the query rows of a group's heads are the columns of one product (the one
 // of topk_gate_few_kernel: the same scores to the last bit).  What it costs hides under the other blocks' loads, the gate is no launch any more, and the
 // chunk of a lone row's own keys is not read.  Decode of 16 requests against 512 to 32768 keys, 32 over 8 heads of 128, top-k 8 of 128-key chunks 119 -> 106 us;
-// one request of 3000 keys 21.3 -> 16.6, of 60000 48.5 -> 36.5; 20 of 256 to 65536, 32 over 32 heads 740 -> 694.
+// one request of 3000 keys 21.3 -> 16.6, of 60000 48.5 -> 36.5; 20 of 256 to 65536, 32 over 32 heads 740 -> 694.  Heads of 256 too, though the query rows leave
+// three waves per SIMD of eight: one request of 60000 keys, 8 heads 81.9 -> 62.4, eight of 1000 to 30000, 32 over 4 heads 61.4 -> 56.2, 32 of 512 to 32768, 32
+// heads 907 -> 878.
 template <typename T, bool MANY, int HD>
 __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x, FewGate few) {
   const int c = blockIdx.x, b = blockIdx.y;

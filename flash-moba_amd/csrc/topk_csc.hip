@@ -170,8 +170,8 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
 // 262144 tokens, 16 heads, top-k 16 of 128-key chunks 3859 -> 2921 us; 1024-row parts of prompts with 9000 to 33000 keys, 32
 // heads, top-k 8 51 -> 29 us (before: winners shared out by lane, lists of entrants, the whole cut of the first group searched).  Bound by
 // the vector instructions (87 % of the clocks at 262144 tokens), most of them the pass of a new winner.  Above 16 winners: 126187 tokens, 16 heads, top-k
-// 28 of 64-key chunks, gating and lists 9514 -> 2340 us, 54437 tokens, 32 heads, top-k 27 2603 -> 1007, 40000 tokens, 16 heads, top-k 50 1748 -> 846 (before: winners in two lists in LDS, an entrant looked for the weakest
-// of all, one workgroup per compute unit).
+// 28 of 64-key chunks, gating and lists 9514 -> 2340 us, 54437 tokens, 32 heads, top-k 27 2603 -> 1007, 40000 tokens, 16 heads, top-k 50 1748 -> 846 (before:
+// winners in two lists in LDS, an entrant looked for the weakest of all, one workgroup per compute unit).
 // ------------------------------------------------------------------------------------
 // A winner is ONE double between 1 and 2: order key of its score and chunk are 48 bits of its fraction, so that the order "score
 // descending, chunk descending" is the order of the doubles and minimum / maximum are single instructions.
@@ -680,8 +680,8 @@ __global__ __launch_bounds__(512) void topk_gate_few_kernel(TopkParams p) {
 }
 
 // How many chunks a row selected below each word of its selection (PREFIX), and its visits, for rows first, first + step, .. of `rows` rows of sequence b from `row0` on;
-// with them, shared out among `nblk` blocks, the rows before the first sequence and after the last one (a buffer longer than its batch), which have no visits: the combine
-// kernels look at every row.
+// with them, shared out among `nblk` blocks, the rows before the first sequence and after the last one (a buffer longer than its batch), which have no visits:
+// the combine kernels look at every row.
 template <bool PREFIX>
 __device__ __forceinline__ void rank_rows(const TopkParams &p, int h, int b, int blk, int nblk, int row0, int rows) {
   const fmoba_fused_topk_args &a = p.a;
@@ -906,12 +906,13 @@ __global__ __launch_bounds__(64) void csc_fill_kernel(TopkParams p) {
 // each wave a quarter, all loads in flight at once), a segment's rows are asked for together with them, and with ranks the chunks of a row below the word column are
 // counted from its words, of which there are few.  grid (nseg * W, + nseg for the visits if ranks are wanted; heads, batch), a wave for each 64 rows of a segment.
 // What bounds it is a chain: launch, counts, 32 ballots and stores.  The scan before it was a launch and a chain of its own whose few workgroups left the chip
-// empty, and one wave per segment walks four times as far: 8192 tokens, 16 heads, ranked lists of 128-key chunks, scan and fill 17.6 us, one wave per segment 15.1, this 10.0 (four waves of
-// eight chunks each, which read the words below four times: 10.9, and 23 where this takes 19); parts of prompts of 1024 rows against 9000 to 33000 keys, 32 heads
-// 22.0 -> 19.4; 8191 tokens of short documents, plain lists 10.7 -> 4.8.  More counts, or longer segments (which calls of many waves have), go to the two launches: there the
-// scan is a small part of the time and the counts of a workgroup would be a large one.  So do calls of many workgroups, each of which counts for itself,
-// earlier where ranks are made beside the lists: ranked, 9856 of them 28.2 us against 21.4 and 5120 of them 22.7 against 18.7, while 3840 win (above); plain, 4800 of them
-// (12037 tokens, 16 heads) 11.8 against 18.0, and 11200 (24571 tokens, 32 heads) as long as the two launches.
+// empty, and one wave per segment walks four times as far: 8192 tokens, 16 heads, ranked lists of 128-key chunks, scan and fill 17.6 us, one wave per segment
+// 15.1, this 10.0 (four waves of eight chunks each, which read the words below four times: 10.9, and 23 where this takes 19); parts of prompts of 1024 rows
+// against 9000 to 33000 keys, 32 heads 22.0 -> 19.4; 8191 tokens of short documents, plain lists 10.7 -> 4.8.  More counts, or longer segments (which calls of
+// many waves have), go to the two launches: there the scan is a small part of the time and the counts of a workgroup would be a large one.  So do calls of many
+// workgroups, each of which counts for itself, earlier where ranks are made beside the lists: ranked, 9856 of them 28.2 us against 21.4 and 5120 of them 22.7
+// against 18.7, while 3840 win (above); plain, 4800 of them (12037 tokens, 16 heads) 11.8 against 18.0, and 11200 (24571 tokens, 32 heads) as long as the two
+// launches.
 constexpr int kListCounts = 4096, kListWords = 16, kListSegRows = 256, kListGroups = 8192, kListRankedGroups = 4096;
 template <bool RANKED>
 __global__ __launch_bounds__(256) void csc_lists_kernel(TopkParams p) {
@@ -1178,8 +1179,9 @@ template <typename T, int HD>
 static int launch_gate_nt(const TopkParams &p, dim3 grid, hipStream_t s) {
   if (p.W <= 2) return launch_gate<T, HD, 2>(p, grid, s);
   if (p.W <= 4) return launch_gate<T, HD, 4>(p, grid, s);
-  // more than 128 chunks and no more than 16 winners: in groups.  (32768 tokens, 32 heads, top-k 16 of 128-key chunks 306 -> 250 us; with up to
-  // 128 chunks all scores in registers are the faster form: 21000 tokens in two sequences, top-k 12 55 against 64 us, 16384 tokens, top-k 8 41 against 43.)
+  // more than 128 chunks and no more than 16 winners: in groups.  (Gating and lists, in groups and with all scores in registers: 32768 tokens, 32 heads, 128-key
+  // chunks, top-k 16 333 and 384 us, top-k 4 246 and 335; 10000 tokens, 16 heads of 64, 157 chunks, top-k 16 55.7 and 59.5.  With up
+  // to 128 chunks registers are the faster form: 21000 tokens in two sequences, top-k 12 55 against 64 us, 16384 tokens, top-k 8 41 against 43.)
   if (gate_winners(p) <= 16) return launch_gate_stream<T, HD>(p, grid, s);
   return launch_gate<T, HD, 8>(p, grid, s);
 }
