@@ -81,10 +81,16 @@ __device__ __forceinline__ uint32_t shift_in_flag(uint32_t w, unsigned long long
 #endif
 }
 
+// Up to this many chunks a row's cut is found by taking its best scores off one by one (two and a half instructions per score and chunk), beyond by bisection
+// (about ten passes of two): both are bound by vector instructions.  Gate of 8192 tokens, 16 heads, up to 64 chunks, bisection and this: top-k 3 16.3 -> 12.2 us, 5 16.3 -> 13.1, 8 16.8 -> 14.5,
+// 11 16.5 -> 15.4, 13 16.8 -> 16.3, 17 15.6 -> 16.1, 25 15.1 -> 18.5; 4096 tokens top-k 3 11.3 -> 8.2, 11 11.9 -> 11.1, 17 11.9 -> 12.5.
+constexpr int kGatePeels = 10;
 // The wave's 32 rows, lane (row l % 32): qf holds the row's slices as the B operand, the chunk means lie in the LDS tile from ldsTile on (rows of HD elements, piece c
 // of row r at c ^ tile_swz<HD>(r)), n_tiles * 32 of them.  The row's candidates are the chunks [0, nc); it keeps the best kp and its own chunk (own; below 0: none).
 // emit(t, w): word t of the row's selection, t < words, the same in both halves of the wave.
-template <typename T, int HD, int NT, typename Emit>
+// PEEL: as the row-block forward does it where several sets of waves wait for the choice (1024 + 2048 tokens, 8 heads of 64, call 30.4 -> 28.6 us), and the gate's own launch; in the workgroups
+// of one set, which overlap each other's choices, the second search of the cut only made the code longer (8191 tokens of short documents 123.6 -> 124.7 us).
+template <typename T, int HD, int NT, bool PEEL, typename Emit>
 __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[HD / 16], int lane, int n_tiles, int nc, int kp, int own, bool valid, int words, const Emit &emit) {
   constexpr int KS = HD / 16, RB = HD * 2;
   const int hh = lane >> 5;
@@ -222,7 +228,30 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
   // bisect the VALUE range (few steps for ordinary score distributions), later ones the key
   // range (at most 32 more steps whatever the values).  If the bracket closes first, the
   // scores inside it are all equal and tie across the cut: the highest chunk indices win.
-  bisect(true);
+  if (PEEL && kp <= kGatePeels && __any(open && nc - kp > 1)) {
+    // The largest score, the largest below it, .., kp of them: the cut lies right below the last.  Exact unless a score of those occurs twice, which
+    // the count below shows.
+    float last = INFINITY;
+    for (int j = 0; j < kp; ++j) {
+      float best = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (t < n_tiles) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) best = fmaxf(best, sc[t][i] < last ? sc[t][i] : -INFINITY);
+        }
+      last = max_xor32_f(best);
+    }
+    if (open) {
+      uint32_t below = float_order_key(last) - 1u;  // (the float below +0 that compares below it is not -0)
+      if (below == 0x7fffffffu) below -= 1u;
+      tau = order_key_float(below);
+      guessed = true;
+      open = false;
+    }
+  } else {
+    bisect(true);
+  }
   bool any_tie = __any(n_eq > 0);  // some row of the wave has a tie across its cut
   // Without a tie in the wave a score is selected iff it lies above tau: the flags of the lane's 16 scores of a tile,
   // shifted in one by one (w + w + flag: one add with carry each), highest first.
@@ -372,7 +401,7 @@ __device__ __forceinline__ void gate_row_block(const fmoba_attn_fwd_args &a, con
     const int rp = row + off, own = causal && valid && rp >= 0 ? rp / Bn : -1;
     const int nc = min(causal ? min(max(own, 0), Cb) : valid ? Cb : 0, nsc);
     uint32_t *selp = gate.sel + (int64_t)h * gate.W * a.total_q + q0 + row;
-    gate_select<T, HD, NT>(ldsTile, qb, lane, n_tiles, nc, causal ? gate.topk - 1 : gate.topk, own, valid, nw, [&](int t, uint32_t w) {
+    gate_select<T, HD, NT, (SPLIT > 1)>(ldsTile, qb, lane, n_tiles, nc, causal ? gate.topk - 1 : gate.topk, own, valid, nw, [&](int t, uint32_t w) {
       if (hh == 0) sBits[t * 32 * RW + wave * 32 + lane] = w;
       if (gate.sel != nullptr) {
         if (valid && hh == 0) selp[(int64_t)t * a.total_q] = w;

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
   const int own = a.is_causal && valid && rp >= 0 ? rp / B : -1;
   const int seg = m0 / p.seg_rows;
   uint32_t *selp = p.sel + (int64_t)h * p.W * a.total_q + q0 + r;
-  gate_select<T, HD, NT>(ldsTile, qf, lane, n_tiles, nc, kp, own, valid, p.W, [&](int t, uint32_t w) {
+  gate_select<T, HD, NT, true>(ldsTile, qf, lane, n_tiles, nc, kp, own, valid, p.W, [&](int t, uint32_t w) {
     if (valid && hh == 0) selp[(int64_t)t * a.total_q] = w;
     // per-chunk counts of this wave's 32 rows (both halves of the wave hold the rows' words)
     if (p.segcnt != nullptr && __any(w != 0u)) {
