@@ -18,9 +18,9 @@ struct FwdRowsDirectSmem {
   static constexpr size_t ring = 4 * tile;                    // K, K, V, V: the rings of one set of waves
   static constexpr size_t oStep = SPLIT * ring;               // int[step_cap]: key block | chunk << 16
   static constexpr int UPW = ROWS / 64;                       // unions of 64 rows' selection words per word
-  // behind the steps, sized by the call: uint32[nw][UPW] unions, uint32[nw][ROWS] the rows' selection words
-  static size_t bytes(int step_cap, int nw) { return oStep + ((size_t)step_cap + (size_t)nw * (UPW + ROWS)) * 4; }
-  static_assert((size_t)RW * 32 * LDO * 2 <= ring && (size_t)RW * HD * 128 <= ring && SPLIT * RW * 512 <= ring, "output tiles must fit the K/V rings");
+  // behind the steps, sized by the call: uint32[nw][UPW] unions, uint32[nw][ROWS] the rows' selection words, int[kRowGateChunks] counts of those that choose their chunks
+  static size_t bytes(int step_cap, int nw) { return oStep + ((size_t)step_cap + (size_t)nw * (UPW + ROWS) + kRowGateChunks) * 4; }
+  static_assert((size_t)RW * 32 * LDO * 2 <= ring && (size_t)RW * HD * 128 <= ring, "output tiles must fit the K/V rings");
 };
 
 // IN_LDS: the rows' words are in sBits already, visible to every thread.
@@ -81,6 +81,34 @@ __device__ __forceinline__ int row_block_steps(const uint32_t *words, int64_t st
   }
   __syncthreads();
   return nstep_all;
+}
+
+// The same steps where the rows' words are in sBits and the chunks no more than kRowGateChunks, by every wave for itself: all write the same list and none waits for
+// another (two barriers and the LDS reads behind them were 1800 clocks in front of a workgroup's first loads, 700 are left).  Ends with the list visible to the wave.
+template <int ROWS>
+__device__ __forceinline__ int gated_row_block_steps(int kend, int Bn, int nw, int step_cap, int *sStep, const uint32_t *sBits) {
+  static_assert(kRowGateChunks == 64, "a chunk per lane");
+  const int lane = threadIdx.x & 63, sub = Bn >> 6;
+  const int nchunk = kend > 0 ? min((kend + Bn - 1) / Bn, nw * 32) : 0;
+  uint32_t x[2] = {0u, 0u};
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+    if (w < nw) {
+#pragma unroll
+      for (int r = 0; r < ROWS; r += 64) x[w] |= sBits[w * ROWS + r + lane];
+    }
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(or_wave(x[0])), hi = __builtin_amdgcn_readfirstlane(or_wave(x[1]));
+  unsigned long long u = ((unsigned long long)hi << 32) | lo;
+  if (nchunk < 64) u &= (1ull << nchunk) - 1ull;
+  if ((u >> lane) & 1ull) {
+    int pos = (int)__popcll(u & ((1ull << lane) - 1ull)) * sub;
+    const int cnt = min(sub, (kend - lane * Bn + 63) >> 6);
+    for (int jb = 0; jb < cnt; ++jb, ++pos)
+      if (pos < step_cap) sStep[pos] = (lane * sub + jb) | (lane << 16);
+  }
+  wave_lds_fence();
+  const int last = nchunk - 1;
+  return u == 0ull ? 0 : (int)__popcll(u) * sub - (((u >> last) & 1ull) ? sub - min(sub, (kend - last * Bn + 63) >> 6) : 0);
 }
 
 }  // namespace fmoba

@@ -462,34 +462,37 @@ __global__ __launch_bounds__(512) void attn_fwd_rows_loader_kernel(fmoba_attn_fw
 // 166; training step of 8191 tokens of short documents 122.2 -> 116.4, 5000 tokens, 8 heads of 112 216 -> 211, 8 x 4096 tokens, 32 over 8 heads, forward 1262
 // -> 1234; nothing from 24571 tokens of training on.  (One to six scalars of these instances are spilled, none without the choice.)
 // RW: waves of a set, which share its tiles.  SPLIT = 2 (4): two (four) sets of waves take turns at the steps of the same rows, with
-// rings of their own; the results of a row meet in LDS at the end.  Which of them: launch_rows.
+// rings of their own; the results of a row meet in LDS at the end.  KH = 2: the tiles of a set are two waves', half kh of the keys each.  Which of them: launch_rows.
 // ------------------------------------------------------------------------------------
-template <typename T, int HD, int RW, int SPLIT, bool GATED>
-__global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, ItemOrder order, RowGate gate) {
+template <typename T, int HD, int RW, int SPLIT, int KH, bool GATED>
+__global__ __launch_bounds__(SPLIT * KH * RW * 64, 2) void attn_fwd_rows_kernel(fmoba_attn_fwd_args a, const uint32_t *bm, int nw, int step_cap, ItemOrder order, RowGate gate) {
   typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
   constexpr int kRows = SM::ROWS;
   constexpr int KS = HD / 16, LDO = SM::LDO, NDT = HD / 32, VPR = HD / 8;
-  constexpr int NTHR = SPLIT * RW * 64;
+  constexpr int NSETS = SPLIT * KH, NTHR = NSETS * RW * 64;
+  constexpr int NKT = 2 / KH;           // 32-key halves of a tile that a wave takes
   constexpr int RB = HD * 2;            // bytes of a tile row
-  constexpr int NI = VPR / RW;          // direct-to-LDS instructions (64 lanes x 16 bytes) per tile and feeding wave
-  static_assert(NI >= 1 && NI * RW == VPR, "the waves of a set share the loads of a tile");
+  constexpr int FW = KH * RW;           // waves that share a ring
+  constexpr int NI = VPR / FW;          // direct-to-LDS instructions (64 lanes x 16 bytes) per tile and wave
+  static_assert(NI >= 1 && NI * FW == VPR, "the waves of a ring share the loads of a tile");
   extern __shared__ __attribute__((aligned(256))) uint8_t smem[];
   int *sStep = reinterpret_cast<int *>(smem + SM::oStep);
   uint32_t *sUnion = reinterpret_cast<uint32_t *>(sStep + step_cap);
   uint32_t *sBits = sUnion + nw * SM::UPW;
 
   // the longest walks (last rows of a causal sequence) start first
-  int b, h, rb, q0, Lq, k0, Lk;
+  int b, h, rb, q0, Lq, k0, Lk, km0 = 0, Cm = 0;  // km0, Cm: the sequence's first chunk mean and how many
   if (order == kListedLongestFirst) {
-    const BlockItem item = listed_item<kRows, true>(blockIdx.x, a.batch, a.heads, a.max_seqlen_q, a.cu_seqlens_q, a.cu_seqlens_k);
+    const BlockItem item = listed_item<kRows, true>(blockIdx.x, a.batch, a.heads, a.max_seqlen_q, a.cu_seqlens_q, a.cu_seqlens_k, GATED ? gate.cu_seqlens_km : nullptr);
     if (item.b < 0) return;
-    b = item.b, h = item.h, rb = item.idx, q0 = item.q0, Lq = item.Lq, k0 = item.k0, Lk = item.Lk;
+    b = item.b, h = item.h, rb = item.idx, q0 = item.q0, Lq = item.Lq, k0 = item.k0, Lk = item.Lk, km0 = item.m0, Cm = item.Cm;
   } else {
     const int nrb = (a.max_seqlen_q + kRows - 1) / kRows;
     const PairItem item = xcd_pair_item(blockIdx.x, a.batch * a.heads, nrb, false, order == kLongestFirst);
     b = item.pair / a.heads, h = item.pair - b * a.heads, rb = nrb - 1 - item.idx;
     q0 = a.cu_seqlens_q[b], Lq = a.cu_seqlens_q[b + 1] - q0;
     k0 = a.cu_seqlens_k[b], Lk = a.cu_seqlens_k[b + 1] - k0;
+    if constexpr (GATED) km0 = gate.cu_seqlens_km[b], Cm = gate.cu_seqlens_km[b + 1] - km0;
   }
   const int r0 = rb * kRows;
   if (r0 >= Lq) return;
@@ -497,7 +500,9 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   const int D = a.head_dim;
   const int hk = h / (a.heads / a.heads_k);
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5;
-  const int wave = wave_all % RW, set = wave_all / RW;  // rows 32 wave .., steps set, set + SPLIT, ..
+  const int wave = wave_all % RW, sid = wave_all / RW;    // rows 32 wave ..
+  const int set = sid / KH, kh = sid % KH;                // steps set, set + SPLIT, .., half kh of the keys of a tile
+  const int feeder = wave_all % FW;
   const bool causal = a.is_causal != 0;
   const int Bn = a.lg_block_n;
   const float scale_log2 = a.softmax_scale * 1.4426950408889634f;
@@ -516,9 +521,9 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   const int kend = min(Lk, causal ? rlast + off + 1 : Lk);  // keys [0, kend) are visible to some row
   int nstep_all;
   if constexpr (GATED) {
-    static_assert(row_gate_lds<HD>() <= SM::ring, "the chunk means and the counts lie where the K/V rings will");
-    gate_row_block<T, HD, RW, SPLIT>(a, gate, smem, sBits, qb, b, h, hk, q0, r0, rlast, Lq, off, nw);
-    nstep_all = row_block_steps<kRows, NTHR, true>(nullptr, 0, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
+    static_assert(row_gate_lds<HD>() <= SM::ring, "the chunk means lie where the K/V rings will");
+    gate_row_block<T, HD, RW, NSETS>(a, gate, smem, sBits, reinterpret_cast<int *>(sBits + nw * kRows), qb, b, h, hk, q0, r0, rlast, Lq, off, nw, km0, Cm);
+    nstep_all = gated_row_block_steps<kRows>(kend, Bn, nw, step_cap, sStep, sBits);
   } else {
     nstep_all = row_block_steps<kRows, NTHR>(bm + (int64_t)h * nw * a.total_q + q0 + r0, a.total_q, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
   }
@@ -537,7 +542,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   typedef std::integral_constant<int, 0> C0;
   typedef std::integral_constant<int, 1> C1;
   if (nstep_wg == 0) {  // no visible selected key: out = 0, lse = +inf for the rows of this block
-    if (valid && set == 0) {
+    if (valid && sid == 0) {
       uint16_t *op = reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + row) * a.o_row_stride + (int64_t)h * a.o_head_stride;
       for (int e = hh * 8; e < D; e += 16) *reinterpret_cast<Pack8 *>(op + e) = zero_pack8();
       if (hh == 0) a.softmax_lse[(int64_t)h * a.total_q + q0 + row] = INFINITY;
@@ -556,23 +561,23 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int v = (wave * NI + i) * 64 + lane, tr = v / VPR, p = v - tr * VPR;
+      const int v = (feeder * NI + i) * 64 + lane, tr = v / VPR, p = v - tr * VPR;
       const uint32_t e = (uint32_t)min((p ^ tile_swz<HD>(tr)) * 8, D - 8);
-      lofK[i] = ((uint32_t)tr * (uint32_t)a.k_row_stride + e) * 2u;
-      lofV[i] = ((uint32_t)tr * (uint32_t)a.v_row_stride + e) * 2u;
+      lofK[i] = run_offset(((uint32_t)tr * (uint32_t)a.k_row_stride + e) * 2u, i % 4);
+      lofV[i] = run_offset(((uint32_t)tr * (uint32_t)a.v_row_stride + e) * 2u, i % 4);
     }
   }
   auto feed = [&](const uint16_t *g, uint32_t row_stride, const uint32_t(&lof)[NI], uint32_t lds_ring, int stage, int t) {
     const int key0 = (entry(t) & 0xffff) << 6;
-    const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + wave * NI * 1024);
+    const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + feeder * NI * 1024);
     if (key0 + 64 <= Lk) {
       const uint16_t *base = g + (uint64_t)(uint32_t)key0 * row_stride;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) global_to_lds16_sbase(lof[i], base, dst + (uint32_t)(i * 1024));
+      global_to_lds16_run<0, (NI < 4 ? NI : 4)>(lof, base, dst);
+      if constexpr (NI > 4) global_to_lds16_run<0, NI - 4>(lof + 4, base, dst + 4096u);
     } else {
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        const int v = (wave * NI + i) * 64 + lane, tr = v / VPR, p = v - tr * VPR;  // row of the tile, piece
+        const int v = (feeder * NI + i) * 64 + lane, tr = v / VPR, p = v - tr * VPR;  // row of the tile, piece
         const uint32_t e = (uint32_t)min((p ^ tile_swz<HD>(tr)) * 8, D - 8);
         const uint32_t key = (uint32_t)min(key0 + tr, Lk - 1);
         global_to_lds16(g + ((uint64_t)key * row_stride + e), dst + (uint32_t)(i * 1024));
@@ -601,14 +606,14 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
-  f32x16 st[2][2];  // S^T of step t in st[t & 1]: register i of tile kt <-> key kt*32 + acc_row(i, hh), this lane's row
+  f32x16 st[2][NKT];  // S^T of step t in st[t & 1]: register i of tile kt <-> key (kh + kt)*32 + acc_row(i, hh), this lane's row
   float m_run = -INFINITY, l_run = 0.f;  // running maximum of the raw scores, running sum (this half of the wave)
   // byte offsets of this lane's pieces inside a tile: row reads (key lane % 32 of a 32-key half, pieces hh * KS ..) and
   // transposing reads (key (lane % 16) / 4 + 4 hh, feature tile 0); every other operand is an exclusive-or on the piece
   // bits plus a constant
-  const uint32_t rowoff = (uint32_t)((lane & 31) * RB + ((tile_frag_piece<HD>(hh, 0) ^ tile_swz<HD>(lane & 31)) * 16));
+  const uint32_t rowoff = (uint32_t)((kh * 32 + (lane & 31)) * RB + ((tile_frag_piece<HD>(hh, 0) ^ tile_swz<HD>(lane & 31)) * 16));
   const int li = lane & 15, r0t = (li >> 2) + 4 * hh;
-  const uint32_t troff = (uint32_t)(r0t * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
+  const uint32_t troff = (uint32_t)((kh * 32 + r0t) * RB + ((((((lane >> 4) & 1) * 2 + ((li & 3) >> 1))) ^ tile_swz<HD>(r0t)) * 16) + (li & 1) * 8);
   auto opaque = [](uint32_t &x) {
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("" : "+v"(x));
@@ -622,9 +627,9 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     return lds_tr8(tile_tr_addr<HD>(tv, dt) + o, tile_tr_addr8<HD>(tv, dt) + o);
   };
   // S of the first step, not overlapped with anything
-  auto s_plain = [&](uint32_t ak, f32x16(&sn)[2]) {
+  auto s_plain = [&](uint32_t ak, f32x16(&sn)[NKT]) {
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+    for (int kt = 0; kt < NKT; ++kt) {
       Pack8 kf[KS];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) kf[ks] = k_frag(ak, kt, ks);
@@ -639,15 +644,15 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
   // A step in three parts.  part0: masks, row maximum and the reference point of step t (vector arithmetic); part1:
   // S(t + 1) on the matrix cores under the exponentials of step t; part2: O^T += V^T P^T of step t (matrix cores).
   // The other wave of the SIMD belongs to another workgroup (or set) and is in whatever part it is in.
-  Pack8 pf[2][2];      // P^T as the B operand of O^T += V^T P^T, straight from the accumulators
+  Pack8 pf[NKT][2];    // P^T as the B operand of O^T += V^T P^T, straight from the accumulators
   Pack8 kf[KS];        // K operands of S(t + 1): read at the start of part0, their latency runs under its arithmetic
-  Pack8 vt[2][2];      // V^T operands of the first feature tile of step t: read at the end of part1
+  Pack8 vt[NKT][2];    // V^T operands of the first feature tile of step t: read at the end of part1
   float neg_mc = 0.f;  // minus the reference point of the row's exponentials, scaled; -inf for a row that skips the step
   int s_nx = entry(0);  // entry of the next step and this row's word of selection bits for its chunk
   uint32_t word_nx = sBits[((s_nx >> 16) >> 5) * kRows + wave * 32 + (lane & 31)];
   auto part0 = [&](auto par, int t) {
     constexpr int P = decltype(par)::value;
-    f32x16(&sc)[2] = st[P];
+    f32x16(&sc)[NKT] = st[P];
     {
       uint32_t akn = ldsK + (uint32_t)(((t + 1) & 1) * (int)SM::tile) + rowoff;  // K(t + 1)
       opaque(akn);
@@ -657,13 +662,13 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     // (the step's entry and this row's selection word were read during the step before: two dependent LDS reads at
     // this place would be waited for with nothing to do, by every wave at the start of every step)
     const int s = s_nx;
-    const int key0 = (s & 0xffff) << 6, c = s >> 16;
+    const int key0 = ((s & 0xffff) << 6) + kh * 32, c = s >> 16;
     const uint32_t myword = word_nx;
     const bool active = valid && ((myword >> (c & 31)) & 1u) != 0u && lim >= key0;
     const int lim_rel = active ? lim - key0 : -1;
-    if (!__all(lim_rel >= 63 || lim_rel < 0)) {
+    if (!__all(lim_rel >= 32 * NKT - 1 || lim_rel < 0)) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int jrel = kt * 32 + 8 * (i >> 2) + (i & 3) + 4 * hh;
@@ -672,7 +677,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     }
     float mloc = -INFINITY;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, sc[kt][i]);
     mloc = max_xor32_f(mloc);
@@ -697,34 +702,35 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     constexpr int P = decltype(par)::value;
     uint32_t akn = ldsK + (uint32_t)(((t + 1) & 1) * (int)SM::tile) + rowoff;  // K(t + 1)
     opaque(akn);
-    f32x16(&sc)[2] = st[P];
-    f32x16(&sn)[2] = st[P ^ 1];
+    f32x16(&sc)[NKT] = st[P];
+    f32x16(&sn)[NKT] = st[P ^ 1];
     uint32_t tv = ldsV + (uint32_t)((t & 1) * (int)SM::tile) + troff;  // V(t)
     opaque(tv);
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) sn[kt][i] = 0.f;
     float lsum = 0.f;
-    static_for<16>([&](auto gi) {
+    constexpr int NG = 8 * NKT;  // pairs of scores of a lane
+    static_for<NG>([&](auto gi) {
       constexpr int g = decltype(gi)::value;
-      constexpr int M0 = g * (2 * KS) / 16, M1 = (g + 1) * (2 * KS) / 16;
+      constexpr int M0 = g * (NKT * KS) / NG, M1 = (g + 1) * (NKT * KS) / NG;
 #pragma unroll
       for (int mi = M0; mi < M1; ++mi) {
         const int kt = mi / KS, ks = mi % KS;
         sn[kt] = mfma32<T>(kf[ks], qb[ks], sn[kt]);
-        if (kt == 0) kf[ks] = k_frag(akn, 1, ks);  // the operand of the second key tile takes the register over
+        if (NKT == 2 && kt == 0) kf[ks] = k_frag(akn, 1, ks);  // the operand of the second key tile takes the register over
       }
       constexpr int kte = g / 8, j = g % 8;
       const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[kte][2 * j], scale_log2, neg_mc));
       const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[kte][2 * j + 1], scale_log2, neg_mc));
       lsum += p0 + p1;
       pf[kte][j / 4].w[j % 4] = pack2<T>(p0, p1);
-      if (g == 2) s_nx = entry(t + 1);
-      if (g == 8) word_nx = sBits[((s_nx >> 16) >> 5) * kRows + wave * 32 + (lane & 31)];
-      if (g == 14) {  // V^T operands of the first feature tile
+      if (g == NG / 8) s_nx = entry(t + 1);
+      if (g == NG / 2) word_nx = sBits[((s_nx >> 16) >> 5) * kRows + wave * 32 + (lane & 31)];
+      if (g == NG - 2) {  // V^T operands of the first feature tile
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
           for (int s2 = 0; s2 < 2; ++s2) vt[kt][s2] = v_frag(tv, 0, kt, s2);
       }
@@ -738,7 +744,7 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     static_for<NDT>([&](auto di) {
       constexpr int dt = decltype(di)::value;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
           o[dt] = mfma32<T>(vt[kt][s2], pf[kt][s2], o[dt]);
@@ -778,69 +784,78 @@ __global__ __launch_bounds__(SPLIT * RW * 64, 2) void attn_fwd_rows_kernel(fmoba
     if (t + 1 < nturn) step(C1{}, t + 1);
   }
   // (every wave is done with the rings and nothing is in flight: they now hold the sets' sums, then the output tiles)
-  if constexpr (SPLIT > 1) {
-    auto sums_of = [&](int st) { return reinterpret_cast<float *>(smem + st * SM::ring) + (size_t)wave * (HD / 2) * 64 + lane; };  // [wave][HD / 2 registers][64 lanes], in the set's rings
-    auto ml_of = [&](int st) { return reinterpret_cast<float *>(smem) + (st * RW + wave) * 128 + lane; };                            // [set][wave][2][64]
-    if (set > 0) {
+  float l_tot = l_run;
+  constexpr int NP = HD / 2 / NSETS;  // registers of O^T whose features a set takes to the end
+  float share[NP];
+  if constexpr (NSETS == 1) {
+    static_for<NP>([&](auto rc) { share[decltype(rc)::value] = o[decltype(rc)::value / 16][decltype(rc)::value % 16]; });
+  } else {
+    static_assert(NP % 4 == 0 && (size_t)NSETS * RW * HD * 128 <= SPLIT * SM::ring, "whole groups of features; the sums fit the rings");
+    // Sums as [set][wave][HD / 2 registers][64 lanes], m and l behind the lists.  Every set adds up an equal share of the features (the first set alone took 8100
+    // clocks for four of them at head dimension 128, 4000 of 64, and all LDS reads).
+    auto sums_of = [&](int st) { return reinterpret_cast<float *>(smem) + (size_t)(st * RW + wave) * (HD / 2) * 64 + lane; };
+    float *ml = reinterpret_cast<float *>(sBits + nw * kRows + kRowGateChunks) + wave * 128 + lane;  // of set st: RW * 128 st further on
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
+    for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sums_of(set)[(dt * 16 + i) * 64] = o[dt][i];
-      ml_of(set)[0] = m_run;
-      ml_of(set)[64] = l_run;
-    }
+      for (int i = 0; i < 16; ++i) sums_of(sid)[(dt * 16 + i) * 64] = o[dt][i];
+    ml[sid * RW * 128] = m_run;
+    ml[sid * RW * 128 + 64] = l_run;
     __syncthreads();
-    if (set == 0) {
+    float f[NSETS], mn = -INFINITY;
 #pragma unroll
-      for (int st = 1; st < SPLIT; ++st) {
-        const float m1 = ml_of(st)[0], l1 = ml_of(st)[64];
-        const float mn = fmaxf(m_run, m1), mref = mn == -INFINITY ? 0.f : mn;
-        const float f0 = __builtin_amdgcn_exp2f((m_run - mref) * scale_log2), f1 = __builtin_amdgcn_exp2f((m1 - mref) * scale_log2);
-        m_run = mn;
-        l_run = l_run * f0 + l1 * f1;
+    for (int st = 0; st < NSETS; ++st) f[st] = ml[st * RW * 128], mn = fmaxf(mn, f[st]);
+    m_run = mn;
+    const float mref = mn == -INFINITY ? 0.f : mn;
+    l_tot = 0.f;
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[dt][i] = o[dt][i] * f0 + sums_of(st)[(dt * 16 + i) * 64] * f1;
-      }
+    for (int st = 0; st < NSETS; ++st) {
+      f[st] = __builtin_amdgcn_exp2f((f[st] - mref) * scale_log2);
+      l_tot += ml[st * RW * 128 + 64] * f[st];
     }
-    __syncthreads();  // (the output tiles lie where m and l of the other sets did)
-    if (set > 0) return;
+#pragma unroll
+    for (int r = 0; r < NP; ++r) {
+      share[r] = 0.f;
+#pragma unroll
+      for (int st = 0; st < NSETS; ++st) share[r] += sums_of(st)[(sid * NP + r) * 64] * f[st];
+    }
+    __syncthreads();  // (the output tiles lie where the sums did)
   }
 
-  const float l_tot = sum_xor32_f(l_run);
+  l_tot = sum_xor32_f(l_tot);
   const bool empty = !(l_tot > 0.f);
   const float inv = empty ? 0.f : 1.f / l_tot;
   uint16_t *sOut = reinterpret_cast<uint16_t *>(smem) + (size_t)wave * 32 * LDO;
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<uint2 *>(sOut + (lane & 31) * LDO + dt * 32 + 8 * g + 4 * hh) =
-          make_uint2(pack2<T>(o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv), pack2<T>(o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv));
-  if (valid && hh == 0)
+  for (int g = 0; g < NP / 4; ++g)  // (features 2 NP sid .., eight to a group)
+    *reinterpret_cast<uint2 *>(sOut + (lane & 31) * LDO + sid * 2 * NP + 8 * g + 4 * hh) =
+        make_uint2(pack2<T>(share[4 * g] * inv, share[4 * g + 1] * inv), pack2<T>(share[4 * g + 2] * inv, share[4 * g + 3] * inv));
+  if (valid && hh == 0 && sid == 0)
     a.softmax_lse[(int64_t)h * a.total_q + q0 + row] = empty ? INFINITY : (m_run * scale_log2 + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f;
-  wave_lds_fence();
+  if constexpr (NSETS > 1)
+    __syncthreads();
+  else
+    wave_lds_fence();
   // rows leave as 16-byte pieces, VPR of them per row, consecutive lanes taking consecutive pieces
 #pragma unroll
-  for (int v0 = 0; v0 < 32 * VPR; v0 += 64) {
-    const int v = v0 + lane, rl = v / VPR, e = (v - rl * VPR) * 8;
+  for (int v0 = 0; v0 < 32 * VPR; v0 += 64 * NSETS) {
+    const int v = v0 + sid * 64 + lane, rl = v / VPR, e = (v - rl * VPR) * 8;
     const int r2 = r0 + wave * 32 + rl;
-    if (r2 < Lq && e < D) {
+    if (rl < 32 && r2 < Lq && e < D) {
       const Pack8 x = *reinterpret_cast<const Pack8 *>(sOut + rl * LDO + e);
       *reinterpret_cast<Pack8 *>(reinterpret_cast<uint16_t *>(a.out) + (int64_t)(q0 + r2) * a.o_row_stride + (int64_t)h * a.o_head_stride + e) = x;
     }
   }
 }
 
-template <typename T, int HD, int RW, int SPLIT>
+template <typename T, int HD, int RW, int SPLIT, int KH>
 static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, const RowGate *gate, hipStream_t s) {
   typedef FwdRowsDirectSmem<HD, RW, SPLIT> SM;
-  auto kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT, false>;
+  auto kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT, KH, false>;
   if constexpr (HD != 96)
-    if (gate != nullptr) kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT, true>;
+    if (gate != nullptr) kern = attn_fwd_rows_kernel<T, HD, RW, SPLIT, KH, true>;
   const int step_cap = ceil_div(a.max_seqlen_k, 64);  // (at most kRowsStepCap: fwd_rows_feasible)
-  const size_t smem = SM::bytes(step_cap, nw);
+  const size_t smem = SM::bytes(step_cap, nw) + (SPLIT * KH > 1 ? SPLIT * KH * RW * 512 : 0);  // (m and l of the sets)
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("attn_fwd: cannot reserve %zu bytes of LDS", smem);
     return 2;
@@ -851,7 +866,7 @@ static int launch_rows_split(const fmoba_attn_fwd_args &a, const uint32_t *bm, i
     set_error("attn_fwd: too many (sequence, head, row block) work items");
     return 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * RW * 64), smem, s, a, bm, nw, step_cap, order, gate != nullptr ? *gate : RowGate{});
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(SPLIT * KH * RW * 64), smem, s, a, bm, nw, step_cap, order, gate != nullptr ? *gate : RowGate{});
   return 0;
 }
 // Four sets share a walk (head dimensions up to 64) where the workgroups of 64 rows are no more than the compute units, as their rings leave a unit
@@ -875,15 +890,26 @@ static int rows_sets(const fmoba_attn_fwd_args &a) {
   if (a.head_dim <= 64 && a.max_seqlen_k >= kRowsFourSetsKeys && a.heads * (((int64_t)a.total_q + 63 * a.batch) / 64) <= kRowsFourSets) return 4;
   return (int64_t)a.heads * (a.total_q / 128 + a.batch) <= (a.head_dim > 64 ? 288 : 544) ? 2 : 1;
 }
+// Two sets of waves whose tiles are shared by two waves each, which take a half of their keys (eight waves, the loads and the rings of four): half of a turn's arithmetic in front of a
+// barrier.  Above head dimension 64, where the rings of two sets leave a unit room for one workgroup anyway, from sequences of 1024 keys on (shorter walks lose
+// in the sums what they gain: heads of 128, two sequences of 128 tokens 13.9 -> 14.9 us, four of 512 19.7 -> 20.0): 2048 tokens, 8 heads of 128 36.9 -> 34.1, 16 heads 49.3 -> 47.4,
+// 4096 tokens, 8 heads 73.8 -> 67.8, 3495 tokens, 8 heads of 96 56.5 -> 52.5.  Up to 64, where two workgroups of four waves fit a unit, for the calls that four sets are
+// too many for, up to half as many workgroups again as there are units and their items longest first: 1024 + 2048 tokens, 8 heads (384) 28.2 -> 26.9, 1120 tokens, 16 heads (288) 21.3 ->
+// 20.3, 4096 tokens, 8 heads (512) 46.0 -> 50.7, 6 heads (384, pair by pair) 53.7 -> 59.7.
+constexpr int kRowsHalves = 400;  // (counted with a block more per sequence)
+static bool rows_halves(const fmoba_attn_fwd_args &a) {
+  if (a.max_seqlen_k < kRowsFourSetsKeys) return false;
+  return a.head_dim > 64 || (a.heads * a.batch % 8 == 0 && a.heads * (((int64_t)a.total_q + 63 * a.batch) / 64) <= kRowsHalves);
+}
 template <typename T, int HD>
 static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s, const RowGate *gate = nullptr) {
   const int sets = rows_sets(a);
   if constexpr (HD <= 64)
-    if (sets == 4) return launch_rows_split<T, HD, 2, 4>(a, bm, nw, gate, s);
-  if (sets == 2) return launch_rows_split<T, HD, 2, 2>(a, bm, nw, gate, s);
+    if (sets == 4) return launch_rows_split<T, HD, 2, 4, 1>(a, bm, nw, gate, s);
+  if (sets == 2) return rows_halves(a) ? launch_rows_split<T, HD, 2, 2, 2>(a, bm, nw, gate, s) : launch_rows_split<T, HD, 2, 2, 1>(a, bm, nw, gate, s);
   if constexpr (HD <= 64)
-    if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1>(a, bm, nw, gate, s);
-  return launch_rows_split<T, HD, 4, 1>(a, bm, nw, gate, s);
+    if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1, 1>(a, bm, nw, gate, s);
+  return launch_rows_split<T, HD, 4, 1, 1>(a, bm, nw, gate, s);
 }
 
 template <typename T, int HD>

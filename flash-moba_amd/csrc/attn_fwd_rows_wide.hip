@@ -66,8 +66,9 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_rows_wide_kernel(fmoba_attn_f
   const int kend = min(Lk, causal ? rlast + off + 1 : Lk);  // keys [0, kend) are visible to some row
   int nstep;
   if constexpr (GATED) {
-    static_assert(row_gate_lds<HD>() <= SM::ring, "the chunk means and the counts lie where the K/V rings will");
-    gate_row_block<T, HD, RW, 1>(a, gate, smem, sBits, qb, b, h, hk, q0, r0, rlast, Lq, off, nw);
+    static_assert(row_gate_lds<HD>() + kRowGateChunks * 4 <= SM::ring, "the chunk means and the counts lie where the K/V rings will");
+    const int km0 = gate.cu_seqlens_km[b], Cm = gate.cu_seqlens_km[b + 1] - km0;
+    gate_row_block<T, HD, RW, 1>(a, gate, smem, sBits, reinterpret_cast<int *>(smem + row_gate_lds<HD>()), qb, b, h, hk, q0, r0, rlast, Lq, off, nw, km0, Cm);
     nstep = row_block_steps<kRows, 256, true>(nullptr, 0, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);
   } else {
     nstep = row_block_steps<kRows, 256>(bm + (int64_t)h * nw * a.total_q + q0 + r0, a.total_q, rlast - r0 + 1, kend, Bn, nw, step_cap, sStep, sUnion, sBits);

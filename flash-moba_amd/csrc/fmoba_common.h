@@ -597,14 +597,18 @@ __host__ __device__ __forceinline__ ItemOrder item_order(int64_t total, int long
 struct BlockItem {
   int b, h, idx;       // b < 0: none
   int q0, Lq, k0, Lk;  // the sequence's bounds
+  int m0, Cm;          // its first chunk mean and how many, if asked for
 };
 // item `id` of listed_blocks * heads: block idx of head h of sequence b.  Blocks of query rows come from the last ones (whose walks are the longest) to the
 // first, blocks of keys (rows = false; the first are seen by most rows) from the first to the last.
 template <int BLOCK, bool ROWS>
-__device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, int longest, const int32_t *cu_q, const int32_t *cu_k) {
+__device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, int longest, const int32_t *cu_q, const int32_t *cu_k, const int32_t *cu_km = nullptr) {
   const int lane = threadIdx.x & 63, nper = (longest + BLOCK - 1) / BLOCK;
-  int q_lo = 0, q_hi = 0, k_lo = 0, k_hi = 0;
-  if (lane < batch) q_lo = cu_q[lane], q_hi = cu_q[lane + 1], k_lo = cu_k[lane], k_hi = cu_k[lane + 1];
+  int q_lo = 0, q_hi = 0, k_lo = 0, k_hi = 0, m_lo = 0, m_hi = 0;
+  if (lane < batch) {
+    q_lo = cu_q[lane], q_hi = cu_q[lane + 1], k_lo = cu_k[lane], k_hi = cu_k[lane + 1];
+    if (cu_km != nullptr) m_lo = cu_km[lane], m_hi = cu_km[lane + 1];
+  }
   const int n = id / heads;
   const int h = id - n * heads;
   const int nb = min((max(ROWS ? q_hi - q_lo : k_hi - k_lo, 0) + BLOCK - 1) / BLOCK, nper);
@@ -628,7 +632,7 @@ __device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, i
   const int at = upto(base + lane);
   const unsigned long long more = __ballot(at > n);
   const int l = ROWS ? (int)__popcll(more) - 1 : 64 - (int)__popcll(more);
-  BlockItem w{-1, h, base + l, 0, 0, 0, 0};
+  BlockItem w{-1, h, base + l, 0, 0, 0, 0, 0, 0};
   if (l < 0 || l > 63) return w;
   const unsigned long long have = __ballot(nb > w.idx);
   // Which of the sequences that have such a block: rotated by one from number to number, as in xcd_pair_item and for the same reason (30000 tokens in four
@@ -640,6 +644,7 @@ __device__ __forceinline__ BlockItem listed_item(int id, int batch, int heads, i
   w.b = (int)__ffsll(it) - 1;
   w.q0 = __builtin_amdgcn_readlane(q_lo, w.b), w.Lq = __builtin_amdgcn_readlane(q_hi, w.b) - w.q0;
   w.k0 = __builtin_amdgcn_readlane(k_lo, w.b), w.Lk = __builtin_amdgcn_readlane(k_hi, w.b) - w.k0;
+  if (cu_km != nullptr) w.m0 = __builtin_amdgcn_readlane(m_lo, w.b), w.Cm = __builtin_amdgcn_readlane(m_hi, w.b) - w.m0;
   return w;
 }
 
@@ -657,7 +662,7 @@ __device__ __forceinline__ BlockItem listed_pair_item(int id, int batch, int hea
     upto += lane >= o ? up : 0;
   }
   const int s = id >> 3;
-  BlockItem w{-1, 0, 0, 0, 0, 0, 0};
+  BlockItem w{-1, 0, 0, 0, 0, 0, 0, 0, 0};
   const int b = (int)__popcll(__ballot(lane < batch && upto * np <= s));
   if (b >= batch) return w;
   const int n = __builtin_amdgcn_readlane(nb, b), rest = s - (__builtin_amdgcn_readlane(upto, b) - n) * np, pl = rest / n;
@@ -868,6 +873,37 @@ __device__ __forceinline__ void global_to_lds16_sbase(uint32_t lane_byte_off, co
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_byte_off), "s"(uniform_base), "s"(lds_base) : "memory");
 #else
   (void)lane_byte_off, (void)uniform_base, (void)lds_base;
+#endif
+}
+// N of these loads to consecutive kilobytes from lds_base + 1024 FIRST on.  The instruction's offset moves both addresses, so that one setting of m0 serves
+// all: load i's lane offsets are run_offset(byte offset from the base, FIRST + i).  (m0 cannot be set before the load in front has taken it: a wave that sets it for each of eight loads
+// issues them in 412 clocks, with one setting for four in 96, where nothing else is in the way of them; with four waves and more the vector memory path is.)
+constexpr uint32_t kRunBias = 4096;
+__device__ __forceinline__ constexpr uint32_t run_offset(uint32_t byte_off, int i) { return byte_off + (kRunBias - 1024u * (uint32_t)i); }
+template <int FIRST, int N>
+__device__ __forceinline__ void global_to_lds16_run(const uint32_t *off, const void *uniform_base, uint32_t lds_base) {
+  static_assert(N >= 1 && N <= 4 && FIRST >= 0 && FIRST + N <= 4, "offsets of twelve bits");
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint8_t *from = reinterpret_cast<const uint8_t *>(uniform_base) - kRunBias;
+  if constexpr (N == 1)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(off[0]), "s"(from), "s"(lds_base), "n"(FIRST * 1024) : "memory");
+  else if constexpr (N == 2)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2 offset:%4\n\tglobal_load_lds_dwordx4 %1, %2 offset:%5" ::"v"(off[0]), "v"(off[1]), "s"(from),
+                 "s"(lds_base), "n"(FIRST * 1024), "n"(FIRST * 1024 + 1024)
+                 : "memory");
+  else if constexpr (N == 3)
+    asm volatile(
+        "s_mov_b32 m0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %3 offset:%5\n\tglobal_load_lds_dwordx4 %1, %3 offset:%6\n\tglobal_load_lds_dwordx4 %2, %3 offset:%7" ::"v"(off[0]),
+        "v"(off[1]), "v"(off[2]), "s"(from), "s"(lds_base), "n"(FIRST * 1024), "n"(FIRST * 1024 + 1024), "n"(FIRST * 1024 + 2048)
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024\n\tglobal_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, "
+        "%4 offset:3072" ::"v"(off[0]),
+        "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(from), "s"(lds_base)
+        : "memory");
+#else
+  (void)off, (void)uniform_base, (void)lds_base;
 #endif
 }
 // a * b of two values below 2^24, b the same in every lane: one full-rate instruction (a 32-bit multiply takes four

@@ -97,7 +97,11 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
   // scores: lane (query l%32) gets chunk t*32 + acc_row(i, hh) in register i of tile t;
   // chunks that are not candidates of the row hold -inf
   float sc[NT][16];
-  float vmin = INFINITY, vmax = -INFINITY;
+  // (Chains of dependent instructions take twice as long as independent ones where a wave has its SIMD to itself: four side by side, as far as registers last.)
+  constexpr int NCH = NT <= 2 ? 4 : 1;
+  float vmins[NCH], vmaxs[NCH];
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) vmins[j] = INFINITY, vmaxs[j] = -INFINITY;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     if (t < n_tiles) {
@@ -115,16 +119,17 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
         const bool cand = c < nc;
         const float x = acc[i];
         sc[t][i] = cand ? x : -INFINITY;
-        vmin = fminf(vmin, cand ? x : INFINITY);
-        vmax = fmaxf(vmax, sc[t][i]);
+        vmins[i % NCH] = fminf(vmins[i % NCH], cand ? x : INFINITY);
+        vmaxs[i % NCH] = fmaxf(vmaxs[i % NCH], sc[t][i]);
       }
     } else {
 #pragma unroll
       for (int i = 0; i < 16; ++i) sc[t][i] = -INFINITY;
     }
   }
-  vmin = min_xor32_f(vmin);
-  vmax = max_xor32_f(vmax);
+#pragma unroll
+  for (int j = 1; j < NCH; ++j) vmins[0] = fminf(vmins[0], vmins[j]), vmaxs[0] = fmaxf(vmaxs[0], vmaxs[j]);
+  const float vmin = min_xor32_f(vmins[0]), vmax = max_xor32_f(vmaxs[0]);
 
   // K' = number of scored chunks to keep (the own chunk takes one slot in causal mode).
   // A row keeps every candidate x with x > tau, plus, among the candidates equal to tau_eq,
@@ -232,15 +237,19 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
     // The largest score, the largest below it, .., kp of them: the cut lies right below the last.  Exact unless a score of those occurs twice, which
     // the count below shows.
     float last = INFINITY;
-    for (int j = 0; j < kp; ++j) {
-      float best = -INFINITY;
+    for (int n = 0; n < kp; ++n) {
+      float best[NCH];
+#pragma unroll
+      for (int j = 0; j < NCH; ++j) best[j] = -INFINITY;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         if (t < n_tiles) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) best = fmaxf(best, sc[t][i] < last ? sc[t][i] : -INFINITY);
+          for (int i = 0; i < 16; ++i) best[i % NCH] = fmaxf(best[i % NCH], sc[t][i] < last ? sc[t][i] : -INFINITY);
         }
-      last = max_xor32_f(best);
+#pragma unroll
+      for (int j = 1; j < NCH; ++j) best[0] = fmaxf(best[0], best[j]);
+      last = max_xor32_f(best[0]);
     }
     if (open) {
       uint32_t below = float_order_key(last) - 1u;  // (the float below +0 that compares below it is not -0)
@@ -367,18 +376,17 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
 
 // The gate of a row block, by the workgroup that is about to walk its keys (SPLIT sets of RW waves of 32 rows each; the first set chooses): candidates of some
 // row of the block, their means into LDS, scores, choice, as topk_gate_kernel does it.  Q is asked for and not awaited when it begins, arranged when it ends.
-// The rows' words go to sBits (word w of row r at w * 32 RW + r), and if column lists follow to memory with their counts.  Takes row_gate_lds bytes of `smem`.
+// The rows' words go to sBits (word w of row r at w * 32 RW + r), and if column lists follow to memory with their counts, by way of sHist (kRowGateChunks words).
+// km0, Cb: the sequence's first mean and how many it has.  Takes row_gate_lds bytes of `smem`, which are free when it ends.
 template <int HD>
-constexpr size_t row_gate_lds() { return (size_t)kRowGateChunks * HD * 2 + kRowGateChunks * 4; }
+constexpr size_t row_gate_lds() { return (size_t)kRowGateChunks * HD * 2; }
 template <typename T, int HD, int RW, int SPLIT>
-__device__ __forceinline__ void gate_row_block(const fmoba_attn_fwd_args &a, const RowGate &gate, uint8_t *smem, uint32_t *sBits, Pack8 (&qb)[HD / 16], int b, int h, int hk, int q0,
-                                               int r0, int rlast, int Lq, int off, int nw) {
-  constexpr int NT = kRowGateChunks / 32, VPR = HD / 8, RPI = 64 / VPR, RB = HD * 2, NTHR = SPLIT * RW * 64, KS = HD / 16;
+__device__ __forceinline__ void gate_row_block(const fmoba_attn_fwd_args &a, const RowGate &gate, uint8_t *smem, uint32_t *sBits, int *sHist, Pack8 (&qb)[HD / 16], int b, int h, int hk,
+                                               int q0, int r0, int rlast, int Lq, int off, int nw, int km0, int Cb) {
+  constexpr int NT = kRowGateChunks / 32, VPR = HD / 8, RPI = 64 / VPR, NTHR = SPLIT * RW * 64, KS = HD / 16;
   const int tid = threadIdx.x, lane = tid & 63, wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), hh = lane >> 5, wave = wave_all % RW, set = wave_all / RW;
   const int Bn = a.lg_block_n, D = a.head_dim, row = r0 + wave * 32 + (lane & 31);
   const bool causal = a.is_causal != 0, valid = row < Lq;
-  int *sHist = reinterpret_cast<int *>(smem + (size_t)NT * 32 * RB);
-  const int km0 = gate.cu_seqlens_km[b], Cb = gate.cu_seqlens_km[b + 1] - km0;
   const int rmax = rlast + off;
   const int nsc = min(causal ? (rmax < 0 ? 0 : min(Cb, rmax / Bn)) : Cb, min(a.max_cols, kRowGateChunks));
   const int n_tiles = (nsc + 31) >> 5;
