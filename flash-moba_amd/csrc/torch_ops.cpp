@@ -272,25 +272,28 @@ struct Attention : public torch::autograd::Function<Attention> {
       // heads of a group that the library does not add up itself are summed below (flash_moba_api.cpp:842-845)
       const int32_t dkv_heads = fmoba_attn_bwd_dkv_heads(&a);
       const bool grouped = dkv_heads != s.heads_k;
-      const Tensor dk_e = grouped ? at::empty({s.total_k, dkv_heads, s.dim}, k.options()) : dk, dv_e = grouped ? at::empty({s.total_k, dkv_heads, s.dim}, v.options()) : dv;
       const Tensor softmax_d = at::empty({s.heads, s.total_q + 128 * s.batch}, q.options().dtype(at::kFloat));
       a.dout = dout.data_ptr(), a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr(), a.out = out.data_ptr(), a.softmax_lse = lse.data_ptr<float>();
-      a.dq = dq.data_ptr(), a.dk = dk_e.data_ptr(), a.dv = dv_e.data_ptr(), a.softmax_d = softmax_d.data_ptr<float>();
+      a.dq = dq.data_ptr(), a.dk = dk.data_ptr(), a.dv = dv.data_ptr(), a.softmax_d = softmax_d.data_ptr<float>();
       a.col_offsets = co.data_ptr<int64_t>(), a.col_nnz = cn.data_ptr<int32_t>(), a.row_indices = ind.data_ptr<int32_t>(), a.num_row_indices = ind.numel();
       a.cu_seqlens_q = cu_q.data_ptr<int32_t>(), a.cu_seqlens_k = cu_k.data_ptr<int32_t>();
       a.q_row_stride = q.stride(0), a.q_head_stride = q.stride(1), a.k_row_stride = k.stride(0), a.k_head_stride = k.stride(1);
       a.v_row_stride = v.stride(0), a.v_head_stride = v.stride(1), a.o_row_stride = out.stride(0), a.o_head_stride = out.stride(1);
       a.do_row_stride = dout.stride(0), a.do_head_stride = dout.stride(1), a.dq_row_stride = dq.stride(0), a.dq_head_stride = dq.stride(1);
-      a.dk_row_stride = dk_e.stride(0), a.dk_head_stride = dk_e.stride(1), a.dv_row_stride = dv_e.stride(0), a.dv_head_stride = dv_e.stride(1);
+      a.dk_row_stride = dk.stride(0), a.dk_head_stride = dk.stride(1), a.dv_row_stride = dv.stride(0), a.dv_head_stride = dv.stride(1);
       const size_t n = fmoba_attn_bwd_workspace_bytes(&a);
-      const Tensor ws = bytes_like(q, n);
+      const int64_t one = grouped ? int64_t(s.total_k) * dkv_heads * s.dim : 0;
+      const Tensor ws = bytes_like(q, up256(n) + 4 * one);  // the heads kept apart lie behind the library's workspace
+      char *apart = static_cast<char *>(ws.data_ptr()) + up256(n);
+      if (grouped) {
+        a.dk = apart, a.dv = apart + 2 * one;
+        a.dk_row_stride = a.dv_row_stride = int64_t(dkv_heads) * s.dim, a.dk_head_stride = a.dv_head_stride = s.dim;
+      }
       a.workspace = ws.data_ptr(), a.workspace_bytes = n;
       check(fmoba_attn_bwd_ranked(&a, visit_ptr(visits), dkv_heads, 7, s.stream));
       t_partials = fmoba_attn_bwd_uses_partials(&a);
-      if (grouped) {
-        at::sum_out(dk, dk_e.view({s.total_k, s.heads_k, dkv_heads / s.heads_k, s.dim}), at::IntArrayRef{2});
-        at::sum_out(dv, dv_e.view({s.total_k, s.heads_k, dkv_heads / s.heads_k, s.dim}), at::IntArrayRef{2});
-      }
+      if (grouped)
+        check(fmoba_sum_grouped_heads(apart, dk.data_ptr(), dv.data_ptr(), s.total_k, dkv_heads, s.heads_k, s.dim, dk.stride(0), dk.stride(1), dv.stride(0), dv.stride(1), s.dtype, s.stream));
       res[0] = dq, res[1] = dk, res[2] = dv;
     }
     if (at::GradMode::is_enabled()) {  // the gradients have no gradients: say so if anything asks for them

@@ -116,6 +116,7 @@ EXPORTS = {
     "fmoba_pool_and_gate_ranked": (c_i32, [ctypes.POINTER(MeanPoolArgs), ctypes.POINTER(FusedTopkArgs), ctypes.POINTER(CscRanks), c_vp]),
     "fmoba_attn_bwd_grouped": (c_i32, [ctypes.POINTER(AttnBwdArgs), c_i32, c_i32, c_vp]),
     "fmoba_attn_bwd_dkv_heads": (c_i32, [ctypes.POINTER(AttnBwdArgs)]),
+    "fmoba_sum_grouped_heads": (c_i32, [c_vp, c_vp, c_vp, c_i64, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64, c_i64, c_i32, c_vp]),
     "fmoba_attn_bwd_workspace_bytes": (c_sz, [ctypes.POINTER(AttnBwdArgs)]),
     "fmoba_attn_bwd_uses_partials": (c_i32, [ctypes.POINTER(AttnBwdArgs)]),
     "fmoba_attn_bwd": (c_i32, [ctypes.POINTER(AttnBwdArgs), c_vp]),
@@ -642,8 +643,8 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
         # side; the rest is summed below (flash_moba_api.cpp:764-771,842-845)
         dkv_heads = lib.fmoba_attn_bwd_dkv_heads(ctypes.byref(a)) if heads_k != heads else heads
         if dkv_heads != heads_k:
-            dk_e = torch.empty((total_k, dkv_heads, d), dtype=dtype, device=dev)
-            dv_e = torch.empty((total_k, dkv_heads, d), dtype=dtype, device=dev)
+            apart = torch.empty((2, total_k, dkv_heads, d), dtype=dtype, device=dev)
+            dk_e, dv_e = apart[0], apart[1]
             a.dk, a.dk_row_stride, a.dk_head_stride = dk_e.data_ptr(), dk_e.stride(0), dk_e.stride(1)
             a.dv, a.dv_row_stride, a.dv_head_stride = dv_e.data_ptr(), dv_e.stride(0), dv_e.stride(1)
         ws_bytes = lib.fmoba_attn_bwd_workspace_bytes(ctypes.byref(a))
@@ -658,6 +659,10 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
             _phases(lambda mask: _check(lib.fmoba_attn_bwd_ranked(ctypes.byref(a), row_visits, dkv_heads, mask, _stream())))
         if dkv_heads != heads_k:
             grp = dkv_heads // heads_k
-            torch.sum(dk_e.view(total_k, heads_k, grp, d), dim=2, out=dk)
-            torch.sum(dv_e.view(total_k, heads_k, grp, d), dim=2, out=dv)
+            if dk_ is None and dv_ is None:
+                _check(lib.fmoba_sum_grouped_heads(apart.data_ptr(), dk.data_ptr(), dv.data_ptr(), total_k, dkv_heads, heads_k, d, dk.stride(0), dk.stride(1),
+                                                   dv.stride(0), dv.stride(1), _dt(q), _stream()))
+            else:  # a caller's tensors may have any strides and start anywhere
+                torch.sum(dk_e.view(total_k, heads_k, grp, d), dim=2, out=dk)
+                torch.sum(dv_e.view(total_k, heads_k, grp, d), dim=2, out=dv)
     return [dq, dk, dv, softmax_d]

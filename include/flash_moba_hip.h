@@ -292,8 +292,11 @@ int fmoba_attn_bwd(const fmoba_attn_bwd_args *a, void *stream);
 int fmoba_attn_bwd_phases(const fmoba_attn_bwd_args *a, int32_t phases, void *stream);
 /* The same with dk/dv (total_k, dkv_heads, d), each head the sum over heads / dkv_heads consecutive query heads, formed in
  * fp32; dkv_heads is a multiple of heads_k.  fmoba_attn_bwd_dkv_heads says how many are best (and possible) for a call; the
- * caller sums what is left of a group. */
+ * caller sums what is left of a group, for instance with fmoba_sum_grouped_heads (flash_moba_api.cpp:842-845): `apart` is
+ * (2, total_k, dkv_heads, head_dim), packed, dK then dV; strides of dk and dv in elements, multiples of 8. */
 int32_t fmoba_attn_bwd_dkv_heads(const fmoba_attn_bwd_args *a);
+int fmoba_sum_grouped_heads(const void *apart, void *dk, void *dv, int64_t total_k, int32_t dkv_heads, int32_t heads_k, int32_t head_dim, int64_t dk_row_stride,
+                            int64_t dk_head_stride, int64_t dv_row_stride, int64_t dv_head_stride, int32_t dtype, void *stream);
 int fmoba_attn_bwd_grouped(const fmoba_attn_bwd_args *a, int32_t dkv_heads, int32_t phases, void *stream);
 /* The same over the lists and visits of fmoba_pool_and_gate_ranked, as fmoba_attn_fwd_ranked. */
 int fmoba_attn_bwd_ranked(const fmoba_attn_bwd_args *a, const uint32_t *visits, int32_t dkv_heads, int32_t phases, void *stream);
