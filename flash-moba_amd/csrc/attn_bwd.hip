@@ -1635,7 +1635,8 @@ __global__ __launch_bounds__(64 * NW, HD > 64 ? 2 : 4) void attn_bwd_dq_kernel(f
 // dQ, second form: the row's partials are added in ascending key-block order (sorted by block id: the slot a visit
 // got is arbitrary, the sum must not depend on it) and scaled.  One 16-lane group per (row, head), four per wave,
 // sixteen per block of 256: a row's chain of dependent steps (count, ids, order, rows) is mostly waiting, so a wave
-// runs four of them side by side.  Lane li of a group owns the 16-byte piece li of the row.
+// runs four of them side by side.  Lane li of a group owns the 16-byte piece li of the row.  Over ranked lists the first rows are asked for beside the count; the next four
+// are on their way while four are added (figures: attn_fwd_combine_kernel).
 // ------------------------------------------------------------------------------------
 template <typename T, bool RANKED>
 __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd_args a, BwdWs ws, int capl) {
@@ -1650,16 +1651,26 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
   const int64_t row = rh / a.heads;
   const int h = (int)(rh - row * a.heads);
   const int D = a.head_dim;
+  const int c8 = li * 8;
+  const bool mine = c8 < D;
+  const int PD = part_row_elems(D, 2);
+  const uint16_t *part = ws.part + rh * ws.cap * PD;
+  // rows t .. of the row's order, as far as there are `have` of them
+  auto fetch = [&](Pack8(&x)[4], int t, int have) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (t + u >= have) break;
+      x[u] = ld_stream16(part + (int64_t)(RANKED ? t + u : sOrd[t + u]) * PD + c8);
+    }
+  };
+  Pack8 x[4];
+  if (RANKED && mine) fetch(x, 0, ws.cap);  // asked for beside the count: what lies behind it is not used
   const int nall = !valid ? 0 : RANKED ? (int)(ws.visits[(int64_t)h * a.total_q + row] >> 16) : ws.cnt[rh];
   const int n = min(nall, ws.cap);
   if (nall > ws.cap && li == 0 && a.visits_overflow != nullptr) atomicMax(a.visits_overflow, nall);  // visits were dropped
   int nmax = max(n, __shfl_xor(n, 16, 64));
   nmax = max(nmax, __shfl_xor(nmax, 32, 64));  // the wave walks the longest of its four rows
-  const int c8 = li * 8;
-  const bool mine = c8 < D;
   const int32_t *pid = ws.pid + rh * ws.cap;
-  const int PD = part_row_elems(D, 2);
-  const uint16_t *part = ws.part + rh * ws.cap * PD;
   float acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
@@ -1673,15 +1684,16 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
         acc[2 * k + 1] += elem_to_float<T>((uint16_t)(x.w[k] >> 16));
       }
     };
-    int t = 0;
-    for (; t + 4 <= n; t += 4) {  // independent loads, four in flight
-      Pack8 x[4];
+    if (!RANKED && n > 0) fetch(x, 0, n);
+    for (int t = 0; t < n; t += 4) {  // the next rows are on their way while these are added
+      Pack8 nx[4];
+      if (t + 4 < n) fetch(nx, t + 4, n);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) x[u] = ld_stream16(part + (int64_t)(RANKED ? t + u : sOrd[t + u]) * PD + c8);
+      for (int u = 0; u < 4; ++u)
+        if (t + u < n) add(x[u]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) add(x[u]);
+      for (int u = 0; u < 4; ++u) x[u] = nx[u];
     }
-    for (; t < n; ++t) add(ld_stream16(part + (int64_t)(RANKED ? t : sOrd[t]) * PD + c8));
   }
   if (valid && mine) {
     const float scale = dq_sum_scale<T>(a.softmax_scale);
