@@ -1706,8 +1706,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
 
 // grid (ceil(max_seqlen_q / rows_per_block), heads, batch), block 256.
 // LPR = 2^lg_lpr lanes cooperate on one row (LPR >= head_dim / 8).
-constexpr int kPrepRows = 4;  // rows per thread: eight 16-byte loads in flight (with one row a thread had two, 4.7 TB/s)
-template <typename T>
+constexpr int kPrepRows = 4;  // consecutive rows per thread: eight 16-byte loads in flight, and the sums of a wave's rows leave in one store
+// Output rows that the caches cannot hold are read past them: reads alone reach 6.9 TB/s so, 5.5 through the caches.  24571 tokens, 32 heads of 128 (201 MB) 87 -> 76 us, 32768 tokens (the forward's
+// rows are still on their way to memory) 145 -> 131, 36427 tokens, 32 heads of 64 55 -> 46; 8191 tokens, 16 heads of 64 (17 MB) with it 9.1 -> 10.5.
+constexpr int64_t kPrepStreamBytes = (int64_t)64 << 20;
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int lg_lpr, int32_t *tab, RunTable rt, int row_mask, int ztab) {
   const int LPR = 1 << lg_lpr, rows_per_pass = 256 >> lg_lpr;
   // Uneven batches have up to millions of blocks past their sequence's end, each of which lives as long as its chain of loads: they leave
@@ -1764,23 +1767,24 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
       for (int i = threadIdx.x; i < q0; i += 256) dh[i] = 0.f;
   }
   if (first >= Lq) return;
-  const int r0 = first + (threadIdx.x >> lg_lpr), sub = threadIdx.x & (LPR - 1);
+  const int r0 = first + (threadIdx.x >> lg_lpr) * kPrepRows, sub = threadIdx.x & (LPR - 1);
   const int e = sub * 8;
   const int D = a.head_dim;
   Pack8 o[kPrepRows], g[kPrepRows];
 #pragma unroll
   for (int k = 0; k < kPrepRows; ++k) {
-    const int r = r0 + k * rows_per_pass;
+    const int r = r0 + k;
     o[k] = zero_pack8();
     g[k] = zero_pack8();
     if (r < Lq && e < D) {
-      o[k] = ld_global16(reinterpret_cast<const uint16_t *>(a.out) + (int64_t)(q0 + r) * a.o_row_stride + (int64_t)h * a.o_head_stride + e);
+      const uint16_t *from = reinterpret_cast<const uint16_t *>(a.out) + (int64_t)(q0 + r) * a.o_row_stride + (int64_t)h * a.o_head_stride + e;
+      o[k] = STREAM ? ld_stream16(from) : ld_global16(from);
       g[k] = ld_global16(reinterpret_cast<const uint16_t *>(a.dout) + (int64_t)(q0 + r) * a.do_row_stride + (int64_t)h * a.do_head_stride + e);
     }
   }
+  float sum[kPrepRows];
 #pragma unroll
   for (int k = 0; k < kPrepRows; ++k) {
-    const int r = r0 + k * rows_per_pass;
     float fo[8], fg[8];
     unpack8<T>(o[k], fo);
     unpack8<T>(g[k], fg);
@@ -1788,7 +1792,18 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc = fmaf(fo[i], fg[i], acc);
     for (int w = LPR >> 1; w >= 1; w >>= 1) acc += __shfl_xor(acc, w, 64);
-    if (r < Lq && sub == 0) a.softmax_d[(int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b + r] = acc;
+    sum[k] = acc;
+  }
+  float *to = a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b + r0;
+  if (LPR >= kPrepRows) {  // the wave's rows side by side
+    float mine = sum[0];
+#pragma unroll
+    for (int k = 1; k < kPrepRows; ++k) mine = sub == k ? sum[k] : mine;
+    if (sub < kPrepRows && r0 + sub < Lq) to[sub] = mine;
+  } else if (sub == 0) {
+#pragma unroll
+    for (int k = 0; k < kPrepRows; ++k)
+      if (r0 + k < Lq) to[k] = sum[k];
   }
 }
 
@@ -1954,11 +1969,12 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
     const int nx = ceil_div(a.max_seqlen_q, (256 >> lg_lpr) * kPrepRows);
     const RunTable rt = bwd_run_table(a);
     const int ztab = partials ? 0 : (int)ceil_div64(ceil_div(rt.cols, 4), nx);
+    auto prep = (int64_t)a.total_q * a.heads * a.head_dim * 2 >= kPrepStreamBytes ? bwd_prep_kernel<T, true> : bwd_prep_kernel<T, false>;
     if (a.batch + ztab <= 65535) {
-      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, ztab);
+      hipLaunchKernelGGL(prep, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, ztab);
     } else {  // (more planes than a launch has)
-      if (ztab > 0) hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(ceil_div(rt.cols, 4), a.heads, 1), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, 1);
-      hipLaunchKernelGGL(bwd_prep_kernel<T>, dim3(nx, a.heads, a.batch), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, 0);
+      if (ztab > 0) hipLaunchKernelGGL(prep, dim3(ceil_div(rt.cols, 4), a.heads, 1), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, 1);
+      hipLaunchKernelGGL(prep, dim3(nx, a.heads, a.batch), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, 0);
     }
   }
   if (a.head_dim > 128) {
