@@ -24,10 +24,14 @@ struct PoolExtra {
 // one request of 3000 keys 21.3 -> 16.6, of 60000 48.5 -> 36.5; 20 of 256 to 65536, 32 over 32 heads 740 -> 694.  Heads of 256 too, though the query rows leave
 // three waves per SIMD of eight: one request of 60000 keys, 8 heads 81.9 -> 62.4, eight of 1000 to 30000, 32 over 4 heads 61.4 -> 56.2, 32 of 512 to 32768, 32
 // heads 907 -> 878.
+// Keys that the chip's last cache (256 MB) cannot hold until the attention comes to them are read past the caches: one sequence of 32768 keys, 32 heads of 128 (268 MB) 67.7 -> 44.6 us,
+// 262144 keys, 16 heads 241 -> 195, decode of 16 requests with 8 key heads (380 MB) 60.1 -> 57.4.  Keys that it holds are read again from there: 67485 keys, 16 heads of 96 (207 MB)
+// 40.7 us, past the caches 44.6, and the decode step after it 30.6 and 35.7.
+constexpr int64_t kPoolStreamBytes = (int64_t)256 << 20;
 template <typename T, bool MANY, int HD>
 __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x, FewGate few) {
   const int c = blockIdx.x, b = blockIdx.y;
-  const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1];
+  const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1], total_k = a.cu_seqlens_k[a.batch];
   const int row0 = seq_start + c * a.chunk;
   if (x.clear_vec16) {
     const int64_t nthr = (int64_t)gridDim.x * gridDim.y * gridDim.z * 256;
@@ -71,48 +75,55 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
   if (active) {
     const uint16_t *base = reinterpret_cast<const uint16_t *>(a.k) + (int64_t)head * a.k_head_stride + d0;
-    int r = wave;  // row of the chunk
-    // Sixteen independent 16-byte loads in flight per lane, added up in the order of the loop of four below: with four, a chunk of 256 rows is
-    // sixteen memory latencies one after the other.  For rows of up to 2 KB (forward of 3334 tokens, 8 heads, 256-key chunks 65.8 -> 62.0 us, decode of
-    // 43 sequences of up to 59161 keys, 2 key heads of 64 102.9 -> 95.5, of 16 sequences, 8 key heads of 128 119.2 -> 118.6, 3072 tokens, 8 heads of 64, 128-key
-    // chunks 34.2 -> 33.5); wider rows read fewer pages of memory at a time with four (decode of 8 sequences of 30000 keys, 32 key heads, 256-key
-    // chunks 370 us, 392 with sixteen), and chunks of 64 rows gain nothing.
-    for (; MANY && r + 60 < n; r += 64) {
-      Pack8 p[16];
+    auto sum_rows = [&](auto stream) {
+      auto load = [](const uint16_t *p) { return decltype(stream)::value ? ld_stream16(p) : ld_global16(p); };
+      int r = wave;  // row of the chunk
+      // Sixteen independent 16-byte loads in flight per lane, added up in the order of the loop of four below: with four, a chunk of 256 rows is
+      // sixteen memory latencies one after the other.  For rows of up to 2 KB (forward of 3334 tokens, 8 heads, 256-key chunks 65.8 -> 62.0 us, decode of
+      // 43 sequences of up to 59161 keys, 2 key heads of 64 102.9 -> 95.5, of 16 sequences, 8 key heads of 128 119.2 -> 118.6, 3072 tokens, 8 heads of 64, 128-key
+      // chunks 34.2 -> 33.5); wider rows read fewer pages of memory at a time with four (decode of 8 sequences of 30000 keys, 32 key heads, 256-key
+      // chunks 370 us, 392 with sixteen), and chunks of 64 rows gain nothing.
+      for (; MANY && r + 60 < n; r += 64) {
+        Pack8 p[16];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) p[j] = ld_global16(base + (int64_t)(row0 + r + 4 * j) * a.k_row_stride);
+        for (int j = 0; j < 16; ++j) p[j] = load(base + (int64_t)(row0 + r + 4 * j) * a.k_row_stride);
 #pragma unroll
-      for (int j = 0; j < 16; j += 4) {
+        for (int j = 0; j < 16; j += 4) {
+          float f0[8], f1[8], f2[8], f3[8];
+          unpack8<T>(p[j], f0);
+          unpack8<T>(p[j + 1], f1);
+          unpack8<T>(p[j + 2], f2);
+          unpack8<T>(p[j + 3], f3);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc[i] += (f0[i] + f1[i]) + (f2[i] + f3[i]);
+        }
+      }
+      // four in flight
+      for (; r + 12 < n; r += 16) {
+        Pack8 p0 = load(base + (int64_t)(row0 + r) * a.k_row_stride);
+        Pack8 p1 = load(base + (int64_t)(row0 + r + 4) * a.k_row_stride);
+        Pack8 p2 = load(base + (int64_t)(row0 + r + 8) * a.k_row_stride);
+        Pack8 p3 = load(base + (int64_t)(row0 + r + 12) * a.k_row_stride);
         float f0[8], f1[8], f2[8], f3[8];
-        unpack8<T>(p[j], f0);
-        unpack8<T>(p[j + 1], f1);
-        unpack8<T>(p[j + 2], f2);
-        unpack8<T>(p[j + 3], f3);
+        unpack8<T>(p0, f0);
+        unpack8<T>(p1, f1);
+        unpack8<T>(p2, f2);
+        unpack8<T>(p3, f3);
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[i] += (f0[i] + f1[i]) + (f2[i] + f3[i]);
       }
-    }
-    // four in flight
-    for (; r + 12 < n; r += 16) {
-      Pack8 p0 = ld_global16(base + (int64_t)(row0 + r) * a.k_row_stride);
-      Pack8 p1 = ld_global16(base + (int64_t)(row0 + r + 4) * a.k_row_stride);
-      Pack8 p2 = ld_global16(base + (int64_t)(row0 + r + 8) * a.k_row_stride);
-      Pack8 p3 = ld_global16(base + (int64_t)(row0 + r + 12) * a.k_row_stride);
-      float f0[8], f1[8], f2[8], f3[8];
-      unpack8<T>(p0, f0);
-      unpack8<T>(p1, f1);
-      unpack8<T>(p2, f2);
-      unpack8<T>(p3, f3);
+      for (; r < n; r += 4) {
+        Pack8 p0 = load(base + (int64_t)(row0 + r) * a.k_row_stride);
+        float f0[8];
+        unpack8<T>(p0, f0);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] += (f0[i] + f1[i]) + (f2[i] + f3[i]);
-    }
-    for (; r < n; r += 4) {
-      Pack8 p0 = ld_global16(base + (int64_t)(row0 + r) * a.k_row_stride);
-      float f0[8];
-      unpack8<T>(p0, f0);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] += f0[i];
-    }
+        for (int i = 0; i < 8; ++i) acc[i] += f0[i];
+      }
+    };
+    if ((int64_t)total_k * nvec * 16 >= kPoolStreamBytes)
+      sum_rows(std::true_type{});
+    else
+      sum_rows(std::false_type{});
   }
   // the query rows of this wave's first key head: on their way during the reduction
   constexpr int KS = HD > 0 ? HD / 16 : 1;
