@@ -1636,7 +1636,8 @@ __global__ __launch_bounds__(64 * NW, HD > 64 ? 2 : 4) void attn_bwd_dq_kernel(f
 // got is arbitrary, the sum must not depend on it) and scaled.  One 16-lane group per (row, head), four per wave,
 // sixteen per block of 256: a row's chain of dependent steps (count, ids, order, rows) is mostly waiting, so a wave
 // runs four of them side by side.  Lane li of a group owns the 16-byte piece li of the row.  Over ranked lists the first rows are asked for beside the count; the next four
-// are on their way while four are added (figures: attn_fwd_combine_kernel).
+// are on their way while four are added (36427 tokens, 32 heads of 64, top-k 4, training step 1408 -> 1359 us; 25298 tokens, 32 heads of 80, top-k 2 1344 -> 1297; plain lists,
+// 82354 tokens, 16 heads of 64, top-k 4, pass alone 268 -> 251; 16 visits as before).
 // ------------------------------------------------------------------------------------
 template <typename T, bool RANKED>
 __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd_args a, BwdWs ws, int capl) {

@@ -428,11 +428,11 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
 // headers, order, rows) is mostly waiting, so a wave runs four of them side by side.  Lane li of a group owns the
 // 16-byte pieces li, li + 16, .. (NP of them) of the row, whose elements are of type E
 // (NORM: divided by the visit's sum of probabilities).
-// RANKED: the slots are in key-block order and none of the first `visits` is empty.  The headers and the first rows are asked for beside the count, and the next U rows are on
-// their way while U are added: a row of few visits, or of a number that U does not divide, was a chain of loads (36427 tokens, 32 heads of 64, top-k 4 of 64-key chunks, training step
-// with both combines 1408 -> 1359 us; 25298 tokens, 32 heads of 80, top-k 2 1344 -> 1297; 8192 tokens, 16 heads of 128, forward 199.4 -> 196.4; rows of 16 visits as before).  What bounds rows of
-// many visits is the memory: their reads alone, by this pattern, reach 7.1 TB/s, with the output rows written between them (a sixteenth of the bytes) 5.7.
-// (Loads past a row's last visit, instead of none: 12200 -> 12300 us where rows have 17.)
+// RANKED: the slots are in key-block order and none of the first `visits` is empty.  The headers and the first rows are asked for beside the count, and what U does not divide
+// together: a row of few visits was a chain of loads (16-bit rows, pass alone: 8192 tokens, 16 heads of 128, top-k 8 52.4 -> 50.6 us; parts of prompts 39.8 -> 37.5; 5312 tokens, top-k 7
+// 32.8 -> 30.4; 16 and 22 visits as before, 790 and 750).  What bounds rows of many visits is the memory: their reads alone, by this pattern, reach 7.1 TB/s, with the output rows
+// written between them (a sixteenth of the bytes) 5.7.  The next rows on their way while rows are added: 22 visits 750 -> 820, for the registers.  Over plain lists the rows' places come from LDS, and whole
+// groups of U stay free of branches (219 us, else 230).
 template <typename T, typename E, int NP, bool NORM, bool RANKED>
 __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_args a, FwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
@@ -468,12 +468,15 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   // and the partials are merged in rank order, 16 at a time.
   if constexpr (!RANKED) group_rank_order(reinterpret_cast<const int *>(hdr) + 2, 4, n, nmax, sOrd, lane);
   // rows i0 .. of the row's order, as far as there are `have` of them
-  constexpr int U = NP == 1 ? 4 : 2;
-  auto fetch = [&](Pack8(&x)[U][NP], int i0, int have) {
+  constexpr int U = 4;
+  auto fetch = [&](auto all, Pack8(&x)[U][NP], int i0, int have) {
+    int slot[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) slot[u] = RANKED ? i0 + u : sOrd[i0 + u];  // (the list's length is a multiple of sixteen)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (i0 + u >= have) break;
-      const E *from = part + (int64_t)(RANKED ? i0 + u : sOrd[i0 + u]) * PD + c0;
+      if (!decltype(all)::value && i0 + u >= have) break;
+      const E *from = part + (int64_t)slot[u] * PD + c0;
 #pragma unroll
       for (int p = 0; p < NP; ++p) x[u][p] = ld_stream16(c0 + p * 16 * PE < D ? from + p * 16 * PE : from);
     }
@@ -482,15 +485,15 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   float2 head = {-INFINITY, 0.f};
   if constexpr (RANKED) {  // asked for beside the count: what lies behind it is not used
     if (li < ws.cap) head = hdr2[li];
-    if (mine) fetch(x, 0, ws.cap);
+    if (mine) fetch(std::false_type{}, x, 0, ws.cap);
   }
   for (int base = 0; base < nmax; base += 16) {
     const int cntb = min(16, max(n - base, 0));
     float mj = -INFINITY, lj = 0.f;
     if (li < cntb) {
       if constexpr (RANKED) {
-        if (base > 0) head = hdr2[base + li];
         mj = head.x, lj = head.y;
+        if (base + 16 + li < n) head = hdr2[base + 16 + li];
       } else {
         const float4 hd = hdr[sOrd[base + li]];
         mj = hd.x, lj = hd.y;
@@ -529,17 +532,19 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
             }
           }
       };
-      if (!RANKED && base == 0 && cntb > 0) fetch(x, 0, n);
-      for (int t = 0; t < cntb; t += U) {  // the next rows are on their way while these are added
-        Pack8 nx[U][NP];
-        if (base + t + U < n) fetch(nx, base + t + U, n);
+      int t = 0;
+      if constexpr (!RANKED) {
+        for (; t + U <= cntb; t += U) {
+          fetch(std::true_type{}, x, base + t, n);
+#pragma unroll
+          for (int u = 0; u < U; ++u) add(x[u], sWgt[sg][t + u]);
+        }
+      }
+      for (; t < cntb; t += U) {
+        if (!RANKED || base + t > 0) fetch(std::false_type{}, x, base + t, n);
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if (t + u < cntb) add(x[u], sWgt[sg][t + u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int p = 0; p < NP; ++p) x[u][p] = nx[u][p];
       }
     }
   }
