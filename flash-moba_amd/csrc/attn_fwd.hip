@@ -431,8 +431,8 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
 // RANKED: the slots are in key-block order and none of the first `visits` is empty.  The headers and the first rows are asked for beside the count, and what U does not divide
 // together: a row of few visits was a chain of loads (16-bit rows, pass alone: 8192 tokens, 16 heads of 128, top-k 8 52.4 -> 50.6 us; parts of prompts 39.8 -> 37.5; 5312 tokens, top-k 7
 // 32.8 -> 30.4; 16 and 22 visits as before, 790 and 750).  What bounds rows of many visits is the memory: their reads alone, by this pattern, reach 7.1 TB/s, with the output rows
-// written between them (a sixteenth of the bytes) 5.7.  The next rows on their way while rows are added: 22 visits 750 -> 820, for the registers.  Over plain lists the rows' places come from LDS, and whole
-// groups of U stay free of branches (219 us, else 230).
+// written between them (a sixteenth of the bytes) 5.7.  The next rows on their way while rows are added: 22 visits 750 -> 820, for the registers.  Over plain lists the rows' places come from LDS: nothing is early, and whole
+// groups of U and single rows take 60 us where groups with branches take 67 (12182 tokens, 16 heads of 64, top-k 4).
 template <typename T, typename E, int NP, bool NORM, bool RANKED>
 __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_args a, FwdWs ws, int capl) {
   extern __shared__ __attribute__((aligned(16))) int sOrdAll[];  // [16 groups][capl]: slot of the partial of rank r
@@ -467,25 +467,25 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
   // its rank in ascending key-block order over the WHOLE row (equal ids, a malformed pattern, are ordered by slot),
   // and the partials are merged in rank order, 16 at a time.
   if constexpr (!RANKED) group_rank_order(reinterpret_cast<const int *>(hdr) + 2, 4, n, nmax, sOrd, lane);
-  // rows i0 .. of the row's order, as far as there are `have` of them
-  constexpr int U = 4;
-  auto fetch = [&](auto all, Pack8(&x)[U][NP], int i0, int have) {
-    int slot[U];
+  auto load = [&](Pack8(&y)[NP], int slot) {
+    const E *from = part + (int64_t)slot * PD + c0;
 #pragma unroll
-    for (int u = 0; u < U; ++u) slot[u] = RANKED ? i0 + u : sOrd[i0 + u];  // (the list's length is a multiple of sixteen)
+    for (int p = 0; p < NP; ++p) y[p] = ld_stream16(c0 + p * 16 * PE < D ? from + p * 16 * PE : from);
+  };
+  // rows i0 .. of a ranked row, as far as there are `have` of them
+  constexpr int U = 4;
+  auto fetch = [&](Pack8(&y)[U][NP], int i0, int have) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (!decltype(all)::value && i0 + u >= have) break;
-      const E *from = part + (int64_t)slot[u] * PD + c0;
-#pragma unroll
-      for (int p = 0; p < NP; ++p) x[u][p] = ld_stream16(c0 + p * 16 * PE < D ? from + p * 16 * PE : from);
+      if (i0 + u >= have) break;
+      load(y[u], i0 + u);
     }
   };
-  Pack8 x[U][NP];
+  Pack8 x[U][NP];  // (of ranked rows)
   float2 head = {-INFINITY, 0.f};
   if constexpr (RANKED) {  // asked for beside the count: what lies behind it is not used
     if (li < ws.cap) head = hdr2[li];
-    if (mine) fetch(std::false_type{}, x, 0, ws.cap);
+    if (mine) fetch(x, 0, ws.cap);
   }
   for (int base = 0; base < nmax; base += 16) {
     const int cntb = min(16, max(n - base, 0));
@@ -532,19 +532,31 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
             }
           }
       };
-      int t = 0;
-      if constexpr (!RANKED) {
-        for (; t + U <= cntb; t += U) {
-          fetch(std::true_type{}, x, base + t, n);
+      if constexpr (RANKED) {
+        for (int t = 0; t < cntb; t += U) {
+          if (base + t > 0) fetch(x, base + t, n);
 #pragma unroll
-          for (int u = 0; u < U; ++u) add(x[u], sWgt[sg][t + u]);
+          for (int u = 0; u < U; ++u)
+            if (t + u < cntb) add(x[u], sWgt[sg][t + u]);
         }
-      }
-      for (; t < cntb; t += U) {
-        if (!RANKED || base + t > 0) fetch(std::false_type{}, x, base + t, n);
+      } else {
+        int t = 0;
+        for (; t + U <= cntb; t += U) {  // independent loads, four in flight
+          Pack8 y[U][NP];
+          float w[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (t + u < cntb) add(x[u], sWgt[sg][t + u]);
+          for (int u = 0; u < U; ++u) {
+            load(y[u], sOrd[base + t + u]);
+            w[u] = sWgt[sg][t + u];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) add(y[u], w[u]);
+        }
+        for (; t < cntb; ++t) {
+          Pack8 y[NP];
+          load(y, sOrd[base + t]);
+          add(y, sWgt[sg][t]);
+        }
       }
     }
   }
