@@ -607,6 +607,8 @@ __global__ __launch_bounds__(256) void csc_row_visits_kernel(fmoba_attn_fwd_args
 }
 // The same with the counts of a range of rows of one (sequence, head) in LDS: no atomics in memory, the maximum on the way out.  Every workgroup
 // reads all lists of the pair (in any order) and counts what falls into its rows; a wave takes 512 entries of two lists at a time.
+// Bound by the latency of those loads, which go out together, past a list's end from its last entry: each under a branch of its own with a wait (entries that exist alone
+// were asked for) took 90 us where this takes 30 (30039 tokens, 8 heads, top-k 14; 12182 tokens, 16 heads, top-k 4 27 -> 12).
 // grid (row ranges, heads, batch); `range` rows in LDS, `max_out` cleared before.
 __global__ __launch_bounds__(1024) void csc_row_visits_lds_kernel(fmoba_attn_fwd_args a, int32_t *cnt, int32_t *max_out, int kb, int range) {
   extern __shared__ int32_t visits[];
@@ -640,15 +642,17 @@ __global__ __launch_bounds__(1024) void csc_row_visits_lds_kernel(fmoba_attn_fwd
         for (int p = 0; p < max(n[0], n[1]); p += 512) {
           int r[2][8];
 #pragma unroll
-          for (int u = 0; u < 2; ++u)
+          for (int u = 0; u < 2; ++u) {
+            if (p >= n[u]) continue;  // (entries past a list's end are not read, not even where the list is empty)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) r[u][i] = p + i * 64 + lane < n[u] ? list[u][p + i * 64 + lane] - r0 : -1;
+            for (int i = 0; i < 8; ++i) r[u][i] = list[u][min(p + i * 64 + lane, n[u] - 1)];
+          }
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             const int add = blocks[u && two ? c + 1 : c];
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-              if ((uint32_t)r[u][i] < (uint32_t)rows) atomicAdd(&visits[r[u][i]], add);
+              if (p + i * 64 + lane < n[u] && (uint32_t)(r[u][i] - r0) < (uint32_t)rows) atomicAdd(&visits[r[u][i] - r0], add);
           }
         }
       }
@@ -842,12 +846,12 @@ static int fwd_check_common(const fmoba_attn_fwd_args *a) {
   return 0;
 }
 
-// Counts in LDS or by atomics in memory.  In LDS a workgroup reads all lists of its (sequence, head), some 2.4 entries per ns, so the longest sequence is the
+// Counts in LDS or by atomics in memory.  In LDS a workgroup reads all lists of its (sequence, head), some 10 entries per ns, so the longest sequence is the
 // call; the whole chip does 27 atomics per ns, up to 60 where the counters of few heads lie close together.  So LDS where a call is worth
-// many heads of its longest sequence.  Atomics and LDS, us: 262144 tokens, top-k 16 of 128-key chunks, 8 heads 1219 and 1497, 16 heads 2530 and 1925;
-// 90000 tokens, top-k 8, 10 heads 279 and 285, 12 heads 336 and 295; sequences of 20000, top-k 16, 4 x 4 heads 146 and 136, 8 x 2 heads 115 and 135, 16 x 2
-// heads 206 and 142, 32 x 1 head 142 and 144; one sequence of 200000 with seven of 2048, 1 head 118 and 1086, 16 heads of 150000 with three of 2000 767
-// and 504.  And where the longest lists are so short that their reading takes less than the two more launches: 8 heads of 1000 tokens.
+// many heads of its longest sequence.  Atomics and LDS, us: 262144 tokens, top-k 16 of 128-key chunks, 1 head 141 and 408, 8 heads 1204 and 436;
+// 90000 tokens, top-k 8, 2 heads 55 and 85, 16 heads 446 and 94; 20000 tokens, 2 heads 16.5 and 19.5, 16 heads 106 and 25; sequences of 20000, 4 x 1 head 21.3 and 20.3, 16 x 2
+// heads 128 and 32; one of 200000 with seven of 2048, 1 head 59 and 186.  And where the longest lists are so short that their reading takes less than the two more launches: 8 heads of
+// 1000 tokens 8.3 and 7.3.  (The line is the one of a pass that read 2.4 entries per ns; LDS has since been the faster from four heads of the longest sequence on.)
 static bool csc_visits_in_lds(const fmoba_attn_fwd_args &a) {
   const int64_t longest = std::max(1, a.max_seqlen_q), alike = (int64_t)a.heads * a.total_q / longest;
   return alike >= std::max(12, 64 / a.heads) || (alike >= 8 && longest * a.max_cols <= 32768);
