@@ -963,7 +963,7 @@ int fwd_check_gated(const fmoba_attn_fwd_args *a) {
   return 0;
 }
 bool pool_scores_feasible(int head_dim, int group, int rows, int batch);                                       // mean_pool.hip
-int mean_pool_with_scores(const fmoba_mean_pool_args *a, const FewGate &few, void *stream);
+int mean_pool_with_scores(const fmoba_mean_pool_args *a, const FewGate &few, int64_t total_k, void *stream);
 void run_fwd_few_scored(const fmoba_attn_fwd_args &a, const FewGate &few, hipStream_t s);                      // attn_fwd_few.hip
 }  // namespace fmoba
 
@@ -995,7 +995,7 @@ extern "C" int fmoba_attn_fwd_gated_few(const fmoba_mean_pool_args *m, const fmo
   few.q = reinterpret_cast<const uint16_t *>(a->q), few.cu_seqlens_q = a->cu_seqlens_q, few.cu_seqlens_km = m->cu_seqlens_km, few.scores = scores;
   few.q_row_stride = a->q_row_stride, few.q_head_stride = a->q_head_stride;
   few.heads = a->heads, few.group = a->heads / a->heads_k, few.rows = a->max_seqlen_q, few.topk = topk, few.is_causal = gate_is_causal;
-  if (int rc = mean_pool_with_scores(m, few, stream)) return rc;
+  if (int rc = mean_pool_with_scores(m, few, a->total_k, stream)) return rc;
   run_fwd_few_scored(*a, few, (hipStream_t)stream);
   FMOBA_LAUNCH_CHECK("attn_fwd_gated_few");
   return 0;

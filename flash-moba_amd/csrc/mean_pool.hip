@@ -28,10 +28,18 @@ struct PoolExtra {
 // 262144 keys, 16 heads 241 -> 195, decode of 16 requests with 8 key heads (380 MB) 60.1 -> 57.4.  Keys that it holds are read again from there: 67485 keys, 16 heads of 96 (207 MB)
 // 40.7 us, past the caches 44.6, and the decode step after it 30.6 and 35.7.
 constexpr int64_t kPoolStreamBytes = (int64_t)256 << 20;
-template <typename T, bool MANY, int HD>
+// STREAM: known at the launch (a second loop in the scoring instances costs a short decode step 0.4 us); the others find out from the offsets.
+template <typename T, bool MANY, int HD, bool STREAM>
 __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x, FewGate few) {
   const int c = blockIdx.x, b = blockIdx.y;
-  const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1], total_k = a.cu_seqlens_k[a.batch];
+  const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1];
+  int total_k = 0;
+  if constexpr (HD == 0) {
+    total_k = a.cu_seqlens_k[a.batch];
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(total_k));  // awaited with the other two, not in front of the rows
+#endif
+  }
   const int row0 = seq_start + c * a.chunk;
   if (x.clear_vec16) {
     const int64_t nthr = (int64_t)gridDim.x * gridDim.y * gridDim.z * 256;
@@ -120,10 +128,14 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
         for (int i = 0; i < 8; ++i) acc[i] += f0[i];
       }
     };
-    if ((int64_t)total_k * nvec * 16 >= kPoolStreamBytes)
-      sum_rows(std::true_type{});
-    else
-      sum_rows(std::false_type{});
+    if constexpr (HD > 0) {
+      sum_rows(std::integral_constant<bool, STREAM>{});
+    } else {
+      if ((int64_t)total_k * nvec * 16 >= kPoolStreamBytes)
+        sum_rows(std::true_type{});
+      else
+        sum_rows(std::false_type{});
+    }
   }
   // the query rows of this wave's first key head: on their way during the reduction
   constexpr int KS = HD > 0 ? HD / 16 : 1;
@@ -214,7 +226,7 @@ extern "C" int fmoba_chunk_offsets(const int32_t *cu_seqlens, int32_t *cu_seqlen
 }
 
 // `extra`: cu_km and clear_* of PoolExtra.  `few`: scores in place of the means (km and its strides are not looked at)
-static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &extra, void *stream, const fmoba::FewGate *few = nullptr) {
+static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &extra, void *stream, const fmoba::FewGate *few = nullptr, int64_t total_k = 0) {
   using namespace fmoba;
   FMOBA_REQUIRE(a != nullptr, "mean_pool: null args");
   FMOBA_REQUIRE(a->dtype == FMOBA_DTYPE_F16 || a->dtype == FMOBA_DTYPE_BF16, "mean_pool: only fp16 and bf16 are supported");
@@ -241,10 +253,15 @@ static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &
   }
   auto pick = [&](auto t) {
     typedef decltype(t) T;
-    if (hd == 64) return many ? mean_pool_kernel<T, true, 64> : mean_pool_kernel<T, false, 64>;
-    if (hd == 128) return many ? mean_pool_kernel<T, true, 128> : mean_pool_kernel<T, false, 128>;
-    if (hd == 256) return many ? mean_pool_kernel<T, true, 256> : mean_pool_kernel<T, false, 256>;
-    return many ? mean_pool_kernel<T, true, 0> : mean_pool_kernel<T, false, 0>;
+    auto scoring = [&](auto hd_) {
+      constexpr int HD = decltype(hd_)::value;
+      if (total_k * nvec * 16 >= kPoolStreamBytes) return many ? mean_pool_kernel<T, true, HD, true> : mean_pool_kernel<T, false, HD, true>;
+      return many ? mean_pool_kernel<T, true, HD, false> : mean_pool_kernel<T, false, HD, false>;
+    };
+    if (hd == 64) return scoring(std::integral_constant<int, 64>{});
+    if (hd == 128) return scoring(std::integral_constant<int, 128>{});
+    if (hd == 256) return scoring(std::integral_constant<int, 256>{});
+    return many ? mean_pool_kernel<T, true, 0, false> : mean_pool_kernel<T, false, 0, false>;
   };
   hipLaunchKernelGGL(a->dtype == FMOBA_DTYPE_BF16 ? pick(bf16_t()) : pick(f16_t()), grid, dim3(256), 0, s, *a, extra, scored);
   FMOBA_LAUNCH_CHECK("mean_pool");
@@ -268,7 +285,7 @@ int mean_pool_with_offsets(const fmoba_mean_pool_args *a, int32_t *clear, int64_
 
 // Whether the pooling pass can score the rows of a call: a product has 32 columns.
 bool pool_scores_feasible(int head_dim, int group, int rows, int batch) { return head_dim <= 256 && group * rows <= 32 && batch <= kPoolOffsetsBatch; }
-int mean_pool_with_scores(const fmoba_mean_pool_args *a, const FewGate &few, void *stream) {
-  return mean_pool_run(a, PoolExtra{const_cast<int32_t *>(a->cu_seqlens_km), nullptr, 0}, stream, &few);
+int mean_pool_with_scores(const fmoba_mean_pool_args *a, const FewGate &few, int64_t total_k, void *stream) {
+  return mean_pool_run(a, PoolExtra{const_cast<int32_t *>(a->cu_seqlens_km), nullptr, 0}, stream, &few, total_k);
 }
 }  // namespace fmoba
