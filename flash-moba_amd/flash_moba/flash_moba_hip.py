@@ -659,7 +659,8 @@ def moba_varlen_bwd(dout, q, k, v, out, softmax_lse, dq_, dk_, dv_, moba_col_off
             _phases(lambda mask: _check(lib.fmoba_attn_bwd_ranked(ctypes.byref(a), row_visits, dkv_heads, mask, _stream())))
         if dkv_heads != heads_k:
             grp = dkv_heads // heads_k
-            if all(given is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for given, t in ((dk_, dk), (dv_, dv))):
+            # (a packed tensor may have any stride where it has one row or one head)
+            if all(given is None or (t.is_contiguous() and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0) for given, t in ((dk_, dk), (dv_, dv))):
                 _check(lib.fmoba_sum_grouped_heads(apart.data_ptr(), dk.data_ptr(), dv.data_ptr(), total_k, dkv_heads, heads_k, d, dk.stride(0), dk.stride(1),
                                                    dv.stride(0), dv.stride(1), _dt(q), _stream()))
             else:  # a caller's tensors may have any strides and start anywhere
