@@ -892,21 +892,19 @@ static int rows_sets(const fmoba_attn_fwd_args &a) {
 }
 // Two sets of waves whose tiles are shared by two waves each, which take a half of their keys (eight waves, the loads and the rings of four): half of a turn's arithmetic in front of a
 // barrier.  Above head dimension 64, where the rings of two sets leave a unit room for one workgroup anyway, from sequences of 1024 keys on (shorter walks lose
-// in the sums what they gain: heads of 128, two sequences of 128 tokens 13.9 -> 14.9 us, four of 512 19.7 -> 20.0): 2048 tokens, 8 heads of 128 36.9 -> 34.1, 16 heads 49.3 -> 47.4,
-// 4096 tokens, 8 heads 73.8 -> 67.8, 3495 tokens, 8 heads of 96 56.5 -> 52.5.  Up to 64, where two workgroups of four waves fit a unit, for the calls that four sets are
-// too many for, up to half as many workgroups again as there are units and their items longest first: 1024 + 2048 tokens, 8 heads (384) 28.2 -> 26.9, 1120 tokens, 16 heads (288) 21.3 ->
-// 20.3, 4096 tokens, 8 heads (512) 46.0 -> 50.7, 6 heads (384, pair by pair) 53.7 -> 59.7.
-constexpr int kRowsHalves = 400;  // (counted with a block more per sequence)
-static bool rows_halves(const fmoba_attn_fwd_args &a) {
-  if (a.max_seqlen_k < kRowsFourSetsKeys) return false;
-  return a.head_dim > 64 || (a.heads * a.batch % 8 == 0 && a.heads * (((int64_t)a.total_q + 63 * a.batch) / 64) <= kRowsHalves);
-}
+// in the sums what they gain: heads of 128, two sequences of 128 tokens 13.9 -> 14.9 us, four of 512 19.7 -> 20.0).  The pass alone: 2048 tokens, 8 heads of 128 33.8 -> 32.1 us, not causal 33.9 ->
+// 31.3, 16 heads 45.4 -> 43.9, 4096 tokens, 8 heads 75.1 -> 70.3, 3495 tokens, 8 heads of 96 45.3 -> 41.3, 3 x 1024 tokens, 8 heads of 128 28.3 -> 28.6, not causal 38.0 -> 36.2.
+// Not up to 64, where two workgroups of four waves fit a unit and one of eight does: in calls of 257 to 400 workgroups 2 x 1536 tokens, 8 heads 21.8 -> 23.9, 3 x 1024 17.2 -> 21.1, not causal
+// 1024 + 2048 tokens 29.9 -> 39.6, 1100 tokens, 16 heads 20.1 -> 27.5; causal 1100 tokens, 16 heads 17.5 -> 17.0, 1024 + 2048, 8 heads 24.3 -> 23.9.
+static bool rows_halves(const fmoba_attn_fwd_args &a) { return a.head_dim > 64 && a.max_seqlen_k >= kRowsFourSetsKeys; }
 template <typename T, int HD>
 static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s, const RowGate *gate = nullptr) {
   const int sets = rows_sets(a);
   if constexpr (HD <= 64)
     if (sets == 4) return launch_rows_split<T, HD, 2, 4, 1>(a, bm, nw, gate, s);
-  if (sets == 2) return rows_halves(a) ? launch_rows_split<T, HD, 2, 2, 2>(a, bm, nw, gate, s) : launch_rows_split<T, HD, 2, 2, 1>(a, bm, nw, gate, s);
+  if constexpr (HD > 64)
+    if (sets == 2 && rows_halves(a)) return launch_rows_split<T, HD, 2, 2, 2>(a, bm, nw, gate, s);
+  if (sets == 2) return launch_rows_split<T, HD, 2, 2, 1>(a, bm, nw, gate, s);
   if constexpr (HD <= 64)
     if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1, 1>(a, bm, nw, gate, s);
   return launch_rows_split<T, HD, 4, 1, 1>(a, bm, nw, gate, s);
@@ -1012,3 +1010,4 @@ int run_fwd_rows(const fmoba_attn_fwd_args &a, int phases, hipStream_t s) {
 }  // namespace fmoba
 
 extern "C" int32_t fmoba_attn_fwd_row_sets(const fmoba_attn_fwd_args *a) { return a != nullptr && a->head_dim > 0 && a->head_dim <= 128 && fmoba::fwd_rows_direct(*a) ? fmoba::rows_sets(*a) : 1; }
+extern "C" int32_t fmoba_attn_fwd_key_halves(const fmoba_attn_fwd_args *a) { return fmoba_attn_fwd_row_sets(a) == 2 && fmoba::rows_halves(*a) ? 1 : 0; }

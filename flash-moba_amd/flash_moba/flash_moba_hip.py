@@ -103,6 +103,7 @@ EXPORTS = {
     "fmoba_attn_fwd_workspace_bytes": (c_sz, [ctypes.POINTER(AttnFwdArgs)]),
     "fmoba_attn_fwd_uses_row_blocks": (c_i32, [ctypes.POINTER(AttnFwdArgs)]),
     "fmoba_attn_fwd_row_sets": (c_i32, [ctypes.POINTER(AttnFwdArgs)]),
+    "fmoba_attn_fwd_key_halves": (c_i32, [ctypes.POINTER(AttnFwdArgs)]),
     "fmoba_csc_row_visits_in_lds": (c_i32, [ctypes.POINTER(AttnFwdArgs)]),
     "fmoba_csc_max_row_visits": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp, c_vp, c_vp]),
     "fmoba_attn_fwd": (c_i32, [ctypes.POINTER(AttnFwdArgs), c_vp]),

@@ -196,6 +196,8 @@ size_t fmoba_attn_fwd_workspace_bytes(const fmoba_attn_fwd_args *a);
 int32_t fmoba_attn_fwd_uses_row_blocks(const fmoba_attn_fwd_args *a);
 /* In the row-block form, of more than a handful of rows: the sets of waves that share a walk (1, 2 or 4; the same fields are read). */
 int32_t fmoba_attn_fwd_row_sets(const fmoba_attn_fwd_args *a);
+/* 1 if two waves of those sets share a tile, half of its keys each (the same fields are read). */
+int32_t fmoba_attn_fwd_key_halves(const fmoba_attn_fwd_args *a);
 /* counts (total_q * heads) int32 and max_out (1) int32 are device outputs: visits per (row, head) and
  * their maximum for the pattern in `a` (q/k/v/out/workspace of `a` are not read).  No counterpart in the
  * reference, whose row-wise scratch needs no bound. */
