@@ -81,15 +81,18 @@ __device__ __forceinline__ uint32_t shift_in_flag(uint32_t w, unsigned long long
 #endif
 }
 
-// Up to this many chunks a row's cut is found by taking its best scores off one by one (two and a half instructions per score and chunk), beyond by bisection
-// (about ten passes of two): both are bound by vector instructions.  Gate of 8192 tokens, 16 heads, up to 64 chunks, bisection and this: top-k 3 16.3 -> 12.2 us, 5 16.3 -> 13.1, 8 16.8 -> 14.5,
-// 11 16.5 -> 15.4, 13 16.8 -> 16.3, 17 15.6 -> 16.1, 25 15.1 -> 18.5; 4096 tokens top-k 3 11.3 -> 8.2, 11 11.9 -> 11.1, 17 11.9 -> 12.5.
+// Up to this many winners a row's cut is found by taking its best scores off one by one (two and a half instructions per score and winner), beyond by bisection
+// (about ten passes of two): both are bound by vector instructions.  Gate of 16 heads, bisection and this: 8192 tokens, 64 chunks, heads of 64 3 winners 14.3 -> 10.6 us, 8 14.2 -> 12.1,
+// 10 14.1 -> 13.6, 12 14.7 -> 15.4, heads of 128 8 16.3 -> 13.9, 10 16.4 -> 15.0, 12 17.7 -> 18.1; 12800 tokens, 100 chunks, heads of 64 8 23.0 -> 19.9, 10 23.6 -> 21.5, 12 23.7 -> 23.9,
+// heads of 128 8 28.6 -> 25.2, 10 30.7 -> 30.2, heads of 256 8 48.2 -> 43.9, 10 48.3 -> 45.3.
 constexpr int kGatePeels = 10;
 // The wave's 32 rows, lane (row l % 32): qf holds the row's slices as the B operand, the chunk means lie in the LDS tile from ldsTile on (rows of HD elements, piece c
 // of row r at c ^ tile_swz<HD>(r)), n_tiles * 32 of them.  The row's candidates are the chunks [0, nc); it keeps the best kp and its own chunk (own; below 0: none).
 // emit(t, w): word t of the row's selection, t < words, the same in both halves of the wave.
-// PEEL: as the row-block forward does it where several sets of waves wait for the choice (1024 + 2048 tokens, 8 heads of 64, call 30.4 -> 28.6 us), and the gate's own launch; in the workgroups
-// of one set, which overlap each other's choices, the second search of the cut only made the code longer (8191 tokens of short documents 123.6 -> 124.7 us).
+// PEEL: the best scores are taken off one by one, up to kGatePeels of them: the gate's own launch (an instance without serves more winners: with both searches it took 0.2 to 0.9 us of 13 to 35
+// more), and the row-block forward where several sets of waves wait for the choice (1024 + 2048 tokens, 8 heads of 64, call 30.4 -> 28.6 us).  In the workgroups of one set, which overlap each
+// other's choices, the second search of the cut only made the code longer (8191 tokens of short documents 123.6 -> 124.7 us).  One chain of comparisons: four side by side are no faster where
+// a wave has its SIMD to itself (1024 + 2048 tokens, 8 heads of 64 24.4 us either way) and cost the gate's launch 12.1 -> 12.8 (64 chunks, heads of 64, 8 winners), 13.9 -> 14.8 (of 128).
 template <typename T, int HD, int NT, bool PEEL, typename Emit>
 __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[HD / 16], int lane, int n_tiles, int nc, int kp, int own, bool valid, int words, const Emit &emit) {
   constexpr int KS = HD / 16, RB = HD * 2;
@@ -97,11 +100,7 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
   // scores: lane (query l%32) gets chunk t*32 + acc_row(i, hh) in register i of tile t;
   // chunks that are not candidates of the row hold -inf
   float sc[NT][16];
-  // (Chains of dependent instructions take twice as long as independent ones where a wave has its SIMD to itself: four side by side, as far as registers last.)
-  constexpr int NCH = NT <= 2 ? 4 : 1;
-  float vmins[NCH], vmaxs[NCH];
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) vmins[j] = INFINITY, vmaxs[j] = -INFINITY;
+  float vmin = INFINITY, vmax = -INFINITY;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     if (t < n_tiles) {
@@ -119,17 +118,16 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
         const bool cand = c < nc;
         const float x = acc[i];
         sc[t][i] = cand ? x : -INFINITY;
-        vmins[i % NCH] = fminf(vmins[i % NCH], cand ? x : INFINITY);
-        vmaxs[i % NCH] = fmaxf(vmaxs[i % NCH], sc[t][i]);
+        vmin = fminf(vmin, cand ? x : INFINITY);
+        vmax = fmaxf(vmax, sc[t][i]);
       }
     } else {
 #pragma unroll
       for (int i = 0; i < 16; ++i) sc[t][i] = -INFINITY;
     }
   }
-#pragma unroll
-  for (int j = 1; j < NCH; ++j) vmins[0] = fminf(vmins[0], vmins[j]), vmaxs[0] = fmaxf(vmaxs[0], vmaxs[j]);
-  const float vmin = min_xor32_f(vmins[0]), vmax = max_xor32_f(vmaxs[0]);
+  vmin = min_xor32_f(vmin);
+  vmax = max_xor32_f(vmax);
 
   // K' = number of scored chunks to keep (the own chunk takes one slot in causal mode).
   // A row keeps every candidate x with x > tau, plus, among the candidates equal to tau_eq,
@@ -225,31 +223,19 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
       }
     }
   };
-  // K' = number of scored chunks to keep (the own chunk takes one slot in causal mode).
-  // A row keeps every candidate x with x > tau, plus, among the candidates equal to tau_eq,
-  // those with chunk index >= iota.  tau is found by bisection between the row's smallest
-  // and largest score and the search stops as soon as exactly K' scores lie above the probe.
-  // The bracket is kept as order-preserving integer keys (lo_k, hi_k]; the first probes
-  // bisect the VALUE range (few steps for ordinary score distributions), later ones the key
-  // range (at most 32 more steps whatever the values).  If the bracket closes first, the
-  // scores inside it are all equal and tie across the cut: the highest chunk indices win.
   if (PEEL && kp <= kGatePeels && __any(open && nc - kp > 1)) {
     // The largest score, the largest below it, .., kp of them: the cut lies right below the last.  Exact unless a score of those occurs twice, which
     // the count below shows.
     float last = INFINITY;
     for (int n = 0; n < kp; ++n) {
-      float best[NCH];
-#pragma unroll
-      for (int j = 0; j < NCH; ++j) best[j] = -INFINITY;
+      float best = -INFINITY;
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         if (t < n_tiles) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) best[i % NCH] = fmaxf(best[i % NCH], sc[t][i] < last ? sc[t][i] : -INFINITY);
+          for (int i = 0; i < 16; ++i) best = fmaxf(best, sc[t][i] < last ? sc[t][i] : -INFINITY);
         }
-#pragma unroll
-      for (int j = 1; j < NCH; ++j) best[0] = fmaxf(best[0], best[j]);
-      last = max_xor32_f(best[0]);
+      last = max_xor32_f(best);
     }
     if (open) {
       uint32_t below = float_order_key(last) - 1u;  // (the float below +0 that compares below it is not -0)

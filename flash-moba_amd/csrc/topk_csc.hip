@@ -59,7 +59,8 @@ __device__ __forceinline__ GateItem gate_item(const TopkParams &p) {
   return GateItem{(int)(gridDim.y - 1 - blockIdx.y), (int)blockIdx.x};
 }
 
-template <typename T, int HD, int NT>
+// PEEL: how a row's cut is found (kGatePeels)
+template <typename T, int HD, bool PEEL, int NT>
 __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_kernel(TopkParams p) {
   constexpr int KS = HD / 16;
   constexpr int VPR = HD / 8;    // 16-byte pieces of a row of chunk means
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(256, (NT == 8 || HD > 128) ? 2 : 4) void topk_gate_
   const int own = a.is_causal && valid && rp >= 0 ? rp / B : -1;
   const int seg = m0 / p.seg_rows;
   uint32_t *selp = p.sel + (int64_t)h * p.W * a.total_q + q0 + r;
-  gate_select<T, HD, NT, true>(ldsTile, qf, lane, n_tiles, nc, kp, own, valid, p.W, [&](int t, uint32_t w) {
+  gate_select<T, HD, NT, PEEL>(ldsTile, qf, lane, n_tiles, nc, kp, own, valid, p.W, [&](int t, uint32_t w) {
     if (valid && hh == 0) selp[(int64_t)t * a.total_q] = w;
     // per-chunk counts of this wave's 32 rows (both halves of the wave hold the rows' words)
     if (p.segcnt != nullptr && __any(w != 0u)) {
@@ -1118,10 +1119,14 @@ extern "C" size_t fmoba_fused_topk_workspace_bytes(int32_t batch, int32_t total_
 }
 
 namespace fmoba {
+// chunks that a row keeps besides its own
+static int gate_winners(const TopkParams &p) { return p.a.is_causal ? p.a.topk - 1 : p.a.topk; }
 template <typename T, int HD, int NT>
 static int launch_gate(const TopkParams &p, dim3 grid, hipStream_t s) {
   const size_t smem = (size_t)NT * 32 * HD * 2 + (size_t)NT * 32 * 4;
-  auto kern = topk_gate_kernel<T, HD, NT>;
+  auto kern = topk_gate_kernel<T, HD, false, NT>;
+  if constexpr (NT < 8)  // (with more chunks so few winners are the stream's)
+    if (gate_winners(p) <= kGatePeels) kern = topk_gate_kernel<T, HD, true, NT>;
   if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     set_error("fused_topk: cannot reserve %zu bytes of LDS", smem);
     return 2;
@@ -1131,8 +1136,6 @@ static int launch_gate(const TopkParams &p, dim3 grid, hipStream_t s) {
 }
 // chunk indices are 16-bit fields of the running winners (topk_gate_stream_kernel) and the forward's step lists
 constexpr int kMaxChunksPerSequence = 65535;
-// chunks that a row keeps besides its own
-static int gate_winners(const TopkParams &p) { return p.a.is_causal ? p.a.topk - 1 : p.a.topk; }
 template <typename T, int HD>
 static int launch_gate_stream(const TopkParams &p, dim3 grid, hipStream_t s) {
   const size_t smem = gate_stream_smem<HD>();
