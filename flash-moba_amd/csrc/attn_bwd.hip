@@ -1637,7 +1637,8 @@ __global__ __launch_bounds__(64 * NW, HD > 64 ? 2 : 4) void attn_bwd_dq_kernel(f
 // sixteen per block of 256: a row's chain of dependent steps (count, ids, order, rows) is mostly waiting, so a wave
 // runs four of them side by side.  Lane li of a group owns the 16-byte piece li of the row.  Over ranked lists the first rows are asked for beside the count; the next four
 // are on their way while four are added (36427 tokens, 32 heads of 64, top-k 4, training step 1408 -> 1359 us; 25298 tokens, 32 heads of 80, top-k 2 1344 -> 1297; plain lists,
-// 82354 tokens, 16 heads of 64, top-k 4, pass alone 268 -> 251; 16 visits as before).
+// 82354 tokens, 16 heads of 64, top-k 4, pass alone 268 -> 251; 16 visits as before).  What it costs: rows at a sequence's beginning that have fewer visits read up to three too many (eleven
+// sequences of 1048 to 8510 tokens, 8 heads of 128, top-k 5, pass alone 91.3 -> 94.3).
 // ------------------------------------------------------------------------------------
 template <typename T, bool RANKED>
 __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd_args a, BwdWs ws, int capl) {
@@ -1707,10 +1708,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
 
 // grid (ceil(max_seqlen_q / rows_per_block), heads, batch), block 256.
 // LPR = 2^lg_lpr lanes cooperate on one row (LPR >= head_dim / 8).
-constexpr int kPrepRows = 4;  // consecutive rows per thread: eight 16-byte loads in flight, and the sums of a wave's rows leave in one store
-// Output rows that the caches cannot hold are read past them: reads alone reach 6.9 TB/s so, 5.5 through the caches.  24571 tokens, 32 heads of 128 (201 MB) 87 -> 76 us, 32768 tokens (the forward's
-// rows are still on their way to memory) 145 -> 131, 36427 tokens, 32 heads of 64 55 -> 46; 8191 tokens, 16 heads of 64 (17 MB) with it 9.1 -> 10.5.
-constexpr int64_t kPrepStreamBytes = (int64_t)64 << 20;
+constexpr int kPrepRows = 4;  // rows per thread: eight 16-byte loads in flight (with one row a thread had two, 4.7 TB/s)
+// Output rows of 128 MB and more are read past the caches.  Through them and past them, us: 16 heads of 128, 48 MB 19.6 and 25.0, 64 MB 25.0 and 26.9, 100 MB 36.5 and 38.0, 128 MB 50.4 and 48.3,
+// 160 MB 69.6 and 60.7, 256 MB 138 and 120, 400 MB 208 and 199, 1 GB 414 and 392; 32 heads of 64, 64 MB 25.1 and 25.2, 100 MB 35.8 and 36.0, 128 MB 48.6 and 45.0, 256 MB 137 and 121.
+// Consecutive rows in a thread, whose sums then leave in one store: 24 MB 11.6 -> 12.4, 160 MB 60.7 -> 63.7, 256 MB 120 -> 127, 1 GB 392 -> 404 (17 to 32 MB of heads of 64 11.9 -> 11.7, 15.9 -> 15.0).
+constexpr int64_t kPrepStreamBytes = (int64_t)128 << 20;
 template <typename T, bool STREAM>
 __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, int lg_lpr, int32_t *tab, RunTable rt, int row_mask, int ztab) {
   const int LPR = 1 << lg_lpr, rows_per_pass = 256 >> lg_lpr;
@@ -1768,13 +1770,13 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
       for (int i = threadIdx.x; i < q0; i += 256) dh[i] = 0.f;
   }
   if (first >= Lq) return;
-  const int r0 = first + (threadIdx.x >> lg_lpr) * kPrepRows, sub = threadIdx.x & (LPR - 1);
+  const int r0 = first + (threadIdx.x >> lg_lpr), sub = threadIdx.x & (LPR - 1);
   const int e = sub * 8;
   const int D = a.head_dim;
   Pack8 o[kPrepRows], g[kPrepRows];
 #pragma unroll
   for (int k = 0; k < kPrepRows; ++k) {
-    const int r = r0 + k;
+    const int r = r0 + k * rows_per_pass;
     o[k] = zero_pack8();
     g[k] = zero_pack8();
     if (r < Lq && e < D) {
@@ -1783,9 +1785,9 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
       g[k] = ld_global16(reinterpret_cast<const uint16_t *>(a.dout) + (int64_t)(q0 + r) * a.do_row_stride + (int64_t)h * a.do_head_stride + e);
     }
   }
-  float sum[kPrepRows];
 #pragma unroll
   for (int k = 0; k < kPrepRows; ++k) {
+    const int r = r0 + k * rows_per_pass;
     float fo[8], fg[8];
     unpack8<T>(o[k], fo);
     unpack8<T>(g[k], fg);
@@ -1793,18 +1795,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(fmoba_attn_bwd_args a, in
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc = fmaf(fo[i], fg[i], acc);
     for (int w = LPR >> 1; w >= 1; w >>= 1) acc += __shfl_xor(acc, w, 64);
-    sum[k] = acc;
-  }
-  float *to = a.softmax_d + (int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b + r0;
-  if (LPR >= kPrepRows) {  // the wave's rows side by side
-    float mine = sum[0];
-#pragma unroll
-    for (int k = 1; k < kPrepRows; ++k) mine = sub == k ? sum[k] : mine;
-    if (sub < kPrepRows && r0 + sub < Lq) to[sub] = mine;
-  } else if (sub == 0) {
-#pragma unroll
-    for (int k = 0; k < kPrepRows; ++k)
-      if (r0 + k < Lq) to[k] = sum[k];
+    if (r < Lq && sub == 0) a.softmax_d[(int64_t)h * ((int64_t)a.total_q + 128 * (int64_t)a.batch) + q0 + 128 * b + r] = acc;
   }
 }
 
