@@ -24,17 +24,19 @@ struct PoolExtra {
 // one request of 3000 keys 21.3 -> 16.6, of 60000 48.5 -> 36.5; 20 of 256 to 65536, 32 over 32 heads 740 -> 694.  Heads of 256 too, though the query rows leave
 // three waves per SIMD of eight: one request of 60000 keys, 8 heads 81.9 -> 62.4, eight of 1000 to 30000, 32 over 4 heads 61.4 -> 56.2, 32 of 512 to 32768, 32
 // heads 907 -> 878.
-// Keys that the chip's last cache (256 MB) cannot hold until the attention comes to them are read past the caches: one sequence of 32768 keys, 32 heads of 128 (268 MB) 67.7 -> 44.6 us,
-// 262144 keys, 16 heads 241 -> 195, decode of 16 requests with 8 key heads (380 MB) 60.1 -> 57.4.  Keys that it holds are read again from there: 67485 keys, 16 heads of 96 (207 MB)
-// 40.7 us, past the caches 44.6, and the decode step after it 30.6 and 35.7.
+// Keys that the chip's last cache (256 MB) cannot hold until the attention comes to them are read past the caches.  The pass alone, through them and past them: plain, 32 heads of 128, 160 MB of keys
+// 39.9 and 33.1 us, 224 MB 55.4 and 40.8, 256 MB 62.2 and 45.4, 400 MB 99 and 71; with scores, 16 requests, 8 key heads of 128, 160 MB 30.5 and 29.0, 256 MB 45.9 and 43.9, 400 MB 70.4 and 65.8.
+// Keys that it holds are read again from there: 67485 keys, 16 heads of 96 (207 MB) 40.7 us, past the caches 44.6, and the decode step after it 30.6 and 35.7.
 constexpr int64_t kPoolStreamBytes = (int64_t)256 << 20;
-// STREAM: known at the launch (a second loop in the scoring instances costs a short decode step 0.4 us); the others find out from the offsets.
+// STREAM: with scores, read past the caches, known at the launch.  Plain pooling, whose arguments do not say how many keys there are: found out from the offsets; calls that are below the line
+// even if every sequence is as long as the longest take the instance without (a third offset and a second loop: 8192 tokens, 16 heads of 128 7.4 -> 7.8 us, of 64 5.1 -> 5.5, 3072 tokens, 8 heads
+// 5.1 -> 5.4, 24571 tokens, 8 heads 11.8 -> 12.1).
 template <typename T, bool MANY, int HD, bool STREAM>
 __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, PoolExtra x, FewGate few) {
   const int c = blockIdx.x, b = blockIdx.y;
   const int seq_start = a.cu_seqlens_k[b], seq_end = a.cu_seqlens_k[b + 1];
   int total_k = 0;
-  if constexpr (HD == 0) {
+  if constexpr (HD == 0 && STREAM) {
     total_k = a.cu_seqlens_k[a.batch];
 #if defined(__HIP_DEVICE_COMPILE__)
     asm volatile("" : "+s"(total_k));  // awaited with the other two, not in front of the rows
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(fmoba_mean_pool_args a, 
         for (int i = 0; i < 8; ++i) acc[i] += f0[i];
       }
     };
-    if constexpr (HD > 0) {
+    if constexpr (HD > 0 || !STREAM) {
       sum_rows(std::integral_constant<bool, STREAM>{});
     } else {
       if ((int64_t)total_k * nvec * 16 >= kPoolStreamBytes)
@@ -251,17 +253,19 @@ static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &
     scored.block_heads = 64 / (a->head_dim / 8);
     grid.z = ceil_div(a->heads_k, scored.block_heads);
   }
+  if (few == nullptr) total_k = (int64_t)a->batch * a->max_chunks * a->chunk;  // (no more than)
+  const bool stream_keys = total_k > (kPoolStreamBytes - 1) / (nvec * 16);
   auto pick = [&](auto t) {
     typedef decltype(t) T;
-    auto scoring = [&](auto hd_) {
+    auto instance = [&](auto hd_) {
       constexpr int HD = decltype(hd_)::value;
-      if (total_k * nvec * 16 >= kPoolStreamBytes) return many ? mean_pool_kernel<T, true, HD, true> : mean_pool_kernel<T, false, HD, true>;
+      if (stream_keys) return many ? mean_pool_kernel<T, true, HD, true> : mean_pool_kernel<T, false, HD, true>;
       return many ? mean_pool_kernel<T, true, HD, false> : mean_pool_kernel<T, false, HD, false>;
     };
-    if (hd == 64) return scoring(std::integral_constant<int, 64>{});
-    if (hd == 128) return scoring(std::integral_constant<int, 128>{});
-    if (hd == 256) return scoring(std::integral_constant<int, 256>{});
-    return many ? mean_pool_kernel<T, true, 0, false> : mean_pool_kernel<T, false, 0, false>;
+    if (hd == 64) return instance(std::integral_constant<int, 64>{});
+    if (hd == 128) return instance(std::integral_constant<int, 128>{});
+    if (hd == 256) return instance(std::integral_constant<int, 256>{});
+    return instance(std::integral_constant<int, 0>{});
   };
   hipLaunchKernelGGL(a->dtype == FMOBA_DTYPE_BF16 ? pick(bf16_t()) : pick(f16_t()), grid, dim3(256), 0, s, *a, extra, scored);
   FMOBA_LAUNCH_CHECK("mean_pool");
