@@ -428,9 +428,11 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
 // headers, order, rows) is mostly waiting, so a wave runs four of them side by side.  Lane li of a group owns the
 // 16-byte pieces li, li + 16, .. (NP of them) of the row, whose elements are of type E
 // (NORM: divided by the visit's sum of probabilities).
-// RANKED: the slots are in key-block order and none of the first `visits` is empty.  The headers and the first rows are asked for beside the count, and what U does not divide
-// together: a row of few visits was a chain of loads (16-bit rows, pass alone: 8192 tokens, 16 heads of 128, top-k 8 52.4 -> 50.6 us; parts of prompts 39.8 -> 37.5; 5312 tokens, top-k 7
-// 32.8 -> 30.4; 16 and 22 visits as before, 790 and 750).  What bounds rows of many visits is the memory: their reads alone, by this pattern, reach 7.1 TB/s, with the output rows
+// RANKED: the slots are in key-block order and none of the first `visits` is empty.  The headers and the first rows are asked for beside the count, whole groups of U together without
+// branches, and what U does not divide together under them: a row of few visits was a chain of loads (16-bit rows, pass alone: 8192 tokens, 16 heads of 128, top-k 8 52.2 -> 50.2 us; parts of prompts
+// 38.4 -> 36.7; 24000 tokens, 8 heads of 128, top-k 5 61.1 -> 54.2; of 96, top-k 7 70.0 -> 57.5; 16 and 22 visits as before, 792 and 750).  Whole groups under the branches of the remainder hold each
+// other up where few workgroups wait for their rows: 137 rows, 8 heads of 128, 16 visits 5.9 -> 6.7, without 6.0; 300 rows of 64, 12 visits 5.3 -> 5.8, without 5.3.
+// What bounds rows of many visits is the memory: their reads alone, by this pattern, reach 7.1 TB/s, with the output rows
 // written between them (a sixteenth of the bytes) 5.7.  The next rows on their way while rows are added: 22 visits 750 -> 820, for the registers.  Over plain lists the rows' places come from LDS: nothing is early, and whole
 // groups of U and single rows take 60 us where groups with branches take 67 (12182 tokens, 16 heads of 64, top-k 4).
 template <typename T, typename E, int NP, bool NORM, bool RANKED>
@@ -533,7 +535,16 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
           }
       };
       if constexpr (RANKED) {
-        for (int t = 0; t < cntb; t += U) {
+        int t = 0;
+        for (; t + U <= cntb; t += U) {
+          if (base + t > 0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) load(x[u], base + t + u);
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) add(x[u], sWgt[sg][t + u]);
+        }
+        if (t < cntb) {
           if (base + t > 0) fetch(x, base + t, n);
 #pragma unroll
           for (int u = 0; u < U; ++u)
