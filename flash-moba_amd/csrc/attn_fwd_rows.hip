@@ -572,8 +572,8 @@ __global__ __launch_bounds__(SPLIT * KH * RW * 64, 2) void attn_fwd_rows_kernel(
     const uint32_t dst = lds_ring + (uint32_t)__builtin_amdgcn_readfirstlane(stage * (int)SM::tile + feeder * NI * 1024);
     if (key0 + 64 <= Lk) {
       const uint16_t *base = g + (uint64_t)(uint32_t)key0 * row_stride;
-      global_to_lds16_run<0, (NI < 4 ? NI : 4)>(lof, base, dst);
-      if constexpr (NI > 4) global_to_lds16_run<0, NI - 4>(lof + 4, base, dst + 4096u);
+      global_to_lds16_run<(NI < 4 ? NI : 4)>(lof, base, dst);
+      if constexpr (NI > 4) global_to_lds16_run<NI - 4>(lof + 4, base, dst + 4096u);
     } else {
 #pragma unroll
       for (int i = 0; i < NI; ++i) {

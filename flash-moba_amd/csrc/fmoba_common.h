@@ -875,27 +875,22 @@ __device__ __forceinline__ void global_to_lds16_sbase(uint32_t lane_byte_off, co
   (void)lane_byte_off, (void)uniform_base, (void)lds_base;
 #endif
 }
-// N of these loads to consecutive kilobytes from lds_base + 1024 FIRST on.  The instruction's offset moves both addresses, so that one setting of m0 serves
-// all: load i's lane offsets are run_offset(byte offset from the base, FIRST + i).  (m0 cannot be set before the load in front has taken it: a wave that sets it for each of eight loads
+// N of these loads to consecutive kilobytes from lds_base on.  The instruction's offset moves both addresses, so that one setting of m0 serves all: load i's lane offsets
+// are run_offset(byte offset from the base, i).  (m0 cannot be set before the load in front has taken it: a wave that sets it for each of eight loads
 // issues them in 412 clocks, with one setting for four in 96, where nothing else is in the way of them; with four waves and more the vector memory path is.)
 constexpr uint32_t kRunBias = 4096;
 __device__ __forceinline__ constexpr uint32_t run_offset(uint32_t byte_off, int i) { return byte_off + (kRunBias - 1024u * (uint32_t)i); }
-template <int FIRST, int N>
+template <int N>
 __device__ __forceinline__ void global_to_lds16_run(const uint32_t *off, const void *uniform_base, uint32_t lds_base) {
-  static_assert(N >= 1 && N <= 4 && FIRST >= 0 && FIRST + N <= 4, "offsets of twelve bits");
+  static_assert(N >= 2 && N <= 4, "offsets of twelve bits");
 #if defined(__HIP_DEVICE_COMPILE__)
   const uint8_t *from = reinterpret_cast<const uint8_t *>(uniform_base) - kRunBias;
-  if constexpr (N == 1)
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(off[0]), "s"(from), "s"(lds_base), "n"(FIRST * 1024) : "memory");
-  else if constexpr (N == 2)
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2 offset:%4\n\tglobal_load_lds_dwordx4 %1, %2 offset:%5" ::"v"(off[0]), "v"(off[1]), "s"(from),
-                 "s"(lds_base), "n"(FIRST * 1024), "n"(FIRST * 1024 + 1024)
-                 : "memory");
+  if constexpr (N == 2)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" ::"v"(off[0]), "v"(off[1]), "s"(from), "s"(lds_base) : "memory");
   else if constexpr (N == 3)
-    asm volatile(
-        "s_mov_b32 m0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %3 offset:%5\n\tglobal_load_lds_dwordx4 %1, %3 offset:%6\n\tglobal_load_lds_dwordx4 %2, %3 offset:%7" ::"v"(off[0]),
-        "v"(off[1]), "v"(off[2]), "s"(from), "s"(lds_base), "n"(FIRST * 1024), "n"(FIRST * 1024 + 1024), "n"(FIRST * 1024 + 2048)
-        : "memory");
+    asm volatile("s_mov_b32 m0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %3\n\tglobal_load_lds_dwordx4 %1, %3 offset:1024\n\tglobal_load_lds_dwordx4 %2, %3 offset:2048" ::"v"(off[0]),
+                 "v"(off[1]), "v"(off[2]), "s"(from), "s"(lds_base)
+                 : "memory");
   else
     asm volatile(
         "s_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024\n\tglobal_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, "
