@@ -894,17 +894,29 @@ static int rows_sets(const fmoba_attn_fwd_args &a) {
 // barrier.  Above head dimension 64, where the rings of two sets leave a unit room for one workgroup anyway, from sequences of 1024 keys on (shorter walks lose
 // in the sums what they gain: heads of 128, two sequences of 128 tokens 13.9 -> 14.9 us, four of 512 19.7 -> 20.0).  The pass alone: 2048 tokens, 8 heads of 128 33.8 -> 32.1 us, not causal 33.9 ->
 // 31.3, 16 heads 45.4 -> 43.9, 4096 tokens, 8 heads 75.1 -> 70.3, 3495 tokens, 8 heads of 96 45.3 -> 41.3, 3 x 1024 tokens, 8 heads of 128 28.3 -> 28.6, not causal 38.0 -> 36.2.
-// Not up to 64, where two workgroups of four waves fit a unit and one of eight does: in calls of 257 to 400 workgroups 2 x 1536 tokens, 8 heads 21.8 -> 23.9, 3 x 1024 17.2 -> 21.1, not causal
-// 1024 + 2048 tokens 29.9 -> 39.6, 1100 tokens, 16 heads 20.1 -> 27.5; causal 1100 tokens, 16 heads 17.5 -> 17.0, 1024 + 2048, 8 heads 24.3 -> 23.9.
-static bool rows_halves(const fmoba_attn_fwd_args &a) { return a.head_dim > 64 && a.max_seqlen_k >= kRowsFourSetsKeys; }
+// Up to 64 a unit holds one such workgroup where it holds two of four waves, and what is more than there are units starts when the first are done.  That is no loss where the longest walk
+// covers it, in causal calls whose items start longest first and whose heads fill the turns of the XCDs (each XCD has its share of every sequence).  A workgroup costs its walk and what ten to
+// fourteen blocks of 64 keys take (start, choice, list, sums); if the sequences are about alike, the `later` workgroups are the rows' first `later` / (heads * batch) blocks, which start when walks
+// of that length are done.  Workgroups that find no block count (a grid for the longest sequence has some in the others).  Calls of heads of 64, us, without and with: 1024 + 2048 tokens,
+// 8 heads 27.7 and 26.6, 1700 + 900 25.5 and 24.3, 2500 + 500 31.2 and 29.5, 3000 35.3 and 33.9, 1100, 16 heads 21.0 and 20.2; refused: 2 x 1536, 8 heads 24.5 and 26.3, 3 x 1024 20.7 and
+// 23.7, 1112 + 1512 25.6 and 28.3, 1400, 16 heads 23.5 and 24.0, 2 x 1200, 8 heads 22.3 and 21.9, 24 heads of 1024 21.0 and 24.1, four sequences of 407 to 2641, 4 heads 35.1 and 51.8, not causal
+// (the pass alone) 1100, 16 heads 20.1 and 27.5, 1024 + 2048, 8 heads 29.9 and 39.6.  Beyond 400 workgroups of uneven sequences: 3000 + 600, 8 heads 35.9 and 37.7, 3500 + 300 + 200 39.1 and 42.8.
+constexpr int kRowsHalves = 400, kRowsHalvesCost = 14;
+static bool rows_halves(const fmoba_attn_fwd_args &a) {
+  if (a.max_seqlen_k < kRowsFourSetsKeys) return false;
+  if (a.head_dim > 64) return true;
+  if (!a.is_causal || a.total_q != a.total_k || a.max_seqlen_q != a.max_seqlen_k || a.heads % 8 != 0) return false;
+  const int nb = ceil_div(a.max_seqlen_q, 64);
+  const bool listed = item_order(a.total_q, a.max_seqlen_q, a.batch, a.heads, 64, true) == kListedLongestFirst;
+  const int64_t items = a.heads * (listed ? ((int64_t)a.total_q + 63 * a.batch) / 64 : (int64_t)a.batch * nb);
+  return items <= kRowsHalves && 2 * (items - kRowsFourSets) <= (int64_t)(nb - kRowsHalvesCost) * a.heads * a.batch;
+}
 template <typename T, int HD>
 static int launch_rows(const fmoba_attn_fwd_args &a, const uint32_t *bm, int nw, hipStream_t s, const RowGate *gate = nullptr) {
   const int sets = rows_sets(a);
   if constexpr (HD <= 64)
     if (sets == 4) return launch_rows_split<T, HD, 2, 4, 1>(a, bm, nw, gate, s);
-  if constexpr (HD > 64)
-    if (sets == 2 && rows_halves(a)) return launch_rows_split<T, HD, 2, 2, 2>(a, bm, nw, gate, s);
-  if (sets == 2) return launch_rows_split<T, HD, 2, 2, 1>(a, bm, nw, gate, s);
+  if (sets == 2) return rows_halves(a) ? launch_rows_split<T, HD, 2, 2, 2>(a, bm, nw, gate, s) : launch_rows_split<T, HD, 2, 2, 1>(a, bm, nw, gate, s);
   if constexpr (HD <= 64)
     if (a.total_q <= (int64_t)1536 * a.batch) return launch_rows_split<T, HD, 2, 1, 1>(a, bm, nw, gate, s);
   return launch_rows_split<T, HD, 4, 1, 1>(a, bm, nw, gate, s);

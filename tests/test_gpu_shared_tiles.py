@@ -35,3 +35,10 @@ def test_output_and_log_sum_exp(lens_q, lens_k, H, Hk, D, chunk, topk, dtype, ca
     seen = torch.isfinite(want_lse)
     assert torch.equal(torch.isfinite(lse), seen) and (lse[~seen] == float("inf")).all()
     assert_close("lse", lse[seen], want_lse[seen], 2e-3, 1e-3)
+
+
+# heads up to 64: more workgroups than units and no more than the longest walk covers
+@pytest.mark.parametrize("lens,H,Hk,D,chunk,topk", [([1024, 2048], 8, 8, 64, 128, 4), ([1057, 1, 64], 16, 4, 40, 64, 9), ([2301], 8, 1, 32, 256, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_narrow_heads(lens, H, Hk, D, chunk, topk, dtype):
+    test_output_and_log_sum_exp(lens, None, H, Hk, D, chunk, topk, dtype, True)
