@@ -432,6 +432,8 @@ __global__ __launch_bounds__((64 * FwdColSmem<HD, KB>::NW), 2) void attn_fwd_col
 // branches, and what U does not divide together under them: a row of few visits was a chain of loads (16-bit rows, pass alone: 8192 tokens, 16 heads of 128, top-k 8 52.2 -> 50.2 us; parts of prompts
 // 38.4 -> 36.7; 24000 tokens, 8 heads of 128, top-k 5 61.1 -> 54.2; of 96, top-k 7 70.0 -> 57.5; 16 and 22 visits as before, 792 and 750).  Whole groups under the branches of the remainder hold each
 // other up where few workgroups wait for their rows: 137 rows, 8 heads of 128, 16 visits 5.9 -> 6.7, without 6.0; 300 rows of 64, 12 visits 5.3 -> 5.8, without 5.3.
+// Rows of fp32 (heads above 128) are awaited: short sequences have rows of fewer visits, and what is read in vain is four times as much (seven sequences of 21 to 652 tokens, 8 heads of 256, top-k 4
+// 11.8 -> 15.0 us with early rows, 11.5 without; 9000 tokens, top-k 7 96.5 -> 94.4 and 92.7).
 // What bounds rows of many visits is the memory: their reads alone, by this pattern, reach 7.1 TB/s, with the output rows
 // written between them (a sixteenth of the bytes) 5.7.  The next rows on their way while rows are added: 22 visits 750 -> 820, for the registers.  Over plain lists the rows' places come from LDS: nothing is early, and whole
 // groups of U and single rows take 60 us where groups with branches take 67 (12182 tokens, 16 heads of 64, top-k 4).
@@ -483,11 +485,12 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
       load(y[u], i0 + u);
     }
   };
+  constexpr bool kEarly = NP == 1;  // (rows of 16 bits)
   Pack8 x[U][NP];  // (of ranked rows)
   float2 head = {-INFINITY, 0.f};
   if constexpr (RANKED) {  // asked for beside the count: what lies behind it is not used
     if (li < ws.cap) head = hdr2[li];
-    if (mine) fetch(x, 0, ws.cap);
+    if (kEarly && mine) fetch(x, 0, ws.cap);
   }
   for (int base = 0; base < nmax; base += 16) {
     const int cntb = min(16, max(n - base, 0));
@@ -537,7 +540,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
       if constexpr (RANKED) {
         int t = 0;
         for (; t + U <= cntb; t += U) {
-          if (base + t > 0) {
+          if (!kEarly || base + t > 0) {
 #pragma unroll
             for (int u = 0; u < U; ++u) load(x[u], base + t + u);
           }
@@ -545,7 +548,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine_kernel(fmoba_attn_fwd_ar
           for (int u = 0; u < U; ++u) add(x[u], sWgt[sg][t + u]);
         }
         if (t < cntb) {
-          if (base + t > 0) fetch(x, base + t, n);
+          if (!kEarly || base + t > 0) fetch(x, base + t, n);
 #pragma unroll
           for (int u = 0; u < U; ++u)
             if (t + u < cntb) add(x[u], sWgt[sg][t + u]);
