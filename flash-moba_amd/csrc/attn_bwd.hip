@@ -1709,7 +1709,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_combine_kernel(fmoba_attn_bwd
 // grid (ceil(max_seqlen_q / rows_per_block), heads, batch), block 256.
 // LPR = 2^lg_lpr lanes cooperate on one row (LPR >= head_dim / 8).
 constexpr int kPrepRows = 4;  // rows per thread: eight 16-byte loads in flight (with one row a thread had two, 4.7 TB/s)
-// Output rows of 128 MB and more are read past the caches.  Through them and past them, us: 16 heads of 128, 48 MB 19.6 and 25.0, 64 MB 25.0 and 26.9, 100 MB 36.5 and 38.0, 128 MB 50.4 and 48.3,
+// Output rows of 128 MB and more whose heads are whole cache lines are read past the caches (a line that two heads share would be read twice: 400 MB of rows, 16 heads of 80 198 -> 220 us, of 96
+// 191 -> 204, of 112 194 -> 212, 32 heads of 40 267 -> 294).  Through them and past them, us: 16 heads of 128, 48 MB 19.6 and 25.0, 64 MB 25.0 and 26.9, 100 MB 36.5 and 38.0, 128 MB 50.4 and 48.3,
 // 160 MB 69.6 and 60.7, 256 MB 138 and 120, 400 MB 208 and 199, 1 GB 414 and 392; 32 heads of 64, 64 MB 25.1 and 25.2, 100 MB 35.8 and 36.0, 128 MB 48.6 and 45.0, 256 MB 137 and 121.
 // Consecutive rows in a thread, whose sums then leave in one store: 24 MB 11.6 -> 12.4, 160 MB 60.7 -> 63.7, 256 MB 120 -> 127, 1 GB 392 -> 404 (17 to 32 MB of heads of 64 11.9 -> 11.7, 15.9 -> 15.0).
 constexpr int64_t kPrepStreamBytes = (int64_t)128 << 20;
@@ -1961,7 +1962,7 @@ static int run_bwd(const fmoba_attn_bwd_args &a, const BwdWs &ws, int phases, hi
     const int nx = ceil_div(a.max_seqlen_q, (256 >> lg_lpr) * kPrepRows);
     const RunTable rt = bwd_run_table(a);
     const int ztab = partials ? 0 : (int)ceil_div64(ceil_div(rt.cols, 4), nx);
-    auto prep = (int64_t)a.total_q * a.heads * a.head_dim * 2 >= kPrepStreamBytes ? bwd_prep_kernel<T, true> : bwd_prep_kernel<T, false>;
+    auto prep = a.head_dim % 64 == 0 && (int64_t)a.total_q * a.heads * a.head_dim * 2 >= kPrepStreamBytes ? bwd_prep_kernel<T, true> : bwd_prep_kernel<T, false>;
     if (a.batch + ztab <= 65535) {
       hipLaunchKernelGGL(prep, dim3(nx, a.heads, a.batch + ztab), dim3(256), 0, s, a, lg_lpr, ws.tab, rt, ws.row_mask, ztab);
     } else {  // (more planes than a launch has)
