@@ -254,7 +254,8 @@ static int mean_pool_run(const fmoba_mean_pool_args *a, const fmoba::PoolExtra &
     grid.z = ceil_div(a->heads_k, scored.block_heads);
   }
   if (few == nullptr) total_k = (int64_t)a->batch * a->max_chunks * a->chunk;  // (no more than)
-  const bool stream_keys = total_k > (kPoolStreamBytes - 1) / (nvec * 16);
+  // (narrow rows that share cache lines: 32 requests, 500 MB of keys of one head of 80 170.5 us, past the caches 174, of two of 40 166.4 and 170.9; two of 80 102.4 and 99.9)
+  const bool stream_keys = (nvec % 8 == 0 || nvec >= 16) && total_k > (kPoolStreamBytes - 1) / (nvec * 16);
   auto pick = [&](auto t) {
     typedef decltype(t) T;
     auto instance = [&](auto hd_) {
