@@ -42,7 +42,7 @@ CONFIGS = {
     "sweep16k": ([16384, 16384], 16, 128, 128, 8, True),
     "sweep64k": ([65536, 65536], 16, 128, 128, 8, True),
 }
-# the arithmetic type of the 16-bit inputs: bf16 as BASELINE.json's configs say, fp16 where the reference's own sweep uses it
+# the arithmetic type of the 16-bit inputs: bf16 for the named configurations, fp16 where the reference's own sweep uses it
 CONFIG_DTYPE = {"sweep16k": "fp16", "sweep64k": "fp16"}
 
 

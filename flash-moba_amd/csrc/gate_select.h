@@ -131,7 +131,7 @@ __device__ __forceinline__ void gate_select(uint32_t ldsTile, const Pack8 (&qf)[
 
   // K' = number of scored chunks to keep (the own chunk takes one slot in causal mode).
   // A row keeps every candidate x with x > tau, plus, among the candidates equal to tau_eq,
-  // those with chunk index >= iota.  tau is found by bisection between the row's smallest
+  // those with chunk index >= iota.  tau is found below the K'-th of the best scores (PEEL), or by bisection between the row's smallest
   // and largest score and the search stops as soon as exactly K' scores lie above the probe.
   // The bracket is kept as order-preserving integer keys (lo_k, hi_k]; the first probes
   // bisect the VALUE range (few steps for ordinary score distributions), later ones the key

@@ -1,7 +1,7 @@
 // Fused top-k block gating and deterministic CSC build.
 //
-//   topk_gate_kernel : scores S^T = KM * Q^T on MFMA, per-row exact top-k by bisection on
-//                      order-preserving keys held in registers (no score matrix, no sorted
+//   topk_gate_kernel : scores S^T = KM * Q^T on MFMA, per-row exact top-k by the best scores one by one or by bisection on
+//                      order-preserving keys, scores held in registers (no score matrix, no sorted
 //                      list and no per-row index list ever reaches HBM); emits one selection
 //                      BIT per (row, chunk) and per-(2048-row segment, chunk) counts.
 //   csc_scan_kernel  : per (sequence, head) scan of the counts -> col_nnz, col_offsets

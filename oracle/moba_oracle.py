@@ -504,7 +504,7 @@ def moba_dense_ref(q, k, v, cu_seqlens_q, cu_seqlens_k, moba_chunk_size: int, mo
 def topk_gap_mask(gates, cu_seqlens_q, moba_topk: int, rel: float = 1e-3) -> torch.Tensor:
     """(T,H) bool: True where the row's selection is unambiguous, i.e. the gap between the
     last selected and the first rejected candidate score exceeds `rel` relative
-    ("bit-exact wherever the reference score gap exceeds 1e-3
+    (the bar of the comparison: "bit-exact wherever the reference score gap exceeds 1e-3
     relative"; moba_test_utils.py:835-843 uses the same idea with an absolute eps).
     `gates` is the list returned by fused_topk(..., return_gate=True)."""
     cuq = cu_seqlens_q.cpu().numpy().astype(np.int64)
